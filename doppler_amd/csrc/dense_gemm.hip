@@ -4,11 +4,9 @@
 //   f16 activations    the same with f16 weights, v_mfma_f32_32x32x16_f16 (products of rows an f16 cache holds)
 //   f32 activations    v_mfma_f32_32x32x2_f32 on the weights widened (exactly) to f32: a true 32-bit product
 //
-// Weights [N][ldw] and activations [M][lda] are both read along k, 64 elements (bf16) or 32 (f32) at a time; K is
-// a multiple of 64, which the owner of the buffers reaches with zero padding.  A tile of each goes through
-// registers into one of two LDS buffers (loads for the next tile are in flight while the current one is
-// multiplied; one barrier per tile).  LDS rows hold their 16-byte pieces at slot (piece ^ row) & 7, so that both
-// the row-wise stores and the column-wise fragment reads touch every bank once.
+// Weights [N][ldw] and activations [M][lda] are both read along k; K is a multiple of 64, which the owner of the buffers
+// reaches with zero padding.  16-bit operands: gemm_wide.h (256 x 256, 256 x 128 or 128 x 128 tiles straight from memory into LDS).
+// 32-bit: 64-row tiles, 32 k at a time through registers.
 //
 // The epilogue serves two outputs, because the projections that read one normalised row are stored as one
 // stacked matrix: columns below n_first are (alpha * acc + bias) * column scale (+ residual) in f32, columns from n_first
@@ -26,6 +24,7 @@
 
 #include "dense_device.h"
 #include "experts.h"
+#include "gemm_wide.h"
 
 namespace {
 
@@ -166,106 +165,31 @@ __device__ __forceinline__ void store_glu(const GemmArgs& a, const TilePlace& p,
   }
 }
 
-// WM x WN waves; a wave computes TM x TN accumulator tiles of 32 x 32.
-template <int WM, int WN, int TM, int TN, bool F16, int ACT, bool GROUPED = false, bool GLU = false>
-__global__ __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : TM * TN == 2 ? 3 : 4) void gemm_16bit_kernel(const GemmArgs a) {
-  static_assert(!GLU || TN == 2, "a wave's two tiles are the gate and the up value");
-  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, THREADS = 64 * WM * WN;
-  constexpr int PA = BM * 8 / THREADS, PB = BN * 8 / THREADS;      // 16-byte pieces per thread and tile
-  static_assert(BM * 8 % THREADS == 0 && BN * 8 % THREADS == 0, "whole pieces per thread");
-  __shared__ __align__(16) u32x4_t lds[2][(BM + BN) * 8];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wm = wave / WN, wn = wave % WN;
+// 16-bit operands (gemm_wide.h).
+template <class Tile, bool F16, int ACT, bool GROUPED = false, bool GLU = false>
+__global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const GemmArgs a) {
+  static_assert(!GLU || Tile::FB == 1, "a wave's two tiles are the gate and the up value");
+  extern __shared__ __align__(16) char smem[];
   const int tile = dh::xcd_contiguous(blockIdx.x, a.tiles_m * a.tiles_n);
   TilePlace place;
-  if (!place_tile<GROUPED>(a, tile % a.tiles_m, BM, &place)) return;
-  const int m0 = place.m0, n0 = (tile / a.tiles_m) * BN;
-
-  // this thread's pieces: rows past the matrix repeat its last row (their products are never stored)
-  const uint16_t* pa[PA];
-  const uint16_t* pb[PB];
-  int sa[PA], sb[PB];
+  if (!place_tile<GROUPED>(a, tile % a.tiles_m, Tile::BM, &place)) return;
+  const int m0 = place.m0, n0 = (tile / a.tiles_m) * Tile::BN;
+  const int k0 = blockIdx.y * a.k_slice, nk = min(a.k_slice, a.K - k0) >> 6;
+  f32x16_t acc[2 * Tile::FA][2 * Tile::FB];
+  const int64_t first = GROUPED ? 0 : m0;       // gathered rows lie anywhere
+  dh::wide_product<Tile, F16>(
+      acc, static_cast<const uint16_t*>(a.A) + first * a.lda,
+      [&](int row) { return (uint32_t)((source_row<GROUPED>(a, place, row) - first) * a.lda * 2); }, place.W + (int64_t)n0 * a.ldw,
+      [&](int row) { return (uint32_t)(min(row, a.N - 1 - n0) * a.ldw * 2); }, 2u * k0, nk, smem);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = m0 + 64 * Tile::FA * (wave / Tile::WN), n = n0 + 64 * Tile::FB * (wave % Tile::WN);
 #pragma unroll
-  for (int r = 0; r < PA; r++) {
-    const int p = tid + THREADS * r, row = p >> 3, c = p & 7;
-    pa[r] = static_cast<const uint16_t*>(a.A) + source_row<GROUPED>(a, place, row) * a.lda + 8 * c;
-    sa[r] = row * 8 + (c ^ (row & 7));
-  }
-#pragma unroll
-  for (int r = 0; r < PB; r++) {
-    const int p = tid + THREADS * r, row = p >> 3, c = p & 7;
-    pb[r] = place.W + (int64_t)min(n0 + row, a.N - 1) * a.ldw + 8 * c;
-    sb[r] = BM * 8 + row * 8 + (c ^ (row & 7));
-  }
-  u32x4_t ra[PA], rb[PB];
-#define DH_GEMM_LOAD(kt_)                                                                                              \
-  do {                                                                                                                 \
-    _Pragma("unroll") for (int r = 0; r < PA; r++) ra[r] = *reinterpret_cast<const u32x4_t*>(pa[r] + 64 * (kt_));      \
-    _Pragma("unroll") for (int r = 0; r < PB; r++) rb[r] = *reinterpret_cast<const u32x4_t*>(pb[r] + 64 * (kt_));      \
-  } while (0)
-#define DH_GEMM_STORE(b_)                                                                                              \
-  do {                                                                                                                 \
-    _Pragma("unroll") for (int r = 0; r < PA; r++) lds[b_][sa[r]] = ra[r];                                             \
-    _Pragma("unroll") for (int r = 0; r < PB; r++) lds[b_][sb[r]] = rb[r];                                             \
-  } while (0)
-
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-
-  const int k0 = blockIdx.y * a.k_slice;
-  const int nk = min(a.k_slice, a.K - k0) >> 6;
-#pragma unroll
-  for (int r = 0; r < PA; r++) pa[r] += k0;
-#pragma unroll
-  for (int r = 0; r < PB; r++) pb[r] += k0;
-  DH_GEMM_LOAD(0);
-  DH_GEMM_STORE(0);
-  __syncthreads();
-  const int frow = lane & 31, fk = lane >> 5;
-  for (int kt = 0; kt < nk; kt++) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) DH_GEMM_LOAD(kt + 1);
-#pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      u32x4_t fa[TM], fb[TN];
-      const int piece = 2 * ks + fk;
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const int row = 32 * (wm * TM + i) + frow;
-        fa[i] = lds[buf][row * 8 + (piece ^ (row & 7))];
-      }
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int row = 32 * (wn * TN + j) + frow;
-        fb[j] = lds[buf][BM * 8 + row * 8 + (piece ^ (row & 7))];
-      }
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-          if constexpr (F16)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, fa[i]), __builtin_bit_cast(f16x8_t, fb[j]), acc[i][j], 0, 0, 0);
-          else
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fa[i]), __builtin_bit_cast(bf16x8_t, fb[j]), acc[i][j], 0, 0, 0);
-        }
-    }
-    if (kt + 1 < nk) DH_GEMM_STORE(buf ^ 1);
-    __syncthreads();
-  }
-#undef DH_GEMM_LOAD
-#undef DH_GEMM_STORE
-#pragma unroll
-  for (int i = 0; i < TM; i++) {
+  for (int i = 0; i < 2 * Tile::FA; i++) {
     if constexpr (GLU) {
-      store_glu(a, place, acc[i][0], acc[i][1], m0 + 32 * (wm * TM + i), n0 + 32 * wn * TN, lane);
+      store_glu(a, place, acc[i][0], acc[i][1], m + 32 * i, n, lane);
     } else {
 #pragma unroll
-      for (int j = 0; j < TN; j++) store_tile<ACT>(a, place, acc[i][j], m0 + 32 * (wm * TM + i), n0 + 32 * (wn * TN + j), lane);
+      for (int j = 0; j < 2 * Tile::FB; j++) store_tile<ACT>(a, place, acc[i][j], m + 32 * i, n + 32 * j, lane);
     }
   }
 }
@@ -350,74 +274,186 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   }
 }
 
+// Sums of the k slices in slice order; blockIdx.y = row, VEC columns per thread (N a multiple of VEC).
+template <int VEC>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int slices) {
+  const int m = blockIdx.y, n = VEC * (blockIdx.x * 256 + threadIdx.x);
+  if (n >= a.N) return;
   const int64_t total = (int64_t)a.M * a.N;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    float s = 0.f;
+  const float* p = a.parts + (int64_t)m * a.N + n;
+  float s[VEC] = {};
 #pragma unroll 4
-    for (int k = 0; k < slices; k++) s += a.parts[k * total + i];
-    put(a, (int)(i / a.N), (int)(i % a.N), s);
+  for (int k = 0; k < slices; k++) {
+    if constexpr (VEC == 4) {
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p + k * total);
+#pragma unroll
+      for (int e = 0; e < 4; e++) s[e] += v[e];
+    } else {
+      s[0] += p[k * total];
+    }
   }
+#pragma unroll
+  for (int e = 0; e < VEC; e++) put(a, m, n + e, s[e]);
 }
 
-template <int WM, int WN, int TM, int TN, bool F16, int ACT>
-int launch_16bit(const char* op, GemmArgs a, int slices) {
-  a.tiles_m = (int)dh::ceil_div(a.M, 32 * WM * TM);
-  a.tiles_n = (int)dh::ceil_div(a.N, 32 * WN * TN);
+// Tiles of the 16-bit products, and what a k step (64 elements) of one costs in ns: `alone` with few workgroups on the device, `one`
+// with one on every compute unit, `full` with as many as fit (the two larger tiles: one, which takes more than half of the LDS).  The
+// device slows its clock under matrix-core load, so a step gets dearer as more compute units join, and idle ones are not all
+// lost.  Fitted to M = 17 .. 2048, N = 1024 .. 18464, K = 1024 .. 16384 with each tile and 1 .. 8 slices: the choice is within
+// 10 % of the best of them at nearly all.  Against the 128 x 128 and 64 x 64 tiles through registers that were here before:
+// 2048 x 18464 x 4096 391 -> 300 us, 2048 x 4096 x 16384 312 -> 253, 1531 x 2048 x 6144 75 -> 45, 512 x 4096 x 4096 38 -> 29,
+// 40 x 4096 x 16384 101 -> 39.
+using Tile256x256 = dh::WideTile<2, 4, 2, 1>;
+using Tile256x128 = dh::WideTile<4, 2, 1, 1>;
+using Tile128x128 = dh::WideTile<2, 2, 1, 1>;
+struct TileCost {
+  int bm, bn, per_cu;
+  float alone, one, full, start;      // start: ns outside the k loop
+};
+constexpr TileCost kTiles[] = {{256, 256, 1, 1000.f, 1720.f, 1720.f, 8000.f},
+                               {256, 128, 1, 520.f, 930.f, 930.f, 5500.f},
+                               {128, 128, 2, 330.f, 480.f, 1050.f, 4500.f}};
+constexpr int kMaxSlices = 8, kMinSliceSteps = 8;
+
+struct TileChoice {
+  int tile, slices;
+};
+// The cheapest tile and number of k slices.  Slices cost the round trip of their raw sums and a second launch.
+TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices) {
+  const int64_t cus = dh::num_cus(), steps = K / 64;
+  TileChoice best{0, 1};
+  double least = 1e30;
+  for (int i = 0; i < 3; i++) {
+    const TileCost& c = kTiles[i];
+    for (int s = 1; s <= most_slices && (s == 1 || steps / s >= kMinSliceSteps); s++) {
+      const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s, slots = cus * c.per_cu, left = groups % slots;
+      const double f = (double)left / cus;
+      const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (0.7 + 0.3 * f / c.per_cu);
+      const double per_group = (double)dh::ceil_div(steps, s);
+      double t = per_group * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + c.start;
+      if (s > 1) t += 3500.0 + 4.0 * M * N * (2 * s + 1) / 4000.0;      // a launch, and 4 bytes a sum at about 4 TB/s
+      if (t < least) {
+        least = t;
+        best = TileChoice{i, s};
+      }
+    }
+  }
+  return best;
+}
+
+// A tile's rows are addressed by 32-bit byte offsets (rows millions of elements long are out of reach).
+bool within_reach(int64_t rows, int64_t ld, int64_t K) { return 2 * (std::min<int64_t>(rows, 256) * ld + K) < (int64_t)1 << 32; }
+
+// LDS beyond 64 KB is asked for once per kernel.
+template <class Tile, bool F16, int ACT, bool GROUPED, bool GLU>
+int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
+  auto kern = gemm_16bit_kernel<Tile, F16, ACT, GROUPED, GLU>;
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLds);
+  DH_CHECK_HIP(op, set);
+  if (!within_reach(a.M, a.lda, a.K) || !within_reach(a.N, a.ldw, a.K))
+    return dh::fail(1, "[%s] rows %lld and %lld elements apart are out of reach", op, (long long)a.lda, (long long)a.ldw);
+  if (!GROUPED) a.tiles_m = (int)dh::ceil_div(a.M, Tile::BM);
+  a.tiles_n = (int)dh::ceil_div(a.N, Tile::BN);
+  hipLaunchKernelGGL(kern, dim3(a.tiles_m * a.tiles_n, slices), dim3(Tile::kThreads), Tile::kLds, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+template <bool F16, int ACT, bool GLU>
+int launch_16bit(const char* op, GemmArgs a, const TileChoice& pick) {
   a.k_slice = a.K;
-  if (slices > 1) {
-    a.k_slice = (int)dh::ceil_div(a.K / 64, slices) * 64;
+  int slices = 1;
+  if (pick.slices > 1) {
+    a.k_slice = (int)dh::ceil_div(a.K / 64, pick.slices) * 64;
     slices = (int)dh::ceil_div(a.K, a.k_slice);
     size_t bytes = 0;
     a.parts = dh::splitk_workspace(&bytes);
   }
-  hipLaunchKernelGGL((gemm_16bit_kernel<WM, WN, TM, TN, F16, ACT>), dim3(a.tiles_m * a.tiles_n, slices), dim3(64 * WM * WN), 0, dh::stream(), a);
-  DH_CHECK_LAUNCH(op);
-  if (a.parts) {
-    const unsigned grid = (unsigned)std::min<int64_t>(dh::ceil_div((int64_t)a.M * a.N, 256), 4096);
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3(grid), dim3(256), 0, dh::stream(), a, slices);
-    DH_CHECK_LAUNCH(op);
+  int rc;
+  switch (pick.tile) {
+    case 0: rc = launch_16bit_kernel<Tile256x256, F16, ACT, false, GLU>(op, a, slices); break;
+    case 1: rc = launch_16bit_kernel<Tile256x128, F16, ACT, false, GLU>(op, a, slices); break;
+    default: rc = launch_16bit_kernel<Tile128x128, F16, ACT, false, GLU>(op, a, slices); break;
   }
+  if (rc || !a.parts) return rc;
+  const bool vec = a.N % 4 == 0;
+  const dim3 grid((unsigned)dh::ceil_div(a.N, vec ? 1024 : 256), (unsigned)a.M);
+  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, dim3(256), 0, dh::stream(), a, slices);
+  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, dim3(256), 0, dh::stream(), a, slices);
+  DH_CHECK_LAUNCH(op);
   return 0;
 }
+int launch_act(const char* op, const GemmArgs& a, bool f16, const TileChoice& pick) {
+  if (f16) return a.n_first == a.N ? launch_16bit<true, kNoSecond, false>(op, a, pick)
+                  : a.act == DH_ACT_NONE ? launch_16bit<true, DH_ACT_NONE, false>(op, a, pick)
+                                         : launch_16bit<true, kAnyAct, false>(op, a, pick);
+  if (a.n_first == a.N) return launch_16bit<false, kNoSecond, false>(op, a, pick);
+  if (a.act == DH_ACT_RELU2) return launch_16bit<false, DH_ACT_RELU2, false>(op, a, pick);
+  if (a.act == DH_ACT_GELU_ERF) return launch_16bit<false, DH_ACT_GELU_ERF, false>(op, a, pick);
+  return launch_16bit<false, kAnyAct, false>(op, a, pick);
+}
 
-template <int WM, int WN, int TM, int TN>
-int launch_tile(const char* op, const GemmArgs& a, bool f16, int slices) {
-  if (f16) return a.n_first == a.N ? launch_16bit<WM, WN, TM, TN, true, kNoSecond>(op, a, slices)
-                  : a.act == DH_ACT_NONE ? launch_16bit<WM, WN, TM, TN, true, DH_ACT_NONE>(op, a, slices)
-                                         : launch_16bit<WM, WN, TM, TN, true, kAnyAct>(op, a, slices);
-  if (a.n_first == a.N) return launch_16bit<WM, WN, TM, TN, false, kNoSecond>(op, a, slices);
-  if (a.act == DH_ACT_RELU2) return launch_16bit<WM, WN, TM, TN, false, DH_ACT_RELU2>(op, a, slices);
-  if (a.act == DH_ACT_GELU_ERF) return launch_16bit<WM, WN, TM, TN, false, DH_ACT_GELU_ERF>(op, a, slices);
-  return launch_16bit<WM, WN, TM, TN, false, kAnyAct>(op, a, slices);
+// A product whose rows are out of reach goes in halves.
+int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
+  if (a.M > 1 && !within_reach(a.M, a.lda, a.K)) {
+    GemmArgs low = a, high = a;
+    const int64_t m = low.M = a.M / 2;
+    high.M = a.M - low.M;
+    high.A = static_cast<const uint16_t*>(a.A) + m * a.lda;
+    if (a.residual) high.residual = a.residual + m * a.ldc;
+    if (a.C) high.C = a.C + m * a.ldc;
+    if (a.C2) high.C2 = static_cast<char*>(a.C2) + m * a.ldc2 * (a.c2_dtype == DH_F32 ? 4 : 2);
+    const int rc = dense_16bit(op, low, f16);
+    return rc ? rc : dense_16bit(op, high, f16);
+  }
+  if (a.N > 1 && !within_reach(a.N, a.ldw, a.K)) {
+    GemmArgs low = a, high = a;
+    const int n = low.N = a.N / 2;
+    high.N = a.N - n;
+    low.n_first = std::min(a.n_first, n);
+    high.n_first = a.n_first - low.n_first;
+    high.W = a.W + (int64_t)n * a.ldw;
+    if (a.bias) high.bias = a.bias + n;
+    if (a.col_scale) high.col_scale = a.col_scale + n;
+    if (a.residual) high.residual = a.residual + n;
+    if (a.C) high.C = a.C + n;
+    if (a.C2) high.C2 = static_cast<char*>(a.C2) + (int64_t)(n - low.n_first) * (a.c2_dtype == DH_F32 ? 4 : 2);
+    const int rc = dense_16bit(op, low, f16);
+    return rc ? rc : dense_16bit(op, high, f16);
+  }
+  size_t ws_bytes = 0;
+  (void)dh::splitk_workspace(&ws_bytes);
+  const int most = (int)std::max<size_t>(1, std::min<size_t>(kMaxSlices, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
+  TileChoice pick = choose_tile(a.M, a.N, a.K, most);
+  const int env_tile = dh::tuning_int("DH_DENSE_TILE", -1), env_slices = dh::tuning_int("DH_DENSE_SLICES", 0);
+  if (env_tile >= 0) pick.tile = env_tile;
+  if (env_slices) pick.slices = std::min(most, env_slices);
+  return launch_act(op, a, f16, pick);
 }
 
 // Expert products; the grouped ones launch as many row tiles as the table has room for.
 template <bool GROUPED, bool GLU>
-int launch_experts(const char* op, GemmArgs a, int a_dtype, int bm) {
+int launch_experts(const char* op, GemmArgs a, int a_dtype) {
   a.k_slice = a.K;
   if (a_dtype == DH_F32) {
     constexpr int TN = GLU ? 2 : 1;
     a.tiles_n = (int)dh::ceil_div(a.N, 64 * TN);
     if (!GROUPED) a.tiles_m = (int)dh::ceil_div(a.M, 64);
     hipLaunchKernelGGL((gemm_f32_kernel<TN, GROUPED, GLU>), dim3(a.tiles_m * a.tiles_n), dim3(256), 0, dh::stream(), a);
-  } else {
-    a.tiles_n = (int)dh::ceil_div(a.N, 128);
-    if (!GROUPED) a.tiles_m = (int)dh::ceil_div(a.M, bm);
-    if (bm == 128)
-      hipLaunchKernelGGL((gemm_16bit_kernel<2, 2, 2, 2, false, kNoSecond, GROUPED, GLU>), dim3(a.tiles_m * a.tiles_n), dim3(256), 0, dh::stream(), a);
-    else
-      hipLaunchKernelGGL((gemm_16bit_kernel<2, 2, 1, 2, false, kNoSecond, GROUPED, GLU>), dim3(a.tiles_m * a.tiles_n), dim3(256), 0, dh::stream(), a);
+    DH_CHECK_LAUNCH(op);
+    return 0;
   }
-  DH_CHECK_LAUNCH(op);
-  return 0;
+  if constexpr (GROUPED) {
+    return launch_16bit_kernel<Tile128x128, false, kNoSecond, true, GLU>(op, a, 1);
+  } else {
+    return launch_16bit<false, kNoSecond, GLU>(op, a, choose_tile(a.M, a.N, a.K, 1));
+  }
 }
 
 }  // namespace
 
 namespace dh {
 
-int expert_tile_rows(int a_dtype, int rows, int groups) { return a_dtype == DH_F32 ? 64 : rows >= 96 * groups ? 128 : 64; }
+int expert_tile_rows(int a_dtype) { return a_dtype == DH_F32 ? 64 : Tile128x128::BM; }
 
 int experts_glu(const char* op, const ExpertRows& rows, const void* A, int a_dtype, int64_t lda, const uint16_t* W, int64_t ldw, int M,
                 int N, int K, void* out, int out_dtype, int64_t ld_out) {
@@ -426,10 +462,9 @@ int experts_glu(const char* op, const ExpertRows& rows, const void* A, int a_dty
   a.C2 = out; a.c2_dtype = out_dtype; a.ldc2 = ld_out; a.rows = rows;
   if (rows.tiles) {
     a.tiles_m = rows.max_tiles;
-    return launch_experts<true, true>(op, a, a_dtype, rows.tile_rows);
+    return launch_experts<true, true>(op, a, a_dtype);
   }
-  const int bm = ceil_div(M, 128) * ceil_div(N, 128) >= num_cus() ? 128 : 64;
-  return launch_experts<false, true>(op, a, a_dtype, bm);
+  return launch_experts<false, true>(op, a, a_dtype);
 }
 
 int experts_down(const char* op, const ExpertRows& rows, const void* A, int a_dtype, int64_t lda, const uint16_t* W, int64_t ldw, int N,
@@ -438,7 +473,7 @@ int experts_down(const char* op, const ExpertRows& rows, const void* A, int a_dt
   a.A = A; a.W = W; a.lda = lda; a.ldw = ldw; a.N = N; a.K = K; a.alpha = 1.f;
   a.C = out; a.ldc = ld_out; a.n_first = N; a.rows = rows;
   a.tiles_m = rows.max_tiles;
-  return launch_experts<true, false>(op, a, a_dtype, rows.tile_rows);
+  return launch_experts<true, false>(op, a, a_dtype);
 }
 
 }  // namespace dh
@@ -480,21 +515,5 @@ extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, con
     DH_CHECK_LAUNCH(op);
     return 0;
   }
-  // 128 x 128 tiles (two workgroups per compute unit) where they fill the device, 64 x 64 otherwise.  (256 x 256 and
-  // 256 x 128 tiles measured the same or slower at every shape tried: one workgroup per compute unit hides less.)
-  const int cus = dh::num_cus();
-  auto tiles = [&](int bm, int bn) { return dh::ceil_div(M, bm) * dh::ceil_div(N, bn); };
-  static const int env_tile = dh::tuning_int("DH_DENSE_TILE", 0);
-  static const int env_slices = dh::tuning_int("DH_DENSE_SLICES", 0);
-  // slices of at least 1024 k, as many as fill the device, within the workspace
-  size_t ws_bytes = 0;
-  (void)dh::splitk_workspace(&ws_bytes);
-  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(K / 1024, (int64_t)(ws_bytes / ((size_t)M * N * sizeof(float)))));
-  auto slices_for = [&](int64_t t, int per_cu) { return std::min(most, std::max<int64_t>(1, (int64_t)per_cu * cus / t)); };
-  const bool big_enough = tiles(128, 128) >= cus || (M > 64 && tiles(128, 128) * most >= cus);
-  const int pick = env_tile ? env_tile : big_enough ? 128 : 64;
-  const int64_t t = tiles(pick, pick);
-  const int slices = env_slices ? (int)std::min<int64_t>(env_slices, most) : t >= cus ? 1 : (int)slices_for(t, pick == 128 ? 2 : 4);
-  const bool f16 = a_dtype == DH_F16;
-  return pick == 128 ? launch_tile<2, 2, 2, 2>(op, a, f16, slices) : launch_tile<2, 2, 1, 1>(op, a, f16, slices);
+  return dense_16bit(op, a, a_dtype == DH_F16);
 }

@@ -366,7 +366,7 @@ PortionSpace portion_space(const dh_experts* s, int operand, int T) {
   const size_t n = (size_t)T * s->top, elem = operand == DH_F32 ? 4 : 2;
   p.ld_z = (logits(s) + 3) / 4 * 4;
   p.ld_y = (s->hidden + 3) / 4 * 4;
-  p.tile_rows = dh::expert_tile_rows(operand, (int)n, s->experts);
+  p.tile_rows = dh::expert_tile_rows(operand);
   p.max_tiles = (int)(n / p.tile_rows + std::min<size_t>(n, s->experts));
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t r = at; at += up256(bytes); return r; };
@@ -442,6 +442,12 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   if (!d_h || !d_x || !d_workspace) return dh::fail(1, "[%s] null pointer", op);
   if (!aligned(d_h) || !aligned(d_workspace)) return dh::fail(1, "[%s] pointers must be 16-byte aligned", op);
   if ((int64_t)T * spec->top > (1 << 24)) return dh::fail(1, "[%s] %d tokens are too many for one portion", op, T);
+  if (operand == DH_BF16 && T > 1 && (int64_t)T * spec->K >= (int64_t)1 << 31) {
+    // gathered rows are addressed by 32-bit byte offsets: more than 4 GB of them go in two portions
+    const int half = T / 2;
+    if (int rc = dh_experts_prefill(spec, d_h, operand, d_x, ld_x, d_workspace, half)) return rc;
+    return dh_experts_prefill(spec, static_cast<const uint16_t*>(d_h) + (int64_t)half * spec->K, operand, d_x + (int64_t)half * ld_x, ld_x, d_workspace, T - half);
+  }
   const PortionSpace p = portion_space(spec, operand, T);
   char* w = static_cast<char*>(d_workspace);
   auto f32 = [&](size_t at) { return reinterpret_cast<float*>(w + at); };

@@ -138,6 +138,29 @@ def test_dense_matmul(L, M, N, K, first, operand):
             assert (got2[:, N - first:] == 9.0).all()
 
 
+# the larger tiles of the 16-bit products: k steps of either parity, edges in both directions, both outputs in one tile
+@pytest.mark.parametrize("M,N,K,first", [(2060, 6150, 1536, 6150), (2060, 6150, 1600, 3001), (1540, 4090, 2048, 33), (1537, 4097, 2112, 4000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_matmul_large_tiles(L, M, N, K, first, dtype):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(dtype)
+    scale, res = torch.randn(N, generator=g, device="cuda"), torch.randn(M, first, generator=g, device="cuda")
+    C, C2 = res.clone(), torch.full((M, N - first + 2), 9.0, dtype=dtype, device="cuda")
+    code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul_scaled(A.data_ptr(), code, K, W.data_ptr(), K, M, N, K, 1.5, None, scale.data_ptr(), C.data_ptr(), C.data_ptr(),
+                                        first, first, C2.data_ptr(), code, N - first + 2, capi.ACT_RELU2))
+    capi.check(L.dh_sync())
+    acc = 1.5 * (A.double() @ W.double().T)
+    # unit products: sums of up to 2112 terms in 32 bits stay within 2^-24 * sqrt(K) * a few of them
+    assert (C.double() - (acc[:, :first] * scale[:first].double() + res.double())).abs().max() < 5e-5
+    if first < N:
+        want = acc[:, first:].clamp(min=0).square()
+        assert ((C2[:, :N - first].double() - want).abs() <= 2.0 ** (-8 if dtype == torch.bfloat16 else -10) * want + 1e-4).all()
+        assert (C2[:, N - first:] == 9.0).all()
+
+
 def test_f32_products_are_not_reduced_precision(L):
     """Activations that differ from a constant in their last bits only: bf16- or TF32-like operands would lose them."""
     M, N, K = 40, 70, 256

@@ -795,7 +795,8 @@ def runScale(input, scale, count=None, outputBuffer=None, inplace=False, **_igno
     n = _nbytes(input) // 4 if count is None else count
     if n * 4 > _nbytes(input):
         raise DopplerHipError("[Scale] count=%d exceeds the input buffer." % n)
-    out = input.buffer if inplace else _out(outputBuffer, n * 4)
+    # the result has the input's shape: a buffer made here holds all of it, also where only `count` elements are scaled
+    out = input.buffer if inplace else _out(outputBuffer, n * 4 if outputBuffer is not None else max(n, int(np.prod(input.shape))) * 4)
     capi.check(_lib().dh_scale(_ptr(input), _ptr(out), n, float(scale)))
     return Tensor(out, input.dtype, input.shape, "scale_output")
 

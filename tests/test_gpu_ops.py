@@ -782,6 +782,16 @@ def test_bias_add_and_scale_bit_exact():
     assert same.buffer is xt.buffer and np.array_equal(ops.readTensor(xt).reshape(x.shape), x * s)
 
 
+def test_scale_of_a_part_holds_its_whole_shape():
+    """readTensor reads a tensor's whole shape: a part's buffer as short as the part sends that read past its end, and the copy is
+    refused where the allocation ends."""
+    x = synth.normal_f32((6, 1536), seed=4452)
+    part = ops.runScale(ops.tensorFromNumpy(x), 0.3, count=1536)
+    assert tuple(part.shape) == x.shape and part.buffer.numel() >= x.nbytes
+    got = ops.readTensor(part).reshape(x.shape)
+    assert np.array_equal(got[0], x[0] * np.float32(0.3)) and not got[1:].any()
+
+
 def test_split_qkv_exact():
     """split_qkv.js: a pure copy, so every output element equals its source bit for bit."""
     T, qs, ks, vs = 7, 2048, 512, 384

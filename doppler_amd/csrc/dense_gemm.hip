@@ -196,29 +196,33 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const Gem
 
 // The 32-bit product: four waves, a 64 x 64 TN tile, 32 k at a time.  Both tiles sit in LDS as f32 rows of 32 + 4
 // words; a lane reads four consecutive k of its row and feeds four instructions with them (k-slot l >> 5 of
-// instruction e stands for k = 8 s + 4 (l >> 5) + e on both sides).
+// instruction e stands for k = 8 s + 4 (l >> 5) + e on both sides).  A matrix-core instruction takes 64 cycles here, so a tile's 16
+// of them cover the loads of the next (registers, then the other LDS buffer; one barrier a tile).  What was far from the 157 TFLOP/s of
+// the part (115 reached at 2048 rows) is a narrow product that leaves compute units without a tile: k slices (blockIdx.y) as for the
+// 16-bit ones, M x N x K without -> with them: 301 x 1024 x 4096 85 -> 36 us, 17 x 1024 x 4096 85 -> 14, 64 x 4096 x 16384 360 -> 86.
 template <int TN, bool GROUPED, bool GLU>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   static_assert(!GLU || TN == 2, "a wave's two tiles are the gate and the up value");
   constexpr int BM = 64, BN = 64 * TN, BK = 32, ROW = BK + 4;
-  __shared__ __align__(16) float la[BM * ROW];
-  __shared__ __align__(16) float lb[BN * ROW];
+  __shared__ __align__(16) float la[2][BM * ROW];
+  __shared__ __align__(16) float lb[2][BN * ROW];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wm = wave >> 1, wn = wave & 1;
   const int tile = dh::xcd_contiguous(blockIdx.x, a.tiles_m * a.tiles_n);
   TilePlace place;
   if (!place_tile<GROUPED>(a, tile % a.tiles_m, BM, &place)) return;
   const int m0 = place.m0, n0 = (tile / a.tiles_m) * BN;
+  const int k0 = blockIdx.y * a.k_slice, nk = min(a.k_slice, a.K - k0) / BK;
   // A: 64 rows x 8 pieces of 4 floats, two per thread; W: 64 TN rows x 4 pieces of 8 elements, TN per thread
   const float* pa[2];
   const uint16_t* pb[TN];
 #pragma unroll
   for (int r = 0; r < 2; r++) {
     const int p = tid + 256 * r;
-    pa[r] = static_cast<const float*>(a.A) + source_row<GROUPED>(a, place, p >> 3) * a.lda + 4 * (p & 7);
+    pa[r] = static_cast<const float*>(a.A) + source_row<GROUPED>(a, place, p >> 3) * a.lda + 4 * (p & 7) + k0;
   }
 #pragma unroll
-  for (int r = 0; r < TN; r++) pb[r] = place.W + (int64_t)min(n0 + 64 * r + (tid >> 2), a.N - 1) * a.ldw + 8 * (tid & 3);
+  for (int r = 0; r < TN; r++) pb[r] = place.W + (int64_t)min(n0 + 64 * r + (tid >> 2), a.N - 1) * a.ldw + 8 * (tid & 3) + k0;
   f32x4_t ra[2];
   u32x4_t rb[TN];
   f32x16_t acc[TN];
@@ -226,45 +230,44 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   for (int j = 0; j < TN; j++)
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[j][e] = 0.f;
-  const int nk = a.K / BK;
+  auto load = [&](int kt) {
 #pragma unroll
-  for (int r = 0; r < 2; r++) ra[r] = *reinterpret_cast<const f32x4_t*>(pa[r]);
+    for (int r = 0; r < 2; r++) ra[r] = *reinterpret_cast<const f32x4_t*>(pa[r] + BK * kt);
 #pragma unroll
-  for (int r = 0; r < TN; r++) rb[r] = *reinterpret_cast<const u32x4_t*>(pb[r]);
-  for (int kt = 0; kt < nk; kt++) {
-    __syncthreads();
+    for (int r = 0; r < TN; r++) rb[r] = *reinterpret_cast<const u32x4_t*>(pb[r] + BK * kt);
+  };
+  auto store = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < 2; r++) {
       const int p = tid + 256 * r;
-      *reinterpret_cast<f32x4_t*>(&la[(p >> 3) * ROW + 4 * (p & 7)]) = ra[r];
+      *reinterpret_cast<f32x4_t*>(&la[buf][(p >> 3) * ROW + 4 * (p & 7)]) = ra[r];
     }
 #pragma unroll
     for (int r = 0; r < TN; r++) {
-      float* wb = &lb[(64 * r + (tid >> 2)) * ROW + 8 * (tid & 3)];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        wb[2 * e] = dh::bf16_low(rb[r][e]);
-        wb[2 * e + 1] = dh::bf16_high(rb[r][e]);
-      }
+      f32x4_t* wb = reinterpret_cast<f32x4_t*>(&lb[buf][(64 * r + (tid >> 2)) * ROW + 8 * (tid & 3)]);
+      wb[0] = f32x4_t{dh::bf16_low(rb[r][0]), dh::bf16_high(rb[r][0]), dh::bf16_low(rb[r][1]), dh::bf16_high(rb[r][1])};
+      wb[1] = f32x4_t{dh::bf16_low(rb[r][2]), dh::bf16_high(rb[r][2]), dh::bf16_low(rb[r][3]), dh::bf16_high(rb[r][3])};
     }
-    __syncthreads();
-    if (kt + 1 < nk) {
-#pragma unroll
-      for (int r = 0; r < 2; r++) ra[r] = *reinterpret_cast<const f32x4_t*>(pa[r] + BK * (kt + 1));
-#pragma unroll
-      for (int r = 0; r < TN; r++) rb[r] = *reinterpret_cast<const u32x4_t*>(pb[r] + BK * (kt + 1));
-    }
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int kt = 0; kt < nk; kt++) {
+    const int buf = kt & 1;
+    if (kt + 1 < nk) load(kt + 1);
 #pragma unroll
     for (int s = 0; s < BK / 8; s++) {
       const int k = 8 * s + 4 * (lane >> 5);
-      const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(&la[(32 * wm + (lane & 31)) * ROW + k]);
+      const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(&la[buf][(32 * wm + (lane & 31)) * ROW + k]);
 #pragma unroll
       for (int j = 0; j < TN; j++) {
-        const f32x4_t fb = *reinterpret_cast<const f32x4_t*>(&lb[(32 * (wn * TN + j) + (lane & 31)) * ROW + k]);
+        const f32x4_t fb = *reinterpret_cast<const f32x4_t*>(&lb[buf][(32 * (wn * TN + j) + (lane & 31)) * ROW + k]);
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc[j], 0, 0, 0);
       }
     }
+    if (kt + 1 < nk) store(buf ^ 1);
+    __syncthreads();
   }
   if constexpr (GLU) {
     store_glu(a, place, acc[0], acc[1], m0 + 32 * wm, n0 + 32 * wn * TN, lane);
@@ -358,6 +361,14 @@ int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
   DH_CHECK_LAUNCH(op);
   return 0;
 }
+int launch_reduce(const char* op, const GemmArgs& a, int slices) {
+  const bool vec = a.N % 4 == 0;
+  const dim3 grid((unsigned)dh::ceil_div(a.N, vec ? 1024 : 256), (unsigned)a.M);
+  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, dim3(256), 0, dh::stream(), a, slices);
+  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, dim3(256), 0, dh::stream(), a, slices);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
 template <bool F16, int ACT, bool GLU>
 int launch_16bit(const char* op, GemmArgs a, const TileChoice& pick) {
   a.k_slice = a.K;
@@ -375,12 +386,7 @@ int launch_16bit(const char* op, GemmArgs a, const TileChoice& pick) {
     default: rc = launch_16bit_kernel<Tile128x128, F16, ACT, false, GLU>(op, a, slices); break;
   }
   if (rc || !a.parts) return rc;
-  const bool vec = a.N % 4 == 0;
-  const dim3 grid((unsigned)dh::ceil_div(a.N, vec ? 1024 : 256), (unsigned)a.M);
-  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, dim3(256), 0, dh::stream(), a, slices);
-  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, dim3(256), 0, dh::stream(), a, slices);
-  DH_CHECK_LAUNCH(op);
-  return 0;
+  return launch_reduce(op, a, slices);
 }
 int launch_act(const char* op, const GemmArgs& a, bool f16, const TileChoice& pick) {
   if (f16) return a.n_first == a.N ? launch_16bit<true, kNoSecond, false>(op, a, pick)
@@ -428,6 +434,36 @@ int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
   if (env_tile >= 0) pick.tile = env_tile;
   if (env_slices) pick.slices = std::min(most, env_slices);
   return launch_act(op, a, f16, pick);
+}
+
+// k slices of a 32-bit product.  Workgroups on a compute unit share its matrix cores, so the one with the most of them ends last: 64 k of a
+// tile take 1.35 us alone there and 1.1 us each in company (0.85 at the full rate).  Slices cost as in choose_tile.
+int dense_f32(const char* op, GemmArgs a) {
+  a.tiles_m = (int)dh::ceil_div(a.M, 64);
+  a.tiles_n = (int)dh::ceil_div(a.N, 64);
+  size_t ws_bytes = 0;
+  float* ws = dh::splitk_workspace(&ws_bytes);
+  const int64_t steps = a.K / 64, tiles = (int64_t)a.tiles_m * a.tiles_n;
+  const int most = (int)std::max<size_t>(1, std::min<size_t>(16, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
+  const int env_slices = dh::tuning_int("DH_F32_SLICES", 0);
+  int slices = 1;
+  double least = 1e30;
+  for (int s = 1; s <= most && (s == 1 || steps / s >= 2); s++) {
+    const int64_t together = dh::ceil_div(tiles * s, dh::num_cus());
+    double t = (together == 1 ? 1350.0 : 1100.0 * together) * dh::ceil_div(steps, s);
+    if (s > 1) t += 3500.0 + 4.0 * a.M * a.N * (2 * s + 1) / 4000.0;
+    if (t < least) {
+      least = t;
+      slices = s;
+    }
+  }
+  if (env_slices) slices = std::min(most, env_slices);
+  a.k_slice = (int)dh::ceil_div(steps, slices) * 64;
+  slices = (int)dh::ceil_div(a.K, a.k_slice);
+  if (slices > 1) a.parts = ws;
+  hipLaunchKernelGGL((gemm_f32_kernel<1, false, false>), dim3((unsigned)tiles, slices), dim3(256), 0, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return slices > 1 ? launch_reduce(op, a, slices) : 0;
 }
 
 // Expert products; the grouped ones launch as many row tiles as the table has room for.
@@ -508,12 +544,6 @@ extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, con
   a.M = M; a.N = N; a.K = K; a.alpha = alpha; a.bias = d_bias; a.residual = d_residual; a.col_scale = d_col_scale;
   a.C = d_C; a.ldc = ldc; a.n_first = n_first;
   a.C2 = d_C2; a.ldc2 = ldc2; a.c2_dtype = c2_dtype; a.act = activation;
-  if (a_dtype == DH_F32) {
-    a.tiles_m = (int)dh::ceil_div(M, 64);
-    a.tiles_n = (int)dh::ceil_div(N, 64);
-    hipLaunchKernelGGL((gemm_f32_kernel<1, false, false>), dim3(a.tiles_m * a.tiles_n), dim3(256), 0, dh::stream(), a);
-    DH_CHECK_LAUNCH(op);
-    return 0;
-  }
+  if (a_dtype == DH_F32) return dense_f32(op, a);
   return dense_16bit(op, a, a_dtype == DH_F16);
 }

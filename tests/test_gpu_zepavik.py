@@ -161,6 +161,22 @@ def test_dense_matmul_large_tiles(L, M, N, K, first, dtype):
         assert (C2[:, N - first:] == 9.0).all()
 
 
+# 32-bit products in k slices: one tile, a ragged last slice, a narrow product, as many slices as there are
+@pytest.mark.parametrize("M,N,K", [(1, 3, 128), (17, 70, 4160), (65, 130, 1088), (301, 1024, 4096), (40, 129, 16448)])
+def test_dense_matmul_f32_slices(L, M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda")
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16)
+    bias, C = torch.randn(N, generator=g, device="cuda"), torch.full((M, N + 4), 9.0, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), capi.F32, K, W.data_ptr(), K, M, N, K, -0.5, bias.data_ptr(), None, C.data_ptr(), N + 4, N, None, 0,
+                                 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    want = -0.5 * (A.double() @ W.double().T) + bias.double()
+    # unit products: sums of up to 16448 terms in 32 bits
+    assert (C[:, :N].double() - want).abs().max() < 5e-5 and (C[:, N:] == 9.0).all()
+
+
 def test_f32_products_are_not_reduced_precision(L):
     """Activations that differ from a constant in their last bits only: bf16- or TF32-like operands would lose them."""
     M, N, K = 40, 70, 256

@@ -1,47 +1,43 @@
 // Q4_K prefill GEMM for gfx950: C[M,N] = alpha * A[M,K] . dequant(W)[N,K]^T for M >= 16, and
 // the fused gate/up projection with gated activation, on the matrix cores.
 //
-// Tiles: a wave computes a 64 x 64 (or 32 x 32) quadrant with v_mfma_f32_32x32x16_f16 (f32
-// accumulators), four waves a 128 x 128 (64 x 64) tile, and a workgroup is one or two such groups
-// stacked along M against the same weight tile: 256 x 128 with eight waves for large problems.
-// K advances 64 at a time: one 32-byte nibble chunk of a super-block (low nibbles = sub-block
-// 2c, high = 2c+1) per weight row.
-//   weights  a thread loads 8 or 16 nibble bytes of a row + the block header and rebuilds the
-//            weights as f16: (w & 0x000F000F) | 0x64006400 is the pair (1024 + q) in f16, one
-//            packed subtract and one packed fma with (d*sc, -dmin*mn) finish them: about 2
-//            vector ops per weight, paid once per workgroup tile (hence the tall tiles).
-//   A        packed once per product by a pre-pass (pack_a_row_kernel / pack_a_kernel): each
-//            row scaled by the power of two that puts its largest element at 2^14, rounded to
-//            f16, k-permuted, rows zero-padded to a multiple of 64.  The GEMM tiles then copy
-//            16-byte pieces into LDS, no conversion in the K loop, and the epilogue divides the
-//            row factor out again, exactly: activations beyond the f16 range (65504) neither
-//            overflow nor lose small rows to subnormals.
-// Both tiles sit in LDS as [row][64 k] with a 16-byte pad (conflict-free 16-byte fragment
-// reads) and are double-buffered, one barrier per K step.
-// The K loop is bound by instruction issue, not by memory (with every load served from the
-// first-level cache it runs 3 % faster) and not by the matrix cores alone (they are busy for
-// half of the loop's cycles at the 1.84 GHz the part holds under this load).  Measured on this
-// part: a wave issues an independent vector instruction every 5 cycles and a dependent one every
-// 8, a matrix-core instruction occupies its pipe for 32, and a wave may issue 4 vector
-// instructions behind a matrix-core instruction at no cost.  Hence:
-//   * every wave both multiplies and produces, and the producer's work of a step (LDS stores of
-//     the A tile, scale unpack, nibble dwords, the loads two tiles ahead) is dealt out in pieces
-//     behind the matrix-core instructions of the same step, in program order pinned with
-//     scheduling barriers;
+// Two kernels.  Both take the activations packed once per product by a pre-pass (pack_a_row_kernel / pack_a_kernel): each row
+// scaled by the power of two that puts its largest element at 2^14, rounded to f16, k-permuted (packed_place: the order in which a
+// dword of nibbles comes out; a contraction index may be permuted freely when both operands agree), rows zero-padded to a
+// multiple of 64.  The K loops copy them as they are, and the epilogue divides the row factor out again, exactly: activations
+// beyond the f16 range (65504) neither overflow nor lose small rows to subnormals.  And both rebuild weights as f16 from the
+// nibbles with magic numbers ((w & 0x000F000F) | 0x64006400 is the pair (1024 + q) in f16), a packed subtract and a packed
+// fma with (d * sc, -dmin * mn).
+//
+// q4k_wide_kernel (large products).  Tiles of up to 256 x 256 (eight waves, 128 x 64 each).  Packed activations and the raw
+// super-blocks go from memory straight into LDS (gemm_wide.h's fetches: 64 k of activations in two buffers, 256 k of weights in
+// two); a wave reads its fragments of the activations, and of the weights the 16 nibble bytes a lane needs for 64 k, and
+// dequantises them in registers, between the matrix-core instructions of the slice before.  So a weight costs 0.56 bytes of LDS
+// traffic instead of two written and two read, at the price of one dequantisation for each wave along M (two): what bounds it is
+// instruction issue (154 vector instructions for 16 or 32 matrix-core ones) and, at 2048 rows, power.  One barrier per 64 k.
+// 2048 rows, against the other kernel: 6144 x 4096 190 -> 130 us, 4096 x 4096 112 -> 95, 4096 x 12288 284 -> 244, gated pair
+// 12288 x 4096 428 -> 397; 512 rows: 77 -> 57, 78 -> 43, 164 -> 87, 151 -> 120.
+// Tried there: four activation buffers instead of two (no change: a fetch is not what a step waits for), the weights
+// dequantised to f16 in memory by a pre-pass for gemm_wide.h (the same at 2048 rows, slower below).
+//
+// q4k_gemm_kernel (the rest): a wave computes a 64 x 64 (or 32 x 32) quadrant with v_mfma_f32_32x32x16_f16, four waves a
+// 128 x 128 (64 x 64) tile, and a workgroup is one or two such groups stacked along M against the same weight tile.  K advances 64
+// at a time; a thread loads 8 or 16 nibble bytes of a row and the block header, and the weights of a tile are dequantised once
+// per workgroup into LDS.  Both tiles sit in LDS as [row][64 k] with a 16-byte pad (conflict-free 16-byte fragment reads) and are
+// double-buffered, one barrier per K step.
+// Its K loop is bound by instruction issue, not by memory and not by the matrix cores alone.  Measured on this part: a wave issues an
+// independent vector instruction every 5 cycles and a dependent one every 8, a matrix-core instruction occupies its pipe for 32.  Hence:
+//   * every wave both multiplies and produces, and the producer's work of a step (LDS stores of the A tile, scale unpack,
+//     nibble dwords, the loads two tiles ahead) is dealt out in pieces behind the matrix-core instructions of the same step,
+//     in program order pinned with scheduling barriers;
 //   * fragments are double-buffered in registers, so LDS latency runs under the previous slice;
-//   * all global loads are unconditional: one conditional load makes the compiler wait for every
-//     outstanding load before a tile is used, which halves the lookahead.
-// Tried and measured slower: producer / multiplier wave specialisation (four waves each: the
-// producers' 250 vector instructions per step at one wave per SIMD took longer than the
-// multipliers' step, 1.3 us per K step against 1.0 us for eight symmetric waves on the same
-// 256 x 128 x 2 problem), two A sub-tiles per wave (one wave per SIMD), 256 x 64 blocks.
-// k order inside every group of 4 is (0, 2, 1, 3) in BOTH tiles: that is the order the masked
-// nibble pairs come out in, and a contraction index may be permuted freely when both operands
-// agree.
+//   * all global loads are unconditional: one conditional load makes the compiler wait for every outstanding load before a
+//     tile is used, which halves the lookahead.
+// Tried there and measured slower: producer / multiplier wave specialisation, two A sub-tiles per wave, 256 x 64 blocks.
 #include <algorithm>
 #include <cstdlib>
 
-#include "dh_common.h"
+#include "gemm_wide.h"
 #include "q4k_device.h"
 
 namespace {
@@ -75,12 +71,20 @@ struct GemmArgs {
   // partial[z][M][N]; splitk_reduce_kernel adds the pieces in order
   int ksplit, kt_per_split;
   float* partial;
+  int tiles_m, tiles_n;
   const float2* row_scale;   // [M] (multiplier applied before the f16 rounding, its inverse)
   // RMSNorm prologue (norm_weight null = off): rows are normalised while they are packed
   const float* norm_weight;  // [K]
   float norm_eps;
   int norm_weight_offset;    // 1: scale by (1 + w)
 };
+
+// Where k .. k + 3 (k a multiple of 4) of a packed row lie: inside every 64, the 16 a matrix-core instruction contracts are, for either half
+// h of the wave, four low nibbles' k = 16 h + 4 i .. and the four high nibbles' 32 + 16 h + 4 i .. of one dword of a weight row.
+__device__ __forceinline__ int packed_place(int k) {
+  const int q = k >> 2;
+  return (k & ~63) + 16 * (q & 3) + 8 * ((q >> 2) & 1) + 4 * ((q >> 3) & 1);
+}
 
 // Packs the activations for the matrix cores, one wave per row (four rows per workgroup):
 // finds the row's largest magnitude, scales by the power of two that puts it at 2^14 ((1, 1) for
@@ -121,7 +125,7 @@ __global__ __launch_bounds__(256) void pack_a_kernel(const float* __restrict__ A
     }
     const half2_t p0 = {(_Float16)(v[0] * mul), (_Float16)(v[2] * mul)};
     const half2_t p1 = {(_Float16)(v[1] * mul), (_Float16)(v[3] * mul)};
-    *reinterpret_cast<uint2*>(dst + k) = make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+    *reinterpret_cast<uint2*>(dst + packed_place(k)) = make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
   }
 }
 
@@ -202,7 +206,7 @@ __global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict
     if (k < kpad) {
       const half2_t p0 = {(_Float16)(v[i][0] * mul), (_Float16)(v[i][2] * mul)};
       const half2_t p1 = {(_Float16)(v[i][1] * mul), (_Float16)(v[i][3] * mul)};
-      *reinterpret_cast<uint2*>(dst + k) = make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
+      *reinterpret_cast<uint2*>(dst + packed_place(k)) = make_uint2(__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1));
     }
   }
 }
@@ -212,40 +216,48 @@ __global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict
 struct PairScales {
   half2_t slo, mlo, shi, mhi;     // (scale, scale), (-min, -min) of the low- and high-nibble sub-block
 };
-__device__ __forceinline__ PairScales pair_scales_f16(const u32x4_t hdr, const int c) {
-  const float d = f16lo(hdr[0]), dmin = f16hi(hdr[0]);
+struct ScaleBits {
+  uint32_t sc, mn;                // 6-bit scales and mins of the low (byte 0) and high (byte 1) sub-block
+};
+__device__ __forceinline__ ScaleBits scale_bits(const u32x4_t hdr, const int c) {
   const int sh = (c & 1) * 16;
   const uint32_t a1 = hdr[1] >> sh, a2 = hdr[2] >> sh, a3 = hdr[3] >> sh;
   const bool low = c < 2;
-  const uint32_t scp = low ? (a1 & 0x3F3Fu) : ((a3 & 0x0F0Fu) | ((a1 >> 2) & 0x3030u));
-  const uint32_t mnp = low ? (a2 & 0x3F3Fu) : (((a3 >> 4) & 0x0F0Fu) | ((a2 >> 2) & 0x3030u));
-  const _Float16 sl = (_Float16)(d * (float)(scp & 0xFFu)), sh_ = (_Float16)(d * (float)((scp >> 8) & 0xFFu));
-  const _Float16 ml = (_Float16)(-dmin * (float)(mnp & 0xFFu)), mh = (_Float16)(-dmin * (float)((mnp >> 8) & 0xFFu));
-  PairScales r;
-  r.slo = half2_t{sl, sl}; r.mlo = half2_t{ml, ml};
-  r.shi = half2_t{sh_, sh_}; r.mhi = half2_t{mh, mh};
-  return r;
+  return ScaleBits{low ? (a1 & 0x3F3Fu) : ((a3 & 0x0F0Fu) | ((a1 >> 2) & 0x3030u)),
+                   low ? (a2 & 0x3F3Fu) : (((a3 >> 4) & 0x0F0Fu) | ((a2 >> 2) & 0x3030u))};
 }
-// One dword of nibbles (8 weights) -> two low-nibble and two high-nibble f16 pairs.
-// `magic` is 0x64006400 held in a vector register (see magic_1024): with the constant visible the
-// compiler emits v_and + v_or, since one instruction may read only one literal or scalar.
-__device__ __forceinline__ void dequant_dword(const uint32_t w, const PairScales& ps, const uint32_t magic, uint32_t& lo0,
-                                              uint32_t& lo1, uint32_t& hi0, uint32_t& hi1) {
-  const half2_t k1024 = {(_Float16)1024.f, (_Float16)1024.f};
-  const half2_t v0 = __builtin_bit_cast(half2_t, (w & 0x000F000Fu) | magic) - k1024;
-  const half2_t v1 = __builtin_bit_cast(half2_t, ((w >> 8) & 0x000F000Fu) | magic) - k1024;
-  const half2_t v2 = __builtin_bit_cast(half2_t, ((w >> 4) & 0x000F000Fu) | magic) - k1024;
-  const half2_t v3 = __builtin_bit_cast(half2_t, ((w >> 12) & 0x000F000Fu) | magic) - k1024;
-  lo0 = __builtin_bit_cast(uint32_t, v0 * ps.slo + ps.mlo);
-  lo1 = __builtin_bit_cast(uint32_t, v1 * ps.slo + ps.mlo);
-  hi0 = __builtin_bit_cast(uint32_t, v2 * ps.shi + ps.mhi);
-  hi1 = __builtin_bit_cast(uint32_t, v3 * ps.shi + ps.mhi);
+__device__ __forceinline__ PairScales pair_scales_f16(const u32x4_t hdr, const ScaleBits b) {
+  const float d = f16lo(hdr[0]), dmin = f16hi(hdr[0]);
+  const _Float16 sl = (_Float16)(d * (float)(b.sc & 0xFFu)), sh = (_Float16)(d * (float)((b.sc >> 8) & 0xFFu));
+  const _Float16 ml = (_Float16)(-dmin * (float)(b.mn & 0xFFu)), mh = (_Float16)(-dmin * (float)((b.mn >> 8) & 0xFFu));
+  return PairScales{half2_t{sl, sl}, half2_t{ml, ml}, half2_t{sh, sh}, half2_t{mh, mh}};
 }
-
-__device__ __forceinline__ uint32_t magic_1024() {
+// One dword of nibbles (8 weights) -> two f16 pairs of low nibbles, two of high ones.  Bits 0..3 of a half under the exponent of 1024 are
+// 1024 + q, bits 4..7 under that of 64 are 64 + q: no shift brings the high nibbles down.
+// The magic numbers are held in vector registers: with the constants visible the compiler emits v_and + v_or, since one instruction may
+// read only one literal or scalar.
+__device__ __forceinline__ uint32_t magic_number(uint32_t value) {
   uint32_t m;
-  asm("v_mov_b32 %0, 0x64006400" : "=v"(m));
+  asm("v_mov_b32 %0, %1" : "=v"(m) : "i"(value));
   return m;
+}
+struct Magic {
+  uint32_t low, high;
+};
+__device__ __forceinline__ Magic magic_numbers() { return Magic{magic_number(0x64006400u), magic_number(0x54005400u)}; }
+__device__ __forceinline__ void dequant_low(const uint32_t w, const PairScales& ps, const Magic& m, uint32_t& p0, uint32_t& p1) {
+  const half2_t k = {(_Float16)1024.f, (_Float16)1024.f};
+  const half2_t v0 = __builtin_bit_cast(half2_t, (w & 0x000F000Fu) | m.low) - k;
+  const half2_t v1 = __builtin_bit_cast(half2_t, ((w >> 8) & 0x000F000Fu) | m.low) - k;
+  p0 = __builtin_bit_cast(uint32_t, v0 * ps.slo + ps.mlo);
+  p1 = __builtin_bit_cast(uint32_t, v1 * ps.slo + ps.mlo);
+}
+__device__ __forceinline__ void dequant_high(const uint32_t w, const PairScales& ps, const Magic& m, uint32_t& p0, uint32_t& p1) {
+  const half2_t k = {(_Float16)64.f, (_Float16)64.f};
+  const half2_t v0 = __builtin_bit_cast(half2_t, (w & 0x00F000F0u) | m.high) - k;
+  const half2_t v1 = __builtin_bit_cast(half2_t, ((w >> 8) & 0x00F000F0u) | m.high) - k;
+  p0 = __builtin_bit_cast(uint32_t, v0 * ps.shi + ps.mhi);
+  p1 = __builtin_bit_cast(uint32_t, v1 * ps.shi + ps.mhi);
 }
 
 // tanh-form GELU with tanh(t) = 1 - 2 / (1 + e^{2t}): a handful of instructions, inlined once per
@@ -307,7 +319,7 @@ __global__ __launch_bounds__(256 * MG) void q4k_gemm_kernel(const GemmArgs a) {
     // a matrix's units are a multiple of 64 threads: uniform per wave, so the base stays scalar
     w_second[j] = NMAT > 1 && __builtin_amdgcn_readfirstlane(mt & 1) != 0;
     w_off[j] = (uint32_t)((int64_t)min(n0 + row, a.N - 1) * row_bytes);
-    w_lds[j] = A_HALVES + (mt % NMAT) * B_HALVES + row * LDS_ROW + 16 * half + 8 * sub;
+    w_lds[j] = A_HALVES + (mt % NMAT) * B_HALVES + row * LDS_ROW + 8 * half + 16 * QD * sub;
   }
   // Two register sets: while tile kt is multiplied, tile kt+1 waits in one set and the loads of
   // tile kt+2 are in flight into the other, so a load has two K steps to arrive.
@@ -416,8 +428,7 @@ __global__ __launch_bounds__(256 * MG) void q4k_gemm_kernel(const GemmArgs a) {
   // its dwords of nibbles, and the last piece issues the loads two tiles ahead.
   constexpr int NPARTS = 2 + (1 + QD) * NW;
   PairScales ps[NW];
-  const uint32_t magic = magic_1024();
-  uint32_t lo_w[NW][2 * QD], hi_w[NW][2 * QD];
+  const Magic magic = magic_numbers();
   auto produce_part = [&](int part, int kt, Staged& nxt) {      // moves tile kt + 1
     _Float16* At = lds + ((kt & 1) ^ 1) * BUF_HALVES;
     if (part == 0) {
@@ -432,14 +443,13 @@ __global__ __launch_bounds__(256 * MG) void q4k_gemm_kernel(const GemmArgs a) {
       const int j = (part - 1) / (1 + QD), d = (part - 1) % (1 + QD) - 1;
       if (ALL_ACTIVE || w_active[j]) {
         if (d < 0) {
-          ps[j] = pair_scales_f16(nxt.h[j], (kt + 1) & 3);
+          ps[j] = pair_scales_f16(nxt.h[j], scale_bits(nxt.h[j], (kt + 1) & 3));
         } else {
-          dequant_dword(nxt.q[j][d], ps[j], magic, lo_w[j][2 * d], lo_w[j][2 * d + 1], hi_w[j][2 * d], hi_w[j][2 * d + 1]);
-          if (d & 1) {
-            _Float16* Bt = At + w_lds[j] + 4 * (d - 1);
-            *reinterpret_cast<uint4*>(Bt) = make_uint4(lo_w[j][2 * d - 2], lo_w[j][2 * d - 1], lo_w[j][2 * d], lo_w[j][2 * d + 1]);
-            *reinterpret_cast<uint4*>(Bt + 32) = make_uint4(hi_w[j][2 * d - 2], hi_w[j][2 * d - 1], hi_w[j][2 * d], hi_w[j][2 * d + 1]);
-          }
+          // a dword's eight weights are one piece of the packed k order (packed_place)
+          uint4 w;
+          dequant_low(nxt.q[j][d], ps[j], magic, w.x, w.y);
+          dequant_high(nxt.q[j][d], ps[j], magic, w.z, w.w);
+          *reinterpret_cast<uint4*>(At + w_lds[j] + 16 * d) = w;
         }
       }
     }
@@ -515,6 +525,244 @@ __global__ __launch_bounds__(256 * MG) void q4k_gemm_kernel(const GemmArgs a) {
     }
 }
 
+// ---- the wide kernel
+// WM x WN waves; a wave computes 32 RA rows x 64 columns (DUAL: 32 columns of both matrices).
+template <int WM_, int WN_, int RA_>
+struct Q4Tile {
+  static constexpr int WM = WM_, WN = WN_, RA = RA_;
+  static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
+  static constexpr int BM = 32 * RA * WM, kRows = 64 * WN;                // weight rows of a tile (of both matrices together)
+  static constexpr int kBufA = BM * 128, kRoundsA = kBufA / (1024 * kWaves);
+  static constexpr int kRowsWave = kRows / kWaves;                        // weight rows a wave fetches: 144 bytes each
+  static constexpr int kRoundsB = (kRowsWave * 9 + 63) / 64, kRegion = kRoundsB * 1024, kBufB = kRegion * kWaves;
+  static constexpr int kLds = 2 * (kBufA + kBufB);
+  static_assert(kBufA % (1024 * kWaves) == 0 && kRowsWave <= 32 * WN && kRowsWave % 32 == 0, "whole loads; a wave fetches rows of one matrix");
+};
+
+template <class Tile, bool DUAL>
+__global__ __launch_bounds__(Tile::kThreads, 2) void q4k_wide_kernel(const GemmArgs a) {
+  constexpr int RA = Tile::RA, WN = Tile::WN, NB = Tile::kRoundsB, NA = Tile::kRoundsA;
+  constexpr int BN = DUAL ? Tile::kRows / 2 : Tile::kRows;
+  extern __shared__ __align__(16) char smem[];
+  __shared__ float rs_lds[Tile::BM];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int tile = dh::xcd_contiguous(blockIdx.x, a.tiles_m * a.tiles_n);
+  const int m0 = (tile % a.tiles_m) * Tile::BM, n0 = (tile / a.tiles_m) * BN;
+  const int fr = lane & 31, fh = lane >> 5;
+  const int kt0 = a.ksplit > 1 ? (int)blockIdx.z * a.kt_per_split : 0;    // a multiple of 4
+  const int nk = (a.ksplit > 1 ? min((a.K + BK - 1) / BK, kt0 + a.kt_per_split) : (a.K + BK - 1) / BK) - kt0;
+  const int sb0 = kt0 >> 2, sb_last = (kt0 + nk - 1) >> 2;
+  for (int r = threadIdx.x; r < Tile::BM; r += Tile::kThreads) rs_lds[r] = a.row_scale[min(m0 + r, a.M - 1)].y;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  // ---- fetches
+  uint32_t va[NA], vb[NB];
+  {
+    const int row_lane = 8 * wave + (lane >> 3);
+    const uint32_t piece = 16 * ((lane & 7) ^ ((row_lane >> 1) & 7));
+#pragma unroll
+    for (int r = 0; r < NA; r++) {
+      const int row = 8 * Tile::kWaves * r + row_lane;
+      va[r] = (uint32_t)min(row, a.M - 1 - m0) * (uint32_t)a.kpad * 2u + piece;
+    }
+  }
+  const int row_first = wave * Tile::kRowsWave;                            // among the tile's: matrix (or column group) first
+  const int frag_first = row_first / (32 * WN);
+  const int64_t row_bytes = (int64_t)a.nb * kBlockBytes;
+#pragma unroll
+  for (int r = 0; r < NB; r++) {
+    const int at = min(64 * r + lane, Tile::kRowsWave * 9 - 1);            // past the rows: the last piece again
+    const int row = row_first % (32 * WN) + at / 9;                        // column group row / 32 of this fragment, column row % 32
+    const int n = DUAL ? row : (row >> 5) * 64 + 32 * frag_first + (row & 31);
+    vb[r] = (uint32_t)((int64_t)min(n, a.N - 1 - n0) * row_bytes) + 16u * (at % 9);
+  }
+  const dh::buffer_words_t wa = dh::buffer_words(a.Apk + (int64_t)m0 * a.kpad);
+  const dh::buffer_words_t wb = dh::buffer_words((DUAL && frag_first ? a.W2 : a.W) + (int64_t)n0 * row_bytes);
+  const uint32_t lds_a = lds0 + 1024 * wave, lds_b = lds0 + 2 * Tile::kBufA + Tile::kRegion * wave;
+  auto fetch_a = [&](int t, int buf) {
+    const uint32_t k = 128u * (uint32_t)(kt0 + min(t, nk - 1));
+#pragma unroll
+    for (int r = 0; r < NA; r++) dh::fetch_to_lds(wa, va[r], k, lds_a + buf * Tile::kBufA + 1024 * Tile::kWaves * r);
+  };
+  auto fetch_b = [&](int r, uint32_t k, uint32_t buf_at) { dh::fetch_to_lds(wb, vb[r], k, lds_b + buf_at + 1024 * r); };
+  auto b_at = [&](int sb) { return (uint32_t)min(sb, sb_last) * kBlockBytes; };
+
+  // ---- LDS reads
+  const char* ra[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ks++) ra[ks] = smem + (32 * RA * wm + fr) * 128 + 16 * ((2 * ks + fh) ^ ((fr >> 1) & 7));
+  const char* rb[2];
+#pragma unroll
+  for (int f = 0; f < 2; f++) {
+    const int row = f * 32 * WN + 32 * wn + fr;
+    rb[f] = smem + 2 * Tile::kBufA + row / Tile::kRowsWave * Tile::kRegion + row % Tile::kRowsWave * kBlockBytes;
+  }
+  u32x4_t fa[2][RA], raw[2][2], hdr[2], fb[2][2];
+  PairScales ps[2][2];
+  ScaleBits bits;
+  const Magic magic = magic_numbers();
+  float16_t acc[RA][2];
+#pragma unroll
+  for (int i = 0; i < RA; i++)
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][f][e] = 0.f;
+
+  auto read_a = [&](int buf, int ks, int set) {
+#pragma unroll
+    for (int i = 0; i < RA; i++) fa[set][i] = *reinterpret_cast<const u32x4_t*>(ra[ks] + buf * Tile::kBufA + i * 4096);
+  };
+  auto read_b = [&](int c, uint32_t buf_at, int set) {
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+      hdr[f] = *reinterpret_cast<const u32x4_t*>(rb[f] + buf_at);
+      raw[set][f] = *reinterpret_cast<const u32x4_t*>(rb[f] + buf_at + 16 + 32 * c + 16 * fh);
+    }
+  };
+  // A slice's weights of fragment f in three stages of independent instructions (a dependent one waits eight cycles for its operand, so
+  // four chains side by side, with matrix-core instructions between the stages, take half the time of one after the other): the nibbles
+  // under their exponents, the numbers themselves, the weights.
+  half2_t nib[2][4];
+  auto dequant = [&](int stage, int f, int ks, int step_set, int set) {
+    const half2_t k1024 = {(_Float16)1024.f, (_Float16)1024.f}, k64 = {(_Float16)64.f, (_Float16)64.f};
+    half2_t(&v)[4] = nib[f];
+    const PairScales& p = ps[step_set][f];
+    if (stage == 0) {
+      const uint32_t w = raw[step_set][f][ks], w8 = w >> 8;
+      v[0] = __builtin_bit_cast(half2_t, (w & 0x000F000Fu) | magic.low);
+      v[2] = __builtin_bit_cast(half2_t, (w & 0x00F000F0u) | magic.high);
+      v[1] = __builtin_bit_cast(half2_t, (w8 & 0x000F000Fu) | magic.low);
+      v[3] = __builtin_bit_cast(half2_t, (w8 & 0x00F000F0u) | magic.high);
+    } else if (stage == 1) {
+      v[0] = v[0] - k1024; v[2] = v[2] - k64; v[1] = v[1] - k1024; v[3] = v[3] - k64;
+    } else {
+      fb[set][f][0] = __builtin_bit_cast(uint32_t, v[0] * p.slo + p.mlo);
+      fb[set][f][2] = __builtin_bit_cast(uint32_t, v[2] * p.shi + p.mhi);
+      fb[set][f][1] = __builtin_bit_cast(uint32_t, v[1] * p.slo + p.mlo);
+      fb[set][f][3] = __builtin_bit_cast(uint32_t, v[3] * p.shi + p.mhi);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int NM = 2 * RA;
+  // multiplies slice ks; behind its matrix-core instruction n `between(n)` is called
+  auto multiply = [&](int ks, auto&& between) {
+    int n = 0;
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int i = 0; i < RA; i++) {
+        acc[i][f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, fa[ks & 1][i]), __builtin_bit_cast(half8_t, fb[ks & 1][f]),
+                                                           acc[i][f], 0, 0, 0);
+        between(n++);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+  // b_now, b_next: where this super-block and the next lie in LDS; k_next: the next one's place in its row
+  auto step = [&](int t, auto chunk, uint32_t b_now, uint32_t b_next, uint32_t k_next) {
+    constexpr int C = decltype(chunk)::value, P = C & 1, Q = P ^ 1;
+    constexpr int per = (NB + 1) / 2, lo = C == 0 ? 0 : C == 1 ? per : NB, hi = C == 0 ? per : NB;
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+      if (ks == 3) dh::arrive_and_wait<hi - lo>();     // step t + 1's activations are there, and with step 2's all of the next super-block
+      multiply(ks, [&](int n) {
+        if (n == 0) {
+          if (ks < 3) {
+            read_a(P, ks + 1, (ks + 1) & 1);
+          } else {
+            read_a(Q, 0, 0);
+            fetch_a(t + 2, P);
+          }
+          if (ks == 0) read_b((C + 1) & 3, C == 3 ? b_next : b_now, Q);
+        }
+        if (ks < 3)
+          for (int r = lo + ks; r < hi; r += 3)
+            if (n == (r - lo) / 3) fetch_b(r, k_next, b_next);
+        // the next slice's weights; in the middle two slices the next step's scales
+        const int next_ks = (ks + 1) & 3, src = ks < 3 ? P : Q, dst = (ks + 1) & 1;
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+          for (int stage = 0; stage < 3; stage++)
+            if (n == (NM == 4 ? f + stage : 3 * f + stage)) dequant(stage, f, next_ks, src, dst);
+        if (ks == 1 || ks == 2) {
+          if (n == (NM == 4 ? 0 : 6)) bits = scale_bits(hdr[ks - 1], (C + 1) & 3);
+          if (n == NM - 1) ps[Q][ks - 1] = pair_scales_f16(hdr[ks - 1], bits);
+        }
+      });
+    }
+  };
+
+#pragma unroll
+  for (int r = 0; r < NB; r++) fetch_b(r, b_at(sb0), 0);
+  fetch_a(0, 0);
+  fetch_a(1, 1);
+  dh::arrive_and_wait<NA>();
+  read_b(0, 0, 0);
+  read_a(0, 0, 0);
+#pragma unroll
+  for (int f = 0; f < 2; f++) ps[0][f] = pair_scales_f16(hdr[f], scale_bits(hdr[f], 0));
+#pragma unroll
+  for (int f = 0; f < 2; f++)
+#pragma unroll
+    for (int stage = 0; stage < 3; stage++) dequant(stage, f, 0, 0, 0);
+  uint32_t now = 0, next = Tile::kBufB;
+  for (int t = 0, sb = sb0;; t += 4, sb++) {
+    const uint32_t k_next = b_at(sb + 1);
+    step(t, std::integral_constant<int, 0>{}, now, next, k_next);
+    if (t + 1 >= nk) break;
+    step(t + 1, std::integral_constant<int, 1>{}, now, next, k_next);
+    if (t + 2 >= nk) break;
+    step(t + 2, std::integral_constant<int, 2>{}, now, next, k_next);
+    if (t + 3 >= nk) break;
+    step(t + 3, std::integral_constant<int, 3>{}, now, next, k_next);
+    if (t + 4 >= nk) break;
+    const uint32_t was = now;
+    now = next;
+    next = was;
+  }
+  dh::arrive_and_wait<0>();                // nothing may be in flight towards LDS when the workgroup ends
+
+  // ---- epilogue: lane holds column l & 31 of rows 8 (e / 4) + 4 (l >> 5) + e % 4
+#pragma unroll
+  for (int i = 0; i < RA; i++)
+#pragma unroll
+    for (int f = 0; f < (DUAL ? 1 : 2); f++) {
+      const int n = n0 + (DUAL ? 32 * wn : 64 * wn + 32 * f) + fr;
+      if (n >= a.N) continue;
+      const int rl0 = 32 * (RA * wm + i) + 4 * fh;
+      float res[16];
+      if (!DUAL && a.residual && a.ksplit == 1) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) res[e] = a.residual[(int64_t)min(m0 + rl0 + 8 * (e >> 2) + (e & 3), a.M - 1) * a.N + n];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; e++) res[e] = 0.f;
+      }
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int rl = rl0 + 8 * (e >> 2) + (e & 3), m = m0 + rl;
+        if (m >= a.M) continue;
+        const float unscale = rs_lds[rl];
+        float v;
+        if (DUAL) {
+          const float g = acc[i][0][e] * unscale, u = acc[i][1][e] * unscale;
+          v = (a.activation == DH_ACT_SILU ? act_silu(g) : gelu_tanh_fast(g)) * u * a.alpha;
+          if (a.activation == DH_ACT_SILU && a.clamp_max > 0.f) v = fminf(fmaxf(v, -a.clamp_max), a.clamp_max);
+        } else {
+          if (a.ksplit > 1) {
+            a.partial[((int64_t)blockIdx.z * a.M + m) * a.N + n] = acc[i][f][e] * unscale;
+            continue;
+          }
+          v = acc[i][f][e] * unscale * a.alpha + res[e];
+        }
+        if (a.c_f16) reinterpret_cast<__half*>(a.C)[(int64_t)m * a.N + n] = __float2half(v);
+        else reinterpret_cast<float*>(a.C)[(int64_t)m * a.N + n] = v;
+      }
+    }
+}
+
 // C = alpha * (sum of the split-K pieces, in split order) + residual.  Four consecutive outputs per
 // thread when the row length allows 16-byte accesses, every piece's load in flight before the sums.
 constexpr int kMaxSplit = 8;
@@ -566,6 +814,18 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs a) {
   }
 }
 
+int launch_reduce(const GemmArgs& a, const char* op) {
+  const int64_t total = (int64_t)a.M * a.N;
+  if (a.ksplit > kMaxSplit) return dh::fail(2, "[%s] internal: K cut into %d pieces, the reduction takes %d", op, a.ksplit, kMaxSplit);
+  const bool vec = total % 4 == 0 && (reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.residual)) % 16 == 0;
+  if (vec)
+    hipLaunchKernelGGL(splitk_reduce_kernel<true>, dim3((unsigned)dh::ceil_div(total / 4, 256)), dim3(256), 0, dh::stream(), a);
+  else
+    hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3((unsigned)dh::ceil_div(total, 256)), dim3(256), 0, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+
 template <bool DUAL, int T, int MG>
 int launch_gemm_cfg(const GemmArgs& a, const char* op) {
   constexpr int BM = 64 * T * MG, BN = 64 * T;
@@ -580,17 +840,70 @@ int launch_gemm_cfg(const GemmArgs& a, const char* op) {
   const dim3 grid((unsigned)dh::ceil_div(a.N, BN), (unsigned)dh::ceil_div(a.M, BM), (unsigned)std::max(1, a.ksplit));
   hipLaunchKernelGGL(kern, grid, dim3(256 * MG), lds, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
-  if (a.ksplit > 1) {
-    const int64_t total = (int64_t)a.M * a.N;
-    if (a.ksplit > kMaxSplit) return dh::fail(2, "[%s] internal: K cut into %d pieces, the reduction takes %d", op, a.ksplit, kMaxSplit);
-    const bool vec = total % 4 == 0 && (reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.residual)) % 16 == 0;
-    if (vec)
-      hipLaunchKernelGGL(splitk_reduce_kernel<true>, dim3((unsigned)dh::ceil_div(total / 4, 256)), dim3(256), 0, dh::stream(), a);
-    else
-      hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3((unsigned)dh::ceil_div(total, 256)), dim3(256), 0, dh::stream(), a);
-    DH_CHECK_LAUNCH(op);
-  }
+  return a.ksplit > 1 ? launch_reduce(a, op) : 0;
+}
+
+template <class Tile, bool DUAL>
+int launch_wide(GemmArgs a, const char* op) {
+  auto kern = q4k_wide_kernel<Tile, DUAL>;
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLds);
+  DH_CHECK_HIP(op, set);
+  a.tiles_m = (int)dh::ceil_div(a.M, Tile::BM);
+  a.tiles_n = (int)dh::ceil_div(a.N, DUAL ? Tile::kRows / 2 : Tile::kRows);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n), 1, (unsigned)std::max(1, a.ksplit)), dim3(Tile::kThreads), Tile::kLds, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
   return 0;
+}
+
+// Tiles of q4k_wide_kernel and what 64 k of one cost in ns, with few workgroups on the device, with one on every compute unit, with as many
+// as fit; start: outside the k loop.  Fitted to M = 64 .. 2048 over the products of models 1024 .. 4096 wide.
+struct WideCost {
+  int bm, rows, per_cu;
+  float alone, one, full, start;
+};
+constexpr WideCost kWide[] = {{256, 256, 1, 1200.f, 1950.f, 1950.f, 8000.f},       // <2, 4, 4>
+                              {128, 256, 1, 760.f, 1120.f, 1250.f, 9000.f},        // <1, 4, 4>
+                              {128, 256, 1, 845.f, 1200.f, 1250.f, 5500.f},        // <2, 4, 2>
+                              {128, 128, 2, 580.f, 720.f, 1280.f, 5000.f}};        // <2, 2, 2>
+// The cheapest of them, with K cut in pieces (of whole super-blocks) where that pays for the reduction.
+template <bool DUAL>
+int launch_wide_best(GemmArgs a, const char* op) {
+  const int64_t cus = dh::num_cus(), steps = dh::ceil_div(a.K, BK);
+  size_t ws_bytes = 0;
+  float* ws = dh::splitk_workspace(&ws_bytes);
+  const int most = DUAL || !ws ? 1 : (int)std::max<size_t>(1, std::min<size_t>(kMaxSplit, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
+  int pick = 0, split = 1;
+  double least = 1e30;
+  for (int i = 0; i < 4; i++) {
+    const WideCost& c = kWide[i];
+    for (int s = 1; s <= most && (s == 1 || steps >= 8 * s); s++) {
+      const int64_t groups = dh::ceil_div(a.M, c.bm) * dh::ceil_div(a.N, DUAL ? c.rows / 2 : c.rows) * s, slots = cus * c.per_cu, left = groups % slots;
+      const double f = (double)left / cus;
+      const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (0.85 + 0.15 * f / c.per_cu);
+      double t = 4.0 * dh::ceil_div(steps, 4 * s) * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + c.start;
+      if (s > 1) t += 3500.0 + 4.0 * a.M * a.N * (2 * s + 1) / 4000.0;
+      if (t < least) {
+        least = t;
+        pick = i;
+        split = s;
+      }
+    }
+  }
+  const int env_tile = dh::tuning_int("DH_Q4_TILE", -1);
+  if (env_tile >= 0) pick = env_tile;
+  if (split > 1) {
+    a.kt_per_split = (int)dh::ceil_div(steps, 4 * split) * 4;
+    a.ksplit = (int)dh::ceil_div(steps, a.kt_per_split);
+    if (a.ksplit > 1) a.partial = ws;
+  }
+  int rc;
+  switch (pick) {
+    case 0: rc = launch_wide<Q4Tile<2, 4, 4>, DUAL>(a, op); break;
+    case 1: rc = launch_wide<Q4Tile<1, 4, 4>, DUAL>(a, op); break;
+    case 2: rc = launch_wide<Q4Tile<2, 4, 2>, DUAL>(a, op); break;
+    default: rc = launch_wide<Q4Tile<2, 2, 2>, DUAL>(a, op); break;
+  }
+  return rc || a.ksplit <= 1 ? rc : launch_reduce(a, op);
 }
 
 // 128 x 128 tiles when they occupy at least half of the compute units (their higher matrix-core
@@ -641,13 +954,15 @@ int launch_gemm(GemmArgs a, const char* op) {
   DH_CHECK_LAUNCH(op);
   a.row_scale = scales;
   a.Apk = packed;
-  // Tile choice, largest first: 256 x 128 (eight waves) when such tiles fill the compute units,
-  // for the fused gate/up pair 128 x 64 (eight waves) next, then 128 x 128 (four waves, two
-  // workgroups per compute unit) when those occupy at least half of them, else 64 x 64.
+  // Products of enough work, or of enough tiles, go to q4k_wide_kernel: where a step's latency counts instead of its throughput the kernel
+  // below is ahead, because its waves share one dequantised tile (us, this one / the wide one: 1300 x 513 x 1100 21 / 28, 512 x 1152 x 6912
+  // 34 / 38, 64 x 4096 x 4096 25 / 27, but 1024 x 2048 x 1024 38 / 27, 200 x 6144 x 4096 43 / 39, 512 x 4096 x 12288 164 / 87).  There: for
+  // the fused gate/up pair 128 x 64 tiles (eight waves), then 128 x 128 (four waves, two workgroups per compute unit) when those
+  // occupy at least half of the compute units, else 64 x 64.
   const int64_t big_tiles = dh::ceil_div(a.M, 128) * dh::ceil_div(a.N, 128);
   const int64_t tall_tiles = dh::ceil_div(a.M, 256) * dh::ceil_div(a.N, 128);
   a.ksplit = 1;
-  if (tall_tiles >= dh::num_cus()) return launch_gemm_cfg<DUAL, 2, 2>(a, op);
+  if (tall_tiles >= dh::num_cus() || (double)a.M * a.N * a.K * (DUAL ? 2 : 1) >= (a.M >= 1024 ? 2e9 : 5e9)) return launch_wide_best<DUAL>(a, op);
   if (2 * big_tiles >= dh::num_cus()) {
     if constexpr (DUAL) {
       return launch_gemm_cfg<true, 1, 2>(a, op);

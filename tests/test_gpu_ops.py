@@ -782,6 +782,39 @@ def test_bias_add_and_scale_bit_exact():
     assert same.buffer is xt.buffer and np.array_equal(ops.readTensor(xt).reshape(x.shape), x * s)
 
 
+# products large enough for the wide prefill kernel: edges of every tile of it in M and N, K off the 64 and the 256, K in pieces, both
+# kinds of output, norm and residual; reference: the dequantised weights (bit-exact above) in 64 bits
+@pytest.mark.parametrize("M,N,K,pair,f16_out", [(1030, 2100, 1100, False, False), (2050, 6150, 1088, False, True), (1041, 4097, 2300, False, False),
+                                                (600, 4100, 4032, False, False), (513, 130, 81920, False, False), (1100, 1030, 1024, True, False),
+                                                (1025, 5000, 300, True, False), (520, 6900, 1152, True, False)])
+def test_prefill_products_of_the_wide_kernel(M, N, K, pair, f16_out):
+    import torch
+    W = [synth.q4k_centred(synth.q4k_tensor(N, K, seed=7000 + i)) for i in range(2 if pair else 1)]
+    wb = [ops.createWeightBuffer(ops.uploadData(ops.acquireBuffer(w.size), w), "q4k", "row", (N, K)) for w in W]
+    nb = (K + 255) // 256
+    D = [ops.runDequantQ4K(b, N * nb).buffer.view(torch.float32).view(N, nb * 256)[:, :K].double() for b in wb]
+    g = torch.Generator().manual_seed(M + N + K)
+    x, res = torch.randn(M, K, generator=g), torch.randn(M, N, generator=g)
+    xt, nw = ops.tensorFromNumpy(x.numpy()), ops.tensorFromNumpy((1 + 0.1 * torch.randn(K, generator=g)).numpy())
+    xd = x.double().cuda()
+    if pair:
+        h = xd / torch.sqrt(xd.square().mean(1, keepdim=True) + 1e-5) * nw.buffer.view(torch.float32).double()
+        out = ops.runFusedNormedFFN(xt, nw, 1e-5, wb[0], wb[1], K, N, batchSize=M, activation="silu")
+        gate = h @ D[0].T
+        want = gate * torch.sigmoid(gate) * (h @ D[1].T)
+    else:
+        rt = ops.tensorFromNumpy(res.numpy())
+        out = ops.runMatmul(xt, wb[0], M, N, K, alpha=0.5, outputDtype="f16" if f16_out else "f32", residualTensor=rt)
+        want = 0.5 * (xd @ D[0].T) + res.double().cuda()
+    got = ops.readTensor(out)
+    got = torch.from_numpy(got.view(np.float16) if f16_out else got).double().reshape(M, N)
+    want = want.cpu()
+    # f16 operands: 2^-11 relative on either side of a product (the gated pair has two factors)
+    assert ((got - want).norm() / want.norm()).item() < (2e-3 if pair else 1e-3)
+    worst = (got - want).norm(dim=1) / want.norm(dim=1)
+    assert worst.max().item() < 4e-3 and ((got - want).norm(dim=0) / want.norm(dim=0)).max().item() < 4e-3
+
+
 def test_scale_of_a_part_holds_its_whole_shape():
     """readTensor reads a tensor's whole shape: a part's buffer as short as the part sends that read past its end, and the copy is
     refused where the allocation ends."""

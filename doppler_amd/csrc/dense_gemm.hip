@@ -5,7 +5,7 @@
 //   f32 activations    v_mfma_f32_32x32x2_f32 on the weights widened (exactly) to f32: a true 32-bit product
 //
 // Weights [N][ldw] and activations [M][lda] are both read along k; K is a multiple of 64, which the owner of the buffers
-// reaches with zero padding.  16-bit operands: gemm_wide.h (256 x 256, 256 x 128 or 128 x 128 tiles straight from memory into LDS).
+// reaches with zero padding.  16-bit operands: gemm_wide.h (tiles of 256 x 256 down to 64 x 64, straight from memory into LDS).
 // 32-bit: 64-row tiles, 32 k at a time through registers.
 //
 // The epilogue serves two outputs, because the projections that read one normalised row are stored as one
@@ -21,6 +21,7 @@
 // A grid of too few tiles for the device cuts k into slices instead (grid.y): every slice leaves its raw sums in the
 // library's split-K workspace and a second launch adds them in slice order and runs the epilogue.
 #include <algorithm>
+#include <type_traits>
 
 #include "dense_device.h"
 #include "experts.h"
@@ -168,28 +169,36 @@ __device__ __forceinline__ void store_glu(const GemmArgs& a, const TilePlace& p,
 // 16-bit operands (gemm_wide.h).
 template <class Tile, bool F16, int ACT, bool GROUPED = false, bool GLU = false>
 __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const GemmArgs a) {
-  static_assert(!GLU || Tile::FB == 1, "a wave's two tiles are the gate and the up value");
+  static_assert(!GLU || Tile::FB == 1 || Tile::FA == 0, "a wave's two tiles are the gate and the up value");
   extern __shared__ __align__(16) char smem[];
   const int tile = dh::xcd_contiguous(blockIdx.x, a.tiles_m * a.tiles_n);
   TilePlace place;
   if (!place_tile<GROUPED>(a, tile % a.tiles_m, Tile::BM, &place)) return;
   const int m0 = place.m0, n0 = (tile / a.tiles_m) * Tile::BN;
   const int k0 = blockIdx.y * a.k_slice, nk = min(a.k_slice, a.K - k0) >> 6;
-  f32x16_t acc[2 * Tile::FA][2 * Tile::FB];
   const int64_t first = GROUPED ? 0 : m0;       // gathered rows lie anywhere
-  dh::wide_product<Tile, F16>(
-      acc, static_cast<const uint16_t*>(a.A) + first * a.lda,
-      [&](int row) { return (uint32_t)((source_row<GROUPED>(a, place, row) - first) * a.lda * 2); }, place.W + (int64_t)n0 * a.ldw,
-      [&](int row) { return (uint32_t)(min(row, a.N - 1 - n0) * a.ldw * 2); }, 2u * k0, nk, smem);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int m = m0 + 64 * Tile::FA * (wave / Tile::WN), n = n0 + 64 * Tile::FB * (wave % Tile::WN);
+  const void *a_base = static_cast<const uint16_t*>(a.A) + first * a.lda, *w_base = place.W + (int64_t)n0 * a.ldw;
+  auto a_off = [&](int row) { return (uint32_t)((source_row<GROUPED>(a, place, row) - first) * a.lda * 2); };
+  auto w_off = [&](int row) { return (uint32_t)(min(row, a.N - 1 - n0) * a.ldw * 2); };
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / Tile::WN, wn = wave % Tile::WN;
+  if constexpr (Tile::FA == 0) {
+    f32x16_t acc[Tile::G];
+    dh::small_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem);
+    const int m = m0 + 32 * wm, n = n0 + 32 * Tile::G * wn;
+    if constexpr (GLU) store_glu(a, place, acc[0], acc[1], m, n, lane);
+    else store_tile<ACT>(a, place, acc[0], m, n, lane);
+  } else {
+    f32x16_t acc[2 * Tile::FA][2 * Tile::FB];
+    dh::wide_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem);
+    const int m = m0 + 64 * Tile::FA * wm, n = n0 + 64 * Tile::FB * wn;
 #pragma unroll
-  for (int i = 0; i < 2 * Tile::FA; i++) {
-    if constexpr (GLU) {
-      store_glu(a, place, acc[i][0], acc[i][1], m + 32 * i, n, lane);
-    } else {
+    for (int i = 0; i < 2 * Tile::FA; i++) {
+      if constexpr (GLU) {
+        store_glu(a, place, acc[i][0], acc[i][1], m + 32 * i, n, lane);
+      } else {
 #pragma unroll
-      for (int j = 0; j < 2 * Tile::FB; j++) store_tile<ACT>(a, place, acc[i][j], m + 32 * i, n + 32 * j, lane);
+        for (int j = 0; j < 2 * Tile::FB; j++) store_tile<ACT>(a, place, acc[i][j], m + 32 * i, n + 32 * j, lane);
+      }
     }
   }
 }
@@ -303,31 +312,35 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
 // with one on every compute unit, `full` with as many as fit (the two larger tiles: one, which takes more than half of the LDS).  The
 // device slows its clock under matrix-core load, so a step gets dearer as more compute units join, and idle ones are not all
 // lost.  Fitted to M = 17 .. 2048, N = 1024 .. 18464, K = 1024 .. 16384 with each tile and 1 .. 8 slices: the choice is within
-// 10 % of the best of them at nearly all.  Against the 128 x 128 and 64 x 64 tiles through registers that were here before:
+// 10 % of the best of them at nearly all.  (full of the smallest: 365 ns at 512 rows, 520 at 2048.)  Against the 128 x 128 and 64 x 64 tiles through registers that were here before:
 // 2048 x 18464 x 4096 391 -> 300 us, 2048 x 4096 x 16384 312 -> 253, 1531 x 2048 x 6144 75 -> 45, 512 x 4096 x 4096 38 -> 29,
-// 40 x 4096 x 16384 101 -> 39.
+// 40 x 4096 x 16384 101 -> 34 (slices), 40 x 5120 x 1024 11.2 -> 7.1, 700 x 1024 x 1024 9.2 -> 7.3 (64 x 64 tiles).
 using Tile256x256 = dh::WideTile<2, 4, 2, 1>;
 using Tile256x128 = dh::WideTile<4, 2, 1, 1>;
 using Tile128x128 = dh::WideTile<2, 2, 1, 1>;
+using Tile64x64 = dh::SmallTile<2, 2, 1>;
+using Tile64x128 = dh::SmallTile<2, 2, 2>;     // gate and up columns
 struct TileCost {
   int bm, bn, per_cu;
   float alone, one, full, start;      // start: ns outside the k loop
 };
-constexpr TileCost kTiles[] = {{256, 256, 1, 1000.f, 1720.f, 1720.f, 8000.f},
+constexpr TileCost kTiles[] = {{256, 256, 1, 900.f, 1720.f, 1720.f, 8000.f},
                                {256, 128, 1, 520.f, 930.f, 930.f, 5500.f},
-                               {128, 128, 2, 330.f, 480.f, 1050.f, 4500.f}};
-constexpr int kMaxSlices = 8, kMinSliceSteps = 8;
+                               {128, 128, 2, 330.f, 480.f, 1080.f, 4500.f},
+                               {64, 64, 2, 210.f, 250.f, 450.f, 3700.f}};
+constexpr TileCost kSmallGlu = {64, 128, 1, 260.f, 330.f, 330.f, 3700.f};
+constexpr int kMaxSlices = 16, kMinSliceSteps = 8;
 
 struct TileChoice {
   int tile, slices;
 };
 // The cheapest tile and number of k slices.  Slices cost the round trip of their raw sums and a second launch.
-TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices) {
+TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool glu) {
   const int64_t cus = dh::num_cus(), steps = K / 64;
   TileChoice best{0, 1};
   double least = 1e30;
-  for (int i = 0; i < 3; i++) {
-    const TileCost& c = kTiles[i];
+  for (int i = 0; i < 4; i++) {
+    const TileCost& c = glu && i == 3 ? kSmallGlu : kTiles[i];
     for (int s = 1; s <= most_slices && (s == 1 || steps / s >= kMinSliceSteps); s++) {
       const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s, slots = cus * c.per_cu, left = groups % slots;
       const double f = (double)left / cus;
@@ -383,7 +396,8 @@ int launch_16bit(const char* op, GemmArgs a, const TileChoice& pick) {
   switch (pick.tile) {
     case 0: rc = launch_16bit_kernel<Tile256x256, F16, ACT, false, GLU>(op, a, slices); break;
     case 1: rc = launch_16bit_kernel<Tile256x128, F16, ACT, false, GLU>(op, a, slices); break;
-    default: rc = launch_16bit_kernel<Tile128x128, F16, ACT, false, GLU>(op, a, slices); break;
+    case 2: rc = launch_16bit_kernel<Tile128x128, F16, ACT, false, GLU>(op, a, slices); break;
+    default: rc = launch_16bit_kernel<std::conditional_t<GLU, Tile64x128, Tile64x64>, F16, ACT, false, GLU>(op, a, slices); break;
   }
   if (rc || !a.parts) return rc;
   return launch_reduce(op, a, slices);
@@ -429,7 +443,7 @@ int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
   size_t ws_bytes = 0;
   (void)dh::splitk_workspace(&ws_bytes);
   const int most = (int)std::max<size_t>(1, std::min<size_t>(kMaxSlices, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
-  TileChoice pick = choose_tile(a.M, a.N, a.K, most);
+  TileChoice pick = choose_tile(a.M, a.N, a.K, most, false);
   const int env_tile = dh::tuning_int("DH_DENSE_TILE", -1), env_slices = dh::tuning_int("DH_DENSE_SLICES", 0);
   if (env_tile >= 0) pick.tile = env_tile;
   if (env_slices) pick.slices = std::min(most, env_slices);
@@ -479,9 +493,10 @@ int launch_experts(const char* op, GemmArgs a, int a_dtype) {
     return 0;
   }
   if constexpr (GROUPED) {
-    return launch_16bit_kernel<Tile128x128, false, kNoSecond, true, GLU>(op, a, 1);
+    if (a.rows.tile_rows == Tile128x128::BM) return launch_16bit_kernel<Tile128x128, false, kNoSecond, true, GLU>(op, a, 1);
+    return launch_16bit_kernel<std::conditional_t<GLU, Tile64x128, Tile64x64>, false, kNoSecond, true, GLU>(op, a, 1);
   } else {
-    return launch_16bit<false, kNoSecond, GLU>(op, a, choose_tile(a.M, a.N, a.K, 1));
+    return launch_16bit<false, kNoSecond, GLU>(op, a, choose_tile(a.M, a.N, a.K, 1, true));
   }
 }
 
@@ -489,7 +504,7 @@ int launch_experts(const char* op, GemmArgs a, int a_dtype) {
 
 namespace dh {
 
-int expert_tile_rows(int a_dtype) { return a_dtype == DH_F32 ? 64 : Tile128x128::BM; }
+int expert_tile_rows(int a_dtype, int rows, int groups) { return a_dtype == DH_F32 || rows < 96 * groups ? 64 : Tile128x128::BM; }
 
 int experts_glu(const char* op, const ExpertRows& rows, const void* A, int a_dtype, int64_t lda, const uint16_t* W, int64_t ldw, int M,
                 int N, int K, void* out, int out_dtype, int64_t ld_out) {

@@ -23,9 +23,8 @@ __device__ __forceinline__ float clamped_glu(float g, float u, float limit) {
   return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
 
-// Rows of a tile of the grouped products.  (16-bit operands: tiles of 64 rows measured the same where experts get few rows: a tile's
-// time there is its steps' latency.)
-int expert_tile_rows(int a_dtype);
+// Row tiles of the grouped products for this many rows in all.
+int expert_tile_rows(int a_dtype, int rows, int groups);
 // act[row] = clamped_glu of a row's gate and up products with interleaved [N = 2 ff][K] weights (32 gate, 32 up rows, ..).
 int experts_glu(const char* op, const ExpertRows& rows, const void* A, int a_dtype, int64_t lda, const uint16_t* W, int64_t ldw, int M,
                 int N, int K, void* out, int out_dtype, int64_t ld_out);

@@ -366,7 +366,7 @@ PortionSpace portion_space(const dh_experts* s, int operand, int T) {
   const size_t n = (size_t)T * s->top, elem = operand == DH_F32 ? 4 : 2;
   p.ld_z = (logits(s) + 3) / 4 * 4;
   p.ld_y = (s->hidden + 3) / 4 * 4;
-  p.tile_rows = dh::expert_tile_rows(operand);
+  p.tile_rows = dh::expert_tile_rows(operand, (int)n, s->experts);
   p.max_tiles = (int)(n / p.tile_rows + std::min<size_t>(n, s->experts));
   size_t at = 0;
   auto take = [&](size_t bytes) { const size_t r = at; at += up256(bytes); return r; };

@@ -1,5 +1,4 @@
-// Matrix products of 16-bit operands in tiles of 256 rows, shared by the products that have enough of them: eight waves,
-// operands from memory straight into LDS, v_mfma_f32_32x32x16 with f32 accumulation.
+// Matrix products of 16-bit operands: operands from memory straight into LDS, v_mfma_f32_32x32x16 with f32 accumulation.
 #pragma once
 #include "dense_device.h"
 
@@ -195,6 +194,89 @@ __device__ __forceinline__ void wide_product(f32x16_t (&acc)[2 * Tile::FA][2 * T
   arrive_and_wait<0>();
 #undef DH_READ_A
 #undef DH_READ_B
+}
+
+// The small relative, for products whose tiles are too few to hide a step's latency: WM x WN waves of 32 rows x 32 G columns, four k
+// steps in LDS, one barrier a step, fetches three steps ahead; a step is 4 G matrix-core instructions for a wave (0.21 us a step with few
+// workgroups on the device, against 0.33 us for the 128 x 128 tile above).  Fetches, LDS layout and fragments as there.
+template <int WM_, int WN_, int G_>
+struct SmallTile {
+  static constexpr int WM = WM_, WN = WN_, G = G_, FA = 0, FB = 0;
+  static constexpr int BM = 32 * WM, BN = 32 * G * WN, kWaves = WM * WN, kThreads = 64 * kWaves;
+  static constexpr int kBufA = BM * 128, kBufB = BN * 128, kRoundsA = kBufA / (1024 * kWaves), kRoundsB = kBufB / (1024 * kWaves);
+  static constexpr int kLds = 4 * (kBufA + kBufB);
+  static_assert(kBufA % (1024 * kWaves) == 0 && kBufB % (1024 * kWaves) == 0 && 4 * kBufA <= 65536 && 4 * kBufB <= 65536, "whole loads");
+};
+template <class Tile, bool F16, class OffA, class OffW>
+__device__ __forceinline__ void small_product(f32x16_t (&acc)[Tile::G], const void* a_base, OffA a_off, const void* w_base, OffW w_off, uint32_t k_bytes, int nk,
+                                              char* smem) {
+  constexpr int G = Tile::G, RA = Tile::kRoundsA, RB = Tile::kRoundsB, R = RA + RB;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / Tile::WN, wn = wave % Tile::WN;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const buffer_words_t wa = buffer_words(a_base), ww = buffer_words(w_base);
+  uint32_t va[RA], vb[RB];
+  const int row_lane = 8 * wave + (lane >> 3);
+  const uint32_t piece = 16 * ((lane & 7) ^ ((row_lane >> 1) & 7));
+#pragma unroll
+  for (int r = 0; r < RA; r++) va[r] = a_off(8 * Tile::kWaves * r + row_lane) + piece;
+#pragma unroll
+  for (int r = 0; r < RB; r++) vb[r] = w_off(8 * Tile::kWaves * r + row_lane) + piece;
+  const uint32_t lds_a = lds0 + 1024 * wave, lds_b = lds0 + 4 * Tile::kBufA + 1024 * wave;
+  auto fetch = [&](int t, int buf) {
+    const uint32_t k = k_bytes + 128u * (uint32_t)min(t, nk - 1);
+#pragma unroll
+    for (int r = 0; r < RA; r++) fetch_to_lds(wa, va[r], k, lds_a + buf * Tile::kBufA + 1024 * Tile::kWaves * r);
+#pragma unroll
+    for (int r = 0; r < RB; r++) fetch_to_lds(ww, vb[r], k, lds_b + buf * Tile::kBufB + 1024 * Tile::kWaves * r);
+  };
+  const int frow = lane & 31;
+  const char *ra[4], *rb[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ks++) {
+    const int at = frow * 128 + 16 * ((2 * ks + (lane >> 5)) ^ ((frow >> 1) & 7));
+    ra[ks] = smem + at + wm * 4096;
+    rb[ks] = smem + at + 4 * Tile::kBufA + wn * (G * 4096);
+  }
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[g][e] = 0.f;
+  auto step = [&](int t, auto buffer) {
+    constexpr int B = decltype(buffer)::value;
+    arrive_and_wait<2 * R>();                // step t is there for all, and all have read step t - 1
+    fetch(t + 3, (B + 3) & 3);
+    u32x4_t fa[4], fb[4][G];
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+      fa[ks] = *reinterpret_cast<const u32x4_t*>(ra[ks] + B * Tile::kBufA);
+#pragma unroll
+      for (int g = 0; g < G; g++) fb[ks][g] = *reinterpret_cast<const u32x4_t*>(rb[ks] + B * Tile::kBufB + g * 4096);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        if constexpr (F16)
+          acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, fa[ks]), __builtin_bit_cast(f16x8_t, fb[ks][g]), acc[g], 0, 0, 0);
+        else
+          acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fa[ks]), __builtin_bit_cast(bf16x8_t, fb[ks][g]), acc[g], 0, 0, 0);
+      }
+  };
+  fetch(0, 0);
+  fetch(1, 1);
+  fetch(2, 2);
+  for (int t = 0;; t += 4) {
+    step(t, std::integral_constant<int, 0>{});
+    if (t + 1 >= nk) break;
+    step(t + 1, std::integral_constant<int, 1>{});
+    if (t + 2 >= nk) break;
+    step(t + 2, std::integral_constant<int, 2>{});
+    if (t + 3 >= nk) break;
+    step(t + 3, std::integral_constant<int, 3>{});
+    if (t + 4 >= nk) break;
+  }
+  arrive_and_wait<0>();                      // nothing may be in flight towards LDS when the workgroup ends
 }
 
 }  // namespace dh

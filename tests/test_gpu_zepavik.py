@@ -161,6 +161,22 @@ def test_dense_matmul_large_tiles(L, M, N, K, first, dtype):
         assert (C2[:, N - first:] == 9.0).all()
 
 
+# the smallest tile: k steps of every remainder by its four buffers, one row and column over and under its edges
+@pytest.mark.parametrize("M,N,K", [(64, 64, 64), (65, 63, 128), (33, 129, 192), (63, 65, 256), (3, 97, 320), (130, 31, 448)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_matmul_small_tiles(L, M, N, K, dtype):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(dtype)
+    C = torch.full((M, N + 3), 9.0, device="cuda")
+    code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), code, K, W.data_ptr(), K, M, N, K, 1.0, None, None, C.data_ptr(), N + 3, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    # unit products: sums of up to 448 exact terms in 32 bits
+    assert (C[:, :N].double() - A.double() @ W.double().T).abs().max() < 2e-5 and (C[:, N:] == 9.0).all()
+
+
 # 32-bit products in k slices: one tile, a ragged last slice, a narrow product, as many slices as there are
 @pytest.mark.parametrize("M,N,K", [(1, 3, 128), (17, 70, 4160), (65, 130, 1088), (301, 1024, 4096), (40, 129, 16448)])
 def test_dense_matmul_f32_slices(L, M, N, K):

@@ -95,6 +95,8 @@ SIGNATURES = {
     "dh_host_alloc": (_I, [_SZ, ctypes.POINTER(_P)]),
     "dh_host_free": (_I, [_P]),
     "dh_download_async": (_I, [_P, _P, _SZ, _SZ]),
+    "dh_set_words": (_I, [_P, _SZ, _P, _I]),
+    "dh_read_words": (_I, [_P, _P, _SZ, _I]),
     "dh_event_synchronize": (_I, [_P]),
     "dh_event_create": (_I, [ctypes.POINTER(_P)]),
     "dh_event_record": (_I, [_P]),

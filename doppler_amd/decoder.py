@@ -124,17 +124,17 @@ class DecoderBase:
         self._enqueue_head(self._step_row(), out_index, self.logits.data_ptr() if want_logits else None)
 
     def set_token(self, token, kv_len=None, pos=None):
-        """Token id of the step (and beside it, in the same upload, the key count of a captured step and the token
+        """Token id of the step (and beside it, with it, the key count of a captured step and the token
         before position pos)."""
         self._host_ids[0] = token
         self._host_ids[1] = 0 if kv_len is None else kv_len
         self._host_ids[2] = 0 if pos is None else self._before(pos)
-        capi.check(self.L.dh_upload(self.ids.data_ptr(), 0, self._host_ids.ctypes.data, self._host_ids.nbytes))
+        capi.check(self.L.dh_set_words(self.ids.data_ptr(), 0, self._host_ids.ctypes.data, 3))
         if pos is not None:
             self._remember(pos, token)
 
     def read_token(self):
-        capi.check(self.L.dh_download(self._host_token.ctypes.data, self.token.data_ptr(), 0, 4))
+        capi.check(self.L.dh_read_words(self._host_token.ctypes.data, self.token.data_ptr(), 0, 1))
         return int(self._host_token[0])
 
     def _reset_finiteness(self):
@@ -163,7 +163,7 @@ class DecoderBase:
             return self.read_token()
         # staging layout of the reference: [token, status, layer, step, pad]
         words = np.empty(5, np.uint32)
-        capi.check(self.L.dh_download(words.ctypes.data, self.token.data_ptr(), 4 * out_index, 20))
+        capi.check(self.L.dh_read_words(words.ctypes.data, self.token.data_ptr(), 4 * out_index, 5))
         self._raise_if_triggered(words, 1, "generation")
         return int(words[0])
 
@@ -283,7 +283,7 @@ class DecoderBase:
         if not self.finiteness_guard:
             return self.read_token()
         words = np.empty(5, np.uint32)
-        capi.check(self.L.dh_download(words.ctypes.data, self.token.data_ptr(), 4 * (self.TOKEN_RING - 1), 20))
+        capi.check(self.L.dh_read_words(words.ctypes.data, self.token.data_ptr(), 4 * (self.TOKEN_RING - 1), 5))
         self._raise_if_triggered(words, 1, "generation")
         return int(words[0])
 

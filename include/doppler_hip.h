@@ -76,6 +76,12 @@ int dh_host_alloc(size_t bytes, void** host_out);
 int dh_host_free(void* host_ptr);
 int dh_download_async(void* host_dst, const void* d_src, size_t src_offset, size_t bytes);
 int dh_event_synchronize(void* ev);
+/* A step's few words either way (its token id and key count in, the sampled token and the finiteness status out) without a
+ * copy command, whose two ends cost more than the words: up to 16 32-bit words as a launch's own arguments, in stream order and
+ * without a wait, and back through pinned memory of the library, behind everything enqueued so far (this one waits, and reports
+ * like dh_download).  offset in bytes, a multiple of 4.  Not while a graph is being captured. */
+int dh_set_words(void* d_dst, size_t offset, const uint32_t* words, int n);
+int dh_read_words(uint32_t* host_dst, const void* d_src, size_t offset, int n);
 
 /* ---- captured decode steps ----
  * The reference records a whole decode step into one command encoder and submits it once

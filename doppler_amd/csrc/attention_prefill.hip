@@ -1,13 +1,23 @@
 // Prefill attention (T query tokens at once) over an f16 KV cache with grouped-query heads, on the
 // matrix cores: the flash-attention recurrence with v_mfma_f32_16x16x32_f16.
 //
-// Grid = (query tiles of 64 QT tokens, query heads); a workgroup is 4 waves, wave w owns QT
-// groups of 16 consecutive query rows of the tile.  Keys advance 64 at a time; the K and V tiles
-// of the head's kv head are staged in LDS once per workgroup and shared by the four waves, and
-// every fragment a wave reads from there feeds QT matrix-core instructions (QT = 2 for prompts
-// long enough to fill the compute units with 128-query tiles: the kernel is bound by
-// instruction issue and LDS round trips per product, not by the matrix cores or by LDS
-// bandwidth; 118 -> 102 us at T = 2048, 32 heads).
+// A workgroup serves 64 QT query tokens of one head with two groups of four waves: wave w of a group owns QT groups of 16
+// consecutive query rows, group 0 takes the even key tiles and group 1 the odd ones, and the groups' accumulators meet in
+// LDS at the end.  Under a causal mask the last queries see many times the keys of the first: two groups on one tile halve that
+// longest chain and keep two waves on every SIMD to its end, where two workgroups of four waves on a compute unit left the longer
+// of them alone.  Long tiles are dispatched first; a head's tiles go to one of the eight L2 caches where the head count allows it.
+//
+// Key and value tiles go from memory straight into LDS (two buffers per group, one barrier per tile, the next tile in
+// flight during the whole of this one), 16-byte pieces of a row permuted so that no fragment read meets a bank conflict; values are
+// read transposed (ds_read_b64_tr_b16).  QT = 2 for prompts long enough to fill the compute units with 128-query tiles: every
+// fragment a wave reads from LDS then feeds two matrix-core instructions.  Fragments are read six ahead of their use.
+//
+// Measured (us; before: one group staged through registers, V transposed on the way into LDS, fragments read as they were
+// needed -> now): H 32/8, T 2048: 101 -> 61 (562 TFLOP/s); 16/8, 4096: 171 -> 96; 32/8, 8192: 1051 -> 605 (908
+// TFLOP/s); 16/8, 512: 14.5 -> 11.2.  SPEC with distance bias, H 16/4, D 128: T 2048 90 -> 44, T 4096 276 -> 129, window 512 33 -> 29; 16 heads of 128 + 64 shared, T 2048: 91 -> 51.
+// What is left at 128 queries a workgroup: 31% of the matrix cores' cycles and about as much vector work (exponentials) in turns.
+// Measured without gain: the groups half a tile apart (one at the products while the other is at its exponentials, two
+// barriers a tile: 61 -> 59 us, but 51 -> 62 us with shared keys); fetches spread between the products (61 -> 65 us).
 //
 // Everything is computed transposed, so that the softmax statistics of a query live in the lanes
 // that also hold its output column and nothing has to be shuffled between the two products:
@@ -19,8 +29,8 @@
 //                   instructions), the sums only once after the last tile; fp32, online rescale.
 //   O^T = V^T . P^T B = P^T is exactly the lane's own probabilities (k-slot (g, i') stands for
 //                   key 16 (2 kb + i'/4) + 4g + i'%4 of 32-key block kb: a contraction index may be
-//                   renumbered as long as both operands agree), A = V^T read from LDS, where the
-//                   V tile was stored transposed with its keys in that same slot order.
+//                   renumbered as long as both operands agree), A = V^T read from LDS in that same
+//                   slot order by two transposing reads, 16 dims x 4 keys each.
 // Causal tiles beyond the tile's last query are never visited.
 // The SPEC form (dh_attn_spec_prefill) serves the attention of decoders without rotary positions: queries are read
 // from stacked projection rows, every score loses r1 log2(1 + r2 (i - j)) (the distance bias in the softmax's own
@@ -28,14 +38,13 @@
 // LDS and registers), probabilities enter the second product as f16 high part + residual (22 bits), and the output is
 // gated per head and written in the operand type of the product that reads it.  A head's key may end in elements that all
 // heads of the token share (dh_attn_spec_prefill_shared): those come from rows of their own.
-// (Measured without effect at T = 2048..4096: a second LDS buffer per tile with one barrier per
-// tile instead of two, and dispatching the long late-query tiles first.)
 #include <algorithm>
 #include <cfloat>
 #include <cstdlib>
 
 #include "attention_spec.h"
 #include "dense_device.h"
+#include "gemm_wide.h"
 
 namespace {
 
@@ -43,7 +52,19 @@ typedef __attribute__((ext_vector_type(8))) _Float16 half8_t;
 typedef __attribute__((ext_vector_type(4))) float float4_t;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;   // plain vector type: arrays of it stay in registers
 
-constexpr int BKEYS = 64;
+// A 16-byte piece's slot in its row of LDS, and back.  Keys: a fragment read takes one piece of 16 rows, and the slots of
+// those rows cover all banks (rows of an odd number of 128 bytes alternate between the banks' halves by themselves).  Values: pairs of
+// pieces (the 16 elements of a transposing read) stay together.
+template <int D>
+__device__ __forceinline__ int swizzled_k(int row, int c) { return D / 64 % 2 ? c ^ ((row >> 1) & 7) : c ^ (row & 15); }
+template <int VD>
+__device__ __forceinline__ int swizzled_v(int row, int c) { return VD / 64 % 2 ? c ^ (2 * ((row >> 1) & 3)) : c ^ (2 * (row & 7)); }
+
+typedef __attribute__((ext_vector_type(4))) _Float16 half4_t;
+typedef __attribute__((ext_vector_type(4))) short short4_t;
+__device__ __forceinline__ half4_t read_transposed(const char* p) {
+  return __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)p));
+}
 
 // The four lanes l, l ^ 16, l ^ 32, l ^ 48 hold one query's scores.  v_permlane32_swap and
 // v_permlane16_swap (gfx950) hand a lane its partner's value through the vector ALU: with both
@@ -81,24 +102,30 @@ struct PrefillArgs {
   uint16_t* O16;        // bf16 output instead of O
 };
 
-// QT = 16-query groups per wave: every K and V fragment read from LDS feeds QT matrix-core
-// instructions, and a workgroup tile (64 QT queries) stages each key tile once.
 template <int D, int VD, int QT, bool SPEC>
-__global__ __launch_bounds__(256, SPEC ? 2 : 1) void attn_prefill_kernel(const PrefillArgs a) {
+__global__ __launch_bounds__(512, 2) void attn_prefill_kernel(const PrefillArgs a) {
   constexpr int BQ = 64 * QT;
+  constexpr int BKEYS = D > 192 ? 32 : 64;      // keys of a tile: four tiles (two groups, two buffers) in 160 KB of LDS
+  constexpr int NJ = BKEYS / 16, NKB = BKEYS / 32;
   constexpr int STEPS = D / 32;            // MFMAs per 16 x 16 score tile
   constexpr int DT = VD / 16;              // output row tiles (of O^T)
-  constexpr int KROW = D + 8;              // halves per K row in LDS (16-byte pad)
-  constexpr int VROW = BKEYS + 8;          // halves per V^T row in LDS
-  constexpr int PIECES = BKEYS * D / 8 / 256;   // 16-byte pieces of a K tile per thread
+  constexpr int AHEAD = 6;                 // fragments on their way from LDS
+  constexpr int PIECES = BKEYS * D / 8 / 256;   // 16-byte pieces of a K tile per thread of a group
   constexpr int VPIECES = BKEYS * VD / 8 / 256;
-  __shared__ __align__(16) _Float16 k_lds[BKEYS * KROW];
-  __shared__ __align__(16) _Float16 v_lds[VD * VROW];
+  constexpr int KBYTES = BKEYS * D * 2, TILE = KBYTES + BKEYS * VD * 2;
+  constexpr int MERGE_BYTES = 4 * QT * (DT * 1024 + 512);        // four waves' accumulators, maxima and sums
+  static_assert(PIECES >= 1 && VPIECES >= 1 && MERGE_BYTES <= 4 * TILE && 4 * TILE <= 160 * 1024, "LDS");
+  __shared__ __align__(1024) char smem[4 * TILE];
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int q = lane & 15, g = lane >> 4;
-  const int h = blockIdx.y, kvh = h / a.G;
-  const int q0 = blockIdx.x * BQ;
+  // late queries first, heads fastest; workgroups go round the eight XCDs, which get H / 8 neighbouring heads each
+  const int id = blockIdx.y * gridDim.x + blockIdx.x;
+  const int q0 = ((int)gridDim.x - 1 - id / a.H) * BQ;
+  int h = id % a.H;
+  if (a.H % 8 == 0) h = (h & 7) * (a.H / 8) + (h >> 3);
+  const int kvh = h / a.G;
   const int dk = SPEC ? a.dk : D, dv = SPEC ? a.dv : VD;
   const int own_k = SPEC ? a.own_k : D;
   const int64_t k_stride = (int64_t)a.Hkv * own_k, v_stride = (int64_t)a.Hkv * dv;
@@ -152,78 +179,115 @@ __global__ __launch_bounds__(256, SPEC ? 2 : 1) void attn_prefill_kernel(const P
     l_run[u] = 0.f;
   }
 
-  u32x4_t kreg[PIECES], vreg[VPIECES];
-  // K piece p = tid + 256 r of a tile: key p / (D/8), 8 consecutive dims starting at 8 (p % (D/8)).
-  // V is fetched by key PAIRS, so that the transposed tile can be written in 32-bit words: item j
-  // of a thread is keys 2 (tid % 32), 2 (tid % 32) + 1 and dims 8 c .. 8 c + 7, c = tid / 32 + 8 j
-  // (vreg[2 j + s] holds key s of the pair).  The 32 pairs of a half wave land in 32 different
-  // LDS banks.
-  const int vpair = tid & 31, vcol = tid >> 5;
-#define DH_PF_LOAD(tile_)                                                                        \
-  _Pragma("unroll") for (int r = 0; r < PIECES; r++) {                                           \
-    const int p_ = tid + 256 * r, key_ = p_ / (D / 8), c_ = p_ % (D / 8);                        \
-    const int row_ = min(kbeg + (tile_) * BKEYS + key_, a.kv_len - 1);                           \
-    kreg[r] = u32x4_t{0u, 0u, 0u, 0u};                                                           \
-    if (SPEC && 8 * c_ >= own_k) {                                                               \
-      if (8 * c_ < dk) kreg[r] = *reinterpret_cast<const u32x4_t*>(a.KS + (int64_t)row_ * a.ld_shared + 8 * c_ - own_k); \
-    } else {                                                                                     \
-      kreg[r] = *reinterpret_cast<const u32x4_t*>(a.K + (int64_t)row_ * k_stride + (int64_t)kvh * own_k + 8 * c_); \
-    }                                                                                            \
-  }                                                                                              \
-  _Pragma("unroll") for (int r = 0; r < VPIECES; r++) {                                          \
-    const int vrow_ = min(kbeg + (tile_) * BKEYS + 2 * vpair + (r & 1), a.kv_len - 1);           \
-    const int c_ = vcol + 8 * (r >> 1);                                                          \
-    vreg[r] = u32x4_t{0u, 0u, 0u, 0u};                                                           \
-    if (!SPEC || 8 * c_ < dv)                                                                    \
-      vreg[r] = *reinterpret_cast<const u32x4_t*>(a.V + (int64_t)vrow_ * v_stride + (int64_t)kvh * dv + 8 * c_); \
-  }
-  if (ntiles > 0) { DH_PF_LOAD(0); }
-
-  for (int kt = 0; kt < ntiles; kt++) {
-    __syncthreads();                                   // the previous tile has been consumed
+  // ---- fetches: piece tid + 256 r of a tile's slots in LDS is loaded from where the swizzle says it belongs
+  uint32_t k_at[PIECES], v_at[VPIECES];
+  auto k_piece = [&](int r, int* row) { *row = (tid + 256 * r) / (D / 8); return swizzled_k<D>(*row, (tid + 256 * r) % (D / 8)); };
+  auto v_piece = [&](int r, int* row) { *row = (tid + 256 * r) / (VD / 8); return swizzled_v<VD>(*row, (tid + 256 * r) % (VD / 8)); };
+  const uint32_t k_row = 2 * (uint32_t)k_stride, s_row = SPEC ? 2 * (uint32_t)a.ld_shared : 0u, v_row = 2 * (uint32_t)v_stride;
+  auto place = [&](int last) {                       // byte offsets of this lane's pieces in a tile whose last row is `last`
 #pragma unroll
     for (int r = 0; r < PIECES; r++) {
-      const int p = tid + 256 * r, key = p / (D / 8), c = p % (D / 8);
-      *reinterpret_cast<u32x4_t*>(&k_lds[key * KROW + 8 * c]) = kreg[r];
+      int row;
+      const int c = k_piece(r, &row);
+      k_at[r] = SPEC && 8 * c >= own_k ? min(row, last) * s_row + 2u * (8 * c - own_k) : min(row, last) * k_row + 16u * c;
     }
-    // V^T with the keys in k-slot order: key = 32 kb + 16 jj + 4 gg + ii -> slot 32 kb + 8 gg + 4 jj + ii;
-    // the two keys of a pair are neighbours there, one 32-bit word per dim
-    {
-      const int key0 = 2 * vpair;
-      const int slot = 32 * (key0 >> 5) + 8 * ((key0 >> 2) & 3) + 4 * ((key0 >> 4) & 1) + (key0 & 3);
 #pragma unroll
-      for (int j = 0; j < VPIECES / 2; j++) {
-        const int c = vcol + 8 * j;
-        const u32x4_t aw = vreg[2 * j];
-        const u32x4_t bw = vreg[2 * j + 1];
+    for (int r = 0; r < VPIECES; r++) {
+      int row;
+      const int c = v_piece(r, &row);
+      v_at[r] = min(row, last) * v_row + 16u * c;
+    }
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + 1024u * wave;
+  auto fetch = [&](int kt, int buf) {
+    const int first = kbeg + kt * BKEYS;
+    if (first + BKEYS > a.kv_len) place(a.kv_len - 1 - first);
+    const uint32_t to = lds0 + (uint32_t)((2 * grp + buf) * TILE);
+    const dh::buffer_words_t wk = dh::buffer_words(a.K + (int64_t)first * k_stride + (int64_t)kvh * own_k);
+    const dh::buffer_words_t wv = dh::buffer_words(a.V + (int64_t)first * v_stride + (int64_t)kvh * dv);
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const uint32_t word = __builtin_amdgcn_perm(bw[e >> 1], aw[e >> 1], (e & 1) ? 0x07060302u : 0x05040100u);
-          reinterpret_cast<uint32_t*>(v_lds)[((8 * c + e) * VROW + slot) >> 1] = word;
-        }
+    for (int r = 0; r < PIECES; r++) {
+      int row;
+      const int c = k_piece(r, &row);
+      if (!SPEC || 8 * c < own_k) {
+        dh::fetch_to_lds(wk, k_at[r], 0, to + 4096u * r);
+      } else if (8 * c < dk) {
+        dh::fetch_to_lds(dh::buffer_words(a.KS + (int64_t)first * a.ld_shared), k_at[r], 0, to + 4096u * r);
       }
     }
-    __syncthreads();
-    if (kt + 1 < ntiles) { DH_PF_LOAD(kt + 1); }
+#pragma unroll
+    for (int r = 0; r < VPIECES; r++) {
+      int row;
+      const int c = v_piece(r, &row);
+      if (!SPEC || 8 * c < dv) dh::fetch_to_lds(wv, v_at[r], 0, to + KBYTES + 4096u * r);
+    }
+  };
+  if (SPEC) {                                        // elements beyond the heads' sizes: nothing is fetched there
+    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    for (int buf = 0; buf < 2; buf++) {
+      char* to = smem + (2 * grp + buf) * TILE + 16 * tid;
+#pragma unroll
+      for (int r = 0; r < PIECES; r++) {
+        int row;
+        if (8 * k_piece(r, &row) >= dk) *reinterpret_cast<u32x4_t*>(to + 4096 * r) = zero;
+      }
+#pragma unroll
+      for (int r = 0; r < VPIECES; r++) {
+        int row;
+        if (8 * v_piece(r, &row) >= dv) *reinterpret_cast<u32x4_t*>(to + KBYTES + 4096 * r) = zero;
+      }
+    }
+  }
+  place(BKEYS - 1);
+  if (grp < ntiles) fetch(grp, 0);
+
+  // fragment addresses in a tile: the swizzles depend on the lane alone, so a step is an exclusive or, a row block an offset
+  const int k_lane = q * (2 * D) + 16 * swizzled_k<D>(q, g);
+  const int v_lane = KBYTES + (4 * g + (q >> 2)) * (2 * VD) + 16 * swizzled_v<VD>(4 * g + (q >> 2), (q & 3) >> 1) + 8 * (q & 1);
+  for (int it = 0; 2 * it < ntiles; it++) {
+    const int kt = 2 * it + grp;
+    dh::arrive_and_wait<0>();                          // the tile is there, and the other buffer read by all
+    if (kt + 2 < ntiles) fetch(kt + 2, (it + 1) & 1);
+    if (kt >= ntiles) continue;
 
     // ---- S^T for this wave's 16 QT queries against the 64 keys
     const int kbase = kbeg + kt * BKEYS;
-    float4_t st[QT][4];
+    if (a.causal && kbase > a.start_pos + q0 + 16 * QT * (wave + 1) - 1) continue;    // behind all of the wave's queries
+    float4_t st[QT][NJ];
+    half8_t ring[AHEAD];
+    const int at = (2 * grp + (it & 1)) * TILE;
+    auto k_fragment = [&](int f) {
+      constexpr int X = D / 64 % 2 ? 1 : 3;            // steps inside the swizzled part of a row
+      const int j = f % NJ, step = f / NJ;
+      return *reinterpret_cast<const half8_t*>(smem + (((at + k_lane) ^ (64 * (step & X))) + 64 * (step & ~X) + 32 * D * j));
+    };
+    auto v_fragment = [&](int f) {
+      const int t = f % DT, kb = f / DT;
+      const char* p = smem + (((at + v_lane) ^ (32 * t)) + 64 * VD * kb);
+      const half4_t lo = read_transposed(p), hi = read_transposed(p + 32 * VD);
+      return half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int f = 0; f < AHEAD; f++) ring[f] = k_fragment(f);
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
       for (int u = 0; u < QT; u++) st[u][j] = {0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < STEPS; s++) {
-        const half8_t ka = *reinterpret_cast<const half8_t*>(&k_lds[(16 * j + q) * KROW + 32 * s + 8 * g]);
+    for (int f = 0; f < NJ * STEPS; f++) {
 #pragma unroll
-        for (int u = 0; u < QT; u++) st[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[u][s], st[u][j], 0, 0, 0);
-      }
+      for (int u = 0; u < QT; u++) st[u][f % NJ] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[f % AHEAD], qb[u][f / NJ], st[u][f % NJ], 0, 0, 0);
+      if (f + AHEAD < NJ * STEPS) ring[f % AHEAD] = k_fragment(f + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int f = 0; f < AHEAD; f++) ring[f] = v_fragment(f);
+    __builtin_amdgcn_sched_barrier(0);
     // ---- mask, soft cap, online softmax (this lane: query my_q, keys kbase + 16 j + 4 g + i).
     // A tile that every query of a 16-query group sees completely needs no per-element masks.
-    half8_t pb[QT][2];
-    half8_t pl[SPEC ? QT : 1][2];            // SPEC: what the f16 probabilities left over
+    half8_t pb[QT][NKB];
+    half8_t pl[SPEC ? QT : 1][NKB];            // SPEC: what the f16 probabilities left over
     float alpha[QT];
     bool rescale = false;
 #pragma unroll
@@ -235,38 +299,43 @@ __global__ __launch_bounds__(256, SPEC ? 2 : 1) void attn_prefill_kernel(const P
       if (SPEC && a.r1) {
         const float d0 = (float)(my_pos[u] - kbase - 4 * g);
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
           for (int i = 0; i < 4; i++)         // keys behind the query give NaN or less; they are masked below
             st[u][j][i] = fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, d0 - (float)(16 * j + i), 1.0f)), st[u][j][i]);
       }
-      if (full && !(a.softcap > 0.f)) {
+      if (a.softcap > 0.f) {
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
-          for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[u][j][i]);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const int key = kbase + 16 * j + 4 * g + i;
-            float s = st[u][j][i];
-            if (a.softcap > 0.f) s = tanhf(s / a.softcap) * (a.softcap * kLog2e);
-            bool ok = key < a.kv_len;
-            if (a.causal) ok = ok && key <= my_pos[u];
-            if (a.window > 0) ok = ok && key > my_pos[u] - a.window;
-            s = ok ? s : -INFINITY;
-            st[u][j][i] = s;
-            mx = fmaxf(mx, s);
-          }
+          for (int i = 0; i < 4; i++) st[u][j][i] = tanhf(st[u][j][i] / a.softcap) * (a.softcap * kLog2e);
       }
+      if (!full) {                            // this lane's keys are 16 j + i behind kbase + 4 g
+        const int last = min(a.causal ? my_pos[u] : a.kv_len - 1, a.kv_len - 1) - kbase - 4 * g;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) st[u][j][i] = 16 * j + i <= last ? st[u][j][i] : -INFINITY;
+        if (a.window > 0) {
+          const int first = my_pos[u] - a.window + 1 - kbase - 4 * g;
+#pragma unroll
+          for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) st[u][j][i] = 16 * j + i >= first ? st[u][j][i] : -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[u][j][i]);
       mx = quad_rows_max(mx);
-      const float m_new = fmaxf(m_run[u], mx);              // finite: m_run starts at -FLT_MAX
+      // m_run need not be the maximum, only near it: up to 2^8 the probabilities keep their precision in f16, and the
+      // accumulators are scaled seldom.  Finite: it starts at -FLT_MAX.
+      const float m_new = mx > m_run[u] + 8.f ? mx : m_run[u];
       alpha[u] = __builtin_amdgcn_exp2f(m_run[u] - m_new);
       float ps = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int j = 0; j < NJ; j++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const float p = __builtin_amdgcn_exp2f(st[u][j][i] - m_new);   // 2^-inf = 0 for masked keys
@@ -277,28 +346,52 @@ __global__ __launch_bounds__(256, SPEC ? 2 : 1) void attn_prefill_kernel(const P
         }
       l_run[u] = l_run[u] * alpha[u] + ps;               // this lane's share: alpha is the query's, the sum is taken once at the end
       m_run[u] = m_new;
-      rescale = rescale || __builtin_amdgcn_ballot_w64(alpha[u] != 1.0f) != 0;   // no new maximum: nothing to scale
+      rescale = rescale || __builtin_amdgcn_ballot_w64(alpha[u] != 1.0f) != 0;   // else nothing to scale
     }
     // ---- O^T = alpha O^T + V^T P^T
+    if (rescale) {
 #pragma unroll
-    for (int t = 0; t < DT; t++) {
-      if (rescale) {
+      for (int t = 0; t < DT; t++)
 #pragma unroll
         for (int u = 0; u < QT; u++) acc[u][t] *= alpha[u];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < NKB * DT; f++) {
+      const int t = f % DT, kb = f / DT;
+#pragma unroll
+      for (int u = 0; u < QT; u++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[f % AHEAD], pb[u][kb], acc[u][t], 0, 0, 0);
+      if constexpr (SPEC) {
+#pragma unroll
+        for (int u = 0; u < QT; u++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[f % AHEAD], pl[u][kb], acc[u][t], 0, 0, 0);
       }
-#pragma unroll
-      for (int kb = 0; kb < 2; kb++) {
-        const half8_t va = *reinterpret_cast<const half8_t*>(&v_lds[(16 * t + q) * VROW + 32 * kb + 8 * g]);
-#pragma unroll
-        for (int u = 0; u < QT; u++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[u][kb], acc[u][t], 0, 0, 0);
-        if constexpr (SPEC) {
-#pragma unroll
-          for (int u = 0; u < QT; u++) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[u][kb], acc[u][t], 0, 0, 0);
-        }
-      }
+      if (f + AHEAD < NKB * DT) ring[f % AHEAD] = v_fragment(f + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-#undef DH_PF_LOAD
+
+  // ---- the two groups' shares of a query, through LDS
+  __syncthreads();
+  float4_t* shared_acc = reinterpret_cast<float4_t*>(smem) + wave * (QT * DT * 64) + lane;
+  float2* shared_ml = reinterpret_cast<float2*>(smem + 4 * QT * DT * 1024) + wave * (QT * 64) + lane;
+  if (grp) {
+#pragma unroll
+    for (int u = 0; u < QT; u++) {
+#pragma unroll
+      for (int t = 0; t < DT; t++) shared_acc[64 * (u * DT + t)] = acc[u][t];
+      shared_ml[64 * u] = make_float2(m_run[u], l_run[u]);
+    }
+  }
+  __syncthreads();
+  if (grp) return;
+#pragma unroll
+  for (int u = 0; u < QT; u++) {
+    const float2 ml = shared_ml[64 * u];
+    const float m = fmaxf(m_run[u], ml.x), mine = __builtin_amdgcn_exp2f(m_run[u] - m), other = __builtin_amdgcn_exp2f(ml.x - m);
+    l_run[u] = l_run[u] * mine + ml.y * other;
+#pragma unroll
+    for (int t = 0; t < DT; t++) acc[u][t] = acc[u][t] * mine + shared_acc[64 * (u * DT + t)] * other;
+  }
 
   // ---- lane (q, g) holds O[my_q][16 t + 4 g + i]
 #pragma unroll
@@ -356,17 +449,17 @@ extern "C" int dh_attn_prefill(const float* d_Q, const void* d_K, const void* d_
   a.Q = d_Q; a.K = static_cast<const __half*>(d_K); a.V = static_cast<const __half*>(d_V); a.O = d_O;
   a.T = T; a.H = H; a.Hkv = Hkv; a.G = H / Hkv; a.kv_len = kv_len; a.start_pos = start_pos;
   a.causal = causal ? 1 : 0; a.window = sliding_window; a.scale = scale; a.softcap = softcap;
-  // Two 16-query groups per wave (128 queries per workgroup) halve the LDS traffic per product;
-  // short prompts keep 64-query tiles so that the grid still covers the compute units.
+  // Two 16-query groups per wave halve the LDS traffic per product (H 32, T 2048: 73 -> 61 us, the fewest workgroups that gain);
+  // short prompts keep 64-query tiles so that the grid still covers the compute units (H 16, T 2048: 37 us, 45 with 128).
   static const int env_qt = dh::tuning_int("DH_ATTN_PREFILL_QT", 0);
   const int qt = env_qt ? env_qt : ((int64_t)dh::ceil_div(T, 128) * H >= 2 * dh::num_cus() ? 2 : 1);
   const dim3 grid((unsigned)dh::ceil_div(T, 64 * qt), (unsigned)H);
   if (D == 64) {
-    if (qt == 2) hipLaunchKernelGGL((attn_prefill_kernel<64, 64, 2, false>), grid, dim3(256), 0, dh::stream(), a);
-    else hipLaunchKernelGGL((attn_prefill_kernel<64, 64, 1, false>), grid, dim3(256), 0, dh::stream(), a);
+    if (qt == 2) hipLaunchKernelGGL((attn_prefill_kernel<64, 64, 2, false>), grid, dim3(512), 0, dh::stream(), a);
+    else hipLaunchKernelGGL((attn_prefill_kernel<64, 64, 1, false>), grid, dim3(512), 0, dh::stream(), a);
   } else {
-    if (qt == 2) hipLaunchKernelGGL((attn_prefill_kernel<128, 128, 2, false>), grid, dim3(256), 0, dh::stream(), a);
-    else hipLaunchKernelGGL((attn_prefill_kernel<128, 128, 1, false>), grid, dim3(256), 0, dh::stream(), a);
+    if (qt == 2) hipLaunchKernelGGL((attn_prefill_kernel<128, 128, 2, false>), grid, dim3(512), 0, dh::stream(), a);
+    else hipLaunchKernelGGL((attn_prefill_kernel<128, 128, 1, false>), grid, dim3(512), 0, dh::stream(), a);
   }
   DH_CHECK_LAUNCH(op);
   return 0;
@@ -379,9 +472,9 @@ int launch_spec(const char* op, const PrefillArgs& a) {
   // keys of more than 128 elements: two query groups would spill registers
   const int qt = D > 128 ? 1 : env_qt ? env_qt : dh::ceil_div(a.T, 128) * a.H >= 2 * dh::num_cus() ? 2 : 1;
   const dim3 grid((unsigned)dh::ceil_div(a.T, 64 * qt), (unsigned)a.H);
-  if constexpr (D > 128) hipLaunchKernelGGL((attn_prefill_kernel<D, VD, 1, true>), grid, dim3(256), 0, dh::stream(), a);
-  else if (qt == 2) hipLaunchKernelGGL((attn_prefill_kernel<D, VD, 2, true>), grid, dim3(256), 0, dh::stream(), a);
-  else hipLaunchKernelGGL((attn_prefill_kernel<D, VD, 1, true>), grid, dim3(256), 0, dh::stream(), a);
+  if constexpr (D > 128) hipLaunchKernelGGL((attn_prefill_kernel<D, VD, 1, true>), grid, dim3(512), 0, dh::stream(), a);
+  else if (qt == 2) hipLaunchKernelGGL((attn_prefill_kernel<D, VD, 2, true>), grid, dim3(512), 0, dh::stream(), a);
+  else hipLaunchKernelGGL((attn_prefill_kernel<D, VD, 1, true>), grid, dim3(512), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   return 0;
 }
@@ -411,7 +504,7 @@ extern "C" int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float
     return dh::fail(1, "[%s] shared key rows must be 16-byte aligned and ld_shared=%d a multiple of 8 that holds %d elements", op, ld_shared, shared_dim);
   if (spec->ld_qkv < spec->H * dk) return dh::fail(1, "[%s] a projection row of %d floats does not hold its queries", op, spec->ld_qkv);
   const dh::SharedKey shared{d_shared_k, shared_dim, ld_shared};
-  if (spec->cache_dtype != DH_F16 || dk > 256 || spec->VD > 128)
+  if (spec->cache_dtype != DH_F16 || dk > 256 || spec->VD > 128 || ld_shared >= 1 << 24)
     return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);
   PrefillArgs a{};
   a.Q = d_qkv; a.K = static_cast<const __half*>(d_cache_k); a.V = static_cast<const __half*>(d_cache_v);

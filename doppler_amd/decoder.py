@@ -124,7 +124,7 @@ class DecoderBase:
         self._enqueue_head(self._step_row(), out_index, self.logits.data_ptr() if want_logits else None)
 
     def set_token(self, token, kv_len=None, pos=None):
-        """Token id of the step (and beside it, with it, the key count of a captured step and the token
+        """Token id of the step (and with it the key count of a captured step and the token
         before position pos)."""
         self._host_ids[0] = token
         self._host_ids[1] = 0 if kv_len is None else kv_len

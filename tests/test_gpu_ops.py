@@ -1113,6 +1113,43 @@ def test_attention_prefill_causal(T, start, H, Hkv, D):
         assert rel_l2(got[t], want[t]) <= REL_L2_F16_MFMA, t
 
 
+@pytest.mark.parametrize("T,start,H,Hkv,D,window,causal,ramp", [
+    (2100, 5, 36, 9, 128, 0, True, 0.0), (2111, 0, 40, 8, 64, 700, True, 0.0),      # 128-query tiles, heads that are and are not whole eights
+    (1, 0, 3, 3, 128, 0, True, 0.0), (130, 62, 8, 2, 128, 0, True, 0.0),            # one key tile (one of the two groups has none), three
+    (65, 64, 8, 8, 64, 0, False, 0.0), (90, 200, 5, 5, 128, 31, False, 0.0),
+    (300, 0, 4, 2, 128, 0, True, 60.0), (2048, 0, 32, 8, 128, 0, True, 60.0),       # maxima that rise from tile to tile
+    (300, 0, 4, 2, 64, 0, True, -60.0)])
+def test_attention_prefill_tiles(T, start, H, Hkv, D, window, causal, ramp):
+    """Against 64 bits: tile remainders, both tile heights, key groups with uneven shares, and scores that climb (ramp: over all keys) so
+    that the running maximum is sometimes only near the true one.  Inputs are exact in f16, so what is left are the roundings of the scaled
+    query, the probabilities (2^-11 each) and, with a ramp, of scores up to ramp: 2^-11 of the query's part in each."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    n, scale = start + T, 0.25
+    q = (torch.randn(T, H, D, generator=g, device="cuda") * 0.5).half().float()
+    k = torch.randn(n, Hkv, D, generator=g, device="cuda").mul_(0.5).half()
+    v = torch.randn(n, Hkv, D, generator=g, device="cuda").half()
+    if ramp:
+        q[:, :, 0] = 8.0
+        k[:, :, 0] = (torch.linspace(0, ramp, n, device="cuda") / (8.0 * scale))[:, None].half()
+    torch.cuda.synchronize()
+    out = ops.runAttention(ops.tensorFromNumpy(q.cpu().numpy()), ops.tensorFromNumpy(k.cpu().numpy().view(np.uint16)),
+                           ops.tensorFromNumpy(v.cpu().numpy().view(np.uint16)), None, H, D, seqLen=T, kvLen=n, numKVHeads=Hkv,
+                           causal=causal, startPos=start, slidingWindow=window, scale=scale)
+    got = torch.from_numpy(ops.readTensor(out).reshape(T, H, D)).cuda().double()
+    pos, key = start + torch.arange(T, device="cuda")[:, None], torch.arange(n, device="cuda")[None]
+    hidden = torch.zeros(T, n, dtype=torch.bool, device="cuda")
+    if causal:
+        hidden |= key > pos
+    if window:
+        hidden |= key <= pos - window
+    for h in range(H):
+        s = (q[:, h].double() @ k[:, h * Hkv // H].double().T) * scale
+        want = torch.softmax(s.masked_fill(hidden, float("-inf")), 1) @ v[:, h * Hkv // H].double()
+        err = (got[:, h] - want).norm(dim=1) / want.norm(dim=1)
+        assert err.max() < (4e-3 if ramp == 0.0 else 8e-3), (h, int(err.argmax()), float(err.max()))
+
+
 def test_attention_prefill_options_and_errors():
     T, start, H, Hkv, D = 96, 40, 8, 4, 128
     kv_len = start + T

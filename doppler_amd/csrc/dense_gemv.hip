@@ -1,7 +1,7 @@
 // Products of ONE f32 activation row with dense bf16 weights (decode), HBM-bound.
 //
-// The row sits in LDS as f32 (optionally RMS-normalised on its way there); a wave streams R weight rows at a time,
-// 16 bytes per lane and load with the non-temporal hint, R * U loads of the next stage in flight while the current
+// The row sits in LDS as f32 (optionally RMS-normalised on its way there); a wave streams one weight row at a time,
+// 16 bytes per lane and load with the non-temporal hint, U loads of the next stage in flight while the current
 // ones are multiplied (f32 fma on the widened weights, so the product is a 32-bit one).  The first stage is requested
 // before the row is prepared and travels meanwhile.  The row is kept as two planes of 16-byte pieces (elements
 // 0..3 and 4..7 of every eight) so that a wave's reads of either plane are consecutive.
@@ -42,12 +42,12 @@ struct GemvArgs {
   int act;
   const float* gate;          // HEADS form: one number per element; norm_weight has one too, eps is the heads'
   int heads, head_padded, head_size;
-  int iters;                  // row groups per wave
+  int iters;                  // rows per wave
   float* part_val;            // argmax: per-workgroup candidates
   uint32_t* part_idx;
 };
 
-template <int R, int U, int WAVES, bool ARGMAX, bool HEADS>
+template <int U, int WAVES, bool ARGMAX, bool HEADS>
 __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   extern __shared__ __align__(16) float4 planes[];      // [2][K / 8]
   __shared__ float red[WAVES];
@@ -58,19 +58,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   const int np = a.K >> 3, nstages = (np + 64 * U - 1) / (64 * U);
   const int units = a.iters * nstages;
 
-  uint4 cur[R][U], nxt[R][U];
-  auto first_row = [&](int it) { return ((int64_t)(it * (int)gridDim.x + (int)blockIdx.x) * WAVES + wave) * R; };
-  auto load = [&](int unit, uint4 (&dst)[R][U]) {
+  uint4 cur[U], nxt[U];
+  auto row_of = [&](int it) { return (int64_t)(it * (int)gridDim.x + (int)blockIdx.x) * WAVES + wave; };
+  auto load = [&](int unit, uint4 (&dst)[U]) {
     const int it = unit / nstages, st = unit - it * nstages;
-    const int64_t row0 = first_row(it);
+    const uint4* w = reinterpret_cast<const uint4*>(a.W + min(row_of(it), (int64_t)a.N - 1) * a.ldw);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-      const uint4* w = reinterpret_cast<const uint4*>(a.W + min(row0 + r, (int64_t)a.N - 1) * a.ldw);
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int p = lane + 64 * (u + U * st);
-        dst[r][u] = p < np ? dh::stream_load_16(w + p) : make_uint4(0, 0, 0, 0);
-      }
+    for (int u = 0; u < U; u++) {
+      const int p = lane + 64 * (u + U * st);
+      dst[u] = p < np ? dh::stream_load_16(w + p) : make_uint4(0, 0, 0, 0);
     }
   };
   load(0, cur);
@@ -148,9 +144,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   }
   __syncthreads();
 
-  float acc[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) acc[r] = 0.f;
+  float acc = 0.f;
   Cand best{-FLT_MAX, 0xFFFFFFFFu};
   int st = 0, it = 0;
   for (int unit = 0; unit < units; unit++) {
@@ -159,43 +153,32 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
     for (int u = 0; u < U; u++) {
       const int p = min(lane + 64 * (u + U * st), np - 1);      // past the row the weights are zeros
       const float4 xa = planes[p], xb = planes[np + p];
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const uint4 w = cur[r][u];
-        float s = acc[r];
-        s = fmaf(xa.x, dh::bf16_low(w.x), s); s = fmaf(xa.y, dh::bf16_high(w.x), s);
-        s = fmaf(xa.z, dh::bf16_low(w.y), s); s = fmaf(xa.w, dh::bf16_high(w.y), s);
-        s = fmaf(xb.x, dh::bf16_low(w.z), s); s = fmaf(xb.y, dh::bf16_high(w.z), s);
-        s = fmaf(xb.z, dh::bf16_low(w.w), s); s = fmaf(xb.w, dh::bf16_high(w.w), s);
-        acc[r] = s;
-      }
+      const uint4 w = cur[u];
+      acc = fmaf(xa.x, dh::bf16_low(w.x), acc); acc = fmaf(xa.y, dh::bf16_high(w.x), acc);
+      acc = fmaf(xa.z, dh::bf16_low(w.y), acc); acc = fmaf(xa.w, dh::bf16_high(w.y), acc);
+      acc = fmaf(xb.x, dh::bf16_low(w.z), acc); acc = fmaf(xb.y, dh::bf16_high(w.z), acc);
+      acc = fmaf(xb.z, dh::bf16_low(w.w), acc); acc = fmaf(xb.w, dh::bf16_high(w.w), acc);
     }
     if (++st == nstages) {
-      const int64_t row0 = first_row(it);
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const float v = dh::wave_sum_uniform(acc[r]) * a.alpha;
-        acc[r] = 0.f;
-        const int64_t n = row0 + r;
-        if (lane == 0 && n < a.N) {
-          if (n < a.n_first) {
-            float y = v + (a.bias ? a.bias[n] : 0.f);
-            if (a.col_scale) y *= a.col_scale[n];
-            if (a.residual) y += a.residual[n];
-            if (a.C) a.C[n] = y;
-          } else {
-            a.C2[n - a.n_first] = dh::activate(v, a.act);
-          }
-          if (ARGMAX && dh::beats(v, (uint32_t)n, best.v, best.i)) { best.v = v; best.i = (uint32_t)n; }
+      const float v = dh::wave_sum_uniform(acc) * a.alpha;
+      acc = 0.f;
+      const int64_t n = row_of(it);
+      if (lane == 0 && n < a.N) {
+        if (n < a.n_first) {
+          float y = v + (a.bias ? a.bias[n] : 0.f);
+          if (a.col_scale) y *= a.col_scale[n];
+          if (a.residual) y += a.residual[n];
+          if (a.C) a.C[n] = y;
+        } else {
+          a.C2[n - a.n_first] = dh::activate(v, a.act);
         }
+        if (ARGMAX && dh::beats(v, (uint32_t)n, best.v, best.i)) { best.v = v; best.i = (uint32_t)n; }
       }
       st = 0;
       it++;
     }
 #pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-      for (int u = 0; u < U; u++) cur[r][u] = nxt[r][u];
+    for (int u = 0; u < U; u++) cur[u] = nxt[u];
   }
   if (ARGMAX) {
     if (lane == 0) { sv[wave] = best.v; si[wave] = best.i; }
@@ -209,16 +192,17 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   }
 }
 
-template <int R, int U, int WAVES, bool ARGMAX, bool HEADS>
+template <int U, int WAVES, bool ARGMAX, bool HEADS>
 int launch(const char* op, GemvArgs a, int max_grid, int* parts) {
-  auto kern = gemv_kernel<R, U, WAVES, ARGMAX, HEADS>;
+  auto kern = gemv_kernel<U, WAVES, ARGMAX, HEADS>;
   static bool attr_set = false;
   if (!attr_set) {
     DH_CHECK_HIP(op, hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                          kMaxK * 4));
     attr_set = true;
   }
-  const int64_t groups = dh::ceil_div(a.N, R * WAVES);
+  if (ARGMAX) max_grid = std::min(max_grid, dh::kMaxParts);
+  const int64_t groups = dh::ceil_div(a.N, WAVES);
   a.iters = (int)std::max<int64_t>(1, dh::ceil_div(groups, max_grid));
   const int grid = (int)dh::ceil_div(groups, a.iters);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WAVES), (size_t)a.K * 4, dh::stream(), a);
@@ -227,25 +211,27 @@ int launch(const char* op, GemvArgs a, int max_grid, int* parts) {
   return 0;
 }
 
+template <int WAVES, bool ARGMAX, bool HEADS>
+int launch_loads(const char* op, const GemvArgs& a, int max_grid, int* parts) {
+  // a stage as long as the row: lanes past the end load nothing and multiply zeros (a row of 1024 in a stage of 4096 leaves a quarter
+  // of the bytes in flight).  Four waves a workgroup are few, so long rows get long stages there.
+  if (a.K <= 1024) return launch<2, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if (WAVES > 4 || a.K <= 2048) return launch<4, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  return launch<8, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+}
+
+// Every workgroup prepares the whole activation row, so workgroups are as wide as leaves one for every compute unit, and as many
+// as are resident at once.  us, N x K with four waves and stages of 4096 (or two rows of 2048) -> now, weights from memory: 10256 x
+// 2048 11.9 -> 10.8, 5136 x 1024 6.5 -> 5.3, 18464 x 4096 31.0 -> 27.8 (5.4 TB/s), 2048 x 8192 10.1 -> 9.2, 6144 x 2048 9.1 -> 7.9; heads 32000 x
+// 2048 28.5 -> 26.8, 32000 x 1024 19.2 -> 17.4.  A launch alone is about 4 of them.
 template <bool ARGMAX, bool HEADS = false>
 int dispatch(const char* op, const GemvArgs& a, int* parts) {
-  // workgroups that are resident at once share the activation row's preparation as widely as the LDS allows
   const int cus = dh::num_cus();
-  static const int env_r = dh::tuning_int("DH_DENSE_GEMV_R", 0);
-  if constexpr (HEADS) {
-    // every workgroup reads three rows to prepare one: wide workgroups, as long as there is one for every compute unit
-    static const int env_w = dh::tuning_int("DH_GEMV_HEADS_WAVES", 0);
-    const int waves = env_w ? env_w : a.N >= 16 * cus ? 16 : a.N >= 8 * cus ? 8 : 4;
-    if (a.K <= 8192 && waves == 16) return launch<1, 8, 16, ARGMAX, HEADS>(op, a, cus, parts);
-    if (a.K <= 8192 && waves == 8) return launch<1, 8, 8, ARGMAX, HEADS>(op, a, 2 * cus, parts);
-  }
-  const bool two = env_r ? env_r == 2 : a.K <= 4096 && (int64_t)a.N >= (int64_t)64 * cus;
-  if (a.K <= 8192) {
-    const int max_grid = ARGMAX ? std::min(4 * cus, dh::kMaxParts) : 4 * cus;
-    return two ? launch<2, 4, 4, ARGMAX, HEADS>(op, a, max_grid, parts) : launch<1, 8, 4, ARGMAX, HEADS>(op, a, max_grid, parts);
-  }
-  const int max_grid = a.K <= 16384 ? 2 * cus : cus;
-  return launch<1, 8, 8, ARGMAX, HEADS>(op, a, std::min(max_grid, dh::kMaxParts), parts);
+  if (a.K > 8192) return launch<8, 8, ARGMAX, HEADS>(op, a, a.K <= 16384 ? 2 * cus : cus, parts);
+  if constexpr (HEADS)          // three rows are read to prepare one
+    if (a.N >= 16 * cus) return launch_loads<16, ARGMAX, HEADS>(op, a, cus, parts);
+  if (a.N >= 8 * cus) return launch_loads<8, ARGMAX, HEADS>(op, a, !HEADS && a.K <= 2048 ? 4 * cus : 2 * cus, parts);
+  return launch_loads<4, ARGMAX, HEADS>(op, a, 4 * cus, parts);
 }
 
 int check(const char* op, const float* x, const float* norm_weight, int hidden, float eps, const void* W, int ldw, int N, int K) {

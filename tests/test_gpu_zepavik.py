@@ -236,6 +236,35 @@ def test_dense_gemv(L, N, K, hidden, first):
         assert got2[-1] == 5.0
 
 
+@pytest.mark.parametrize("K", [960, 1024, 1088, 2048, 2112, 4160, 8192])
+@pytest.mark.parametrize("N", [5, 2047, 2049, 4101])
+def test_dense_gemv_widths(L, N, K):
+    """Either side of where the stage's length and the workgroup's width change; a product of K terms of size 1 / sqrt(K) in f32 in at
+    most K / 64 + 6 roundings a lane and sum: 2^-24 (K / 64 + 6) <= 8e-6 of terms below 6."""
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x, w = torch.randn(K, generator=g, device="cuda"), torch.rand(K, generator=g, device="cuda") + 0.5
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16)
+    C = torch.full((N + 1,), 5.0, device="cuda")
+    torch.cuda.synchronize()
+    for normed in (True, False):
+        capi.check(L.dh_dense_gemv(x.data_ptr(), w.data_ptr() if normed else None, K, 1e-5, W.data_ptr(), K, N, K, 1.0, None, None,
+                                   C.data_ptr(), N, None, capi.ACT_NONE))
+        capi.check(L.dh_sync())
+        xn = x.double()
+        if normed:
+            xn = xn / torch.sqrt(xn.square().mean() + 1e-5) * w.double()
+        assert (C[:N].double() - W.double() @ xn).abs().max() < 2e-5 and C[N] == 5.0
+    # heads of 64 in front of the product
+    H = K // 64
+    y, gate = torch.zeros(N, device="cuda"), torch.randn(K, generator=g, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_gemv_heads(x.data_ptr(), gate.data_ptr(), w.data_ptr(), H, 64, 64, 1e-5, W.data_ptr(), K, N, K, None, None, y.data_ptr()))
+    capi.check(L.dh_sync())
+    heads = x.double().reshape(H, 64)
+    heads = (heads / torch.sqrt(heads.square().mean(1, keepdim=True) + 1e-5)).reshape(-1) * w.double() * torch.sigmoid(gate.double())
+    assert (y.double() - W.double() @ heads).abs().max() < 2e-5
+
+
 @pytest.mark.parametrize("vocab,K,hidden", [(301, 192, 136), (70001, 512, 500), (900, 9024, 9000)])
 def test_dense_head_argmax(L, vocab, K, hidden):
     g = torch.Generator().manual_seed(vocab)

@@ -102,6 +102,18 @@ struct PrefillArgs {
   uint16_t* O16;        // bf16 output instead of O
 };
 
+// Four elements of an output row in the type of the product that reads it.
+__device__ __forceinline__ void store_spec(const PrefillArgs& a, int64_t at, float4_t v) {
+  if (a.O16) {
+    uint2 two;
+    two.x = (uint32_t)dh::f32_to_bf16_bits(v[0]) | ((uint32_t)dh::f32_to_bf16_bits(v[1]) << 16);
+    two.y = (uint32_t)dh::f32_to_bf16_bits(v[2]) | ((uint32_t)dh::f32_to_bf16_bits(v[3]) << 16);
+    *reinterpret_cast<uint2*>(a.O16 + at) = two;
+  } else {
+    *reinterpret_cast<float4*>(a.O + at) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+}
+
 template <int D, int VD, int QT, bool SPEC>
 __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(const PrefillArgs a) {
   constexpr int BQ = 64 * QT;
@@ -405,15 +417,7 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(const PrefillArgs 
 #pragma unroll
         for (int t = 0; t < DT; t++) {
           if (16 * t + 4 * g >= dv) continue;
-          if (a.O16) {
-            uint2 two;
-            two.x = (uint32_t)dh::f32_to_bf16_bits(acc[u][t][0] * inv) | ((uint32_t)dh::f32_to_bf16_bits(acc[u][t][1] * inv) << 16);
-            two.y = (uint32_t)dh::f32_to_bf16_bits(acc[u][t][2] * inv) | ((uint32_t)dh::f32_to_bf16_bits(acc[u][t][3] * inv) << 16);
-            *reinterpret_cast<uint2*>(a.O16 + at + 16 * t) = two;
-          } else {
-            *reinterpret_cast<float4*>(a.O + at + 16 * t) =
-                make_float4(acc[u][t][0] * inv, acc[u][t][1] * inv, acc[u][t][2] * inv, acc[u][t][3] * inv);
-          }
+          store_spec(a, at + 16 * t, acc[u][t] * inv);
         }
         continue;
       }
@@ -423,6 +427,138 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(const PrefillArgs 
         *reinterpret_cast<float4*>(op + 16 * t) =
             make_float4(acc[u][t][0] * inv, acc[u][t][1] * inv, acc[u][t][2] * inv, acc[u][t][3] * inv);
     }
+  }
+}
+
+// The same over a 32-bit cache, everything in 32 bits (v_mfma_f32_16x16x4_f32; a lane's four consecutive elements of a key row feed
+// four instructions, whose k-slot g stands for element 4 g + e on both sides).  A workgroup is eight waves on the same
+// 16 queries of a head; a wave takes every eighth tile of 32 keys, straight from memory into registers (values requested before the
+// scores are computed, the next keys before the exponentials), and the waves meet in LDS at the end.  The general kernel reads every
+// key again for each query: us, H 16/8, D 64, before -> now: T 301 28 -> 11, T 1024 164 -> 52, T 4096 1926 -> 549 (63 of 136 TFLOP/s;
+// each workgroup reads its keys from L2 on its own); D 128, window 1024, T 2048 845 -> 251.
+template <int D, int VD>
+__global__ __launch_bounds__(512) void attn_prefill_f32_kernel(const PrefillArgs a) {
+  constexpr int WAVES = 8, STEPS = D / 16, DT = VD / 16, BKEYS = 32;
+  __shared__ __align__(16) float4_t acc_s[WAVES][DT][64];
+  __shared__ float2 ml_s[WAVES][16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int q = lane & 15, g = lane >> 4;
+  const int id = blockIdx.y * gridDim.x + blockIdx.x;            // late queries first
+  const int q0 = ((int)gridDim.x - 1 - id / a.H) * 16, h = id % a.H, kvh = h / a.G;
+  const int my_q = q0 + q, my_pos = a.start_pos + my_q;
+  const float* K = reinterpret_cast<const float*>(a.K) + (int64_t)kvh * a.own_k;
+  const float* V = reinterpret_cast<const float*>(a.V) + (int64_t)kvh * a.dv;
+  const float* KS = reinterpret_cast<const float*>(a.KS);
+  const int64_t k_stride = (int64_t)a.Hkv * a.own_k, v_stride = (int64_t)a.Hkv * a.dv;
+  const int kend = min(a.kv_len, a.start_pos + min(q0 + 16, a.T));
+  const int kbeg = a.window > 0 ? max(0, a.start_pos + q0 - a.window + 1) / BKEYS * BKEYS : 0;
+  const int ntiles = (kend - kbeg + BKEYS - 1) / BKEYS;
+
+  float4_t kf[2][STEPS], qb[STEPS];
+  float vf[8][DT];
+  auto load_k = [&](int kt) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int64_t row = min(kbeg + kt * BKEYS + 16 * j + q, a.kv_len - 1);
+#pragma unroll
+      for (int s = 0; s < STEPS; s++) {
+        const int dim = 16 * s + 4 * g;
+        kf[j][s] = float4_t{0.f, 0.f, 0.f, 0.f};
+        if (dim < a.own_k) kf[j][s] = *reinterpret_cast<const float4_t*>(K + row * k_stride + dim);
+        else if (dim < a.dk) kf[j][s] = *reinterpret_cast<const float4_t*>(KS + row * a.ld_shared + dim - a.own_k);
+      }
+    }
+  };
+  if (wave < ntiles) load_k(wave);
+  const float* qp = a.Q + (int64_t)min(my_q, a.T - 1) * a.ld_q + (int64_t)h * a.dk + 4 * g;
+  constexpr float kLog2e = 1.4426950408889634f;
+#pragma unroll
+  for (int s = 0; s < STEPS; s++) {
+    qb[s] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (16 * s + 4 * g < a.dk) qb[s] = *reinterpret_cast<const float4_t*>(qp + 16 * s) * (a.scale * kLog2e);
+  }
+  float r1 = 0.f, r2 = 0.f;
+  if (a.r1) {
+    r1 = a.r1[h];
+    r2 = a.r2[h];
+  }
+  float4_t acc[DT];
+#pragma unroll
+  for (int t = 0; t < DT; t++) acc[t] = {0.f, 0.f, 0.f, 0.f};
+  float m_run = -FLT_MAX, l_run = 0.f;
+  for (int kt = wave; kt < ntiles; kt += WAVES) {
+    const int kbase = kbeg + kt * BKEYS;
+#pragma unroll
+    for (int n = 0; n < 8; n++) {
+      const int64_t row = min(kbase + 16 * (n >> 2) + 4 * g + (n & 3), a.kv_len - 1);
+#pragma unroll
+      for (int t = 0; t < DT; t++) vf[n][t] = 16 * t + q < a.dv ? V[row * v_stride + 16 * t + q] : 0.f;
+    }
+    float4_t st[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) st[j] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STEPS; s++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][s][e], qb[s][e], st[j], 0, 0, 0);
+    if (kt + WAVES < ntiles) load_k(kt + WAVES);
+    const float d0 = (float)(my_pos - kbase - 4 * g);
+    const int last = min(my_pos, a.kv_len - 1) - kbase - 4 * g, first = a.window > 0 ? my_pos - a.window + 1 - kbase - 4 * g : -BKEYS;
+    float mx = -FLT_MAX;
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {           // keys behind the query give NaN or less; they are masked
+        float v = st[j][i];
+        if (a.r1) v = fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, d0 - (float)(16 * j + i), 1.0f)), v);
+        v = 16 * j + i <= last && 16 * j + i >= first ? v : -INFINITY;
+        st[j][i] = v;
+        mx = fmaxf(mx, v);
+      }
+    const float m_new = fmaxf(m_run, quad_rows_max(mx));         // finite: m_run starts at -FLT_MAX
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    float ps = 0.f;
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        st[j][i] = __builtin_amdgcn_exp2f(st[j][i] - m_new);     // 2^-inf = 0 for masked keys
+        ps += st[j][i];
+      }
+    l_run = l_run * alpha + ps;
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < DT; t++) acc[t] *= alpha;
+#pragma unroll
+    for (int n = 0; n < 8; n++)
+#pragma unroll
+      for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[n][t], st[n >> 2][n & 3], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < DT; t++) acc_s[wave][t][lane] = acc[t];
+  l_run = quad_rows_sum(l_run);
+  if (g == 0) ml_s[wave][q] = make_float2(m_run, l_run);
+  __syncthreads();
+  if (my_q >= a.T) return;
+  float m = -FLT_MAX, l = 0.f, part[WAVES];
+#pragma unroll
+  for (int w = 0; w < WAVES; w++) m = fmaxf(m, ml_s[w][q].x);
+#pragma unroll
+  for (int w = 0; w < WAVES; w++) {
+    part[w] = __builtin_amdgcn_exp2f(ml_s[w][q].x - m);
+    l = fmaf(part[w], ml_s[w][q].y, l);
+  }
+  float inv = l > 0.f ? 1.0f / l : 0.f;
+  if (a.gate) inv *= 1.0f / (1.0f + expf(-a.gate[(int64_t)my_q * a.ld_q + h]));
+  const int64_t at = (int64_t)my_q * a.ld_o + (int64_t)h * a.dv + 4 * g;
+  for (int t = wave; t < DT; t += WAVES) {
+    if (16 * t + 4 * g >= a.dv) continue;
+    float4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) o += acc_s[w][t][lane] * part[w];
+    store_spec(a, at + 16 * t, o * inv);
   }
 }
 
@@ -504,7 +640,11 @@ extern "C" int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float
     return dh::fail(1, "[%s] shared key rows must be 16-byte aligned and ld_shared=%d a multiple of 8 that holds %d elements", op, ld_shared, shared_dim);
   if (spec->ld_qkv < spec->H * dk) return dh::fail(1, "[%s] a projection row of %d floats does not hold its queries", op, spec->ld_qkv);
   const dh::SharedKey shared{d_shared_k, shared_dim, ld_shared};
-  if (spec->cache_dtype != DH_F16 || dk > 256 || spec->VD > 128 || ld_shared >= 1 << 24)
+  // fewer than 16 queries leave most of a 32-bit tile empty (5 at 100: 7.8 us by the general kernel, 9.2; 16 at 4000: 67 and 66)
+  const bool wide_cache = spec->cache_dtype != DH_F16;
+  if (wide_cache ? dk > 128 || T < 16 : dk > 256 || ld_shared >= 1 << 24)
+    return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);
+  if (spec->VD > 128)
     return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);
   PrefillArgs a{};
   a.Q = d_qkv; a.K = static_cast<const __half*>(d_cache_k); a.V = static_cast<const __half*>(d_cache_v);
@@ -516,6 +656,15 @@ extern "C" int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float
   a.ld_q = spec->ld_qkv; a.ld_o = ld_out;
   a.r1 = spec->d_bias_r1; a.r2 = spec->d_bias_r2;
   a.gate = spec->gate_offset >= 0 ? d_qkv + spec->gate_offset : nullptr;
+  if (wide_cache) {
+    const dim3 grid((unsigned)dh::ceil_div(T, 16), (unsigned)spec->H);
+    if (dk <= 64 && spec->VD <= 64) hipLaunchKernelGGL((attn_prefill_f32_kernel<64, 64>), grid, dim3(512), 0, dh::stream(), a);
+    else if (dk <= 64) hipLaunchKernelGGL((attn_prefill_f32_kernel<64, 128>), grid, dim3(512), 0, dh::stream(), a);
+    else if (spec->VD <= 64) hipLaunchKernelGGL((attn_prefill_f32_kernel<128, 64>), grid, dim3(512), 0, dh::stream(), a);
+    else hipLaunchKernelGGL((attn_prefill_f32_kernel<128, 128>), grid, dim3(512), 0, dh::stream(), a);
+    DH_CHECK_LAUNCH(op);
+    return 0;
+  }
   if (dk <= 64) return spec->VD <= 64 ? launch_spec<64, 64>(op, a) : launch_spec<64, 128>(op, a);
   if (dk <= 128) return spec->VD <= 64 ? launch_spec<128, 64>(op, a) : launch_spec<128, 128>(op, a);
   return dk <= 192 ? launch_spec<192, 128>(op, a) : launch_spec<256, 128>(op, a);

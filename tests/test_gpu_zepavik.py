@@ -395,6 +395,18 @@ def test_attention_window_edges(L, window, cache):
                 assert np.abs(want[outside] - want[edge]).max() > 0.1
 
 
+@pytest.mark.parametrize("start,T", [(0, 15), (0, 16), (3, 17), (30, 33), (255, 2), (1, 257), (40, 130)])
+@pytest.mark.parametrize("H,G,d,e,window", [(4, 2, 64, 64, 0), (3, 1, 72, 40, 33), (2, 2, 128, 128, 0), (2, 1, 24, 104, 100)])
+def test_attention_f32_tiles(L, H, G, d, e, window, start, T):
+    """Tiles of 16 queries and 32 keys dealt to eight waves, remainders of both, either output type; the tolerance is the shapes test's."""
+    a = Attn(L, H, G, d, e, window, "f32", n=start + T, seed=T)
+    want = a.want()[start:]
+    portions = [start, T] if start else [T]
+    got = a.run(portions)[start:, :, :e]
+    assert max(rel(got[t], want[t]) for t in range(T)) < 3e-6
+    assert max(rel(x, y) for x, y in zip(a.run(portions, "bf16")[start:, :, :e], want)) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("bias,gate,norm", [(False, True, True), (True, False, True), (True, True, False), (False, False, False)])
 def test_attention_mechanisms_one_at_a_time(L, bias, gate, norm):
     for cache, tol in (("f16", 3e-3), ("f32", 3e-6)):

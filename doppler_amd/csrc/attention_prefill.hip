@@ -642,7 +642,7 @@ extern "C" int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float
   const dh::SharedKey shared{d_shared_k, shared_dim, ld_shared};
   // fewer than 16 queries leave most of a 32-bit tile empty (5 at 100: 7.8 us by the general kernel, 9.2; 16 at 4000: 67 and 66)
   const bool wide_cache = spec->cache_dtype != DH_F16;
-  if (wide_cache ? dk > 128 || T < 16 : dk > 256 || ld_shared >= 1 << 24)
+  if (wide_cache ? dk > 128 || T < 16 || spec->H > 65535 : dk > 256 || ld_shared >= 1 << 24)
     return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);
   if (spec->VD > 128)
     return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);

@@ -755,6 +755,35 @@ def test_split_qkv_rmsnorm_rope_kvwrite(T, H, Hkv, D):
     assert np.mean(got_k != wk) < 0.02
 
 
+@pytest.mark.parametrize("norm", [0, 1])
+@pytest.mark.parametrize("T,H,Hkv,D", [(1, 1, 1, 64), (7, 6, 2, 64), (33, 9, 3, 128), (5, 4, 1, 256), (300, 16, 8, 128)])
+def test_qkv_norm_rope_whole_rows(T, H, Hkv, D, norm):
+    """Rows moved in 16-byte pieces against the general kernel, which an offset of one element in the caches still takes: the sums of
+    squares add in another order (f32, relative 2^-21), so a rounding of K to f16 may fall to the other side."""
+    start, n = 3, T * Hkv * D
+    cos, sin = synth.rope_tables(D, start + T, 1e4)
+    t = {k: ops.tensorFromNumpy(v).buffer for k, v in dict(
+        qkv=synth.normal_f32((T, (H + 2 * Hkv) * D), seed=T + D), qw=1 + synth.normal_f32(D, seed=1, scale=0.1),
+        kw=1 + synth.normal_f32(D, seed=2, scale=0.1), cos=cos, sin=sin).items()}
+    L, outs = capi.load(), []
+    for offset in (8, 1):
+        q = ops.acquireBuffer(T * H * D * 4)
+        ck, cv = ops.acquireBuffer((n + 16) * 2), ops.acquireBuffer((n + 16) * 2)
+        for b in (ck, cv):
+            capi.check(L.dh_fill_zero(b.data_ptr(), 0, (n + 16) * 2))
+        capi.check(L.dh_qkv_norm_rope_kvwrite(t["qkv"].data_ptr(), t["qw"].data_ptr() if norm else None, t["kw"].data_ptr() if norm else None,
+                                              t["cos"].data_ptr(), t["sin"].data_ptr(), q.data_ptr(), ck.data_ptr(), cv.data_ptr(), T, H, Hkv, D,
+                                              start, D, 0, 1e-6, 1, offset, norm))
+        k, v = (ops.readBuffer(b, dtype=np.uint16)[:n + 16] for b in (ck, cv))
+        for a in (k, v):
+            assert not a[:offset].any() and not a[offset + n:].any()
+        outs.append((ops.readBuffer(q, dtype=np.float32)[:T * H * D], k[offset:offset + n], v[offset:offset + n]))
+    (q0, k0, v0), (q1, k1, v1) = outs
+    assert np.array_equal(v0, v1) and np.mean(k0 != k1) < 2e-3
+    assert np.abs(q0 - q1).max() <= 2.0 ** -20 * np.abs(q1).max()
+    assert rel_l2(k0.view(np.float16).astype(np.float64), k1.view(np.float16).astype(np.float64)) < 1e-4
+
+
 def test_bias_add_and_scale_bit_exact():
     """residual.js runBiasAdd (in place, byte offsets, f32 or f16 bias) and scale.js runScale: one IEEE add or
     multiply per element, so the f32 results are fixed bit for bit."""

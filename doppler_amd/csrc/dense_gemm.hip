@@ -176,7 +176,8 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const Gem
   if (!place_tile<GROUPED>(a, tile % a.tiles_m, Tile::BM, &place)) return;
   const int m0 = place.m0, n0 = (tile / a.tiles_m) * Tile::BN;
   const int k0 = blockIdx.y * a.k_slice, nk = min(a.k_slice, a.K - k0) >> 6;
-  const int64_t first = GROUPED ? 0 : m0;       // gathered rows lie anywhere
+  // offsets count from the tile's first row, which may lie anywhere; those of gathered rows from the first of all
+  const int64_t first = GROUPED && a.rows.row_index ? 0 : (int64_t)place.base + m0;
   const void *a_base = static_cast<const uint16_t*>(a.A) + first * a.lda, *w_base = place.W + (int64_t)n0 * a.ldw;
   auto a_off = [&](int row) { return (uint32_t)((source_row<GROUPED>(a, place, row) - first) * a.lda * 2); };
   auto w_off = [&](int row) { return (uint32_t)(min(row, a.N - 1 - n0) * a.ldw * 2); };
@@ -366,7 +367,8 @@ int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
   auto kern = gemm_16bit_kernel<Tile, F16, ACT, GROUPED, GLU>;
   static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLds);
   DH_CHECK_HIP(op, set);
-  if (!within_reach(a.M, a.lda, a.K) || !within_reach(a.N, a.ldw, a.K))
+  const bool gathered = GROUPED && a.rows.row_index;
+  if (!(gathered ? (int64_t)2 * a.rows.source_rows * a.lda < (int64_t)1 << 32 : within_reach(GROUPED ? Tile::BM : a.M, a.lda, a.K)) || !within_reach(a.N, a.ldw, a.K))
     return dh::fail(1, "[%s] rows %lld and %lld elements apart are out of reach", op, (long long)a.lda, (long long)a.ldw);
   if (!GROUPED) a.tiles_m = (int)dh::ceil_div(a.M, Tile::BM);
   a.tiles_n = (int)dh::ceil_div(a.N, Tile::BN);

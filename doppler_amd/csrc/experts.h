@@ -8,7 +8,8 @@ namespace dh {
 struct ExpertRows {
   const int* tiles;        // [max_tiles][2]: expert (-1: no tile), first row inside its group; null: one group, rows as they are
   const int* group_off;    // [experts + 1] first row of every group
-  const int* row_index;    // activation row of every sorted row, or null
+  const int* row_index;    // activation row of every sorted row (one of source_rows), or null: the rows themselves
+  int source_rows;
   int64_t w_stride;        // elements between the experts' matrices
   int max_tiles, tile_rows;
   const float* row_in;     // factor of a row's input (gate and up before the clamps), or null

@@ -463,7 +463,7 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
                      p.max_tiles, i32(p.off), i32(p.slot), i32(p.row_token), f32(p.row_weight), i32(p.tiles));
   DH_CHECK_LAUNCH(op);
   dh::ExpertRows rows{};
-  rows.tiles = i32(p.tiles); rows.group_off = i32(p.off); rows.row_index = i32(p.row_token); rows.w_stride = (int64_t)2 * spec->ff * spec->K;
+  rows.tiles = i32(p.tiles); rows.group_off = i32(p.off); rows.row_index = i32(p.row_token); rows.source_rows = T; rows.w_stride = (int64_t)2 * spec->ff * spec->K;
   rows.max_tiles = p.max_tiles; rows.tile_rows = p.tile_rows; rows.row_in = f32(p.row_weight); rows.limit = spec->limit;
   if (int rc = dh::experts_glu(op, rows, d_h, operand, spec->K, static_cast<const uint16_t*>(spec->d_up), spec->K, n, 2 * spec->ff, spec->K, w + p.act,
                                operand, spec->ff))

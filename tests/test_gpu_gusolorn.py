@@ -370,6 +370,33 @@ def test_many_experts_are_chosen_exactly(L, tmp_path, E, top):
         assert parts_error(dec, want, t, portions, n)[clear].max() < PART["float32"]
 
 
+# widths and counts where a portion's rows end past 4 GB: the experts' activations (12 million rows of 192), the tokens' own rows (gathered)
+@pytest.mark.parametrize("T,W,K,E,top,ff", [(1500000, 64, 64, 9, 8, 192), ((1 << 20) + 77, 64, 2048, 3, 1, 64)])
+def test_expert_rows_past_4_gb(L, T, W, K, E, top, ff):
+    """A token's result does not depend on the portion it comes in: the last ones (and some in the middle) again, alone.  Both calls add the
+    same bf16 products in 32 bits, so what differs is the order of a few sums and a rounding of an activation to bf16 behind it."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    h = torch.zeros(T, K, dtype=torch.bfloat16, device="cuda")
+    for i in range(0, T, 1 << 18):
+        h[i:i + (1 << 18), :W] = torch.randn(min(1 << 18, T - i), W, generator=g, device="cuda")
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") * 0.2).to(torch.bfloat16)
+    router, up, down, norm = w(E, K), w(E, 2 * ff, K), w(E, W, ff), torch.ones(W, device="cuda")
+    spec = capi.Experts(W, K, E, top, ff, 0, 1e-5, 7.0, 0.0, norm.data_ptr(), None, router.data_ptr(), up.data_ptr(), down.data_ptr(), None, None)
+    ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T), dtype=torch.uint8, device="cuda")
+
+    def run(rows):
+        x = torch.zeros(len(rows), W, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_experts_prefill(ctypes.byref(spec), rows.data_ptr(), capi.BF16, x.data_ptr(), W, ws.data_ptr(), len(rows)))
+        capi.check(L.dh_sync())
+        return x
+    whole, size = run(h), 1000
+    for at in (0, T // 3, T // 2 - 500, T * 5 // 6, T - size):
+        alone = run(h[at:at + size].contiguous())
+        assert alone.norm() > 0
+        assert ((whole[at:at + size] - alone).norm(dim=1) <= 2.0 ** -8 * alone.norm(dim=1)).all(), at
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

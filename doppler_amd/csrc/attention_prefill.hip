@@ -486,6 +486,8 @@ __global__ __launch_bounds__(512) void attn_prefill_f32_kernel(const PrefillArgs
 #pragma unroll
   for (int t = 0; t < DT; t++) acc[t] = {0.f, 0.f, 0.f, 0.f};
   float m_run = -FLT_MAX, l_run = 0.f;
+  bool left_out = false;
+  auto in_part = [&](int kbase) { return kbase + BKEYS - 1 > a.start_pos + q0 || (a.window > 0 && kbase + a.window < a.start_pos + q0 + 16); };
   for (int kt = wave; kt < ntiles; kt += WAVES) {
     const int kbase = kbeg + kt * BKEYS;
 #pragma unroll
@@ -531,33 +533,67 @@ __global__ __launch_bounds__(512) void attn_prefill_f32_kernel(const PrefillArgs
     m_run = m_new;
 #pragma unroll
     for (int t = 0; t < DT; t++) acc[t] *= alpha;
+    // Where not every query sees the whole tile, values that are not finite count as zero here (a masked probability of 0 would make
+    // them NaN); the queries that see them get them behind the loop.
+    if (in_part(kbase)) {
+      float z = 0.f;
+#pragma unroll
+      for (int n = 0; n < 8; n++)
+#pragma unroll
+        for (int t = 0; t < DT; t++) z = fmaf(vf[n][t], 0.f, z);
+      if (__builtin_amdgcn_ballot_w64(!(z == 0.f))) {
+        left_out = true;
+#pragma unroll
+        for (int n = 0; n < 8; n++)
+#pragma unroll
+          for (int t = 0; t < DT; t++) vf[n][t] = fabsf(vf[n][t]) < INFINITY ? vf[n][t] : 0.f;
+      }
+    }
 #pragma unroll
     for (int n = 0; n < 8; n++)
 #pragma unroll
       for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[n][t], st[n >> 2][n & 3], acc[t], 0, 0, 0);
   }
+  // The lane's place once more, from the hardware: kept through the loop it would cost the registers of the largest form (128, 128) that
+  // the loop needs (addresses spilled, 248 -> 267 us at T 2048).
+  const int out_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), out_g = out_lane >> 4;
+  const int out_q = q0 + (out_lane & 15), out_pos = a.start_pos + out_q;
+  if (left_out) {
+    for (int kt = wave; kt < ntiles; kt += WAVES) {
+      if (!in_part(kbeg + kt * BKEYS)) continue;
+      const int last = min(kbeg + (kt + 1) * BKEYS - 1, min(out_pos, a.kv_len - 1));
+      for (int key = max(kbeg + kt * BKEYS, a.window > 0 ? out_pos - a.window + 1 : 0); key <= last; key++)
 #pragma unroll
-  for (int t = 0; t < DT; t++) acc_s[wave][t][lane] = acc[t];
+        for (int t = 0; t < DT; t++) {
+          if (16 * t + 4 * out_g >= a.dv) continue;
+          const float4_t v = *reinterpret_cast<const float4_t*>(V + key * v_stride + 16 * t + 4 * out_g);
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[t][e] = fabsf(v[e]) < INFINITY ? acc[t][e] : acc[t][e] + v[e];
+        }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < DT; t++) acc_s[wave][t][out_lane] = acc[t];
   l_run = quad_rows_sum(l_run);
-  if (g == 0) ml_s[wave][q] = make_float2(m_run, l_run);
+  if (out_g == 0) ml_s[wave][out_lane & 15] = make_float2(m_run, l_run);
   __syncthreads();
-  if (my_q >= a.T) return;
+  if (out_q >= a.T) return;
   float m = -FLT_MAX, l = 0.f, part[WAVES];
 #pragma unroll
-  for (int w = 0; w < WAVES; w++) m = fmaxf(m, ml_s[w][q].x);
+  for (int w = 0; w < WAVES; w++) m = fmaxf(m, ml_s[w][out_lane & 15].x);
 #pragma unroll
   for (int w = 0; w < WAVES; w++) {
-    part[w] = __builtin_amdgcn_exp2f(ml_s[w][q].x - m);
-    l = fmaf(part[w], ml_s[w][q].y, l);
+    part[w] = __builtin_amdgcn_exp2f(ml_s[w][out_lane & 15].x - m);
+    l = fmaf(part[w], ml_s[w][out_lane & 15].y, l);
   }
   float inv = l > 0.f ? 1.0f / l : 0.f;
-  if (a.gate) inv *= 1.0f / (1.0f + expf(-a.gate[(int64_t)my_q * a.ld_q + h]));
-  const int64_t at = (int64_t)my_q * a.ld_o + (int64_t)h * a.dv + 4 * g;
+  if (a.gate) inv *= 1.0f / (1.0f + expf(-a.gate[(int64_t)out_q * a.ld_q + h]));
+  const int64_t at = (int64_t)out_q * a.ld_o + (int64_t)h * a.dv + 4 * out_g;
   for (int t = wave; t < DT; t += WAVES) {
-    if (16 * t + 4 * g >= a.dv) continue;
+    if (16 * t + 4 * out_g >= a.dv) continue;
     float4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < WAVES; w++) o += acc_s[w][t][lane] * part[w];
+    for (int w = 0; w < WAVES; w++) o += acc_s[w][t][out_lane] * part[w];
     store_spec(a, at + 16 * t, o * inv);
   }
 }

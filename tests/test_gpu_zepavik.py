@@ -407,6 +407,27 @@ def test_attention_f32_tiles(L, H, G, d, e, window, start, T):
     assert max(rel(x, y) for x, y in zip(a.run(portions, "bf16")[start:, :, :e], want)) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("H,G,d,e,window,at", [(2, 2, 64, 64, 0, 37), (2, 1, 128, 104, 40, 50), (1, 1, 64, 128, 33, 95), (2, 1, 120, 24, 1, 64),
+                                                   (1, 1, 64, 64, 70, 0), (1, 1, 64, 64, 0, 149)])
+def test_a_non_finite_value_stays_with_the_queries_that_see_it(L, H, G, d, e, window, at, bad):
+    """f32 caches: every query in front of the value's token, or past its window, has the same bits as without it; those that see it do
+    not, in that element alone."""
+    n = 150
+    a = Attn(L, H, G, d, e, window, "f32", n=n, seed=at)
+    clean = a.run([n])
+    rows, out = a.rows(), torch.zeros(n, H * a.VD, device="cuda")
+    a.vc.view(-1, a.vc.numel() // a.vc.shape[0])[at, 3] = bad                # one element of the first key-value head's value
+    torch.cuda.synchronize()
+    capi.check(L.dh_attn_spec_prefill(ctypes.byref(a.spec), rows.data_ptr(), a.kc.data_ptr(), a.vc.data_ptr(), out.data_ptr(), capi.F32, H * a.VD, n, 0))
+    got = host(out).reshape(n, H, a.VD)
+    sees = np.zeros(n, bool)
+    sees[at:at + window if window else n] = True
+    hit = np.zeros(got.shape, bool)
+    hit[sees, :H // G, 3] = True                                            # the query heads of that key-value head
+    assert not np.isfinite(got[hit]).any() and np.array_equal(got[~hit], clean[~hit])
+
+
 @pytest.mark.parametrize("bias,gate,norm", [(False, True, True), (True, False, True), (True, True, False), (False, False, False)])
 def test_attention_mechanisms_one_at_a_time(L, bias, gate, norm):
     for cache, tol in (("f16", 3e-3), ("f32", 3e-6)):

@@ -287,26 +287,29 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   }
 }
 
-// Sums of the k slices in slice order; blockIdx.y = row, VEC columns per thread (N a multiple of VEC).
+// Sums of the k slices in slice order.  VEC columns per thread (N a multiple of VEC), a block's threads as wide as the row allows and the
+// rest of them on further rows; a grid's second dimension holds 65535 blocks, so rows go round.
 template <int VEC>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int slices) {
-  const int m = blockIdx.y, n = VEC * (blockIdx.x * 256 + threadIdx.x);
+  const int n = VEC * (blockIdx.x * blockDim.x + threadIdx.x);
   if (n >= a.N) return;
   const int64_t total = (int64_t)a.M * a.N;
-  const float* p = a.parts + (int64_t)m * a.N + n;
-  float s[VEC] = {};
+  for (int m = blockIdx.y * blockDim.y + threadIdx.y; m < a.M; m += gridDim.y * blockDim.y) {
+    const float* p = a.parts + (int64_t)m * a.N + n;
+    float s[VEC] = {};
 #pragma unroll 4
-  for (int k = 0; k < slices; k++) {
-    if constexpr (VEC == 4) {
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p + k * total);
+    for (int k = 0; k < slices; k++) {
+      if constexpr (VEC == 4) {
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p + k * total);
 #pragma unroll
-      for (int e = 0; e < 4; e++) s[e] += v[e];
-    } else {
-      s[0] += p[k * total];
+        for (int e = 0; e < 4; e++) s[e] += v[e];
+      } else {
+        s[0] += p[k * total];
+      }
     }
-  }
 #pragma unroll
-  for (int e = 0; e < VEC; e++) put(a, m, n + e, s[e]);
+    for (int e = 0; e < VEC; e++) put(a, m, n + e, s[e]);
+  }
 }
 
 // Tiles of the 16-bit products, and what a k step (64 elements) of one costs in ns: `alone` with few workgroups on the device, `one`
@@ -378,9 +381,13 @@ int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
 }
 int launch_reduce(const char* op, const GemmArgs& a, int slices) {
   const bool vec = a.N % 4 == 0;
-  const dim3 grid((unsigned)dh::ceil_div(a.N, vec ? 1024 : 256), (unsigned)a.M);
-  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, dim3(256), 0, dh::stream(), a, slices);
-  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, dim3(256), 0, dh::stream(), a, slices);
+  const int64_t columns = vec ? a.N / 4 : a.N;
+  unsigned wide = 256;
+  while (wide > 4 && wide / 2 >= columns) wide /= 2;
+  const dim3 block(wide, 256 / wide);
+  const dim3 grid((unsigned)dh::ceil_div(columns, wide), (unsigned)std::min<int64_t>(dh::ceil_div(a.M, block.y), 65535));
+  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, block, 0, dh::stream(), a, slices);
+  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, block, 0, dh::stream(), a, slices);
   DH_CHECK_LAUNCH(op);
   return 0;
 }

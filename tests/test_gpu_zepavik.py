@@ -193,6 +193,22 @@ def test_dense_matmul_f32_slices(L, M, N, K):
     assert (C[:, :N].double() - want).abs().max() < 5e-5 and (C[:, N:] == 9.0).all()
 
 
+@pytest.mark.parametrize("M,N,K,operand", [(70000, 16, 4096, "f32"), (66000, 17, 12288, "bf16"), (66000, 20, 12288, "f16")])
+def test_tall_narrow_products_in_slices(L, M, N, K, operand):
+    """More rows than a grid's second dimension holds, and few enough columns that k is cut into slices."""
+    dtype, code = dict(f32=(torch.float32, capi.F32), bf16=(torch.bfloat16, capi.BF16), f16=(torch.float16, capi.F16))[operand]
+    g = torch.Generator(device="cuda").manual_seed(N)
+    A = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16 if operand == "f32" else dtype)
+    C = torch.full((M, N + 3), 9.0, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), code, K, W.data_ptr(), K, M, N, K, 1.0, None, None, C.data_ptr(), N + 3, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    want = torch.cat([A[i:i + 8192].double() @ W.double().T for i in range(0, M, 8192)])
+    # unit products: sums of up to 12288 terms in 32 bits
+    assert (C[:, :N].double() - want).abs().max() < 5e-5 and (C[:, N:] == 9.0).all()
+
+
 def test_f32_products_are_not_reduced_precision(L):
     """Activations that differ from a constant in their last bits only: bf16- or TF32-like operands would lose them."""
     M, N, K = 40, 70, 256

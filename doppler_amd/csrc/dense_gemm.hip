@@ -361,8 +361,8 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool gl
   return best;
 }
 
-// A tile's rows are addressed by 32-bit byte offsets (rows millions of elements long are out of reach).
-bool within_reach(int64_t rows, int64_t ld, int64_t K) { return 2 * (std::min<int64_t>(rows, 256) * ld + K) < (int64_t)1 << 32; }
+// A tile's rows are addressed by 32-bit byte offsets from its first (rows millions of elements long are out of reach; a single row never is).
+bool within_reach(int64_t rows, int64_t ld, int64_t K) { return 2 * ((std::min<int64_t>(rows, 256) - 1) * ld + K) < (int64_t)1 << 32; }
 
 // LDS beyond 64 KB is asked for once per kernel.
 template <class Tile, bool F16, int ACT, bool GROUPED, bool GLU>

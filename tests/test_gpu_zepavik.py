@@ -209,6 +209,24 @@ def test_tall_narrow_products_in_slices(L, M, N, K, operand):
     assert (C[:, :N].double() - want).abs().max() < 5e-5 and (C[:, N:] == 9.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("far", ["activations", "weights"])
+def test_dense_matmul_rows_4_gb_apart(L, far, dtype):
+    """Two rows as far apart as a 32-bit stride allows."""
+    M, N, K, ld = (2, 70, 64, 2 ** 31 - 64) if far == "activations" else (70, 2, 64, 2 ** 31 - 64)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    A, W = torch.randn(M, K, generator=g, device="cuda").to(dtype), torch.randn(N, K, generator=g, device="cuda").to(dtype)
+    wide = torch.zeros(ld + K, dtype=dtype, device="cuda")
+    wide[:K], wide[ld:] = (A if far == "activations" else W)
+    C, code = torch.zeros(M, N, device="cuda"), capi.BF16 if dtype == torch.bfloat16 else capi.F16
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(wide.data_ptr() if M == 2 else A.data_ptr(), code, ld if M == 2 else K, wide.data_ptr() if N == 2 else W.data_ptr(),
+                                 ld if N == 2 else K, M, N, K, 1.0, None, None, C.data_ptr(), N, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    # 64 terms of size up to 4 x 4 in 32 bits
+    assert (C.double() - A.double() @ W.double().T).abs().max() < 64 * 16 * 2.0 ** -23
+
+
 def test_f32_products_are_not_reduced_precision(L):
     """Activations that differ from a constant in their last bits only: bf16- or TF32-like operands would lose them."""
     M, N, K = 40, 70, 256

@@ -795,10 +795,13 @@ def runScale(input, scale, count=None, outputBuffer=None, inplace=False, **_igno
     n = _nbytes(input) // 4 if count is None else count
     if n * 4 > _nbytes(input):
         raise DopplerHipError("[Scale] count=%d exceeds the input buffer." % n)
-    # the result has the input's shape: a buffer made here holds all of it, also where only `count` elements are scaled
-    out = input.buffer if inplace else _out(outputBuffer, n * 4 if outputBuffer is not None else max(n, int(np.prod(input.shape))) * 4)
+    # the result has the input's shape: a buffer made here holds all of it, also where only `count` elements are scaled; a caller's
+    # buffer that does not is described by those elements
+    whole = int(np.prod(input.shape))
+    out = input.buffer if inplace else _out(outputBuffer, n * 4 if outputBuffer is not None else max(n, whole) * 4)
+    shape = input.shape if _nbytes(out) >= 4 * whole else (n,)
     capi.check(_lib().dh_scale(_ptr(input), _ptr(out), n, float(scale)))
-    return Tensor(out, input.dtype, input.shape, "scale_output")
+    return Tensor(out, input.dtype, shape, "scale_output")
 
 
 def runGather(indices, embeddings, numTokens, hiddenSize, vocabSize, outputBuffer=None, embeddingDtype=None,

@@ -852,6 +852,13 @@ def test_scale_of_a_part_holds_its_whole_shape():
     assert tuple(part.shape) == x.shape and part.buffer.numel() >= x.nbytes
     got = ops.readTensor(part).reshape(x.shape)
     assert np.array_equal(got[0], x[0] * np.float32(0.3)) and not got[1:].any()
+    # a caller's buffer: of the whole shape, and of the part alone (described by what it holds)
+    for nbytes, shape in ((x.nbytes, x.shape), (1536 * 4, (1536,)), (x.nbytes - 4, (1536,))):
+        part = ops.runScale(ops.tensorFromNumpy(x), 0.3, count=1536, outputBuffer=ops.acquireBuffer(nbytes))
+        assert tuple(part.shape) == shape
+        assert np.array_equal(ops.readTensor(part)[:1536], x[0] * np.float32(0.3))
+    with pytest.raises(capi.DopplerHipError, match="too small"):
+        ops.runScale(ops.tensorFromNumpy(x), 0.3, count=1536, outputBuffer=ops.acquireBuffer(1536 * 4 - 4))
 
 
 def test_split_qkv_exact():

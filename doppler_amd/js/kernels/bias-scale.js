@@ -44,16 +44,21 @@ async function scaleTensor(recorder, input, scale, options = {}) {
   if (count * 4 > input.buffer.size) {
     throw new Error(`[Scale] count=${count} exceeds the input buffer.`);
   }
-  const owned = !inplace && !outputBuffer ? acquireBuffer(count * 4, undefined, 'scale_output') : null;
+  // The result has the input's shape: a buffer made here holds all of it (zeros behind the scaled elements, which a buffer from the pool
+  // need not have), also where only `count` elements are scaled; a caller's buffer that does not is described by those elements.
+  const whole = input.shape.reduce((a, b) => a * b, 1);
+  const elements = Math.max(count, whole);
+  const owned = !inplace && !outputBuffer ? acquireBuffer(elements * 4, undefined, 'scale_output') : null;
   const output = inplace ? input.buffer : (outputBuffer || owned);
   try {
+    if (owned && count < elements) getNative().fillZero(output.ptr, count * 4, (elements - count) * 4);
     getNative().scale(input.buffer.ptr, output.ptr, count, scale);
   } catch (error) {
     if (owned) releaseBuffer(owned);
     throw error;
   }
   noteDispatch(recorder, 'scale');
-  return createTensor(output, input.dtype, [...input.shape], 'scale_output');
+  return createTensor(output, input.dtype, output.size >= whole * 4 ? [...input.shape] : [count], 'scale_output');
 }
 
 export async function runScale(input, scale, options = {}) {

@@ -126,6 +126,18 @@ async function main() {
       const s = await dh.runScale(b, c.scale);
       await save(c.name + '.bias.out.bin', b.buffer, c.tokens * c.dim * 4);
       await save(c.name + '.scale.out.bin', s.buffer, c.tokens * c.dim * 4);
+    } else if (c.op === 'scale_part') {
+      const x = tensor(c.x, 'f32', [c.rows, c.dim]);
+      const used = dh.acquireBuffer(c.rows * c.dim * 4);           // the pool hands out buffers that were used before
+      dh.uploadData(used, new Float32Array(c.rows * c.dim).fill(5));
+      dh.releaseBuffer(used);
+      const s = await dh.runScale(x, c.scale, { count: c.dim });
+      if (s.shape.join() !== x.shape.join() || s.buffer.size < c.rows * c.dim * 4) throw new Error('runScale: the buffer must hold the shape');
+      await save(out, s.buffer, s.buffer.size);
+      const short = await dh.runScale(x, c.scale, { count: c.dim, outputBuffer: dh.acquireBuffer(c.dim * 4) });
+      if (short.shape.join() !== String(c.dim)) throw new Error('runScale: the shape of a short buffer');
+      const full = await dh.runScale(x, c.scale, { count: c.dim, outputBuffer: dh.acquireBuffer(c.rows * c.dim * 4) });
+      if (full.shape.join() !== x.shape.join()) throw new Error('runScale: the shape of a full buffer');
     } else if (c.op === 'split_qkv') {
       const ck = dh.acquireBuffer(c.maxSeq * c.kvHeads * c.headDim * 2);
       const cv = dh.acquireBuffer(c.maxSeq * c.kvHeads * c.headDim * 2);

@@ -236,6 +236,10 @@ def test_js_host_path_parity(tmp_path):
     cases.append(dict(name="biasscale", op="bias_scale", x=put("bs.x", bx), bias=put("bs.b", bb), tokens=3, dim=1024, scale=0.125))
     checks.append(lambda: np.array_equal(get("biasscale.bias.out.bin", np.float32).reshape(3, 1024), bx + bb[1]))
     checks.append(lambda: np.array_equal(get("biasscale.scale.out.bin", np.float32).reshape(3, 1024), (bx + bb[1]) * np.float32(0.125)))
+    part = synth.normal_f32((6, 1536), 9512)
+    part_want = np.concatenate([part[:1] * np.float32(0.3), np.zeros((5, 1536), np.float32)])
+    cases.append(dict(name="scalepart", op="scale_part", x=put("scalepart.x", part), rows=6, dim=1536, scale=0.3))
+    checks.append(lambda: np.array_equal(get("scalepart.out.bin", np.float32).reshape(6, 1536), part_want))
     sx = synth.normal_f32((3, 1024 + 256 + 256), 9520)
     cases.append(dict(name="splitplain", op="split_plain", x=put("sp.x", sx), tokens=3, q=1024, k=256, v=256))
     checks.append(lambda: np.array_equal(get("splitplain.q.out.bin", np.float32).reshape(3, 1024), sx[:, :1024]))

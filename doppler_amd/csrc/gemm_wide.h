@@ -26,10 +26,13 @@ __device__ __forceinline__ buffer_words_t buffer_words(const void* base) {
 // 16 bytes per lane from base + v_off + s_off to LDS at lds + 16 * lane.  Inline assembly without register results: to the
 // compiler the fetch does not exist, so its own LDS reads wait for no fetch in flight; the waits are written where the data is due.
 // (s_nop: wait states between a vector instruction that writes a scalar operand, or the write of m0, and the fetch.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void fetch_to_lds(const buffer_words_t& words, uint32_t v_off, uint32_t s_off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
-               : "memory");
+               : "m0", "memory");
 }
+#pragma clang diagnostic pop
 // At most `fetches` of this wave's fetches still in flight, all its LDS reads done, then the other waves.
 template <int fetches>
 __device__ __forceinline__ void arrive_and_wait() {

@@ -15,6 +15,11 @@ not on the source, and a change of either turns a correct kernel into one that r
 Both are checked here on the assembly hipcc emits for gfx950 (device pass only, a few seconds).  The first
 check runs in program order and starts over at every label, so it can miss a hazard across a branch but
 never reports a false one; the second is a data-flow analysis over the kernels' control-flow graphs.
+
+Kernels that fetch from memory straight into LDS (gemm_wide.h) have no destination registers, but the first point
+holds for them too, and three more: m0, which names the fetch's place in LDS, belongs to the hand-written statements
+alone; no spill lies in a loop that fetches (it would wait for the fetches in flight, once per use); and a
+workgroup does not end with a fetch in flight (its LDS may be another's by then).
 """
 import os
 import re
@@ -24,9 +29,13 @@ import tempfile
 
 import pytest
 
+from doppler_amd import build as native
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "doppler_amd", "csrc")
 SOURCES = ["q4k_gemv_rows.hip", "q4k_gemv_i8.hip", "q4k_gemv_chain.hip"]
+# kernels whose hand-written fetches go straight into LDS (m0 names the place): no destination registers, waits counted by hand
+FETCHING = ["attention_prefill.hip", "dense_gemm.hip", "q4k_gemm.hip"]
 VMEM_PREFIXES = ("global_", "buffer_", "flat_", "scratch_")
 SREG = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]")
 VREG = re.compile(r"\bv(\d+)\b|\bv\[(\d+):(\d+)\]")
@@ -165,11 +174,9 @@ def assembly():
         pytest.skip("hipcc not available")
     d = tempfile.mkdtemp(prefix="doppler_amd_asm_")
     procs = []
-    for src in SOURCES:
+    for src in SOURCES + FETCHING:
         out = os.path.join(d, src.replace(".hip", ".s"))
-        cmd = [hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-I" + CSRC, "-I" + os.path.join(ROOT, "include"),
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "--cuda-device-only", "-S",
-               os.path.join(CSRC, src), "-o", out]
+        cmd = [hipcc] + native.HIP_FLAGS + native.FILE_FLAGS.get(src, []) + ["--cuda-device-only", "-S", os.path.join(CSRC, src), "-o", out]
         procs.append((src, out, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)))
     paths = {}
     for src, out, p in procs:
@@ -180,7 +187,7 @@ def assembly():
     shutil.rmtree(d, ignore_errors=True)
 
 
-@pytest.mark.parametrize("src", SOURCES)
+@pytest.mark.parametrize("src", SOURCES + FETCHING)
 def test_no_scalar_register_hazard_in_front_of_hand_written_loads(assembly, src):
     assert scalar_operand_hazards(assembly[src]) == []
 
@@ -206,6 +213,73 @@ def test_no_scratch_memory_in_the_streaming_kernels(assembly, src):
     assert {k: v for k, v in used.items() if not any(a in k for a in allowed)} == {}
 
 
+def _is_fetch(s, in_asm):
+    return in_asm and s.startswith("buffer_load") and s.split()[-1] == "lds"
+
+
+def foreign_m0(path):
+    return ["%s line %d: `%s`" % (k, ln, s) for ln, s, in_asm, k in _instructions(path) if not in_asm and re.search(r"\bm0\b", s)]
+
+
+def spills_in_fetching_loops(path):
+    """Loops: from a label to a later branch back to it."""
+    ins = list(_instructions(path))
+    label_at = {s[:-1]: i for i, (_, s, _, _) in enumerate(ins) if s.endswith(":")}
+    hits, loops = set(), 0
+    for i, (_, s, _, kernel) in enumerate(ins):
+        first = label_at.get(s.split()[-1], i) if s.startswith(("s_branch", "s_cbranch")) else i
+        body = ins[first:i]
+        if any(_is_fetch(t, a) for _, t, a, _ in body):
+            loops += 1
+            hits.update("%s line %d: `%s`" % (kernel, ln, t) for ln, t, _, _ in body if t.startswith("scratch_"))
+    return sorted(hits), loops
+
+
+def ends_with_fetches_in_flight(path):
+    """Whether a fetch can reach the program's end with no wait for all vector-memory operations behind it, on any path."""
+    ins = list(_instructions(path))
+    label_at = {s[:-1]: i for i, (_, s, _, _) in enumerate(ins) if s.endswith(":")}
+    hits, seen, fetches = [], set(), 0
+    work = [i for i, (_, s, a, _) in enumerate(ins) if _is_fetch(s, a)]
+    fetches = len(work)
+    work = [i + 1 for i in work]
+    while work:
+        i = work.pop()
+        if i in seen or i >= len(ins):
+            continue
+        seen.add(i)
+        ln, s, _, kernel = ins[i]
+        if s.startswith("s_waitcnt") and _vmcnt(s) == 0:
+            continue
+        if s.startswith("s_endpgm"):
+            hits.append("%s line %d" % (kernel, ln))
+            continue
+        if s.startswith(("s_branch", "s_cbranch")):
+            work.append(label_at[s.split()[-1]])
+        if not s.startswith("s_branch"):
+            work.append(i + 1)
+    return hits, fetches
+
+
+@pytest.mark.parametrize("src", FETCHING)
+def test_m0_belongs_to_the_fetches(assembly, src):
+    assert foreign_m0(assembly[src]) == []
+
+
+@pytest.mark.parametrize("src", FETCHING)
+def test_no_spills_in_loops_that_fetch(assembly, src):
+    hits, loops = spills_in_fetching_loops(assembly[src])
+    assert loops > 0, "the scan found no loop with a fetch in %s: the parser no longer matches the assembly" % src
+    assert hits == []
+
+
+# the prefill attention's last fetch is waited for by a later turn of its loop, which a path through the code need not take
+@pytest.mark.parametrize("src", [s for s in FETCHING if s != "attention_prefill.hip"])
+def test_no_fetch_in_flight_at_the_end(assembly, src):
+    hits, fetches = ends_with_fetches_in_flight(assembly[src])
+    assert fetches > 0 and hits == []
+
+
 def test_the_scans_see_what_they_look_for(tmp_path):
     """The assembly of the build that faulted, reduced to the lines that matter, and a register reuse."""
     bad = tmp_path / "bad.s"
@@ -223,3 +297,9 @@ def test_the_scans_see_what_they_look_for(tmp_path):
         "\tv_mov_b32_e32 v17, 0\n", ""))
     assert scalar_operand_hazards(str(good)) == []
     assert in_flight_destination_hazards(str(good))[0] == []
+    fetch = "\t;;#ASMSTART\n\ts_mov_b32 m0, s4\n\ts_nop 4\n\tbuffer_load_dwordx4 v1, s[8:11], s5 offen lds\n\t;;#ASMEND\n"
+    loop = tmp_path / "loop.s"
+    loop.write_text("kernel_b:\n.LBB0_1:\n" + fetch + "%s\ts_cbranch_scc1 .LBB0_1\n%s\ts_endpgm\n" % ("\tscratch_load_dword v2, off, off\n\ts_mov_b32 m0, 0\n", ""))
+    assert len(foreign_m0(str(loop))) == 1 and len(spills_in_fetching_loops(str(loop))[0]) == 1 and len(ends_with_fetches_in_flight(str(loop))[0]) == 1
+    loop.write_text("kernel_b:\n.LBB0_1:\n" + fetch + "\ts_cbranch_scc1 .LBB0_1\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier\n\tscratch_load_dword v2, off, off\n\ts_endpgm\n")
+    assert foreign_m0(str(loop)) == [] and spills_in_fetching_loops(str(loop)) == ([], 1) and ends_with_fetches_in_flight(str(loop)) == ([], 1)

@@ -421,6 +421,21 @@ int launch_act(const char* op, const GemmArgs& a, bool f16, const TileChoice& pi
   return launch_16bit<false, kAnyAct, false>(op, a, pick);
 }
 
+// k slices that the library's workspace holds the sums of.
+int slices_in_workspace(int64_t M, int64_t N, int most) {
+  size_t ws_bytes = 0;
+  (void)dh::splitk_workspace(&ws_bytes);
+  return (int)std::max<size_t>(1, std::min<size_t>(most, ws_bytes / ((size_t)M * N * sizeof(float))));
+}
+TileChoice choose_16bit(int64_t M, int64_t N, int64_t K) {
+  const int most = slices_in_workspace(M, N, kMaxSlices);
+  TileChoice pick = choose_tile(M, N, K, most, false);
+  const int env_tile = dh::tuning_int("DH_DENSE_TILE", -1), env_slices = dh::tuning_int("DH_DENSE_SLICES", 0);
+  if (env_tile >= 0) pick.tile = env_tile;
+  if (env_slices) pick.slices = std::min(most, env_slices);
+  return pick;
+}
+
 // A product whose rows are out of reach goes in halves.
 int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
   if (a.M > 1 && !within_reach(a.M, a.lda, a.K)) {
@@ -449,42 +464,39 @@ int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
     const int rc = dense_16bit(op, low, f16);
     return rc ? rc : dense_16bit(op, high, f16);
   }
-  size_t ws_bytes = 0;
-  (void)dh::splitk_workspace(&ws_bytes);
-  const int most = (int)std::max<size_t>(1, std::min<size_t>(kMaxSlices, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
-  TileChoice pick = choose_tile(a.M, a.N, a.K, most, false);
-  const int env_tile = dh::tuning_int("DH_DENSE_TILE", -1), env_slices = dh::tuning_int("DH_DENSE_SLICES", 0);
-  if (env_tile >= 0) pick.tile = env_tile;
-  if (env_slices) pick.slices = std::min(most, env_slices);
-  return launch_act(op, a, f16, pick);
+  return launch_act(op, a, f16, choose_16bit(a.M, a.N, a.K));
 }
 
 // k slices of a 32-bit product.  Workgroups on a compute unit share its matrix cores, so the one with the most of them ends last: 64 k of a
 // tile take 1.35 us alone there and 1.1 us each in company (0.85 at the full rate).  Slices cost as in choose_tile.
-int dense_f32(const char* op, GemmArgs a) {
-  a.tiles_m = (int)dh::ceil_div(a.M, 64);
-  a.tiles_n = (int)dh::ceil_div(a.N, 64);
-  size_t ws_bytes = 0;
-  float* ws = dh::splitk_workspace(&ws_bytes);
-  const int64_t steps = a.K / 64, tiles = (int64_t)a.tiles_m * a.tiles_n;
-  const int most = (int)std::max<size_t>(1, std::min<size_t>(16, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
-  const int env_slices = dh::tuning_int("DH_F32_SLICES", 0);
+int choose_f32_slices(int64_t M, int64_t N, int64_t K) {
+  const int64_t steps = K / 64, tiles = dh::ceil_div(M, 64) * dh::ceil_div(N, 64);
+  const int most = slices_in_workspace(M, N, 16), env_slices = dh::tuning_int("DH_F32_SLICES", 0);
+  if (env_slices) return std::min(most, env_slices);
   int slices = 1;
   double least = 1e30;
   for (int s = 1; s <= most && (s == 1 || steps / s >= 2); s++) {
     const int64_t together = dh::ceil_div(tiles * s, dh::num_cus());
     double t = (together == 1 ? 1350.0 : 1100.0 * together) * dh::ceil_div(steps, s);
-    if (s > 1) t += 3500.0 + 4.0 * a.M * a.N * (2 * s + 1) / 4000.0;
+    if (s > 1) t += 3500.0 + 4.0 * M * N * (2 * s + 1) / 4000.0;
     if (t < least) {
       least = t;
       slices = s;
     }
   }
-  if (env_slices) slices = std::min(most, env_slices);
-  a.k_slice = (int)dh::ceil_div(steps, slices) * 64;
-  slices = (int)dh::ceil_div(a.K, a.k_slice);
-  if (slices > 1) a.parts = ws;
-  hipLaunchKernelGGL((gemm_f32_kernel<1, false, false>), dim3((unsigned)tiles, slices), dim3(256), 0, dh::stream(), a);
+  return slices;
+}
+// k of a slice (whole steps of 64).
+int slice_extent(int64_t K, int slices) { return (int)dh::ceil_div(K / 64, slices) * 64; }
+
+int dense_f32(const char* op, GemmArgs a) {
+  a.tiles_m = (int)dh::ceil_div(a.M, 64);
+  a.tiles_n = (int)dh::ceil_div(a.N, 64);
+  a.k_slice = slice_extent(a.K, choose_f32_slices(a.M, a.N, a.K));
+  const int slices = (int)dh::ceil_div(a.K, a.k_slice);
+  size_t ws_bytes = 0;
+  if (slices > 1) a.parts = dh::splitk_workspace(&ws_bytes);
+  hipLaunchKernelGGL((gemm_f32_kernel<1, false, false>), dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n), slices), dim3(256), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   return slices > 1 ? launch_reduce(op, a, slices) : 0;
 }
@@ -570,4 +582,18 @@ extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, con
   a.C2 = d_C2; a.ldc2 = ldc2; a.c2_dtype = c2_dtype; a.act = activation;
   if (a_dtype == DH_F32) return dense_f32(op, a);
   return dense_16bit(op, a, a_dtype == DH_F16);
+}
+
+extern "C" int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int glu, int num_cus, int64_t* out3) {
+  const char* op = "dh_dense_matmul_layout";
+  if (!out3 || M <= 0 || N <= 0 || K <= 0 || K % 64) return dh::fail(1, "[%s] M=%d, N=%d, K=%d (a multiple of 64), or no place for the result", op, M, N, K);
+  dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
+  const bool wide = a_dtype == DH_F32;
+  const TileChoice pick = wide ? TileChoice{0, glu ? 1 : choose_f32_slices(M, N, K)} : glu ? choose_tile(M, N, K, 1, true) : choose_16bit(M, N, K);
+  dh::plan_end();
+  const TileCost& c = glu && pick.tile == 3 ? kSmallGlu : kTiles[pick.tile];
+  out3[0] = wide ? 64 : c.bm;
+  out3[1] = wide ? (glu ? 128 : 64) : c.bn;
+  out3[2] = dh::ceil_div(K, slice_extent(K, pick.slices));
+  return 0;
 }

@@ -105,7 +105,7 @@ void graph_note_finiteness(const GraphFiniteCall& call) {
   g->fin[g->n_fin++] = call;
 }
 float* splitk_workspace(size_t* bytes) {
-  *bytes = g_splitk_ws ? kSplitKWsBytes : 0;
+  *bytes = g_splitk_ws || t_plan_cus > 0 ? kSplitKWsBytes : 0;      // a plan counts on it
   return g_splitk_ws;
 }
 float* gemm_row_scale() { return g_row_scale; }

@@ -865,45 +865,62 @@ constexpr WideCost kWide[] = {{256, 256, 1, 1200.f, 1950.f, 1950.f, 8000.f},    
                               {128, 256, 1, 760.f, 1120.f, 1250.f, 9000.f},        // <1, 4, 4>
                               {128, 256, 1, 845.f, 1200.f, 1250.f, 5500.f},        // <2, 4, 2>
                               {128, 128, 2, 580.f, 720.f, 1280.f, 5000.f}};        // <2, 2, 2>
+struct WideChoice {
+  int tile, pieces;
+};
 // The cheapest of them, with K cut in pieces (of whole super-blocks) where that pays for the reduction.
-template <bool DUAL>
-int launch_wide_best(GemmArgs a, const char* op) {
-  const int64_t cus = dh::num_cus(), steps = dh::ceil_div(a.K, BK);
+WideChoice choose_wide(int64_t M, int64_t N, int64_t K, bool dual) {
+  const int64_t cus = dh::num_cus(), steps = dh::ceil_div(K, BK);
   size_t ws_bytes = 0;
-  float* ws = dh::splitk_workspace(&ws_bytes);
-  const int most = DUAL || !ws ? 1 : (int)std::max<size_t>(1, std::min<size_t>(kMaxSplit, ws_bytes / ((size_t)a.M * a.N * sizeof(float))));
-  int pick = 0, split = 1;
+  (void)dh::splitk_workspace(&ws_bytes);
+  const int most = dual ? 1 : (int)std::max<size_t>(1, std::min<size_t>(kMaxSplit, ws_bytes / ((size_t)M * N * sizeof(float))));
+  WideChoice best{0, 1};
   double least = 1e30;
   for (int i = 0; i < 4; i++) {
     const WideCost& c = kWide[i];
     for (int s = 1; s <= most && (s == 1 || steps >= 8 * s); s++) {
-      const int64_t groups = dh::ceil_div(a.M, c.bm) * dh::ceil_div(a.N, DUAL ? c.rows / 2 : c.rows) * s, slots = cus * c.per_cu, left = groups % slots;
+      const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, dual ? c.rows / 2 : c.rows) * s, slots = cus * c.per_cu, left = groups % slots;
       const double f = (double)left / cus;
       const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (0.85 + 0.15 * f / c.per_cu);
       double t = 4.0 * dh::ceil_div(steps, 4 * s) * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + c.start;
-      if (s > 1) t += 3500.0 + 4.0 * a.M * a.N * (2 * s + 1) / 4000.0;
+      if (s > 1) t += 3500.0 + 4.0 * M * N * (2 * s + 1) / 4000.0;
       if (t < least) {
         least = t;
-        pick = i;
-        split = s;
+        best = WideChoice{i, s};
       }
     }
   }
   const int env_tile = dh::tuning_int("DH_Q4_TILE", -1);
-  if (env_tile >= 0) pick = env_tile;
-  if (split > 1) {
-    a.kt_per_split = (int)dh::ceil_div(steps, 4 * split) * 4;
-    a.ksplit = (int)dh::ceil_div(steps, a.kt_per_split);
-    if (a.ksplit > 1) a.partial = ws;
+  if (env_tile >= 0) best.tile = env_tile;
+  return best;
+}
+// Steps of 64 k in a piece.
+int64_t steps_per_piece(int64_t K, int pieces) { return dh::ceil_div(dh::ceil_div(K, BK), 4 * pieces) * 4; }
+
+template <bool DUAL>
+int launch_wide_best(GemmArgs a, const char* op) {
+  const WideChoice pick = choose_wide(a.M, a.N, a.K, DUAL);
+  if (pick.pieces > 1) {
+    a.kt_per_split = (int)steps_per_piece(a.K, pick.pieces);
+    a.ksplit = (int)dh::ceil_div(dh::ceil_div(a.K, BK), a.kt_per_split);
+    size_t ws_bytes = 0;
+    if (a.ksplit > 1) a.partial = dh::splitk_workspace(&ws_bytes);
   }
   int rc;
-  switch (pick) {
+  switch (pick.tile) {
     case 0: rc = launch_wide<Q4Tile<2, 4, 4>, DUAL>(a, op); break;
     case 1: rc = launch_wide<Q4Tile<1, 4, 4>, DUAL>(a, op); break;
     case 2: rc = launch_wide<Q4Tile<2, 4, 2>, DUAL>(a, op); break;
     default: rc = launch_wide<Q4Tile<2, 2, 2>, DUAL>(a, op); break;
   }
   return rc || a.ksplit <= 1 ? rc : launch_reduce(a, op);
+}
+
+// Products of enough work, or of enough tiles, go to q4k_wide_kernel: where a step's latency counts instead of its throughput the other
+// kernel is ahead, because its waves share one dequantised tile (us, that one / the wide one: 1300 x 513 x 1100 21 / 28, 512 x 1152 x 6912
+// 34 / 38, 64 x 4096 x 4096 25 / 27, but 1024 x 2048 x 1024 38 / 27, 200 x 6144 x 4096 43 / 39, 512 x 4096 x 12288 164 / 87).
+bool takes_wide(int64_t M, int64_t N, int64_t K, bool dual) {
+  return dh::ceil_div(M, 256) * dh::ceil_div(N, 128) >= dh::num_cus() || (double)M * N * K * (dual ? 2 : 1) >= (M >= 1024 ? 2e9 : 5e9);
 }
 
 // 128 x 128 tiles when they occupy at least half of the compute units (their higher matrix-core
@@ -954,15 +971,11 @@ int launch_gemm(GemmArgs a, const char* op) {
   DH_CHECK_LAUNCH(op);
   a.row_scale = scales;
   a.Apk = packed;
-  // Products of enough work, or of enough tiles, go to q4k_wide_kernel: where a step's latency counts instead of its throughput the kernel
-  // below is ahead, because its waves share one dequantised tile (us, this one / the wide one: 1300 x 513 x 1100 21 / 28, 512 x 1152 x 6912
-  // 34 / 38, 64 x 4096 x 4096 25 / 27, but 1024 x 2048 x 1024 38 / 27, 200 x 6144 x 4096 43 / 39, 512 x 4096 x 12288 164 / 87).  There: for
-  // the fused gate/up pair 128 x 64 tiles (eight waves), then 128 x 128 (four waves, two workgroups per compute unit) when those
-  // occupy at least half of the compute units, else 64 x 64.
-  const int64_t big_tiles = dh::ceil_div(a.M, 128) * dh::ceil_div(a.N, 128);
-  const int64_t tall_tiles = dh::ceil_div(a.M, 256) * dh::ceil_div(a.N, 128);
   a.ksplit = 1;
-  if (tall_tiles >= dh::num_cus() || (double)a.M * a.N * a.K * (DUAL ? 2 : 1) >= (a.M >= 1024 ? 2e9 : 5e9)) return launch_wide_best<DUAL>(a, op);
+  if (takes_wide(a.M, a.N, a.K, DUAL)) return launch_wide_best<DUAL>(a, op);
+  // The other kernel: for the fused gate/up pair 128 x 64 tiles (eight waves), then 128 x 128 (four waves, two workgroups per compute
+  // unit) when those occupy at least half of the compute units, else 64 x 64.
+  const int64_t big_tiles = dh::ceil_div(a.M, 128) * dh::ceil_div(a.N, 128);
   if (2 * big_tiles >= dh::num_cus()) {
     if constexpr (DUAL) {
       return launch_gemm_cfg<true, 1, 2>(a, op);
@@ -1041,3 +1054,16 @@ int q4k_gemm_gate_up(const char* op, const float* A, const uint8_t* Wg, const ui
 }
 
 }  // namespace dh
+
+extern "C" int dh_q4k_gemm_layout(int M, int N, int K, int dual, int num_cus, int64_t* out4) {
+  if (!out4 || M < 16 || N <= 0 || K <= 0) return 0;
+  dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
+  const int wide = takes_wide(M, N, K, dual != 0) ? 1 : 0;
+  const WideChoice pick = choose_wide(M, N, K, dual != 0);
+  dh::plan_end();
+  const int64_t steps = dh::ceil_div(K, BK);
+  constexpr int rows_per_wave[] = {128, 128, 64, 64};
+  const int64_t out[4] = {kWide[pick.tile].bm, kWide[pick.tile].rows, rows_per_wave[pick.tile], dh::ceil_div(steps, steps_per_piece(K, pick.pieces))};
+  for (int i = 0; i < 4; i++) out4[i] = wide ? out[i] : 0;
+  return wide;
+}

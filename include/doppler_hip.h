@@ -167,6 +167,11 @@ int dh_q4k_matmul_plan(int M, int N, int K, int normed, int dual, int num_cus);
  * arithmetic on the host; other families leave the record zero.  No counterpart in the reference. */
 int dh_q4k_gemv_layout(int M, int N, int K, int normed, int dual, int num_cus, int64_t* out12);
 
+/* The tiles dh_q4k_matmul (dual = 0) or dh_q4k_ffn_gate_up (dual = 1) would take from 16 rows on, for one pass of M rows: out4 = { rows of
+ * a tile, weight rows of a tile (of both matrices of a pair), rows of a wave, pieces K is cut into }.  Returns 1, or 0 with zeros where the
+ * kernel for smaller products serves the shape.  For tests that have to reach every tile; needs no device. */
+int dh_q4k_gemm_layout(int M, int N, int K, int dual, int num_cus, int64_t* out4);
+
 /* out[M,inter] = clamp(act(x.Wgate^T) * (x.Wup^T) * alpha).
  * Replaces runFusedFFN/recordFusedFFN, src/gpu/kernels/fused_ffn.js:501,605
  * (fused_ffn_q4k.wgsl:129-363).  clamp (swigluLimit) applies to DH_ACT_SILU only;
@@ -379,6 +384,9 @@ int dh_dense_matmul(const void* d_A, int a_dtype, int lda, const void* d_W, int 
 int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K, float alpha,
                            const float* d_bias, const float* d_col_scale, const float* d_residual, float* d_C, int ldc,
                            int n_first, void* d_C2, int c2_dtype, int ldc2, int activation);
+/* The tile dh_dense_matmul would take for activations of a_dtype (glu = 1: the shared expert's gate and up product of dh_experts_prefill):
+ * out3 = { rows, columns, slices k is cut into }.  For tests that have to reach every tile; needs no device. */
+int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int glu, int num_cus, int64_t* out3);
 
 /* The same product for ONE f32 activation row (decode; HBM-bound), d_C2 in f32, with an optional RMSNorm of the
  * row in its prologue: x * rsqrt(mean of the first `hidden` elements squared + eps) * w.  d_x and d_norm_weight

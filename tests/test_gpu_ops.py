@@ -5,6 +5,8 @@ Bars: bit-exact for Q4_K unpacking / dequantized weights, 
 results (argmax, gather, f16 narrowing); relative L2 <= 1e-3 for f32-accumulate matmul,
 attention and logits.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -209,7 +211,7 @@ def test_matmul_prefill_gemm(M, N, K, kw):
 @pytest.mark.parametrize("M,N,K,kw", [(1000, 8200, 320, dict(residual=True)), (1024, 8192, 256, dict(outputDtype="f16")),
                                       (2048, 4224, 192, dict(alpha=0.5))])
 def test_matmul_prefill_gemm_tall_tiles(M, N, K, kw):
-    """Enough 256 x 128 tiles to fill 256 compute units: the eight-wave tall-tile kernel, with ragged edges in M
+    """Enough rows and columns for 256 tiles of 256 x 128, which makes it the wide kernel however short K is: ragged edges in M
     and N, an odd number of K steps and a K that ends inside a super-block."""
     assert -(-M // 256) * -(-N // 128) >= 256
     assert _matmul_case(M, N, K, seed=1560 + K, **kw) <= REL_L2_F16_MFMA
@@ -217,7 +219,7 @@ def test_matmul_prefill_gemm_tall_tiles(M, N, K, kw):
 
 @pytest.mark.parametrize("M,hidden,inter,activation", [(1000, 320, 8200, "silu"), (1024, 256, 8192, "gelu")])
 def test_fused_ffn_prefill_tall_tiles(M, hidden, inter, activation):
-    """The fused gate/up pair on 256 x 128 x 2 tiles."""
+    """The same of the fused gate/up pair."""
     Wg, wg = q4k_weight(inter, hidden, seed=2410)
     Wu, wu = q4k_weight(inter, hidden, seed=2411)
     X = synth.normal_f32((M, hidden), seed=2412, scale=0.05)
@@ -811,13 +813,28 @@ def test_bias_add_and_scale_bit_exact():
     assert same.buffer is xt.buffer and np.array_equal(ops.readTensor(xt).reshape(x.shape), x * s)
 
 
-# products large enough for the wide prefill kernel: edges of every tile of it in M and N, K off the 64 and the 256, K in pieces, both
-# kinds of output, norm and residual; reference: the dequantised weights (bit-exact above) in 64 bits
-@pytest.mark.parametrize("M,N,K,pair,f16_out", [(1030, 2100, 1100, False, False), (2050, 6150, 1088, False, True), (1041, 4097, 2300, False, False),
-                                                (600, 4100, 4032, False, False), (513, 130, 81920, False, False), (1100, 1030, 1024, True, False),
-                                                (1025, 5000, 300, True, False), (520, 6900, 1152, True, False)])
-def test_prefill_products_of_the_wide_kernel(M, N, K, pair, f16_out):
+# Products large enough for the wide prefill kernel, with the tile each takes on 256 compute units: rows, weight rows (of both matrices of a
+# pair), rows of a wave, pieces of K.  Every tile, whole and in pieces, plain and gated; edges in M and N, K off the 64 and the 256.
+WIDE_PRODUCTS = [
+    (1030, 2100, 1100, False, False, (128, 128, 64, 1)), (2050, 6150, 1088, False, True, (256, 256, 128, 1)), (1041, 4097, 2300, False, False, (128, 256, 64, 1)),
+    (600, 4100, 4032, False, False, (128, 128, 64, 1)), (513, 130, 81920, False, False, (128, 128, 64, 8)), (1100, 1030, 1024, True, False, (128, 128, 64, 1)),
+    (1025, 5000, 300, True, False, (128, 128, 64, 1)), (520, 6900, 1152, True, False, (256, 256, 128, 1)),
+    (1049, 1061, 1861, False, True, (128, 128, 64, 2)), (1829, 2215, 554, False, True, (128, 256, 64, 1)), (946, 1350, 4612, False, False, (128, 256, 64, 5)),
+    (1582, 2529, 2601, False, False, (128, 256, 128, 1)), (1255, 1583, 7763, False, True, (128, 256, 128, 3)), (1703, 4807, 523, False, False, (256, 256, 128, 1)),
+    (1538, 2528, 10169, False, False, (256, 256, 128, 2)), (1652, 1225, 511, True, False, (128, 256, 64, 1)), (1676, 1190, 2575, True, False, (128, 256, 128, 1)),
+    (1673, 2351, 548, True, False, (256, 256, 128, 1))]
+
+
+def wide_tile(M, N, K, pair, num_cus=0):
+    out = (ctypes.c_int64 * 4)()
+    return tuple(out) if capi.load().dh_q4k_gemm_layout(M, N, K, int(pair), num_cus, out) else None
+
+
+# reference: the dequantised weights (bit-exact above) in 64 bits
+@pytest.mark.parametrize("M,N,K,pair,f16_out,tile", WIDE_PRODUCTS)
+def test_prefill_products_of_the_wide_kernel(M, N, K, pair, f16_out, tile):
     import torch
+    assert wide_tile(M, N, K, pair) == tile
     W = [synth.q4k_centred(synth.q4k_tensor(N, K, seed=7000 + i)) for i in range(2 if pair else 1)]
     wb = [ops.createWeightBuffer(ops.uploadData(ops.acquireBuffer(w.size), w), "q4k", "row", (N, K)) for w in W]
     nb = (K + 255) // 256

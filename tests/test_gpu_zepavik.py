@@ -161,6 +161,72 @@ def test_dense_matmul_large_tiles(L, M, N, K, first, dtype):
         assert (C2[:, N - first:] == 9.0).all()
 
 
+# every tile of the 16-bit products, whole and in k slices (with a short last one), k steps of either parity, ragged in both directions; the
+# tile and the slices are those of 256 compute units
+TILES = [(129, 130, 192, (64, 64, 1)), (2, 33, 1664, (64, 64, 3)), (1928, 1074, 640, (128, 128, 1)), (1073, 1932, 704, (128, 128, 1)),
+         (645, 457, 4608, (128, 128, 6)), (649, 486, 4864, (128, 128, 7)), (1299, 3078, 640, (256, 128, 1)), (1299, 3078, 704, (256, 128, 1)),
+         (1165, 1684, 9664, (256, 128, 3)), (2720, 4759, 1152, (256, 256, 1)), (2060, 6150, 1600, (256, 256, 1)), (129, 11422, 14144, (256, 256, 5))]
+# gate and up products of a shared expert (32 gate rows, 32 up rows, ..)
+GLU_TILES = [(300, 256, 704, (64, 128, 1)), (1234, 1664, 704, (128, 128, 1)), (1928, 2176, 640, (256, 128, 1)), (2224, 5632, 1344, (256, 256, 1))]
+
+
+def tile_of(L, M, N, K, code, glu=False, num_cus=0):
+    out = (ctypes.c_int64 * 3)()
+    capi.check(L.dh_dense_matmul_layout(M, N, K, code, int(glu), num_cus, out))
+    return tuple(out)
+
+
+@pytest.mark.parametrize("M,N,K,tile", TILES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_matmul_every_tile(L, M, N, K, tile, dtype):
+    code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
+    assert tile_of(L, M, N, K, code) == tile
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda").to(dtype)
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(dtype)
+    acc = A.double() @ W.double().T
+    for first, act, fn in ((N, capi.ACT_NONE, None), (N // 3, capi.ACT_NONE, lambda z: z), (N // 3, capi.ACT_RELU2, lambda z: z.clamp(min=0).square()),
+                           (N // 3, capi.ACT_GELU_ERF, lambda z: 0.5 * z * (1 + torch.erf(z * 0.5 ** 0.5)))):
+        C, C2 = torch.full((M, first + 3), 9.0, device="cuda"), torch.full((M, N - first + 2), 9.0, dtype=dtype, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_dense_matmul(A.data_ptr(), code, K, W.data_ptr(), K, M, N, K, 1.0, None, None, C.data_ptr(), first + 3, first,
+                                     C2.data_ptr(), code, N - first + 2, act))
+        capi.check(L.dh_sync())
+        # unit products: sums of up to 14144 exact terms in 32 bits; a second output is rounded once more
+        assert (C[:, :first].double() - acc[:, :first]).abs().max() < 5e-5 and (C[:, first:] == 9.0).all()
+        if first < N:
+            want = fn(acc[:, first:])
+            assert ((C2[:, :N - first].double() - want).abs() <= 2.0 ** (-8 if code == capi.BF16 else -10) * want.abs() + 2e-4).all()
+            assert (C2[:, N - first:] == 9.0).all()
+
+
+@pytest.mark.parametrize("T,N,K,tile", GLU_TILES)
+def test_shared_expert_on_every_tile(L, T, N, K, tile):
+    """The routed expert's weights are zero, so that what is added to the rows is the shared expert's result alone.  Its activations are
+    rounded to bf16 in front of the down product (2^-9 of each, added up over ff of them in a product of random signs)."""
+    assert tile_of(L, T, N, K, capi.BF16, glu=True) == tile
+    ff, hidden, limit = N // 2, 128, 1.5
+    g = torch.Generator(device="cuda").manual_seed(T)
+    h = torch.randn(T, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = lambda rows, k: (torch.randn(rows, k, generator=g, device="cuda") / k ** 0.5).to(torch.bfloat16)
+    up, down, router, norm = w(N, K), w(K, ff)[:hidden].contiguous(), w(2, K), torch.ones(K, device="cuda")
+    none = torch.zeros(max(128, K), max(64, K), dtype=torch.bfloat16, device="cuda")
+    spec = capi.Experts(hidden, K, 1, 1, 64, ff, 1e-5, 7.0, limit, norm.data_ptr(), None, router.data_ptr(), none.data_ptr(), none.data_ptr(), up.data_ptr(),
+                        down.data_ptr())
+    ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T), dtype=torch.uint8, device="cuda")
+    x = torch.zeros(T, hidden, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_experts_prefill(ctypes.byref(spec), h.data_ptr(), capi.BF16, x.data_ptr(), hidden, ws.data_ptr(), T))
+    capi.check(L.dh_sync())
+    z = (h.double() @ up.double().T).view(T, ff // 32, 2, 32)
+    gate, lin = (z[:, :, i].reshape(T, ff) for i in (0, 1))
+    gate = gate.clamp(max=limit)
+    act = gate * torch.sigmoid(1.702 * gate) * (lin.clamp(-limit, limit) + 1) * torch.sigmoid(h.double() @ router[1].double())[:, None]
+    want = act @ down.double().T
+    assert ((x.double() - want).norm(dim=1) <= 2.0 ** -8 * want.norm(dim=1)).all()
+    assert ((x.double() - want).norm(dim=0) <= 2.0 ** -8 * want.norm(dim=0)).all()
+
+
 # the smallest tile: k steps of every remainder by its four buffers, one row and column over and under its edges
 @pytest.mark.parametrize("M,N,K", [(64, 64, 64), (65, 63, 128), (33, 129, 192), (63, 65, 256), (3, 97, 320), (130, 31, 448)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

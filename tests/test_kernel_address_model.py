@@ -292,3 +292,24 @@ def test_a_smaller_device_changes_the_layout_not_the_bounds():
     check_i8(2, 4096, 12288, 0, 0, ncu=304)
     check_rows(8, 4096, 4096, 0, 0, ncu=64)
     check_rows(4, 4096, 12288, 0, 0, ncu=304)
+
+
+def test_the_product_tests_reach_every_tile():
+    """The shapes of the matrix products' GPU tests take the tiles named beside them, and together every one a product of many shapes takes."""
+    from tests import test_gpu_ops, test_gpu_zepavik
+    L, rng = capi.load(), np.random.Generator(np.random.PCG64(5))
+    for M, N, K, pair, _, tile in test_gpu_ops.WIDE_PRODUCTS:
+        assert test_gpu_ops.wide_tile(M, N, K, pair, NCU) == tile, (M, N, K, pair)
+    for glu, cases in ((False, test_gpu_zepavik.TILES), (True, test_gpu_zepavik.GLU_TILES)):
+        for M, N, K, tile in cases:
+            assert test_gpu_zepavik.tile_of(L, M, N, K, capi.BF16, glu, NCU) == tile, (M, N, K, glu)
+    wide = {(pair, tile[:3], tile[3] > 1) for *_, pair, _, tile in test_gpu_ops.WIDE_PRODUCTS}
+    dense = {(glu, tile[:2], tile[2] > 1) for glu, cases in ((False, test_gpu_zepavik.TILES), (True, test_gpu_zepavik.GLU_TILES)) for *_, tile in cases}
+    for M, N, K in np.exp2(rng.uniform((4, 6, 6), (11.5, 14, 14.2), (20000, 3))).astype(int).tolist():
+        K64 = -(-K // 64) * 64
+        for two in (False, True):
+            t = test_gpu_ops.wide_tile(M, N, K, two, NCU)
+            assert t is None or (two, t[:3], t[3] > 1) in wide, (M, N, K, two, t)
+            n = -(-N // 128) * 128 if two else N
+            t = test_gpu_zepavik.tile_of(L, M, n, K64, capi.BF16, two, NCU)
+            assert (two, t[:2], t[2] > 1) in dense, (M, n, K64, two, t)

@@ -29,7 +29,7 @@ __device__ __forceinline__ buffer_words_t buffer_words(const void* base) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void fetch_to_lds(const buffer_words_t& words, uint32_t v_off, uint32_t s_off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
                : "m0", "memory");
 }
 #pragma clang diagnostic pop

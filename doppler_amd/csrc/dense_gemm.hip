@@ -288,13 +288,13 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
 }
 
 // Sums of the k slices in slice order.  VEC columns per thread (N a multiple of VEC), a block's threads as wide as the row allows and the
-// rest of them on further rows; a grid's second dimension holds 65535 blocks, so rows go round.
+// rest of them on further rows (thread t: column t % wide, row t / wide); a grid's second dimension holds 65535 blocks, so rows go round.
 template <int VEC>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int slices) {
-  const int n = VEC * (blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int slices, int log2_wide, int round) {
+  const int n = VEC * ((blockIdx.x << log2_wide) + (threadIdx.x & ((1 << log2_wide) - 1)));
   if (n >= a.N) return;
   const int64_t total = (int64_t)a.M * a.N;
-  for (int m = blockIdx.y * blockDim.y + threadIdx.y; m < a.M; m += gridDim.y * blockDim.y) {
+  for (int m = (blockIdx.y << (8 - log2_wide)) + (threadIdx.x >> log2_wide); m < a.M; m += round) {
     const float* p = a.parts + (int64_t)m * a.N + n;
     float s[VEC] = {};
 #pragma unroll 4
@@ -382,12 +382,12 @@ int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
 int launch_reduce(const char* op, const GemmArgs& a, int slices) {
   const bool vec = a.N % 4 == 0;
   const int64_t columns = vec ? a.N / 4 : a.N;
-  unsigned wide = 256;
-  while (wide > 4 && wide / 2 >= columns) wide /= 2;
-  const dim3 block(wide, 256 / wide);
-  const dim3 grid((unsigned)dh::ceil_div(columns, wide), (unsigned)std::min<int64_t>(dh::ceil_div(a.M, block.y), 65535));
-  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, block, 0, dh::stream(), a, slices);
-  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, block, 0, dh::stream(), a, slices);
+  int log2_wide = 8;
+  while (log2_wide > 2 && 1 << (log2_wide - 1) >= columns) log2_wide--;
+  const int rows = 256 >> log2_wide;
+  const dim3 grid((unsigned)dh::ceil_div(columns, 1 << log2_wide), (unsigned)std::min<int64_t>(dh::ceil_div(a.M, rows), 65535));
+  if (vec) hipLaunchKernelGGL(gemm_reduce_kernel<4>, grid, dim3(256), 0, dh::stream(), a, slices, log2_wide, rows * (int)grid.y);
+  else hipLaunchKernelGGL(gemm_reduce_kernel<1>, grid, dim3(256), 0, dh::stream(), a, slices, log2_wide, rows * (int)grid.y);
   DH_CHECK_LAUNCH(op);
   return 0;
 }

@@ -152,6 +152,7 @@ SIGNATURES = {
     "dh_attn_spec_kv_write": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _P, _I, _I]),
     "dh_attn_spec_prefill": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _P, _P, _I, _I, _I, _I]),
     "dh_attn_spec_prefill_shared": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _P, _I, _I, _P, _P, _I, _I, _I, _I]),
+    "dh_attn_spec_prefill_plan": (_I, [ctypes.POINTER(AttnSpec), _I, _I, _I, _I]),
     "dh_latent_rows": (_I, [ctypes.POINTER(Latent), _P, _P, _I, _I]),
     "dh_latent_prefill_workspace_bytes": (_SZ, [ctypes.POINTER(Latent), _I, _I]),
     "dh_latent_prefill": (_I, [ctypes.POINTER(Latent), _P, _P, _P, _P, _I, _I, _I, _I]),

@@ -650,6 +650,29 @@ int launch_spec(const char* op, const PrefillArgs& a) {
   DH_CHECK_LAUNCH(op);
   return 0;
 }
+
+// Prompts over f32 caches: attn_prefill_f32_kernel, or the general kernel where that is the faster of the two, which few queries over few
+// key-value heads are (a workgroup of it is one query and up to eight heads of a key-value head, so its time goes with the heads at
+// once; a workgroup here is 16 queries of one head).  Both take a start and a time for each key the last query sees, in us: the general
+// kernel's by lanes a key (heads of at most 64 elements, of 128) and heads at once, and by how many workgroups a compute unit has; this
+// one's by its instance and rounds of one workgroup on every compute unit.  Fitted to 4800 calls (heads of 32 .. 128, 4 .. 64 of them,
+// 16 .. 200 queries, 16 .. 3200 keys) and checked on 1584 with windows of 16 .. 1024: the choice is 0.2 and 0.6 % behind the better of the
+// two on average, at worst 1.2 us on 4.8.  General / this, H 8/8, D 128: 16 queries 4.4 / 8.3 us, 33 behind 500 keys 18 / 25, 200 21 / 13;
+// H 16/8: 16 behind 3000 83 / 104, 100 behind 3000 209 / 104; H 32/8: 64 behind 500 38 / 27.  Fewer than 16 queries leave most of a tile
+// empty.
+bool takes_f32_tiles(const dh_attn_spec* s, int dk, int T, int start_pos) {
+  if (dk > 128 || s->VD > 128 || T < 16 || s->H > 65535) return false;
+  constexpr double general_start[2] = {5.1, 6.1};
+  constexpr double general_key[2][4] = {{0.0084, 0.0147, 0.0231, 0.0398}, {0.0190, 0.0250, 0.0402, 0.0774}};
+  constexpr double tiles_start[4] = {5.1, 6.4, 6.6, 6.8}, tiles_key[4] = {0.0141, 0.0228, 0.0239, 0.0313};
+  const double cus = dh::num_cus(), keys = std::min<int64_t>((int64_t)start_pos + T, s->window > 0 ? s->window : INT32_MAX);
+  const int G = s->H / s->Hkv, wide = dk > 64 || s->VD > 64, log2_heads = G <= 1 ? 0 : G <= 2 ? 1 : G <= 4 ? 2 : 3;
+  const double per_cu = (double)s->Hkv * dh::ceil_div(G, 1 << log2_heads) * T / cus;
+  const double general = general_start[wide] + keys * general_key[wide][log2_heads] * (per_cu <= 1.0 ? 1.0 : per_cu <= 2.0 ? 1.29 : 0.82 * per_cu);
+  const int instance = 2 * (dk > 64) + (s->VD > 64);
+  const int64_t rounds = dh::ceil_div(dh::ceil_div(T, 16) * s->H, dh::num_cus());
+  return tiles_start[instance] + keys * tiles_key[instance] * rounds <= general;
+}
 }  // namespace
 
 extern "C" int dh_attn_spec_prefill(const dh_attn_spec* spec, const float* d_qkv, const void* d_cache_k, const void* d_cache_v,
@@ -676,11 +699,8 @@ extern "C" int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float
     return dh::fail(1, "[%s] shared key rows must be 16-byte aligned and ld_shared=%d a multiple of 8 that holds %d elements", op, ld_shared, shared_dim);
   if (spec->ld_qkv < spec->H * dk) return dh::fail(1, "[%s] a projection row of %d floats does not hold its queries", op, spec->ld_qkv);
   const dh::SharedKey shared{d_shared_k, shared_dim, ld_shared};
-  // fewer than 16 queries leave most of a 32-bit tile empty (5 at 100: 7.8 us by the general kernel, 9.2; 16 at 4000: 67 and 66)
   const bool wide_cache = spec->cache_dtype != DH_F16;
-  if (wide_cache ? dk > 128 || T < 16 || spec->H > 65535 : dk > 256 || ld_shared >= 1 << 24)
-    return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);
-  if (spec->VD > 128)
+  if (wide_cache ? !takes_f32_tiles(spec, dk, T, start_pos) : dk > 256 || spec->VD > 128 || ld_shared >= 1 << 24)
     return dh::attn_spec_prefill_general(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, out_dtype, ld_out, T, start_pos, shared);
   PrefillArgs a{};
   a.Q = d_qkv; a.K = static_cast<const __half*>(d_cache_k); a.V = static_cast<const __half*>(d_cache_v);
@@ -704,4 +724,19 @@ extern "C" int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float
   if (dk <= 64) return spec->VD <= 64 ? launch_spec<64, 64>(op, a) : launch_spec<64, 128>(op, a);
   if (dk <= 128) return spec->VD <= 64 ? launch_spec<128, 64>(op, a) : launch_spec<128, 128>(op, a);
   return dk <= 192 ? launch_spec<192, 128>(op, a) : launch_spec<256, 128>(op, a);
+}
+
+extern "C" int dh_attn_spec_prefill_plan(const dh_attn_spec* spec, int shared_dim, int T, int start_pos, int num_cus) {
+  const char* op = "dh_attn_spec_prefill_plan";
+  if (dh::attn_spec_check(op, spec)) return -1;
+  if (T <= 0 || start_pos < 0 || shared_dim < 0) {
+    dh::fail(1, "[%s] seqLen must be positive, startPos and the shared elements non-negative", op);
+    return -1;
+  }
+  const int dk = spec->D + shared_dim;
+  if (spec->cache_dtype == DH_F16) return dk <= 256 && spec->VD <= 128 ? 1 : 0;
+  dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
+  const bool tiles = takes_f32_tiles(spec, dk, T, start_pos);
+  dh::plan_end();
+  return tiles ? 1 : 0;
 }

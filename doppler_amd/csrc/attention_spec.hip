@@ -1,6 +1,6 @@
 // Attention with a logarithmic distance bias, a sliding window, normed values, an output gate and key and value heads
 // of different sizes (dh_attn_spec): decode steps, and prefill for what the matrix-core kernels
-// (attention_prefill.hip) do not serve (heads of more than 128 elements, f32 caches with fewer than 16 queries).
+// (attention_prefill.hip) do not serve (heads of more than 128 elements, f32 caches with few queries).
 //
 // attn_spec_kernel: grid = (kv head x query-head group, key split, query token), four waves.  Keys advance in chunks;
 // every wave takes its own keys of a chunk and keeps its own online-softmax state, so the loop has no barrier.

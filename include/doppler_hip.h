@@ -445,7 +445,8 @@ typedef struct dh_attn_spec {
 int dh_attn_spec_kv_write(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, int T,
                           int start_pos);
 /* T queries at positions start_pos .. against the cache rows up to their own (already written).  Output rows of H * VD
- * elements, ld_out apart, f32 or bf16.  f16 caches with D, VD <= 128 run on the matrix cores. */
+ * elements, ld_out apart, f32 or bf16.  f16 caches with keys of at most 256 and values of at most 128 elements run on the matrix cores;
+ * f32 caches with both at most 128 where that is faster. */
 int dh_attn_spec_prefill(const dh_attn_spec* spec, const float* d_qkv, const void* d_cache_k, const void* d_cache_v,
                          void* d_out, int out_dtype, int ld_out, int T, int start_pos);
 /* One step from its raw projection row: key and value are appended at row `pos`, the token attends to its window;
@@ -460,6 +461,9 @@ int dh_attn_spec_decode(const dh_attn_spec* spec, const float* d_qkv, void* d_ca
 int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float* d_qkv, const void* d_cache_k, const void* d_shared_k,
                                 int shared_dim, int ld_shared, const void* d_cache_v, void* d_out, int out_dtype, int ld_out,
                                 int T, int start_pos);
+/* 1 where the call (with `shared_dim` shared key elements) runs on the matrix cores, 0 where the general kernel serves it, -1 for a spec
+ * that is refused.  For tests that have to reach both; needs no device (num_cus <= 0: the initialised device's, or 256). */
+int dh_attn_spec_prefill_plan(const dh_attn_spec* spec, int shared_dim, int T, int start_pos, int num_cus);
 
 /* ---- attention over a low-rank latent ----
  *   k_h = [W_uk,h c | k_rot],  v_h = W_uv,h c,  softmax over 0 <= i - j < window of scale * (q_h . k_h)

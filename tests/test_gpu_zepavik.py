@@ -507,6 +507,24 @@ def test_attention_f32_tiles(L, H, G, d, e, window, start, T):
     assert max(rel(x, y) for x, y in zip(a.run(portions, "bf16")[start:, :, :e], want)) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("start,T", [(0, 31), (3, 17), (30, 33), (1, 257), (40, 130), (700, 40)])
+@pytest.mark.parametrize("H,G,d,e,window", [(16, 2, 64, 64, 0), (5, 1, 72, 40, 33), (8, 1, 128, 128, 0), (7, 1, 24, 104, 100)])
+def test_attention_f32_tiles_of_many_heads(L, H, G, d, e, window, start, T):
+    """The same where the tiles serve the call whatever its length: five and more heads to a key-value head."""
+    a = Attn(L, H, G, d, e, window, "f32", n=start + T, seed=T)
+    assert L.dh_attn_spec_prefill_plan(ctypes.byref(a.spec), 0, T, start, 256) == 1
+    test_attention_f32_tiles(L, H, G, d, e, window, start, T)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("H,G,d,e,window,at", [(8, 1, 64, 64, 0, 37), (5, 1, 128, 104, 40, 50), (16, 2, 64, 128, 33, 95), (7, 1, 120, 24, 20, 64),
+                                                   (8, 1, 64, 64, 70, 0), (16, 2, 64, 64, 0, 149)])
+def test_a_non_finite_value_in_a_tile_stays_with_the_queries_that_see_it(L, H, G, d, e, window, at, bad):
+    a = Attn(L, H, G, d, e, window, "f32", n=150, seed=at)
+    assert L.dh_attn_spec_prefill_plan(ctypes.byref(a.spec), 0, 150, 0, 256) == 1
+    test_a_non_finite_value_stays_with_the_queries_that_see_it(L, H, G, d, e, window, at, bad)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
 @pytest.mark.parametrize("H,G,d,e,window,at", [(2, 2, 64, 64, 0, 37), (2, 1, 128, 104, 40, 50), (1, 1, 64, 128, 33, 95), (2, 1, 120, 24, 1, 64),
                                                    (1, 1, 64, 64, 70, 0), (1, 1, 64, 64, 0, 149)])

@@ -313,3 +313,14 @@ def test_the_product_tests_reach_every_tile():
             n = -(-N // 128) * 128 if two else N
             t = test_gpu_zepavik.tile_of(L, M, n, K64, capi.BF16, two, NCU)
             assert (two, t[:2], t[2] > 1) in dense, (M, n, K64, two, t)
+
+
+@pytest.mark.parametrize("H,G,d,e,window,start,T,tiles", [
+    (8, 8, 128, 128, 0, 0, 16, 0), (8, 8, 128, 128, 0, 500, 33, 0), (8, 8, 128, 128, 0, 3000, 64, 0), (8, 8, 128, 128, 0, 0, 200, 1),
+    (16, 8, 128, 128, 0, 3000, 16, 0), (16, 8, 128, 128, 0, 3000, 100, 1), (16, 8, 128, 128, 512, 3000, 16, 0), (32, 8, 128, 128, 0, 500, 64, 1),
+    (4, 4, 64, 64, 0, 0, 64, 0), (16, 8, 64, 64, 0, 0, 301, 1), (16, 8, 64, 64, 0, 0, 15, 0), (8, 1, 64, 64, 0, 400, 16, 1)])
+def test_prompts_over_f32_caches_take_the_kernel_measured_faster(H, G, d, e, window, start, T, tiles):
+    import ctypes
+    ld = H * d + G * (d + e)
+    spec = capi.AttnSpec(H, G, d, e, e, window, capi.F32, 0, H * d, H * d + G * d, -1, ld, d ** -0.5, 1e-6, None, None)
+    assert capi.load().dh_attn_spec_prefill_plan(ctypes.byref(spec), 0, T, start, NCU) == tiles

@@ -312,13 +312,15 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
   }
 }
 
-// Tiles of the 16-bit products, and what a k step (64 elements) of one costs in ns: `alone` with few workgroups on the device, `one`
-// with one on every compute unit, `full` with as many as fit (the two larger tiles: one, which takes more than half of the LDS).  The
-// device slows its clock under matrix-core load, so a step gets dearer as more compute units join, and idle ones are not all
-// lost.  Fitted to M = 17 .. 2048, N = 1024 .. 18464, K = 1024 .. 16384 with each tile and 1 .. 8 slices: the choice is within
-// 10 % of the best of them at nearly all.  (full of the smallest: 365 ns at 512 rows, 520 at 2048.)  Against the 128 x 128 and 64 x 64 tiles through registers that were here before:
-// 2048 x 18464 x 4096 391 -> 300 us, 2048 x 4096 x 16384 312 -> 253, 1531 x 2048 x 6144 75 -> 45, 512 x 4096 x 4096 38 -> 29,
-// 40 x 4096 x 16384 101 -> 34 (slices), 40 x 5120 x 1024 11.2 -> 7.1, 700 x 1024 x 1024 9.2 -> 7.3 (64 x 64 tiles).
+// Tiles of the 16-bit products, and what they cost in ns: a k step (64 elements) `alone` with few workgroups on the device, `one` with one
+// on every compute unit, `full` with as many as fit (the two larger tiles: one, which takes more than half of the LDS); outside the k
+// loop `start`, and `again` for every further round of workgroups.  The device slows its clock under matrix-core load, so a step gets
+// dearer as more compute units join, and idle ones are not all lost.  Fitted to 446 products (M 2 .. 2048, N 16 .. 32000, K 64 .. 16384) with each
+// tile and up to 16 slices, weights from HBM as a model's layers in turn have them (a step waits for those: 2048 x 1152 x 6912 on
+// 128 x 128 tiles takes 46 us with weights from the cache, 68 from HBM): the choice is 0.7 % behind the best on average, 20 % at worst.
+// Against the 128 x 128 and 64 x 64 tiles through registers that were here before, us: 2048 x 18464 x 4096
+// 421 -> 306, 2048 x 4096 x 16384 329 -> 261, 1531 x 2048 x 6144 70 -> 63, 300 x 2048 x 2048 18.4 -> 11.3, 33 x 5120 x 1024 14.6 -> 7.2,
+// 700 x 1024 x 1024 14.1 -> 7.4; behind them still: 33 x 4096 x 16384 30.6 -> 33.1 (2 rows 28.5 -> 32.7) and few rows at K 64.
 using Tile256x256 = dh::WideTile<2, 4, 2, 1>;
 using Tile256x128 = dh::WideTile<4, 2, 1, 1>;
 using Tile128x128 = dh::WideTile<2, 2, 1, 1>;
@@ -326,32 +328,42 @@ using Tile64x64 = dh::SmallTile<2, 2, 1>;
 using Tile64x128 = dh::SmallTile<2, 2, 2>;     // gate and up columns
 struct TileCost {
   int bm, bn, per_cu;
-  float alone, one, full, start;      // start: ns outside the k loop
+  float alone, one, full, start, again;
 };
-constexpr TileCost kTiles[] = {{256, 256, 1, 900.f, 1720.f, 1720.f, 8000.f},
-                               {256, 128, 1, 520.f, 930.f, 930.f, 5500.f},
-                               {128, 128, 2, 330.f, 480.f, 1080.f, 4500.f},
-                               {64, 64, 2, 210.f, 250.f, 450.f, 3700.f}};
-constexpr TileCost kSmallGlu = {64, 128, 1, 260.f, 330.f, 330.f, 3700.f};
+constexpr TileCost kTiles[] = {{256, 256, 1, 1075.f, 1590.f, 1840.f, 9300.f, 5300.f},
+                               {256, 128, 1, 610.f, 825.f, 825.f, 12300.f, 6000.f},
+                               {128, 128, 2, 360.f, 645.f, 1415.f, 5000.f, 3100.f},
+                               {64, 64, 2, 232.f, 294.f, 516.f, 4100.f, 1400.f}};
+// gate and up products, never sliced
+constexpr TileCost kGluTiles[] = {{256, 256, 1, 900.f, 1720.f, 1720.f, 8000.f, 0.f},
+                                  {256, 128, 1, 520.f, 930.f, 930.f, 5500.f, 0.f},
+                                  {128, 128, 2, 330.f, 480.f, 1080.f, 4500.f, 0.f},
+                                  {64, 128, 1, 260.f, 330.f, 330.f, 3700.f, 0.f}};
 constexpr int kMaxSlices = 16, kMinSliceSteps = 8;
 
 struct TileChoice {
   int tile, slices;
 };
-// The cheapest tile and number of k slices.  Slices cost the round trip of their raw sums and a second launch.
-TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool glu) {
+// The cheapest tile and number of k slices.  Slices cost the round trip of their raw sums (about 4 TB/s) and a second launch, and no
+// number of them is faster than the weights come in.
+// erf: a second output through the exact gelu, whose epilogue takes a compute unit about 60 ns for each element a lane holds of a wave, 40
+// where another workgroup's loop runs beside it (1531 x 6144 x 2048 without it 52 us on 128 x 128 tiles, 47 on 256 x 256; with it 76 and
+// 111); behind slices it is the reduce launch's.
+TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool glu, bool erf) {
   const int64_t cus = dh::num_cus(), steps = K / 64;
   TileChoice best{0, 1};
   double least = 1e30;
   for (int i = 0; i < 4; i++) {
-    const TileCost& c = glu && i == 3 ? kSmallGlu : kTiles[i];
+    const TileCost& c = glu ? kGluTiles[i] : kTiles[i];
     for (int s = 1; s <= most_slices && (s == 1 || steps / s >= kMinSliceSteps); s++) {
       const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s, slots = cus * c.per_cu, left = groups % slots;
       const double f = (double)left / cus;
-      const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (0.7 + 0.3 * f / c.per_cu);
-      const double per_group = (double)dh::ceil_div(steps, s);
-      double t = per_group * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + c.start;
-      if (s > 1) t += 3500.0 + 4.0 * M * N * (2 * s + 1) / 4000.0;      // a launch, and 4 bytes a sum at about 4 TB/s
+      const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (0.76 + 0.24 * f / c.per_cu);
+      const int64_t rounds = groups / slots + (left ? 1 : 0);
+      const double loop = dh::ceil_div(steps, s) * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + (double)(rounds - 1) * c.again;
+      double t = std::max(loop, 2.0 * N * K / 6450.0) + c.start;
+      if (s > 1) t += 2250.0 + 4.0 * M * N * (2 * s + 1) / 4150.0;
+      else if (erf) t += (c.per_cu == 1 ? 60.0 : 40.0) * (c.bm * c.bn / 64) * dh::ceil_div(groups, cus);
       if (t < least) {
         least = t;
         best = TileChoice{i, s};
@@ -427,9 +439,9 @@ int slices_in_workspace(int64_t M, int64_t N, int most) {
   (void)dh::splitk_workspace(&ws_bytes);
   return (int)std::max<size_t>(1, std::min<size_t>(most, ws_bytes / ((size_t)M * N * sizeof(float))));
 }
-TileChoice choose_16bit(int64_t M, int64_t N, int64_t K) {
+TileChoice choose_16bit(int64_t M, int64_t N, int64_t K, bool erf) {
   const int most = slices_in_workspace(M, N, kMaxSlices);
-  TileChoice pick = choose_tile(M, N, K, most, false);
+  TileChoice pick = choose_tile(M, N, K, most, false, erf);
   const int env_tile = dh::tuning_int("DH_DENSE_TILE", -1), env_slices = dh::tuning_int("DH_DENSE_SLICES", 0);
   if (env_tile >= 0) pick.tile = env_tile;
   if (env_slices) pick.slices = std::min(most, env_slices);
@@ -464,11 +476,11 @@ int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
     const int rc = dense_16bit(op, low, f16);
     return rc ? rc : dense_16bit(op, high, f16);
   }
-  return launch_act(op, a, f16, choose_16bit(a.M, a.N, a.K));
+  return launch_act(op, a, f16, choose_16bit(a.M, a.N, a.K, a.n_first < a.N && a.act == DH_ACT_GELU_ERF));
 }
 
 // k slices of a 32-bit product.  Workgroups on a compute unit share its matrix cores, so the one with the most of them ends last: 64 k of a
-// tile take 1.35 us alone there and 1.1 us each in company (0.85 at the full rate).  Slices cost as in choose_tile.
+// tile take 1.35 us alone there and 1.1 us each in company (0.85 at the full rate).  Slices cost a launch and 4 bytes a sum at 4 TB/s.
 int choose_f32_slices(int64_t M, int64_t N, int64_t K) {
   const int64_t steps = K / 64, tiles = dh::ceil_div(M, 64) * dh::ceil_div(N, 64);
   const int most = slices_in_workspace(M, N, 16), env_slices = dh::tuning_int("DH_F32_SLICES", 0);
@@ -517,7 +529,7 @@ int launch_experts(const char* op, GemmArgs a, int a_dtype) {
     if (a.rows.tile_rows == Tile128x128::BM) return launch_16bit_kernel<Tile128x128, false, kNoSecond, true, GLU>(op, a, 1);
     return launch_16bit_kernel<std::conditional_t<GLU, Tile64x128, Tile64x64>, false, kNoSecond, true, GLU>(op, a, 1);
   } else {
-    return launch_16bit<false, kNoSecond, GLU>(op, a, choose_tile(a.M, a.N, a.K, 1, true));
+    return launch_16bit<false, kNoSecond, GLU>(op, a, choose_tile(a.M, a.N, a.K, 1, true, false));
   }
 }
 
@@ -584,14 +596,14 @@ extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, con
   return dense_16bit(op, a, a_dtype == DH_F16);
 }
 
-extern "C" int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int glu, int num_cus, int64_t* out3) {
+extern "C" int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int form, int num_cus, int64_t* out3) {
   const char* op = "dh_dense_matmul_layout";
   if (!out3 || M <= 0 || N <= 0 || K <= 0 || K % 64) return dh::fail(1, "[%s] M=%d, N=%d, K=%d (a multiple of 64), or no place for the result", op, M, N, K);
   dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
-  const bool wide = a_dtype == DH_F32;
-  const TileChoice pick = wide ? TileChoice{0, glu ? 1 : choose_f32_slices(M, N, K)} : glu ? choose_tile(M, N, K, 1, true) : choose_16bit(M, N, K);
+  const bool wide = a_dtype == DH_F32, glu = form == 1;
+  const TileChoice pick = wide ? TileChoice{0, glu ? 1 : choose_f32_slices(M, N, K)} : glu ? choose_tile(M, N, K, 1, true, false) : choose_16bit(M, N, K, form == 2);
   dh::plan_end();
-  const TileCost& c = glu && pick.tile == 3 ? kSmallGlu : kTiles[pick.tile];
+  const TileCost& c = glu ? kGluTiles[pick.tile] : kTiles[pick.tile];
   out3[0] = wide ? 64 : c.bm;
   out3[1] = wide ? (glu ? 128 : 64) : c.bn;
   out3[2] = dh::ceil_div(K, slice_extent(K, pick.slices));

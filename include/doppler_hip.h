@@ -384,9 +384,10 @@ int dh_dense_matmul(const void* d_A, int a_dtype, int lda, const void* d_W, int 
 int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K, float alpha,
                            const float* d_bias, const float* d_col_scale, const float* d_residual, float* d_C, int ldc,
                            int n_first, void* d_C2, int c2_dtype, int ldc2, int activation);
-/* The tile dh_dense_matmul would take for activations of a_dtype (glu = 1: the shared expert's gate and up product of dh_experts_prefill):
- * out3 = { rows, columns, slices k is cut into }.  For tests that have to reach every tile; needs no device. */
-int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int glu, int num_cus, int64_t* out3);
+/* The tile dh_dense_matmul would take for activations of a_dtype (form 1: the shared expert's gate and up product of dh_experts_prefill;
+ * 2: with a second output through DH_ACT_GELU_ERF): out3 = { rows, columns, slices k is cut into }.  For tests that have to reach every
+ * tile; needs no device. */
+int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int form, int num_cus, int64_t* out3);
 
 /* The same product for ONE f32 activation row (decode; HBM-bound), d_C2 in f32, with an optional RMSNorm of the
  * row in its prologue: x * rsqrt(mean of the first `hidden` elements squared + eps) * w.  d_x and d_norm_weight

@@ -163,30 +163,44 @@ def test_dense_matmul_large_tiles(L, M, N, K, first, dtype):
 
 # every tile of the 16-bit products, whole and in k slices (with a short last one), k steps of either parity, ragged in both directions; the
 # tile and the slices are those of 256 compute units
-TILES = [(129, 130, 192, (64, 64, 1)), (2, 33, 1664, (64, 64, 3)), (1928, 1074, 640, (128, 128, 1)), (1073, 1932, 704, (128, 128, 1)),
-         (645, 457, 4608, (128, 128, 6)), (649, 486, 4864, (128, 128, 7)), (1299, 3078, 640, (256, 128, 1)), (1299, 3078, 704, (256, 128, 1)),
+TILES = [(129, 130, 192, (64, 64, 1)), (2, 33, 1664, (64, 64, 3)), (195, 9798, 640, (128, 128, 1)), (148, 11027, 704, (128, 128, 1)),
+         (67, 4706, 4096, (128, 128, 6)), (1274, 65, 11776, (128, 128, 16)), (1412, 2912, 896, (256, 128, 1)), (1540, 4090, 2112, (256, 128, 1)),
          (1165, 1684, 9664, (256, 128, 3)), (2720, 4759, 1152, (256, 256, 1)), (2060, 6150, 1600, (256, 256, 1)), (129, 11422, 14144, (256, 256, 5))]
+# with a second output through the exact gelu, whose epilogue counts
+ERF_TILES = [(129, 130, 192, (64, 64, 1)), (2, 33, 1664, (64, 64, 3)), (330, 5525, 768, (128, 128, 1)), (67, 4706, 4096, (128, 128, 6)),
+             (1224, 4121, 2176, (256, 128, 1)), (1165, 1684, 9664, (256, 128, 3)), (2441, 5063, 1216, (256, 256, 1)), (129, 11422, 14144, (256, 256, 5))]
 # gate and up products of a shared expert (32 gate rows, 32 up rows, ..)
 GLU_TILES = [(300, 256, 704, (64, 128, 1)), (1234, 1664, 704, (128, 128, 1)), (1928, 2176, 640, (256, 128, 1)), (2224, 5632, 1344, (256, 256, 1))]
 
 
-def tile_of(L, M, N, K, code, glu=False, num_cus=0):
+def tile_of(L, M, N, K, code, glu=False, num_cus=0, erf=False):
     out = (ctypes.c_int64 * 3)()
-    capi.check(L.dh_dense_matmul_layout(M, N, K, code, int(glu), num_cus, out))
+    capi.check(L.dh_dense_matmul_layout(M, N, K, code, 2 if erf else int(glu), num_cus, out))
     return tuple(out)
 
 
 @pytest.mark.parametrize("M,N,K,tile", TILES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_dense_matmul_every_tile(L, M, N, K, tile, dtype):
+    assert tile_of(L, M, N, K, capi.BF16 if dtype == torch.bfloat16 else capi.F16) == tile
+    check_forms(L, M, N, K, dtype, ((N, capi.ACT_NONE, None), (N // 3, capi.ACT_NONE, lambda z: z),
+                                    (N // 3, capi.ACT_RELU2, lambda z: z.clamp(min=0).square())))
+
+
+@pytest.mark.parametrize("M,N,K,tile", ERF_TILES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_matmul_gelu_on_every_tile(L, M, N, K, tile, dtype):
+    assert tile_of(L, M, N, K, capi.BF16 if dtype == torch.bfloat16 else capi.F16, erf=True) == tile
+    check_forms(L, M, N, K, dtype, ((N // 3, capi.ACT_GELU_ERF, lambda z: 0.5 * z * (1 + torch.erf(z * 0.5 ** 0.5))),))
+
+
+def check_forms(L, M, N, K, dtype, forms):
     code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
-    assert tile_of(L, M, N, K, code) == tile
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     A = torch.randn(M, K, generator=g, device="cuda").to(dtype)
     W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(dtype)
     acc = A.double() @ W.double().T
-    for first, act, fn in ((N, capi.ACT_NONE, None), (N // 3, capi.ACT_NONE, lambda z: z), (N // 3, capi.ACT_RELU2, lambda z: z.clamp(min=0).square()),
-                           (N // 3, capi.ACT_GELU_ERF, lambda z: 0.5 * z * (1 + torch.erf(z * 0.5 ** 0.5)))):
+    for first, act, fn in forms:
         C, C2 = torch.full((M, first + 3), 9.0, device="cuda"), torch.full((M, N - first + 2), 9.0, dtype=dtype, device="cuda")
         torch.cuda.synchronize()
         capi.check(L.dh_dense_matmul(A.data_ptr(), code, K, W.data_ptr(), K, M, N, K, 1.0, None, None, C.data_ptr(), first + 3, first,

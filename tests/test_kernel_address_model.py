@@ -304,6 +304,9 @@ def test_the_product_tests_reach_every_tile():
         for M, N, K, tile in cases:
             assert test_gpu_zepavik.tile_of(L, M, N, K, capi.BF16, glu, NCU) == tile, (M, N, K, glu)
     wide = {(pair, tile[:3], tile[3] > 1) for *_, pair, _, tile in test_gpu_ops.WIDE_PRODUCTS}
+    for M, N, K, tile in test_gpu_zepavik.ERF_TILES:
+        assert test_gpu_zepavik.tile_of(L, M, N, K, capi.BF16, False, NCU, erf=True) == tile, (M, N, K)
+    erf = {(tile[:2], tile[2] > 1) for *_, tile in test_gpu_zepavik.ERF_TILES}
     dense = {(glu, tile[:2], tile[2] > 1) for glu, cases in ((False, test_gpu_zepavik.TILES), (True, test_gpu_zepavik.GLU_TILES)) for *_, tile in cases}
     for M, N, K in np.exp2(rng.uniform((4, 6, 6), (11.5, 14, 14.2), (20000, 3))).astype(int).tolist():
         K64 = -(-K // 64) * 64
@@ -313,6 +316,8 @@ def test_the_product_tests_reach_every_tile():
             n = -(-N // 128) * 128 if two else N
             t = test_gpu_zepavik.tile_of(L, M, n, K64, capi.BF16, two, NCU)
             assert (two, t[:2], t[2] > 1) in dense, (M, n, K64, two, t)
+        t = test_gpu_zepavik.tile_of(L, M, N, K64, capi.BF16, False, NCU, erf=True)
+        assert (t[:2], t[2] > 1) in erf, (M, N, K64, t)
 
 
 @pytest.mark.parametrize("H,G,d,e,window,start,T,tiles", [

@@ -918,9 +918,12 @@ int launch_wide_best(GemmArgs a, const char* op) {
 
 // Products of enough work, or of enough tiles, go to q4k_wide_kernel: where a step's latency counts instead of its throughput the other
 // kernel is ahead, because its waves share one dequantised tile (us, that one / the wide one: 1300 x 513 x 1100 21 / 28, 512 x 1152 x 6912
-// 34 / 38, 64 x 4096 x 4096 25 / 27, but 1024 x 2048 x 1024 38 / 27, 200 x 6144 x 4096 43 / 39, 512 x 4096 x 12288 164 / 87).
+// 34 / 38, 64 x 4096 x 4096 25 / 27, but 1024 x 2048 x 1024 38 / 27, 200 x 6144 x 4096 43 / 39, 512 x 4096 x 12288 164 / 87).  Pairs of
+// few steps stay there at any height (2048 x 1024 x 512 18 / 21, 1024 x 2048 x 1024 22 / 24), and up to 64 rows as long as its 64-row tiles
+// are resident at once (64 x 12288 x 4096 44 / 50, 48 x 16000 x 4096 44 / 51, but 64 x 20000 x 4096 80 / 62).
 bool takes_wide(int64_t M, int64_t N, int64_t K, bool dual) {
-  return dh::ceil_div(M, 256) * dh::ceil_div(N, 128) >= dh::num_cus() || (double)M * N * K * (dual ? 2 : 1) >= (M >= 1024 ? 2e9 : 5e9);
+  if (dual && M <= 64 && dh::ceil_div(N, 64) <= dh::num_cus()) return false;
+  return dh::ceil_div(M, 256) * dh::ceil_div(N, 128) >= dh::num_cus() || (double)M * N * K * (dual ? 2 : 1) >= (M >= 1024 && !dual ? 2e9 : 5e9);
 }
 
 // 128 x 128 tiles when they occupy at least half of the compute units (their higher matrix-core

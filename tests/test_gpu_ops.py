@@ -817,12 +817,12 @@ def test_bias_add_and_scale_bit_exact():
 # pair), rows of a wave, pieces of K.  Every tile, whole and in pieces, plain and gated; edges in M and N, K off the 64 and the 256.
 WIDE_PRODUCTS = [
     (1030, 2100, 1100, False, False, (128, 128, 64, 1)), (2050, 6150, 1088, False, True, (256, 256, 128, 1)), (1041, 4097, 2300, False, False, (128, 256, 64, 1)),
-    (600, 4100, 4032, False, False, (128, 128, 64, 1)), (513, 130, 81920, False, False, (128, 128, 64, 8)), (1100, 1030, 1024, True, False, (128, 128, 64, 1)),
-    (1025, 5000, 300, True, False, (128, 128, 64, 1)), (520, 6900, 1152, True, False, (256, 256, 128, 1)),
+    (600, 4100, 4032, False, False, (128, 128, 64, 1)), (513, 130, 81920, False, False, (128, 128, 64, 8)), (1335, 498, 3761, True, False, (128, 128, 64, 1)),
+    (284, 3297, 2670, True, False, (128, 128, 64, 1)), (520, 6900, 1152, True, False, (256, 256, 128, 1)),
     (1049, 1061, 1861, False, True, (128, 128, 64, 2)), (1829, 2215, 554, False, True, (128, 256, 64, 1)), (946, 1350, 4612, False, False, (128, 256, 64, 5)),
     (1582, 2529, 2601, False, False, (128, 256, 128, 1)), (1255, 1583, 7763, False, True, (128, 256, 128, 3)), (1703, 4807, 523, False, False, (256, 256, 128, 1)),
-    (1538, 2528, 10169, False, False, (256, 256, 128, 2)), (1652, 1225, 511, True, False, (128, 256, 64, 1)), (1676, 1190, 2575, True, False, (128, 256, 128, 1)),
-    (1673, 2351, 548, True, False, (256, 256, 128, 1))]
+    (1538, 2528, 10169, False, False, (256, 256, 128, 2)), (525, 11517, 366, True, False, (128, 256, 64, 1)), (993, 2642, 953, True, False, (128, 256, 64, 1)), (1676, 1190, 2575, True, False, (128, 256, 128, 1)),
+    (1207, 3570, 582, True, False, (256, 256, 128, 1))]
 
 
 def wide_tile(M, N, K, pair, num_cus=0):

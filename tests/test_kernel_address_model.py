@@ -329,3 +329,10 @@ def test_prompts_over_f32_caches_take_the_kernel_measured_faster(H, G, d, e, win
     ld = H * d + G * (d + e)
     spec = capi.AttnSpec(H, G, d, e, e, window, capi.F32, 0, H * d, H * d + G * d, -1, ld, d ** -0.5, 1e-6, None, None)
     assert capi.load().dh_attn_spec_prefill_plan(ctypes.byref(spec), 0, T, start, NCU) == tiles
+
+
+@pytest.mark.parametrize("M,inter,hidden,wide", [(2048, 1024, 512, 0), (1024, 2048, 1024, 0), (64, 12288, 4096, 0), (48, 16000, 4096, 0), (64, 20000, 4096, 1),
+                                                  (65, 12288, 4096, 1), (200, 6144, 2048, 1), (2048, 12288, 4096, 1)])
+def test_gated_pairs_take_the_kernel_measured_faster(M, inter, hidden, wide):
+    import ctypes
+    assert capi.load().dh_q4k_gemm_layout(M, inter, hidden, 1, NCU, (ctypes.c_int64 * 4)()) == wide

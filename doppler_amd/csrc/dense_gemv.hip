@@ -214,23 +214,41 @@ int launch(const char* op, GemvArgs a, int max_grid, int* parts) {
 template <int WAVES, bool ARGMAX, bool HEADS>
 int launch_loads(const char* op, const GemvArgs& a, int max_grid, int* parts) {
   // a stage as long as the row: lanes past the end load nothing and multiply zeros (a row of 1024 in a stage of 4096 leaves a quarter
-  // of the bytes in flight).  Four waves a workgroup are few, so long rows get long stages there.
+  // of the bytes in flight).  Four waves a workgroup are few, so long rows get long stages there, and gated heads where a row is all a wave
+  // has (2048 x 4096 7.5 -> 7.1 us) or very long (4096 x 8192 19.3 -> 16.9); two stages of 1536 fit rows up to 3072 better than two of
+  // 2048 (2560 x 2560 5.9 -> 5.5).
   if (a.K <= 1024) return launch<2, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
-  if (WAVES > 4 || a.K <= 2048) return launch<4, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
-  return launch<8, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if (a.K <= 2048) return launch<4, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if constexpr (WAVES == 4) return launch<8, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if constexpr (HEADS) {
+    if (WAVES == 8 ? a.N <= 8 * dh::num_cus() : a.K > 4096) return launch<8, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  } else {
+    if (a.K <= 3072) return launch<3, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  }
+  return launch<4, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+}
+
+// Rows of each of its workgroups that the busiest compute unit goes through, with at most `per_cu` workgroups on every one.
+int64_t busiest(int64_t N, int waves, int per_cu) {
+  const int64_t cus = dh::num_cus(), groups = dh::ceil_div(N, waves), iters = dh::ceil_div(groups, per_cu * cus);
+  return dh::ceil_div(dh::ceil_div(groups, iters), cus) * iters;
 }
 
 // Every workgroup prepares the whole activation row, so workgroups are as wide as leaves one for every compute unit, and as many
-// as are resident at once.  us, N x K with four waves and stages of 4096 (or two rows of 2048) -> now, weights from memory: 10256 x
-// 2048 11.9 -> 10.8, 5136 x 1024 6.5 -> 5.3, 18464 x 4096 31.0 -> 27.8 (5.4 TB/s), 2048 x 8192 10.1 -> 9.2, 6144 x 2048 9.1 -> 7.9; heads 32000 x
-// 2048 28.5 -> 26.8, 32000 x 1024 19.2 -> 17.4.  A launch alone is about 4 of them.
+// as are resident at once; of rows beyond 2048 two to a compute unit, or four where that spreads them better (5136 rows are 642 groups:
+// two rounds of 321, or one of 642; x 2560 8.9 -> 6.9 us, x 8192 17.4 -> 16.7).  us, N x K with four waves and stages of 4096 (or two rows of 2048) -> now,
+// weights from memory: 10256 x 2048 11.9 -> 10.8, 5136 x 1024 6.5 -> 5.3, 18464 x 4096 31.0 -> 27.8 (5.4 TB/s), 2048 x 8192 10.1 -> 9.2,
+// 6144 x 2048 9.1 -> 7.9; heads 32000 x 2048 28.5 -> 26.8, 32000 x 1024 19.2 -> 17.4.  A launch alone is about 4 of them.
 template <bool ARGMAX, bool HEADS = false>
 int dispatch(const char* op, const GemvArgs& a, int* parts) {
   const int cus = dh::num_cus();
   if (a.K > 8192) return launch<8, 8, ARGMAX, HEADS>(op, a, a.K <= 16384 ? 2 * cus : cus, parts);
   if constexpr (HEADS)          // three rows are read to prepare one
     if (a.N >= 16 * cus) return launch_loads<16, ARGMAX, HEADS>(op, a, cus, parts);
-  if (a.N >= 8 * cus) return launch_loads<8, ARGMAX, HEADS>(op, a, !HEADS && a.K <= 2048 ? 4 * cus : 2 * cus, parts);
+  if (a.N >= 8 * cus) {
+    const bool four = !HEADS && (a.K <= 2048 || busiest(a.N, 8, 4) < busiest(a.N, 8, 2));
+    return launch_loads<8, ARGMAX, HEADS>(op, a, four ? 4 * cus : 2 * cus, parts);
+  }
   return launch_loads<4, ARGMAX, HEADS>(op, a, 4 * cus, parts);
 }
 

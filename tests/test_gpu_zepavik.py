@@ -350,8 +350,8 @@ def test_dense_gemv(L, N, K, hidden, first):
         assert got2[-1] == 5.0
 
 
-@pytest.mark.parametrize("K", [960, 1024, 1088, 2048, 2112, 4160, 8192])
-@pytest.mark.parametrize("N", [5, 2047, 2049, 4101])
+@pytest.mark.parametrize("K", [960, 1024, 1088, 2048, 2112, 3072, 3136, 4160, 8192])
+@pytest.mark.parametrize("N", [5, 2047, 2048, 2049, 4101, 5136])
 def test_dense_gemv_widths(L, N, K):
     """Either side of where the stage's length and the workgroup's width change; a product of K terms of size 1 / sqrt(K) in f32 in at
     most K / 64 + 6 roundings a lane and sum: 2^-24 (K / 64 + 6) <= 8e-6 of terms below 6."""

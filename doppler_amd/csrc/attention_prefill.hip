@@ -382,28 +382,32 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_kernel(const PrefillArgs 
     }
   }
 
-  // ---- the two groups' shares of a query, through LDS
-  __syncthreads();
-  float4_t* shared_acc = reinterpret_cast<float4_t*>(smem) + wave * (QT * DT * 64) + lane;
-  float2* shared_ml = reinterpret_cast<float2*>(smem + 4 * QT * DT * 1024) + wave * (QT * 64) + lane;
-  if (grp) {
+  // ---- the two groups' shares of a query, through LDS; a single tile is group 0's alone (prompts of 64 tokens, D 128: 6.2 -> 5.7 us)
+  if (ntiles > 1) {
+    __syncthreads();
+    float4_t* shared_acc = reinterpret_cast<float4_t*>(smem) + wave * (QT * DT * 64) + lane;
+    float2* shared_ml = reinterpret_cast<float2*>(smem + 4 * QT * DT * 1024) + wave * (QT * 64) + lane;
+    if (grp) {
 #pragma unroll
-    for (int u = 0; u < QT; u++) {
+      for (int u = 0; u < QT; u++) {
 #pragma unroll
-      for (int t = 0; t < DT; t++) shared_acc[64 * (u * DT + t)] = acc[u][t];
-      shared_ml[64 * u] = make_float2(m_run[u], l_run[u]);
+        for (int t = 0; t < DT; t++) shared_acc[64 * (u * DT + t)] = acc[u][t];
+        shared_ml[64 * u] = make_float2(m_run[u], l_run[u]);
+      }
+    }
+    __syncthreads();
+    if (!grp) {
+#pragma unroll
+      for (int u = 0; u < QT; u++) {
+        const float2 ml = shared_ml[64 * u];
+        const float m = fmaxf(m_run[u], ml.x), mine = __builtin_amdgcn_exp2f(m_run[u] - m), other = __builtin_amdgcn_exp2f(ml.x - m);
+        l_run[u] = l_run[u] * mine + ml.y * other;
+#pragma unroll
+        for (int t = 0; t < DT; t++) acc[u][t] = acc[u][t] * mine + shared_acc[64 * (u * DT + t)] * other;
+      }
     }
   }
-  __syncthreads();
   if (grp) return;
-#pragma unroll
-  for (int u = 0; u < QT; u++) {
-    const float2 ml = shared_ml[64 * u];
-    const float m = fmaxf(m_run[u], ml.x), mine = __builtin_amdgcn_exp2f(m_run[u] - m), other = __builtin_amdgcn_exp2f(ml.x - m);
-    l_run[u] = l_run[u] * mine + ml.y * other;
-#pragma unroll
-    for (int t = 0; t < DT; t++) acc[u][t] = acc[u][t] * mine + shared_acc[64 * (u * DT + t)] * other;
-  }
 
   // ---- lane (q, g) holds O[my_q][16 t + 4 g + i]
 #pragma unroll

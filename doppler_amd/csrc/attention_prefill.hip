@@ -15,7 +15,7 @@
 // Measured (us; before: one group staged through registers, V transposed on the way into LDS, fragments read as they were
 // needed -> now): H 32/8, T 2048: 101 -> 61 (562 TFLOP/s); 16/8, 4096: 171 -> 96; 32/8, 8192: 1051 -> 605 (908
 // TFLOP/s); 16/8, 512: 14.5 -> 11.2.  SPEC with distance bias, H 16/4, D 128: T 2048 90 -> 44, T 4096 276 -> 129, window 512 33 -> 29; 16 heads of 128 + 64 shared, T 2048: 91 -> 51.
-// What is left at 128 queries a workgroup: 31% of the matrix cores' cycles and about as much vector work (exponentials) in turns.
+// What is left at 128 queries a workgroup: 34% of the matrix cores' cycles and about as much other vector work (exponentials) in turns.
 // Measured without gain: the groups half a tile apart (one at the products while the other is at its exponentials, two
 // barriers a tile: 61 -> 59 us, but 51 -> 62 us with shared keys); fetches spread between the products (61 -> 65 us).
 //

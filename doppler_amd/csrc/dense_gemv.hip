@@ -237,8 +237,8 @@ int64_t busiest(int64_t N, int waves, int per_cu) {
 // Every workgroup prepares the whole activation row, so workgroups are as wide as leaves one for every compute unit, and as many
 // as are resident at once; of rows beyond 2048 two to a compute unit, or four where that spreads them better (5136 rows are 642 groups:
 // two rounds of 321, or one of 642; x 2560 8.9 -> 6.9 us, x 8192 17.4 -> 16.7).  us, N x K with four waves and stages of 4096 (or two rows of 2048) -> now,
-// weights from memory: 10256 x 2048 11.9 -> 10.8, 5136 x 1024 6.5 -> 5.3, 18464 x 4096 31.0 -> 27.8 (5.4 TB/s), 2048 x 8192 10.1 -> 9.2,
-// 6144 x 2048 9.1 -> 7.9; heads 32000 x 2048 28.5 -> 26.8, 32000 x 1024 19.2 -> 17.4.  A launch alone is about 4 of them.
+// weights from memory: 10256 x 2048 10.6 -> 9.8, 5136 x 1024 5.9 -> 4.5, 18464 x 4096 28.0 -> 25.8 (5.9 TB/s), 2050 x 8192 9.8 -> 9.1; with
+// a norm 5136 x 1024 6.3 -> 5.1, 5136 x 2048 8.1 -> 7.1; heads 32000 x 2048 27.1 -> 25.6, 32000 x 1024 18.6 -> 16.9.  A launch alone is about 4 of them.
 template <bool ARGMAX, bool HEADS = false>
 int dispatch(const char* op, const GemvArgs& a, int* parts) {
   const int cus = dh::num_cus();

@@ -14,9 +14,9 @@
 // two); a wave reads its fragments of the activations, and of the weights the 16 nibble bytes a lane needs for 64 k, and
 // dequantises them in registers, between the matrix-core instructions of the slice before.  So a weight costs 0.56 bytes of LDS
 // traffic instead of two written and two read, at the price of one dequantisation for each wave along M (two): what bounds it is
-// instruction issue (154 vector instructions for 16 or 32 matrix-core ones) and, at 2048 rows, power.  One barrier per 64 k.
-// 2048 rows, against the other kernel: 6144 x 4096 190 -> 130 us, 4096 x 4096 112 -> 95, 4096 x 12288 284 -> 244, gated pair
-// 12288 x 4096 428 -> 397; 512 rows: 77 -> 57, 78 -> 43, 164 -> 87, 151 -> 120.
+// instruction issue (154 vector instructions for 16 or 32 matrix-core ones; the matrix cores are busy 60 % of the time at 2048
+// rows).  One barrier per 64 k.  Against the other kernel in tiles of its own, weights from memory, 2048 rows: 6144 x 4096 159 -> 124 us,
+// 4096 x 4096 96 -> 95, 4096 x 12288 257 -> 261, gated pair 12288 x 4096 423 -> 400; 512 rows: 64 -> 57, 58 -> 42, 149 -> 83, 152 -> 118.
 // Tried there: four activation buffers instead of two (no change: a fetch is not what a step waits for), the weights
 // dequantised to f16 in memory by a pre-pass for gemm_wide.h (the same at 2048 rows, slower below).
 //
@@ -917,8 +917,9 @@ int launch_wide_best(GemmArgs a, const char* op) {
 }
 
 // Products of enough work, or of enough tiles, go to q4k_wide_kernel: where a step's latency counts instead of its throughput the other
-// kernel is ahead, because its waves share one dequantised tile (us, that one / the wide one: 1300 x 513 x 1100 21 / 28, 512 x 1152 x 6912
-// 34 / 38, 64 x 4096 x 4096 25 / 27, but 1024 x 2048 x 1024 38 / 27, 200 x 6144 x 4096 43 / 39, 512 x 4096 x 12288 164 / 87).  Pairs of
+// kernel is ahead, because its waves share one dequantised tile (us, that one / the wide one, weights from memory: 128 x 1152 x 6912 20 / 28,
+// 512 x 1152 x 6912 33.2 / 33.2, 64 x 4096 x 4096 23.5 / 24.7, but 1024 x 2048 x 1024 25.3 / 24.3, 200 x 6144 x 4096 39.5 / 37.3, 512 x 4096 x 12288
+// 142 / 82; a threshold of the product's size, as the costs of the other kernel are not in the table: over 236 shapes 1.5 % behind the best).  Pairs of
 // few steps stay there at any height (2048 x 1024 x 512 18 / 21, 1024 x 2048 x 1024 22 / 24), and up to 64 rows as long as its 64-row tiles
 // are resident at once (64 x 12288 x 4096 44 / 50, 48 x 16000 x 4096 44 / 51, but 64 x 20000 x 4096 80 / 62).
 bool takes_wide(int64_t M, int64_t N, int64_t K, bool dual) {

@@ -2,11 +2,12 @@
 //
 //   bf16 activations   v_mfma_f32_32x32x16_bf16, f32 accumulation
 //   f16 activations    the same with f16 weights, v_mfma_f32_32x32x16_f16 (products of rows an f16 cache holds)
-//   f32 activations    v_mfma_f32_32x32x2_f32 on the weights widened (exactly) to f32: a true 32-bit product
+//   f32 activations    each the sum of three bf16, which makes every product exact, v_mfma_f32_32x32x16_bf16 (gemm_split.h)
 //
 // Weights [N][ldw] and activations [M][lda] are both read along k; K is a multiple of 64, which the owner of the buffers
 // reaches with zero padding.  16-bit operands: gemm_wide.h (tiles of 256 x 256 down to 64 x 64, straight from memory into LDS).
-// 32-bit: 64-row tiles, 32 k at a time through registers.
+// 32-bit: tiles of 128 x 128 down to 32 x 64, the same way; products of experts, of one step, and of rows out of reach go
+// through registers, 32 k at a time, to v_mfma_f32_32x32x2_f32 on the weights widened (exactly) to f32.
 //
 // The epilogue serves two outputs, because the projections that read one normalised row are stored as one
 // stacked matrix: columns below n_first are (alpha * acc + bias) * column scale (+ residual) in f32, columns from n_first
@@ -25,7 +26,7 @@
 
 #include "dense_device.h"
 #include "experts.h"
-#include "gemm_wide.h"
+#include "gemm_split.h"
 
 namespace {
 
@@ -207,9 +208,8 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const Gem
 // The 32-bit product: four waves, a 64 x 64 TN tile, 32 k at a time.  Both tiles sit in LDS as f32 rows of 32 + 4
 // words; a lane reads four consecutive k of its row and feeds four instructions with them (k-slot l >> 5 of
 // instruction e stands for k = 8 s + 4 (l >> 5) + e on both sides).  A matrix-core instruction takes 64 cycles here, so a tile's 16
-// of them cover the loads of the next (registers, then the other LDS buffer; one barrier a tile).  What was far from the 157 TFLOP/s of
-// the part (115 reached at 2048 rows) is a narrow product that leaves compute units without a tile: k slices (blockIdx.y) as for the
-// 16-bit ones, M x N x K without -> with them: 301 x 1024 x 4096 85 -> 36 us, 17 x 1024 x 4096 85 -> 14, 64 x 4096 x 16384 360 -> 86.
+// of them cover the loads of the next (registers, then the other LDS buffer; one barrier a tile).  k slices (blockIdx.y) as for the
+// 16-bit ones.
 template <int TN, bool GROUPED, bool GLU>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   static_assert(!GLU || TN == 2, "a wave's two tiles are the gate and the up value");
@@ -287,6 +287,49 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   }
 }
 
+// 32-bit products of rows within reach (gemm_split.h).  Bound by the matrix cores where tiles are many (at 600 x 18464 x 4096 the three
+// instructions' rate is 1060 TFLOP/s, what the 16-bit products reach), by the steps' latency where they are few; us against 32-bit
+// instructions: 301 x 5136 x 1024 43 -> 18, 301 x 1024 x 4096 37 -> 18, 600 x 18464 x 4096 893 -> 257, 2 x 4096 x 16384 83 -> 34.
+// Distance from 64 bits (2-norm) there 5.7e-7 -> 1.0e-7, 4.7e-7 -> 1.4e-7, 8.1e-7 -> 2.7e-7, 8.1e-7 -> 2.2e-7.  A sum that is not finite is made again by itself: the parts of an infinite value, and
+// a part that is zero times an infinite weight, are no numbers where the product is infinite.  So is one of up to 2^-80: parts lose what lies
+// below bf16's smallest number, 2^-133, which a sum of that size may consist of.
+template <class Tile>
+__global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_kernel(const GemmArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  const int tile = dh::xcd_contiguous(blockIdx.x, a.tiles_m * a.tiles_n);
+  TilePlace place;
+  place_tile<false>(a, tile % a.tiles_m, Tile::BM, &place);
+  const int m0 = place.m0, n0 = (tile / a.tiles_m) * Tile::BN;
+  const int k0 = blockIdx.y * a.k_slice, k_end = min(k0 + a.k_slice, a.K);
+  const float* a_base = static_cast<const float*>(a.A) + (int64_t)m0 * a.lda + k0;
+  const uint16_t* w_base = a.W + (int64_t)n0 * a.ldw + k0;
+  auto a_off = [&](int row) { return (uint32_t)((int64_t)min(row, a.M - 1 - m0) * a.lda * 4); };
+  auto w_off = [&](int row) { return (uint32_t)((int64_t)min(row, a.N - 1 - n0) * a.ldw * 2); };
+  dh::split_product<Tile>(a_base, a_off, w_base, w_off, (k_end - k0) >> 6, smem);
+  const int lane = threadIdx.x & 63;
+#pragma unroll 1
+  for (int u = threadIdx.x >> 6; u < Tile::WM * Tile::NF * 4; u += Tile::kWaves) {
+    const int q = u & 3, j = (u >> 2) % Tile::NF, wm = (u >> 2) / Tile::NF;
+    f32x4_t sum = dh::split_sums<Tile>(smem, 0, wm, j, q)[lane];
+#pragma unroll
+    for (int g = 1; g < Tile::KG; g++) sum += dh::split_sums<Tile>(smem, g, wm, j, q)[lane];
+    const int n = n0 + 32 * j + (lane & 31), row = 32 * wm + 8 * q + 4 * (lane >> 5);
+    if (n >= a.N) continue;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int m = m0 + row + e;
+      if (m >= a.M) break;
+      float v = sum[e];
+      if (__builtin_expect(!(fabsf(v) <= 3.402823466e38f) || (v != 0.f && fabsf(v) < 0x1p-80f), 0)) {
+        v = 0.f;
+        for (int k = 0; k < k_end - k0; k++) v = fmaf(a_base[(int64_t)(row + e) * a.lda + k], dh::bf16_bits_to_f32(w_base[(int64_t)(n - n0) * a.ldw + k]), v);
+      }
+      if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = v;
+      else put(a, m, n, v);
+    }
+  }
+}
+
 // Sums of the k slices in slice order.  VEC columns per thread (N a multiple of VEC), a block's threads as wide as the row allows and the
 // rest of them on further rows (thread t: column t % wide, row t / wide); a grid's second dimension holds 65535 blocks, so rows go round.
 template <int VEC>
@@ -344,26 +387,30 @@ constexpr int kMaxSlices = 16, kMinSliceSteps = 8;
 struct TileChoice {
   int tile, slices;
 };
+// The k loops of so many workgroups; `lone`: how much of the full step's time a single workgroup on every compute unit would take.
+double loops_ns(const TileCost& c, int64_t groups, int64_t steps, double lone) {
+  const int64_t cus = dh::num_cus(), slots = cus * c.per_cu, left = groups % slots;
+  const double f = (double)left / cus;
+  const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (lone + (1.0 - lone) * f / c.per_cu);
+  const int64_t rounds = groups / slots + (left ? 1 : 0);
+  return steps * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + (double)(rounds - 1) * c.again;
+}
 // The cheapest tile and number of k slices.  Slices cost the round trip of their raw sums (about 4 TB/s) and a second launch, and no
 // number of them is faster than the weights come in.
 // erf: a second output through the exact gelu, whose epilogue takes a compute unit about 60 ns for each element a lane holds of a wave, 40
 // where another workgroup's loop runs beside it (1531 x 6144 x 2048 without it 52 us on 128 x 128 tiles, 47 on 256 x 256; with it 76 and
 // 111); behind slices it is the reduce launch's.
 TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool glu, bool erf) {
-  const int64_t cus = dh::num_cus(), steps = K / 64;
+  const int64_t steps = K / 64;
   TileChoice best{0, 1};
   double least = 1e30;
   for (int i = 0; i < 4; i++) {
     const TileCost& c = glu ? kGluTiles[i] : kTiles[i];
     for (int s = 1; s <= most_slices && (s == 1 || steps / s >= kMinSliceSteps); s++) {
-      const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s, slots = cus * c.per_cu, left = groups % slots;
-      const double f = (double)left / cus;
-      const double step = f <= 1.0 ? c.alone + (c.one - c.alone) * f : c.full * (0.76 + 0.24 * f / c.per_cu);
-      const int64_t rounds = groups / slots + (left ? 1 : 0);
-      const double loop = dh::ceil_div(steps, s) * ((double)(groups / slots) * c.full + (left ? step : 0.0)) + (double)(rounds - 1) * c.again;
-      double t = std::max(loop, 2.0 * N * K / 6450.0) + c.start;
+      const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s;
+      double t = std::max(loops_ns(c, groups, dh::ceil_div(steps, s), 0.76), 2.0 * N * K / 6450.0) + c.start;
       if (s > 1) t += 2250.0 + 4.0 * M * N * (2 * s + 1) / 4150.0;
-      else if (erf) t += (c.per_cu == 1 ? 60.0 : 40.0) * (c.bm * c.bn / 64) * dh::ceil_div(groups, cus);
+      else if (erf) t += (c.per_cu == 1 ? 60.0 : 40.0) * (c.bm * c.bn / 64) * dh::ceil_div(groups, dh::num_cus());
       if (t < least) {
         least = t;
         best = TileChoice{i, s};
@@ -479,37 +526,70 @@ int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
   return launch_act(op, a, f16, choose_16bit(a.M, a.N, a.K, a.n_first < a.N && a.act == DH_ACT_GELU_ERF));
 }
 
-// k slices of a 32-bit product.  Workgroups on a compute unit share its matrix cores, so the one with the most of them ends last: 64 k of a
-// tile take 1.35 us alone there and 1.1 us each in company (0.85 at the full rate).  Slices cost a launch and 4 bytes a sum at 4 TB/s.
-int choose_f32_slices(int64_t M, int64_t N, int64_t K) {
-  const int64_t steps = K / 64, tiles = dh::ceil_div(M, 64) * dh::ceil_div(N, 64);
-  const int most = slices_in_workspace(M, N, 16), env_slices = dh::tuning_int("DH_F32_SLICES", 0);
-  if (env_slices) return std::min(most, env_slices);
-  int slices = 1;
+// Tiles of the 32-bit products, and their costs as above, fitted to 318 products (M 2 .. 2048, N 64 .. 20000, K 64 .. 16384) with each tile and
+// up to 16 slices, weights from HBM: the choice is 0.7 % behind the best on average, 15 % at worst.
+using Split32x64 = dh::SplitTile<1, 2, 4, 4, 2>;
+using Split64x64 = dh::SplitTile<2, 2, 4, 3, 4>;
+using Split128x128 = dh::SplitTile<4, 4, 2, 3, 2>;
+constexpr TileCost kSplitTiles[] = {{32, 64, 2, 201.f, 287.f, 503.f, 4500.f, 2730.f},
+                                    {64, 64, 2, 304.f, 411.f, 800.f, 4730.f, 2600.f},
+                                    {128, 128, 1, 737.f, 1190.f, 1293.f, 9470.f, 7970.f}};
+constexpr int kSplitK = 128;                     // two steps
+TileChoice choose_f32(int64_t M, int64_t N, int64_t K) {
+  const int64_t steps = K / 64;
+  const int most = slices_in_workspace(M, N, kMaxSlices);
+  TileChoice best{0, 1};
   double least = 1e30;
-  for (int s = 1; s <= most && (s == 1 || steps / s >= 2); s++) {
-    const int64_t together = dh::ceil_div(tiles * s, dh::num_cus());
-    double t = (together == 1 ? 1350.0 : 1100.0 * together) * dh::ceil_div(steps, s);
-    if (s > 1) t += 3500.0 + 4.0 * M * N * (2 * s + 1) / 4000.0;
-    if (t < least) {
-      least = t;
-      slices = s;
+  for (int i = 0; i < 3; i++)
+    for (int s = 1; s <= most && (s == 1 || steps / s >= 2); s++) {
+      const TileCost& c = kSplitTiles[i];
+      const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s;
+      double t = std::max(loops_ns(c, groups, dh::ceil_div(steps, s), 0.9), 2.0 * N * K / 6165.0) + c.start;
+      if (s > 1) t += 2450.0 + 4.0 * M * N * (2 * s + 1) / 6300.0;
+      if (t < least) {
+        least = t;
+        best = TileChoice{i, s};
+      }
     }
-  }
-  return slices;
+  const int env_tile = dh::tuning_int("DH_F32_TILE", -1), env_slices = dh::tuning_int("DH_F32_SLICES", 0);
+  if (env_tile >= 0) best.tile = env_tile;
+  if (env_slices) best.slices = std::min(most, env_slices);
+  return best;
 }
 // k of a slice (whole steps of 64).
 int slice_extent(int64_t K, int slices) { return (int)dh::ceil_div(K / 64, slices) * 64; }
 
+template <class Tile>
+int launch_split(const char* op, GemmArgs a, int slices) {
+  auto kern = gemm_split_kernel<Tile>;
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLds);
+  DH_CHECK_HIP(op, set);
+  a.tiles_m = (int)dh::ceil_div(a.M, Tile::BM);
+  a.tiles_n = (int)dh::ceil_div(a.N, Tile::BN);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n), slices), dim3(Tile::kThreads), Tile::kLds, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+// Rows below 4 GB apart within a tile and at least two steps take the bf16 matrix cores.  A single step has nothing to hide its start
+// behind: 361 x 8204 x 64 takes 9.4 us with 32-bit instructions and 12.1 without, 2024 x 3594 x 64 17.9 and 21.9; at two steps it is even or ahead.
 int dense_f32(const char* op, GemmArgs a) {
-  a.tiles_m = (int)dh::ceil_div(a.M, 64);
-  a.tiles_n = (int)dh::ceil_div(a.N, 64);
-  a.k_slice = slice_extent(a.K, choose_f32_slices(a.M, a.N, a.K));
+  const bool split = a.K >= kSplitK && 4 * (std::min<int64_t>(a.M, Split128x128::BM) * a.lda + a.K) < (int64_t)1 << 32 && within_reach(a.N, a.ldw, a.K);
+  const TileChoice pick = choose_f32(a.M, a.N, a.K);
+  a.k_slice = slice_extent(a.K, pick.slices);
   const int slices = (int)dh::ceil_div(a.K, a.k_slice);
   size_t ws_bytes = 0;
   if (slices > 1) a.parts = dh::splitk_workspace(&ws_bytes);
-  hipLaunchKernelGGL((gemm_f32_kernel<1, false, false>), dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n), slices), dim3(256), 0, dh::stream(), a);
-  DH_CHECK_LAUNCH(op);
+  if (!split) {
+    a.tiles_m = (int)dh::ceil_div(a.M, 64);
+    a.tiles_n = (int)dh::ceil_div(a.N, 64);
+    hipLaunchKernelGGL((gemm_f32_kernel<1, false, false>), dim3((unsigned)((int64_t)a.tiles_m * a.tiles_n), slices), dim3(256), 0, dh::stream(), a);
+    DH_CHECK_LAUNCH(op);
+  } else {
+    const int rc = pick.tile == 0 ? launch_split<Split32x64>(op, a, slices)
+                 : pick.tile == 1 ? launch_split<Split64x64>(op, a, slices)
+                                  : launch_split<Split128x128>(op, a, slices);
+    if (rc) return rc;
+  }
   return slices > 1 ? launch_reduce(op, a, slices) : 0;
 }
 
@@ -601,11 +681,12 @@ extern "C" int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int form
   if (!out3 || M <= 0 || N <= 0 || K <= 0 || K % 64) return dh::fail(1, "[%s] M=%d, N=%d, K=%d (a multiple of 64), or no place for the result", op, M, N, K);
   dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
   const bool wide = a_dtype == DH_F32, glu = form == 1;
-  const TileChoice pick = wide ? TileChoice{0, glu ? 1 : choose_f32_slices(M, N, K)} : glu ? choose_tile(M, N, K, 1, true, false) : choose_16bit(M, N, K, form == 2);
+  const TileChoice pick = wide ? (glu ? TileChoice{0, 1} : choose_f32(M, N, K)) : glu ? choose_tile(M, N, K, 1, true, false) : choose_16bit(M, N, K, form == 2);
   dh::plan_end();
-  const TileCost& c = glu ? kGluTiles[pick.tile] : kTiles[pick.tile];
-  out3[0] = wide ? 64 : c.bm;
-  out3[1] = wide ? (glu ? 128 : 64) : c.bn;
+  const bool registers = wide && (glu || K < kSplitK);
+  const TileCost& c = wide ? kSplitTiles[pick.tile] : glu ? kGluTiles[pick.tile] : kTiles[pick.tile];
+  out3[0] = registers ? 64 : c.bm;
+  out3[1] = registers ? (glu ? 128 : 64) : c.bn;
   out3[2] = dh::ceil_div(K, slice_extent(K, pick.slices));
   return 0;
 }

@@ -4,6 +4,7 @@ loading, step, cache, prefill and generation.
 Tolerances: 32-bit paths must agree with the float64 restatement to ~1e-5; bf16 paths to what rounding operands to bf16
 (products) and f16 (cached keys and values, queries) explains."""
 import ctypes
+import math
 import json
 import os
 import subprocess
@@ -271,6 +272,71 @@ def test_dense_matmul_f32_slices(L, M, N, K):
     want = -0.5 * (A.double() @ W.double().T) + bias.double()
     # unit products: sums of up to 16448 terms in 32 bits
     assert (C[:, :N].double() - want).abs().max() < 5e-5 and (C[:, N:] == 9.0).all()
+
+
+# the tiles of the 32-bit products, whole and in k slices, ragged in both directions; one of a single step, which goes through registers
+F32_TILES = [(33, 65, 64, (64, 64, 1)), (2, 33, 128, (32, 64, 1)), (33, 70, 960, (32, 64, 1)), (17, 70, 4160, (32, 64, 13)), (200, 4000, 192, (64, 64, 1)),
+             (400, 3001, 2112, (64, 64, 1)), (301, 1024, 4096, (64, 64, 3)), (590, 10255, 2112, (128, 128, 1)), (600, 2050, 8256, (128, 128, 3))]
+
+
+@pytest.mark.parametrize("M,N,K,tile", F32_TILES)
+def test_dense_matmul_f32_tiles(L, M, N, K, tile):
+    """Both outputs, in place, rows further apart than they are long.  Of K terms a sum is rounded fewer than K / 8 times, by 2^-25 of its size
+    on average: within 2^-24 sqrt(K) / 4 of the exact one (2-norm), and 2^-22 for what the epilogue adds."""
+    assert tile_of(L, M, N, K, capi.F32, num_cus=256) == tile
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K + 8, generator=g, device="cuda")
+    W = (torch.randn(N, K + 16, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16)
+    first = N // 2
+    bias, scale, res = (torch.randn(*s, generator=g, device="cuda") for s in ((first,), (first,), (M, first + 3)))
+    C, C2 = res.clone(), torch.full((M, N - first + 2), 9.0, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul_scaled(A.data_ptr(), capi.F32, K + 8, W.data_ptr(), K + 16, M, N, K, 0.5, bias.data_ptr(), scale.data_ptr(), C.data_ptr(),
+                                        C.data_ptr(), first + 3, first, C2.data_ptr(), capi.F32, N - first + 2, capi.ACT_RELU2))
+    capi.check(L.dh_sync())
+    acc = 0.5 * (A[:, :K].double() @ W[:, :K].double().T)
+    want, near = (acc[:, :first] + bias.double()) * scale.double() + res[:, :first].double(), 2.0 ** -24 * K ** 0.5 / 4 + 2.0 ** -22
+    assert (C[:, :first].double() - want).norm() < near * want.norm() and torch.equal(C[:, first:], res[:, first:])
+    want = acc[:, first:].clamp(min=0).square()
+    assert (C2[:, :N - first].double() - want).norm() < 2 * near * want.norm() and (C2[:, N - first:] == 9.0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 70, 128), (300, 1030, 1024), (301, 1024, 4096), (600, 10255, 2112)])
+def test_dense_matmul_f32_extreme_values(L, M, N, K):
+    """Infinities, no numbers and overflow stay where they belong; rows and products near the smallest numbers keep their bits."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A = torch.randn(M, K, generator=g, device="cuda")
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16)
+    A[0, 3], A[1, K - 1] = math.inf, -math.inf
+    A[2, 7] = torch.tensor([0x7f800001], dtype=torch.int32, device="cuda").view(torch.float32)[0]        # a NaN whose upper half is an infinity
+    W[3, 9], A[3, 9] = math.inf, 0.5           # the lower parts of 0.5 are zero
+    W[N - 1, 0] = -math.inf
+    A[4] *= 2.0 ** -122
+    A[0, 4:], W[5, 4:] = 0, 0
+    A[3, 11], W[6, 11] = 3.4e38, 1.0
+    got, want = torch.zeros(M, N, device="cuda"), A.double() @ W.double().T
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), capi.F32, K, W.data_ptr(), K, M, N, K, 1.0, None, None, got.data_ptr(), N, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    finite = want.float().isfinite()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()].double(), want[want.isinf()])
+    # row 4's products are rounded at 2^-149 each
+    assert (got[4].double() - want[4])[finite[4]].abs().max() < 1e-6 * 2.0 ** -122 * 6 + K * 2.0 ** -150
+    rows = [m for m in range(M) if m not in (3, 4)]
+    assert (got.double() - want)[rows][finite[rows]].abs().max() < 5e-5
+
+
+def test_dense_matmul_f32_rows_2_gb_apart(L):
+    M, N, K, ld = 2, 70, 192, 2 ** 29
+    g = torch.Generator(device="cuda").manual_seed(7)
+    A, W, C = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda").to(torch.bfloat16), torch.zeros(M, N, device="cuda")
+    wide = torch.zeros(ld + K, device="cuda")
+    wide[:K], wide[ld:] = A
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(wide.data_ptr(), capi.F32, ld, W.data_ptr(), K, M, N, K, 1.0, None, None, C.data_ptr(), N, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    # 192 terms of size up to 4 x 4 in 32 bits
+    assert (C.double() - A.double() @ W.double().T).abs().max() < 192 * 16 * 2.0 ** -23
 
 
 @pytest.mark.parametrize("M,N,K,operand", [(70000, 16, 4096, "f32"), (66000, 17, 12288, "bf16"), (66000, 20, 12288, "f16")])

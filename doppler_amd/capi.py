@@ -121,6 +121,8 @@ SIGNATURES = {
     "dh_q4k_gemv_chain_limited": (_I, [_P, ctypes.POINTER(ChainPhase), _I, _I, _I]),
     "dh_q4k_gemv_chain_attn_supported": (_I, [_I, _I, _I, _I]),
     "dh_q4k_gemv_chain_attn": (_I, [ctypes.POINTER(ChainAttnSource), ctypes.POINTER(ChainPhase), _I]),
+    "dh_q4k_layer_chain_supported": (_I, [_I, _I, _I, _I]),
+    "dh_q4k_gemv_chain_short": (_I, [_P, ctypes.POINTER(ChainAttnSource), ctypes.POINTER(ChainPhase), _I]),
     "dh_f16w_matmul": (_I, [_P, _P, _P, _I, _I, _I, _F]),
     "dh_lmhead_argmax_workspace_bytes": (_SZ, [_I]),
     "dh_lmhead_argmax_f16": (_I, [_P, _P, _I, _I, _I64, _F, _P, _P, _I, _P]),

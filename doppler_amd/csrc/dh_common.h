@@ -21,6 +21,10 @@ constexpr int kWave = 64;
 // Records a message for dh_last_error() and returns the code to hand back to the caller.
 int fail(int code, const char* fmt, ...);
 hipStream_t stream();
+// Around a launch that uses the library's one exchange area (q4k_gemv_chain.hip): launches of several streams (dh_set_stream) follow one
+// another.
+int exchange_begin(const char* op);
+int exchange_end(const char* op);
 bool ready();
 int num_cus();
 // Scratch for the split-K prefill GEMM's partial products (allocated by dh_init, shared by all

@@ -60,22 +60,24 @@ constexpr int kStage = 3 * 1024;                   // a wave's ring: one unit (1
                                                    // land in the stage's own tail, so no load needs a lane mask
 constexpr int kUnitLoads = 3;                     // load instructions of a full unit: ceil(16 rows * 9 pieces / 64 lanes)
 constexpr int kMaxPhases = DH_CHAIN_MAX_PHASES;
-constexpr int kSlots = 8;                         // tiles whose partial sums may be in LDS at once (a power of two)
-constexpr int kSlotShift = 3;
+// Tiles whose partial sums may be in LDS at once (a power of two).  Rows below 1536 are so few units that those in flight span more tiles:
+// ten at 1024.  A layer of width 1024 (feed-forward 3072, 16 heads, 517 keys) is 23.0 us in two launches against 30.5 in six; the token of
+// 28 layers 865 -> 655 us.  Such a layer is bound by its chain of exchanges, 3.2 us each: 0.4 a unit, 0.3 + 0.7 the tile's end, 1.5 the trip
+// through memory to the other compute dies.
+constexpr int kSlots = 8, kSlotsShort = 16;
 constexpr int kZeroBytes = 144;                   // what a lane without an operand reads
 constexpr size_t kMaxLds = 160 * 1024;
 constexpr int kMaxChainN = 32768;                 // longest exchanged vector
 constexpr int kDefaultSpinLimit = 1 << 17;        // polls of one bounded wait
-constexpr int kColsPerPass = 3;                   // columns whose loads a wave has in flight at once in the prologue
 // counters in LDS: [p] next unit of phase p to draw, [kCtrArrived + s] units delivered to slot s,
-// [kCtrGen + s] tiles completed in slot s, [kCtrAbort] a wave has given up, [kCtrDone + p] tiles of
+// [kGen + s] tiles completed in slot s, [kAbort] a wave has given up, [kDone + p] tiles of
 // phase p this workgroup has finished, then the column flags of the two record areas
 constexpr int kCtrNext = 0;
 constexpr int kCtrArrived = kMaxPhases;
-constexpr int kCtrGen = kCtrArrived + kSlots;
-constexpr int kCtrAbort = kCtrGen + kSlots;
-constexpr int kCtrDone = kCtrAbort + 1;
-constexpr int kCtrFlags = kCtrDone + kMaxPhases;
+template <int SLOTS>
+struct Ctr {
+  static constexpr int kGen = kCtrArrived + SLOTS, kAbort = kGen + SLOTS, kDone = kAbort + 1, kFlags = kDone + kMaxPhases;
+};
 // a tile's partial sums are read four columns at a time: the last read may reach past the counters
 constexpr int kLdsPad = 1024;
 
@@ -108,6 +110,7 @@ struct Phase {
   int tiles_base, tiles_rem;   // tiles per workgroup: floor and remainder of tiles / grid
   int activation, norm_weight_offset;
   int wait_stores;             // a later phase reads this phase's C as its residual
+  int residual_ahead;          // the residual is there when the phase begins, for a workgroup whose own tiles of the phases before are done
   float alpha, clamp_max, norm_eps;
 };
 
@@ -149,7 +152,12 @@ __device__ __forceinline__ uint32_t lds_read_u32(uint32_t addr) {
   return v;
 }
 
+template <int SLOTS>
 __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const ChainArgs a) {
+  constexpr int kSlotShift = SLOTS == 8 ? 3 : 4, kCtrGen = Ctr<SLOTS>::kGen, kCtrAbort = Ctr<SLOTS>::kAbort, kCtrDone = Ctr<SLOTS>::kDone, kCtrFlags = Ctr<SLOTS>::kFlags;
+  static_assert(SLOTS == 1 << kSlotShift, "a power of two");
+  // columns whose loads a wave has in flight at once in the prologue
+  constexpr int kColsPerPass = SLOTS == kSlots ? 3 : 1;
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -162,13 +170,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
   asm volatile("" :: "s"(a.ph[0].norm_weight), "s"(a.ph[0].nb));
 
   // ---- LDS: ring [16 waves][3072], record areas 0 and 1, zeros [144], partial sums
-  // [kSlots][red_stride], counters
+  // [SLOTS][red_stride], counters
   unsigned char* ring = lds;
   unsigned char* xq0 = ring + (size_t)kWaves * kStage;
   unsigned char* xq1 = xq0 + a.xq_bytes[0];
   unsigned char* zeros = xq1 + a.xq_bytes[1];
   float* red = reinterpret_cast<float*>(zeros + kZeroBytes);
-  unsigned* ctr = reinterpret_cast<unsigned*>(red + (size_t)kSlots * a.red_stride);
+  unsigned* ctr = reinterpret_cast<unsigned*>(red + (size_t)SLOTS * a.red_stride);
   const int nflags = a.nb_max[0] + a.nb_max[1];
   // (every wave takes unit `wave` of a phase without drawing: the unit counters start behind those)
   for (int i = tid; i < kCtrFlags + nflags; i += 64 * kWaves) ctr[i] = i < kMaxPhases ? (unsigned)kWaves : 0u;
@@ -288,9 +296,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
     }
     if (2 * lane < a.attn_D) {
 #pragma unroll
-      for (int i = 0; i < kMergePre; i++) {
-        const float* q = m_base + (int64_t)min(i, smax - 1) * (a.attn_D + 2) + 2 * lane;
-        asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(m_ov[i]) : "v"(q) : "memory");
+      for (int i0 = 0; i0 < kMergePre; i0 += 4) {
+        if (i0 >= smax) break;             // (what is read for nothing is waited for: 1650 -> 1634 us with 17 of 32)
+#pragma unroll
+        for (int i = i0; i < i0 + 4; i++) {
+          const float* q = m_base + (int64_t)min(i, smax - 1) * (a.attn_D + 2) + 2 * lane;
+          asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(m_ov[i]) : "v"(q) : "memory");
+        }
       }
     }
     m_nsplit = a.attn_nsplit;
@@ -485,6 +497,9 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
     const uint32_t next_abs = ctr_abs + 4 * (kCtrNext + p);
     const uint32_t flag_want = (uint32_t)p + 1u;
     const bool last_phase = p == nph - 1;
+    // (short rows: a wave has one unit, so what a tile's end needs is fetched here as well, out of the chain of things that are waited for)
+    if constexpr (SLOTS == kSlotsShort)
+      asm volatile("" :: "s"(Q.C), "s"(Q.residual), "s"(Q.alpha), "s"(Q.activation), "s"(Q.clamp_max), "s"(Q.norm_eps), "s"(Q.K), "s"(Q.wait_stores));
 
     if (p > 0 || from_attn) {
       // ---- the wave's first unit of the phase: unit `wave`, no draw
@@ -537,7 +552,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
           if (++spins > a.spin_limit || __builtin_amdgcn_readfirstlane(lds_read_u32(abort_addr)) != 0u) {
             give_up(DH_KSTATUS_EXCHANGE_WAIT, p);
           }
-          __builtin_amdgcn_s_sleep(8);
+          __builtin_amdgcn_s_sleep(SLOTS == kSlots ? 8 : 1);
         }
 #pragma unroll
         for (int i = 0; i < kColsPerPass; i++)
@@ -547,6 +562,14 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
     }
 
     // ---- the phase's units
+    // A workgroup's only tile: its residual is requested here, not when the tile's sums are there (a trip to memory in the chain of
+    // things the other workgroups wait for; a token of 36 layers of width 4096 1675 -> 1650 us).
+    const bool ahead = ntl == 1 && Q.residual_ahead;
+    float res_ahead = 0.f;
+    if (ahead) {
+      const int64_t row = (int64_t)bid * S.rows + j;
+      if (row < S.N) res_ahead = __hip_atomic_load(const_cast<float*>(Q.residual) + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     float inv_rms = 1.f;
     bool have_rms = false;
 #pragma unroll 1
@@ -554,7 +577,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
       if (cur >= total) break;              // draws only grow: nothing behind this one either
       DH_DECODE(S, cur, tl, mat, col)
       const int tord = tb + tl;                         // tile ordinal of the workgroup, over all phases
-      const int slot = tord & (kSlots - 1);
+      const int slot = tord & (SLOTS - 1);
       // draw the unit that will go into the ring once this one has been read (the answer is collected
       // with the reads below)
       unsigned nxt = 0;
@@ -719,7 +742,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
             v = sg * Q.alpha;
             const float* const residual = Q.residual;
             // device-scope load: an earlier phase of this launch may have written the residual
-            if (residual) v += __hip_atomic_load(const_cast<float*>(residual) + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (residual) v += ahead ? res_ahead : __hip_atomic_load(const_cast<float*>(residual) + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
           __hip_atomic_store(Q.C + row, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           if (!last_phase) {
@@ -752,14 +775,15 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_chain_kernel(const Ch
 // ---- host side ----------------------------------------------------------------------------------
 v2u* g_ll = nullptr;          // exchange pairs, 2 x kMaxChainN
 uint32_t* g_epoch = nullptr;  // launch counter
-bool g_coresident = false;
 
 struct Plan {
   ChainArgs a;
   size_t lds;
+  bool short_rows;             // kSlotsShort
 };
 
-int make_plan(const char* op, const float* d_x0, const dh_chain_attn_source* src, const dh_chain_phase* ph, int n, Plan* out) {
+// short_rows: rows below 1536 are served.
+int make_plan(const char* op, const float* d_x0, const dh_chain_attn_source* src, const dh_chain_phase* ph, int n, bool short_rows, Plan* out) {
   if (n < 1 || n > kMaxPhases) return dh::fail(1, "[%s] a chain holds 1..%d products, got %d", op, kMaxPhases, n);
   if ((!d_x0 && !src) || !ph) return dh::fail(1, "[%s] null pointer", op);
   if (reinterpret_cast<uintptr_t>(d_x0) & 15) return dh::fail(1, "[%s] x0 must be 16-byte aligned", op);
@@ -818,12 +842,19 @@ int make_plan(const char* op, const float* d_x0, const dh_chain_attn_source* src
     // outputs that a later product reads back as its residual must have reached memory by then
     for (int q = p + 1; q < n; q++)
       if (ph[q].d_residual == s.d_C) P.wait_stores = 1;
+    // as many rows are the same tiles in the same workgroups
+    P.residual_ahead = s.d_residual != nullptr;
+    for (int q = 0; q < p; q++)
+      if (ph[q].d_C == s.d_residual && ph[q].N != s.N) P.residual_ahead = 0;
     // a product may not overwrite what an earlier or later one of the launch still reads elsewhere
     if (d_x0 && s.d_C == d_x0) return dh::fail(1, "[%s] product %d writes over the chain's input", op, p);
   }
   // the units in flight (16 waves x 2 draws) must not span more tiles than there are slots
-  if ((kWaves * 2 + min_upt - 1) / min_upt + 2 > kSlots)
-    return dh::fail(1, "[%s] K=%d is too short for a chain (at least 1536)", op, min_upt * kQK);
+  const int spanned = (kWaves * 2 + min_upt - 1) / min_upt + 2;
+  if (spanned > (short_rows ? kSlotsShort : kSlots))
+    return dh::fail(1, "[%s] K=%d is too short for a chain (at least %d)", op, min_upt * kQK, short_rows ? 768 : 1536);
+  out->short_rows = spanned > kSlots;
+  const int slots = out->short_rows ? kSlotsShort : kSlots, counters = out->short_rows ? Ctr<kSlotsShort>::kFlags : Ctr<kSlots>::kFlags;
   if (src) {
     // the first product's input is the merge of a decode attention's split-K partial results
     const int ncus = dh::num_cus();
@@ -858,15 +889,16 @@ int make_plan(const char* op, const float* d_x0, const dh_chain_attn_source* src
   a.xq_bytes[1] = a.nb_max[1] * kRec;
   a.red_stride = 16 * max_upt;
   out->lds = (size_t)kWaves * kStage + a.xq_bytes[0] + a.xq_bytes[1] + kZeroBytes +
-             sizeof(float) * kSlots * a.red_stride + sizeof(unsigned) * (kCtrFlags + a.nb_max[0] + a.nb_max[1]) + kLdsPad;
+             sizeof(float) * slots * a.red_stride + sizeof(unsigned) * (counters + a.nb_max[0] + a.nb_max[1]) + kLdsPad;
   if (out->lds > kMaxLds)
     return dh::fail(1, "[%s] the chain's activations do not fit the LDS (%zu of %zu bytes)", op, out->lds, kMaxLds);
   return 0;
 }
 
-int launch(const char* op, Plan& plan, int workgroups) {
-  auto kern = q4k_gemv_chain_kernel;
-  static bool attr_set = false;
+template <int SLOTS>
+int launch_slots(const char* op, Plan& plan, int workgroups) {
+  auto kern = q4k_gemv_chain_kernel<SLOTS>;
+  static bool attr_set = false, coresident = false;
   if (!attr_set) {
     DH_CHECK_HIP(op, hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)kMaxLds));
@@ -874,13 +906,17 @@ int launch(const char* op, Plan& plan, int workgroups) {
     int per_cu = 0;
     DH_CHECK_HIP(op, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kern), 64 * kWaves,
                                                                   kMaxLds));
-    g_coresident = per_cu >= 1;
+    coresident = per_cu >= 1;
     attr_set = true;
   }
-  if (!g_coresident) return dh::fail(1, "[%s] the device cannot hold one workgroup of the chain per compute unit", op);
+  if (!coresident) return dh::fail(1, "[%s] the device cannot hold one workgroup of the chain per compute unit", op);
+  if (int rc = dh::exchange_begin(op)) return rc;
   hipLaunchKernelGGL(kern, dim3(workgroups), dim3(64 * kWaves), plan.lds, dh::stream(), plan.a);
   DH_CHECK_LAUNCH(op);
-  return 0;
+  return dh::exchange_end(op);
+}
+int launch(const char* op, Plan& plan, int workgroups) {
+  return plan.short_rows ? launch_slots<kSlotsShort>(op, plan, workgroups) : launch_slots<kSlots>(op, plan, workgroups);
 }
 
 // Exchange area and launch counter.
@@ -922,7 +958,7 @@ int dh_q4k_gemv_chain(const float* d_x0, const dh_chain_phase* phases, int n_pha
   DH_REQUIRE_INIT(op);
   Plan plan;
   if (!d_x0) return dh::fail(1, "[%s] null pointer", op);
-  if (int rc = make_plan(op, d_x0, nullptr, phases, n_phases, &plan)) return rc;
+  if (int rc = make_plan(op, d_x0, nullptr, phases, n_phases, false, &plan)) return rc;
   return launch(op, plan, plan.a.grid);
 }
 
@@ -937,7 +973,33 @@ int dh_q4k_gemv_chain_attn(const dh_chain_attn_source* source, const dh_chain_ph
   DH_REQUIRE_INIT(op);
   if (!source) return dh::fail(1, "[%s] null pointer", op);
   Plan plan;
-  if (int rc = make_plan(op, nullptr, source, phases, n_phases, &plan)) return rc;
+  if (int rc = make_plan(op, nullptr, source, phases, n_phases, false, &plan)) return rc;
+  return launch(op, plan, plan.a.grid);
+}
+
+int dh_q4k_layer_chain_supported(int hidden, int inter, int q_size, int qkv_size) {
+  if (!dh::ready()) return 0;
+  // a layer's four products, on addresses that nothing reads
+  float* const at = reinterpret_cast<float*>(uintptr_t{16});
+  dh_chain_phase ph[4] = {};
+  const int n[4] = {hidden, inter, hidden, qkv_size}, k[4] = {q_size, hidden, inter, hidden};
+  for (int p = 0; p < 4; p++) {
+    ph[p].d_W = at;
+    ph[p].d_C = at + 4 * (p + 1);
+    ph[p].N = n[p];
+    ph[p].K = k[p];
+  }
+  ph[1].d_W2 = at;
+  Plan plan;
+  return make_plan("dh_q4k_layer_chain_supported", at, nullptr, ph, 4, true, &plan) == 0 ? 1 : 0;
+}
+
+int dh_q4k_gemv_chain_short(const float* d_x0, const dh_chain_attn_source* source, const dh_chain_phase* phases, int n_phases) {
+  const char* op = "dh_q4k_gemv_chain_short";
+  DH_REQUIRE_INIT(op);
+  if (!d_x0 == !source) return dh::fail(1, "[%s] the first product reads either x0 or an attention's partial results", op);
+  Plan plan;
+  if (int rc = make_plan(op, d_x0, source, phases, n_phases, true, &plan)) return rc;
   return launch(op, plan, plan.a.grid);
 }
 
@@ -947,7 +1009,7 @@ int dh_q4k_gemv_chain_limited(const float* d_x0, const dh_chain_phase* phases, i
   DH_REQUIRE_INIT(op);
   Plan plan;
   if (!d_x0) return dh::fail(1, "[%s] null pointer", op);
-  if (int rc = make_plan(op, d_x0, nullptr, phases, n_phases, &plan)) return rc;
+  if (int rc = make_plan(op, d_x0, nullptr, phases, n_phases, false, &plan)) return rc;
   if (workgroups < 1 || workgroups > plan.a.grid)
     return dh::fail(1, "[%s] workgroups must be 1..%d", op, plan.a.grid);
   if (spin_limit < 1 || spin_limit > kDefaultSpinLimit) return dh::fail(1, "[%s] spin_limit must be 1..%d", op, kDefaultSpinLimit);

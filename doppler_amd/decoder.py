@@ -477,10 +477,11 @@ class HipDecoder(DecoderBase):
 
     def chain_gemvs_served(self):
         """Whether set_chain_gemvs(True) accepts this model: hidden, FFN and attention widths that are
-        multiples of 256 in 2048..32768, norms fused, finiteness guard off."""
+        multiples of 256 in 768..32768 and fit the launch, norms fused, finiteness guard off."""
         c = self.cfg
-        dims = (c["hidden"], c["inter"], c["heads"] * c["head_dim"])
-        return bool(all(k % 256 == 0 and 2048 <= k <= 32768 for k in dims) and self.fuse_norm and not self.finiteness_guard)
+        qs, ks = c["heads"] * c["head_dim"], c["kv_heads"] * c["head_dim"]
+        return bool(self.fuse_norm and not self.finiteness_guard and
+                    self.L.dh_q4k_layer_chain_supported(c["hidden"], c["inter"], qs, qs + 2 * ks))
 
     def set_chain_gemvs(self, on, merge_attention=True):
         """on: the four products between two attentions (o, gate/up, down, next q/k/v) go out as one
@@ -491,7 +492,7 @@ class HipDecoder(DecoderBase):
         c = self.cfg
         if on and not self.chain_gemvs_served():
             raise ValueError("chain_gemvs serves hidden, FFN and attention widths that are multiples of 256 in "
-                             "2048..32768, with the norms fused and the finiteness guard off (got %s)"
+                             "768..32768 and fit one launch, with the norms fused and the finiteness guard off (got %s)"
                              % ((c["hidden"], c["inter"], c["heads"] * c["head_dim"]),))
         self.chain_gemvs = bool(on)
         self.chain_merges_attention = bool(on and merge_attention and self.fuse_qkv_attention and
@@ -600,7 +601,7 @@ class HipDecoder(DecoderBase):
             # the library moves that launch with the position, a split count handed to the chain it could not)
             if not self.chain_merges_attention or (getattr(self, "_capturing", False) and not device_kv_len):
                 self._enqueue_attention(d, pos, device_kv_len)
-                ck(L.dh_q4k_gemv_chain(self.attn.data_ptr(), arr, n))
+                ck(L.dh_q4k_gemv_chain_short(self.attn.data_ptr(), None, arr, n))
                 continue
             # the key splits' partial results stay in the workspace; the chain's first waves merge them
             src = capi.ChainAttnSource(self.attn_ws.data_ptr(), H, Hkv, D, 0, None, 0, 0, 0)
@@ -619,7 +620,7 @@ class HipDecoder(DecoderBase):
                     self.sin.data_ptr(), d["cache_k"].data_ptr(), d["cache_v"].data_ptr(), H, Hkv, D, pos, D, 0, c["eps"],
                     0, use_norm, self.scale, 0.0, 0, 0, capi.KV_CONTIGUOUS, self.attn_ws.data_ptr(), ctypes.byref(nsplit)))
                 src.nsplit = nsplit.value
-            ck(L.dh_q4k_gemv_chain_attn(ctypes.byref(src), arr, n))
+            ck(L.dh_q4k_gemv_chain_short(None, ctypes.byref(src), arr, n))
 
     def _enqueue_attention(self, d, pos, device_kv_len=False):
         """self.qkv (raw stacked projection of the step's token) -> self.attn, appending the

@@ -204,7 +204,8 @@ int dh_q4k_ffn_gate_up_rmsnorm(const float* d_x, const float* d_norm_weight, flo
  * Limits: K of every product a multiple of 256 and at least 2048, N and K at most 32768,
  * K_p = N_{p-1}, f32 vectors, 16-byte aligned pointers; a product's d_residual may be an earlier
  * product's d_C (or d_x0's producer's output), d_C must not be d_x0.  Launches are ordered on the
- * op stream and share one exchange area of the library: one chain at a time per device.
+ * op stream and share one exchange area of the library: one chain at a time per device (chains of several streams set with
+ * dh_set_stream follow one another).
  * Every wait inside the launch is bounded: if one gives up (it cannot while the launch has the
  * device's compute units to itself) all waves exit, the outputs are undefined, and the next call
  * that waits for the stream (dh_sync, dh_download, dh_upload, dh_free) fails with the reason. */
@@ -245,6 +246,11 @@ typedef struct dh_chain_attn_source {
   int max_kv_len, sliding_window, kv_start;
 } dh_chain_attn_source;
 int dh_q4k_gemv_chain_attn(const dh_chain_attn_source* source, const dh_chain_phase* phases, int n_phases);
+/* The same for models with short rows: K of every product from 768 on.  The first product reads d_x0, or with `source` the merged
+ * attention (the other one is NULL). */
+/* 1 when a layer's products (o, gate/up, down, next q/k/v) fit one such chain (after dh_init), else 0. */
+int dh_q4k_layer_chain_supported(int hidden, int inter, int q_size, int qkv_size);
+int dh_q4k_gemv_chain_short(const float* d_x0, const dh_chain_attn_source* source, const dh_chain_phase* phases, int n_phases);
 /* 1 when dh_q4k_gemv_chain_attn serves this head geometry for key counts up to max_kv_len on the
  * current device (after dh_init), else 0. */
 int dh_q4k_gemv_chain_attn_supported(int H, int Hkv, int D, int max_kv_len);

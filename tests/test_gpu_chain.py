@@ -314,3 +314,86 @@ def test_chain_attn_argument_errors():
     fails(capi.ChainAttnSource(ws, 32, 8, 128, 0, lay.kvlen.data_ptr(), 0, 0, 0), "max_kv_len >= 1")
     assert L.dh_q4k_gemv_chain_attn_supported(32, 8, 96, 1024) == 0
     assert L.dh_q4k_gemv_chain_attn_supported(32, 5, 128, 1024) == 0
+
+
+# ---- short rows: more tiles in flight than the wide models' launches hold ----------------------------------------
+
+@pytest.mark.parametrize("dims", [(768, 768, 768, 768), (1024, 3072, 1024, 2048), (1280, 4096, 768, 1100), (1024, 2304, 2048, 515), (1280, 12288, 1280, 20000)])
+def test_short_rows_against_oracle_and_separate_calls(dims):
+    """Rows of 768 to 1280 elements, the shortest and the last before the wide models', and many tiles a workgroup."""
+    L = capi.init(0)
+    lay = Layer(*dims, seed=7600 + dims[1] + dims[0])
+    sep = {k: torch.zeros_like(v) for k, v in lay.out.items()}
+    lay.separate(L, sep)
+    capi.check(L.dh_sync())
+    want = lay.oracle_chain()
+    arr = capi.chain_phases(lay.phases())
+    for rep in range(3):
+        for t in lay.out.values():
+            t.fill_(float("nan"))
+        capi.check(L.dh_q4k_gemv_chain_short(lay.d["attn"].data_ptr(), None, arr, 4))
+        capi.check(L.dh_sync())
+        for name in ("x2", "act", "x3", "qkv"):
+            assert rel_l2(_read(lay.out[name]), want[name]) <= 1e-3, (rep, name)
+            assert _read(lay.out[name]).tobytes() == _read(sep[name]).tobytes(), (rep, name)
+    with pytest.raises(DopplerHipError, match="too short for a chain"):
+        capi.check(L.dh_q4k_gemv_chain_short(lay.d["attn"].data_ptr(), None, capi.chain_phases(
+            [dict(W=lay.d["wo"].data_ptr(), C=lay.out["x2"].data_ptr(), N=256, K=512)]), 1))
+    with pytest.raises(DopplerHipError, match="either x0 or"):
+        capi.check(L.dh_q4k_gemv_chain_short(None, None, arr, 4))
+
+
+def test_layers_that_fit_a_chain():
+    L = capi.init(0)
+    for dims, fits in (((1024, 3072, 1024, 2048), 1), ((4096, 12288, 4096, 6144), 1), ((768, 768, 768, 768), 1), ((512, 1024, 512, 1024), 0),
+                       ((1024, 3000, 1024, 2048), 0), ((1024, 32768, 1024, 2048), 0), ((1024, 16384, 1024, 2048), 0)):
+        assert L.dh_q4k_layer_chain_supported(*dims) == fits, dims
+
+
+def test_residual_of_other_rows_is_read_when_its_tile_ends():
+    """A product whose residual is the head of a longer product's outputs (other rows, so other workgroups') is not read ahead."""
+    L = capi.init(0)
+    N0, N1, N2, K = 2048, 4096, 2048, 2048
+    w = [dev(synth.q4k_tensor(n, k, 7700 + i)) for i, (n, k) in enumerate([(N1, K), (N0, N1), (N2, N0)])]
+    x = dev(synth.normal_f32(K, 7710) * np.float32(0.01))
+    c = [f32(N1), f32(N0), f32(N2)]
+    ph = [dict(W=w[0].data_ptr(), C=c[0].data_ptr(), N=N1, K=K), dict(W=w[1].data_ptr(), C=c[1].data_ptr(), N=N0, K=N1),
+          dict(W=w[2].data_ptr(), C=c[2].data_ptr(), residual=c[0].data_ptr(), N=N2, K=N0)]
+    capi.check(L.dh_q4k_gemv_chain(x.data_ptr(), capi.chain_phases(ph), 3))
+    capi.check(L.dh_sync())
+    got = [_read(t) for t in c]
+    ck, o = capi.check, [f32(N1), f32(N0), f32(N2)]
+    ck(L.dh_q4k_matmul(x.data_ptr(), capi.F32, w[0].data_ptr(), o[0].data_ptr(), capi.F32, 1, N1, K, 1.0, None))
+    ck(L.dh_q4k_matmul(o[0].data_ptr(), capi.F32, w[1].data_ptr(), o[1].data_ptr(), capi.F32, 1, N0, N1, 1.0, None))
+    ck(L.dh_q4k_matmul(o[1].data_ptr(), capi.F32, w[2].data_ptr(), o[2].data_ptr(), capi.F32, 1, N2, N0, 1.0, o[0].data_ptr()))
+    ck(L.dh_sync())
+    for a, b in zip(got, o):
+        assert a.tobytes() == _read(b).tobytes()
+
+
+def test_chains_of_several_streams_follow_one_another():
+    L = capi.init(0)
+    lays = [Layer(1024, 3072, 1024, 2048, seed=7800), Layer(2048, 4096, 2048, 3072, seed=7850), Layer(1024, 3072, 1024, 2048, seed=7900)]
+    arrs = [capi.chain_phases(l.phases()) for l in lays]
+    sep = [{k: torch.zeros_like(v) for k, v in l.out.items()} for l in lays]
+    for l, s in zip(lays, sep):
+        l.separate(L, s)
+    capi.check(L.dh_sync())
+    streams = [None, torch.cuda.Stream(), torch.cuda.Stream()]
+    try:
+        for rep in range(5):
+            for l in lays:
+                for t in l.out.values():
+                    t.zero_()
+            torch.cuda.synchronize()
+            for again in range(4):
+                for l, arr, s in zip(lays, arrs, streams):
+                    capi.check(L.dh_set_stream(s.cuda_stream if s else None))
+                    capi.check(L.dh_q4k_gemv_chain_short(l.d["attn"].data_ptr(), None, arr, 4))
+            torch.cuda.synchronize()
+            for i, l in enumerate(lays):
+                for k, v in l.out.items():
+                    assert _read(v).tobytes() == _read(sep[i][k]).tobytes(), (rep, i, k)
+    finally:
+        capi.check(L.dh_set_stream(None))
+    capi.check(L.dh_sync())

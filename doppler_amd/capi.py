@@ -234,6 +234,6 @@ _initialised = False
 
 def init(device=0):
     global _initialised
-    check(load().dh_init(device))
+    check((_lib or load()).dh_init(device))
     _initialised = True
     return _lib

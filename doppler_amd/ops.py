@@ -52,7 +52,8 @@ def createWeightBuffer(buffer, dtype, layout, shape, label=None):
 
 
 def _lib():
-    if not torch.cuda.is_available():
+    # (asking for a GPU again costs half a microsecond of a call of seven; a library that is up has one)
+    if not capi._initialised and not torch.cuda.is_available():
         raise DopplerHipError("no GPU visible: the HIP path cannot run (there is no CPU fallback)")
     return capi.init(torch.cuda.current_device())
 
@@ -116,8 +117,7 @@ def _ptr(x):
 
 
 def _nbytes(x):
-    b = _buf(x)
-    return b.numel() * b.element_size()
+    return _buf(x).nbytes
 
 
 def _out(outputBuffer, nbytes):
@@ -146,9 +146,10 @@ def runMatmul(A, B, M, N, K, alpha=1.0, outputBuffer=None, transposeB=True, outp
     `useFusedRmsnormWideTile` the RMSNorm of A runs inside the matmul
     (src/gpu/kernels/matmul-selection.js:609-620)."""
     op = "runMatmul"
-    for v in (M, N, K):
-        if not isinstance(v, (int, np.integer)):
-            raise DopplerHipError("[%s] Invalid dimensions: M=%s, N=%s, K=%s" % (op, M, N, K))
+    if not (type(M) is type(N) is type(K) is int):
+        for v in (M, N, K):
+            if not isinstance(v, (int, np.integer)):
+                raise DopplerHipError("[%s] Invalid dimensions: M=%s, N=%s, K=%s" % (op, M, N, K))
     if M <= 0 or N <= 0 or K <= 0:
         raise DopplerHipError("[%s] Dimensions must be positive: M=%s, N=%s, K=%s" % (op, M, N, K))
     if outputDtype not in ("f16", "f32"):
@@ -158,11 +159,12 @@ def runMatmul(A, B, M, N, K, alpha=1.0, outputBuffer=None, transposeB=True, outp
         raise DopplerHipError("[%s] B dtype is required for matmul dispatch%s." % (op, " (role=%s)" % role if role else ""))
     if A.dtype not in ("f32", "f16"):
         raise DopplerHipError("[%s] f32 or f16 activations required, got %s" % (op, A.dtype))
-    a_elem = 2 if A.dtype == "f16" else 4
+    a_f16 = A.dtype == "f16"
+    a_elem = 2 if a_f16 else 4
     if _nbytes(A) < M * K * a_elem:
         raise DopplerHipError("[%s] A buffer too small: %d < %d (M=%d, K=%d, aDtype=%s)"
                               % (op, _nbytes(A), M * K * a_elem, M, K, A.dtype))
-    if A.dtype == "f16" and (bdtype != "q4k" or (normWeight is not None and useFusedRmsnormWideTile)):
+    if a_f16 and (bdtype != "q4k" or (normWeight is not None and useFusedRmsnormWideTile)):
         raise DopplerHipError("[%s] f16 activations are served for q4k weights without the fused RMSNorm only" % op)
     L = _lib()
     if bdtype == "q4k":
@@ -181,8 +183,8 @@ def runMatmul(A, B, M, N, K, alpha=1.0, outputBuffer=None, transposeB=True, outp
                                                1 if rmsNormOffset else 0, _ptr(B), out.data_ptr(), cdt,
                                                M, N, K, alpha, _ptr(residualTensor)))
         else:
-            capi.check(L.dh_q4k_matmul(_ptr(A), capi.F16 if A.dtype == "f16" else capi.F32, _ptr(B),
-                                       out.data_ptr(), cdt, M, N, K, alpha, _ptr(residualTensor)))
+            capi.check(L.dh_q4k_matmul(_ptr(A), capi.F16 if a_f16 else capi.F32, B.buffer.data_ptr(), out.data_ptr(), cdt, M, N, K, alpha,
+                                       _ptr(residualTensor)))
         return Tensor(out, outputDtype, (M, N), "matmul_output")
     if bdtype == "f16":
         if transposeB not in (True, "auto"):

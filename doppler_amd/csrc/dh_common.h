@@ -98,6 +98,9 @@ struct Family {
 };
 int register_family(const Family& f);
 
+// C = alpha * (sum of the slices [M][N] at parts, in order; at most 8) + residual (q4k_gemm.hip).
+int q4k_sum_slices(const char* op, float* parts, int slices, void* C, int c_f16, int M, int N, float alpha, const float* residual);
+
 // Matrix-core GEMM for prefill-sized batches (q4k_gemm.hip).  `serves`: M >= 16, K a multiple
 // of 4, A 16-byte aligned.
 bool q4k_gemm_serves(int M, int K, const void* A);

@@ -1031,6 +1031,12 @@ int launch_gemm(GemmArgs a, const char* op) {
 
 namespace dh {
 
+int q4k_sum_slices(const char* op, float* parts, int slices, void* C, int c_f16, int M, int N, float alpha, const float* residual) {
+  GemmArgs a{};
+  a.partial = parts; a.ksplit = slices; a.C = C; a.c_f16 = c_f16; a.M = M; a.N = N; a.alpha = alpha; a.residual = residual;
+  return launch_reduce(a, op);
+}
+
 bool q4k_gemm_serves(int M, int K, const void* A) {
   (void)K; (void)A;          // any K and alignment: the packing pre-pass has a scalar path
   return M >= 16;

@@ -87,6 +87,7 @@ struct RowsArgs {
   int acc_max;           // accumulators per wave the LDS block was sized for: (tiles_base + 1 if tiles_rem) * matrices
   int c_f16, activation, norm_weight_offset;
   float alpha, clamp_max, norm_eps;
+  float* parts;          // [slices][M][N] raw sums of a slice of the columns (blockIdx.y) each, or null
 };
 
 // value of lane ^ 1
@@ -159,7 +160,9 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_rows_kernel(const Row
   const int64_t row_bytes = (int64_t)nb * kBlockBytes;
   const int ntl = a.tiles_base + ((int)blockIdx.x < a.tiles_rem ? 1 : 0);   // this workgroup's tiles: blockIdx.x + i * grid
   const int nacc = ntl * NMAT;
-  const int total = nb * nacc;                 // units of the workgroup, ordered (column, tile, matrix)
+  // slices of the columns (blockIdx.y of gridDim.y)
+  const int col0 = (int)(blockIdx.y * nb) / (int)gridDim.y, cols = (int)((blockIdx.y + 1) * nb) / (int)gridDim.y - col0;
+  const int total = cols * nacc;               // units of the workgroup, ordered (column, tile, matrix)
   const int q0 = (wave * total) >> 4, q1 = ((wave + 1) * total) >> 4;
   const int nun = q1 - q0;                     // this wave's run
   unsigned char* my_ring = ring + (size_t)wave * D * kStage;
@@ -369,6 +372,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_rows_kernel(const Row
   if (nun > 0) {
     colc = q0 / nacc;
     accc = q0 - colc * nacc;
+    colc += col0;
   }
   int coli = colc, acci = accc;
   int issued = 0, consumed = 0;
@@ -536,6 +540,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_rows_kernel(const Row
     const int tile = (int)blockIdx.x + tl * a.grid;
     const int64_t row = (int64_t)tile * a.rows + oj;
     if (oj < a.rows && m < a.M && row < a.N) {
+      if (!DUAL && a.parts) {
+        a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + row] = sg;
+        continue;
+      }
       float v;
       if (DUAL) {
         const float act = a.activation == DH_ACT_SILU ? act_silu(sg) : act_gelu(sg);
@@ -555,21 +563,66 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_rows_kernel(const Row
 
 int env_int(const char* name, int dflt) { return dh::tuning_int(name, dflt); }
 
+// A launch for so many compute units: rows per tile, the largest count <= 16 that gives every workgroup the same number of tiles, and the
+// tiles dealt to workgroups.
+struct Deal {
+  int rows, grid, base, rem;
+};
+Deal deal(int64_t N, int64_t cus) {
+  const int64_t per_cu = dh::ceil_div(N, cus * kTileRows);
+  const int rows = (int)std::max<int64_t>(1, std::min<int64_t>(kTileRows, dh::ceil_div(N, cus * per_cu)));
+  const int64_t tiles = dh::ceil_div(N, rows), grid = std::min(tiles, cus);
+  return {rows, (int)grid, (int)(tiles / grid), (int)(tiles % grid)};
+}
+
+// Slices of the columns, whose sums a second launch adds up.  A wave's columns follow one another: loads of its eight activation rows,
+// conversion, products.  Many columns over few tiles are therefore cut so that a wave meets one of them and uses it for several tiles: M x N x K
+// in us, weights from memory, one slice against the choice: 8 x 4096 x 12288 18.9 -> 15.9 (weights from the cache 15.2 -> 14.2), 8 x 2048 x 12288
+// 16.2 -> 12.0, 8 x 1024 x 12288 15.0 -> 10.9, 8 x 12288 x 12288 29.9 -> 27.1, 8 x 2048 x 6144 11.4 -> 10.2, 4 x 600 x 9000 14.9 -> 10.7.  The costs
+// below (us) were read off these: a column, a unit, the second launch; up to 16 columns over 256 workgroups stay whole (8 x 4096 x 4096 8.5, 11.4 in
+// two slices).
+int choose_slices(int64_t M, int64_t N, int64_t nb) {
+  constexpr double kColumn = 4.0, kUnit = 0.7, kUnitRow = 1.3 / kTileRows, kSecondLaunch = 3.0;
+  if (nb <= kWaves) return 1;
+  size_t bytes = 0;
+  (void)dh::splitk_workspace(&bytes);
+  const int most = (int)std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)bytes / (4 * M * N)));
+  int best = 1;
+  double least = 1e30;
+  for (int s = 1; s <= most; s++) {
+    const Deal d = deal(N, std::max(1, dh::num_cus() / s));
+    const int tiles = d.base + (d.rem ? 1 : 0);
+    const int64_t units = dh::ceil_div(nb, s) * tiles;
+    int64_t columns = 0, run = 0;              // the most that a wave meets
+    for (int w = 0; w < kWaves; w++) {
+      const int64_t q0 = w * units / kWaves, q1 = (w + 1) * units / kWaves;
+      run = std::max(run, q1 - q0);
+      if (q1 > q0) columns = std::max(columns, (q1 - 1) / tiles - q0 / tiles + 1);
+    }
+    const double t = kColumn * columns + (kUnit + kUnitRow * d.rows) * run + (s > 1 ? kSecondLaunch : 0.0);
+    if (t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  const int env = env_int("DH_GEMV_ROWS_SLICES", 0);
+  return env ? std::min(env, most) : best;
+}
+
 template <bool DUAL, bool VEC, bool AF16 = false>
 int launch_rows(RowsArgs a, const char* op) {
   constexpr int NMAT = DUAL ? 2 : 1;
   auto kern = q4k_gemv_rows_kernel<DUAL, VEC, AF16>;
-  const int ncu = dh::num_cus();
-  // rows per tile: the largest count <= 16 that gives every workgroup the same number of tiles
-  const int per_cu = (int)dh::ceil_div(a.N, (int64_t)ncu * kTileRows);
-  a.rows = std::max(1, std::min(kTileRows, (int)dh::ceil_div(a.N, (int64_t)ncu * per_cu)));
-  a.nlw = (9 * a.rows + 63) / 64;
-  const int64_t ntiles = dh::ceil_div(a.N, a.rows);
-  const int grid = (int)std::min<int64_t>(ntiles, ncu);
-  a.grid = grid;
-  a.tiles_base = (int)(ntiles / grid);
-  a.tiles_rem = (int)(ntiles % grid);
-  a.acc_max = (a.tiles_base + (a.tiles_rem ? 1 : 0)) * NMAT;
+  auto lay_out = [&](int slices) {
+    const Deal d = deal(a.N, std::max(1, dh::num_cus() / slices));
+    a.rows = d.rows;
+    a.nlw = (9 * a.rows + 63) / 64;
+    a.grid = d.grid;
+    a.tiles_base = d.base;
+    a.tiles_rem = d.rem;
+    a.acc_max = (a.tiles_base + (a.tiles_rem ? 1 : 0)) * NMAT;
+  };
+  lay_out(1);
   // about a run per wave: with far fewer units than waves most of the workgroup idles, and the
   // kernel that spreads a tile's columns over the waves is faster (measured on 1024 x 3072 and smaller)
   static const int env_min_units = env_int("DH_GEMV_ROWS_MIN_UNITS", 12);
@@ -578,26 +631,51 @@ int launch_rows(RowsArgs a, const char* op) {
     return (size_t)kWaves * dep * kStage + (a.norm_weight ? sizeof(float) * kWaves * kQK : 0) +
            sizeof(float) * kWaves * kSsqFloats + (size_t)kWaves * a.acc_max * kAccBytes;
   };
-  static const int env_depth = env_int("DH_GEMV_ROWS_DEPTH", 0);
-  int depth = env_depth > 0 ? std::min(kMaxDepth, env_depth) : kMaxDepth;
-  while (depth > 1 && lds_for(depth) > kLdsCap) depth--;
-  if (lds_for(depth) > kLdsCap) return -1;
-  a.depth = depth;
+  // ring stages that fit; 0: none does
+  auto fit_depth = [&]() {
+    static const int env_depth = env_int("DH_GEMV_ROWS_DEPTH", 0);
+    int depth = env_depth > 0 ? std::min(kMaxDepth, env_depth) : kMaxDepth;
+    while (depth > 0 && lds_for(depth) > kLdsCap) depth--;
+    return depth;
+  };
+  a.depth = fit_depth();
+  if (a.depth == 0) return -1;
+  // the record is the launch of one slice; several are this launch for so many times fewer compute units, with fewer columns
   {
-    const int64_t rec[12] = {a.rows, a.nlw, grid, a.tiles_base, a.tiles_rem, depth, (int64_t)lds_for(depth), 0, 0, 0, a.acc_max,
+    const int64_t rec[12] = {a.rows, a.nlw, a.grid, a.tiles_base, a.tiles_rem, a.depth, (int64_t)lds_for(a.depth), 0, 0, 0, a.acc_max,
                              a.M};
     for (int i = 0; i < 12; i++) dh::plan_layout(i, rec[i]);
   }
   if (dh::plan_note(DH_PLAN_GEMV_ROWS)) return 0;
+  int slices = DUAL || a.norm_weight ? 1 : choose_slices(a.M, a.N, a.nb);
+  if (slices > 1) {
+    lay_out(slices);
+    a.depth = fit_depth();
+    if (a.depth == 0) {
+      slices = 1;
+      lay_out(1);
+      a.depth = fit_depth();
+    }
+  }
+  const size_t lds = lds_for(a.depth);
   static bool attr_set = false;   // once per instantiation: the call costs microseconds
   if (!attr_set) {
     DH_CHECK_HIP(op, hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsCap));
     attr_set = true;
   }
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kWaves), lds_for(depth), dh::stream(), a);
+  if (slices == 1) {
+    hipLaunchKernelGGL(kern, dim3(a.grid), dim3(64 * kWaves), lds, dh::stream(), a);
+    DH_CHECK_LAUNCH(op);
+    return 0;
+  }
+  size_t bytes = 0;
+  a.parts = dh::splitk_workspace(&bytes);
+  if (int rc = dh::exchange_begin(op)) return rc;
+  hipLaunchKernelGGL(kern, dim3(a.grid, slices), dim3(64 * kWaves), lds, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
-  return 0;
+  if (int rc = dh::q4k_sum_slices(op, a.parts, slices, a.C, a.c_f16, a.M, a.N, a.alpha, a.residual)) return rc;
+  return dh::exchange_end(op);
 }
 
 }  // namespace

@@ -88,6 +88,24 @@ def _matmul_case(M, N, K, seed, alpha=1.0, outputDtype="f32", residual=False):
     return rel_l2(got, want)
 
 
+@pytest.mark.parametrize("M,N,K,alpha,outputDtype,residual,f16", [
+    (3, 1100, 4352, 1.0, "f32", False, False),                                   # 17 columns: the first count that may be cut
+    (8, 4096, 12288, 1.0, "f32", True, False), (4, 600, 9000, 0.5, "f32", True, False), (15, 1024, 12288, 1.0, "f16", True, False),
+    (5, 2047, 6148, 1.0, "f32", False, True), (8, 33, 32768, -2.0, "f32", True, True), (7, 3001, 5000, 1.0, "f16", False, False)])
+def test_few_rows_of_many_columns(M, N, K, alpha, outputDtype, residual, f16):
+    """Long rows whose columns are cut into slices.  Operands keep 22 bits and sums are f32: 1e-5 of the result; an f16 output rounds to 2^-11."""
+    W, wb = q4k_weight(N, K, 1350 + M)
+    A = synth.normal_f32((M, K), 1351 + M)
+    A = A.astype(np.float16) if f16 else A
+    res = synth.normal_f32((M, N), 1352 + M) if residual else None
+    for rep in range(2):
+        got = ops.readTensor(ops.runMatmul(ops.tensorFromNumpy(A.view(np.uint16) if f16 else A), wb, M, N, K, alpha=alpha, outputDtype=outputDtype,
+                                           residualTensor=ops.tensorFromNumpy(res) if residual else None))
+        got = got.view(np.float16).astype(np.float32) if outputDtype == "f16" else got
+        want = oracle.q4k_matmul(A.astype(np.float32), W, M, N, K, alpha)
+        assert rel_l2(got, want + res if residual else want) <= 1e-5 + (5e-4 if outputDtype == "f16" else 0)
+
+
 @pytest.mark.parametrize("M,N,K,outputDtype,residual", [
     (4, 6144, 1536, "f16", False),      # the shape of the reference's f16-activation parity test
     (1, 1024, 4096, "f16", False), (1, 4096, 4096, "f32", True), (8, 512, 1152, "f32", False),

@@ -294,6 +294,14 @@ def test_a_smaller_device_changes_the_layout_not_the_bounds():
     check_rows(4, 4096, 12288, 0, 0, ncu=304)
 
 
+@pytest.mark.parametrize("slices", range(2, 9))
+def test_few_row_gemv_slices_are_launches_for_fewer_compute_units(slices):
+    """Rows of more than 16 columns go in slices of the columns, each dealt to so many times fewer compute units."""
+    for M, N, K in ((8, 4096, 12288), (3, 600, 9000), (8, 12288, 32768), (5, 33, 4100)):
+        if layout(M, N, K, 0, 0, NCU // slices)[0] == ROWS:
+            check_rows(M, N, K, 0, 0, ncu=NCU // slices)
+
+
 def test_the_product_tests_reach_every_tile():
     """The shapes of the matrix products' GPU tests take the tiles named beside them, and together every one a product of many shapes takes."""
     from tests import test_gpu_ops, test_gpu_zepavik

@@ -162,6 +162,51 @@ def test_memory_state_starts_at_zero_whatever_the_buffers_hold(L, tmp_path):
         assert parts_error(dec, want, t, portions, 150).max() < PART["float32"]
 
 
+@pytest.mark.parametrize("H,D,V,T,start", [(1, 32, 32, 1, 0), (2, 64, 96, 64, 0), (3, 96, 32, 65, 0), (2, 160, 64, 191, 5), (1, 256, 512, 130, 64)])
+def test_memory_state_behind_a_prompt(L, H, D, V, T, start):
+    """State and normaliser behind a portion against the recurrence in 64 bits, on tiles that are whole and half full; and an infinite key and value,
+    which stay with their row and column.  A chunk's 64 products are summed and rounded in f32: 64 * 2^-24 of the largest terms at worst."""
+    import ctypes
+    from doppler_amd.capi import MLSTM
+    g = rng(100 + D + T)
+    n_qkv, ld = H * (2 * D + V), H * (2 * D + V) + 2 * H + 2 * H % 4
+    for bad in (False, True):
+        rows = g.standard_normal((T, ld)).astype(np.float32)
+        k, v = rows[:, H * D:2 * H * D].reshape(T, H, D), rows[:, 2 * H * D:n_qkv].reshape(T, H, V)
+        if bad:
+            v[:] = np.abs(v) + 0.5
+            v[T // 2, 0, 7] = 1.0                       # (a value bf16 holds: its lower parts are zero)
+            k[T // 2, 0, 3], v[T - 1, H - 1, 9] = np.inf, -np.inf
+            k[T - 1] = np.abs(k[T - 1]) + 0.5
+        zi, zf = rows[:, n_qkv:n_qkv + H].astype(np.float64), rows[:, n_qkv + H:n_qkv + 2 * H].astype(np.float64)
+        spec = MLSTM()
+        spec.H, spec.dim, spec.vdim, spec.DP, spec.VP = H, D, V, D, V
+        spec.gate_cap, spec.ld_row, spec.k_offset, spec.v_offset, spec.i_offset, spec.f_offset = 15.0, ld, H * D, 2 * H * D, n_qkv, n_qkv + H
+        state = np.zeros(int(L.dh_mlstm_state_bytes(ctypes.byref(spec))) // 4, np.float32)
+        S, n, m = state[:H * D * V].reshape(H, D, V), state[H * D * V:H * D * (V + 2)].reshape(2, H, D), state[H * D * (V + 2):][:2 * H].reshape(2, H)
+        if start:
+            S[:], n[start & 1], m[start & 1] = g.standard_normal(S.shape), g.standard_normal((H, D)), 0.5
+        want_S, want_n, mm = S.astype(np.float64), n[start & 1].astype(np.float64), m[start & 1].astype(np.float64)
+        for t in range(T):
+            i, f = 15 * np.tanh(zi[t] / 15), 15 * np.tanh(zf[t] / 15)
+            f = np.minimum(f, 0) - np.log1p(np.exp(-np.abs(f)))
+            to = np.maximum(f + mm, i)
+            keep, put, mm = np.exp(f + mm - to), np.exp(i - to), to
+            want_n = keep[:, None] * want_n + put[:, None] * k[t]
+            want_S = keep[:, None, None] * want_S + put[:, None, None] * k[t][:, :, None].astype(np.float64) * v[t][:, None, :]
+        dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+        d_rows, d_state, out = dev(rows), dev(state), torch.zeros(T * H * V, device="cuda")
+        ws = torch.zeros(int(L.dh_mlstm_prefill_workspace_bytes(ctypes.byref(spec), T)), dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_mlstm_prefill(ctypes.byref(spec), d_rows.data_ptr(), d_state.data_ptr(), ws.data_ptr(), out.data_ptr(), H * V, T, start))
+        capi.check(L.dh_sync())
+        got = d_state.cpu().numpy()
+        for name, a, b in (("S", got[:H * D * V].reshape(H, D, V), want_S), ("n", got[H * D * V:H * D * (V + 2)].reshape(2, H, D)[(start + T) & 1], want_n)):
+            assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b)) and np.array_equal(a[np.isinf(b)], b[np.isinf(b)]), (name, bad)
+            fin = np.isfinite(b)
+            assert np.abs(a[fin] - b[fin]).max() <= 64 * 2.0 ** -24 * max(1.0, np.abs(b[fin]).max()) * 4, (name, bad)
+
+
 def test_more_heads_than_the_fused_output_product_takes(L, tmp_path):
     x = rng(10).standard_normal((70, 40))
     for dtype in DTYPES:

@@ -7,15 +7,6 @@ namespace dh {
 // An f32 is the exact sum of three bf16: its upper 16 bits, those of what remains, and the rest (8 + 8 + 8 significand bits; what a
 // subtraction leaves fits the next).  A product of two bf16 is exact in f32, so three bf16 instructions give what an f32 one gives of an
 // activation and a bf16 weight, in 3 x 32 cycles for 16 k against 8 x 64.  Of a pair of values the words hold (first, second).
-__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& high, uint32_t& mid, uint32_t& low) {
-  const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
-  const float r0 = x0 - __uint_as_float(u0 & 0xffff0000u), r1 = x1 - __uint_as_float(u1 & 0xffff0000u);
-  const uint32_t v0 = __float_as_uint(r0), v1 = __float_as_uint(r1);
-  const float q0 = r0 - __uint_as_float(v0 & 0xffff0000u), q1 = r1 - __uint_as_float(v1 & 0xffff0000u);
-  high = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-  mid = __builtin_amdgcn_perm(v1, v0, 0x07060302u);
-  low = __builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
-}
 struct SplitWords {
   u32x4_t high, mid, low;
 };
@@ -23,11 +14,14 @@ __device__ __forceinline__ SplitWords split_words(const f32x4_t& a, const f32x4_
   SplitWords s;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    uint32_t h, m, l;
-    split_pair(i < 2 ? a[2 * i] : b[2 * i - 4], i < 2 ? a[2 * i + 1] : b[2 * i - 3], h, m, l);
-    s.high[i] = h;
-    s.mid[i] = m;
-    s.low[i] = l;
+    const float x0 = i < 2 ? a[2 * i] : b[2 * i - 4], x1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+    const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+    const float r0 = x0 - __uint_as_float(u0 & 0xffff0000u), r1 = x1 - __uint_as_float(u1 & 0xffff0000u);
+    const uint32_t v0 = __float_as_uint(r0), v1 = __float_as_uint(r1);
+    const float q0 = r0 - __uint_as_float(v0 & 0xffff0000u), q1 = r1 - __uint_as_float(v1 & 0xffff0000u);
+    s.high[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+    s.mid[i] = __builtin_amdgcn_perm(v1, v0, 0x07060302u);
+    s.low[i] = __builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
   }
   return s;
 }

@@ -14,17 +14,18 @@
 // masked product inside it:
 //
 //   mlstm_gates_kernel     F, i, m of every token; one workgroup per head
-//   mlstm_states_kernel    the state in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + what chunk c adds,
-//                          sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T; a workgroup a tile of the state
+//   mlstm_chunks_kernel    what every chunk adds to the state behind it, sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T: independent of
+//                          one another, because m is known
+//   mlstm_scan_kernel      the state in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + what chunk c adds,
+//                          element by element and in place
 //   mlstm_outputs_kernel   o of (chunk, head, value columns): Q K^T and Q S in one walk over dim, decay mask, then (Q K^T) V
 //
-// the outputs on the 32-bit matrix-core instruction v_mfma_f32_32x32x2_f32.  head_norm_gate_kernel then divides every head's output by its root
+// on the 32-bit matrix-core instruction v_mfma_f32_32x32x2_f32.  head_norm_gate_kernel then divides every head's output by its root
 // mean square and applies the weight and the output gate.
 #include <algorithm>
 #include <cfloat>
 
 #include "dense_device.h"
-#include "gemm_split.h"
 
 namespace {
 
@@ -33,8 +34,6 @@ using dh::f32x4_t;
 
 constexpr int kChunk = 64;           // tokens per chunk
 constexpr int kCols = 32;            // value columns per workgroup of a step
-constexpr int kStateCols = 32;       // value columns of a workgroup's tile of the state
-constexpr int kStateLds = 2 * 3 * (64 + kStateCols) * 2 * kChunk + 4096;
 constexpr float kDenominatorEps = 1e-6f;
 
 struct MemArgs {
@@ -54,7 +53,6 @@ struct MemArgs {
   float* mt;               // m after every token
   float* mc;               // [H][chunks + 1] m in front of every chunk, and at the end
   float* keep;             // [H][chunks] what a chunk leaves of the state in front of it
-  float* wt;               // [H][T] what a token's k v^T counts in the state behind its chunk
   float* Sc;               // [chunks + 1][H][DP][VP]
   float* nc;               // [chunks + 1][H][DP]
 };
@@ -177,174 +175,94 @@ __global__ __launch_bounds__(1024) void mlstm_gates_kernel(const MemArgs a) {
     const double start = c > 0 ? F[c * kChunk - 1] : 0.0, end = F[min((c + 1) * kChunk, a.T) - 1];
     a.keep[(int64_t)h * a.chunks + c] = expf((float)(end - start + (double)mc[c] - (double)mc[c + 1]));
   }
-  for (int t = tid; t < a.T; t += 1024) {
-    const int c = t / kChunk;
-    a.wt[(int64_t)h * a.T + t] = expf((float)(F[min((c + 1) * kChunk, a.T) - 1] - F[t] + (double)li[t] - (double)mc[c + 1]));
+}
+
+// Grid = (64 x 64 tiles of a head's state, heads, chunks); wave w: rows 32 (w >> 1), columns 32 (w & 1) of the tile.
+__global__ __launch_bounds__(256) void mlstm_chunks_kernel(const MemArgs a) {
+  constexpr int ROW = 64 + 4;
+  __shared__ __align__(16) float ks[kChunk * ROW];     // weighted keys [token][dim]
+  __shared__ __align__(16) float vs[kChunk * ROW];     // values [token][column]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y, c = blockIdx.z;
+  const int tiles_v = (a.VP + 63) / 64, d0 = 64 * (blockIdx.x / tiles_v), v0 = 64 * (blockIdx.x % tiles_v);
+  const double* F = a.F + (int64_t)h * a.T;
+  const int first = c * kChunk, count = min(kChunk, a.T - first);
+  const double F_end = F[first + count - 1];
+  const float m_end = a.mc[(int64_t)h * (a.chunks + 1) + c + 1];
+  f32x4_t kr[4], vr[4];
+  float w[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int p = tid + 256 * r, tok = first + min(p >> 4, count - 1), x = 4 * (p & 15);
+    const float* row = a.rows + (int64_t)tok * a.ld_row;
+    kr[r] = vr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (d0 + x < a.DP) kr[r] = *reinterpret_cast<const f32x4_t*>(row + a.k_off + (int64_t)h * a.DP + d0 + x);
+    if (v0 + x < a.VP) vr[r] = *reinterpret_cast<const f32x4_t*>(row + a.v_off + (int64_t)h * a.VP + v0 + x);
+    w[r] = (p >> 4) < count ? expf((float)(F_end - F[tok] + (double)a.i[(int64_t)h * a.T + tok] - (double)m_end)) : 0.f;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int p = tid + 256 * r, tok = p >> 4, x = 4 * (p & 15);
+    // (rows past the last repeat it: an infinite one times a weight of zero is no number)
+    if ((p >> 4) < count) kr[r] *= w[r];
+    else kr[r] = vr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f32x4_t*>(&ks[tok * ROW + x]) = kr[r];
+    *reinterpret_cast<f32x4_t*>(&vs[tok * ROW + x]) = vr[r];
+  }
+  __syncthreads();
+  const int wd = 32 * (wave >> 1), wv = 32 * (wave & 1);
+  if (d0 + wd < a.DP && v0 + wv < a.VP) {              // wave-uniform (sizes are multiples of 32)
+    f32x16_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+#pragma unroll 8
+    for (int j = 0; j < kChunk / 2; j++) {
+      const int tok = 2 * j + (lane >> 5);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[tok * ROW + wd + (lane & 31)], vs[tok * ROW + wv + (lane & 31)], acc, 0, 0, 0);
+    }
+    // accumulator element e of a lane: state row 8 (e / 4) + 4 (lane >> 5) + e % 4, column lane & 31
+    float* U = a.Sc + ((int64_t)(c + 1) * a.H + h) * a.DP * a.VP + (int64_t)(d0 + wd + 4 * (lane >> 5)) * a.VP + v0 + wv + (lane & 31);
+#pragma unroll
+    for (int e = 0; e < 16; e++) U[(int64_t)(8 * (e >> 2) + (e & 3)) * a.VP] = acc[e];
+  }
+  if (v0 == 0 && tid < 64 && d0 + tid < a.DP) {
+    float s = 0.f;
+#pragma unroll 8
+    for (int t = 0; t < kChunk; t++) s += ks[t * ROW + tid];
+    a.nc[((int64_t)(c + 1) * a.H + h) * a.DP + d0 + tid] = s;
   }
 }
 
-// Grid = 64 x 32 tiles of the heads' states: a workgroup walks the chunks with its tile in registers; wave w: rows 16 (w & 3), columns
-// 16 (w >> 2).
-// What a chunk adds is a product of f32 operands, each the sum of three bf16 (gemm_split.h): of the nine products of parts the six that
-// reach f32's last bit, on v_mfma_f32_16x16x32_bf16 in 192 cycles where v_mfma_f32_32x32x2_f32 takes 512.  Operands lie in LDS along the
-// tokens, one plane a part: a row's 16-byte piece p (tokens 8 p .. 8 p + 7) at slot p ^ key(row), which spreads fragment reads over all
-// banks and the writes over half of them.  The next chunk's rows are loaded while this one is multiplied.
-// Bound by that chain, 1.4 us a chunk: about 250 instructions a wave, two waves on a SIMD (deeper prefetch, wider or conflict-free LDS traffic
-// and scalar addressing changed nothing; four waves took 2.2 us).  1531 tokens, 4 heads of 256 x 512: 36 us; before, each chunk's sum by
-// itself (38 us, 50 MB written) and a scan over them (18 us, 100 MB).
-__global__ __launch_bounds__(512) void mlstm_states_kernel(const MemArgs a) {
-  constexpr int KB = 64 * 2 * kChunk, VB = kStateCols * 2 * kChunk;    // bytes of a plane
-  static_assert(kStateLds == 2 * 3 * (KB + VB) + 2 * 8 * 64 * 4, "the launch's");
-  extern __shared__ __align__(16) char smem[];         // two chunks' planes of the keys and of the values, sums of keys
-  float* const nsums = reinterpret_cast<float*>(smem + 2 * 3 * (KB + VB));
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // tiles of a head, which read the same rows, on as few compute dies as hold them
-  const int tiles_v = a.VP / kStateCols, tiles = (a.DP + 63) / 64 * tiles_v, place_at = dh::xcd_contiguous(blockIdx.x, gridDim.x);
-  const int h = __builtin_amdgcn_readfirstlane(place_at / tiles), d0 = 64 * (place_at % tiles / tiles_v), v0 = kStateCols * (place_at % tiles_v);
-  const float* keep = a.keep + (int64_t)h * a.chunks;
-  const float* wt = a.wt + (int64_t)h * a.T;
-  auto key = [](int row) { return ((row >> 1) ^ (row >> 4)) & 7; };
-  // a thread's share of a chunk: two tokens, four dims of the keys and two columns of the values (dims past the last repeat: no wave
-  // multiplies them)
-  const int dq = 4 * (tid & 15), cq = 2 * (tid & 15), tp = tid >> 4, kd = min(d0 + dq, a.DP - 4);
-  const float* k_at = a.rows + a.k_off + (int64_t)h * a.DP + kd;
-  const float* v_at = a.rows + a.v_off + (int64_t)h * a.VP + v0 + cq;
-  struct Loads {
-    f32x4_t k[2];
-    float2 v[2];
-    float w[2], kept;
-  } x;
-  auto load = [&](int c) {
-    x.kept = keep[c];
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-      const int tok = min(c * kChunk + 2 * tp + r, a.T - 1);
-      x.w[r] = wt[tok];
-      x.k[r] = *reinterpret_cast<const f32x4_t*>(k_at + (int64_t)tok * a.ld_row);
-      x.v[r] = *reinterpret_cast<const float2*>(v_at + (int64_t)tok * a.ld_row);
-    }
-  };
-  const int wd = 16 * (wave & 3), wv = 16 * (wave >> 2);
-  const int row = d0 + wd + 4 * (lane >> 4), col = v0 + wv + (lane & 15);       // of accumulator element 0
-  const bool live = d0 + wd < a.DP;                    // (sizes are multiples of 32)
-  float* S = a.S + (int64_t)h * a.DP * a.VP + (int64_t)row * a.VP + col;
-  const bool sums = v0 == 0 && tid < 64 && d0 + tid < a.DP;
+// Grid = (groups of 1024 elements of a head's [S | n], heads), four per thread; slot 0 of Sc and nc is filled here.
+__global__ __launch_bounds__(256) void mlstm_scan_kernel(const MemArgs a) {
+  constexpr int AHEAD = 16;
+  const int h = blockIdx.y, size = a.DP * a.VP;
+  const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (i >= size + a.DP) return;
+  const bool is_n = i >= size;
+  const int64_t stride = is_n ? (int64_t)a.H * a.DP : (int64_t)a.H * size;
+  float* at = is_n ? a.nc + (int64_t)h * a.DP + (i - size) : a.Sc + (int64_t)h * size + i;
   const int64_t slots = (int64_t)a.H * a.DP;
+  const float* from = is_n ? a.n + (a.pos & 1) * slots + (int64_t)h * a.DP + (i - size) : a.S + (int64_t)h * size + i;
+  float* to = is_n ? a.n + ((a.pos + a.T) & 1) * slots + (int64_t)h * a.DP + (i - size) : a.S + (int64_t)h * size + i;
+  const float* keep = a.keep + (int64_t)h * a.chunks;
   f32x4_t s = {0.f, 0.f, 0.f, 0.f};
-  float n = 0.f;
-  if (a.pos > 0) {
-    if (live)
+  if (a.pos > 0) s = *reinterpret_cast<const f32x4_t*>(from);
+  *reinterpret_cast<f32x4_t*>(at) = s;
+  for (int c0 = 0; c0 < a.chunks; c0 += AHEAD) {
+    f32x4_t u[AHEAD];
 #pragma unroll
-      for (int e = 0; e < 4; e++) s[e] = S[(int64_t)e * a.VP];
-    if (sums) n = a.n[(a.pos & 1) * slots + (int64_t)h * a.DP + d0 + tid];
+    for (int k = 0; k < AHEAD; k++)
+      if (c0 + k < a.chunks) u[k] = *reinterpret_cast<const f32x4_t*>(at + (c0 + k + 1) * stride);
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+      const int c = c0 + k;
+      if (c < a.chunks) {
+        s = s * keep[c] + u[k];
+        if (c + 1 < a.chunks) *reinterpret_cast<f32x4_t*>(at + (c + 1) * stride) = s;
+      }
+    }
   }
-  // a chunk's operands into LDS
-  auto place = [&](int c) {
-    const int count = min(kChunk, a.T - c * kChunk);
-    char* const ks = smem + (c & 1) * 3 * (KB + VB);
-    char* const vs = ks + 3 * KB;
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) x.k[r][e] = 2 * tp + r < count ? x.k[r][e] * x.w[r] : 0.f;      // (rows past the last repeat it)
-    if (v0 == 0) {
-      f32x4_t part = x.k[0] + x.k[1];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        part[e] += __shfl_xor(part[e], 16, 64);
-        part[e] += __shfl_xor(part[e], 32, 64);
-      }
-      if (lane < 16) *reinterpret_cast<f32x4_t*>(nsums + ((c & 1) * 8 + wave) * 64 + dq) = part;
-    }
-    const int piece = tp >> 2, word = 4 * (tp & 3);
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      uint32_t w[3];
-      dh::split_pair(x.k[0][e], x.k[1][e], w[0], w[1], w[2]);
-      char* at = ks + (dq + e) * 128 + 16 * (piece ^ key(dq + e)) + word;
-#pragma unroll
-      for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t*>(at + p * KB) = w[p];
-    }
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-      uint32_t w[3];
-      dh::split_pair(e ? x.v[0].y : x.v[0].x, e ? x.v[1].y : x.v[1].x, w[0], w[1], w[2]);
-      char* at = vs + (cq + e) * 128 + 16 * (piece ^ key(cq + e)) + word;
-#pragma unroll
-      for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t*>(at + p * VB) = w[p];
-    }
-  };
-  auto chunk = [&](int c, float kept) {
-    const int first = c * kChunk, count = min(kChunk, a.T - first);
-    const char* const ks = smem + (c & 1) * 3 * (KB + VB);
-    const char* const vs = ks + 3 * KB;
-    // the state in front of the chunk
-    if (live) {
-      float* at = a.Sc + ((int64_t)c * a.H + h) * a.DP * a.VP + (int64_t)row * a.VP + col;
-#pragma unroll
-      for (int e = 0; e < 4; e++) at[(int64_t)e * a.VP] = s[e];
-      f32x4_t sum = {0.f, 0.f, 0.f, 0.f}, rest = sum;
-#pragma unroll
-      for (int k = 0; k < kChunk / 32; k++) {
-        const int d = wd + (lane & 15), v = wv + (lane & 15), at8 = 4 * k + (lane >> 4);
-        dh::bf16x8_t fa[3], fb[3];
-#pragma unroll
-        for (int p = 0; p < 3; p++) {
-          fa[p] = *reinterpret_cast<const dh::bf16x8_t*>(ks + p * KB + d * 128 + 16 * (at8 ^ key(d)));
-          fb[p] = *reinterpret_cast<const dh::bf16x8_t*>(vs + p * VB + v * 128 + 16 * (at8 ^ key(v)));
-        }
-        // parts 0, 1, 2: high, mid, low; the small products are added up by themselves
-        rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[2], fb[0], rest, 0, 0, 0);
-        rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0], fb[2], rest, 0, 0, 0);
-        rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[1], fb[1], rest, 0, 0, 0);
-        rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[1], fb[0], rest, 0, 0, 0);
-        rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0], fb[1], rest, 0, 0, 0);
-        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[0], fb[0], sum, 0, 0, 0);
-      }
-      sum += rest;
-      bool sound = true;
-#pragma unroll
-      for (int e = 0; e < 4; e++) sound = sound && fabsf(sum[e]) <= FLT_MAX;
-      // the parts of an infinite value, and a part that is zero times one, are no numbers: such sums are made again by themselves
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!sound) != 0ull, 0)) {
-        sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-        for (int t = first; t < first + count; t++) {
-          const float* r = a.rows + (int64_t)t * a.ld_row;
-          const float w = wt[t], v = r[a.v_off + (int64_t)h * a.VP + col];
-#pragma unroll
-          for (int e = 0; e < 4; e++) sum[e] = fmaf(r[a.k_off + (int64_t)h * a.DP + row + e] * w, v, sum[e]);
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 4; e++) s[e] = fmaf(kept, s[e], sum[e]);
-    }
-    if (sums) {
-      a.nc[((int64_t)c * a.H + h) * a.DP + d0 + tid] = n;
-      float u = 0.f;
-#pragma unroll
-      for (int t = 0; t < 8; t++) u += nsums[((c & 1) * 8 + t) * 64 + tid];
-      n = fmaf(kept, n, u);
-    }
-  };
-  // while a chunk is multiplied, the next one is placed and the one after that is on its way
-  load(0);
-  place(0);
-  float kept = x.kept;
-  load(min(1, a.chunks - 1));
-  __syncthreads();
-  for (int c = 0; c < a.chunks; c++) {
-    const float next = x.kept;
-    if (c + 1 < a.chunks) place(c + 1);
-    load(min(c + 2, a.chunks - 1));
-    chunk(c, kept);
-    kept = next;
-    __syncthreads();
-  }
-  if (live)
-#pragma unroll
-    for (int e = 0; e < 4; e++) S[(int64_t)e * a.VP] = s[e];
-  if (sums) a.n[((a.pos + a.T) & 1) * slots + (int64_t)h * a.DP + d0 + tid] = n;
+  *reinterpret_cast<f32x4_t*>(to) = s;
 }
 
 // Grid = (chunks, heads, groups of 64 TN value columns); wave w: tokens 32 (w >> 1), columns 32 TN (w & 1) + 0 .. 32 TN - 1.
@@ -580,7 +498,7 @@ int dh_mlstm_step(const dh_mlstm* spec, const float* d_row, void* d_state, float
 size_t dh_mlstm_prefill_workspace_bytes(const dh_mlstm* s, int T) {
   if (!s || T <= 0) return 256;
   const size_t chunks = (size_t)dh::ceil_div(T, kChunk), HT = (size_t)s->H * T;
-  return up256(HT * 8) + 3 * up256(HT * 4) + 2 * up256((size_t)s->H * (chunks + 1) * 4) + up256((chunks + 1) * s->H * s->DP * 4) +
+  return up256(HT * 8) + 2 * up256(HT * 4) + 2 * up256((size_t)s->H * (chunks + 1) * 4) + up256((chunks + 1) * s->H * s->DP * 4) +
          up256((chunks + 1) * s->H * s->DP * s->VP * 4);
 }
 
@@ -603,16 +521,16 @@ int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, v
   a.mt = reinterpret_cast<float*>(take(HT * 4));
   a.mc = reinterpret_cast<float*>(take((size_t)spec->H * (a.chunks + 1) * 4));
   a.keep = reinterpret_cast<float*>(take((size_t)spec->H * (a.chunks + 1) * 4));
-  a.wt = reinterpret_cast<float*>(take(HT * 4));
   a.nc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * 4));
   a.Sc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * spec->VP * 4));
   hipLaunchKernelGGL(mlstm_gates_kernel, dim3(spec->H), dim3(1024), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
+  const int tiles = (int)(dh::ceil_div(spec->DP, 64) * dh::ceil_div(spec->VP, 64));
   // the grid's third dimension holds at most 65535 chunks
   if (a.chunks > 65535) return dh::fail(1, "[%s] %d tokens are too many for one portion", op, T);
-  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(mlstm_states_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kStateLds);
-  DH_CHECK_HIP(op, set);
-  hipLaunchKernelGGL(mlstm_states_kernel, dim3((unsigned)(dh::ceil_div(spec->DP, 64) * (spec->VP / kStateCols) * spec->H)), dim3(512), kStateLds, dh::stream(), a);
+  hipLaunchKernelGGL(mlstm_chunks_kernel, dim3(tiles, spec->H, a.chunks), dim3(256), 0, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  hipLaunchKernelGGL(mlstm_scan_kernel, dim3((unsigned)dh::ceil_div((int64_t)spec->DP * spec->VP + spec->DP, 1024), spec->H), dim3(256), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   // wide column groups repeat Q K^T less often; narrow ones where those would not fill the device
   const bool wide = spec->VP > 64 && (int64_t)a.chunks * spec->H * dh::ceil_div(spec->VP, 128) >= dh::num_cus();

@@ -207,6 +207,40 @@ def test_memory_state_behind_a_prompt(L, H, D, V, T, start):
             assert np.abs(a[fin] - b[fin]).max() <= 64 * 2.0 ** -24 * max(1.0, np.abs(b[fin]).max()) * 4, (name, bad)
 
 
+@pytest.mark.parametrize("live,before", [(1, 0), (2, 0), (4, 0), (1, 64)])
+def test_memory_state_of_few_live_tokens(L, live, before):
+    """A chunk that few tokens count in (a portion of one, two or four tokens, and one whose last token closes the forget gate over 64 others)
+    has few roundings: a weight's (at most 2^-23; that of the last token is exp(0)), the weighted key's, the product's and one a sum, so (3 + live)
+    * 2^-24 of the terms, and 2 * 2^-24 for a single token."""
+    from doppler_amd.capi import MLSTM
+    H, D, V, T = 2, 256, 512, before + live
+    g = rng(310 + live + before)
+    n_qkv, ld = H * (2 * D + V), H * (2 * D + V) + 2 * H
+    rows = g.standard_normal((T, ld)).astype(np.float32)
+    rows[:, n_qkv:n_qkv + H], rows[:, n_qkv + H:] = 0.0, 1e3        # i = 0, f = log of sigmoid(15)
+    if before:
+        rows[before, n_qkv + H:] = -1e3                             # f = log of sigmoid(-15)
+    k, v = rows[:, H * D:2 * H * D].reshape(T, H, D).astype(np.float64), rows[:, 2 * H * D:n_qkv].reshape(T, H, V).astype(np.float64)
+    spec = MLSTM()
+    spec.H, spec.dim, spec.vdim, spec.DP, spec.VP = H, D, V, D, V
+    spec.gate_cap, spec.ld_row, spec.k_offset, spec.v_offset, spec.i_offset, spec.f_offset = 15.0, ld, H * D, 2 * H * D, n_qkv, n_qkv + H
+    S, terms, m = np.zeros((H, D, V)), np.zeros((H, D, V)), 0.0
+    for t in range(T):
+        f = -15.0 - np.log1p(np.exp(-15.0)) if before and t == before else -np.log1p(np.exp(-15.0))
+        to = max(f + m, 0.0)
+        kv = k[t][:, :, None] * v[t][:, None, :]
+        S, terms, m = np.exp(f + m - to) * S + np.exp(-to) * kv, np.exp(f + m - to) * terms + np.exp(-to) * np.abs(kv), to
+    d_rows, out = torch.from_numpy(rows).cuda(), torch.zeros(T * H * V, device="cuda")
+    state = torch.zeros(int(L.dh_mlstm_state_bytes(ctypes.byref(spec))) // 4, device="cuda")
+    ws = torch.zeros(int(L.dh_mlstm_prefill_workspace_bytes(ctypes.byref(spec), T)), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_mlstm_prefill(ctypes.byref(spec), d_rows.data_ptr(), state.data_ptr(), ws.data_ptr(), out.data_ptr(), H * V, T, 0))
+    capi.check(L.dh_sync())
+    got = state.cpu().numpy()[:H * D * V].reshape(H, D, V).astype(np.float64)
+    worst = (np.abs(got - S) / terms).max()
+    assert worst <= (2 if live == 1 else 3 + live) * 2.0 ** -24, worst * 2.0 ** 24
+
+
 def test_more_heads_than_the_fused_output_product_takes(L, tmp_path):
     x = rng(10).standard_normal((70, 40))
     for dtype in DTYPES:

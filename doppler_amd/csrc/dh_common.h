@@ -21,10 +21,14 @@ constexpr int kWave = 64;
 // Records a message for dh_last_error() and returns the code to hand back to the caller.
 int fail(int code, const char* fmt, ...);
 hipStream_t stream();
-// Around a launch that uses the library's one exchange area (q4k_gemv_chain.hip): launches of several streams (dh_set_stream) follow one
-// another.
-int exchange_begin(const char* op);
-int exchange_end(const char* op);
+// Memory that launches of every stream share and that is theirs for the length of a launch: the exchange of chained products
+// (q4k_gemv_chain.hip), the sums of slices of few-row products (q4k_gemv_rows.hip).  Around the launches that use one: those of several streams
+// (dh_set_stream) follow one another.
+enum Area { kExchangeArea, kSlicesArea, kAreas };
+int area_begin(const char* op, Area area);
+int area_end(const char* op, Area area);
+// Whether the op stream is being captured into a graph that is not the library's (dh_graph_begin): replays of it follow nothing.
+bool foreign_capture();
 bool ready();
 int num_cus();
 // Scratch for the split-K prefill GEMM's partial products (allocated by dh_init, shared by all

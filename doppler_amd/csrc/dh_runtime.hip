@@ -11,8 +11,10 @@ bool g_ready = false;
 int g_device = -1;
 hipStream_t g_own_stream = nullptr;
 hipStream_t g_stream = nullptr;
-hipStream_t g_exchange_stream = nullptr;    // where the last launch that uses the library's exchange area went
-hipEvent_t g_exchange_event = nullptr;      // behind it (on the library's own stream: recorded when that is left)
+struct LastUse {
+  hipStream_t stream;                 // where the last launch that uses the area went
+  hipEvent_t event;                   // behind it (on the library's own stream: recorded when that is left)
+} g_areas[dh::kAreas];
 int g_num_cus = 0;
 constexpr int kMaxFamilies = 16;
 dh::Family g_families[kMaxFamilies];  // filled while the library is being loaded (zero-initialised before that)
@@ -63,16 +65,18 @@ static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
-int exchange_begin(const char* op) {
-  if (g_exchange_stream && g_exchange_stream != g_stream && !capturing(g_stream)) DH_CHECK_HIP(op, hipStreamWaitEvent(g_stream, g_exchange_event, 0));
+int area_begin(const char* op, Area area) {
+  const LastUse& last = g_areas[area];
+  if (last.stream && last.stream != g_stream && !capturing(g_stream)) DH_CHECK_HIP(op, hipStreamWaitEvent(g_stream, last.event, 0));
   return 0;
 }
-int exchange_end(const char* op) {
-  g_exchange_stream = g_stream;
+int area_end(const char* op, Area area) {
+  g_areas[area].stream = g_stream;
   // (a stream of the caller's may be gone by the time another one is set)
-  if (g_stream != g_own_stream && !capturing(g_stream)) DH_CHECK_HIP(op, hipEventRecord(g_exchange_event, g_stream));
+  if (g_stream != g_own_stream && !capturing(g_stream)) DH_CHECK_HIP(op, hipEventRecord(g_areas[area].event, g_stream));
   return 0;
 }
+bool foreign_capture() { return !g_capturing && capturing(g_stream); }
 bool ready() { return g_ready || t_plan_cus > 0; }
 int num_cus() { return t_plan_cus > 0 ? t_plan_cus : g_num_cus; }
 void plan_begin(int cus) {
@@ -174,9 +178,10 @@ static int release_all(const char* op) {
     delete g_capturing;
     g_capturing = nullptr;
   }
-  if (g_exchange_event) note(hipEventDestroy(g_exchange_event));
-  g_exchange_event = nullptr;
-  g_exchange_stream = nullptr;
+  for (LastUse& last : g_areas) {
+    if (last.event) note(hipEventDestroy(last.event));
+    last = LastUse{};
+  }
   if (g_own_stream) note(hipStreamDestroy(g_own_stream));
   if (g_splitk_ws) note(hipFree(g_splitk_ws));
   if (g_row_scale) note(hipFree(g_row_scale));
@@ -214,7 +219,7 @@ static int init_locked(int device_ordinal) {
                     prop.gcnArchName);
   DH_CHECK_HIP("dh_init", hipStreamCreateWithFlags(&g_own_stream, hipStreamDefault));
   g_stream = g_own_stream;
-  DH_CHECK_HIP("dh_init", hipEventCreateWithFlags(&g_exchange_event, hipEventDisableTiming));
+  for (LastUse& last : g_areas) DH_CHECK_HIP("dh_init", hipEventCreateWithFlags(&last.event, hipEventDisableTiming));
   g_num_cus = prop.multiProcessorCount;
   DH_CHECK_HIP("dh_init", hipMalloc(reinterpret_cast<void**>(&g_splitk_ws), kSplitKWsBytes));
   DH_CHECK_HIP("dh_init", hipMalloc(reinterpret_cast<void**>(&g_row_scale), (size_t)kRowScaleRows * 2 * sizeof(float)));
@@ -261,8 +266,8 @@ int dh_set_stream(void* hip_stream) {
   DH_REQUIRE_INIT("dh_set_stream");
   if (g_capturing) return dh::fail(1, "[dh_set_stream] not possible while a graph is being captured (the capture belongs to the current stream)");
   hipStream_t next = hip_stream ? static_cast<hipStream_t>(hip_stream) : g_own_stream;
-  if (next != g_stream && g_stream == g_own_stream && g_exchange_stream == g_own_stream)
-    DH_CHECK_HIP("dh_set_stream", hipEventRecord(g_exchange_event, g_own_stream));
+  for (LastUse& last : g_areas)
+    if (next != g_stream && g_stream == g_own_stream && last.stream == g_own_stream) DH_CHECK_HIP("dh_set_stream", hipEventRecord(last.event, g_own_stream));
   g_stream = next;
   return 0;
 }
@@ -438,7 +443,8 @@ int dh_graph_begin(void) {
   DH_REQUIRE_INIT("dh_graph_begin");
   if (g_capturing) return dh::fail(1, "[dh_graph_begin] a capture is already in progress");
   DH_CHECK_HIP("dh_graph_begin", hipStreamSynchronize(g_stream));
-  if (g_exchange_stream && g_exchange_stream != g_stream) DH_CHECK_HIP("dh_graph_begin", hipEventSynchronize(g_exchange_event));
+  for (const LastUse& last : g_areas)
+    if (last.stream && last.stream != g_stream) DH_CHECK_HIP("dh_graph_begin", hipEventSynchronize(last.event));
   g_capturing = new dh::Graph();
   const hipError_t e = hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) {
@@ -523,9 +529,12 @@ int dh_graph_launch(void* graph, int position) {
   if (position != g->position) {
     if (int rc = graph_move(g, position)) return rc;
   }
-  if (int rc = dh::exchange_begin("dh_graph_launch")) return rc;        // it may hold such launches
+  for (int i = 0; i < dh::kAreas; i++)        // it may hold such launches
+    if (int rc = dh::area_begin("dh_graph_launch", static_cast<dh::Area>(i))) return rc;
   DH_CHECK_HIP("dh_graph_launch", hipGraphLaunch(g->exec, g_stream));
-  return dh::exchange_end("dh_graph_launch");
+  for (int i = 0; i < dh::kAreas; i++)
+    if (int rc = dh::area_end("dh_graph_launch", static_cast<dh::Area>(i))) return rc;
+  return 0;
 }
 
 int dh_graph_prepare(void* graph, int position) {

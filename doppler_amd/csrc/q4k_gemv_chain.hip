@@ -910,10 +910,10 @@ int launch_slots(const char* op, Plan& plan, int workgroups) {
     attr_set = true;
   }
   if (!coresident) return dh::fail(1, "[%s] the device cannot hold one workgroup of the chain per compute unit", op);
-  if (int rc = dh::exchange_begin(op)) return rc;
+  if (int rc = dh::area_begin(op, dh::kExchangeArea)) return rc;
   hipLaunchKernelGGL(kern, dim3(workgroups), dim3(64 * kWaves), plan.lds, dh::stream(), plan.a);
   DH_CHECK_LAUNCH(op);
-  return dh::exchange_end(op);
+  return dh::area_end(op, dh::kExchangeArea);
 }
 int launch(const char* op, Plan& plan, int workgroups) {
   return plan.short_rows ? launch_slots<kSlotsShort>(op, plan, workgroups) : launch_slots<kSlots>(op, plan, workgroups);

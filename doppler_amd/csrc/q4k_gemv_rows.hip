@@ -563,6 +563,20 @@ __global__ __launch_bounds__(64 * kWaves, 1) void q4k_gemv_rows_kernel(const Row
 
 int env_int(const char* name, int dflt) { return dh::tuning_int(name, dflt); }
 
+// Sums of the slices of one launch.  Not the split-K workspace: its other users go by one stream's order alone, and products of few rows may
+// run beside them on another stream.
+constexpr size_t kSliceBytes = (size_t)32 << 20;
+float* g_slice_sums = nullptr;
+int rows_init(int) {
+  DH_CHECK_HIP("dh_init", hipMalloc(reinterpret_cast<void**>(&g_slice_sums), kSliceBytes));
+  return 0;
+}
+void rows_release() {
+  if (g_slice_sums) (void)hipFree(g_slice_sums);
+  g_slice_sums = nullptr;
+}
+const int g_family = dh::register_family({rows_init, rows_release, nullptr, nullptr, nullptr});
+
 // A launch for so many compute units: rows per tile, the largest count <= 16 that gives every workgroup the same number of tiles, and the
 // tiles dealt to workgroups.
 struct Deal {
@@ -584,9 +598,7 @@ Deal deal(int64_t N, int64_t cus) {
 int choose_slices(int64_t M, int64_t N, int64_t nb) {
   constexpr double kColumn = 4.0, kUnit = 0.7, kUnitRow = 1.3 / kTileRows, kSecondLaunch = 3.0;
   if (nb <= kWaves) return 1;
-  size_t bytes = 0;
-  (void)dh::splitk_workspace(&bytes);
-  const int most = (int)std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)bytes / (4 * M * N)));
+  const int most = (int)std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)kSliceBytes / (4 * M * N)));
   int best = 1;
   double least = 1e30;
   for (int s = 1; s <= most; s++) {
@@ -647,7 +659,9 @@ int launch_rows(RowsArgs a, const char* op) {
     for (int i = 0; i < 12; i++) dh::plan_layout(i, rec[i]);
   }
   if (dh::plan_note(DH_PLAN_GEMV_ROWS)) return 0;
+  // (a caller's own graph is replayed beside whatever it likes: it shares no memory with other launches)
   int slices = DUAL || a.norm_weight ? 1 : choose_slices(a.M, a.N, a.nb);
+  if (slices > 1 && dh::foreign_capture()) slices = 1;
   if (slices > 1) {
     lay_out(slices);
     a.depth = fit_depth();
@@ -669,13 +683,12 @@ int launch_rows(RowsArgs a, const char* op) {
     DH_CHECK_LAUNCH(op);
     return 0;
   }
-  size_t bytes = 0;
-  a.parts = dh::splitk_workspace(&bytes);
-  if (int rc = dh::exchange_begin(op)) return rc;
+  a.parts = g_slice_sums;
+  if (int rc = dh::area_begin(op, dh::kSlicesArea)) return rc;
   hipLaunchKernelGGL(kern, dim3(a.grid, slices), dim3(64 * kWaves), lds, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   if (int rc = dh::q4k_sum_slices(op, a.parts, slices, a.C, a.c_f16, a.M, a.N, a.alpha, a.residual)) return rc;
-  return dh::exchange_end(op);
+  return dh::area_end(op, dh::kSlicesArea);
 }
 
 }  // namespace

@@ -9,6 +9,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from doppler_amd import capi, ops, synth
@@ -104,6 +105,77 @@ def test_few_rows_of_many_columns(M, N, K, alpha, outputDtype, residual, f16):
         got = got.view(np.float16).astype(np.float32) if outputDtype == "f16" else got
         want = oracle.q4k_matmul(A.astype(np.float32), W, M, N, K, alpha)
         assert rel_l2(got, want + res if residual else want) <= 1e-5 + (5e-4 if outputDtype == "f16" else 0)
+
+
+def _q4k_products(*shapes):
+    """(weights, rows, output, call) of products M x N x K with f32 rows and outputs."""
+    L, made = capi.load(), []
+    for i, (M, N, K) in enumerate(shapes):
+        w = torch.from_numpy(synth.q4k_tensor(N, K, 1370 + i)).cuda()
+        a, out = torch.from_numpy(synth.normal_f32((M, K), 1380 + i)).cuda(), torch.zeros(M, N, device="cuda")
+        call = lambda w=w, a=a, out=out, M=M, N=N, K=K: capi.check(
+            L.dh_q4k_matmul(a.data_ptr(), capi.F32, w.data_ptr(), out.data_ptr(), capi.F32, M, N, K, 1.0, None))
+        made.append((w, a, out, call))
+    return made
+
+
+def test_products_of_few_rows_beside_prompts_on_other_streams():
+    """Sliced products of few rows on two streams and a prompt's products, cut along K, on the library's own: each as it is alone."""
+    L = capi.init(torch.cuda.current_device())
+    products = _q4k_products((32, 1024, 12288), (8, 4096, 12288), (5, 2048, 12288))
+    streams = [None, torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    alone = []
+    for _, _, out, call in products:
+        call()
+        capi.check(L.dh_sync())
+        alone.append(out.clone())
+    try:
+        for rep in range(5):
+            for _, _, out, _ in products:
+                out.zero_()
+            torch.cuda.synchronize()
+            for again in range(6):
+                for (_, _, _, call), stream in zip(products, streams):
+                    capi.check(L.dh_set_stream(stream.cuda_stream if stream else None))
+                    call()
+            torch.cuda.synchronize()
+            for i, (_, _, out, _) in enumerate(products):
+                assert torch.equal(out, alone[i]), (rep, i)
+    finally:
+        capi.check(L.dh_set_stream(None))
+
+
+def test_few_rows_in_a_graph_of_the_callers_beside_others():
+    """Replays of a product that a caller captured run beside sliced products on another stream: it is one launch that shares no memory."""
+    L = capi.init(torch.cuda.current_device())
+    (_, _, captured, capture), (_, _, other, beside) = _q4k_products((8, 4096, 12288), (5, 4096, 12288))
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    capture()
+    beside()
+    capi.check(L.dh_sync())
+    eager, alone = captured.clone(), other.clone()
+    try:
+        capi.check(L.dh_set_stream(stream.cuda_stream))
+        with torch.cuda.graph(graph, stream=stream):
+            capture()
+    finally:
+        capi.check(L.dh_set_stream(None))
+    want = None
+    for rep in range(5):
+        captured.zero_()
+        other.zero_()
+        torch.cuda.synchronize()
+        for again in range(4):
+            with torch.cuda.stream(stream):
+                graph.replay()
+            beside()
+        torch.cuda.synchronize()
+        want = captured.clone() if want is None else want
+        assert torch.equal(captured, want) and torch.equal(other, alone), rep
+    # sums in another order: 1e-5 as the products above
+    assert float((want.double() - eager.double()).norm() / eager.double().norm()) <= 1e-5
 
 
 @pytest.mark.parametrize("M,N,K,outputDtype,residual", [

@@ -65,15 +65,19 @@ static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
+// A launch that is captured uses nothing yet: it neither waits nor is waited for.
 int area_begin(const char* op, Area area) {
   const LastUse& last = g_areas[area];
-  if (last.stream && last.stream != g_stream && !capturing(g_stream)) DH_CHECK_HIP(op, hipStreamWaitEvent(g_stream, last.event, 0));
+  // (a stream of the caller's may be gone, and its handle another stream's by now: only the library's own is known to be the same one)
+  if (last.stream && (last.stream != g_stream || g_stream != g_own_stream) && !capturing(g_stream))
+    DH_CHECK_HIP(op, hipStreamWaitEvent(g_stream, last.event, 0));
   return 0;
 }
 int area_end(const char* op, Area area) {
-  g_areas[area].stream = g_stream;
-  // (a stream of the caller's may be gone by the time another one is set)
-  if (g_stream != g_own_stream && !capturing(g_stream)) DH_CHECK_HIP(op, hipEventRecord(g_areas[area].event, g_stream));
+  LastUse& last = g_areas[area];
+  if ((last.stream == g_stream && g_stream == g_own_stream) || capturing(g_stream)) return 0;
+  last.stream = g_stream;
+  if (g_stream != g_own_stream) DH_CHECK_HIP(op, hipEventRecord(last.event, g_stream));
   return 0;
 }
 bool foreign_capture() { return !g_capturing && capturing(g_stream); }

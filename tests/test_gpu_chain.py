@@ -397,3 +397,38 @@ def test_chains_of_several_streams_follow_one_another():
     finally:
         capi.check(L.dh_set_stream(None))
     capi.check(L.dh_sync())
+
+
+def test_a_captured_chain_is_not_the_last_one():
+    """Chains in flight on one stream, a chain that a caller captures on another, then one launched there: it still follows those in flight."""
+    L = capi.init(0)
+    lays = [Layer(4096, 12288, 4096, 6144, seed=7950), Layer(1024, 3072, 1024, 2048, seed=7980)]
+    arrs = [capi.chain_phases(l.phases()) for l in lays]
+    sep = [{k: torch.zeros_like(v) for k, v in l.out.items()} for l in lays]
+    for l, s in zip(lays, sep):
+        l.separate(L, s)
+    run = lambda i: capi.check(L.dh_q4k_gemv_chain_short(lays[i].d["attn"].data_ptr(), None, arrs[i], 4))
+    for i in range(2):
+        run(i)
+    capi.check(L.dh_sync())
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    for l in lays:
+        for t in l.out.values():
+            t.zero_()
+    torch.cuda.synchronize()
+    try:
+        for again in range(8):
+            run(0)
+        capi.check(L.dh_set_stream(stream.cuda_stream))
+        with torch.cuda.stream(stream):
+            graph.capture_begin(capture_error_mode="thread_local")
+            run(1)
+            graph.capture_end()
+        run(1)
+        torch.cuda.synchronize()
+    finally:
+        capi.check(L.dh_set_stream(None))
+    for i, l in enumerate(lays):
+        for k, v in l.out.items():
+            assert _read(v).tobytes() == _read(sep[i][k]).tobytes(), (i, k)
+    capi.check(L.dh_sync())

@@ -162,6 +162,7 @@ struct Graph {
   int n_attn = 0, cap_attn = 0;
   GraphFiniteCall* fin = nullptr;
   int n_fin = 0, cap_fin = 0;
+  unsigned areas = 0;                     // bit i: a captured launch uses Area i
 };
 // The graph being captured on the op stream, or null.
 Graph* capturing_graph();

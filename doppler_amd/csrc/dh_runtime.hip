@@ -65,8 +65,9 @@ static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
-// A launch that is captured uses nothing yet: it neither waits nor is waited for.
+// A launch that is captured uses nothing yet: it neither waits nor is waited for, and the graph notes what its launches will use.
 int area_begin(const char* op, Area area) {
+  if (g_capturing) g_capturing->areas |= 1u << area;
   const LastUse& last = g_areas[area];
   // (a stream of the caller's may be gone, and its handle another stream's by now: only the library's own is known to be the same one)
   if (last.stream && (last.stream != g_stream || g_stream != g_own_stream) && !capturing(g_stream))
@@ -447,8 +448,6 @@ int dh_graph_begin(void) {
   DH_REQUIRE_INIT("dh_graph_begin");
   if (g_capturing) return dh::fail(1, "[dh_graph_begin] a capture is already in progress");
   DH_CHECK_HIP("dh_graph_begin", hipStreamSynchronize(g_stream));
-  for (const LastUse& last : g_areas)
-    if (last.stream && last.stream != g_stream) DH_CHECK_HIP("dh_graph_begin", hipEventSynchronize(last.event));
   g_capturing = new dh::Graph();
   const hipError_t e = hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) {
@@ -533,11 +532,13 @@ int dh_graph_launch(void* graph, int position) {
   if (position != g->position) {
     if (int rc = graph_move(g, position)) return rc;
   }
-  for (int i = 0; i < dh::kAreas; i++)        // it may hold such launches
-    if (int rc = dh::area_begin("dh_graph_launch", static_cast<dh::Area>(i))) return rc;
+  for (int i = 0; i < dh::kAreas; i++)
+    if (g->areas >> i & 1)
+      if (int rc = dh::area_begin("dh_graph_launch", static_cast<dh::Area>(i))) return rc;
   DH_CHECK_HIP("dh_graph_launch", hipGraphLaunch(g->exec, g_stream));
   for (int i = 0; i < dh::kAreas; i++)
-    if (int rc = dh::area_end("dh_graph_launch", static_cast<dh::Area>(i))) return rc;
+    if (g->areas >> i & 1)
+      if (int rc = dh::area_end("dh_graph_launch", static_cast<dh::Area>(i))) return rc;
   return 0;
 }
 

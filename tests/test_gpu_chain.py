@@ -432,3 +432,53 @@ def test_a_captured_chain_is_not_the_last_one():
         for k, v in l.out.items():
             assert _read(v).tobytes() == _read(sep[i][k]).tobytes(), (i, k)
     capi.check(L.dh_sync())
+
+
+def test_graphs_without_shared_memory_run_beside_one_another():
+    """A graph of launches that share nothing ends while one launched on another stream, behind long work, is still waiting to begin."""
+    L = capi.init(0)
+    bufs, graphs = [torch.ones(64, device="cuda") for _ in range(2)], []
+    torch.cuda.synchronize()
+    for b in bufs:
+        capi.check(L.dh_graph_begin())
+        capi.check(L.dh_fill_zero(b.data_ptr(), 0, 256))
+        g = ctypes.c_void_p()
+        capi.check(L.dh_graph_end(0, ctypes.byref(g)))
+        graphs.append(g)
+    x = torch.zeros(8192, 8192, device="cuda")
+    long, side = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(4)]
+
+    def ends_first(stream, launch):
+        """launch(on the long stream), then on `stream`: whether the second ends while the long stream's work goes on"""
+        with torch.cuda.stream(long):
+            for _ in range(20):
+                torch.mm(x, x)             # some 10 ms each in f32
+        launch(0, long)
+        launch(1, stream)
+        done = torch.cuda.Event()
+        done.record(stream)
+        done.synchronize()
+        first = not long.query()
+        torch.cuda.synchronize()
+        return first
+
+    def plain(i, stream):
+        with torch.cuda.stream(stream):
+            bufs[i].fill_(1)
+
+    def graph(i, stream):
+        capi.check(L.dh_set_stream(stream.cuda_stream))
+        capi.check(L.dh_graph_launch(graphs[i], 0))
+
+    plain(0, long)
+    ends_first(side[0], plain)             # (the library's own first call)
+    # streams share the hardware's queues: one that runs beside the long one's
+    beside = [s for s in side if ends_first(s, plain)]
+    assert beside
+    try:
+        assert ends_first(beside[0], graph)
+        assert float(sum(b.sum() for b in bufs)) == 0.0
+    finally:
+        capi.check(L.dh_set_stream(None))
+        for g in graphs:
+            capi.check(L.dh_graph_destroy(g))

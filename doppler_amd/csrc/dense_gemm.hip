@@ -290,9 +290,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
 // 32-bit products of rows within reach (gemm_split.h).  Bound by the matrix cores where tiles are many (at 600 x 18464 x 4096 the three
 // instructions' rate is 1060 TFLOP/s, what the 16-bit products reach), by the steps' latency where they are few; us against 32-bit
 // instructions: 301 x 5136 x 1024 43 -> 18, 301 x 1024 x 4096 37 -> 18, 600 x 18464 x 4096 893 -> 257, 2 x 4096 x 16384 83 -> 34.
-// Distance from 64 bits (2-norm) there 5.7e-7 -> 1.0e-7, 4.7e-7 -> 1.4e-7, 8.1e-7 -> 2.7e-7, 8.1e-7 -> 2.2e-7.  A sum that is not finite is made again by itself: the parts of an infinite value, and
-// a part that is zero times an infinite weight, are no numbers where the product is infinite.  So is one of up to 2^-80: parts lose what lies
-// below bf16's smallest number, 2^-133, which a sum of that size may consist of.
+// Distance from 64 bits (2-norm) there 5.7e-7 -> 1.0e-7, 4.7e-7 -> 1.4e-7, 8.1e-7 -> 2.7e-7, 8.1e-7 -> 2.2e-7.  A tile whose sums the parts do not
+// give (join_sums) is multiplied again by 32-bit instructions.
 template <class Tile>
 __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_kernel(const GemmArgs a) {
   extern __shared__ __align__(16) char smem[];
@@ -305,29 +304,26 @@ __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_ker
   const uint16_t* w_base = a.W + (int64_t)n0 * a.ldw + k0;
   auto a_off = [&](int row) { return (uint32_t)((int64_t)min(row, a.M - 1 - m0) * a.lda * 4); };
   auto w_off = [&](int row) { return (uint32_t)((int64_t)min(row, a.N - 1 - n0) * a.ldw * 2); };
-  dh::split_product<Tile>(a_base, a_off, w_base, w_off, (k_end - k0) >> 6, smem);
+  const int nk = (k_end - k0) >> 6;
+  dh::split_product<Tile>(a_base, a_off, w_base, w_off, nk, smem);
+  if (__builtin_expect(!dh::everywhere<Tile>(dh::join_sums<Tile>(smem), smem), 0)) {
+    dh::exact_product<Tile>(a_base, a_off, w_base, w_off, nk, smem);
+    __syncthreads();
+    (void)dh::join_sums<Tile>(smem);
+  }
   const int lane = threadIdx.x & 63;
-#pragma unroll 1
-  for (int u = threadIdx.x >> 6; u < Tile::WM * Tile::NF * 4; u += Tile::kWaves) {
-    const int q = u & 3, j = (u >> 2) % Tile::NF, wm = (u >> 2) / Tile::NF;
-    f32x4_t sum = dh::split_sums<Tile>(smem, 0, wm, j, q)[lane];
-#pragma unroll
-    for (int g = 1; g < Tile::KG; g++) sum += dh::split_sums<Tile>(smem, g, wm, j, q)[lane];
+  dh::each_sum<Tile>(smem, [&](const f32x4_t* at, int wm, int j, int q) {
+    const f32x4_t sum = *at;
     const int n = n0 + 32 * j + (lane & 31), row = 32 * wm + 8 * q + 4 * (lane >> 5);
-    if (n >= a.N) continue;
+    if (n >= a.N) return;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int m = m0 + row + e;
       if (m >= a.M) break;
-      float v = sum[e];
-      if (__builtin_expect(!(fabsf(v) <= 3.402823466e38f) || (v != 0.f && fabsf(v) < 0x1p-80f), 0)) {
-        v = 0.f;
-        for (int k = 0; k < k_end - k0; k++) v = fmaf(a_base[(int64_t)(row + e) * a.lda + k], dh::bf16_bits_to_f32(w_base[(int64_t)(n - n0) * a.ldw + k]), v);
-      }
-      if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = v;
-      else put(a, m, n, v);
+      if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = sum[e];
+      else put(a, m, n, sum[e]);
     }
-  }
+  });
 }
 
 // Sums of the k slices in slice order.  VEC columns per thread (N a multiple of VEC), a block's threads as wide as the row allows and the

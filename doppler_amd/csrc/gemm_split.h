@@ -35,12 +35,95 @@ struct SplitTile {
   static constexpr int kBufA = BM * 256, kBufB = BN * 128, kRoundsA = kBufA / (1024 * kWaves), kRoundsB = kBufB / (1024 * kWaves);
   static constexpr int kSums = kWaves * NF * 4096, kLds = S * (kBufA + kBufB) > kSums ? S * (kBufA + kBufB) : kSums;
   static_assert(kBufA % (1024 * kWaves) == 0 && kBufB % (1024 * kWaves) == 0 && kLds <= 163840, "whole loads");
+  static_assert(kLds >= kSums + 4 * kWaves, "a word a wave behind the sums");
 };
 
 // Where a group's sums lie when the loop is over: lane l's four are rows 32 wm + 8 q + 4 (l >> 5) + 0 .. 3 of column 32 j + (l & 31).
 template <class Tile>
 __device__ __forceinline__ f32x4_t* split_sums(char* smem, int kg, int wm, int j, int q) {
   return reinterpret_cast<f32x4_t*>(smem) + (((kg * Tile::WM + wm) * Tile::NF + j) * 4 + q) * 64;
+}
+
+// A wave's share of a tile's sums, columns and rows as above: f(sum's place in the first group, wm, j, q).
+template <class Tile, class F>
+__device__ __forceinline__ void each_sum(char* smem, F f) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll 1
+  for (int u = threadIdx.x >> 6; u < Tile::WM * Tile::NF * 4; u += Tile::kWaves) {
+    const int q = u & 3, j = (u >> 2) % Tile::NF, wm = (u >> 2) / Tile::NF;
+    f(split_sums<Tile>(smem, 0, wm, j, q) + lane, wm, j, q);
+  }
+}
+// Adds the groups' sums into the first's; whether they are what the product's are.  Not if one is not finite: the parts of an infinite value, and
+// a part that is zero times an infinite weight, are no numbers where the product is infinite.  Nor if one is of up to 2^-80: parts lose what
+// lies below bf16's smallest number, 2^-133, which a sum of that size may consist of.
+template <class Tile>
+__device__ __forceinline__ bool join_sums(char* smem) {
+  bool sound = true;
+  each_sum<Tile>(smem, [&](f32x4_t* at, int wm, int j, int q) {
+    f32x4_t sum = *at;
+#pragma unroll
+    for (int g = 1; g < Tile::KG; g++) sum += *(split_sums<Tile>(smem, g, wm, j, q) + (threadIdx.x & 63));
+    *at = sum;
+#pragma unroll
+    for (int e = 0; e < 4; e++) sound = sound && fabsf(sum[e]) <= 3.402823466e38f && (sum[e] == 0.f || fabsf(sum[e]) >= 0x1p-80f);
+  });
+  return sound;
+}
+// Whether it holds for the whole workgroup.
+template <class Tile>
+__device__ __forceinline__ bool everywhere(bool here, char* smem) {
+  int* const words = reinterpret_cast<int*>(smem + Tile::kSums);
+  const int all = __builtin_amdgcn_ballot_w64(!here) == 0ull;
+  if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = all;
+  __syncthreads();
+  int every = 1;
+#pragma unroll
+  for (int w = 0; w < Tile::kWaves; w++) every &= words[w];
+  return __builtin_amdgcn_readfirstlane(every) != 0;
+}
+
+// The same tile on v_mfma_f32_32x32x2_f32, operands from memory into registers: for a tile whose sums the parts do not give.  Waves take the
+// rows and the share of k that they have in split_product, a lane four k at a time.  Bound by the instruction, 64 cycles for 2 k: a row that is
+// no number takes a call of 600 x 18464 x 4096 from 280 to 700 us, infinite rows in every tile to 1230 (each such sum by a lane of its own: 1000
+// and 90000).
+template <class Tile, class OffA, class OffW>
+__device__ __forceinline__ void exact_product(const void* a_base, OffA a_off, const void* w_base, OffW w_off, int nk, char* smem) {
+  constexpr int NF = Tile::NF, KS = 4 / Tile::KG;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wave / Tile::WM, wm = wave % Tile::WM, row = lane & 31, half = lane >> 5;
+  const char *pa = static_cast<const char*>(a_base) + a_off(32 * wm + row) + 64 * KS * kg + 16 * half, *pw[NF];
+  f32x16_t acc[NF];
+#pragma unroll
+  for (int j = 0; j < NF; j++) {
+    pw[j] = static_cast<const char*>(w_base) + w_off(32 * j + row) + 32 * KS * kg + 8 * half;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[j][e] = 0.f;
+  }
+#pragma unroll 1
+  for (int t = 0; t < nk; t++) {
+    f32x4_t fa[2 * KS];
+    uint2 fw[2 * KS][NF];
+#pragma unroll
+    for (int s = 0; s < 2 * KS; s++) {
+      fa[s] = *reinterpret_cast<const f32x4_t*>(pa + 256 * (int64_t)t + 32 * s);
+#pragma unroll
+      for (int j = 0; j < NF; j++) fw[s][j] = *reinterpret_cast<const uint2*>(pw[j] + 128 * (int64_t)t + 16 * s);
+    }
+#pragma unroll
+    for (int s = 0; s < 2 * KS; s++)
+#pragma unroll
+      for (int j = 0; j < NF; j++) {
+        const f32x4_t w = {bf16_low(fw[s][j].x), bf16_high(fw[s][j].x), bf16_low(fw[s][j].y), bf16_high(fw[s][j].y)};
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[s][e], w[e], acc[j], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < NF; j++)
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      split_sums<Tile>(smem, kg, wm, j, q)[lane] = f32x4_t{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
 }
 
 // One tile; operands, offsets and fetches as in gemm_wide.h, with 4-byte rows of A.  An A row's 64 k are 256 bytes whose 16-byte piece p

@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
 // instructions' rate is 1060 TFLOP/s, what the 16-bit products reach), by the steps' latency where they are few; us against 32-bit
 // instructions: 301 x 5136 x 1024 43 -> 18, 301 x 1024 x 4096 37 -> 18, 600 x 18464 x 4096 893 -> 257, 2 x 4096 x 16384 83 -> 34.
 // Distance from 64 bits (2-norm) there 5.7e-7 -> 1.0e-7, 4.7e-7 -> 1.4e-7, 8.1e-7 -> 2.7e-7, 8.1e-7 -> 2.2e-7.  A tile whose sums the parts do not
-// give (join_sums) is multiplied again by 32-bit instructions.
+// give (an activation that is not the sum of its parts, join_sums) is multiplied again by 32-bit instructions.
 template <class Tile>
 __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_kernel(const GemmArgs a) {
   extern __shared__ __align__(16) char smem[];
@@ -305,25 +305,27 @@ __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_ker
   auto a_off = [&](int row) { return (uint32_t)((int64_t)min(row, a.M - 1 - m0) * a.lda * 4); };
   auto w_off = [&](int row) { return (uint32_t)((int64_t)min(row, a.N - 1 - n0) * a.ldw * 2); };
   const int nk = (k_end - k0) >> 6;
-  dh::split_product<Tile>(a_base, a_off, w_base, w_off, nk, smem);
-  if (__builtin_expect(!dh::everywhere<Tile>(dh::join_sums<Tile>(smem), smem), 0)) {
+  dh::f32x4_t sums[Tile::kShare];
+  const bool whole = dh::split_product<Tile>(a_base, a_off, w_base, w_off, nk, smem), sound = dh::join_sums<Tile>(sums, smem);
+  if (__builtin_expect(!dh::everywhere<Tile>(whole && sound, smem), 0)) {
     dh::exact_product<Tile>(a_base, a_off, w_base, w_off, nk, smem);
     __syncthreads();
-    (void)dh::join_sums<Tile>(smem);
+    (void)dh::join_sums<Tile>(sums, smem);
   }
   const int lane = threadIdx.x & 63;
-  dh::each_sum<Tile>(smem, [&](const f32x4_t* at, int wm, int j, int q) {
-    const f32x4_t sum = *at;
-    const int n = n0 + 32 * j + (lane & 31), row = 32 * wm + 8 * q + 4 * (lane >> 5);
-    if (n >= a.N) return;
+#pragma unroll
+  for (int u = 0; u < Tile::kShare; u++) {
+    const dh::SumPlace<Tile> at(u);
+    const int n = n0 + 32 * at.j + (lane & 31), row = 32 * at.wm + 8 * at.q + 4 * (lane >> 5);
+    if (n >= a.N) continue;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int m = m0 + row + e;
       if (m >= a.M) break;
-      if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = sum[e];
-      else put(a, m, n, sum[e]);
+      if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = sums[u][e];
+      else put(a, m, n, sums[u][e]);
     }
-  });
+  }
 }
 
 // Sums of the k slices in slice order.  VEC columns per thread (N a multiple of VEC), a block's threads as wide as the row allows and the

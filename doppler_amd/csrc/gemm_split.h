@@ -5,12 +5,13 @@
 namespace dh {
 
 // An f32 is the exact sum of three bf16: its upper 16 bits, those of what remains, and the rest (8 + 8 + 8 significand bits; what a
-// subtraction leaves fits the next).  A product of two bf16 is exact in f32, so three bf16 instructions give what an f32 one gives of an
+// subtraction leaves fits the next) - unless it has bits below bf16's smallest number, 2^-133, which only one below 2^-110 can have: then the rest's lower
+// half is not zero, and `lost` collects that.  A product of two bf16 is exact in f32, so three bf16 instructions give what an f32 one gives of an
 // activation and a bf16 weight, in 3 x 32 cycles for 16 k against 8 x 64.  Of a pair of values the words hold (first, second).
 struct SplitWords {
   u32x4_t high, mid, low;
 };
-__device__ __forceinline__ SplitWords split_words(const f32x4_t& a, const f32x4_t& b) {
+__device__ __forceinline__ SplitWords split_words(const f32x4_t& a, const f32x4_t& b, uint32_t& lost) {
   SplitWords s;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
@@ -22,6 +23,7 @@ __device__ __forceinline__ SplitWords split_words(const f32x4_t& a, const f32x4_
     s.high[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
     s.mid[i] = __builtin_amdgcn_perm(v1, v0, 0x07060302u);
     s.low[i] = __builtin_amdgcn_perm(__float_as_uint(q1), __float_as_uint(q0), 0x07060302u);
+    lost |= __float_as_uint(q0) | __float_as_uint(q1);
   }
   return s;
 }
@@ -33,9 +35,9 @@ struct SplitTile {
   static constexpr int WM = WM_, NF = NF_, KG = KG_, S = S_, kPerSimd = PER_SIMD_;
   static constexpr int BM = 32 * WM, BN = 32 * NF, kWaves = WM * KG, kThreads = 64 * kWaves;
   static constexpr int kBufA = BM * 256, kBufB = BN * 128, kRoundsA = kBufA / (1024 * kWaves), kRoundsB = kBufB / (1024 * kWaves);
-  static constexpr int kSums = kWaves * NF * 4096, kLds = S * (kBufA + kBufB) > kSums ? S * (kBufA + kBufB) : kSums;
+  static constexpr int kSums = kWaves * NF * 4096, kShare = WM * NF * 4 / kWaves, kLds = S * (kBufA + kBufB) > kSums ? S * (kBufA + kBufB) : kSums;
   static_assert(kBufA % (1024 * kWaves) == 0 && kBufB % (1024 * kWaves) == 0 && kLds <= 163840, "whole loads");
-  static_assert(kLds >= kSums + 4 * kWaves, "a word a wave behind the sums");
+  static_assert(kLds >= kSums + 4 * kWaves && WM * NF * 4 % kWaves == 0, "a word a wave behind the sums, whole shares");
 };
 
 // Where a group's sums lie when the loop is over: lane l's four are rows 32 wm + 8 q + 4 (l >> 5) + 0 .. 3 of column 32 j + (l & 31).
@@ -44,30 +46,30 @@ __device__ __forceinline__ f32x4_t* split_sums(char* smem, int kg, int wm, int j
   return reinterpret_cast<f32x4_t*>(smem) + (((kg * Tile::WM + wm) * Tile::NF + j) * 4 + q) * 64;
 }
 
-// A wave's share of a tile's sums, columns and rows as above: f(sum's place in the first group, wm, j, q).
-template <class Tile, class F>
-__device__ __forceinline__ void each_sum(char* smem, F f) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll 1
-  for (int u = threadIdx.x >> 6; u < Tile::WM * Tile::NF * 4; u += Tile::kWaves) {
-    const int q = u & 3, j = (u >> 2) % Tile::NF, wm = (u >> 2) / Tile::NF;
-    f(split_sums<Tile>(smem, 0, wm, j, q) + lane, wm, j, q);
-  }
-}
-// Adds the groups' sums into the first's; whether they are what the product's are.  Not if one is not finite: the parts of an infinite value, and
-// a part that is zero times an infinite weight, are no numbers where the product is infinite.  Nor if one is of up to 2^-80: parts lose what
-// lies below bf16's smallest number, 2^-133, which a sum of that size may consist of.
+// A wave's share of a tile's sums: groups of four rows and 32 columns, u-th at (wm, j, q) as above.
 template <class Tile>
-__device__ __forceinline__ bool join_sums(char* smem) {
+struct SumPlace {
+  int wm, j, q;
+  __device__ __forceinline__ SumPlace(int u) {
+    const int at = (threadIdx.x >> 6) + Tile::kWaves * u;
+    q = at & 3, j = (at >> 2) % Tile::NF, wm = (at >> 2) / Tile::NF;
+  }
+};
+// Adds up the groups' sums; whether they are what the product's are.  Not if one is not finite: the parts of an infinite value, and
+// a part that is zero times an infinite weight, are no numbers where the product is infinite.  Nor if one is of up to 2^-80, which may consist
+// of products of parts that f32 does not hold.
+template <class Tile>
+__device__ __forceinline__ bool join_sums(f32x4_t (&sums)[Tile::kShare], char* smem) {
   bool sound = true;
-  each_sum<Tile>(smem, [&](f32x4_t* at, int wm, int j, int q) {
-    f32x4_t sum = *at;
 #pragma unroll
-    for (int g = 1; g < Tile::KG; g++) sum += *(split_sums<Tile>(smem, g, wm, j, q) + (threadIdx.x & 63));
-    *at = sum;
+  for (int u = 0; u < Tile::kShare; u++) {
+    const SumPlace<Tile> at(u);
+    sums[u] = split_sums<Tile>(smem, 0, at.wm, at.j, at.q)[threadIdx.x & 63];
 #pragma unroll
-    for (int e = 0; e < 4; e++) sound = sound && fabsf(sum[e]) <= 3.402823466e38f && (sum[e] == 0.f || fabsf(sum[e]) >= 0x1p-80f);
-  });
+    for (int g = 1; g < Tile::KG; g++) sums[u] += split_sums<Tile>(smem, g, at.wm, at.j, at.q)[threadIdx.x & 63];
+#pragma unroll
+    for (int e = 0; e < 4; e++) sound = sound && fabsf(sums[u][e]) <= 3.402823466e38f && (sums[u][e] == 0.f || fabsf(sums[u][e]) >= 0x1p-80f);
+  }
   return sound;
 }
 // Whether it holds for the whole workgroup.
@@ -127,9 +129,9 @@ __device__ __forceinline__ void exact_product(const void* a_base, OffA a_off, co
 }
 
 // One tile; operands, offsets and fetches as in gemm_wide.h, with 4-byte rows of A.  An A row's 64 k are 256 bytes whose 16-byte piece p
-// lies at slot p ^ (row & 15); W rows as there.  Leaves every group's sums in LDS.
+// lies at slot p ^ (row & 15); W rows as there.  Leaves every group's sums in LDS; whether the parts of what this lane has split are the whole.
 template <class Tile, class OffA, class OffW>
-__device__ __forceinline__ void split_product(const void* a_base, OffA a_off, const void* w_base, OffW w_off, int nk, char* smem) {
+__device__ __forceinline__ bool split_product(const void* a_base, OffA a_off, const void* w_base, OffW w_off, int nk, char* smem) {
   constexpr int NF = Tile::NF, KG = Tile::KG, S = Tile::S, RA = Tile::kRoundsA, RB = Tile::kRoundsB, KS = 4 / KG;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kg = wave / Tile::WM, wm = wave % Tile::WM;
@@ -172,6 +174,7 @@ __device__ __forceinline__ void split_product(const void* a_base, OffA a_off, co
   f32x4_t fa[2];
   u32x4_t fb[2][NF];
   SplitWords words[2];
+  uint32_t lost = 0;
   auto read = [&](int i, int buf, int set) {
 #pragma unroll
     for (int e = 0; e < 2; e++) fa[e] = *reinterpret_cast<const f32x4_t*>(ra[i][e] + buf * Tile::kBufA);
@@ -199,11 +202,11 @@ __device__ __forceinline__ void split_product(const void* a_base, OffA a_off, co
       multiply(words[cur].low, cur, rest);
       multiply(words[cur].mid, cur, rest);
       multiply(words[cur].high, cur, acc);
-      words[next] = split_words(fa[0], fa[1]);
+      words[next] = split_words(fa[0], fa[1], lost);
       __builtin_amdgcn_sched_group_barrier(0x008, NF, 0);
 #pragma unroll
       for (int n = 0; n < 2 * NF; n++) {
-        __builtin_amdgcn_sched_group_barrier(0x002, 48 / (2 * NF), 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 56 / (2 * NF), 0);
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       }
     }
@@ -212,7 +215,7 @@ __device__ __forceinline__ void split_product(const void* a_base, OffA a_off, co
   for (int t = 0; t < S; t++) fetch(t, t);
   arrive_and_wait<(S - 1) * (RA + RB)>();
   read(0, 0, 0);
-  words[0] = split_words(fa[0], fa[1]);
+  words[0] = split_words(fa[0], fa[1], lost);
   constexpr int U = S * KS % 2 ? 2 * S : S;      // steps after which buffers and sets of registers repeat
   bool more = true;
   for (int t = 0; more; t += U) {
@@ -231,6 +234,7 @@ __device__ __forceinline__ void split_product(const void* a_base, OffA a_off, co
       split_sums<Tile>(smem, kg, wm, j, q)[lane] = f32x4_t{acc[j][4 * q] + rest[j][4 * q], acc[j][4 * q + 1] + rest[j][4 * q + 1],
                                                            acc[j][4 * q + 2] + rest[j][4 * q + 2], acc[j][4 * q + 3] + rest[j][4 * q + 3]};
   __syncthreads();
+  return (lost & 0xffffu) == 0u;
 }
 
 }  // namespace dh

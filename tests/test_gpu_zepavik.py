@@ -327,6 +327,45 @@ def test_dense_matmul_f32_extreme_values(L, M, N, K):
     assert (got.double() - want)[rows][finite[rows]].abs().max() < 5e-5
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 70, 128), (300, 1030, 1024), (301, 1024, 4096), (600, 10255, 2112)])
+def test_dense_matmul_f32_far_from_one(L, M, N, K):
+    """Activations with bits below bf16's smallest number, down to f32's, against small, ordinary and huge weights.  f32 sums: half a unit of the
+    last place of K / 8 partial sums at worst, which are no larger than the terms together, and 2^-150 for each product and sum below f32's normal numbers."""
+    g = torch.Generator(device="cuda").manual_seed(K + 1)
+    A = torch.randn(M, K, generator=g, device="cuda")
+    W = torch.randn(N, K, generator=g, device="cuda")
+    for rows, power in ((slice(0, 2), -136), (slice(2, 4), -124), (slice(4, 6), -110), (slice(6, 7), -100)):
+        A[rows] *= 2.0 ** (power // 2)
+        A[rows] *= 2.0 ** (power - power // 2)
+    for columns, power in ((slice(0, 9), 100), (slice(9, 20), 50), (slice(20, 30), 30), (slice(30, 40), -60)):
+        W[columns] *= 2.0 ** power
+    A[7, 1:] = 0
+    A[7, 0] = 2.0 ** -140
+    W = W.to(torch.bfloat16)
+    got, a, w = torch.zeros(M, N, device="cuda"), A.double(), W.double()
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), capi.F32, K, W.data_ptr(), K, M, N, K, 1.0, None, None, got.data_ptr(), N, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    bound = K / 8 * 2.0 ** -25 * (a.abs() @ w.abs().T) + 2 * K * 2.0 ** -150
+    assert bool(((got.double() - a @ w.T).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 70, 128), (301, 1024, 4096), (600, 10255, 2112)])
+def test_dense_matmul_f32_parts_below_normal_numbers(L, M, N, K):
+    """What parts that bf16 holds only below its normal numbers leave of two activations, where the rest of them cancels; and weights there."""
+    A, W = torch.zeros(M, K, device="cuda"), torch.full((N, K), 2.0 ** 60, device="cuda").to(torch.bfloat16)
+    A[:, 5], A[:, K - 1] = 2.0 ** -104 * (1 + 2.0 ** -22), -2.0 ** -104
+    A[3], W[7] = 0, 2.0 ** -130
+    A[3, 9], A[3, 11] = 2.0 ** 67 * (1 + 2.0 ** -16), -2.0 ** 67
+    got = torch.zeros(M, N, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), capi.F32, K, W.data_ptr(), K, M, N, K, 1.0, None, None, got.data_ptr(), N, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    want = A.double() @ W.double().T
+    want[:, 7] = torch.where(torch.arange(M, device="cuda") == 3, want[:, 7], torch.zeros(()).double().cuda())       # 2^-256
+    assert torch.equal(got.double(), want)
+
+
 def test_dense_matmul_f32_rows_that_are_no_numbers_cost_little(L):
     """Sums that the split operands do not give are made again a tile at a time: with one such row of 600 the call takes 2.5 times as long, with all of
     them what 32-bit instructions take besides, 4.4 times."""

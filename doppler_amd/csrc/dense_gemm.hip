@@ -554,6 +554,25 @@ TileChoice choose_f32(int64_t M, int64_t N, int64_t K) {
   if (env_slices) best.slices = std::min(most, env_slices);
   return best;
 }
+// k slices of a product that goes through registers.  Workgroups on a compute unit share its matrix cores, so the one with the most of them
+// ends last: 64 k of a tile take 1.35 us alone there and 1.1 us each in company (0.85 at the full rate).  Slices cost a launch and 4 bytes a sum
+// at 4 TB/s.
+int choose_register_slices(int64_t M, int64_t N, int64_t K) {
+  const int64_t steps = K / 64, tiles = dh::ceil_div(M, 64) * dh::ceil_div(N, 64);
+  const int most = slices_in_workspace(M, N, kMaxSlices);
+  int slices = 1;
+  double least = 1e30;
+  for (int s = 1; s <= most && (s == 1 || steps / s >= 2); s++) {
+    const int64_t together = dh::ceil_div(tiles * s, dh::num_cus());
+    double t = (together == 1 ? 1350.0 : 1100.0 * together) * dh::ceil_div(steps, s);
+    if (s > 1) t += 3500.0 + 4.0 * M * N * (2 * s + 1) / 4000.0;
+    if (t < least) {
+      least = t;
+      slices = s;
+    }
+  }
+  return slices;
+}
 // k of a slice (whole steps of 64).
 int slice_extent(int64_t K, int slices) { return (int)dh::ceil_div(K / 64, slices) * 64; }
 
@@ -572,7 +591,7 @@ int launch_split(const char* op, GemmArgs a, int slices) {
 // behind: 361 x 8204 x 64 takes 9.4 us with 32-bit instructions and 12.1 without, 2024 x 3594 x 64 17.9 and 21.9; at two steps it is even or ahead.
 int dense_f32(const char* op, GemmArgs a) {
   const bool split = a.K >= kSplitK && 4 * (std::min<int64_t>(a.M, Split128x128::BM) * a.lda + a.K) < (int64_t)1 << 32 && within_reach(a.N, a.ldw, a.K);
-  const TileChoice pick = choose_f32(a.M, a.N, a.K);
+  const TileChoice pick = split ? choose_f32(a.M, a.N, a.K) : TileChoice{0, choose_register_slices(a.M, a.N, a.K)};
   a.k_slice = slice_extent(a.K, pick.slices);
   const int slices = (int)dh::ceil_div(a.K, a.k_slice);
   size_t ws_bytes = 0;
@@ -679,9 +698,9 @@ extern "C" int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int form
   if (!out3 || M <= 0 || N <= 0 || K <= 0 || K % 64) return dh::fail(1, "[%s] M=%d, N=%d, K=%d (a multiple of 64), or no place for the result", op, M, N, K);
   dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
   const bool wide = a_dtype == DH_F32, glu = form == 1;
-  const TileChoice pick = wide ? (glu ? TileChoice{0, 1} : choose_f32(M, N, K)) : glu ? choose_tile(M, N, K, 1, true, false) : choose_16bit(M, N, K, form == 2);
+  const bool registers = wide && (glu || K < kSplitK || form == 3);
+  const TileChoice pick = registers ? TileChoice{0, glu ? 1 : choose_register_slices(M, N, K)} : wide ? choose_f32(M, N, K) : glu ? choose_tile(M, N, K, 1, true, false) : choose_16bit(M, N, K, form == 2);
   dh::plan_end();
-  const bool registers = wide && (glu || K < kSplitK);
   const TileCost& c = wide ? kSplitTiles[pick.tile] : glu ? kGluTiles[pick.tile] : kTiles[pick.tile];
   out3[0] = registers ? 64 : c.bm;
   out3[1] = registers ? (glu ? 128 : 64) : c.bn;

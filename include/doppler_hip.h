@@ -391,7 +391,7 @@ int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, const void* d_
                            const float* d_bias, const float* d_col_scale, const float* d_residual, float* d_C, int ldc,
                            int n_first, void* d_C2, int c2_dtype, int ldc2, int activation);
 /* The tile dh_dense_matmul would take for activations of a_dtype (form 1: the shared expert's gate and up product of dh_experts_prefill;
- * 2: with a second output through DH_ACT_GELU_ERF): out3 = { rows, columns, slices k is cut into }.  For tests that have to reach every
+ * 2: with a second output through DH_ACT_GELU_ERF; 3: f32 rows too far apart for 32-bit offsets): out3 = { rows, columns, slices k is cut into }.  For tests that have to reach every
  * tile; needs no device. */
 int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int form, int num_cus, int64_t* out3);
 

@@ -344,3 +344,16 @@ def test_prompts_over_f32_caches_take_the_kernel_measured_faster(H, G, d, e, win
 def test_gated_pairs_take_the_kernel_measured_faster(M, inter, hidden, wide):
     import ctypes
     assert capi.load().dh_q4k_gemm_layout(M, inter, hidden, 1, NCU, (ctypes.c_int64 * 4)()) == wide
+
+
+@pytest.mark.parametrize("M,N,K", [(301, 1024, 4096), (2, 4096, 16384), (64, 4096, 16384), (17, 1024, 4096), (600, 18464, 4096), (33, 65, 64)])
+def test_f32_rows_out_of_reach_are_sliced_by_their_own_kernels_costs(M, N, K):
+    """64 x 64 tiles through registers: 64 k of one take 1.35 us alone on a compute unit and 1.1 us each in company, a second launch 3.5 us and 4
+    bytes a sum at 4 TB/s."""
+    def cost(s):
+        together, steps = ceil_div(ceil_div(M, 64) * ceil_div(N, 64) * s, NCU), ceil_div(K // 64, s)
+        return (1350 if together == 1 else 1100 * together) * steps + (3500 + 4 * M * N * (2 * s + 1) / 4000 if s > 1 else 0)
+    best = min(range(1, min(16, max(1, K // 128)) + 1), key=cost)
+    out = (ctypes.c_int64 * 3)()
+    capi.check(capi.load().dh_dense_matmul_layout(M, N, K, capi.F32, 3, NCU, out))
+    assert tuple(out) == (64, 64, ceil_div(K // 64, ceil_div(K // 64, best)))

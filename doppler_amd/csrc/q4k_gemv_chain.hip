@@ -991,7 +991,12 @@ int dh_q4k_layer_chain_supported(int hidden, int inter, int q_size, int qkv_size
   }
   ph[1].d_W2 = at;
   Plan plan;
-  return make_plan("dh_q4k_layer_chain_supported", at, nullptr, ph, 4, true, &plan) == 0 ? 1 : 0;
+  // (no is an answer, not an error: the last one's message stays)
+  char message[1024];
+  snprintf(message, sizeof(message), "%s", dh_last_error());
+  const bool fits = make_plan("dh_q4k_layer_chain_supported", at, nullptr, ph, 4, true, &plan) == 0;
+  if (!fits) dh::fail(0, "%s", message);
+  return fits ? 1 : 0;
 }
 
 int dh_q4k_gemv_chain_short(const float* d_x0, const dh_chain_attn_source* source, const dh_chain_phase* phases, int n_phases) {

@@ -348,6 +348,9 @@ def test_layers_that_fit_a_chain():
     for dims, fits in (((1024, 3072, 1024, 2048), 1), ((4096, 12288, 4096, 6144), 1), ((768, 768, 768, 768), 1), ((512, 1024, 512, 1024), 0),
                        ((1024, 3000, 1024, 2048), 0), ((1024, 32768, 1024, 2048), 0), ((1024, 16384, 1024, 2048), 0)):
         assert L.dh_q4k_layer_chain_supported(*dims) == fits, dims
+    assert L.dh_malloc(0, ctypes.byref(ctypes.c_void_p())) != 0
+    message = L.dh_last_error()
+    assert b"dh_malloc" in message and L.dh_q4k_layer_chain_supported(512, 1024, 512, 1024) == 0 and L.dh_last_error() == message
 
 
 def test_residual_of_other_rows_is_read_when_its_tile_ends():

@@ -652,25 +652,22 @@ int launch_rows(RowsArgs a, const char* op) {
   };
   a.depth = fit_depth();
   if (a.depth == 0) return -1;
-  // the record is the launch of one slice; several are this launch for so many times fewer compute units, with fewer columns
+  int slices = DUAL || a.norm_weight ? 1 : choose_slices(a.M, a.N, a.nb);
+  auto take = [&](int s) {
+    slices = s;
+    lay_out(s);
+    a.depth = fit_depth();
+  };
+  take(slices);
+  if (a.depth == 0) take(1);
   {
-    const int64_t rec[12] = {a.rows, a.nlw, a.grid, a.tiles_base, a.tiles_rem, a.depth, (int64_t)lds_for(a.depth), 0, 0, 0, a.acc_max,
+    const int64_t rec[12] = {a.rows, a.nlw, a.grid, a.tiles_base, a.tiles_rem, a.depth, (int64_t)lds_for(a.depth), slices, 0, 0, a.acc_max,
                              a.M};
     for (int i = 0; i < 12; i++) dh::plan_layout(i, rec[i]);
   }
   if (dh::plan_note(DH_PLAN_GEMV_ROWS)) return 0;
-  // (a caller's own graph is replayed beside whatever it likes: it shares no memory with other launches)
-  int slices = DUAL || a.norm_weight ? 1 : choose_slices(a.M, a.N, a.nb);
-  if (slices > 1 && dh::foreign_capture()) slices = 1;
-  if (slices > 1) {
-    lay_out(slices);
-    a.depth = fit_depth();
-    if (a.depth == 0) {
-      slices = 1;
-      lay_out(1);
-      a.depth = fit_depth();
-    }
-  }
+  // a caller's own graph is replayed beside whatever it likes: it shares no memory with other launches
+  if (slices > 1 && dh::foreign_capture()) take(1);
   const size_t lds = lds_for(a.depth);
   static bool attr_set = false;   // once per instantiation: the call costs microseconds
   if (!attr_set) {

@@ -89,12 +89,18 @@ def _matmul_case(M, N, K, seed, alpha=1.0, outputDtype="f32", residual=False):
     return rel_l2(got, want)
 
 
-@pytest.mark.parametrize("M,N,K,alpha,outputDtype,residual,f16", [
-    (3, 1100, 4352, 1.0, "f32", False, False),                                   # 17 columns: the first count that may be cut
-    (8, 4096, 12288, 1.0, "f32", True, False), (4, 600, 9000, 0.5, "f32", True, False), (15, 1024, 12288, 1.0, "f16", True, False),
-    (5, 2047, 6148, 1.0, "f32", False, True), (8, 33, 32768, -2.0, "f32", True, True), (7, 3001, 5000, 1.0, "f16", False, False)])
-def test_few_rows_of_many_columns(M, N, K, alpha, outputDtype, residual, f16):
+SLICED_PRODUCTS = [
+    (3, 1100, 4352, 1.0, "f32", False, False, 2),                                # 17 columns: the first count that may be cut
+    (8, 4096, 12288, 1.0, "f32", True, False, 3), (4, 600, 9000, 0.5, "f32", True, False, 3), (15, 1024, 12288, 1.0, "f16", True, False, 3),
+    (5, 2047, 6148, 1.0, "f32", False, True, 5), (8, 33, 32768, -2.0, "f32", True, True, 8), (7, 3001, 5000, 1.0, "f16", False, False, 5),
+    (8, 4096, 4096, 1.0, "f32", False, False, 1)]
+
+
+@pytest.mark.parametrize("M,N,K,alpha,outputDtype,residual,f16,slices", SLICED_PRODUCTS)
+def test_few_rows_of_many_columns(M, N, K, alpha, outputDtype, residual, f16, slices):
     """Long rows whose columns are cut into slices.  Operands keep 22 bits and sums are f32: 1e-5 of the result; an f16 output rounds to 2^-11."""
+    out12 = (ctypes.c_int64 * 12)()
+    assert capi.load().dh_q4k_gemv_layout(M, N, K, 0, 0, 256, out12) == capi.PLAN_GEMV_ROWS and out12[7] == slices
     W, wb = q4k_weight(N, K, 1350 + M)
     A = synth.normal_f32((M, K), 1351 + M)
     A = A.astype(np.float16) if f16 else A

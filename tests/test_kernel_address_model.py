@@ -28,7 +28,10 @@ def layout(M, N, K, normed, dual, ncu=NCU):
     out = (ctypes.c_int64 * 12)()
     fam = capi.load().dh_q4k_gemv_layout(M, N, K, int(normed), int(dual), ncu, out)
     keys = ("rows", "nlw", "grid", "tiles_base", "tiles_rem", "depth", "lds", "upt", "upt_mul", "nslots", "acc_max", "mt")
-    return fam, dict(zip(keys, [int(v) for v in out]))
+    lay = dict(zip(keys, [int(v) for v in out]))
+    if fam == ROWS:
+        lay["slices"] = lay["upt"]
+    return fam, lay
 
 
 def ceil_div(a, b):
@@ -186,20 +189,59 @@ def test_int8_gemv_refuses_what_its_32_bit_unit_decode_cannot_hold():
 
 # --------------------------------------------------------------------------------------- few-row kernel
 
-def check_rows(M, N, K, normed, dual, ncu=NCU):
+SLICE_BYTES = 32 << 20
+SSQ_FLOATS, ACC_BYTES = 16, 512
+
+
+def deal(N, cus):
+    """rows of a tile, workgroups, tiles of a workgroup: floor and how many have one more"""
+    rows = tile_rows(N, cus)
+    grid = min(ceil_div(N, rows), cus)
+    return (rows, grid) + divmod(ceil_div(N, rows), grid)
+
+
+def rows_lds(tiles, nmat, normed, depth):
+    return WAVES * depth * STAGE + (4 * WAVES * QK if normed else 0) + 4 * WAVES * SSQ_FLOATS + WAVES * tiles * nmat * ACC_BYTES
+
+
+def slices_of(M, N, nb, ncu):
+    """The cheapest number of slices: 4 us for each column a wave meets, 0.7 and 1.3 / 16 a row for each unit, 3 for the second launch; one where a
+    workgroup's accumulators do not fit."""
+    if nb <= WAVES:
+        return 1
+
+    def tiles_of(s):
+        _, _, base, rem = deal(N, ncu // s)
+        return base + (1 if rem else 0)
+
+    def cost(s):
+        tiles = tiles_of(s)
+        units = ceil_div(nb, s) * tiles
+        runs = [(w * units // WAVES, (w + 1) * units // WAVES) for w in range(WAVES)]
+        columns = max((q1 - 1) // tiles - q0 // tiles + 1 for q0, q1 in runs if q1 > q0)
+        return 4 * columns + (0.7 + 1.3 / 16 * deal(N, ncu // s)[0]) * max(q1 - q0 for q0, q1 in runs) + (3 if s > 1 else 0)
+    best = min(range(1, max(1, min(8, SLICE_BYTES // (4 * M * N))) + 1), key=cost)
+    return best if rows_lds(tiles_of(best), 1, False, 1) <= 160 * 1024 else 1
+
+
+def check_rows(M, N, K, normed, dual, ncu=NCU, slices=None):
     fam, lay = layout(M, N, K, normed, dual, ncu)
     assert fam == ROWS, (M, N, K, fam)
     Mp = min(M, 8)                                 # rows of the first pass
     nb, nmat = ceil_div(K, QK), 2 if dual else 1
-    rows = tile_rows(N, ncu)
+    S = 1 if normed or dual else slices_of(Mp, N, nb, ncu)
+    assert lay["slices"] == S and slices in (None, S), (lay["slices"], S, slices)
+    # a slice's columns: whole, each in one slice, none empty; its sums in the slices' own memory
+    cuts = [y * nb // S for y in range(S + 1)]
+    assert cuts[0] == 0 and cuts[S] == nb and all(a < b for a, b in zip(cuts, cuts[1:]))
+    assert S == 1 or 4 * ((S - 1) * Mp * N + (Mp - 1) * N + N) <= SLICE_BYTES
+    rows, grid, tiles_base, tiles_rem = deal(N, ncu // S)
     ntiles = ceil_div(N, rows)
-    grid = min(ntiles, ncu)
-    tiles_base, tiles_rem = ntiles // grid, ntiles % grid
     acc_max = (tiles_base + (1 if tiles_rem else 0)) * nmat
-    ssq_floats, acc_bytes = 16, 512
+    ssq_floats, acc_bytes = SSQ_FLOATS, ACC_BYTES
 
     def lds_for(depth):
-        return WAVES * depth * STAGE + (4 * WAVES * QK if normed else 0) + 4 * WAVES * ssq_floats + WAVES * acc_max * acc_bytes
+        return rows_lds(acc_max // nmat, nmat, normed, depth)
 
     depth = 2
     while depth > 1 and lds_for(depth) > 160 * 1024:
@@ -219,10 +261,10 @@ def check_rows(M, N, K, normed, dual, ncu=NCU):
     xk = 8 * kg + 4 * part
     # ring reads: header of row j, eight bytes of nibbles of the lane's k-group in each of the four chunks
     assert np.all(j * BLOCK + 16 <= STAGE) and np.all(j * BLOCK + 16 + 8 * kg + 96 + 8 <= STAGE)
-    for bid in sorted({0, 1, grid // 2, tiles_rem - 1, tiles_rem, grid - 1} & set(range(grid))):
+    for bid, y in itertools.product(sorted({0, 1, grid // 2, tiles_rem - 1, tiles_rem, grid - 1} & set(range(grid))), sorted({0, S // 2, S - 1})):
         ntl = tiles_base + (1 if bid < tiles_rem else 0)
         nacc = ntl * nmat
-        total = nb * nacc
+        total = (cuts[y + 1] - cuts[y]) * nacc
         assert nacc <= acc_max
         for wave in range(WAVES):
             q0, q1 = (wave * total) >> 4, ((wave + 1) * total) >> 4
@@ -234,8 +276,8 @@ def check_rows(M, N, K, normed, dual, ncu=NCU):
                 assert o_wn + 4 * wave * QK + 63 * 16 + 16 <= o_ssq                  # what the load unit writes
             assert o_ssq + 4 * (wave * ssq_floats + 7) + 4 <= o_acc
             for u in sorted({q0, q0 + 1, (q0 + q1) // 2, q1 - 1} & set(range(q0, q1))):
-                col, acc = u // nacc, u % nacc
-                assert col < nb
+                col, acc = cuts[y] + u // nacc, u % nacc
+                assert cuts[y] <= col < cuts[y + 1]
                 itl, imat = (acc >> 1, acc & 1) if dual else (acc, 0)
                 tile = bid + itl * grid
                 assert tile < ntiles and imat < nmat
@@ -270,7 +312,7 @@ def check_rows(M, N, K, normed, dual, ncu=NCU):
             for oj in range(16):
                 row = tile * rows + oj
                 if oj < rows and row < N:
-                    assert (Mp - 1) * N + row < Mp * N
+                    assert (Mp - 1) * N + row < Mp * N and (y * Mp + Mp - 1) * N + row < (y + 1) * Mp * N
 
 
 ROWS_SHAPES = [
@@ -294,12 +336,28 @@ def test_a_smaller_device_changes_the_layout_not_the_bounds():
     check_rows(4, 4096, 12288, 0, 0, ncu=304)
 
 
-@pytest.mark.parametrize("slices", range(2, 9))
-def test_few_row_gemv_slices_are_launches_for_fewer_compute_units(slices):
+SLICED = [   # (M, N, K), slices on 256 compute units
+    ((8, 4096, 4096), 1), ((3, 1100, 4352), 2), ((8, 8192, 8192), 2), ((8, 4096, 12288), 3), ((4, 600, 9000), 3), ((15, 1024, 12288), 3), ((8, 5000, 16384), 4),
+    ((5, 2047, 6148), 5), ((6, 3520, 5280), 6), ((5, 4222, 6228), 7), ((8, 33, 32768), 8),
+    ((8, 12288, 32768), 1),                                         # eight would not fit the LDS
+]
+
+
+@pytest.mark.parametrize("shape,slices", SLICED)
+def test_few_row_gemv_slices_stay_inside_their_buffers(shape, slices):
     """Rows of more than 16 columns go in slices of the columns, each dealt to so many times fewer compute units."""
-    for M, N, K in ((8, 4096, 12288), (3, 600, 9000), (8, 12288, 32768), (5, 33, 4100)):
-        if layout(M, N, K, 0, 0, NCU // slices)[0] == ROWS:
-            check_rows(M, N, K, 0, 0, ncu=NCU // slices)
+    check_rows(*shape, 0, 0, slices=slices)
+    for ncu in (64, 120, 304):
+        check_rows(*shape, 0, 0, ncu=ncu)
+
+
+def test_the_slices_tests_reach_several_counts():
+    """The shapes of the few-row products' GPU test take the slices named beside them."""
+    from tests import test_gpu_ops
+    for M, N, K, _, _, _, _, slices in test_gpu_ops.SLICED_PRODUCTS:
+        fam, lay = layout(M, N, K, 0, 0)
+        assert fam == ROWS and lay["slices"] == slices, (M, N, K, lay)
+    assert {1, 2, 3} < {s[7] for s in test_gpu_ops.SLICED_PRODUCTS}
 
 
 def test_the_product_tests_reach_every_tile():

@@ -590,13 +590,16 @@ Deal deal(int64_t N, int64_t cus) {
 }
 
 // Slices of the columns, whose sums a second launch adds up.  A wave's columns follow one another: loads of its eight activation rows,
-// conversion, products.  Many columns over few tiles are therefore cut so that a wave meets one of them and uses it for several tiles: M x N x K
-// in us, weights from memory, one slice against the choice: 8 x 4096 x 12288 18.9 -> 15.9 (weights from the cache 15.2 -> 14.2), 8 x 2048 x 12288
-// 16.2 -> 12.0, 8 x 1024 x 12288 15.0 -> 10.9, 8 x 12288 x 12288 29.9 -> 27.1, 8 x 2048 x 6144 11.4 -> 10.2, 4 x 600 x 9000 14.9 -> 10.7.  The costs
-// below (us) were read off these: a column, a unit, the second launch; up to 16 columns over 256 workgroups stay whole (8 x 4096 x 4096 8.5, 11.4 in
-// two slices).
+// conversion, products.  Many columns over few tiles are therefore cut so that a wave meets one of them and uses it for several tiles.
+// The costs (us: a unit of the longest run, a column that a wave of the workgroup meets, the second launch, 10^6 bytes of sums) are fitted to
+// 206 products of 200 .. 40000 x 4100 .. 32768 with 1 to 8 slices, weights from memory and from the cache.  Over 206 others the choice takes
+// 0.83 of one slice's time, 1.07 at worst (6 above 1.03).
+// M x N x K in us, weights from memory, one slice and the choice: 8 x 4096 x 12288 18.9, 15.8 (from the cache 15.3, 14.1), 8 x 1024 x 12288 15.3,
+// 9.9, 8 x 12288 x 12288 29.7, 26.3, 4 x 600 x 9000 14.2, 8.4; whole, against the two to six slices they would be with a second launch of 3 us
+// (and up to 16 columns always): 8 x 4096 x 4608 10.2, 11.7, 3 x 3642 x 4624 9.3, 11.5, 6 x 3520 x 5280 10.2, 11.9.
 int choose_slices(int64_t M, int64_t N, int64_t nb) {
-  constexpr double kColumn = 4.0, kUnit = 0.7, kUnitRow = 1.3 / kTileRows, kSecondLaunch = 3.0;
+  constexpr double kUnit = 1.22, kColumn = 0.305, kSecondLaunch = 4.62, kSums = 0.24e-6;
+  constexpr int kMostTiles = (int)((kLdsCap - kWaves * kStage - sizeof(float) * kWaves * kSsqFloats) / (kWaves * kAccBytes));     // of a workgroup, in LDS
   if (nb <= kWaves) return 1;
   const int most = (int)std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)kSliceBytes / (4 * M * N)));
   int best = 1;
@@ -604,14 +607,15 @@ int choose_slices(int64_t M, int64_t N, int64_t nb) {
   for (int s = 1; s <= most; s++) {
     const Deal d = deal(N, std::max(1, dh::num_cus() / s));
     const int tiles = d.base + (d.rem ? 1 : 0);
+    if (s > 1 && tiles > kMostTiles) continue;
     const int64_t units = dh::ceil_div(nb, s) * tiles;
-    int64_t columns = 0, run = 0;              // the most that a wave meets
+    int64_t columns = 0, run = 0;
     for (int w = 0; w < kWaves; w++) {
       const int64_t q0 = w * units / kWaves, q1 = (w + 1) * units / kWaves;
       run = std::max(run, q1 - q0);
-      if (q1 > q0) columns = std::max(columns, (q1 - 1) / tiles - q0 / tiles + 1);
+      if (q1 > q0) columns += (q1 - 1) / tiles - q0 / tiles + 1;
     }
-    const double t = kColumn * columns + (kUnit + kUnitRow * d.rows) * run + (s > 1 ? kSecondLaunch : 0.0);
+    const double t = kUnit * run + kColumn * columns + (s > 1 ? kSecondLaunch + kSums * 4 * s * M * N : 0.0);
     if (t < least) {
       least = t;
       best = s;
@@ -659,7 +663,6 @@ int launch_rows(RowsArgs a, const char* op) {
     a.depth = fit_depth();
   };
   take(slices);
-  if (a.depth == 0) take(1);
   {
     const int64_t rec[12] = {a.rows, a.nlw, a.grid, a.tiles_base, a.tiles_rem, a.depth, (int64_t)lds_for(a.depth), slices, 0, 0, a.acc_max,
                              a.M};

@@ -90,10 +90,10 @@ def _matmul_case(M, N, K, seed, alpha=1.0, outputDtype="f32", residual=False):
 
 
 SLICED_PRODUCTS = [
-    (3, 1100, 4352, 1.0, "f32", False, False, 2),                                # 17 columns: the first count that may be cut
-    (8, 4096, 12288, 1.0, "f32", True, False, 3), (4, 600, 9000, 0.5, "f32", True, False, 3), (15, 1024, 12288, 1.0, "f16", True, False, 3),
-    (5, 2047, 6148, 1.0, "f32", False, True, 5), (8, 33, 32768, -2.0, "f32", True, True, 8), (7, 3001, 5000, 1.0, "f16", False, False, 5),
-    (8, 4096, 4096, 1.0, "f32", False, False, 1)]
+    (3, 1100, 4352, 1.0, "f32", False, False, 1), (8, 300, 4352, 1.0, "f32", False, False, 6),       # 17 columns: the first count that may be cut
+    (8, 4096, 12288, 1.0, "f32", True, False, 3), (4, 600, 9000, 0.5, "f32", True, False, 6), (15, 1024, 12288, 1.0, "f16", True, False, 4),
+    (5, 2047, 6148, 1.0, "f32", False, True, 2), (8, 33, 32768, -2.0, "f32", True, True, 8), (7, 3001, 5000, 1.0, "f16", False, False, 1),
+    (7, 2605, 9408, 1.0, "f16", False, False, 5)]
 
 
 @pytest.mark.parametrize("M,N,K,alpha,outputDtype,residual,f16,slices", SLICED_PRODUCTS)

@@ -205,8 +205,8 @@ def rows_lds(tiles, nmat, normed, depth):
 
 
 def slices_of(M, N, nb, ncu):
-    """The cheapest number of slices: 4 us for each column a wave meets, 0.7 and 1.3 / 16 a row for each unit, 3 for the second launch; one where a
-    workgroup's accumulators do not fit."""
+    """The cheapest number of slices whose accumulators fit: 1.22 us for each unit of the longest run, 0.305 for each column that a wave of the
+    workgroup meets, 4.62 for the second launch and 0.24 for a million bytes of sums."""
     if nb <= WAVES:
         return 1
 
@@ -218,10 +218,9 @@ def slices_of(M, N, nb, ncu):
         tiles = tiles_of(s)
         units = ceil_div(nb, s) * tiles
         runs = [(w * units // WAVES, (w + 1) * units // WAVES) for w in range(WAVES)]
-        columns = max((q1 - 1) // tiles - q0 // tiles + 1 for q0, q1 in runs if q1 > q0)
-        return 4 * columns + (0.7 + 1.3 / 16 * deal(N, ncu // s)[0]) * max(q1 - q0 for q0, q1 in runs) + (3 if s > 1 else 0)
-    best = min(range(1, max(1, min(8, SLICE_BYTES // (4 * M * N))) + 1), key=cost)
-    return best if rows_lds(tiles_of(best), 1, False, 1) <= 160 * 1024 else 1
+        columns = sum((q1 - 1) // tiles - q0 // tiles + 1 for q0, q1 in runs if q1 > q0)
+        return 1.22 * max(q1 - q0 for q0, q1 in runs) + 0.305 * columns + (4.62 + 0.24e-6 * 4 * s * M * N if s > 1 else 0)
+    return min([s for s in range(1, max(1, min(8, SLICE_BYTES // (4 * M * N))) + 1) if s == 1 or rows_lds(tiles_of(s), 1, False, 1) <= 160 * 1024], key=cost)
 
 
 def check_rows(M, N, K, normed, dual, ncu=NCU, slices=None):
@@ -337,9 +336,10 @@ def test_a_smaller_device_changes_the_layout_not_the_bounds():
 
 
 SLICED = [   # (M, N, K), slices on 256 compute units
-    ((8, 4096, 4096), 1), ((3, 1100, 4352), 2), ((8, 8192, 8192), 2), ((8, 4096, 12288), 3), ((4, 600, 9000), 3), ((15, 1024, 12288), 3), ((8, 5000, 16384), 4),
-    ((5, 2047, 6148), 5), ((6, 3520, 5280), 6), ((5, 4222, 6228), 7), ((8, 33, 32768), 8),
-    ((8, 12288, 32768), 1),                                         # eight would not fit the LDS
+    ((8, 4096, 4096), 1), ((8, 4096, 4608), 1), ((3, 3642, 4624), 1), ((6, 3520, 5280), 1), ((8, 12288, 4352), 1),
+    ((5, 2047, 6148), 2), ((8, 8192, 8192), 2), ((8, 4096, 12288), 3), ((15, 1024, 12288), 4), ((8, 5000, 16384), 4), ((7, 9695, 9384), 5),
+    ((4, 600, 9000), 6), ((5, 4222, 6228), 7), ((8, 33, 32768), 8),
+    ((8, 12288, 32768), 4),                                         # eight would not fit the LDS
 ]
 
 

@@ -290,8 +290,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
 // 32-bit products of rows within reach (gemm_split.h).  Bound by the matrix cores where tiles are many (at 600 x 18464 x 4096 the three
 // instructions' rate is 1060 TFLOP/s, what the 16-bit products reach), by the steps' latency where they are few; us against 32-bit
 // instructions: 301 x 5136 x 1024 43 -> 18, 301 x 1024 x 4096 37 -> 18, 600 x 18464 x 4096 893 -> 257, 2 x 4096 x 16384 83 -> 34.
-// Distance from 64 bits (2-norm) there 5.7e-7 -> 1.0e-7, 4.7e-7 -> 1.4e-7, 8.1e-7 -> 2.7e-7, 8.1e-7 -> 2.2e-7.  A tile whose sums the parts do not
-// give (an activation that is not the sum of its parts, join_sums) is multiplied again by 32-bit instructions.
+// Distance from 64 bits (2-norm) there 5.7e-7 -> 1.0e-7, 4.7e-7 -> 1.4e-7, 8.1e-7 -> 2.7e-7, 8.1e-7 -> 2.2e-7.  A tile with sums the parts do not
+// give (an activation that is not the sum of its parts, sound_sum) is multiplied again by 32-bit instructions, and those sums are taken from there.
 template <class Tile>
 __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_kernel(const GemmArgs a) {
   extern __shared__ __align__(16) char smem[];
@@ -308,9 +308,19 @@ __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_ker
   dh::f32x4_t sums[Tile::kShare];
   const bool whole = dh::split_product<Tile>(a_base, a_off, w_base, w_off, nk, smem), sound = dh::join_sums<Tile>(sums, smem);
   if (__builtin_expect(!dh::everywhere<Tile>(whole && sound, smem), 0)) {
+    const int* const short_rows = dh::short_rows<Tile>(whole, smem);
     dh::exact_product<Tile>(a_base, a_off, w_base, w_off, nk, smem);
     __syncthreads();
-    (void)dh::join_sums<Tile>(sums, smem);
+    dh::f32x4_t exact[Tile::kShare];
+    (void)dh::join_sums<Tile>(exact, smem);
+    // (the other sums stay what they are whatever the rest of their tile holds)
+#pragma unroll
+    for (int u = 0; u < Tile::kShare; u++) {
+      const dh::SumPlace<Tile> at(u);
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (short_rows[32 * at.wm + 8 * at.q + 4 * ((threadIdx.x & 63) >> 5) + e] || !dh::sound_sum(sums[u][e])) sums[u][e] = exact[u][e];
+    }
   }
   const int lane = threadIdx.x & 63;
 #pragma unroll

@@ -37,7 +37,7 @@ struct SplitTile {
   static constexpr int kBufA = BM * 256, kBufB = BN * 128, kRoundsA = kBufA / (1024 * kWaves), kRoundsB = kBufB / (1024 * kWaves);
   static constexpr int kSums = kWaves * NF * 4096, kShare = WM * NF * 4 / kWaves, kLds = S * (kBufA + kBufB) > kSums ? S * (kBufA + kBufB) : kSums;
   static_assert(kBufA % (1024 * kWaves) == 0 && kBufB % (1024 * kWaves) == 0 && kLds <= 163840, "whole loads");
-  static_assert(kLds >= kSums + 4 * kWaves && WM * NF * 4 % kWaves == 0, "a word a wave behind the sums, whole shares");
+  static_assert(kLds >= kSums + 4 * (kWaves + BM) && WM * NF * 4 % kWaves == 0, "a word a wave and a row behind the sums, whole shares");
 };
 
 // Where a group's sums lie when the loop is over: lane l's four are rows 32 wm + 8 q + 4 (l >> 5) + 0 .. 3 of column 32 j + (l & 31).
@@ -55,9 +55,11 @@ struct SumPlace {
     q = at & 3, j = (at >> 2) % Tile::NF, wm = (at >> 2) / Tile::NF;
   }
 };
-// Adds up the groups' sums; whether they are what the product's are.  Not if one is not finite: the parts of an infinite value, and
-// a part that is zero times an infinite weight, are no numbers where the product is infinite.  Nor if one is of up to 2^-80, which may consist
-// of products of parts that f32 does not hold.
+// Whether a sum of parts is the product's.  Not if it is not finite: the parts of an infinite value, and a part that is zero times an infinite
+// weight, are no numbers where the product is infinite.  Nor if it is of up to 2^-80, which may consist of products of parts that f32 does not
+// hold.
+__device__ __forceinline__ bool sound_sum(float v) { return fabsf(v) <= 3.402823466e38f && (v == 0.f || fabsf(v) >= 0x1p-80f); }
+// Adds up the groups' sums; whether all are sound.
 template <class Tile>
 __device__ __forceinline__ bool join_sums(f32x4_t (&sums)[Tile::kShare], char* smem) {
   bool sound = true;
@@ -68,7 +70,7 @@ __device__ __forceinline__ bool join_sums(f32x4_t (&sums)[Tile::kShare], char* s
 #pragma unroll
     for (int g = 1; g < Tile::KG; g++) sums[u] += split_sums<Tile>(smem, g, at.wm, at.j, at.q)[threadIdx.x & 63];
 #pragma unroll
-    for (int e = 0; e < 4; e++) sound = sound && fabsf(sums[u][e]) <= 3.402823466e38f && (sums[u][e] == 0.f || fabsf(sums[u][e]) >= 0x1p-80f);
+    for (int e = 0; e < 4; e++) sound = sound && sound_sum(sums[u][e]);
   }
   return sound;
 }
@@ -83,6 +85,17 @@ __device__ __forceinline__ bool everywhere(bool here, char* smem) {
 #pragma unroll
   for (int w = 0; w < Tile::kWaves; w++) every &= words[w];
   return __builtin_amdgcn_readfirstlane(every) != 0;
+}
+
+// A word for each of the tile's rows, not zero where a lane that has split some of it found the parts short of it (`whole` is split_product's).
+// In place behind the next barrier.
+template <class Tile>
+__device__ __forceinline__ const int* short_rows(bool whole, char* smem) {
+  int* const rows = reinterpret_cast<int*>(smem + Tile::kSums) + Tile::kWaves;
+  for (int r = threadIdx.x; r < Tile::BM; r += Tile::kThreads) rows[r] = 0;
+  __syncthreads();
+  if (!whole) rows[32 * ((threadIdx.x >> 6) % Tile::WM) + (threadIdx.x & 31)] = 1;
+  return rows;
 }
 
 // The same tile on v_mfma_f32_32x32x2_f32, operands from memory into registers: for a tile whose sums the parts do not give.  Waves take the

@@ -348,6 +348,13 @@ def test_dense_matmul_f32_far_from_one(L, M, N, K):
     capi.check(L.dh_sync())
     bound = K / 8 * 2.0 ** -25 * (a.abs() @ w.abs().T) + 2 * K * 2.0 ** -150
     assert bool(((got.double() - a @ w.T).abs() <= bound).all())
+    # the rows beside them are what they are without them
+    A[:8] = A[8]
+    beside = torch.zeros(M, N, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul(A.data_ptr(), capi.F32, K, W.data_ptr(), K, M, N, K, 1.0, None, None, beside.data_ptr(), N, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_sync())
+    assert torch.equal(got[8:], beside[8:])
 
 
 @pytest.mark.parametrize("M,N,K", [(9, 70, 128), (301, 1024, 4096), (600, 10255, 2112)])
@@ -389,9 +396,8 @@ def test_dense_matmul_f32_rows_that_are_no_numbers_cost_little(L):
     A[200, 17] = math.nan
     torch.cuda.synchronize()
     one = fastest()
-    assert C[200].isnan().all() and torch.equal(C[:128], sums[:128]) and torch.equal(C[256:], sums[256:])
-    rows = [m for m in range(128, 256) if m != 200]
-    assert ((C - sums)[rows].norm() / sums[rows].norm()) < 4e-6
+    rows = [m for m in range(M) if m != 200]
+    assert C[200].isnan().all() and torch.equal(C[rows], sums[rows])
     A[:, 5] = math.inf
     torch.cuda.synchronize()
     every = fastest()

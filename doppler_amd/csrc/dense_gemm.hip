@@ -183,15 +183,16 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const Gem
   auto a_off = [&](int row) { return (uint32_t)((source_row<GROUPED>(a, place, row) - first) * a.lda * 2); };
   auto w_off = [&](int row) { return (uint32_t)(min(row, a.N - 1 - n0) * a.ldw * 2); };
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / Tile::WN, wn = wave % Tile::WN;
+  const dh::Company company{m0 / Tile::BM, (place.rows + Tile::BM - 1) / Tile::BM};
   if constexpr (Tile::FA == 0) {
     f32x16_t acc[Tile::G];
-    dh::small_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem);
+    dh::small_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
     const int m = m0 + 32 * wm, n = n0 + 32 * Tile::G * wn;
     if constexpr (GLU) store_glu(a, place, acc[0], acc[1], m, n, lane);
     else store_tile<ACT>(a, place, acc[0], m, n, lane);
   } else {
     f32x16_t acc[2 * Tile::FA][2 * Tile::FB];
-    dh::wide_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem);
+    dh::wide_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
     const int m = m0 + 64 * Tile::FA * wm, n = n0 + 64 * Tile::FB * wn;
 #pragma unroll
     for (int i = 0; i < 2 * Tile::FA; i++) {
@@ -366,11 +367,11 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
 // Tiles of the 16-bit products, and what they cost in ns: a k step (64 elements) `alone` with few workgroups on the device, `one` with one
 // on every compute unit, `full` with as many as fit (the two larger tiles: one, which takes more than half of the LDS); outside the k
 // loop `start`, and `again` for every further round of workgroups.  The device slows its clock under matrix-core load, so a step gets
-// dearer as more compute units join, and idle ones are not all lost.  Fitted to 446 products (M 2 .. 2048, N 16 .. 32000, K 64 .. 16384) with each
-// tile and up to 16 slices, weights from HBM as a model's layers in turn have them (a step waits for those: 2048 x 1152 x 6912 on
-// 128 x 128 tiles takes 46 us with weights from the cache, 68 from HBM): the choice is 0.7 % behind the best on average, 20 % at worst.
+// dearer as more compute units join, and idle ones are not all lost.  Fitted to 300 products (M 16 .. 2100, N 200 .. 20000, K 256 .. 16384) with each
+// tile and up to 16 slices, weights from HBM as a model's layers in turn have them: the choice is 0.5 % behind the best on average, 15 % at
+// worst (1.1 % and 30 % with the costs of tiles that did not ask for their weights ahead).
 // Against the 128 x 128 and 64 x 64 tiles through registers that were here before, us: 2048 x 18464 x 4096
-// 421 -> 306, 2048 x 4096 x 16384 329 -> 261, 1531 x 2048 x 6144 70 -> 63, 300 x 2048 x 2048 18.4 -> 11.3, 33 x 5120 x 1024 14.6 -> 7.2,
+// 421 -> 299, 2048 x 4096 x 16384 329 -> 224, 1531 x 2048 x 6144 70 -> 51, 300 x 2048 x 2048 18.4 -> 11.3, 33 x 5120 x 1024 14.6 -> 7.2,
 // 700 x 1024 x 1024 14.1 -> 7.4; behind them still: 33 x 4096 x 16384 30.6 -> 33.1 (2 rows 28.5 -> 32.7) and few rows at K 64.
 using Tile256x256 = dh::WideTile<2, 4, 2, 1>;
 using Tile256x128 = dh::WideTile<4, 2, 1, 1>;
@@ -381,10 +382,10 @@ struct TileCost {
   int bm, bn, per_cu;
   float alone, one, full, start, again;
 };
-constexpr TileCost kTiles[] = {{256, 256, 1, 1075.f, 1590.f, 1840.f, 9300.f, 5300.f},
-                               {256, 128, 1, 610.f, 825.f, 825.f, 12300.f, 6000.f},
-                               {128, 128, 2, 360.f, 645.f, 1415.f, 5000.f, 3100.f},
-                               {64, 64, 2, 232.f, 294.f, 516.f, 4100.f, 1400.f}};
+constexpr TileCost kTiles[] = {{256, 256, 1, 993.f, 1464.f, 1627.f, 8987.f, 8447.f},
+                               {256, 128, 1, 457.f, 808.f, 899.f, 11078.f, 4801.f},
+                               {128, 128, 2, 396.f, 619.f, 1337.f, 5092.f, 2173.f},
+                               {64, 64, 2, 163.f, 294.f, 498.f, 5060.f, 803.f}};
 // gate and up products, never sliced
 constexpr TileCost kGluTiles[] = {{256, 256, 1, 900.f, 1720.f, 1720.f, 8000.f, 0.f},
                                   {256, 128, 1, 520.f, 930.f, 930.f, 5500.f, 0.f},
@@ -416,8 +417,8 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool gl
     const TileCost& c = glu ? kGluTiles[i] : kTiles[i];
     for (int s = 1; s <= most_slices && (s == 1 || steps / s >= kMinSliceSteps); s++) {
       const int64_t groups = dh::ceil_div(M, c.bm) * dh::ceil_div(N, c.bn) * s;
-      double t = std::max(loops_ns(c, groups, dh::ceil_div(steps, s), 0.76), 2.0 * N * K / 6450.0) + c.start;
-      if (s > 1) t += 2250.0 + 4.0 * M * N * (2 * s + 1) / 4150.0;
+      double t = std::max(loops_ns(c, groups, dh::ceil_div(steps, s), 0.76), 2.0 * N * K / (glu ? 6450.0 : 6950.0)) + c.start;
+      if (s > 1) t += 2550.0 + 4.0 * M * N * (2 * s + 1) / 4300.0;
       else if (erf) t += (c.per_cu == 1 ? 60.0 : 40.0) * (c.bm * c.bn / 64) * dh::ceil_div(groups, dh::num_cus());
       if (t < least) {
         least = t;

@@ -13,7 +13,8 @@ struct WideTile {
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kRound = 1024 * kWaves;                             // bytes all waves fetch with one load each: 8 rows a wave
   static constexpr int kRoundsA = kHalfA / kRound, kRoundsB = kHalfB / kRound;
-  static constexpr int kLds = 4 * (kHalfA + kHalfB);
+  static constexpr int kAhead = BM * BN < 256 * 256 ? 4 : 0, kScratch = 4 * (kHalfA + kHalfB);   // WeightLines
+  static constexpr int kLds = kScratch + (kAhead ? 256 : 0);
   static_assert(kHalfA % kRound == 0 && kHalfB % kRound == 0, "whole loads");
 };
 
@@ -32,12 +33,48 @@ __device__ __forceinline__ void fetch_to_lds(const buffer_words_t& words, uint32
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
                : "m0", "memory");
 }
+// The same with 4 bytes per lane, at lds + 4 * lane.
+__device__ __forceinline__ void touch_to_lds(const buffer_words_t& words, uint32_t v_off, uint32_t s_off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
+               : "m0", "memory");
+}
 #pragma clang diagnostic pop
 // At most `fetches` of this wave's fetches still in flight, all its LDS reads done, then the other waves.
 template <int fetches>
 __device__ __forceinline__ void arrive_and_wait() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(fetches) : "memory");
 }
+
+// The workgroups whose tiles lie in one stretch of columns read the same weights at about the same time.  Those come from HBM, about 1 us
+// away, which the fetches of a tile below 256 x 256 are not far enough ahead for, and every one of the company then waits for the
+// same lines.  So they take turns: at step t of every `count` one of them asks for a word of every line of step t + kAhead (64 lines a wave and
+// instruction), which brings the line into the L2 of their die; the words land in 256 bytes of LDS that nobody reads.  us, weights from HBM:
+// 1531 x 2048 x 6144 on 128 x 128 tiles 62 -> 51 (44 with weights that the 256 MB cache still holds), 1531 x 2048 x 3072 34 -> 27, 600 x 4096 x 4096
+// 36 -> 32, 2048 x 4096 x 16384 on 256 x 128 264 -> 226, 300 x 6144 x 2048 on 64 x 64 19.2 -> 18.1.  Fewer than four tiles gain nothing (100 x 4096 x 12288
+// on 64 x 64 54 -> 55), a 256 x 256 tile's step is longer than the way to HBM (47 -> 47.5), and activations asked for in the same way cost what
+// they give (they are in the cache, having just been written).
+// The waits below count fetches; a line asked for in between makes a wait reach one fetch further than it must, never less far.
+struct Company {
+  int index, count;
+};
+template <class Tile>
+struct WeightLines {
+  static constexpr int kLeast = 4;
+  const buffer_words_t& words;
+  uint32_t v_off, s_off, lds;
+  int next, every, last;
+  template <class OffW>
+  __device__ __forceinline__ WeightLines(const buffer_words_t& ww, OffW w_off, uint32_t k_bytes, int nk, uint32_t lds0, int wave, int lane, Company c)
+      : words(ww), v_off(w_off((wave % (Tile::BN / 64)) * 64 + lane)), s_off(k_bytes), lds(lds0 + Tile::kScratch), next(c.index),
+        every(c.count), last(c.count >= kLeast && wave < Tile::BN / 64 ? nk : 0) {
+    for (int t = next; t < Tile::kAhead && t < last; t += every) touch_to_lds(words, v_off, s_off + 128u * (uint32_t)t, lds);
+  }
+  __device__ __forceinline__ void at(int t) {
+    if (t != next) return;
+    next += every;
+    if (t + Tile::kAhead < last) touch_to_lds(words, v_off, s_off + 128u * (uint32_t)(t + Tile::kAhead), lds);
+  }
+};
 
 // One tile.  a_off / w_off give the byte offset of a tile's row from the base (below 4 GB); rows of both operands hold nk * 64
 // elements of k from there, 16-byte aligned.  Results: acc[i][j], 32 x 32 each, wave (wm, wn) at rows 64 FA wm, columns 64 FB wn.
@@ -58,7 +95,7 @@ __device__ __forceinline__ void arrive_and_wait() {
 // banks, and since a fetch writes 64 consecutive pieces, every lane fetches the piece that belongs there.
 template <class Tile, bool F16, class OffA, class OffW>
 __device__ __forceinline__ void wide_product(f32x16_t (&acc)[2 * Tile::FA][2 * Tile::FB], const void* a_base, OffA a_off, const void* w_base,
-                                             OffW w_off, uint32_t k_bytes, int nk, char* smem) {
+                                             OffW w_off, uint32_t k_bytes, int nk, char* smem, Company company) {
   constexpr int FA = Tile::FA, FB = Tile::FB, RA = Tile::kRoundsA, RB = Tile::kRoundsB, HA = Tile::kHalfA, HB = Tile::kHalfB;
   constexpr int kStep = 2 * (RA + RB);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -141,7 +178,15 @@ __device__ __forceinline__ void wide_product(f32x16_t (&acc)[2 * Tile::FA][2 * T
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
 
-  auto step = [&](int t, auto parity) {
+  struct NoLines {
+    __device__ __forceinline__ void at(int) {}
+  };
+  auto weight_lines = [&] {
+    if constexpr (Tile::kAhead > 0) return WeightLines<Tile>(ww, w_off, k_bytes, nk, lds0, wave, lane, company);
+    else return NoLines{};
+  };
+  auto step = [&](int t, auto parity, auto& lines) {
+    lines.at(t);
     constexpr int P = decltype(parity)::value, Q = P ^ 1;
     using IP = std::integral_constant<int, P>;
     using IQ = std::integral_constant<int, Q>;
@@ -179,6 +224,7 @@ __device__ __forceinline__ void wide_product(f32x16_t (&acc)[2 * Tile::FA][2 * T
   fetch_b(0, 1, 1);
   fetch_b(1, 1, 1);
   fetch_a(1, 1, 1);
+  auto lines = weight_lines();
   arrive_and_wait<2 * kStep - RA - RB>();  // A0 (0), B0 (0)
 #pragma unroll
   for (int i = 0; i < 4 * FA; i++) DH_READ_A(0, 0, i >> 2, i & 3);
@@ -189,10 +235,10 @@ __device__ __forceinline__ void wide_product(f32x16_t (&acc)[2 * Tile::FA][2 * T
   arrive_and_wait<kStep + 2 * RA>();       // B1 (0)
   int t = 0;
   for (; t + 2 <= nk; t += 2) {
-    step(t, I0{});
-    step(t + 1, I1{});
+    step(t, I0{}, lines);
+    step(t + 1, I1{}, lines);
   }
-  if (t < nk) step(t, I0{});
+  if (t < nk) step(t, I0{}, lines);
   // nothing may be in flight towards LDS when the workgroup ends, and the next tile starts from an idle LDS
   arrive_and_wait<0>();
 #undef DH_READ_A
@@ -207,12 +253,12 @@ struct SmallTile {
   static constexpr int WM = WM_, WN = WN_, G = G_, FA = 0, FB = 0;
   static constexpr int BM = 32 * WM, BN = 32 * G * WN, kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kBufA = BM * 128, kBufB = BN * 128, kRoundsA = kBufA / (1024 * kWaves), kRoundsB = kBufB / (1024 * kWaves);
-  static constexpr int kLds = 4 * (kBufA + kBufB);
+  static constexpr int kAhead = 8, kScratch = 4 * (kBufA + kBufB), kLds = kScratch + 256;      // WeightLines
   static_assert(kBufA % (1024 * kWaves) == 0 && kBufB % (1024 * kWaves) == 0 && 4 * kBufA <= 65536 && 4 * kBufB <= 65536, "whole loads");
 };
 template <class Tile, bool F16, class OffA, class OffW>
 __device__ __forceinline__ void small_product(f32x16_t (&acc)[Tile::G], const void* a_base, OffA a_off, const void* w_base, OffW w_off, uint32_t k_bytes, int nk,
-                                              char* smem) {
+                                              char* smem, Company company) {
   constexpr int G = Tile::G, RA = Tile::kRoundsA, RB = Tile::kRoundsB, R = RA + RB;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / Tile::WN, wn = wave % Tile::WN;
@@ -245,8 +291,13 @@ __device__ __forceinline__ void small_product(f32x16_t (&acc)[Tile::G], const vo
   for (int g = 0; g < G; g++)
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[g][e] = 0.f;
+  fetch(0, 0);
+  fetch(1, 1);
+  fetch(2, 2);
+  WeightLines<Tile> lines(ww, w_off, k_bytes, nk, lds0, wave, lane, company);
   auto step = [&](int t, auto buffer) {
     constexpr int B = decltype(buffer)::value;
+    lines.at(t);
     arrive_and_wait<2 * R>();                // step t is there for all, and all have read step t - 1
     fetch(t + 3, (B + 3) & 3);
     u32x4_t fa[4], fb[4][G];
@@ -266,9 +317,6 @@ __device__ __forceinline__ void small_product(f32x16_t (&acc)[Tile::G], const vo
           acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fa[ks]), __builtin_bit_cast(bf16x8_t, fb[ks][g]), acc[g], 0, 0, 0);
       }
   };
-  fetch(0, 0);
-  fetch(1, 1);
-  fetch(2, 2);
   for (int t = 0;; t += 4) {
     step(t, std::integral_constant<int, 0>{});
     if (t + 1 >= nk) break;

@@ -66,17 +66,28 @@ __device__ __forceinline__ void put_c2(const GemmArgs& a, int64_t at, float v) {
   else static_cast<float*>(a.C2)[at] = v;
 }
 
-// The two outputs of one element.
-__device__ __forceinline__ void put(const GemmArgs& a, int m, int n, float acc) {
+// The two outputs of one element; what the first adds and multiplies in is requested before anything is stored (see below).
+struct PutTerms {
+  float bias, scale, residual;
+};
+__device__ __forceinline__ PutTerms put_terms(const GemmArgs& a, int m, int n) {
+  PutTerms t{0.f, 1.f, 0.f};
   if (n < a.n_first) {
-    const int64_t at = (int64_t)m * a.ldc + n;
-    float v = fmaf(acc, a.alpha, a.bias ? a.bias[n] : 0.f);
-    if (a.col_scale) v *= a.col_scale[n];
-    if (a.residual) v += a.residual[at];
-    a.C[at] = v;
-  } else {
-    put_c2(a, (int64_t)m * a.ldc2 + (n - a.n_first), dh::activate(acc * a.alpha, a.act));
+    if (a.bias) t.bias = a.bias[n];
+    if (a.col_scale) t.scale = a.col_scale[n];
+    if (a.residual) t.residual = a.residual[(int64_t)m * a.ldc + n];
   }
+  return t;
+}
+__device__ __forceinline__ float first_output(const GemmArgs& a, const PutTerms& t, float acc) {
+  float v = fmaf(acc, a.alpha, t.bias);
+  if (a.col_scale) v *= t.scale;
+  if (a.residual) v += t.residual;
+  return v;
+}
+__device__ __forceinline__ void put(const GemmArgs& a, const PutTerms& t, int m, int n, float acc) {
+  if (n < a.n_first) a.C[(int64_t)m * a.ldc + n] = first_output(a, t, acc);
+  else put_c2(a, (int64_t)m * a.ldc2 + (n - a.n_first), dh::activate(acc * a.alpha, a.act));
 }
 
 // Where a workgroup's tile lies: its rows (base + 0 .. rows - 1 of the outputs), its first row among them, its weights.
@@ -105,65 +116,117 @@ __device__ __forceinline__ int64_t source_row(const GemmArgs& a, const TilePlace
 }
 
 // One 32 x 32 accumulator tile: lane l holds column l & 31 and rows 8 (i / 4) + 4 (l >> 5) + i % 4.
+//
+// An epilogue requests all it adds and multiplies in (several tiles' residuals at a time) in front of its first store, and computes a tile's
+// values before it stores them: a load behind a store waits for the store's trip to memory as well, and values between the branches of
+// ragged rows are computed one after the other.  Sixteen round trips for a tile of gated pairs took 18 us of 68 (1531 x 6144 x 2048).
+__device__ __forceinline__ int tile_row(int mb, int i) { return mb + 8 * (i >> 2) + (i & 3); }
+
+struct ColumnTerms {       // of one column of the first output
+  float alpha, bias;
+};
+__device__ __forceinline__ ColumnTerms column_terms(const GemmArgs& a, int n0, int lane) {
+  const int n = n0 + (lane & 31);
+  const bool here = n < a.n_first;
+  const float scale = here && a.col_scale ? a.col_scale[n] : 1.f;
+  return {a.alpha * scale, (here && a.bias ? a.bias[n] : 0.f) * scale};
+}
+// (every read in front of the first write, also because the residual may be the output itself)
+__device__ __forceinline__ void load_residual(const GemmArgs& a, const TilePlace& p, float (&r)[16], int m0, int n0, int lane) {
+  const int n = n0 + (lane & 31), mb = m0 + 4 * (lane >> 5);
+  const float* res = a.residual + (int64_t)p.base * a.ldc + min(n, a.n_first - 1);
+#pragma unroll
+  for (int i = 0; i < 16; i++) r[i] = res[(int64_t)min(tile_row(mb, i), p.rows - 1) * a.ldc];
+}
+template <class T, class Value>
+__device__ __forceinline__ void store_rows(T* c, int64_t ld, int mb, int rows, Value&& value) {
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int m = tile_row(mb, i);
+    if (m < rows) c[(int64_t)m * ld] = value(i);
+  }
+}
+__device__ __forceinline__ void store_c2(const GemmArgs& a, int64_t at, int mb, int rows, const float (&v)[16]) {
+  if (a.c2_dtype == DH_BF16) store_rows(static_cast<uint16_t*>(a.C2) + at, a.ldc2, mb, rows, [&](int i) { return dh::f32_to_bf16_bits(v[i]); });
+  else if (a.c2_dtype == DH_F16) store_rows(static_cast<_Float16*>(a.C2) + at, a.ldc2, mb, rows, [&](int i) { return (_Float16)v[i]; });
+  else store_rows(static_cast<float*>(a.C2) + at, a.ldc2, mb, rows, [&](int i) { return v[i]; });
+}
 template <int ACT>
-__device__ __forceinline__ void store_tile(const GemmArgs& a, const TilePlace& p, const f32x16_t& acc, int m0, int n0, int lane) {
+__device__ __forceinline__ void store_tile(const GemmArgs& a, const TilePlace& p, const f32x16_t& acc, const ColumnTerms& col, const float (&r)[16], int m0,
+                                           int n0, int lane) {
   const int n = n0 + (lane & 31);
   if (n >= a.N) return;
   const int mb = m0 + 4 * (lane >> 5);
   if (a.parts) {
-    float* q = a.parts + (int64_t)blockIdx.y * a.M * a.N;
+    store_rows(a.parts + (int64_t)blockIdx.y * a.M * a.N + n, a.N, mb, a.M, [&](int i) { return acc[i]; });
+  } else if (ACT == kNoSecond || n < a.n_first) {
+    float* c = a.C + (int64_t)p.base * a.ldc + n;
+    if (a.residual) store_rows(c, a.ldc, mb, p.rows, [&](int i) { return fmaf(acc[i], col.alpha, col.bias) + r[i]; });
+    else store_rows(c, a.ldc, mb, p.rows, [&](int i) { return fmaf(acc[i], col.alpha, col.bias); });
+  } else if constexpr (ACT == kAnyAct) {      // (one value at a time: sixteen of each activation are too much code)
+    const int64_t at = (int64_t)p.base * a.ldc2 + (n - a.n_first);
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-      const int m = mb + 8 * (i >> 2) + (i & 3);
-      if (m < a.M) q[(int64_t)m * a.N + n] = acc[i];
-    }
-    return;
-  }
-  if (ACT == kNoSecond || n < a.n_first) {
-    const float scale = a.col_scale ? a.col_scale[n] : 1.f, bias = (a.bias ? a.bias[n] : 0.f) * scale, alpha = a.alpha * scale;
-    float* c = a.C + (int64_t)p.base * a.ldc + n;
-    if (a.residual) {
-      // every read in front of the first write: the residual may be the output itself
-      const float* res = a.residual + (int64_t)p.base * a.ldc + n;
-      float r[16];
-#pragma unroll
-      for (int i = 0; i < 16; i++) r[i] = res[(int64_t)min(mb + 8 * (i >> 2) + (i & 3), p.rows - 1) * a.ldc];
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        const int m = mb + 8 * (i >> 2) + (i & 3);
-        if (m < p.rows) c[(int64_t)m * a.ldc] = fmaf(acc[i], alpha, bias) + r[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        const int m = mb + 8 * (i >> 2) + (i & 3);
-        if (m < p.rows) c[(int64_t)m * a.ldc] = fmaf(acc[i], alpha, bias);
-      }
+      const int m = tile_row(mb, i);
+      if (m < p.rows) put_c2(a, at + (int64_t)m * a.ldc2, dh::activate(acc[i] * a.alpha, a.act));
     }
   } else {
-    const int64_t at = (int64_t)p.base * a.ldc2 + (n - a.n_first);
-    const int act = ACT == kAnyAct ? a.act : ACT;
+    float v[16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int m = mb + 8 * (i >> 2) + (i & 3);
-      if (m < p.rows) put_c2(a, at + (int64_t)m * a.ldc2, dh::activate(acc[i] * a.alpha, act));
-    }
+    for (int i = 0; i < 16; i++) v[i] = dh::activate(acc[i] * a.alpha, ACT);
+    store_c2(a, (int64_t)p.base * a.ldc2 + (n - a.n_first), mb, p.rows, v);
   }
 }
-// The same for a gate tile and the up tile beside it (first weight row n0 of the gate block).
-__device__ __forceinline__ void store_glu(const GemmArgs& a, const TilePlace& p, const f32x16_t& gate, const f32x16_t& up, int m0, int n0,
-                                          int lane) {
-  if (n0 >= a.N) return;
-  const int col = (n0 >> 1) + (lane & 31), mb = m0 + 4 * (lane >> 5);
+// Tiles AT .. of a wave's R x C; residuals of four tiles at a time.
+template <int ACT, int AT, int R, int C>
+__device__ __forceinline__ void store_from(const GemmArgs& a, const TilePlace& p, const f32x16_t (&acc)[R][C], const ColumnTerms (&col)[C],
+                                           bool with_residual, int m0, int n0, int lane) {
+  constexpr int kBatch = R * C < 4 ? R * C : 4;
+  float r[kBatch][16];
+  if (with_residual) {
 #pragma unroll
-  for (int i = 0; i < 16; i++) {
-    const int m = mb + 8 * (i >> 2) + (i & 3);
-    if (m >= p.rows) continue;
-    const int64_t r = p.base + m;
-    const float w = a.rows.row_in ? a.rows.row_in[r] : 1.f;
-    float y = dh::clamped_glu(w * gate[i], w * up[i], a.rows.limit);
-    if (a.rows.row_out) y *= a.rows.row_out[r];
-    put_c2(a, r * a.ldc2 + col, y);
+    for (int u = 0; u < kBatch; u++) load_residual(a, p, r[u], m0 + 32 * ((AT + u) / C), n0 + 32 * ((AT + u) % C), lane);
+  }
+#pragma unroll
+  for (int u = 0; u < kBatch; u++)
+    store_tile<ACT>(a, p, acc[(AT + u) / C][(AT + u) % C], col[(AT + u) % C], r[u], m0 + 32 * ((AT + u) / C), n0 + 32 * ((AT + u) % C), lane);
+  if constexpr (AT + kBatch < R * C) store_from<ACT, AT + kBatch>(a, p, acc, col, with_residual, m0, n0, lane);
+}
+template <int ACT, int R, int C>
+__device__ __forceinline__ void store_tiles(const GemmArgs& a, const TilePlace& p, const f32x16_t (&acc)[R][C], int m0, int n0, int lane) {
+  ColumnTerms col[C];
+#pragma unroll
+  for (int j = 0; j < C; j++) col[j] = column_terms(a, n0 + 32 * j, lane);
+  store_from<ACT, 0>(a, p, acc, col, a.residual && !a.parts && (ACT == kNoSecond || n0 < a.n_first), m0, n0, lane);
+}
+// The same for R gate tiles and the up tiles beside them (first weight row n0 of the gate block).
+template <int R>
+__device__ __forceinline__ void store_glu(const GemmArgs& a, const TilePlace& p, const f32x16_t (&acc)[R][2], int m0, int n0, int lane) {
+  if (n0 >= a.N) return;
+  const int mb = m0 + 4 * (lane >> 5);
+  float f[R][16];          // a row's factor, on what goes in or on what comes out
+  const float* factors = a.rows.row_in ? a.rows.row_in : a.rows.row_out;
+  if (factors) {
+#pragma unroll
+    for (int t = 0; t < R; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) f[t][i] = factors[p.base + min(tile_row(mb + 32 * t, i), p.rows - 1)];
+  } else {
+#pragma unroll
+    for (int t = 0; t < R; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) f[t][i] = 1.f;
+  }
+  const bool in = a.rows.row_in != nullptr;
+#pragma unroll
+  for (int t = 0; t < R; t++) {
+    float y[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const float w = in ? f[t][i] : 1.f;
+      y[i] = dh::clamped_glu(w * acc[t][0][i], w * acc[t][1][i], a.rows.limit) * (in ? 1.f : f[t][i]);
+    }
+    store_c2(a, (int64_t)p.base * a.ldc2 + (n0 >> 1) + (lane & 31), mb + 32 * t, p.rows, y);
   }
 }
 
@@ -185,24 +248,17 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_16bit_kernel(const Gem
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave / Tile::WN, wn = wave % Tile::WN;
   const dh::Company company{m0 / Tile::BM, (place.rows + Tile::BM - 1) / Tile::BM};
   if constexpr (Tile::FA == 0) {
-    f32x16_t acc[Tile::G];
-    dh::small_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
+    f32x16_t acc[1][Tile::G];
+    dh::small_product<Tile, F16>(acc[0], a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
     const int m = m0 + 32 * wm, n = n0 + 32 * Tile::G * wn;
-    if constexpr (GLU) store_glu(a, place, acc[0], acc[1], m, n, lane);
-    else store_tile<ACT>(a, place, acc[0], m, n, lane);
+    if constexpr (GLU) store_glu(a, place, acc, m, n, lane);
+    else store_tiles<ACT>(a, place, acc, m, n, lane);
   } else {
     f32x16_t acc[2 * Tile::FA][2 * Tile::FB];
     dh::wide_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
     const int m = m0 + 64 * Tile::FA * wm, n = n0 + 64 * Tile::FB * wn;
-#pragma unroll
-    for (int i = 0; i < 2 * Tile::FA; i++) {
-      if constexpr (GLU) {
-        store_glu(a, place, acc[i][0], acc[i][1], m + 32 * i, n, lane);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2 * Tile::FB; j++) store_tile<ACT>(a, place, acc[i][j], m + 32 * i, n + 32 * j, lane);
-      }
-    }
+    if constexpr (GLU) store_glu(a, place, acc, m, n, lane);
+    else store_tiles<ACT>(a, place, acc, m, n, lane);
   }
 }
 
@@ -236,11 +292,11 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
   for (int r = 0; r < TN; r++) pb[r] = place.W + (int64_t)min(n0 + 64 * r + (tid >> 2), a.N - 1) * a.ldw + 8 * (tid & 3) + k0;
   f32x4_t ra[2];
   u32x4_t rb[TN];
-  f32x16_t acc[TN];
+  f32x16_t acc[1][TN];
 #pragma unroll
   for (int j = 0; j < TN; j++)
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[j][e] = 0.f;
+    for (int e = 0; e < 16; e++) acc[0][j][e] = 0.f;
   auto load = [&](int kt) {
 #pragma unroll
     for (int r = 0; r < 2; r++) ra[r] = *reinterpret_cast<const f32x4_t*>(pa[r] + BK * kt);
@@ -274,18 +330,14 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
       for (int j = 0; j < TN; j++) {
         const f32x4_t fb = *reinterpret_cast<const f32x4_t*>(&lb[buf][(32 * (wn * TN + j) + (lane & 31)) * ROW + k]);
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc[j], 0, 0, 0);
+        for (int e = 0; e < 4; e++) acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc[0][j], 0, 0, 0);
       }
     }
     if (kt + 1 < nk) store(buf ^ 1);
     __syncthreads();
   }
-  if constexpr (GLU) {
-    store_glu(a, place, acc[0], acc[1], m0 + 32 * wm, n0 + 32 * wn * TN, lane);
-  } else {
-#pragma unroll
-    for (int j = 0; j < TN; j++) store_tile<kAnyAct>(a, place, acc[j], m0 + 32 * wm, n0 + 32 * (wn * TN + j), lane);
-  }
+  if constexpr (GLU) store_glu(a, place, acc, m0 + 32 * wm, n0 + 32 * wn * TN, lane);
+  else store_tiles<kAnyAct>(a, place, acc, m0 + 32 * wm, n0 + 32 * wn * TN, lane);
 }
 
 // 32-bit products of rows within reach (gemm_split.h).  Bound by the matrix cores where tiles are many (at 600 x 18464 x 4096 the three
@@ -324,6 +376,16 @@ __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_ker
     }
   }
   const int lane = threadIdx.x & 63;
+  PutTerms terms[Tile::kShare][4];
+  if (!a.parts) {
+#pragma unroll
+    for (int u = 0; u < Tile::kShare; u++) {
+      const dh::SumPlace<Tile> at(u);
+      const int n = n0 + 32 * at.j + (lane & 31), row = 32 * at.wm + 8 * at.q + 4 * (lane >> 5);
+#pragma unroll
+      for (int e = 0; e < 4; e++) terms[u][e] = put_terms(a, min(m0 + row + e, a.M - 1), n);
+    }
+  }
 #pragma unroll
   for (int u = 0; u < Tile::kShare; u++) {
     const dh::SumPlace<Tile> at(u);
@@ -334,7 +396,7 @@ __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_ker
       const int m = m0 + row + e;
       if (m >= a.M) break;
       if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = sums[u][e];
-      else put(a, m, n, sums[u][e]);
+      else put(a, terms[u][e], m, n, sums[u][e]);
     }
   }
 }
@@ -349,6 +411,15 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
   for (int m = (blockIdx.y << (8 - log2_wide)) + (threadIdx.x >> log2_wide); m < a.M; m += round) {
     const float* p = a.parts + (int64_t)m * a.N + n;
     float s[VEC] = {};
+    PutTerms terms[VEC];
+    const bool whole = VEC == 4 && n + 3 < a.n_first && a.ldc % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.residual)) & 15) == 0;
+    f32x4_t residual = {0.f, 0.f, 0.f, 0.f};
+    if (whole && a.residual) residual = *reinterpret_cast<const f32x4_t*>(a.residual + (int64_t)m * a.ldc + n);
+#pragma unroll
+    for (int e = 0; e < VEC; e++) {
+      if (whole) terms[e] = PutTerms{a.bias ? a.bias[n + e] : 0.f, a.col_scale ? a.col_scale[n + e] : 1.f, residual[e]};
+      else terms[e] = put_terms(a, m, n + e);
+    }
 #pragma unroll 4
     for (int k = 0; k < slices; k++) {
       if constexpr (VEC == 4) {
@@ -359,8 +430,15 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
         s[0] += p[k * total];
       }
     }
+    if (whole) {
+      f32x4_t v;
 #pragma unroll
-    for (int e = 0; e < VEC; e++) put(a, m, n + e, s[e]);
+      for (int e = 0; e < VEC; e++) v[e] = first_output(a, terms[e], s[e]);
+      *reinterpret_cast<f32x4_t*>(a.C + (int64_t)m * a.ldc + n) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; e++) put(a, terms[e], m, n + e, s[e]);
+    }
   }
 }
 

@@ -268,6 +268,65 @@ __device__ __forceinline__ float gelu_tanh_fast(float x) {
 }
 
 
+// A wave's 32 x 32 accumulator tiles: value(q, matrix, e), row(q, e) of the workgroup's tile, column col(q), a row's factor unscale(row).  A tile's
+// values are computed before they are stored, and several tiles' residuals requested in front of their first store: a load behind a store waits
+// for the store's trip to memory as well (sixteen of them a tile took half of 64 x 4096 x 4096 with a residual).
+template <bool DUAL, int TILES, class Value, class Row, class Col, class Unscale>
+__device__ __forceinline__ void store_results(const GemmArgs& a, int m0, Value&& value, Row&& row, Col&& col, Unscale&& unscale) {
+  constexpr int kBatch = TILES > 4 ? 2 : TILES;         // (eight tiles leave registers for two more)
+  const bool with_residual = !DUAL && a.residual && a.ksplit <= 1;
+#pragma unroll
+  for (int q0 = 0; q0 < TILES; q0 += kBatch) {
+    float res[kBatch][16];
+    if (with_residual) {
+#pragma unroll
+      for (int u = 0; u < kBatch; u++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) res[u][e] = a.residual[(int64_t)min(m0 + row(q0 + u, e), a.M - 1) * a.N + min(col(q0 + u), a.N - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; u++) {
+      const int q = q0 + u, n = col(q);
+      float v[16];
+      if constexpr (DUAL) {
+        auto gated = [&](auto&& act) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) {
+            const float factor = unscale(row(q, e));
+            v[e] = act(value(q, 0, e) * factor) * (value(q, 1, e) * factor) * a.alpha;
+          }
+        };
+        if (a.activation == DH_ACT_SILU) {
+          gated([](float g) { return act_silu(g); });
+          if (a.clamp_max > 0.f)
+#pragma unroll
+            for (int e = 0; e < 16; e++) v[e] = fminf(fmaxf(v[e], -a.clamp_max), a.clamp_max);
+        } else {
+          gated([](float g) { return gelu_tanh_fast(g); });
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; e++) v[e] = value(q, 0, e) * unscale(row(q, e));
+        if (a.ksplit <= 1) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) v[e] = v[e] * a.alpha + (with_residual ? res[u][e] : 0.f);
+        }
+      }
+      if (n >= a.N) continue;
+      auto store = [&](auto* c, auto&& as) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          const int m = m0 + row(q, e);
+          if (m < a.M) c[(int64_t)m * a.N + n] = as(v[e]);
+        }
+      };
+      if (!DUAL && a.ksplit > 1) store(a.partial + (int64_t)blockIdx.z * a.M * a.N, [](float x) { return x; });
+      else if (a.c_f16) store(reinterpret_cast<__half*>(a.C), [](float x) { return __float2half(x); });
+      else store(reinterpret_cast<float*>(a.C), [](float x) { return x; });
+    }
+  }
+}
+
 // T = MFMA tiles per wave along each of M and N (T = 2: a 64 x 64 quadrant per wave, T = 1:
 // 32 x 32 when larger tiles would leave most compute units idle).  Four waves cover a
 // 64T x 64T tile; MG = groups of four waves stacked along M, all multiplying against the same
@@ -491,38 +550,10 @@ __global__ __launch_bounds__(256 * MG) void q4k_gemm_kernel(const GemmArgs a) {
   // the matrix-core instructions above are inline asm, invisible to the compiler's hazard
   // checks: give the last one time to retire before its accumulators are read
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-  // ---- epilogue: lane holds column n = lane & 31 of rows 8 (e / 4) + 4 fg + (e % 4)
-#pragma unroll
-  for (int i = 0; i < T; i++)
-#pragma unroll
-    for (int j = 0; j < T; j++) {
-      const int n = n0 + wn + 32 * j + fr;
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int rl = wm + 32 * i + 8 * (e >> 2) + 4 * fg + (e & 3);
-        const int m = m0 + rl;
-        if (m < a.M && n < a.N) {
-          float v;
-          const float unscale = rs_lds[rl].y;
-          if (!DUAL && a.ksplit > 1) {
-            a.partial[((int64_t)blockIdx.z * a.M + m) * a.N + n] = acc[0][i][j][e] * unscale;
-            continue;
-          }
-          if (DUAL) {
-            const float g = acc[0][i][j][e] * unscale, u = acc[NMAT - 1][i][j][e] * unscale;
-            v = (a.activation == DH_ACT_SILU ? act_silu(g) : gelu_tanh_fast(g)) * u * a.alpha;
-            if (a.activation == DH_ACT_SILU && a.clamp_max > 0.f) v = fminf(fmaxf(v, -a.clamp_max), a.clamp_max);
-          } else {
-            v = acc[0][i][j][e] * unscale * a.alpha;
-            if (a.residual) v += a.residual[(int64_t)m * a.N + n];
-          }
-          if (a.c_f16)
-            reinterpret_cast<__half*>(a.C)[(int64_t)m * a.N + n] = __float2half(v);
-          else
-            reinterpret_cast<float*>(a.C)[(int64_t)m * a.N + n] = v;
-        }
-      }
-    }
+  store_results<DUAL, T * T>(
+      a, m0, [&](int q, int matrix, int e) { return acc[DUAL ? matrix : 0][q / T][q % T][e]; },
+      [&](int q, int e) { return wm + 32 * (q / T) + 8 * (e >> 2) + 4 * fg + (e & 3); }, [&](int q) { return n0 + wn + 32 * (q % T) + fr; },
+      [&](int row) { return rs_lds[row].y; });
 }
 
 // ---- the wide kernel
@@ -724,43 +755,10 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void q4k_wide_kernel(const GemmA
   }
   dh::arrive_and_wait<0>();                // nothing may be in flight towards LDS when the workgroup ends
 
-  // ---- epilogue: lane holds column l & 31 of rows 8 (e / 4) + 4 (l >> 5) + e % 4
-#pragma unroll
-  for (int i = 0; i < RA; i++)
-#pragma unroll
-    for (int f = 0; f < (DUAL ? 1 : 2); f++) {
-      const int n = n0 + (DUAL ? 32 * wn : 64 * wn + 32 * f) + fr;
-      if (n >= a.N) continue;
-      const int rl0 = 32 * (RA * wm + i) + 4 * fh;
-      float res[16];
-      if (!DUAL && a.residual && a.ksplit == 1) {
-#pragma unroll
-        for (int e = 0; e < 16; e++) res[e] = a.residual[(int64_t)min(m0 + rl0 + 8 * (e >> 2) + (e & 3), a.M - 1) * a.N + n];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 16; e++) res[e] = 0.f;
-      }
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int rl = rl0 + 8 * (e >> 2) + (e & 3), m = m0 + rl;
-        if (m >= a.M) continue;
-        const float unscale = rs_lds[rl];
-        float v;
-        if (DUAL) {
-          const float g = acc[i][0][e] * unscale, u = acc[i][1][e] * unscale;
-          v = (a.activation == DH_ACT_SILU ? act_silu(g) : gelu_tanh_fast(g)) * u * a.alpha;
-          if (a.activation == DH_ACT_SILU && a.clamp_max > 0.f) v = fminf(fmaxf(v, -a.clamp_max), a.clamp_max);
-        } else {
-          if (a.ksplit > 1) {
-            a.partial[((int64_t)blockIdx.z * a.M + m) * a.N + n] = acc[i][f][e] * unscale;
-            continue;
-          }
-          v = acc[i][f][e] * unscale * a.alpha + res[e];
-        }
-        if (a.c_f16) reinterpret_cast<__half*>(a.C)[(int64_t)m * a.N + n] = __float2half(v);
-        else reinterpret_cast<float*>(a.C)[(int64_t)m * a.N + n] = v;
-      }
-    }
+  store_results<DUAL, DUAL ? RA : 2 * RA>(
+      a, m0, [&](int q, int matrix, int e) { return DUAL ? acc[q][matrix][e] : acc[q >> 1][q & 1][e]; },
+      [&](int q, int e) { return 32 * (RA * wm + (DUAL ? q : q >> 1)) + 4 * fh + 8 * (e >> 2) + (e & 3); },
+      [&](int q) { return n0 + (DUAL ? 32 * wn : 64 * wn + 32 * (q & 1)) + fr; }, [&](int row) { return rs_lds[row]; });
 }
 
 // C = alpha * (sum of the split-K pieces, in split order) + residual.  Four consecutive outputs per

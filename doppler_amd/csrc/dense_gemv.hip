@@ -2,9 +2,11 @@
 //
 // The row sits in LDS as f32 (optionally RMS-normalised on its way there); a wave streams one weight row at a time,
 // 16 bytes per lane and load with the non-temporal hint, U loads of the next stage in flight while the current
-// ones are multiplied (f32 fma on the widened weights, so the product is a 32-bit one).  The first stage is requested
-// before the row is prepared and travels meanwhile.  The row is kept as two planes of 16-byte pieces (elements
-// 0..3 and 4..7 of every eight) so that a wave's reads of either plane are consecutive.
+// ones are multiplied (f32 fma on the widened weights, so the product is a 32-bit one).  The row (as far as a few pieces a thread hold it) and its norm's
+// weights are requested first, the first stage of weights behind them: loads arrive in order, so the row is prepared while the weights
+// still travel, and what an output adds and multiplies in comes with its row's weights: short products are a chain of such trips (2048 x 8192
+// with a residual 10.8 -> 9.3 us in a step, gated heads 1024 x 1024 4.9 -> 4.5, 32000 x 1024 14.5 -> 13.6).
+// The row is kept as two planes of 16-byte pieces (elements 0..3 and 4..7 of every eight) so that a wave's reads of either plane are consecutive.
 //
 // Outputs as in the multi-row product (dense_gemm.hip): columns below n_first with bias, column scale and residual, the rest
 // through an activation; or the argmax over all of them (output head).
@@ -59,8 +61,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   const int units = a.iters * nstages;
 
   uint4 cur[U], nxt[U];
+  struct Terms {               // of a row's output
+    float bias, scale, residual;
+  };
+  Terms cur_terms, nxt_terms;
   auto row_of = [&](int it) { return (int64_t)(it * (int)gridDim.x + (int)blockIdx.x) * WAVES + wave; };
-  auto load = [&](int unit, uint4 (&dst)[U]) {
+  auto load = [&](int unit, uint4 (&dst)[U], Terms& terms) {
     const int it = unit / nstages, st = unit - it * nstages;
     const uint4* w = reinterpret_cast<const uint4*>(a.W + min(row_of(it), (int64_t)a.N - 1) * a.ldw);
 #pragma unroll
@@ -68,42 +74,48 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
       const int p = lane + 64 * (u + U * st);
       dst[u] = p < np ? dh::stream_load_16(w + p) : make_uint4(0, 0, 0, 0);
     }
+    if (!ARGMAX && st == 0) {
+      const int64_t n = min(row_of(it), (int64_t)a.n_first - 1);
+      terms = Terms{0.f, 1.f, 0.f};
+      if (n >= 0) {
+        if (a.bias) terms.bias = a.bias[n];
+        if (a.col_scale) terms.scale = a.col_scale[n];
+        if (a.residual) terms.residual = a.residual[n];
+      }
+    }
   };
-  load(0, cur);
 
   // ---- the activation row
+  constexpr int BATCH = HEADS || WAVES < 8 ? 4 : 2;       // 16-byte pieces of a thread requested at once (four workgroups of eight waves: 64 registers)
   if constexpr (HEADS) {
     // weighted and gated on the way in; the squares are summed by eight lanes (whole heads: their sizes are multiples of 32), then by
     // head, and the row in LDS is scaled last: one trip to memory
     __shared__ float inv_s[kMaxHeads];
     __shared__ float squares[kMaxK / 32];
     const int hp = a.head_padded >> 2, live = a.heads * hp;       // 16-byte pieces of a head, of all heads
-    constexpr int BATCH = 4;                              // pieces requested at once
-    for (int i0 = tid; i0 < (a.K >> 2); i0 += THREADS * BATCH) {
-      float4 v[BATCH], w[BATCH], g[BATCH];
+    auto piece_of = [&](const float* row, int i) {
+      const float4 x = reinterpret_cast<const float4*>(row)[min(i, live - 1)];
+      return i < live ? x : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    auto put = [&](int i, float4 y, const float4& w, const float4& g) {
+      float ss = fmaf(y.x, y.x, fmaf(y.y, y.y, fmaf(y.z, y.z, y.w * y.w)));
+      y.x = y.x * w.x * __frcp_rn(1.0f + __expf(-g.x)); y.y = y.y * w.y * __frcp_rn(1.0f + __expf(-g.y));
+      y.z = y.z * w.z * __frcp_rn(1.0f + __expf(-g.z)); y.w = y.w * w.w * __frcp_rn(1.0f + __expf(-g.w));
+      planes[(i & 1) * np + (i >> 1)] = y;
+      ss = dh::group_combine<1, 8>(ss, dh::AddOp());
+      if ((i & 7) == 0) squares[i >> 3] = ss;
+    };
+    float4 v[BATCH], w[BATCH], g[BATCH];
 #pragma unroll
-      for (int b = 0; b < BATCH; b++) {
-        const int i = i0 + THREADS * b;
-        v[b] = w[b] = g[b] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (i < live) {
-          v[b] = reinterpret_cast<const float4*>(a.x)[i];
-          w[b] = reinterpret_cast<const float4*>(a.norm_weight)[i];
-          g[b] = reinterpret_cast<const float4*>(a.gate)[i];
-        }
-      }
-#pragma unroll
-      for (int b = 0; b < BATCH; b++) {
-        const int i = i0 + THREADS * b;
-        if (i >= (a.K >> 2)) break;                       // sixteen lanes at a time: K is a multiple of 64
-        float4 y = v[b];
-        float ss = fmaf(y.x, y.x, fmaf(y.y, y.y, fmaf(y.z, y.z, y.w * y.w)));
-        y.x = y.x * w[b].x * __frcp_rn(1.0f + __expf(-g[b].x)); y.y = y.y * w[b].y * __frcp_rn(1.0f + __expf(-g[b].y));
-        y.z = y.z * w[b].z * __frcp_rn(1.0f + __expf(-g[b].z)); y.w = y.w * w[b].w * __frcp_rn(1.0f + __expf(-g[b].w));
-        planes[(i & 1) * np + (i >> 1)] = y;
-        ss = dh::group_combine<1, 8>(ss, dh::AddOp());
-        if ((i & 7) == 0) squares[i >> 3] = ss;
-      }
+    for (int b = 0; b < BATCH; b++) {
+      const int i = tid + THREADS * b;
+      v[b] = piece_of(a.x, i); w[b] = piece_of(a.norm_weight, i); g[b] = piece_of(a.gate, i);
     }
+    load(0, cur, cur_terms);
+#pragma unroll
+    for (int b = 0; b < BATCH; b++)
+      if (tid + THREADS * b < (a.K >> 2)) put(tid + THREADS * b, v[b], w[b], g[b]);      // sixteen lanes at a time: K is a multiple of 64
+    for (int i = tid + THREADS * BATCH; i < (a.K >> 2); i += THREADS) put(i, piece_of(a.x, i), piece_of(a.norm_weight, i), piece_of(a.gate, i));
     __syncthreads();
     for (int h = tid; h < a.heads; h += THREADS) {
       float ss = 0.f;
@@ -117,14 +129,26 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
       v.x *= f; v.y *= f; v.z *= f; v.w *= f;
     }
   } else {
-    const float4* xg = reinterpret_cast<const float4*>(a.x);
+    const float4 *xg = reinterpret_cast<const float4*>(a.x), *wg = reinterpret_cast<const float4*>(a.norm_weight);
+    const int pieces = a.K >> 2;
+    float4 v[BATCH], w[BATCH];
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) {
+      const int i = min(tid + THREADS * b, pieces - 1);
+      v[b] = xg[i];
+      w[b] = wg ? wg[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+    }
+    load(0, cur, cur_terms);
     float inv = 1.f;
-    if (a.norm_weight) {
+    if (wg) {
       float ss = 0.f;
-      for (int i = tid; i < (a.K >> 2); i += THREADS) {
-        const float4 v = xg[i];
-        ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss); ss = fmaf(v.w, v.w, ss);
-      }
+      auto square = [&](const float4& p) {
+        ss = fmaf(p.x, p.x, ss); ss = fmaf(p.y, p.y, ss); ss = fmaf(p.z, p.z, ss); ss = fmaf(p.w, p.w, ss);
+      };
+#pragma unroll
+      for (int b = 0; b < BATCH; b++)
+        if (tid + THREADS * b < pieces) square(v[b]);
+      for (int i = tid + THREADS * BATCH; i < pieces; i += THREADS) square(xg[i]);
       ss = dh::wave_sum_uniform(ss);
       if (lane == 0) red[wave] = ss;
       __syncthreads();
@@ -133,14 +157,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
       for (int w = 0; w < WAVES; w++) total += red[w];
       inv = 1.0f / sqrtf(total / (float)a.hidden + a.eps);
     }
-    for (int i = tid; i < (a.K >> 2); i += THREADS) {
-      float4 v = xg[i];
-      if (a.norm_weight) {
-        const float4 w = reinterpret_cast<const float4*>(a.norm_weight)[i];
-        v.x = v.x * inv * w.x; v.y = v.y * inv * w.y; v.z = v.z * inv * w.z; v.w = v.w * inv * w.w;
-      }
-      planes[(i & 1) * np + (i >> 1)] = v;
-    }
+    auto put = [&](int i, float4 y, const float4& f) {
+      if (wg) y = make_float4(y.x * inv * f.x, y.y * inv * f.y, y.z * inv * f.z, y.w * inv * f.w);
+      planes[(i & 1) * np + (i >> 1)] = y;
+    };
+#pragma unroll
+    for (int b = 0; b < BATCH; b++)
+      if (tid + THREADS * b < pieces) put(tid + THREADS * b, v[b], w[b]);
+#pragma unroll 2
+    for (int i = tid + THREADS * BATCH; i < pieces; i += THREADS) put(i, xg[i], wg ? wg[i] : make_float4(1.f, 1.f, 1.f, 1.f));
   }
   __syncthreads();
 
@@ -148,7 +173,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   Cand best{-FLT_MAX, 0xFFFFFFFFu};
   int st = 0, it = 0;
   for (int unit = 0; unit < units; unit++) {
-    if (unit + 1 < units) load(unit + 1, nxt);
+    nxt_terms = cur_terms;
+    if (unit + 1 < units) load(unit + 1, nxt, nxt_terms);
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int p = min(lane + 64 * (u + U * st), np - 1);      // past the row the weights are zeros
@@ -165,9 +191,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
       const int64_t n = row_of(it);
       if (lane == 0 && n < a.N) {
         if (n < a.n_first) {
-          float y = v + (a.bias ? a.bias[n] : 0.f);
-          if (a.col_scale) y *= a.col_scale[n];
-          if (a.residual) y += a.residual[n];
+          float y = v;
+          if constexpr (!ARGMAX) {
+            y += cur_terms.bias;
+            if (a.col_scale) y *= cur_terms.scale;
+            if (a.residual) y += cur_terms.residual;
+          }
           if (a.C) a.C[n] = y;
         } else {
           a.C2[n - a.n_first] = dh::activate(v, a.act);
@@ -179,6 +208,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < U; u++) cur[u] = nxt[u];
+    cur_terms = nxt_terms;
   }
   if (ARGMAX) {
     if (lane == 0) { sv[wave] = best.v; si[wave] = best.i; }

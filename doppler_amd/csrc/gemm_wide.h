@@ -33,7 +33,14 @@ __device__ __forceinline__ void fetch_to_lds(const buffer_words_t& words, uint32
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
                : "m0", "memory");
 }
-// The same with 4 bytes per lane, at lds + 4 * lane.
+// The same from an address of its own per lane.
+__device__ __forceinline__ void fetch_global_to_lds(const void* from, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from) : "m0", "memory");
+}
+__device__ __forceinline__ void fetch_words_to_lds(const void* from, uint32_t lds) {      // 4 bytes per lane, to lds + 4 * lane
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(from) : "m0", "memory");
+}
+// 4 bytes per lane as in the first, to lds + 4 * lane.
 __device__ __forceinline__ void touch_to_lds(const buffer_words_t& words, uint32_t v_off, uint32_t s_off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(words), "s"(s_off)
                : "m0", "memory");

@@ -14,10 +14,7 @@
 // masked product inside it:
 //
 //   mlstm_gates_kernel     F, i, m of every token; one workgroup per head
-//   mlstm_chunks_kernel    what every chunk adds to the state behind it, sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T: independent of
-//                          one another, because m is known
-//   mlstm_scan_kernel      the state in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + what chunk c adds,
-//                          element by element and in place
+//   mlstm_states_kernel    the state in front of every chunk, walking the chunks with a tile of it in registers
 //   mlstm_outputs_kernel   o of (chunk, head, value columns): Q K^T and Q S in one walk over dim, decay mask, then (Q K^T) V
 //
 // on the 32-bit matrix-core instruction v_mfma_f32_32x32x2_f32.  head_norm_gate_kernel then divides every head's output by its root
@@ -25,7 +22,7 @@
 #include <algorithm>
 #include <cfloat>
 
-#include "dense_device.h"
+#include "gemm_wide.h"
 
 namespace {
 
@@ -53,6 +50,7 @@ struct MemArgs {
   float* mt;               // m after every token
   float* mc;               // [H][chunks + 1] m in front of every chunk, and at the end
   float* keep;             // [H][chunks] what a chunk leaves of the state in front of it
+  float* w;                // [H][chunks][64] weight of a token's key and value in the state behind its chunk, zero past the last
   float* Sc;               // [chunks + 1][H][DP][VP]
   float* nc;               // [chunks + 1][H][DP]
 };
@@ -197,94 +195,214 @@ __global__ __launch_bounds__(1024) void mlstm_gates_kernel(const MemArgs a) {
     const double start = c > 0 ? F[c * kChunk - 1] : 0.0, end = F[min((c + 1) * kChunk, a.T) - 1];
     a.keep[(int64_t)h * a.chunks + c] = expf((float)(end - start + (double)mc[c] - (double)mc[c + 1]));
   }
-}
-
-// Grid = (64 x 64 tiles of a head's state, heads, chunks); wave w: rows 32 (w >> 1), columns 32 (w & 1) of the tile.
-__global__ __launch_bounds__(256) void mlstm_chunks_kernel(const MemArgs a) {
-  constexpr int ROW = 64 + 4;
-  __shared__ __align__(16) float ks[kChunk * ROW];     // weighted keys [token][dim]
-  __shared__ __align__(16) float vs[kChunk * ROW];     // values [token][column]
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y, c = blockIdx.z;
-  const int tiles_v = (a.VP + 63) / 64, d0 = 64 * (blockIdx.x / tiles_v), v0 = 64 * (blockIdx.x % tiles_v);
-  const double* F = a.F + (int64_t)h * a.T;
-  const int first = c * kChunk, count = min(kChunk, a.T - first);
-  const double F_end = F[first + count - 1];
-  const float m_end = a.mc[(int64_t)h * (a.chunks + 1) + c + 1];
-  f32x4_t kr[4], vr[4];
-  float w[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int p = tid + 256 * r, tok = first + min(p >> 4, count - 1), x = 4 * (p & 15);
-    const float* row = a.rows + (int64_t)tok * a.ld_row;
-    kr[r] = vr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (d0 + x < a.DP) kr[r] = *reinterpret_cast<const f32x4_t*>(row + a.k_off + (int64_t)h * a.DP + d0 + x);
-    if (v0 + x < a.VP) vr[r] = *reinterpret_cast<const f32x4_t*>(row + a.v_off + (int64_t)h * a.VP + v0 + x);
-    w[r] = (p >> 4) < count ? expf((float)(F_end - F[tok] + (double)a.i[(int64_t)h * a.T + tok] - (double)m_end)) : 0.f;
-  }
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int p = tid + 256 * r, tok = p >> 4, x = 4 * (p & 15);
-    // (rows past the last repeat it: an infinite one times a weight of zero is no number)
-    if ((p >> 4) < count) kr[r] *= w[r];
-    else kr[r] = vr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<f32x4_t*>(&ks[tok * ROW + x]) = kr[r];
-    *reinterpret_cast<f32x4_t*>(&vs[tok * ROW + x]) = vr[r];
-  }
-  __syncthreads();
-  const int wd = 32 * (wave >> 1), wv = 32 * (wave & 1);
-  if (d0 + wd < a.DP && v0 + wv < a.VP) {              // wave-uniform (sizes are multiples of 32)
-    f32x16_t acc;
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = 0.f;
-#pragma unroll 8
-    for (int j = 0; j < kChunk / 2; j++) {
-      const int tok = 2 * j + (lane >> 5);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[tok * ROW + wd + (lane & 31)], vs[tok * ROW + wv + (lane & 31)], acc, 0, 0, 0);
-    }
-    // accumulator element e of a lane: state row 8 (e / 4) + 4 (lane >> 5) + e % 4, column lane & 31
-    float* U = a.Sc + ((int64_t)(c + 1) * a.H + h) * a.DP * a.VP + (int64_t)(d0 + wd + 4 * (lane >> 5)) * a.VP + v0 + wv + (lane & 31);
-#pragma unroll
-    for (int e = 0; e < 16; e++) U[(int64_t)(8 * (e >> 2) + (e & 3)) * a.VP] = acc[e];
-  }
-  if (v0 == 0 && tid < 64 && d0 + tid < a.DP) {
-    float s = 0.f;
-#pragma unroll 8
-    for (int t = 0; t < kChunk; t++) s += ks[t * ROW + tid];
-    a.nc[((int64_t)(c + 1) * a.H + h) * a.DP + d0 + tid] = s;
+  for (int t = tid; t < a.chunks * kChunk; t += 1024) {
+    const int c = t / kChunk, last = min((c + 1) * kChunk, a.T) - 1;
+    // in fours of tokens, a token of every four beside those of the others
+    a.w[((int64_t)h * a.chunks + c) * kChunk + 16 * (t & 3) + ((t & (kChunk - 1)) >> 2)] = t <= last ? expf((float)(F[last] - F[t] + (double)li[t] - (double)mc[c + 1])) : 0.f;
   }
 }
 
-// Grid = (groups of 1024 elements of a head's [S | n], heads), four per thread; slot 0 of Sc and nc is filled here.
-__global__ __launch_bounds__(256) void mlstm_scan_kernel(const MemArgs a) {
-  constexpr int AHEAD = 16;
-  const int h = blockIdx.y, size = a.DP * a.VP;
-  const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
-  if (i >= size + a.DP) return;
-  const bool is_n = i >= size;
-  const int64_t stride = is_n ? (int64_t)a.H * a.DP : (int64_t)a.H * size;
-  float* at = is_n ? a.nc + (int64_t)h * a.DP + (i - size) : a.Sc + (int64_t)h * size + i;
-  const int64_t slots = (int64_t)a.H * a.DP;
-  const float* from = is_n ? a.n + (a.pos & 1) * slots + (int64_t)h * a.DP + (i - size) : a.S + (int64_t)h * size + i;
-  float* to = is_n ? a.n + ((a.pos + a.T) & 1) * slots + (int64_t)h * a.DP + (i - size) : a.S + (int64_t)h * size + i;
-  const float* keep = a.keep + (int64_t)h * a.chunks;
-  f32x4_t s = {0.f, 0.f, 0.f, 0.f};
-  if (a.pos > 0) s = *reinterpret_cast<const f32x4_t*>(from);
-  *reinterpret_cast<f32x4_t*>(at) = s;
-  for (int c0 = 0; c0 < a.chunks; c0 += AHEAD) {
-    f32x4_t u[AHEAD];
+// The states in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T, in one walk.
+//
+// One workgroup of eight waves for 64 x 32 of a head's state, a head's tiles on one die.  Wave w holds rows 16 (w >> 1), columns 16 (w & 1) in
+// registers, adds up a chunk's products apart from it (16 of v_mfma_f32_16x16x4_f32: with 32 x 32 tiles half of the SIMDs would have none) and
+// writes the state in front of every chunk once.  Keys, values and weights go straight into three buffers of LDS, two chunks ahead, by waits that count:
+// through registers the compiler waited for the youngest load and store at every chunk (2.3 us each).  Four tokens make an instruction, so their
+// rows' 16-byte pieces are kept apart by 16 banks (slot = piece ^ 4 (token & 3) of 16, piece ^ 4 (token / 2 & 1) of 8).
+// The workgroups behind the tiles walk the normaliser.
+// us, against a launch for what every chunk adds (to memory and back) and another for the scan: four heads of 256 x 512, 1531 tokens 38 + 18.6 -> 35.5, eight, 900
+// tokens 46.6 + 21.6 -> 41, four of 128 x 256, 2000 tokens 17.7 + 11.3 -> 28.3, 40 tokens 6.9 + 2.7 -> 4.8.  Of 35.5 the matrix cores take 15.
+template <int ROWS>
+struct StateTile {           // ROWS x 32 of a state; a wave 16 x 16 of it
+  static constexpr int kWaves = ROWS / 8, kThreads = 64 * kWaves;
+  static constexpr int kKeys = kChunk * ROWS * 4, kValues = kChunk * 32 * 4, kBuffer = kKeys + kValues, kBuffers = 3;
+  static constexpr int kPieces = ROWS / 4, kKeyTokens = 64 / kPieces, kKeyFetches = kChunk / (kKeyTokens * kWaves);      // of a fetch, of a wave
+  static constexpr int kValueFetches = kChunk / (8 * kWaves), kFetches = kKeyFetches + kValueFetches + 1;
+  static constexpr int kWeights = kBuffers * kBuffer, kBytes = kWeights + 4 * kChunk * 4;      // four chunks' weights
+  // 16-byte piece p of a token's keys (values) lies at slot p ^ key_swap (value_swap)
+  static __device__ __forceinline__ int key_swap(int token) { return ROWS == 64 ? 4 * (token & 3) : 4 * ((token >> 1) & 1); }
+  static __device__ __forceinline__ int value_swap(int token) { return 4 * ((token >> 1) & 1); }
+};
+// 64 elements of a head's normaliser: a wave sums a chunk's weighted keys, the first wave then takes the waves' chunks in turn.
+template <int WAVES>
+__device__ __forceinline__ void walk_normaliser(const MemArgs& a, int part, float* sums) {      // [WAVES][64]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int parts = (a.DP + 63) / 64, h = part / parts, d = 64 * (part % parts) + lane;
+  const int64_t slots = (int64_t)a.H * a.DP, at = (int64_t)h * a.DP + min(d, a.DP - 1);
+  const float* rows = a.rows + a.k_off + (int64_t)h * a.DP + 64 * (part % parts);
+  const uint32_t column = (uint32_t)min(lane, a.DP - 1 - 64 * (part % parts));
+  const float* w = a.w + (int64_t)h * a.chunks * kChunk;
+  const bool live = d < a.DP;
+  float n = a.pos > 0 ? a.n[(a.pos & 1) * slots + at] : 0.f;
+  if (wave == 0 && live) a.nc[at] = n;
+  for (int c0 = 0; c0 < a.chunks; c0 += WAVES) {
+    const int c = min(c0 + wave, a.chunks - 1), first = c * kChunk, count = min(kChunk, a.T - first);
+    const float weight = w[first + lane];              // that of token 4 (lane % 16) + lane / 16
+    float u = 0.f;
 #pragma unroll
-    for (int k = 0; k < AHEAD; k++)
-      if (c0 + k < a.chunks) u[k] = *reinterpret_cast<const f32x4_t*>(at + (c0 + k + 1) * stride);
+    for (int half = 0; half < kChunk; half += kChunk / 2) {
+      float k[kChunk / 2];
 #pragma unroll
-    for (int k = 0; k < AHEAD; k++) {
-      const int c = c0 + k;
-      if (c < a.chunks) {
-        s = s * keep[c] + u[k];
-        if (c + 1 < a.chunks) *reinterpret_cast<f32x4_t*>(at + (c + 1) * stride) = s;
+      for (int i = 0; i < kChunk / 2; i++) k[i] = (rows + (int64_t)(first + min(half + i, count - 1)) * a.ld_row)[column];
+#pragma unroll
+      for (int i = 0; i < kChunk / 2; i++) {
+        const int t = half + i;
+        u = fmaf(t < count ? k[i] : 0.f, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), 16 * (t & 3) + (t >> 2))), u);
       }
     }
+    sums[64 * wave + lane] = u;
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int i = 0; i < WAVES; i++) {
+        if (c0 + i >= a.chunks) break;
+        n = n * a.keep[(int64_t)h * a.chunks + c0 + i] + sums[64 * i + lane];
+        if (live) a.nc[(c0 + i + 1) * slots + at] = n;
+      }
+    }
+    __syncthreads();
   }
-  *reinterpret_cast<f32x4_t*>(to) = s;
+  if (wave == 0 && live) a.n[((a.pos + a.T) & 1) * slots + at] = n;
+}
+
+template <int ROWS>
+__global__ __launch_bounds__(StateTile<ROWS>::kThreads, ROWS == 64 ? 4 : 2) void mlstm_states_kernel(const MemArgs a) {
+  using Tile = StateTile<ROWS>;
+  extern __shared__ __align__(16) char lds[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int tiles_v = a.VP / 32, per_head = (a.DP + ROWS - 1) / ROWS * tiles_v, tiles = per_head * a.H;
+  if ((int)blockIdx.x >= tiles) {
+    walk_normaliser<Tile::kWaves>(a, (int)blockIdx.x - tiles, reinterpret_cast<float*>(lds));
+    return;
+  }
+  const int tile = dh::xcd_contiguous(blockIdx.x, tiles);
+  const int h = tile / per_head, d0 = ROWS * (tile % per_head / tiles_v), v0 = 32 * (tile % per_head % tiles_v);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const float* keep = a.keep + (int64_t)h * a.chunks;
+
+  // state rows of waves past the last: those 32 up, computed twice
+  const int wd = d0 + 16 * (wave >> 1) < a.DP ? 16 * (wave >> 1) : 16 * (wave >> 1) - 32, wv = 16 * (wave & 1);
+  const int64_t size = (int64_t)a.DP * a.VP;
+  // accumulator element e of a lane: state row 4 (lane / 16) + e, column lane % 16
+  const int64_t at = (int64_t)h * size + (int64_t)(d0 + wd + 4 * (lane >> 4)) * a.VP + v0 + wv + (lane & 15);
+  f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+  if (a.pos > 0) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) s[e] = a.S[at + (int64_t)e * a.VP];
+  }
+  float* front = a.Sc + at;                            // in front of the next chunk
+  auto store = [&](float* to) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) to[(int64_t)e * a.VP] = s[e];
+  };
+  store(front);
+  float kept = keep[min(lane, a.chunks - 1)];          // of 64 chunks
+  asm volatile("" : "+v"(kept));                       // the compiler's own loads are over before fetches are counted
+
+  // a wave's fetches of a chunk: its tokens' keys and values, and the weights (every wave the same); past the last chunk that again, unread
+  const float* rows = a.rows + (int64_t)h * a.DP;
+  auto key_token = [&](int r) { return Tile::kKeyTokens * (Tile::kKeyFetches * wave + r) + lane / Tile::kPieces; };
+  auto value_token = [&](int r) { return 8 * (Tile::kValueFetches * wave + r) + (lane >> 3); };
+  auto key_at = [&](int t) { return a.k_off + min(d0 + 4 * ((lane % Tile::kPieces) ^ Tile::key_swap(t)), a.DP - 4); };
+  auto value_at = [&](int t) { return a.v_off + h * (a.VP - a.DP) + v0 + 4 * ((lane & 7) ^ Tile::value_swap(t)); };
+  const float *key_from[Tile::kKeyFetches], *value_from[Tile::kValueFetches];
+#pragma unroll
+  for (int r = 0; r < Tile::kKeyFetches; r++) key_from[r] = rows + (int64_t)key_token(r) * a.ld_row + key_at(key_token(r));
+#pragma unroll
+  for (int r = 0; r < Tile::kValueFetches; r++) value_from[r] = rows + (int64_t)value_token(r) * a.ld_row + value_at(value_token(r));
+  const float* weights_from = a.w + (int64_t)h * a.chunks * kChunk + lane;
+  const int64_t chunk_step = (int64_t)kChunk * a.ld_row;
+  int next = 0;                                        // the chunk to be fetched next
+  uint32_t next_buf = lds0;
+  auto fetch = [&](int i) {                            // the i-th of kFetches
+    const bool tail = (next + 1) * kChunk >= a.T;      // the last chunk, or past it
+    const int first = (a.chunks - 1) * kChunk, last = a.T - 1;
+    if (i < Tile::kKeyFetches) {
+      const int t = key_token(i);
+      const float* from = key_from[i];
+      if (tail) from = rows + (int64_t)min(first + t, last) * a.ld_row + key_at(t);
+      dh::fetch_global_to_lds(from, next_buf + 1024 * (Tile::kKeyFetches * wave + i));
+      key_from[i] += chunk_step;
+    } else if (i < Tile::kKeyFetches + Tile::kValueFetches) {
+      const int r = i - Tile::kKeyFetches, t = value_token(r);
+      const float* from = value_from[r];
+      if (tail) from = rows + (int64_t)min(first + t, last) * a.ld_row + value_at(t);
+      dh::fetch_global_to_lds(from, next_buf + Tile::kKeys + 1024 * (Tile::kValueFetches * wave + r));
+      value_from[r] += chunk_step;
+    } else {
+      dh::fetch_words_to_lds(weights_from, lds0 + Tile::kWeights + 4 * kChunk * (next & 3));
+      if (!tail) weights_from += kChunk;
+      next++;
+      next_buf = next_buf == lds0 + (Tile::kBuffers - 1) * Tile::kBuffer ? lds0 : next_buf + Tile::kBuffer;
+    }
+  };
+#pragma unroll
+  for (int n = 0; n < 3; n++)
+#pragma unroll
+    for (int i = 0; i < Tile::kFetches; i++) fetch(i);
+  // a lane's operands: token 4 j + tq, row wd + lane % 16 and column wv + lane % 16
+  const int tq = lane >> 4, kd = wd + (lane & 15), vc = wv + (lane & 15);
+  const uint32_t k_at = 4 * ROWS * tq + 16 * ((kd >> 2) ^ Tile::key_swap(tq)) + 4 * (kd & 3);
+  const uint32_t v_at = Tile::kKeys + 128 * tq + 16 * ((vc >> 2) ^ Tile::value_swap(tq)) + 4 * (vc & 3);
+  struct Operands {
+    float k[kChunk / 4], v[kChunk / 4];
+  };
+  const char* buf = lds;
+  auto read = [&](Operands& o, int j) {
+    o.k[j] = *reinterpret_cast<const float*>(buf + k_at + 16 * ROWS * j);
+    o.v[j] = *reinterpret_cast<const float*>(buf + v_at + 512 * j);
+  };
+  auto next_buffer = [&] { buf = buf == lds + (Tile::kBuffers - 1) * Tile::kBuffer ? lds : buf + Tile::kBuffer; };
+  // a chunk is multiplied while the next one's operands are read and the third after it is fetched into the buffer it came from
+  auto step = [&](int c, Operands& now, Operands& next) {
+    // chunk c + 1 is there: younger than its fetches are those of c + 2 and the stores of the two chunks before this
+    if (c >= 2) dh::arrive_and_wait<Tile::kFetches + 8>();
+    else if (c == 1) dh::arrive_and_wait<Tile::kFetches + 4>();
+    else dh::arrive_and_wait<Tile::kFetches>();
+    const int count = a.T - c * kChunk;
+#pragma unroll
+    for (int j = 0; j < kChunk / 16; j++) {            // a quarter's weights lie side by side (mlstm_gates_kernel)
+      const f32x4_t w = *reinterpret_cast<const f32x4_t*>(lds + Tile::kWeights + 4 * kChunk * (c & 3) + 64 * tq + 16 * j);
+#pragma unroll
+      for (int e = 0; e < 4; e++) now.k[4 * j + e] *= w[e];
+    }
+    if (count < kChunk) {                              // (rows past the last repeat it: an infinite one times a weight of zero is no number)
+#pragma unroll
+      for (int j = 0; j < kChunk / 4; j++)
+        if (4 * j + tq >= count) now.k[j] = now.v[j] = 0.f;
+    }
+    f32x4_t u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < kChunk / 4; j++) {
+      u = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j], now.v[j], u, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      read(next, j);
+      if (j % 2 && j / 2 < Tile::kFetches) fetch(j / 2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    static_assert(Tile::kFetches <= kChunk / 8, "all of them in between");
+    if ((c & 63) == 0 && c > 0) {
+      kept = keep[min(c + lane, a.chunks - 1)];
+      asm volatile("" : "+v"(kept));                   // waited for here, not at every chunk
+    }
+    const float left = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kept), c & 63));
+    s = s * left + u;
+    front += a.H * size;
+    store(front);
+    next_buffer();
+  };
+  Operands even, odd;
+  dh::arrive_and_wait<2 * Tile::kFetches>();
+#pragma unroll
+  for (int j = 0; j < kChunk / 4; j++) read(even, j);
+  next_buffer();
+  for (int c = 0; c < a.chunks; c += 2) {
+    step(c, even, odd);
+    if (c + 1 >= a.chunks) break;
+    step(c + 1, odd, even);
+  }
+  dh::arrive_and_wait<0>();                            // nothing may be in flight towards LDS when the workgroup ends
+  store(a.S + at);
 }
 
 // Grid = (chunks, heads, groups of 64 TN value columns); wave w: tokens 32 (w >> 1), columns 32 TN (w & 1) + 0 .. 32 TN - 1.
@@ -494,6 +612,17 @@ MemArgs make_args(const dh_mlstm* s, const float* rows, float* state, float* out
 }
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+template <int ROWS>
+int launch_states(const char* op, const MemArgs& a) {
+  using Tile = StateTile<ROWS>;
+  auto kern = mlstm_states_kernel<ROWS>;
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kBytes);
+  DH_CHECK_HIP(op, set);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((dh::ceil_div(a.DP, ROWS) * (a.VP / 32) + dh::ceil_div(a.DP, 64)) * a.H)), dim3(Tile::kThreads), Tile::kBytes, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -520,7 +649,7 @@ int dh_mlstm_step(const dh_mlstm* spec, const float* d_row, void* d_state, float
 size_t dh_mlstm_prefill_workspace_bytes(const dh_mlstm* s, int T) {
   if (!s || T <= 0) return 256;
   const size_t chunks = (size_t)dh::ceil_div(T, kChunk), HT = (size_t)s->H * T;
-  return up256(HT * 8) + 2 * up256(HT * 4) + 2 * up256((size_t)s->H * (chunks + 1) * 4) + up256((chunks + 1) * s->H * s->DP * 4) +
+  return up256(HT * 8) + 2 * up256(HT * 4) + 2 * up256((size_t)s->H * (chunks + 1) * 4) + up256((size_t)s->H * chunks * kChunk * 4) + up256((chunks + 1) * s->H * s->DP * 4) +
          up256((chunks + 1) * s->H * s->DP * s->VP * 4);
 }
 
@@ -543,17 +672,16 @@ int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, v
   a.mt = reinterpret_cast<float*>(take(HT * 4));
   a.mc = reinterpret_cast<float*>(take((size_t)spec->H * (a.chunks + 1) * 4));
   a.keep = reinterpret_cast<float*>(take((size_t)spec->H * (a.chunks + 1) * 4));
+  a.w = reinterpret_cast<float*>(take((size_t)spec->H * a.chunks * kChunk * 4));
   a.nc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * 4));
   a.Sc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * spec->VP * 4));
+  // (more chunks than a grid's smaller dimensions hold have always been refused)
+  if (a.chunks > 65535) return dh::fail(1, "[%s] %d tokens are too many for one portion", op, T);
   hipLaunchKernelGGL(mlstm_gates_kernel, dim3(spec->H), dim3(1024), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
-  const int tiles = (int)(dh::ceil_div(spec->DP, 64) * dh::ceil_div(spec->VP, 64));
-  // the grid's third dimension holds at most 65535 chunks
-  if (a.chunks > 65535) return dh::fail(1, "[%s] %d tokens are too many for one portion", op, T);
-  hipLaunchKernelGGL(mlstm_chunks_kernel, dim3(tiles, spec->H, a.chunks), dim3(256), 0, dh::stream(), a);
-  DH_CHECK_LAUNCH(op);
-  hipLaunchKernelGGL(mlstm_scan_kernel, dim3((unsigned)dh::ceil_div((int64_t)spec->DP * spec->VP + spec->DP, 1024), spec->H), dim3(256), 0, dh::stream(), a);
-  DH_CHECK_LAUNCH(op);
+  // tiles of 64 rows, or of 32 where those would not fill the device (us, 64 / 32: 128 x 256 34 / 28.4, 256 x 512 36 / 41)
+  const int64_t tall = dh::ceil_div(spec->DP, 64) * (spec->VP / 32) * spec->H;
+  if (int rc = tall >= dh::num_cus() ? launch_states<64>(op, a) : launch_states<32>(op, a)) return rc;
   // wide column groups repeat Q K^T less often; narrow ones where those would not fill the device
   const bool wide = spec->VP > 64 && (int64_t)a.chunks * spec->H * dh::ceil_div(spec->VP, 128) >= dh::num_cus();
   if (wide) hipLaunchKernelGGL(mlstm_outputs_kernel<2>, dim3(a.chunks, spec->H, (unsigned)dh::ceil_div(spec->VP, 128)), dim3(256), 0, dh::stream(), a);

@@ -207,6 +207,12 @@ def test_memory_state_behind_a_prompt(L, H, D, V, T, start):
             assert np.abs(a[fin] - b[fin]).max() <= 64 * 2.0 ** -24 * max(1.0, np.abs(b[fin]).max()) * 4, (name, bad)
 
 
+@pytest.mark.parametrize("H,D,V,T,start", [(8, 96, 512, 130, 3), (16, 64, 512, 63, 0), (1, 32, 64, 64 * 65 + 1, 0)])
+def test_memory_state_walks(L, H, D, V, T, start):
+    """The same on tiles of 64 rows, the last of them half full, and over more chunks than one read of what they keep holds (64)."""
+    test_memory_state_behind_a_prompt(L, H, D, V, T, start)
+
+
 @pytest.mark.parametrize("live,before", [(1, 0), (2, 0), (4, 0), (1, 64)])
 def test_memory_state_of_few_live_tokens(L, live, before):
     """A chunk that few tokens count in (a portion of one, two or four tokens, and one whose last token closes the forget gate over 64 others)

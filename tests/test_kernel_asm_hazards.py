@@ -35,7 +35,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "doppler_amd", "csrc")
 SOURCES = ["q4k_gemv_rows.hip", "q4k_gemv_i8.hip", "q4k_gemv_chain.hip"]
 # kernels whose hand-written fetches go straight into LDS (m0 names the place): no destination registers, waits counted by hand
-FETCHING = ["attention_prefill.hip", "dense_gemm.hip", "q4k_gemm.hip"]
+FETCHING = ["attention_prefill.hip", "dense_gemm.hip", "matrix_memory.hip", "q4k_gemm.hip"]
 VMEM_PREFIXES = ("global_", "buffer_", "flat_", "scratch_")
 SREG = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]")
 VREG = re.compile(r"\bv(\d+)\b|\bv\[(\d+):(\d+)\]")
@@ -214,7 +214,7 @@ def test_no_scratch_memory_in_the_streaming_kernels(assembly, src):
 
 
 def _is_fetch(s, in_asm):
-    return in_asm and s.startswith("buffer_load") and s.split()[-1] == "lds"
+    return in_asm and (s.startswith("buffer_load") and s.split()[-1] == "lds" or s.startswith("global_load_lds"))
 
 
 def foreign_m0(path):

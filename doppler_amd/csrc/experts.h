@@ -24,6 +24,21 @@ __device__ __forceinline__ float clamped_glu(float g, float u, float limit) {
   return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
 
+// A bf16 product of experts, all of it: gate and up (out: bf16 activations) or down (out: f32, times col_scale, plus residual).
+struct ExpertProduct {
+  ExpertRows rows;
+  const void* A;
+  int64_t lda;
+  const uint16_t* W;
+  int64_t ldw;
+  int M, N, K;
+  void* out;
+  int64_t ld_out;
+  const float *col_scale, *residual;
+};
+// Whether the routed experts' product (rows.tiles) and the shared expert's go in one launch, and that launch.
+bool experts_together(const ExpertProduct& routed, const ExpertProduct& shared, bool glu);
+int experts_pair(const char* op, const ExpertProduct& routed, const ExpertProduct& shared, bool glu);
 // Row tiles of the grouped products for this many rows in all.
 int expert_tile_rows(int a_dtype, int rows, int groups);
 // act[row] = clamped_glu of a row's gate and up products with interleaved [N = 2 ff][K] weights (32 gate, 32 up rows, ..).

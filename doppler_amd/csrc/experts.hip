@@ -493,23 +493,43 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   dh::ExpertRows rows{};
   rows.tiles = i32(p.tiles); rows.group_off = i32(p.off); rows.row_index = i32(p.row_token); rows.source_rows = T; rows.w_stride = (int64_t)2 * spec->ff * spec->K;
   rows.max_tiles = p.max_tiles; rows.tile_rows = p.tile_rows; rows.row_in = f32(p.row_weight); rows.limit = spec->limit;
-  if (int rc = dh::experts_glu(op, rows, d_h, operand, spec->K, static_cast<const uint16_t*>(spec->d_up), spec->K, n, 2 * spec->ff, spec->K, w + p.act,
-                               operand, spec->ff))
-    return rc;
+  dh::ExpertRows one{};
+  one.row_out = f32(p.sg); one.limit = spec->shared_limit;
+  const uint16_t *up = static_cast<const uint16_t*>(spec->d_up), *down = static_cast<const uint16_t*>(spec->d_down);
+  const uint16_t *shared_up = static_cast<const uint16_t*>(spec->d_shared_up), *shared_down = static_cast<const uint16_t*>(spec->d_shared_down);
+  const bool shared = spec->shared_ff > 0, pairs = shared && operand == DH_BF16;
+  // gate and up products; the shared expert's beside the routed ones' or behind them
+  const dh::ExpertProduct routed_up{rows, d_h, spec->K, up, spec->K, n, 2 * spec->ff, spec->K, w + p.act, spec->ff, nullptr, nullptr};
+  const dh::ExpertProduct own_up{one, d_h, spec->K, shared_up, spec->K, T, 2 * spec->shared_ff, spec->K, w + p.shared_act, spec->shared_ff, nullptr, nullptr};
+  const bool up_pair = pairs && dh::experts_together(routed_up, own_up, true);
+  if (up_pair) {
+    if (int rc = dh::experts_pair(op, routed_up, own_up, true)) return rc;
+  } else {
+    if (int rc = dh::experts_glu(op, rows, d_h, operand, spec->K, up, spec->K, n, 2 * spec->ff, spec->K, w + p.act, operand, spec->ff)) return rc;
+  }
   rows.row_index = nullptr; rows.row_in = nullptr; rows.w_stride = (int64_t)spec->hidden * spec->ff;
-  if (int rc = dh::experts_down(op, rows, w + p.act, operand, spec->ff, static_cast<const uint16_t*>(spec->d_down), spec->ff, spec->hidden, spec->ff,
-                                f32(p.y), p.ld_y))
-    return rc;
+  auto shared_gate_up = [&] {
+    return dh::experts_glu(op, one, d_h, operand, spec->K, shared_up, spec->K, T, 2 * spec->shared_ff, spec->K, w + p.shared_act, operand, spec->shared_ff);
+  };
+  // down products: together, the shared expert's reaches x in front of the routed ones' sum
+  const dh::ExpertProduct routed_down{rows, w + p.act, spec->ff, down, spec->ff, n, spec->hidden, spec->ff, f32(p.y), p.ld_y, nullptr, nullptr};
+  const dh::ExpertProduct own_down{dh::ExpertRows{}, w + p.shared_act, spec->shared_ff, shared_down, spec->shared_ff, T, spec->hidden, spec->shared_ff,
+                                   d_x, ld_x, spec->d_layer_scale, d_x};
+  const bool down_pair = pairs && dh::experts_together(routed_down, own_down, false);
+  if (down_pair) {
+    if (!up_pair)
+      if (int rc = shared_gate_up()) return rc;
+    if (int rc = dh::experts_pair(op, routed_down, own_down, false)) return rc;
+  } else {
+    if (int rc = dh::experts_down(op, rows, w + p.act, operand, spec->ff, down, spec->ff, spec->hidden, spec->ff, f32(p.y), p.ld_y)) return rc;
+  }
   hipLaunchKernelGGL(experts_combine_kernel, dim3(T, (unsigned)dh::ceil_div(spec->hidden, 1024)), dim3(256), 0, dh::stream(), f32(p.y), (int64_t)p.ld_y,
                      i32(p.slot), spec->top, spec->d_layer_scale, d_x, (int64_t)ld_x, spec->hidden);
   DH_CHECK_LAUNCH(op);
-  if (spec->shared_ff) {
-    dh::ExpertRows one{};
-    one.row_out = f32(p.sg); one.limit = spec->shared_limit;
-    if (int rc = dh::experts_glu(op, one, d_h, operand, spec->K, static_cast<const uint16_t*>(spec->d_shared_up), spec->K, T, 2 * spec->shared_ff, spec->K,
-                                 w + p.shared_act, operand, spec->shared_ff))
-      return rc;
-    return dh_dense_matmul_scaled(w + p.shared_act, operand, spec->shared_ff, spec->d_shared_down, spec->shared_ff, T, spec->hidden, spec->shared_ff, 1.f,
+  if (shared && !down_pair) {
+    if (!up_pair)
+      if (int rc = shared_gate_up()) return rc;
+    return dh_dense_matmul_scaled(w + p.shared_act, operand, spec->shared_ff, shared_down, spec->shared_ff, T, spec->hidden, spec->shared_ff, 1.f,
                                   nullptr, spec->d_layer_scale, d_x, d_x, ld_x, spec->hidden, nullptr, 0, 0, DH_ACT_NONE);
   }
   return 0;

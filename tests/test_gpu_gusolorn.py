@@ -482,6 +482,48 @@ def test_expert_rows_past_4_gb(L, T, W, K, E, top, ff):
         assert ((whole[at:at + size] - alone).norm(dim=1) <= 2.0 ** -8 * alone.norm(dim=1)).all(), at
 
 
+# shared and routed products of one size share a launch: 128-row tiles (ragged ones, an expert that nobody uses), 64-row tiles, and rows past the first
+# eight workgroups' edge; the last keeps them apart (the shared expert is eight times as wide)
+@pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(1531, 1024, 4, 2, 512, 1024), (1000, 1024, 5, 2, 512, 1024), (40, 256, 8, 2, 64, 128), (7, 64, 3, 1, 64, 64),
+                                                    (300, 256, 4, 1, 64, 512)])
+def test_shared_and_routed_products(L, T, K, E, top, ff, shared_ff):
+    """Rows behind both kinds of experts against 64 bits.  Activations are rounded to bf16 in front of the down products, and a routed product behind
+    them: 2^-9 of every term each, 2^-8 of the terms' sizes together; over a row of random signs the norms keep 2^-8 as well."""
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    h, x0, ls, norm = torch.randn(T, K, generator=g, device="cuda").to(torch.bfloat16), *(torch.randn(n, generator=g, device="cuda") for n in (T * K, K)), torch.ones(K, device="cuda")
+    router, up, down, s_up, s_down = w(E + 1, K), w(E, 2 * ff, K), w(E, K, ff), w(2 * shared_ff, K), w(K, shared_ff)
+    if E == 5:
+        router[2] = 0.0
+        router[2, 0], h[:, 0] = -8.0, 4.0
+    spec = capi.Experts(K, K, E, top, ff, shared_ff, 1e-5, 7.0, 1.5, norm.data_ptr(), ls.data_ptr(), *(a.data_ptr() for a in (router, up, down, s_up, s_down)))
+    ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T), dtype=torch.uint8, device="cuda")
+    x = x0.clone().view(T, K)
+    torch.cuda.synchronize()
+    capi.check(L.dh_experts_prefill(ctypes.byref(spec), h.data_ptr(), capi.BF16, x.data_ptr(), K, ws.data_ptr(), T))
+    capi.check(L.dh_sync())
+
+    def glu(z, limit, scale):
+        z = (z * scale).view(len(z), z.shape[1] // 64, 2, 32)
+        gate, lin = (z[:, :, i].reshape(len(z), z.shape[1] * z.shape[3]) for i in (0, 1))
+        gate = gate.clamp(max=limit)
+        return gate * torch.sigmoid(1.702 * gate) * (lin.clamp(-limit, limit) + 1)
+    hd = h.double()
+    z = hd @ router.double().T
+    best, ids = z[:, :E].topk(top, dim=1)
+    own = glu(hd @ s_up.double().T, 1.5, 1.0) * torch.sigmoid(z[:, E:])
+    want, size = own @ s_down.double().T, own.abs() @ s_down.double().abs().T
+    for e in range(E):
+        at, place = (ids == e).nonzero(as_tuple=True)
+        act = glu(hd[at] @ up[e].double().T, 7.0, torch.sigmoid(best[at, place])[:, None])
+        want[at] += act @ down[e].double().T
+        size[at] += act.abs() @ down[e].double().abs().T
+    want *= ls.double()
+    got = x.double() - x0.view(T, K).double()
+    assert ((got - want).norm(dim=1) <= 2.0 ** -8 * want.norm(dim=1)).all()
+    assert ((got - want).abs() <= 2.0 ** -8 * size * ls.double().abs() + 2.0 ** -22 * x.double().abs()).all()
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

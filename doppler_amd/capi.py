@@ -163,6 +163,7 @@ SIGNATURES = {
     "dh_mlstm_state_bytes": (_SZ, [ctypes.POINTER(MLSTM)]),
     "dh_mlstm_step": (_I, [ctypes.POINTER(MLSTM), _P, _P, _P, _I, _P]),
     "dh_mlstm_prefill_workspace_bytes": (_SZ, [ctypes.POINTER(MLSTM), _I]),
+    "dh_mlstm_prefill_layout": (_I, [ctypes.POINTER(MLSTM), _I, _I, ctypes.POINTER(ctypes.c_int64)]),
     "dh_mlstm_prefill": (_I, [ctypes.POINTER(MLSTM), _P, _P, _P, _P, _I, _I, _I]),
     "dh_head_norm_gate": (_I, [_P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F]),
     "dh_experts_step_workspace_bytes": (_SZ, [ctypes.POINTER(Experts)]),

@@ -14,7 +14,12 @@
 // masked product inside it:
 //
 //   mlstm_gates_kernel     F, i, m of every token; one workgroup per head
-//   mlstm_states_kernel    the state in front of every chunk, walking the chunks with a tile of it in registers
+//   mlstm_states_kernel    the state in front of every chunk, walking the chunks with a tile of it in registers; or, where few tiles would
+//                          walk far, in two launches:
+//   mlstm_chunks_kernel    what every chunk adds to the state behind it, sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T: independent of
+//                          one another, because m is known
+//   mlstm_scan_kernel      the state in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + what chunk c adds,
+//                          element by element and in place
 //   mlstm_outputs_kernel   o of (chunk, head, value columns): Q K^T and Q S in one walk over dim, decay mask, then (Q K^T) V
 //
 // on the 32-bit matrix-core instruction v_mfma_f32_32x32x2_f32.  head_norm_gate_kernel then divides every head's output by its root
@@ -50,7 +55,7 @@ struct MemArgs {
   float* mt;               // m after every token
   float* mc;               // [H][chunks + 1] m in front of every chunk, and at the end
   float* keep;             // [H][chunks] what a chunk leaves of the state in front of it
-  float* w;                // [H][chunks][64] weight of a token's key and value in the state behind its chunk, zero past the last
+  float* w;                // [H][chunks][64] weight of a token's key and value in the state behind its chunk, zero past the last; null: no walk
   float* Sc;               // [chunks + 1][H][DP][VP]
   float* nc;               // [chunks + 1][H][DP]
 };
@@ -195,11 +200,100 @@ __global__ __launch_bounds__(1024) void mlstm_gates_kernel(const MemArgs a) {
     const double start = c > 0 ? F[c * kChunk - 1] : 0.0, end = F[min((c + 1) * kChunk, a.T) - 1];
     a.keep[(int64_t)h * a.chunks + c] = expf((float)(end - start + (double)mc[c] - (double)mc[c + 1]));
   }
+  if (!a.w) return;
   for (int t = tid; t < a.chunks * kChunk; t += 1024) {
     const int c = t / kChunk, last = min((c + 1) * kChunk, a.T) - 1;
     // in fours of tokens, a token of every four beside those of the others
     a.w[((int64_t)h * a.chunks + c) * kChunk + 16 * (t & 3) + ((t & (kChunk - 1)) >> 2)] = t <= last ? expf((float)(F[last] - F[t] + (double)li[t] - (double)mc[c + 1])) : 0.f;
   }
+}
+
+// Grid = (64 x 64 tiles of a head's state, heads, chunks); wave w: rows 32 (w >> 1), columns 32 (w & 1) of the tile.
+__global__ __launch_bounds__(256) void mlstm_chunks_kernel(const MemArgs a) {
+  constexpr int ROW = 64 + 4;
+  __shared__ __align__(16) float ks[kChunk * ROW];     // weighted keys [token][dim]
+  __shared__ __align__(16) float vs[kChunk * ROW];     // values [token][column]
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y, c = blockIdx.z;
+  const int tiles_v = (a.VP + 63) / 64, d0 = 64 * (blockIdx.x / tiles_v), v0 = 64 * (blockIdx.x % tiles_v);
+  const double* F = a.F + (int64_t)h * a.T;
+  const int first = c * kChunk, count = min(kChunk, a.T - first);
+  const double F_end = F[first + count - 1];
+  const float m_end = a.mc[(int64_t)h * (a.chunks + 1) + c + 1];
+  f32x4_t kr[4], vr[4];
+  float w[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int p = tid + 256 * r, tok = first + min(p >> 4, count - 1), x = 4 * (p & 15);
+    const float* row = a.rows + (int64_t)tok * a.ld_row;
+    kr[r] = vr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (d0 + x < a.DP) kr[r] = *reinterpret_cast<const f32x4_t*>(row + a.k_off + (int64_t)h * a.DP + d0 + x);
+    if (v0 + x < a.VP) vr[r] = *reinterpret_cast<const f32x4_t*>(row + a.v_off + (int64_t)h * a.VP + v0 + x);
+    w[r] = (p >> 4) < count ? expf((float)(F_end - F[tok] + (double)a.i[(int64_t)h * a.T + tok] - (double)m_end)) : 0.f;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int p = tid + 256 * r, tok = p >> 4, x = 4 * (p & 15);
+    // (rows past the last repeat it: an infinite one times a weight of zero is no number)
+    if ((p >> 4) < count) kr[r] *= w[r];
+    else kr[r] = vr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f32x4_t*>(&ks[tok * ROW + x]) = kr[r];
+    *reinterpret_cast<f32x4_t*>(&vs[tok * ROW + x]) = vr[r];
+  }
+  __syncthreads();
+  const int wd = 32 * (wave >> 1), wv = 32 * (wave & 1);
+  if (d0 + wd < a.DP && v0 + wv < a.VP) {              // wave-uniform (sizes are multiples of 32)
+    f32x16_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+#pragma unroll 8
+    for (int j = 0; j < kChunk / 2; j++) {
+      const int tok = 2 * j + (lane >> 5);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[tok * ROW + wd + (lane & 31)], vs[tok * ROW + wv + (lane & 31)], acc, 0, 0, 0);
+    }
+    // accumulator element e of a lane: state row 8 (e / 4) + 4 (lane >> 5) + e % 4, column lane & 31
+    float* U = a.Sc + ((int64_t)(c + 1) * a.H + h) * a.DP * a.VP + (int64_t)(d0 + wd + 4 * (lane >> 5)) * a.VP + v0 + wv + (lane & 31);
+#pragma unroll
+    for (int e = 0; e < 16; e++) U[(int64_t)(8 * (e >> 2) + (e & 3)) * a.VP] = acc[e];
+  }
+  if (v0 == 0 && tid < 64 && d0 + tid < a.DP) {
+    float s = 0.f;
+#pragma unroll 8
+    for (int t = 0; t < kChunk; t++) s += ks[t * ROW + tid];
+    a.nc[((int64_t)(c + 1) * a.H + h) * a.DP + d0 + tid] = s;
+  }
+}
+
+// Grid = (groups of 1024 elements of a head's [S | n], heads), four per thread; slot 0 of Sc and nc is filled here.
+__global__ __launch_bounds__(256) void mlstm_scan_kernel(const MemArgs a) {
+  constexpr int AHEAD = 16;
+  const int h = blockIdx.y, size = a.DP * a.VP;
+  const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (i >= size + a.DP) return;
+  const bool is_n = i >= size;
+  const int64_t stride = is_n ? (int64_t)a.H * a.DP : (int64_t)a.H * size;
+  float* at = is_n ? a.nc + (int64_t)h * a.DP + (i - size) : a.Sc + (int64_t)h * size + i;
+  const int64_t slots = (int64_t)a.H * a.DP;
+  const float* from = is_n ? a.n + (a.pos & 1) * slots + (int64_t)h * a.DP + (i - size) : a.S + (int64_t)h * size + i;
+  float* to = is_n ? a.n + ((a.pos + a.T) & 1) * slots + (int64_t)h * a.DP + (i - size) : a.S + (int64_t)h * size + i;
+  const float* keep = a.keep + (int64_t)h * a.chunks;
+  f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+  if (a.pos > 0) s = *reinterpret_cast<const f32x4_t*>(from);
+  *reinterpret_cast<f32x4_t*>(at) = s;
+  for (int c0 = 0; c0 < a.chunks; c0 += AHEAD) {
+    f32x4_t u[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+      if (c0 + k < a.chunks) u[k] = *reinterpret_cast<const f32x4_t*>(at + (c0 + k + 1) * stride);
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+      const int c = c0 + k;
+      if (c < a.chunks) {
+        s = s * keep[c] + u[k];
+        if (c + 1 < a.chunks) *reinterpret_cast<f32x4_t*>(at + (c + 1) * stride) = s;
+      }
+    }
+  }
+  *reinterpret_cast<f32x4_t*>(to) = s;
 }
 
 // The states in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T, in one walk.
@@ -612,6 +706,16 @@ MemArgs make_args(const dh_mlstm* s, const float* rows, float* state, float* out
 }
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Rows of the states' tiles, 0: two launches.  Tiles of 64 rows, or of 32 where those would not fill the device (us, 64 / 32: 128 x 256 34 /
+// 28.4, 256 x 512 36 / 41).  A walk takes 0.79 us a chunk however few its tiles are, two launches 0.22 where few and 0.65 where there are
+// 32 of 64 x 64 (one workgroup a chunk each): us for state and chunks, walk / two launches: 1 x 64 x 64 (one tile) 1000 tokens 14.3 / 12.4, 2048 27 / 15.6,
+// 8192 102 / 36; 2 x 128 x 256 (16 tiles) 1500 21.8 / 20.8, 8192 103 / 64; 4 x 128 x 256 (32) 2048 29.2 / 28.6, 8192 105 / 94.
+int walk_rows(const dh_mlstm& s, int chunks) {
+  const int64_t tiles = dh::ceil_div(s.DP, 64) * dh::ceil_div(s.VP, 64) * s.H;
+  if (tiles < 32 && chunks > 12 + tiles / 2) return 0;
+  return dh::ceil_div(s.DP, 64) * (s.VP / 32) * s.H >= dh::num_cus() ? 64 : 32;
+}
+
 template <int ROWS>
 int launch_states(const char* op, const MemArgs& a) {
   using Tile = StateTile<ROWS>;
@@ -653,6 +757,16 @@ size_t dh_mlstm_prefill_workspace_bytes(const dh_mlstm* s, int T) {
          up256((chunks + 1) * s->H * s->DP * s->VP * 4);
 }
 
+int dh_mlstm_prefill_layout(const dh_mlstm* spec, int T, int num_cus, int64_t* out1) {
+  const char* op = "dh_mlstm_prefill_layout";
+  if (int rc = check(op, spec)) return rc;
+  if (!out1 || T <= 0) return dh::fail(1, "[%s] T=%d, or no place for the result", op, T);
+  dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
+  *out1 = walk_rows(*spec, (int)dh::ceil_div(T, kChunk));
+  dh::plan_end();
+  return 0;
+}
+
 int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, void* d_workspace, float* d_out, int ld_out, int T,
                      int start_pos) {
   const char* op = "dh_mlstm_prefill";
@@ -677,11 +791,19 @@ int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, v
   a.Sc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * spec->VP * 4));
   // (more chunks than a grid's smaller dimensions hold have always been refused)
   if (a.chunks > 65535) return dh::fail(1, "[%s] %d tokens are too many for one portion", op, T);
+  const int rows = walk_rows(*spec, a.chunks);
+  if (!rows) a.w = nullptr;
   hipLaunchKernelGGL(mlstm_gates_kernel, dim3(spec->H), dim3(1024), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
-  // tiles of 64 rows, or of 32 where those would not fill the device (us, 64 / 32: 128 x 256 34 / 28.4, 256 x 512 36 / 41)
-  const int64_t tall = dh::ceil_div(spec->DP, 64) * (spec->VP / 32) * spec->H;
-  if (int rc = tall >= dh::num_cus() ? launch_states<64>(op, a) : launch_states<32>(op, a)) return rc;
+  if (rows) {
+    if (int rc = rows == 64 ? launch_states<64>(op, a) : launch_states<32>(op, a)) return rc;
+  } else {
+    const int tiles = (int)(dh::ceil_div(spec->DP, 64) * dh::ceil_div(spec->VP, 64));
+    hipLaunchKernelGGL(mlstm_chunks_kernel, dim3(tiles, spec->H, a.chunks), dim3(256), 0, dh::stream(), a);
+    DH_CHECK_LAUNCH(op);
+    hipLaunchKernelGGL(mlstm_scan_kernel, dim3((unsigned)dh::ceil_div((int64_t)spec->DP * spec->VP + spec->DP, 1024), spec->H), dim3(256), 0, dh::stream(), a);
+    DH_CHECK_LAUNCH(op);
+  }
   // wide column groups repeat Q K^T less often; narrow ones where those would not fill the device
   const bool wide = spec->VP > 64 && (int64_t)a.chunks * spec->H * dh::ceil_div(spec->VP, 128) >= dh::num_cus();
   if (wide) hipLaunchKernelGGL(mlstm_outputs_kernel<2>, dim3(a.chunks, spec->H, (unsigned)dh::ceil_div(spec->VP, 128)), dim3(256), 0, dh::stream(), a);

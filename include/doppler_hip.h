@@ -525,6 +525,9 @@ int dh_mlstm_step(const dh_mlstm* spec, const float* d_row, void* d_state, float
 size_t dh_mlstm_prefill_workspace_bytes(const dh_mlstm* spec, int T);
 int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, void* d_workspace, float* d_out, int ld_out, int T,
                      int start_pos);
+/* How dh_mlstm_prefill would make the states in front of a portion's chunks: out1 = rows of the tiles that walk the chunks (64, 32), or 0 for
+ * two launches.  For tests that have to reach every form; needs no device. */
+int dh_mlstm_prefill_layout(const dh_mlstm* spec, int T, int num_cus, int64_t* out1);
 /* y = x_h / sqrt(mean of the head's `size` elements squared + eps) * weight * sigmoid(gate), per head of `padded` elements;
  * output DH_BF16 or DH_F32. */
 int dh_head_norm_gate(const float* d_x, int ld_x, const float* d_gate, int ld_gate, const float* d_weight, void* d_out, int out_dtype,

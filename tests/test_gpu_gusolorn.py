@@ -207,9 +207,23 @@ def test_memory_state_behind_a_prompt(L, H, D, V, T, start):
             assert np.abs(a[fin] - b[fin]).max() <= 64 * 2.0 ** -24 * max(1.0, np.abs(b[fin]).max()) * 4, (name, bad)
 
 
-@pytest.mark.parametrize("H,D,V,T,start", [(8, 96, 512, 130, 3), (16, 64, 512, 63, 0), (1, 32, 64, 64 * 65 + 1, 0)])
-def test_memory_state_walks(L, H, D, V, T, start):
-    """The same on tiles of 64 rows, the last of them half full, and over more chunks than one read of what they keep holds (64)."""
+def memory_spec(H, D, V):
+    """A memory whose sizes need no padding, and the lengths of its rows of q, k, v and of whole ones."""
+    qkv = H * (2 * D + V)
+    ld = qkv + 2 * H + 2 * H % 4
+    return capi.MLSTM(H, D, V, D, V, H * D, 2 * H * D, qkv, qkv + H, ld, 15.0), qkv, ld
+
+
+def walk_rows(L, spec, T):
+    out = ctypes.c_int64(-1)
+    capi.check(L.dh_mlstm_prefill_layout(ctypes.byref(spec), T, 0, ctypes.byref(out)))
+    return out.value
+
+
+@pytest.mark.parametrize("H,D,V,T,start,rows", [(8, 96, 512, 130, 3, 64), (16, 64, 512, 63, 0, 64), (1, 32, 64, 64 * 65 + 1, 0, 0), (2, 96, 32, 1500, 7, 0)])
+def test_memory_state_walks(L, H, D, V, T, start, rows):
+    """The same on tiles of 64 rows, the last of them half full, and in two launches, over more chunks than one read of what they keep holds (64)."""
+    assert walk_rows(L, memory_spec(H, D, V)[0], T) == rows
     test_memory_state_behind_a_prompt(L, H, D, V, T, start)
 
 

@@ -259,3 +259,13 @@ def test_spec_sizes_without_a_device():
     assert L.dh_mlstm_state_bytes(ctypes.byref(spec)) == -(-(3 * 32 * 64 + 2 * 3 * 32 + 2 * 3) * 4 // 256) * 256
     assert L.dh_mlstm_step(ctypes.byref(spec), None, None, None, 0, None) != 0
     assert L.dh_experts_prefill(None, None, capi.BF16, None, 0, None, 1) != 0
+
+
+@pytest.mark.parametrize("H,D,V,T,rows", [(1, 32, 32, 300, 32), (1, 64, 64, 2048, 0), (1, 32, 64, 64 * 65 + 1, 0), (4, 64, 128, 8192, 0), (2, 128, 256, 40, 32),
+                                          (2, 128, 256, 8192, 0), (4, 128, 256, 2000, 32), (4, 256, 512, 40, 64), (8, 256, 512, 8192, 64), (16, 64, 512, 1, 64)])
+def test_states_of_a_prompt_walk_where_tiles_are_many_or_the_way_is_short(H, D, V, T, rows):
+    import ctypes
+    nq, n = H * D, H * (2 * D + V)
+    spec, out = capi.MLSTM(H, D, V, D, V, nq, 2 * nq, n, n + H, n + 4 * H, 2.0), ctypes.c_int64(-1)
+    capi.check(capi.load().dh_mlstm_prefill_layout(ctypes.byref(spec), T, 256, ctypes.byref(out)))
+    assert out.value == rows

@@ -317,44 +317,54 @@ struct StateTile {           // ROWS x 32 of a state; a wave 16 x 16 of it
   static __device__ __forceinline__ int key_swap(int token) { return ROWS == 64 ? 4 * (token & 3) : 4 * ((token >> 1) & 1); }
   static __device__ __forceinline__ int value_swap(int token) { return 4 * ((token >> 1) & 1); }
 };
-// 64 elements of a head's normaliser: a wave sums a chunk's weighted keys, the first wave then takes the waves' chunks in turn.
+// 64 elements of a head's normaliser: a wave sums a chunk's weighted keys, rounded and added token by token as mlstm_chunks_kernel does, then
+// every wave takes the waves' chunks in turn and stores the one in front of which is its own.  The next chunks' keys are requested in front of that.
 template <int WAVES>
-__device__ __forceinline__ void walk_normaliser(const MemArgs& a, int part, float* sums) {      // [WAVES][64]
+__device__ __forceinline__ void walk_normaliser(const MemArgs& a, int part, float* sums) {      // [2][WAVES][64]
+  constexpr int HALF = kChunk / 2;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int parts = (a.DP + 63) / 64, h = part / parts, d = 64 * (part % parts) + lane;
   const int64_t slots = (int64_t)a.H * a.DP, at = (int64_t)h * a.DP + min(d, a.DP - 1);
   const float* rows = a.rows + a.k_off + (int64_t)h * a.DP + 64 * (part % parts);
   const uint32_t column = (uint32_t)min(lane, a.DP - 1 - 64 * (part % parts));
-  const float* w = a.w + (int64_t)h * a.chunks * kChunk;
+  const float *w = a.w + (int64_t)h * a.chunks * kChunk, *keep = a.keep + (int64_t)h * a.chunks;
   const bool live = d < a.DP;
   float n = a.pos > 0 ? a.n[(a.pos & 1) * slots + at] : 0.f;
   if (wave == 0 && live) a.nc[at] = n;
-  for (int c0 = 0; c0 < a.chunks; c0 += WAVES) {
-    const int c = min(c0 + wave, a.chunks - 1), first = c * kChunk, count = min(kChunk, a.T - first);
-    const float weight = w[first + lane];              // that of token 4 (lane % 16) + lane / 16
+  float k[2][HALF], weight = 0.f, kept = 0.f;          // weight: that of token 4 (lane % 16) + lane / 16; kept: of 64 chunks
+  auto chunk_of = [&](int c0) { return min(c0 + wave, a.chunks - 1); };
+  auto request = [&](int c0, int half) {
+    const int first = chunk_of(c0) * kChunk, last = min(first + kChunk, a.T) - 1;
+#pragma unroll
+    for (int i = 0; i < HALF; i++) k[half][i] = (rows + (int64_t)min(first + half * HALF + i, last) * a.ld_row)[column];
+  };
+  auto request_first = [&](int c0) {
+    if ((c0 & 63) == 0) kept = keep[min(c0 + lane, a.chunks - 1)];
+    weight = w[chunk_of(c0) * kChunk + lane];
+    request(c0, 0);
+  };
+  request_first(0);
+  for (int c0 = 0; c0 < a.chunks; c0 += WAVES, sums = c0 / WAVES & 1 ? sums + WAVES * 64 : sums - WAVES * 64) {
+    const int count = a.T - chunk_of(c0) * kChunk;
+    const float held = kept;
+    request(c0, 1);
     float u = 0.f;
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int half = 0; half < kChunk; half += kChunk / 2) {
-      float k[kChunk / 2];
-#pragma unroll
-      for (int i = 0; i < kChunk / 2; i++) k[i] = (rows + (int64_t)(first + min(half + i, count - 1)) * a.ld_row)[column];
-#pragma unroll
-      for (int i = 0; i < kChunk / 2; i++) {
-        const int t = half + i;
-        u = fmaf(t < count ? k[i] : 0.f, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), 16 * (t & 3) + (t >> 2))), u);
-      }
+      for (int t = 0; t < kChunk; t++)
+        u = u + (t < count ? k[t / HALF][t % HALF] : 0.f) * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), 16 * (t & 3) + (t >> 2)));
     }
+    if (c0 + WAVES < a.chunks) request_first(c0 + WAVES);
     sums[64 * wave + lane] = u;
-    __syncthreads();
-    if (wave == 0) {
+    __syncthreads();                                   // (the other half of the sums is written next)
 #pragma unroll
-      for (int i = 0; i < WAVES; i++) {
-        if (c0 + i >= a.chunks) break;
-        n = n * a.keep[(int64_t)h * a.chunks + c0 + i] + sums[64 * i + lane];
-        if (live) a.nc[(c0 + i + 1) * slots + at] = n;
-      }
+    for (int i = 0; i < WAVES; i++) {
+      const int c = c0 + i;
+      if (c >= a.chunks) break;
+      n = fmaf(n, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(held), c & 63)), sums[64 * i + lane]);
+      if (i == wave && live && c + 1 < a.chunks) a.nc[(c + 1) * slots + at] = n;
     }
-    __syncthreads();
   }
   if (wave == 0 && live) a.n[((a.pos + a.T) & 1) * slots + at] = n;
 }
@@ -707,12 +717,12 @@ MemArgs make_args(const dh_mlstm* s, const float* rows, float* state, float* out
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Rows of the states' tiles, 0: two launches.  Tiles of 64 rows, or of 32 where those would not fill the device (us, 64 / 32: 128 x 256 34 /
-// 28.4, 256 x 512 36 / 41).  A walk takes 0.79 us a chunk however few its tiles are, two launches 0.22 where few and 0.65 where there are
-// 32 of 64 x 64 (one workgroup a chunk each): us for state and chunks, walk / two launches: 1 x 64 x 64 (one tile) 1000 tokens 14.3 / 12.4, 2048 27 / 15.6,
-// 8192 102 / 36; 2 x 128 x 256 (16 tiles) 1500 21.8 / 20.8, 8192 103 / 64; 4 x 128 x 256 (32) 2048 29.2 / 28.6, 8192 105 / 94.
+// 28.4, 256 x 512 36 / 41).  A walk takes 0.64 us a chunk however few its tiles are, two launches 0.22 where few and 0.65 where there are
+// 32 of 64 x 64 (one workgroup a chunk each): us for state and chunks, walk / two launches: 1 x 64 x 64 (one tile) 1000 tokens 12.3 / 12.4, 2048 22 / 15.6,
+// 8192 82 / 36; 2 x 128 x 256 (16 tiles) 1500 19 / 20.8, 8192 83 / 64; 4 x 128 x 256 (32) 2048 24.7 / 28.6, 8192 86 / 94.
 int walk_rows(const dh_mlstm& s, int chunks) {
   const int64_t tiles = dh::ceil_div(s.DP, 64) * dh::ceil_div(s.VP, 64) * s.H;
-  if (tiles < 32 && chunks > 12 + tiles / 2) return 0;
+  if (tiles < 32 && chunks > 16 + tiles / 2) return 0;
   return dh::ceil_div(s.DP, 64) * (s.VP / 32) * s.H >= dh::num_cus() ? 64 : 32;
 }
 

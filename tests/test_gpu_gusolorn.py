@@ -227,6 +227,43 @@ def test_memory_state_walks(L, H, D, V, T, start, rows):
     test_memory_state_behind_a_prompt(L, H, D, V, T, start)
 
 
+@pytest.mark.parametrize("H,D,V,T,start,rows,alone", [(16, 64, 512, 64 * 65 + 1, 0, 64, 0), (8, 96, 512, 64 * 28 + 5, 7, 64, 0), (32, 64, 64, 64 * 129 + 2, 3, 32, 0),
+                                                      (8, 96, 512, 600, 3, 64, 32), (300, 32, 32, 70, 1, 64, 32)])
+def test_memory_walks_give_the_bits_of_two_launches(L, H, D, V, T, start, rows, alone):
+    """A head's outputs and state do not depend on the form that the states are made in: among many heads its tiles walk the chunks, alone they are
+    smaller or the chunks are summed and scanned in two launches.  The walks pass every turn of their buffers, weights and normaliser sums."""
+    spec, qkv, ld = memory_spec(H, D, V)
+    one, one_qkv, one_ld = memory_spec(1, D, V)
+    assert (walk_rows(L, spec, T), walk_rows(L, one, T)) == (rows, alone)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, ld, generator=g, device="cuda")
+    state = torch.randn(int(L.dh_mlstm_state_bytes(ctypes.byref(spec))) // 4, generator=g, device="cuda")
+    q, k, v = H * D, H * D * V, H * D * (V + 2)
+
+    def run(spec, x, state, V):
+        ws = torch.full((int(L.dh_mlstm_prefill_workspace_bytes(ctypes.byref(spec), T)),), 255, dtype=torch.uint8, device="cuda")
+        out = torch.zeros(T, spec.H * V, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_mlstm_prefill(ctypes.byref(spec), x.data_ptr(), state.data_ptr(), ws.data_ptr(), out.data_ptr(), spec.H * V, T, start))
+        capi.check(L.dh_sync())
+        return out
+    parts = []
+    for h in (0, H // 2, H - 1):
+        row = torch.zeros(T, one_ld, device="cuda")
+        row[:, :D], row[:, D:2 * D], row[:, 2 * D:one_qkv] = x[:, h * D:(h + 1) * D], x[:, q + h * D:q + (h + 1) * D], x[:, 2 * q + h * V:2 * q + (h + 1) * V]
+        row[:, one_qkv], row[:, one_qkv + 1] = x[:, qkv + h], x[:, qkv + H + h]
+        own = torch.zeros(int(L.dh_mlstm_state_bytes(ctypes.byref(one))) // 4, device="cuda")
+        own[:D * V], own[D * V:D * (V + 2)] = state[h * D * V:(h + 1) * D * V], state[k:v].view(2, H, D)[:, h].reshape(-1)
+        own[D * (V + 2):D * (V + 2) + 2] = state[v:v + 2 * H].view(2, H)[:, h]
+        parts.append((h, run(one, row, own, V), own))
+    out, to = run(spec, x, state, V), (start + T) & 1
+    for h, alone, own in parts:
+        assert torch.equal(out[:, h * V:(h + 1) * V], alone), h
+        assert torch.equal(state[h * D * V:(h + 1) * D * V], own[:D * V]), h
+        assert torch.equal(state[k:v].view(2, H, D)[to, h], own[D * V:D * (V + 2)].view(2, D)[to]), h
+        assert state[v:].view(-1)[to * H + h] == own[D * (V + 2) + to], h
+
+
 @pytest.mark.parametrize("live,before", [(1, 0), (2, 0), (4, 0), (1, 64)])
 def test_memory_state_of_few_live_tokens(L, live, before):
     """A chunk that few tokens count in (a portion of one, two or four tokens, and one whose last token closes the forget gate over 64 others)

@@ -304,8 +304,8 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const MemArgs a) {
 // through registers the compiler waited for the youngest load and store at every chunk (2.3 us each).  Four tokens make an instruction, so their
 // rows' 16-byte pieces are kept apart by 16 banks (slot = piece ^ 4 (token & 3) of 16, piece ^ 4 (token / 2 & 1) of 8).
 // The workgroups behind the tiles walk the normaliser.
-// us, against a launch for what every chunk adds (to memory and back) and another for the scan: four heads of 256 x 512, 1531 tokens 38 + 18.6 -> 35.5, eight, 900
-// tokens 46.6 + 21.6 -> 41, four of 128 x 256, 2000 tokens 17.7 + 11.3 -> 28.3, 40 tokens 6.9 + 2.7 -> 4.8.  Of 35.5 the matrix cores take 15.
+// us, against a launch for what every chunk adds (to memory and back) and another for the scan: four heads of 256 x 512, 1500 tokens 37.7 + 18.1 -> 33, eight, 1000
+// tokens 46 + 21.7 -> 38.5, four of 128 x 256, 2048 tokens 17.2 + 11.4 -> 24.7, 40 tokens 6 + 4.8 -> 4.9.  Of 33 the matrix cores take 15.
 template <int ROWS>
 struct StateTile {           // ROWS x 32 of a state; a wave 16 x 16 of it
   static constexpr int kWaves = ROWS / 8, kThreads = 64 * kWaves;
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(StateTile<ROWS>::kThreads, ROWS == 64 ? 4 : 2) void
     }
     const float left = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kept), c & 63));
     s = s * left + u;
-    front += a.H * size;
+    front = c + 1 < a.chunks ? front + a.H * size : a.S + at;      // (nobody reads the state behind the last chunk from the workspace)
     store(front);
     next_buffer();
   };
@@ -506,7 +506,6 @@ __global__ __launch_bounds__(StateTile<ROWS>::kThreads, ROWS == 64 ? 4 : 2) void
     step(c + 1, odd, even);
   }
   dh::arrive_and_wait<0>();                            // nothing may be in flight towards LDS when the workgroup ends
-  store(a.S + at);
 }
 
 // Grid = (chunks, heads, groups of 64 TN value columns); wave w: tokens 32 (w >> 1), columns 32 TN (w & 1) + 0 .. 32 TN - 1.

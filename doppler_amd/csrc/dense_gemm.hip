@@ -205,19 +205,18 @@ __device__ __forceinline__ void store_glu(const GemmArgs& a, const TilePlace& p,
   if (n0 >= a.N) return;
   const int mb = m0 + 4 * (lane >> 5);
   float f[R][16];          // a row's factor, on what goes in or on what comes out
-  const float* factors = a.rows.row_in ? a.rows.row_in : a.rows.row_out;
-  if (factors) {
+  if (a.rows.factor) {
 #pragma unroll
     for (int t = 0; t < R; t++)
 #pragma unroll
-      for (int i = 0; i < 16; i++) f[t][i] = factors[p.base + min(tile_row(mb + 32 * t, i), p.rows - 1)];
+      for (int i = 0; i < 16; i++) f[t][i] = a.rows.factor[p.base + min(tile_row(mb + 32 * t, i), p.rows - 1)];
   } else {
 #pragma unroll
     for (int t = 0; t < R; t++)
 #pragma unroll
       for (int i = 0; i < 16; i++) f[t][i] = 1.f;
   }
-  const bool in = a.rows.row_in != nullptr;
+  const bool in = a.rows.factor_in;
 #pragma unroll
   for (int t = 0; t < R; t++) {
     float y[16];

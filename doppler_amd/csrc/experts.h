@@ -12,8 +12,8 @@ struct ExpertRows {
   int source_rows;
   int64_t w_stride;        // elements between the experts' matrices
   int max_tiles, tile_rows;
-  const float* row_in;     // factor of a row's input (gate and up before the clamps), or null
-  const float* row_out;    // factor of a row's output, or null
+  const float* factor;     // a row's factor, or null: of its input (gate and up before the clamps) or of its output
+  bool factor_in;
   float limit;
 };
 

@@ -492,9 +492,9 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   DH_CHECK_LAUNCH(op);
   dh::ExpertRows rows{};
   rows.tiles = i32(p.tiles); rows.group_off = i32(p.off); rows.row_index = i32(p.row_token); rows.source_rows = T; rows.w_stride = (int64_t)2 * spec->ff * spec->K;
-  rows.max_tiles = p.max_tiles; rows.tile_rows = p.tile_rows; rows.row_in = f32(p.row_weight); rows.limit = spec->limit;
+  rows.max_tiles = p.max_tiles; rows.tile_rows = p.tile_rows; rows.factor = f32(p.row_weight); rows.factor_in = true; rows.limit = spec->limit;
   dh::ExpertRows one{};
-  one.row_out = f32(p.sg); one.limit = spec->shared_limit;
+  one.factor = f32(p.sg); one.limit = spec->shared_limit;
   const uint16_t *up = static_cast<const uint16_t*>(spec->d_up), *down = static_cast<const uint16_t*>(spec->d_down);
   const uint16_t *shared_up = static_cast<const uint16_t*>(spec->d_shared_up), *shared_down = static_cast<const uint16_t*>(spec->d_shared_down);
   const bool shared = spec->shared_ff > 0, pairs = shared && operand == DH_BF16;
@@ -507,7 +507,7 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   } else {
     if (int rc = dh::experts_glu(op, rows, d_h, operand, spec->K, up, spec->K, n, 2 * spec->ff, spec->K, w + p.act, operand, spec->ff)) return rc;
   }
-  rows.row_index = nullptr; rows.row_in = nullptr; rows.w_stride = (int64_t)spec->hidden * spec->ff;
+  rows.row_index = nullptr; rows.factor = nullptr; rows.w_stride = (int64_t)spec->hidden * spec->ff;
   auto shared_gate_up = [&] {
     return dh::experts_glu(op, one, d_h, operand, spec->K, shared_up, spec->K, T, 2 * spec->shared_ff, spec->K, w + p.shared_act, operand, spec->shared_ff);
   };

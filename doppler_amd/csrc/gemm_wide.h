@@ -13,7 +13,8 @@ struct WideTile {
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kRound = 1024 * kWaves;                             // bytes all waves fetch with one load each: 8 rows a wave
   static constexpr int kRoundsA = kHalfA / kRound, kRoundsB = kHalfB / kRound;
-  static constexpr int kAhead = BM * BN < 256 * 256 ? 4 : 0, kScratch = 4 * (kHalfA + kHalfB);   // WeightLines
+  static constexpr int kAhead = BM * BN < 256 * 256 ? 4 : 0, kBegun = 2;                    // WeightLines; steps fetched in front of them
+  static constexpr int kScratch = 4 * (kHalfA + kHalfB);
   static constexpr int kLds = kScratch + (kAhead ? 256 : 0);
   static_assert(kHalfA % kRound == 0 && kHalfB % kRound == 0, "whole loads");
 };
@@ -72,12 +73,13 @@ struct WeightLines {
   int next, every, last;
   template <class OffW>
   __device__ __forceinline__ WeightLines(const buffer_words_t& ww, OffW w_off, uint32_t k_bytes, int nk, uint32_t lds0, int wave, int lane, Company c)
-      : words(ww), v_off(w_off((wave % (Tile::BN / 64)) * 64 + lane)), s_off(k_bytes), lds(lds0 + Tile::kScratch), next(c.index),
-        every(c.count), last(c.count >= kLeast && wave < Tile::BN / 64 ? nk : 0) {
-    for (int t = next; t < Tile::kAhead && t < last; t += every) touch_to_lds(words, v_off, s_off + 128u * (uint32_t)t, lds);
+      : words(ww), v_off(w_off((wave % (Tile::BN / 64)) * 64 + lane)), s_off(k_bytes), lds(lds0 + Tile::kScratch),
+        next(c.count >= kLeast && wave < Tile::BN / 64 ? c.index : -1), every(c.count), last(nk) {
+    for (int t = next; (uint32_t)t < Tile::kAhead && t < last; t += every)
+      if (t >= Tile::kBegun) touch_to_lds(words, v_off, s_off + 128u * (uint32_t)t, lds);      // (the tile itself has fetched those in front)
   }
   __device__ __forceinline__ void at(int t) {
-    if (t != next) return;
+    if (t != next) return;                   // (-1: never, and nothing to count: 16 steps of few rows take 0.2 us more with it)
     next += every;
     if (t + Tile::kAhead < last) touch_to_lds(words, v_off, s_off + 128u * (uint32_t)(t + Tile::kAhead), lds);
   }
@@ -260,7 +262,7 @@ struct SmallTile {
   static constexpr int WM = WM_, WN = WN_, G = G_, FA = 0, FB = 0;
   static constexpr int BM = 32 * WM, BN = 32 * G * WN, kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kBufA = BM * 128, kBufB = BN * 128, kRoundsA = kBufA / (1024 * kWaves), kRoundsB = kBufB / (1024 * kWaves);
-  static constexpr int kAhead = 8, kScratch = 4 * (kBufA + kBufB), kLds = kScratch + 256;      // WeightLines
+  static constexpr int kAhead = 8, kBegun = 3, kScratch = 4 * (kBufA + kBufB), kLds = kScratch + 256;      // WeightLines
   static_assert(kBufA % (1024 * kWaves) == 0 && kBufB % (1024 * kWaves) == 0 && 4 * kBufA <= 65536 && 4 * kBufB <= 65536, "whole loads");
 };
 template <class Tile, bool F16, class OffA, class OffW>

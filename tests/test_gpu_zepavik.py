@@ -196,6 +196,29 @@ def test_dense_matmul_gelu_on_every_tile(L, M, N, K, tile, dtype):
     check_forms(L, M, N, K, dtype, ((N // 3, capi.ACT_GELU_ERF, lambda z: 0.5 * z * (1 + torch.erf(z * 0.5 ** 0.5))),))
 
 
+@pytest.mark.parametrize("M,N,K,tile", TILES + [(1, 70, 64, (64, 64, 1)), (9, 100, 128, (64, 64, 1)), (33, 64, 64, (64, 64, 1))])
+def test_dense_matmul_with_a_residual_in_place_on_every_tile(L, M, N, K, tile):
+    """(acc + bias) * scale + what the output held, alone and in front of a second output.  5e-5 of the sums as in check_forms, times scales of
+    up to 4; squared, twice a sum of up to 5."""
+    assert tile_of(L, M, N, K, capi.BF16) == tile
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    W = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16)
+    bias, scale = (torch.randn(N, generator=g, device="cuda") for _ in range(2))
+    acc = A.double() @ W.double().T
+    for first in (N, N // 3):
+        C, C2 = torch.randn(M, first + 3, generator=g, device="cuda"), torch.full((M, N - first + 2), 9.0, device="cuda")
+        want = (acc[:, :first] + bias[:first].double()) * scale[:first].double() + C[:, :first].double()
+        beside = C[:, first:].clone()
+        torch.cuda.synchronize()
+        capi.check(L.dh_dense_matmul_scaled(A.data_ptr(), capi.BF16, K, W.data_ptr(), K, M, N, K, 1.0, bias.data_ptr(), scale.data_ptr(), C.data_ptr(),
+                                            C.data_ptr(), first + 3, first, C2.data_ptr(), capi.F32, N - first + 2, capi.ACT_RELU2))
+        capi.check(L.dh_sync())
+        assert (C[:, :first].double() - want).abs().max() < 2e-4 and torch.equal(C[:, first:], beside)
+        if first < N:
+            assert (C2[:, :N - first].double() - acc[:, first:].clamp(min=0).square()).abs().max() < 5e-4 and (C2[:, N - first:] == 9.0).all()
+
+
 def check_forms(L, M, N, K, dtype, forms):
     code = capi.BF16 if dtype == torch.bfloat16 else capi.F16
     g = torch.Generator(device="cuda").manual_seed(M + N + K)

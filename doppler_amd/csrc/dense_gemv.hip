@@ -2,10 +2,11 @@
 //
 // The row sits in LDS as f32 (optionally RMS-normalised on its way there); a wave streams one weight row at a time,
 // 16 bytes per lane and load with the non-temporal hint, U loads of the next stage in flight while the current
-// ones are multiplied (f32 fma on the widened weights, so the product is a 32-bit one).  The row (as far as a few pieces a thread hold it) and its norm's
-// weights are requested first, the first stage of weights behind them: loads arrive in order, so the row is prepared while the weights
-// still travel, and what an output adds and multiplies in comes with its row's weights: short products are a chain of such trips (2048 x 8192
-// with a residual 10.8 -> 9.3 us in a step, gated heads 1024 x 1024 4.9 -> 4.5, 32000 x 1024 14.5 -> 13.6).
+// ones are multiplied (f32 fma on the widened weights, so the product is a 32-bit one).  The row (as far as a few pieces a thread hold it), its norm's
+// weights, the first stage of weights and what an output adds and multiplies in are requested together: short products are a chain of trips to
+// memory, and this makes them one.  (The weights' loads are conditional, so the compiler cannot count them, and the row is prepared when all of it has
+// arrived, not while the weights travel.)  us, alone, weights from memory, against weights in front of a row that was requested when they had come: 2048 x 8192 with a
+// residual 9.5 -> 8.9, 2048 x 1024 4.1 -> 3.7, 4096 x 4096 with a norm 8.7 -> 7.9, 3080 x 1024 4.6 -> 4.6, gated heads 1024 x 1024 4.8 -> 4.2, 32000 x 1024 18.7 -> 14.4.
 // The row is kept as two planes of 16-byte pieces (elements 0..3 and 4..7 of every eight) so that a wave's reads of either plane are consecutive.
 //
 // Outputs as in the multi-row product (dense_gemm.hip): columns below n_first with bias, column scale and residual, the rest
@@ -49,7 +50,7 @@ struct GemvArgs {
   uint32_t* part_idx;
 };
 
-template <int U, int WAVES, bool ARGMAX, bool HEADS>
+template <int U, int WAVES, int BATCH, bool ARGMAX, bool HEADS>
 __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   extern __shared__ __align__(16) float4 planes[];      // [2][K / 8]
   __shared__ float red[WAVES];
@@ -86,7 +87,6 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   };
 
   // ---- the activation row
-  constexpr int BATCH = HEADS || WAVES < 8 ? 4 : 2;       // 16-byte pieces of a thread requested at once (four workgroups of eight waves: 64 registers)
   if constexpr (HEADS) {
     // weighted and gated on the way in; the squares are summed by eight lanes (whole heads: their sizes are multiples of 32), then by
     // head, and the row in LDS is scaled last: one trip to memory
@@ -222,9 +222,10 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   }
 }
 
-template <int U, int WAVES, bool ARGMAX, bool HEADS>
+// BATCH: 16-byte pieces of the row that a thread requests in front of the weights.
+template <int U, int WAVES, int BATCH, bool ARGMAX, bool HEADS>
 int launch(const char* op, GemvArgs a, int max_grid, int* parts) {
-  auto kern = gemv_kernel<U, WAVES, ARGMAX, HEADS>;
+  auto kern = gemv_kernel<U, WAVES, BATCH, ARGMAX, HEADS>;
   static bool attr_set = false;
   if (!attr_set) {
     DH_CHECK_HIP(op, hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -247,15 +248,19 @@ int launch_loads(const char* op, const GemvArgs& a, int max_grid, int* parts) {
   // of the bytes in flight).  Four waves a workgroup are few, so long rows get long stages there, and gated heads where a row is all a wave
   // has (2048 x 4096 7.5 -> 7.1 us) or very long (4096 x 8192 19.3 -> 16.9); two stages of 1536 fit rows up to 3072 better than two of
   // 2048 (2560 x 2560 5.9 -> 5.5).
-  if (a.K <= 1024) return launch<2, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
-  if (a.K <= 2048) return launch<4, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
-  if constexpr (WAVES == 4) return launch<8, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  // Pieces: what a row up to the stage's length has for a thread.  Requests for more of them stand in front of the weights for nothing (us, two or
+  // four pieces / one: norm 1536 x 1024 4.2 -> 3.9, 3080 x 1024 4.8 -> 4.6, 2050 x 2048 5.1 -> 4.9, heads 1024 x 1024 4.4 -> 4.2); output heads, with
+  // many rows a wave, go better with two (32000 x 2048 21.1 against 22.0).  Longer rows: as many as registers allow (four workgroups of eight waves: 64).
+  constexpr int BATCH = HEADS || WAVES == 4 ? 4 : 2;
+  if (a.K <= 1024) return launch<2, WAVES, ARGMAX ? 2 : 1, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if (a.K <= 2048) return launch<4, WAVES, ARGMAX || WAVES == 4 ? 2 : 1, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if constexpr (WAVES == 4) return launch<8, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
   if constexpr (HEADS) {
-    if (WAVES == 8 ? a.N <= 8 * dh::num_cus() : a.K > 4096) return launch<8, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+    if (WAVES == 8 ? a.N <= 8 * dh::num_cus() : a.K > 4096) return launch<8, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
   } else {
-    if (a.K <= 3072) return launch<3, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+    if (a.K <= 3072) return launch<3, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
   }
-  return launch<4, WAVES, ARGMAX, HEADS>(op, a, max_grid, parts);
+  return launch<4, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
 }
 
 // Rows of each of its workgroups that the busiest compute unit goes through, with at most `per_cu` workgroups on every one.
@@ -272,7 +277,7 @@ int64_t busiest(int64_t N, int waves, int per_cu) {
 template <bool ARGMAX, bool HEADS = false>
 int dispatch(const char* op, const GemvArgs& a, int* parts) {
   const int cus = dh::num_cus();
-  if (a.K > 8192) return launch<8, 8, ARGMAX, HEADS>(op, a, a.K <= 16384 ? 2 * cus : cus, parts);
+  if (a.K > 8192) return launch<8, 8, HEADS ? 4 : 2, ARGMAX, HEADS>(op, a, a.K <= 16384 ? 2 * cus : cus, parts);
   if constexpr (HEADS)          // three rows are read to prepare one
     if (a.N >= 16 * cus) return launch_loads<16, ARGMAX, HEADS>(op, a, cus, parts);
   if (a.N >= 8 * cus) {

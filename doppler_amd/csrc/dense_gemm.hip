@@ -796,12 +796,13 @@ bool experts_together(const ExpertProduct& routed, const ExpertProduct& shared, 
   const TileCost& c = glu ? kGluTiles[at] : kTiles[at];
   const double work[2] = {(double)routed.M * routed.N * routed.K, (double)shared.M * shared.N * shared.K};
   if (4.0 * std::min(work[0], work[1]) < std::max(work[0], work[1])) return false;
-  const bool gathered = routed.rows.row_index;
-  if (!(gathered ? (int64_t)2 * routed.rows.source_rows * routed.lda < (int64_t)1 << 32 : within_reach(c.bm, routed.lda, routed.K)) ||
+  // (gate and up products gather their rows)
+  if (!(glu ? (int64_t)2 * routed.rows.source_rows * routed.lda < (int64_t)1 << 32 : within_reach(c.bm, routed.lda, routed.K)) ||
       !within_reach(routed.N, routed.ldw, routed.K) || !within_reach(shared.M, shared.lda, shared.K) || !within_reach(shared.N, shared.ldw, shared.K))
     return false;
   const int64_t tiles_n = dh::ceil_div(routed.N, c.bn), own = dh::ceil_div(shared.M, c.bm) * dh::ceil_div(shared.N, c.bn);
   if ((own + 8 + routed.rows.max_tiles * tiles_n) * 256 >= (int64_t)1 << 32) return false;   // threads of one launch
+  if (!glu && (dh::tuning_int("DH_DENSE_TILE", -1) >= 0 || dh::tuning_int("DH_DENSE_SLICES", 0))) return false;     // asked for by name: apart, as asked
   const TileChoice best = glu ? choose_tile(shared.M, shared.N, shared.K, 1, true, false) : choose_16bit(shared.M, shared.N, shared.K, false);
   return loops_ns(c, own, shared.K / 64, 0.76) + c.start <= 1.15 * best.ns;
 }

@@ -36,7 +36,7 @@ struct ExpertProduct {
   int64_t ld_out;
   const float *col_scale, *residual;
 };
-// Whether the routed experts' product (rows.tiles) and the shared expert's go in one launch, and that launch.
+// Whether the routed experts' product and the shared expert's go in one launch (from the sizes alone), and that launch.
 bool experts_together(const ExpertProduct& routed, const ExpertProduct& shared, bool glu);
 int experts_pair(const char* op, const ExpertProduct& routed, const ExpertProduct& shared, bool glu);
 // Row tiles of the grouped products for this many rows in all.

@@ -409,6 +409,23 @@ PortionSpace portion_space(const dh_experts* s, int operand, int T) {
   return p;
 }
 
+// Sizes of a portion's four products: routed and shared, gate and up (glu) or down.
+dh::ExpertProduct routed_product(const dh_experts* s, const PortionSpace& p, int T, bool glu) {
+  dh::ExpertProduct r{};
+  r.M = T * s->top; r.N = glu ? 2 * s->ff : s->hidden; r.lda = r.ldw = r.K = glu ? s->K : s->ff; r.ld_out = glu ? s->ff : p.ld_y;
+  r.rows.source_rows = T; r.rows.w_stride = (int64_t)r.N * r.K; r.rows.max_tiles = p.max_tiles; r.rows.tile_rows = p.tile_rows; r.rows.limit = s->limit;
+  return r;
+}
+dh::ExpertProduct shared_product(const dh_experts* s, int T, int ld_x, bool glu) {
+  dh::ExpertProduct r{};
+  r.M = T; r.N = glu ? 2 * s->shared_ff : s->hidden; r.lda = r.ldw = r.K = glu ? s->K : s->shared_ff; r.ld_out = glu ? s->shared_ff : ld_x;
+  r.rows.limit = s->shared_limit;
+  return r;
+}
+bool together(const dh_experts* s, int operand, const PortionSpace& p, int T, bool glu) {
+  return s->shared_ff > 0 && operand == DH_BF16 && dh::experts_together(routed_product(s, p, T, glu), shared_product(s, T, s->hidden, glu), glu);
+}
+
 }  // namespace
 
 extern "C" {
@@ -461,6 +478,20 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace) {
 
 size_t dh_experts_prefill_workspace_bytes(const dh_experts* s, int operand, int T) { return s && T > 0 ? portion_space(s, operand, T).end : 256; }
 
+int dh_experts_prefill_layout(const dh_experts* spec, int operand, int T, int num_cus, int64_t* out3) {
+  const char* op = "dh_experts_prefill_layout";
+  if (int rc = check(op, spec)) return rc;
+  if (!out3 || T <= 0 || (int64_t)T * spec->top > (1 << 24) || (operand != DH_BF16 && operand != DH_F32))
+    return dh::fail(1, "[%s] T=%d, dtype %d, or no place for the result", op, T, operand);
+  dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
+  const PortionSpace p = portion_space(spec, operand, T);
+  out3[0] = p.tile_rows;
+  out3[1] = together(spec, operand, p, T, true);
+  out3[2] = together(spec, operand, p, T, false);
+  dh::plan_end();
+  return 0;
+}
+
 int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T) {
   const char* op = "dh_experts_prefill";
   DH_REQUIRE_INIT(op);
@@ -490,45 +521,34 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   hipLaunchKernelGGL(experts_sort_kernel, dim3(1), dim3(1024), 0, dh::stream(), i32(p.ids), f32(p.weights), n, spec->top, spec->experts, p.tile_rows,
                      p.max_tiles, i32(p.off), i32(p.slot), i32(p.row_token), f32(p.row_weight), i32(p.tiles));
   DH_CHECK_LAUNCH(op);
-  dh::ExpertRows rows{};
-  rows.tiles = i32(p.tiles); rows.group_off = i32(p.off); rows.row_index = i32(p.row_token); rows.source_rows = T; rows.w_stride = (int64_t)2 * spec->ff * spec->K;
-  rows.max_tiles = p.max_tiles; rows.tile_rows = p.tile_rows; rows.factor = f32(p.row_weight); rows.factor_in = true; rows.limit = spec->limit;
-  dh::ExpertRows one{};
-  one.factor = f32(p.sg); one.limit = spec->shared_limit;
   const uint16_t *up = static_cast<const uint16_t*>(spec->d_up), *down = static_cast<const uint16_t*>(spec->d_down);
   const uint16_t *shared_up = static_cast<const uint16_t*>(spec->d_shared_up), *shared_down = static_cast<const uint16_t*>(spec->d_shared_down);
-  const bool shared = spec->shared_ff > 0, pairs = shared && operand == DH_BF16;
+  const bool shared = spec->shared_ff > 0, up_pair = together(spec, operand, p, T, true), down_pair = together(spec, operand, p, T, false);
   // gate and up products; the shared expert's beside the routed ones' or behind them
-  const dh::ExpertProduct routed_up{rows, d_h, spec->K, up, spec->K, n, 2 * spec->ff, spec->K, w + p.act, spec->ff, nullptr, nullptr};
-  const dh::ExpertProduct own_up{one, d_h, spec->K, shared_up, spec->K, T, 2 * spec->shared_ff, spec->K, w + p.shared_act, spec->shared_ff, nullptr, nullptr};
-  const bool up_pair = pairs && dh::experts_together(routed_up, own_up, true);
-  if (up_pair) {
-    if (int rc = dh::experts_pair(op, routed_up, own_up, true)) return rc;
-  } else {
-    if (int rc = dh::experts_glu(op, rows, d_h, operand, spec->K, up, spec->K, n, 2 * spec->ff, spec->K, w + p.act, operand, spec->ff)) return rc;
-  }
-  rows.row_index = nullptr; rows.factor = nullptr; rows.w_stride = (int64_t)spec->hidden * spec->ff;
-  auto shared_gate_up = [&] {
-    return dh::experts_glu(op, one, d_h, operand, spec->K, shared_up, spec->K, T, 2 * spec->shared_ff, spec->K, w + p.shared_act, operand, spec->shared_ff);
+  dh::ExpertProduct routed = routed_product(spec, p, T, true), own = shared_product(spec, T, ld_x, true);
+  routed.A = own.A = d_h; routed.W = up; routed.out = w + p.act; own.W = shared_up; own.out = w + p.shared_act;
+  routed.rows.tiles = i32(p.tiles); routed.rows.group_off = i32(p.off); routed.rows.row_index = i32(p.row_token); routed.rows.factor = f32(p.row_weight);
+  routed.rows.factor_in = true; own.rows.factor = f32(p.sg);
+  auto glu = [&](const dh::ExpertProduct& g) {
+    return dh::experts_glu(op, g.rows, g.A, operand, g.lda, g.W, g.ldw, g.M, g.N, g.K, g.out, operand, g.ld_out);
   };
+  if (int rc = up_pair ? dh::experts_pair(op, routed, own, true) : glu(routed)) return rc;
+  auto shared_gate_up = [&] { return up_pair ? 0 : glu(own); };
   // down products: together, the shared expert's reaches x in front of the routed ones' sum
-  const dh::ExpertProduct routed_down{rows, w + p.act, spec->ff, down, spec->ff, n, spec->hidden, spec->ff, f32(p.y), p.ld_y, nullptr, nullptr};
-  const dh::ExpertProduct own_down{dh::ExpertRows{}, w + p.shared_act, spec->shared_ff, shared_down, spec->shared_ff, T, spec->hidden, spec->shared_ff,
-                                   d_x, ld_x, spec->d_layer_scale, d_x};
-  const bool down_pair = pairs && dh::experts_together(routed_down, own_down, false);
+  dh::ExpertProduct routed_down = routed_product(spec, p, T, false), own_down = shared_product(spec, T, ld_x, false);
+  routed_down.A = w + p.act; routed_down.W = down; routed_down.out = f32(p.y); routed_down.rows.tiles = i32(p.tiles); routed_down.rows.group_off = i32(p.off);
+  own_down.A = w + p.shared_act; own_down.W = shared_down; own_down.out = d_x; own_down.col_scale = spec->d_layer_scale; own_down.residual = d_x;
   if (down_pair) {
-    if (!up_pair)
-      if (int rc = shared_gate_up()) return rc;
+    if (int rc = shared_gate_up()) return rc;
     if (int rc = dh::experts_pair(op, routed_down, own_down, false)) return rc;
   } else {
-    if (int rc = dh::experts_down(op, rows, w + p.act, operand, spec->ff, down, spec->ff, spec->hidden, spec->ff, f32(p.y), p.ld_y)) return rc;
+    if (int rc = dh::experts_down(op, routed_down.rows, w + p.act, operand, spec->ff, down, spec->ff, spec->hidden, spec->ff, f32(p.y), p.ld_y)) return rc;
   }
   hipLaunchKernelGGL(experts_combine_kernel, dim3(T, (unsigned)dh::ceil_div(spec->hidden, 1024)), dim3(256), 0, dh::stream(), f32(p.y), (int64_t)p.ld_y,
                      i32(p.slot), spec->top, spec->d_layer_scale, d_x, (int64_t)ld_x, spec->hidden);
   DH_CHECK_LAUNCH(op);
   if (shared && !down_pair) {
-    if (!up_pair)
-      if (int rc = shared_gate_up()) return rc;
+    if (int rc = shared_gate_up()) return rc;
     return dh_dense_matmul_scaled(w + p.shared_act, operand, spec->shared_ff, shared_down, spec->shared_ff, T, spec->hidden, spec->shared_ff, 1.f,
                                   nullptr, spec->d_layer_scale, d_x, d_x, ld_x, spec->hidden, nullptr, 0, 0, DH_ACT_NONE);
   }

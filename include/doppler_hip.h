@@ -557,6 +557,9 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace);
 /* T rows: d_h their normed rows [T][K] in the operand type (DH_BF16 or DH_F32), d_x the residual rows. */
 size_t dh_experts_prefill_workspace_bytes(const dh_experts* spec, int operand, int T);
 int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T);
+/* How dh_experts_prefill would multiply a portion: out3 = rows of the routed experts' tiles, whether the shared expert's gate and up product goes in
+ * their launch, whether its down product does.  For tests that have to reach every form; needs no device. */
+int dh_experts_prefill_layout(const dh_experts* spec, int operand, int T, int num_cus, int64_t* out3);
 
 /* ---- normalisation / rotary / KV ---- */
 

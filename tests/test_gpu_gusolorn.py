@@ -535,11 +535,12 @@ def test_expert_rows_past_4_gb(L, T, W, K, E, top, ff):
         assert ((whole[at:at + size] - alone).norm(dim=1) <= 2.0 ** -8 * alone.norm(dim=1)).all(), at
 
 
-# shared and routed products of one size share a launch: 128-row tiles (ragged ones, an expert that nobody uses), 64-row tiles, and rows past the first
-# eight workgroups' edge; the last keeps them apart (the shared expert is eight times as wide)
-@pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(1531, 1024, 4, 2, 512, 1024), (1000, 1024, 5, 2, 512, 1024), (40, 256, 8, 2, 64, 128), (7, 64, 3, 1, 64, 64),
-                                                    (300, 256, 4, 1, 64, 512)])
-def test_shared_and_routed_products(L, T, K, E, top, ff, shared_ff):
+# rows of the routed experts' tiles, and whether the shared expert's products go in their launch: gate and up, down.  With five experts nobody uses one.
+@pytest.mark.parametrize("T,K,E,top,ff,shared_ff,form", [
+    (1531, 1024, 4, 2, 512, 1024, (128, 1, 1)), (1300, 1024, 5, 2, 512, 1024, (128, 1, 1)), (1000, 1024, 5, 2, 512, 1024, (128, 0, 0)),
+    (600, 1024, 5, 4, 768, 3072, (128, 1, 0)), (1500, 256, 5, 2, 128, 256, (128, 0, 1)), (100, 1024, 5, 4, 768, 3072, (64, 1, 0)), (500, 1024, 16, 2, 768, 3072, (64, 0, 1)),
+    (200, 1024, 5, 2, 512, 1024, (64, 1, 1)), (40, 256, 8, 2, 64, 128, (64, 1, 1)), (7, 64, 3, 1, 64, 64, (64, 1, 1)), (300, 256, 4, 1, 64, 512, (64, 0, 0))])
+def test_shared_and_routed_products(L, T, K, E, top, ff, shared_ff, form):
     """Rows behind both kinds of experts against 64 bits.  Activations are rounded to bf16 in front of the down products, and a routed product behind
     them: 2^-9 of every term each, 2^-8 of the terms' sizes together; over a row of random signs the norms keep 2^-8 as well."""
     g = torch.Generator(device="cuda").manual_seed(T + K)
@@ -550,6 +551,9 @@ def test_shared_and_routed_products(L, T, K, E, top, ff, shared_ff):
         router[2] = 0.0
         router[2, 0], h[:, 0] = -8.0, 4.0
     spec = capi.Experts(K, K, E, top, ff, shared_ff, 1e-5, 7.0, 1.5, norm.data_ptr(), ls.data_ptr(), *(a.data_ptr() for a in (router, up, down, s_up, s_down)))
+    took = (ctypes.c_int64 * 3)()
+    capi.check(L.dh_experts_prefill_layout(ctypes.byref(spec), capi.BF16, T, 0, took))
+    assert tuple(took) == form
     ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T), dtype=torch.uint8, device="cuda")
     x = x0.clone().view(T, K)
     torch.cuda.synchronize()
@@ -564,6 +568,7 @@ def test_shared_and_routed_products(L, T, K, E, top, ff, shared_ff):
     hd = h.double()
     z = hd @ router.double().T
     best, ids = z[:, :E].topk(top, dim=1)
+    assert E != 5 or not (ids == 2).any()
     own = glu(hd @ s_up.double().T, 1.5, 1.0) * torch.sigmoid(z[:, E:])
     want, size = own @ s_down.double().T, own.abs() @ s_down.double().abs().T
     for e in range(E):

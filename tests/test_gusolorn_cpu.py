@@ -269,3 +269,20 @@ def test_states_of_a_prompt_walk_where_tiles_are_many_or_the_way_is_short(H, D, 
     spec, out = capi.MLSTM(H, D, V, D, V, nq, 2 * nq, n, n + H, n + 4 * H, 2.0), ctypes.c_int64(-1)
     capi.check(capi.load().dh_mlstm_prefill_layout(ctypes.byref(spec), T, 256, ctypes.byref(out)))
     assert out.value == rows
+
+
+@pytest.mark.parametrize("T,K,E,top,ff,shared_ff,form", [(1531, 2048, 16, 4, 768, 3072, (128, 1, 1)), (1531, 1024, 4, 2, 512, 1024, (128, 1, 1)),
+                                                         (1000, 1024, 5, 2, 512, 1024, (128, 0, 0)), (600, 1024, 5, 4, 768, 3072, (128, 1, 0)),
+                                                         (1500, 256, 5, 2, 128, 256, (128, 0, 1)), (100, 1024, 5, 4, 768, 3072, (64, 1, 0)),
+                                                         (500, 1024, 16, 2, 768, 3072, (64, 0, 1)), (40, 256, 8, 2, 64, 128, (64, 1, 1)),
+                                                         (1, 64, 4, 1, 64, 512, (64, 0, 0)), (40, 256, 8, 2, 64, 0, (64, 0, 0))])
+def test_experts_share_launches_where_neither_is_small(T, K, E, top, ff, shared_ff, form):
+    import ctypes
+    L, some = capi.load(), 256
+    spec, out = capi.Experts(K, K, E, top, ff, shared_ff, 1e-5, 7.0, 1.5, some, None, *[some] * 5), (ctypes.c_int64 * 3)()
+
+    def took(dtype=capi.BF16):
+        capi.check(L.dh_experts_prefill_layout(ctypes.byref(spec), dtype, T, 256, out))
+        return tuple(out)
+    assert took() == form and took(capi.F32) == (64, 0, 0)
+    assert L.dh_experts_prefill_layout(ctypes.byref(spec), capi.BF16, 0, 256, out) != 0 and L.dh_experts_prefill_layout(ctypes.byref(spec), capi.F16, 1, 256, out) != 0

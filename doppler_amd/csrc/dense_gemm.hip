@@ -290,7 +290,7 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void gemm_experts_kernel(const G
   extern __shared__ __align__(16) char smem[];
   const int block = blockIdx.x;
   if (block >= own_blocks) gemm_16bit<Tile, false, kNoSecond, true, GLU>(routed, block - own_blocks, smem);
-  else if (block < shared.tiles_m * shared.tiles_n) gemm_16bit<Tile, false, GLU ? kNoSecond : kResidual, false, GLU>(shared, block, smem);
+  else if (block < shared.tiles_m * shared.tiles_n) gemm_16bit<Tile, false, kNoSecond, false, GLU>(shared, block, smem);
 }
 
 // The 32-bit product: four waves, a 64 x 64 TN tile, 32 k at a time.  Both tiles sit in LDS as f32 rows of 32 + 4
@@ -778,7 +778,7 @@ GemmArgs expert_args(const dh::ExpertProduct& p, bool glu) {
   if (glu) {
     a.C2 = p.out; a.c2_dtype = DH_BF16; a.ldc2 = (int)p.ld_out;
   } else {
-    a.C = static_cast<float*>(p.out); a.ldc = (int)p.ld_out; a.n_first = p.N; a.col_scale = p.col_scale; a.residual = p.residual;
+    a.C = static_cast<float*>(p.out); a.ldc = (int)p.ld_out; a.n_first = p.N;
   }
   return a;
 }
@@ -804,7 +804,8 @@ bool experts_together(const ExpertProduct& routed, const ExpertProduct& shared, 
   if ((own + 8 + routed.rows.max_tiles * tiles_n) * 256 >= (int64_t)1 << 32) return false;   // threads of one launch
   if (!glu && (dh::tuning_int("DH_DENSE_TILE", -1) >= 0 || dh::tuning_int("DH_DENSE_SLICES", 0))) return false;     // asked for by name: apart, as asked
   const TileChoice best = glu ? choose_tile(shared.M, shared.N, shared.K, 1, true, false) : choose_16bit(shared.M, shared.N, shared.K, false);
-  return loops_ns(c, own, shared.K / 64, 0.76) + c.start <= 1.15 * best.ns;
+  // (slices of the shared one would be sums in another order)
+  return best.slices == 1 && loops_ns(c, own, shared.K / 64, 0.76) + c.start <= 1.15 * best.ns;
 }
 int experts_pair(const char* op, const ExpertProduct& routed, const ExpertProduct& shared, bool glu) {
   const GemmArgs r = expert_args(routed, glu), s = expert_args(shared, glu);

@@ -24,7 +24,7 @@ __device__ __forceinline__ float clamped_glu(float g, float u, float limit) {
   return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
 
-// A bf16 product of experts, all of it: gate and up (out: bf16 activations) or down (out: f32, times col_scale, plus residual).
+// A bf16 product of experts, all of it: gate and up (out: bf16 activations) or down (out: f32).
 struct ExpertProduct {
   ExpertRows rows;
   const void* A;
@@ -34,7 +34,6 @@ struct ExpertProduct {
   int M, N, K;
   void* out;
   int64_t ld_out;
-  const float *col_scale, *residual;
 };
 // Whether the routed experts' product and the shared expert's go in one launch (from the sizes alone), and that launch.
 bool experts_together(const ExpertProduct& routed, const ExpertProduct& shared, bool glu);

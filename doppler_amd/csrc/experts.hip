@@ -349,22 +349,28 @@ __global__ __launch_bounds__(1024) void experts_sort_kernel(const int* __restric
   }
 }
 
-// x[t] += ls * sum of the token's rows.  Four columns per thread.
+// x[t] += ls * sum of the token's rows, then ls * the shared expert's row where that is not null (rounded as an epilogue with scale and residual
+// does: a token has the same bits whether the products share a launch or not).  Four columns per thread.
 __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __restrict__ y, int64_t ld_y, const int* __restrict__ slot, int top,
-                                                              const float* __restrict__ ls, float* __restrict__ x, int64_t ld_x, int hidden) {
+                                                              const float* __restrict__ shared, const float* __restrict__ ls, float* __restrict__ x,
+                                                              int64_t ld_x, int hidden) {
   const int t = blockIdx.x, i = 4 * (blockIdx.y * 256 + threadIdx.x);
   if (i >= hidden) return;
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f), own = s;
+  if (shared) own = *reinterpret_cast<const float4*>(shared + (int64_t)t * ld_y + i);
   for (int k = 0; k < top; k++) {
     const float4 v = *reinterpret_cast<const float4*>(y + (int64_t)slot[(int64_t)t * top + k] * ld_y + i);
     s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
   }
-  const float sv[4] = {s.x, s.y, s.z, s.w};
+  const float sv[4] = {s.x, s.y, s.z, s.w}, ov[4] = {own.x, own.y, own.z, own.w};
 #pragma unroll
   for (int e = 0; e < 4; e++) {
     if (i + e >= hidden) break;
     float* o = x + (int64_t)t * ld_x + i + e;
-    *o = fmaf(ls ? ls[i + e] : 1.f, sv[e], *o);
+    const float f = ls ? ls[i + e] : 1.f;
+    float v = fmaf(f, sv[e], *o);
+    if (shared) v = fmaf(ov[e], f, 0.f) + v;
+    *o = v;
   }
 }
 
@@ -386,7 +392,7 @@ int logits(const dh_experts* s) { return s->experts + (s->shared_ff ? 1 : 0); }
 
 // Where a portion's intermediate rows lie in the workspace.
 struct PortionSpace {
-  size_t z, ids, weights, sg, off, slot, row_token, row_weight, tiles, act, shared_act, y, end;
+  size_t z, ids, weights, sg, off, slot, row_token, row_weight, tiles, act, shared_act, y, shared_y, end;
   int ld_z, ld_y, max_tiles, tile_rows;
 };
 PortionSpace portion_space(const dh_experts* s, int operand, int T) {
@@ -405,6 +411,7 @@ PortionSpace portion_space(const dh_experts* s, int operand, int T) {
   p.act = take(n * s->ff * elem);
   p.shared_act = take((size_t)T * s->shared_ff * elem);
   p.y = take(n * p.ld_y * 4);
+  p.shared_y = take(s->shared_ff && operand == DH_BF16 ? (size_t)T * p.ld_y * 4 : 0);
   p.end = at;
   return p;
 }
@@ -416,14 +423,14 @@ dh::ExpertProduct routed_product(const dh_experts* s, const PortionSpace& p, int
   r.rows.source_rows = T; r.rows.w_stride = (int64_t)r.N * r.K; r.rows.max_tiles = p.max_tiles; r.rows.tile_rows = p.tile_rows; r.rows.limit = s->limit;
   return r;
 }
-dh::ExpertProduct shared_product(const dh_experts* s, int T, int ld_x, bool glu) {
+dh::ExpertProduct shared_product(const dh_experts* s, const PortionSpace& p, int T, bool glu) {
   dh::ExpertProduct r{};
-  r.M = T; r.N = glu ? 2 * s->shared_ff : s->hidden; r.lda = r.ldw = r.K = glu ? s->K : s->shared_ff; r.ld_out = glu ? s->shared_ff : ld_x;
+  r.M = T; r.N = glu ? 2 * s->shared_ff : s->hidden; r.lda = r.ldw = r.K = glu ? s->K : s->shared_ff; r.ld_out = glu ? s->shared_ff : p.ld_y;
   r.rows.limit = s->shared_limit;
   return r;
 }
 bool together(const dh_experts* s, int operand, const PortionSpace& p, int T, bool glu) {
-  return s->shared_ff > 0 && operand == DH_BF16 && dh::experts_together(routed_product(s, p, T, glu), shared_product(s, T, s->hidden, glu), glu);
+  return s->shared_ff > 0 && operand == DH_BF16 && dh::experts_together(routed_product(s, p, T, glu), shared_product(s, p, T, glu), glu);
 }
 
 }  // namespace
@@ -525,7 +532,7 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   const uint16_t *shared_up = static_cast<const uint16_t*>(spec->d_shared_up), *shared_down = static_cast<const uint16_t*>(spec->d_shared_down);
   const bool shared = spec->shared_ff > 0, up_pair = together(spec, operand, p, T, true), down_pair = together(spec, operand, p, T, false);
   // gate and up products; the shared expert's beside the routed ones' or behind them
-  dh::ExpertProduct routed = routed_product(spec, p, T, true), own = shared_product(spec, T, ld_x, true);
+  dh::ExpertProduct routed = routed_product(spec, p, T, true), own = shared_product(spec, p, T, true);
   routed.A = own.A = d_h; routed.W = up; routed.out = w + p.act; own.W = shared_up; own.out = w + p.shared_act;
   routed.rows.tiles = i32(p.tiles); routed.rows.group_off = i32(p.off); routed.rows.row_index = i32(p.row_token); routed.rows.factor = f32(p.row_weight);
   routed.rows.factor_in = true; own.rows.factor = f32(p.sg);
@@ -534,10 +541,10 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   };
   if (int rc = up_pair ? dh::experts_pair(op, routed, own, true) : glu(routed)) return rc;
   auto shared_gate_up = [&] { return up_pair ? 0 : glu(own); };
-  // down products: together, the shared expert's reaches x in front of the routed ones' sum
-  dh::ExpertProduct routed_down = routed_product(spec, p, T, false), own_down = shared_product(spec, T, ld_x, false);
+  // down products: together, the shared expert's waits in the workspace until the routed ones' sum has reached x
+  dh::ExpertProduct routed_down = routed_product(spec, p, T, false), own_down = shared_product(spec, p, T, false);
   routed_down.A = w + p.act; routed_down.W = down; routed_down.out = f32(p.y); routed_down.rows.tiles = i32(p.tiles); routed_down.rows.group_off = i32(p.off);
-  own_down.A = w + p.shared_act; own_down.W = shared_down; own_down.out = d_x; own_down.col_scale = spec->d_layer_scale; own_down.residual = d_x;
+  own_down.A = w + p.shared_act; own_down.W = shared_down; own_down.out = f32(p.shared_y);
   if (down_pair) {
     if (int rc = shared_gate_up()) return rc;
     if (int rc = dh::experts_pair(op, routed_down, own_down, false)) return rc;
@@ -545,7 +552,7 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
     if (int rc = dh::experts_down(op, routed_down.rows, w + p.act, operand, spec->ff, down, spec->ff, spec->hidden, spec->ff, f32(p.y), p.ld_y)) return rc;
   }
   hipLaunchKernelGGL(experts_combine_kernel, dim3(T, (unsigned)dh::ceil_div(spec->hidden, 1024)), dim3(256), 0, dh::stream(), f32(p.y), (int64_t)p.ld_y,
-                     i32(p.slot), spec->top, spec->d_layer_scale, d_x, (int64_t)ld_x, spec->hidden);
+                     i32(p.slot), spec->top, down_pair ? f32(p.shared_y) : nullptr, spec->d_layer_scale, d_x, (int64_t)ld_x, spec->hidden);
   DH_CHECK_LAUNCH(op);
   if (shared && !down_pair) {
     if (int rc = shared_gate_up()) return rc;

@@ -582,6 +582,36 @@ def test_shared_and_routed_products(L, T, K, E, top, ff, shared_ff, form):
     assert ((got - want).abs() <= 2.0 ** -8 * size * ls.double().abs() + 2.0 ** -22 * x.double().abs()).all()
 
 
+@pytest.mark.parametrize("K,E,top,ff,shared_ff,together,apart", [(1024, 5, 2, 512, 1024, (1300, 128, 1, 1), (1000, 128, 0, 0)),
+                                                                (1024, 5, 2, 512, 1024, (200, 64, 1, 1), (1000, 128, 0, 0)),
+                                                                (1024, 16, 2, 768, 3072, (700, 64, 1, 1), (1000, 128, 1, 0)),
+                                                                (256, 8, 2, 64, 128, (500, 128, 0, 1), (300, 64, 1, 1))])
+def test_products_that_share_a_launch_give_the_bits_of_those_apart(L, K, E, top, ff, shared_ff, together, apart):
+    """A token has the same bits in portions of either form, where no product is cut into k slices and the router's alike."""
+    (T, *form), (rows, *other) = together, apart
+    g = torch.Generator(device="cuda").manual_seed(T + rows)
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    n = max(T, rows)
+    h, x0, ls = torch.randn(n, K, generator=g, device="cuda").to(torch.bfloat16), torch.randn(n, K, generator=g, device="cuda"), torch.randn(K, generator=g, device="cuda")
+    router, up, down, s_up, s_down, norm = w(E + 1, K), w(E, 2 * ff, K), w(E, K, ff), w(2 * shared_ff, K), w(K, shared_ff), torch.ones(K, device="cuda")
+    spec = capi.Experts(K, K, E, top, ff, shared_ff, 1e-5, 7.0, 1.5, norm.data_ptr(), ls.data_ptr(), *(a.data_ptr() for a in (router, up, down, s_up, s_down)))
+    took = (ctypes.c_int64 * 3)()
+    slices = lambda M, N, K: capi.check(L.dh_dense_matmul_layout(M, N, K, capi.BF16, 0, 0, took)) or took[2]
+    assert slices(T, K, shared_ff) == slices(rows, K, shared_ff) == 1 and slices(T, E + 1, K) == slices(rows, E + 1, K)
+
+    def run(T, form):
+        capi.check(L.dh_experts_prefill_layout(ctypes.byref(spec), capi.BF16, T, 0, took))
+        assert list(took) == form
+        x, ws = x0[:T].clone(), torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T), dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_experts_prefill(ctypes.byref(spec), h.data_ptr(), capi.BF16, x.data_ptr(), K, ws.data_ptr(), T))
+        capi.check(L.dh_sync())
+        return x
+    a, b = run(T, form), run(rows, other)
+    both = min(T, rows)
+    assert torch.equal(a[:both], b[:both]) and not torch.equal(a, x0[:T])
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

@@ -280,6 +280,47 @@ def test_no_fetch_in_flight_at_the_end(assembly, src):
     assert fetches > 0 and hits == []
 
 
+def between_counted_waits(path, kernel):
+    """{(count waited for, next count waited for): {(fetches, then stores, mixed) between}} over all paths from one hand-written wait at a barrier to
+    the next in a kernel whose name holds `kernel`.  A wait that counts is right only while nothing between the two is merged, dropped or moved."""
+    ins = [t for t in _instructions(path)]
+    label_at = {s[:-1]: i for i, (_, s, _, _) in enumerate(ins) if s.endswith(":")}
+    wait = lambda i: _vmcnt(ins[i][1]) if i < len(ins) and ins[i][2] and ins[i][1].startswith("s_waitcnt") else None
+    found = {}
+    for start in [i for i in range(len(ins)) if kernel in (ins[i][3] or "") and wait(i) is not None]:
+        seen, work = set(), [(start + 1, 0, 0, False)]
+        while work:
+            i, fetches, stores, mixed = at = work.pop()
+            if at in seen or i >= len(ins):
+                continue
+            seen.add(at)
+            _, s, in_asm, _ = ins[i]
+            if wait(i) is not None:
+                found.setdefault((wait(start), wait(i)), set()).add((fetches, stores, mixed))
+                continue
+            if s.startswith("s_endpgm"):
+                continue
+            if _is_fetch(s, in_asm):
+                fetches, mixed = min(fetches + 1, 99), mixed or stores > 0
+            elif s.startswith(("global_store", "flat_store", "buffer_store")):
+                stores = min(stores + 1, 99)
+            if s.startswith(("s_branch", "s_cbranch")):
+                work.append((label_at[s.split()[-1]], fetches, stores, mixed))
+            if not s.startswith("s_branch"):
+                work.append((i + 1, fetches, stores, mixed))
+    return found
+
+
+@pytest.mark.parametrize("rows,fetches", [(64, 4), (32, 5)])
+def test_memory_walks_have_the_fetches_and_stores_that_their_waits_count(assembly, rows, fetches):
+    """In front of the loop three chunks are fetched; a chunk fetches another and then stores the four rows of a lane's state."""
+    found = between_counted_waits(assembly["matrix_memory.hip"], "mlstm_states_kernelILi%dE" % rows)
+    begin, steps = 2 * fetches, {fetches, fetches + 4, fetches + 8}
+    assert steps <= {b for _, b in found} and {a for a, _ in found} <= steps | {begin}
+    for (a, b), between in found.items():
+        assert between <= {(fetches, 4, False)} | ({(0, 0, False)} if a == begin else set()), (a, b, between)
+
+
 def test_the_scans_see_what_they_look_for(tmp_path):
     """The assembly of the build that faulted, reduced to the lines that matter, and a register reuse."""
     bad = tmp_path / "bad.s"
@@ -303,3 +344,8 @@ def test_the_scans_see_what_they_look_for(tmp_path):
     assert len(foreign_m0(str(loop))) == 1 and len(spills_in_fetching_loops(str(loop))[0]) == 1 and len(ends_with_fetches_in_flight(str(loop))[0]) == 1
     loop.write_text("kernel_b:\n.LBB0_1:\n" + fetch + "\ts_cbranch_scc1 .LBB0_1\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier\n\tscratch_load_dword v2, off, off\n\ts_endpgm\n")
     assert foreign_m0(str(loop)) == [] and spills_in_fetching_loops(str(loop)) == ([], 1) and ends_with_fetches_in_flight(str(loop)) == ([], 1)
+    wait = "\t;;#ASMSTART\n\ts_waitcnt vmcnt(%d) lgkmcnt(0)\n\ts_barrier\n\t;;#ASMEND\n"
+    loop.write_text("kernel_c:\n" + wait % 2 + ".LBB0_1:\n" + wait % 5 + fetch + "%s\tglobal_store_dword v[2:3], v1, off\n%s\ts_cbranch_scc1 .LBB0_1\n" % ("", "") + wait % 0 + "\ts_endpgm\n")
+    assert between_counted_waits(str(loop), "kernel_c") == {(2, 5): {(0, 0, False)}, (5, 5): {(1, 1, False)}, (5, 0): {(1, 1, False)}}
+    loop.write_text(loop.read_text().replace(fetch, "\ts_cbranch_scc0 .LBB0_2\n\tglobal_store_dword v[4:5], v1, off\n.LBB0_2:\n" + fetch))
+    assert between_counted_waits(str(loop), "kernel_c")[5, 5] == {(1, 1, False), (1, 2, True)}

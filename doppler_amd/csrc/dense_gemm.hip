@@ -500,7 +500,7 @@ constexpr TileCost kTiles[] = {{256, 256, 1, 993.f, 1464.f, 1627.f, 8987.f, 8447
                                {256, 128, 1, 457.f, 808.f, 899.f, 11078.f, 4801.f},
                                {128, 128, 2, 396.f, 619.f, 1337.f, 5092.f, 2173.f},
                                {64, 64, 2, 163.f, 294.f, 498.f, 5060.f, 803.f}};
-// gate and up products, never sliced
+// gate and up products, never sliced (costs of tiles that did not ask for their weights ahead, not fitted again since)
 constexpr TileCost kGluTiles[] = {{256, 256, 1, 900.f, 1720.f, 1720.f, 8000.f, 0.f},
                                   {256, 128, 1, 520.f, 930.f, 930.f, 5500.f, 0.f},
                                   {128, 128, 2, 330.f, 480.f, 1080.f, 4500.f, 0.f},
@@ -787,7 +787,8 @@ GemmArgs expert_args(const dh::ExpertProduct& p, bool glu) {
 
 namespace dh {
 
-// One launch where neither product is small beside the other and the shared one loses little on the routed ones' tiles.  Each fills one to
+// One launch where neither product is small beside the other and the shared one loses little on the routed ones' tiles (what the shared last round
+// gains is not weighed against that loss).  Each fills one to
 // two rounds of workgroups and leaves most of its last round empty, together they leave one: apart and together, us, the gate and up products and
 // the down products of prompts of 2000 rows of 1024: 25.7 + 22.1 to 45.1, 24.9 + 17.0 to 31.1; 1531 of 2048: 65.6 + 52.2 to 102, 48.2 + 31.5 to
 // 68.6; 900 of 4096: 130 + 105 to 220, 92 + 50 to 143.

@@ -22,8 +22,8 @@
 //                          element by element and in place
 //   mlstm_outputs_kernel   o of (chunk, head, value columns): Q K^T and Q S in one walk over dim, decay mask, then (Q K^T) V
 //
-// on the 32-bit matrix-core instruction v_mfma_f32_32x32x2_f32.  head_norm_gate_kernel then divides every head's output by its root
-// mean square and applies the weight and the output gate.
+// on the 32-bit matrix-core instructions v_mfma_f32_32x32x2_f32 and, in the walk, v_mfma_f32_16x16x4_f32 (which add in the same order).
+// head_norm_gate_kernel then divides every head's output by its root mean square and applies the weight and the output gate.
 #include <algorithm>
 #include <cfloat>
 
@@ -66,7 +66,7 @@ __device__ __forceinline__ float log_forget_gate(const MemArgs& a, float z) {
   return fminf(t, 0.f) - log1pf(expf(-fabsf(t)));
 }
 
-// Eight lanes x four columns, 32 rows at a time.  Four heads of 128 x 256: 5.3 -> 4.0 us with everything requested in front of the gates.
+// Eight lanes x four columns, 32 rows at a time.  Four heads of 128 x 256: 5.3 -> 4.0 us with what 128 rows need requested in front of the gates.
 __global__ __launch_bounds__(256) void mlstm_step_kernel(const MemArgs a) {
   __shared__ float red[4];
   __shared__ float4 o_lds[4][8];
@@ -76,7 +76,8 @@ __global__ __launch_bounds__(256) void mlstm_step_kernel(const MemArgs a) {
   const int from = pos & 1, to = from ^ 1;
   const float* q = a.rows + (int64_t)h * a.DP;
   const float* k = a.rows + a.k_off + (int64_t)h * a.DP;
-  // everything the step reads is requested before anything is computed from it (rows of the state four at a time): one trip to memory
+  // what the first four rows of a thread need is requested before anything is computed from it: one trip to memory up to 128 rows (a longer state's
+  // next four are requested behind the stores of these)
   constexpr int BATCH = 4;
   float* S = a.S + (int64_t)h * a.DP * a.VP + col;
   const float* n_old = a.n + ((int64_t)from * a.H + h) * a.DP;
@@ -298,10 +299,10 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const MemArgs a) {
 
 // The states in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T, in one walk.
 //
-// One workgroup of eight waves for 64 x 32 of a head's state, a head's tiles on one die.  Wave w holds rows 16 (w >> 1), columns 16 (w & 1) in
-// registers, adds up a chunk's products apart from it (16 of v_mfma_f32_16x16x4_f32: with 32 x 32 tiles half of the SIMDs would have none) and
-// writes the state in front of every chunk once.  Keys, values and weights go straight into three buffers of LDS, two chunks ahead, by waits that count:
-// through registers the compiler waited for the youngest load and store at every chunk (2.3 us each).  Four tokens make an instruction, so their
+// One workgroup of eight (four) waves for 64 x 32 (32 x 32) of a head's state, a head's tiles on one die.  Wave w holds rows 16 (w >> 1), columns
+// 16 (w & 1) in registers, adds up a chunk's products apart from it (16 of v_mfma_f32_16x16x4_f32: of 32 x 32 for a wave half of the SIMDs would have
+// none) and writes the state in front of every chunk once.  Keys, values and weights go straight into three buffers of LDS, two chunks ahead of the one
+// being read, by waits that count: through registers the compiler waited for the youngest load and store at every chunk (2.3 us each).  Four tokens make an instruction, so their
 // rows' 16-byte pieces are kept apart by 16 banks (slot = piece ^ 4 (token & 3) of 16, piece ^ 4 (token / 2 & 1) of 8).
 // The workgroups behind the tiles walk the normaliser.
 // us, against a launch for what every chunk adds (to memory and back) and another for the scan: four heads of 256 x 512, 1500 tokens 37.7 + 18.1 -> 33, eight, 1000

@@ -71,6 +71,7 @@ __device__ __forceinline__ void put_c2(const GemmArgs& a, int64_t at, float v) {
 struct PutTerms {
   float bias, scale, residual;
 };
+__device__ __forceinline__ bool has_terms(const GemmArgs& a) { return a.bias || a.col_scale || a.residual; }
 __device__ __forceinline__ PutTerms put_terms(const GemmArgs& a, int m, int n) {
   PutTerms t{0.f, 1.f, 0.f};
   if (n < a.n_first) {
@@ -86,9 +87,8 @@ __device__ __forceinline__ float first_output(const GemmArgs& a, const PutTerms&
   if (a.residual) v += t.residual;
   return v;
 }
-__device__ __forceinline__ void put(const GemmArgs& a, const PutTerms& t, int m, int n, float acc) {
-  if (n < a.n_first) a.C[(int64_t)m * a.ldc + n] = first_output(a, t, acc);
-  else put_c2(a, (int64_t)m * a.ldc2 + (n - a.n_first), dh::activate(acc * a.alpha, a.act));
+__device__ __forceinline__ void put_second(const GemmArgs& a, int m, int n, float acc) {
+  put_c2(a, (int64_t)m * a.ldc2 + (n - a.n_first), dh::activate(acc * a.alpha, a.act));
 }
 
 // Where a workgroup's tile lies: its rows (base + 0 .. rows - 1 of the outputs), its first row among them, its weights.
@@ -122,18 +122,18 @@ __device__ __forceinline__ int64_t source_row(const GemmArgs& a, const TilePlace
 // values before it stores them: a load behind a store waits for the store's trip to memory as well, and values between the branches of
 // ragged rows are computed one after the other.  Sixteen round trips for a tile of gated pairs took 18 us of 68 (1531 x 6144 x 2048).
 // A small product waits for every instruction of it, so kernels with and without a residual are two, addresses are a multiplication of 32
-// bits a row, and fours of rows that a tile does not have are left out (us, one form and sixteen rows for all -> now: 40 x 1024 x 1024 6.96 -> 6.6,
-// 4 x 119 x 192 with the exact gelu 4.36 -> 3.65, 500 x 500 x 448 with a residual 5.36 -> 5.3).
+// bits a row, fours of rows that a tile does not have are left out, raw sums of k slices are one kernel's, and first and second outputs follow one
+// another: settled at every value, each steps over the other's code (us, one form and sixteen rows for all -> now: 40 x 1024 x 1024 6.96 -> 6.6, 4 x 119 x 192
+// with the exact gelu 4.36 -> 3.65, 500 x 500 x 448 with a residual 5.36 -> 5.3, 996 x 3600 x 1472 with both outputs 34.1 -> 27.5).
 __device__ __forceinline__ int tile_row(int mb, int i) { return mb + 8 * (i >> 2) + (i & 3); }
 
 struct ColumnTerms {       // of one column of the first output
   float alpha, bias;
 };
 __device__ __forceinline__ ColumnTerms column_terms(const GemmArgs& a, int n0, int lane) {
-  const int n = n0 + (lane & 31);
-  const bool here = n < a.n_first;
-  const float scale = here && a.col_scale ? a.col_scale[n] : 1.f;
-  return {a.alpha * scale, (here && a.bias ? a.bias[n] : 0.f) * scale};
+  const int n = min(n0 + (lane & 31), a.n_first - 1);
+  const float bias = a.bias ? a.bias[n] : 0.f, scale = a.col_scale ? a.col_scale[n] : 1.f;
+  return {a.alpha * scale, bias * scale};
 }
 // (every read in front of the first write, also because the residual may be the output itself)
 __device__ __forceinline__ void load_residual(const GemmArgs& a, const TilePlace& p, float (&r)[16], int m0, int n0, int lane) {
@@ -164,33 +164,34 @@ __device__ __forceinline__ void store_c2(const GemmArgs& a, int64_t at, int mb, 
   else if (a.c2_dtype == DH_F16) store_rows(static_cast<_Float16*>(a.C2) + at, a.ldc2, mb, rows, [&](int i) { return (_Float16)v[i]; });
   else store_rows(static_cast<float*>(a.C2) + at, a.ldc2, mb, rows, [&](int i) { return v[i]; });
 }
-template <int ACT, class Flag>
-__device__ __forceinline__ void store_tile(const GemmArgs& a, const TilePlace& p, const f32x16_t& acc, const ColumnTerms& col, Flag with_residual,
-                                           const float (&r)[16], int m0, int n0, int lane) {
-  const int n = n0 + (lane & 31);
-  if (n >= a.N) return;
-  const int mb = m0 + 4 * (lane >> 5);
-  if (a.parts) {
-    store_rows(a.parts + (int64_t)blockIdx.y * a.M * a.N + n, a.N, mb, a.M, [&](int i) { return acc[i]; });
-  } else if (only_first(ACT) || n < a.n_first) {
-    float* c = a.C + (int64_t)p.base * a.ldc + n;
-    if (with_residual) store_rows(c, a.ldc, mb, p.rows, [&](int i) { return fmaf(acc[i], col.alpha, col.bias) + r[i]; });
-    else store_rows(c, a.ldc, mb, p.rows, [&](int i) { return fmaf(acc[i], col.alpha, col.bias); });
-  } else if constexpr (ACT == kAnyAct) {      // (one value at a time: sixteen of each activation are too much code)
-    const int64_t at = (int64_t)p.base * a.ldc2 + (n - a.n_first);
+template <class Flag>
+__device__ __forceinline__ void store_first(const GemmArgs& a, const TilePlace& p, const f32x16_t& acc, const ColumnTerms& col, Flag with_residual,
+                                            const float (&r)[16], int m0, int n0, int lane) {
+  const int n = n0 + (lane & 31), mb = m0 + 4 * (lane >> 5);
+  if (n >= a.n_first) return;
+  float* c = a.C + (int64_t)p.base * a.ldc + n;
+  if (with_residual) store_rows(c, a.ldc, mb, p.rows, [&](int i) { return fmaf(acc[i], col.alpha, col.bias) + r[i]; });
+  else store_rows(c, a.ldc, mb, p.rows, [&](int i) { return fmaf(acc[i], col.alpha, col.bias); });
+}
+template <int ACT, bool FEW>
+__device__ __forceinline__ void store_second(const GemmArgs& a, const TilePlace& p, const f32x16_t& acc, int m0, int n0, int lane) {
+  const int n = n0 + (lane & 31), mb = m0 + 4 * (lane >> 5);
+  if (n < a.n_first || n >= a.N) return;
+  const int64_t at = (int64_t)p.base * a.ldc2 + (n - a.n_first);
+  if (ACT == kAnyAct || (FEW && m0 + 8 >= p.rows)) {      // one value at a time: sixteen of each activation are too much code, and few rows have few values
 #pragma unroll
     for (int i = 0; i < 16; i++) {
       const int m = tile_row(mb, i);
-      if (m < p.rows) put_c2(a, at + (int64_t)m * a.ldc2, dh::activate(acc[i] * a.alpha, a.act));
+      if (m < p.rows) put_c2(a, at + (int64_t)m * a.ldc2, dh::activate(acc[i] * a.alpha, ACT == kAnyAct ? a.act : ACT));
     }
   } else {
     float v[16];
     by_fours(m0, p.rows, [&](int i) { v[i] = dh::activate(acc[i] * a.alpha, ACT); });
-    store_c2(a, (int64_t)p.base * a.ldc2 + (n - a.n_first), mb, p.rows, v);
+    store_c2(a, at, mb, p.rows, v);
   }
 }
-// Tiles AT .. of a wave's R x C; residuals of four tiles at a time.
-template <int ACT, int AT, int R, int C, class Flag>
+// First outputs of tiles AT .. of a wave's R x C; residuals of four tiles at a time.
+template <int AT, int R, int C, class Flag>
 __device__ __forceinline__ void store_from(const GemmArgs& a, const TilePlace& p, const f32x16_t (&acc)[R][C], const ColumnTerms (&col)[C],
                                            Flag with_residual, int m0, int n0, int lane) {
   constexpr int kBatch = R * C < 4 ? R * C : 4;
@@ -201,22 +202,33 @@ __device__ __forceinline__ void store_from(const GemmArgs& a, const TilePlace& p
   }
 #pragma unroll
   for (int u = 0; u < kBatch; u++)
-    store_tile<ACT>(a, p, acc[(AT + u) / C][(AT + u) % C], col[(AT + u) % C], with_residual, r[u], m0 + 32 * ((AT + u) / C), n0 + 32 * ((AT + u) % C), lane);
-  if constexpr (AT + kBatch < R * C) store_from<ACT, AT + kBatch>(a, p, acc, col, with_residual, m0, n0, lane);
+    store_first(a, p, acc[(AT + u) / C][(AT + u) % C], col[(AT + u) % C], with_residual, r[u], m0 + 32 * ((AT + u) / C), n0 + 32 * ((AT + u) % C), lane);
+  if constexpr (AT + kBatch < R * C) store_from<AT + kBatch>(a, p, acc, col, with_residual, m0, n0, lane);
 }
-template <int ACT, int R, int C>
+// A wave's tiles: raw sums of a k slice (kernels that are launched with slices), or first outputs and then second ones.
+template <int ACT, bool SLICES, int R, int C>
 __device__ __forceinline__ void store_tiles(const GemmArgs& a, const TilePlace& p, const f32x16_t (&acc)[R][C], int m0, int n0, int lane) {
-  ColumnTerms col[C];
+  if (SLICES && a.parts) {
 #pragma unroll
-  for (int j = 0; j < C; j++) col[j] = column_terms(a, n0 + 32 * j, lane);
-  if constexpr (only_first(ACT)) {
-    if constexpr (ACT == kResidual && R * C > 4) store_from<ACT, 0>(a, p, acc, col, a.residual != nullptr, m0, n0, lane);    // (known, registers are spilled here)
-    else store_from<ACT, 0>(a, p, acc, col, std::bool_constant<ACT == kResidual>{}, m0, n0, lane);
-  } else {
-    const bool with_residual = a.residual && !a.parts && n0 < a.n_first;
-    if constexpr (R * C > 4) store_from<ACT, 0>(a, p, acc, col, with_residual, m0, n0, lane);    // (two copies spill registers here)
-    else if (with_residual) store_from<ACT, 0>(a, p, acc, col, std::true_type{}, m0, n0, lane);
-    else store_from<ACT, 0>(a, p, acc, col, std::false_type{}, m0, n0, lane);
+    for (int t = 0; t < R * C; t++) {
+      const int n = n0 + 32 * (t % C) + (lane & 31);
+      if (n < a.N) store_rows(a.parts + (int64_t)blockIdx.y * a.M * a.N + n, a.N, m0 + 32 * (t / C) + 4 * (lane >> 5), a.M, [&](int i) { return acc[t / C][t % C][i]; });
+    }
+    return;
+  }
+  if (n0 < a.n_first) {
+    ColumnTerms col[C];
+#pragma unroll
+    for (int j = 0; j < C; j++) col[j] = column_terms(a, n0 + 32 * j, lane);
+    if constexpr (ACT == kNoSecond) store_from<0>(a, p, acc, col, std::false_type{}, m0, n0, lane);
+    else if constexpr (R * C > 4) store_from<0>(a, p, acc, col, a.residual != nullptr, m0, n0, lane);    // (known, registers are spilled here)
+    else if (ACT == kResidual || a.residual) store_from<0>(a, p, acc, col, std::true_type{}, m0, n0, lane);
+    else store_from<0>(a, p, acc, col, std::false_type{}, m0, n0, lane);
+  }
+  if constexpr (!only_first(ACT)) {
+    if (n0 + 32 * C > a.n_first)
+#pragma unroll
+      for (int t = 0; t < R * C; t++) store_second<ACT, R * C == 1>(a, p, acc[t / C][t % C], m0 + 32 * (t / C), n0 + 32 * (t % C), lane);
   }
 }
 // The same for R gate tiles and the up tiles beside them (first weight row n0 of the gate block).
@@ -269,13 +281,13 @@ __device__ __forceinline__ void gemm_16bit(const GemmArgs& a, int block, char* s
     dh::small_product<Tile, F16>(acc[0], a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
     const int m = m0 + 32 * wm, n = n0 + 32 * Tile::G * wn;
     if constexpr (GLU) store_glu(a, place, acc, m, n, lane);
-    else store_tiles<ACT>(a, place, acc, m, n, lane);
+    else store_tiles<ACT, ACT == kNoSecond && !GROUPED>(a, place, acc, m, n, lane);
   } else {
     f32x16_t acc[2 * Tile::FA][2 * Tile::FB];
     dh::wide_product<Tile, F16>(acc, a_base, a_off, w_base, w_off, 2u * k0, nk, smem, company);
     const int m = m0 + 64 * Tile::FA * wm, n = n0 + 64 * Tile::FB * wn;
     if constexpr (GLU) store_glu(a, place, acc, m, n, lane);
-    else store_tiles<ACT>(a, place, acc, m, n, lane);
+    else store_tiles<ACT, ACT == kNoSecond && !GROUPED>(a, place, acc, m, n, lane);
   }
 }
 
@@ -368,7 +380,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmArgs a) {
     __syncthreads();
   }
   if constexpr (GLU) store_glu(a, place, acc, m0 + 32 * wm, n0 + 32 * wn * TN, lane);
-  else store_tiles<kAnyAct>(a, place, acc, m0 + 32 * wm, n0 + 32 * wn * TN, lane);
+  else store_tiles<kAnyAct, !GROUPED>(a, place, acc, m0 + 32 * wm, n0 + 32 * wn * TN, lane);
 }
 
 // 32-bit products of rows within reach (gemm_split.h).  Bound by the matrix cores where tiles are many (at 600 x 18464 x 4096 the three
@@ -407,29 +419,39 @@ __global__ __launch_bounds__(Tile::kThreads, Tile::kPerSimd) void gemm_split_ker
     }
   }
   const int lane = threadIdx.x & 63;
-  PutTerms terms[Tile::kShare][4];
-  if (!a.parts) {
+  // (which output a tile has is settled in front of the loops over its sums: stepping over the other's code at each of them took 0.7 us)
+  auto each = [&](auto&& f) {
 #pragma unroll
     for (int u = 0; u < Tile::kShare; u++) {
       const dh::SumPlace<Tile> at(u);
-      const int n = n0 + 32 * at.j + (lane & 31), row = 32 * at.wm + 8 * at.q + 4 * (lane >> 5);
+      const int n = n0 + 32 * at.j + (lane & 31), m = m0 + 32 * at.wm + 8 * at.q + 4 * (lane >> 5);
 #pragma unroll
-      for (int e = 0; e < 4; e++) terms[u][e] = put_terms(a, min(m0 + row + e, a.M - 1), n);
+      for (int e = 0; e < 4; e++) f(u, e, m + e, n);
+    }
+  };
+  if (a.parts) {
+    each([&](int u, int e, int m, int n) {
+      if (m < a.M && n < a.N) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = sums[u][e];
+    });
+    return;
+  }
+  if (n0 < a.n_first) {
+    if (has_terms(a)) {
+      PutTerms terms[Tile::kShare][4];
+      each([&](int u, int e, int m, int n) { terms[u][e] = put_terms(a, min(m, a.M - 1), n); });
+      each([&](int u, int e, int m, int n) {
+        if (m < a.M && n < a.n_first) a.C[(int64_t)m * a.ldc + n] = first_output(a, terms[u][e], sums[u][e]);
+      });
+    } else {
+      each([&](int u, int e, int m, int n) {
+        if (m < a.M && n < a.n_first) a.C[(int64_t)m * a.ldc + n] = fmaf(sums[u][e], a.alpha, 0.f);
+      });
     }
   }
-#pragma unroll
-  for (int u = 0; u < Tile::kShare; u++) {
-    const dh::SumPlace<Tile> at(u);
-    const int n = n0 + 32 * at.j + (lane & 31), row = 32 * at.wm + 8 * at.q + 4 * (lane >> 5);
-    if (n >= a.N) continue;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int m = m0 + row + e;
-      if (m >= a.M) break;
-      if (a.parts) a.parts[((int64_t)blockIdx.y * a.M + m) * a.N + n] = sums[u][e];
-      else put(a, terms[u][e], m, n, sums[u][e]);
-    }
-  }
+  if (n0 + Tile::BN > a.n_first)
+    each([&](int u, int e, int m, int n) {
+      if (m < a.M && n >= a.n_first && n < a.N) put_second(a, m, n, sums[u][e]);
+    });
 }
 
 // Sums of the k slices in slice order.  VEC columns per thread (N a multiple of VEC), a block's threads as wide as the row allows and the
@@ -444,9 +466,10 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
     float s[VEC] = {};
     PutTerms terms[VEC];
     const bool whole = VEC == 4 && n + 3 < a.n_first && a.ldc % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.residual)) & 15) == 0;
-    f32x4_t residual = {0.f, 0.f, 0.f, 0.f};
-    if (whole && a.residual) residual = *reinterpret_cast<const f32x4_t*>(a.residual + (int64_t)m * a.ldc + n);
-    if (n < a.n_first) {
+    const bool with_terms = has_terms(a) && n < a.n_first;
+    if (with_terms) {
+      f32x4_t residual = {0.f, 0.f, 0.f, 0.f};
+      if (whole && a.residual) residual = *reinterpret_cast<const f32x4_t*>(a.residual + (int64_t)m * a.ldc + n);
 #pragma unroll
       for (int e = 0; e < VEC; e++) {
         if (whole) terms[e] = PutTerms{a.bias ? a.bias[n + e] : 0.f, a.col_scale ? a.col_scale[n + e] : 1.f, residual[e]};
@@ -463,17 +486,17 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
         s[0] += p[k * total];
       }
     }
+    float v[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; e++) v[e] = with_terms ? first_output(a, terms[e], s[e]) : fmaf(s[e], a.alpha, 0.f);
     if (whole) {
-      f32x4_t v;
-#pragma unroll
-      for (int e = 0; e < VEC; e++) v[e] = first_output(a, terms[e], s[e]);
-      *reinterpret_cast<f32x4_t*>(a.C + (int64_t)m * a.ldc + n) = v;
-    } else if (n >= a.n_first) {
-#pragma unroll
-      for (int e = 0; e < VEC; e++) put_c2(a, (int64_t)m * a.ldc2 + (n + e - a.n_first), dh::activate(s[e] * a.alpha, a.act));
+      *reinterpret_cast<f32x4_t*>(a.C + (int64_t)m * a.ldc + n) = f32x4_t{v[0], v[VEC > 1 ? 1 : 0], v[VEC > 2 ? 2 : 0], v[VEC > 3 ? 3 : 0]};
     } else {
 #pragma unroll
-      for (int e = 0; e < VEC; e++) put(a, terms[e], m, n + e, s[e]);
+      for (int e = 0; e < VEC; e++) {
+        if (n + e < a.n_first) a.C[(int64_t)m * a.ldc + n + e] = v[e];
+        else put_second(a, m, n + e, s[e]);
+      }
     }
   }
 }
@@ -547,6 +570,9 @@ TileChoice choose_tile(int64_t M, int64_t N, int64_t K, int most_slices, bool gl
 // A tile's rows are addressed by 32-bit byte offsets from its first (rows millions of elements long are out of reach; a single row never is).
 bool within_reach(int64_t rows, int64_t ld, int64_t K) { return 2 * ((std::min<int64_t>(rows, 256) - 1) * ld + K) < (int64_t)1 << 32; }
 
+// k of a slice (whole steps of 64).
+int slice_extent(int64_t K, int slices) { return (int)dh::ceil_div(K / 64, slices) * 64; }
+
 // LDS beyond 64 KB is asked for once per kernel.
 template <class Tile, bool F16, int ACT, bool GROUPED, bool GLU>
 int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
@@ -595,11 +621,13 @@ int launch_16bit(const char* op, GemmArgs a, const TileChoice& pick) {
   return launch_reduce(op, a, slices);
 }
 int launch_act(const char* op, const GemmArgs& a, bool f16, const TileChoice& pick) {
-  const bool residual = a.residual && pick.slices == 1;       // (behind slices it is the reduce launch's)
-  if (f16) return a.n_first == a.N ? residual ? launch_16bit<true, kResidual, false>(op, a, pick) : launch_16bit<true, kNoSecond, false>(op, a, pick)
+  // (behind slices terms and second outputs are the reduce launch's)
+  if (a.K > slice_extent(a.K, pick.slices) || (a.n_first == a.N && !a.residual))
+    return f16 ? launch_16bit<true, kNoSecond, false>(op, a, pick) : launch_16bit<false, kNoSecond, false>(op, a, pick);
+  if (f16) return a.n_first == a.N ? launch_16bit<true, kResidual, false>(op, a, pick)
                   : a.act == DH_ACT_NONE ? launch_16bit<true, DH_ACT_NONE, false>(op, a, pick)
                                          : launch_16bit<true, kAnyAct, false>(op, a, pick);
-  if (a.n_first == a.N) return residual ? launch_16bit<false, kResidual, false>(op, a, pick) : launch_16bit<false, kNoSecond, false>(op, a, pick);
+  if (a.n_first == a.N) return launch_16bit<false, kResidual, false>(op, a, pick);
   if (a.act == DH_ACT_RELU2) return launch_16bit<false, DH_ACT_RELU2, false>(op, a, pick);
   if (a.act == DH_ACT_GELU_ERF) return launch_16bit<false, DH_ACT_GELU_ERF, false>(op, a, pick);
   return launch_16bit<false, kAnyAct, false>(op, a, pick);
@@ -700,8 +728,6 @@ int choose_register_slices(int64_t M, int64_t N, int64_t K) {
   }
   return slices;
 }
-// k of a slice (whole steps of 64).
-int slice_extent(int64_t K, int slices) { return (int)dh::ceil_div(K / 64, slices) * 64; }
 
 template <class Tile>
 int launch_split(const char* op, GemmArgs a, int slices) {

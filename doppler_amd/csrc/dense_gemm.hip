@@ -814,10 +814,10 @@ GemmArgs expert_args(const dh::ExpertProduct& p, bool glu) {
 namespace dh {
 
 // One launch where neither product is small beside the other and the shared one loses little on the routed ones' tiles (what the shared last round
-// gains is not weighed against that loss).  Each fills one to
-// two rounds of workgroups and leaves most of its last round empty, together they leave one: apart and together, us, the gate and up products and
-// the down products of prompts of 2000 rows of 1024: 25.7 + 22.1 to 45.1, 24.9 + 17.0 to 31.1; 1531 of 2048: 65.6 + 52.2 to 102, 48.2 + 31.5 to
-// 68.6; 900 of 4096: 130 + 105 to 220, 92 + 50 to 143.
+// gains is not weighed against that loss).  Each fills one to two rounds of workgroups and leaves most of its last round empty, together they leave one:
+// apart and together, us, the gate and up products and the down products of prompts of 2000 rows of 1024: 25.7 + 22.1 to 45.1, 24.9 + 17.0 to 31.1; 1531 of
+// 2048: 65.6 + 52.2 to 102, 48.2 + 31.5 to 66 (and 1 more in the launch that sums); 900 of 4096: 130 + 105 to 220, 92 + 50 to 143.  Whole layers of experts, widths
+// 1024 to 4096, 2 to 2047 rows, by this rule against all apart on tiles that did not ask for their weights ahead: 0.99 to 1.41 times as fast.
 bool experts_together(const ExpertProduct& routed, const ExpertProduct& shared, bool glu) {
   const int at = routed.rows.tile_rows == Tile128x128::BM ? 2 : 3;
   const TileCost& c = glu ? kGluTiles[at] : kTiles[at];

@@ -13,19 +13,20 @@
 // exponents), m is known for every token from a max-plus scan, and a chunk's outputs are a product with the state before it plus a
 // masked product inside it:
 //
-//   mlstm_gates_kernel     F, i, m of every token; one workgroup per head
+//   mlstm_gates_kernel     F, i, m of every token, one workgroup per head; beside them every chunk's scores Q K^T
 //   mlstm_states_kernel    the state in front of every chunk, walking the chunks with a tile of it in registers; or, where few tiles would
 //                          walk far, in two launches:
 //   mlstm_chunks_kernel    what every chunk adds to the state behind it, sum_s e^(F_end - F_s + i_s - m_end) k_s v_s^T: independent of
 //                          one another, because m is known
 //   mlstm_scan_kernel      the state in front of every chunk, S_(c+1) = e^(F_end - F_start + m_start - m_end) S_c + what chunk c adds,
 //                          element by element and in place
-//   mlstm_outputs_kernel   o of (chunk, head, value columns): Q K^T and Q S in one walk over dim, decay mask, then (Q K^T) V
+//   mlstm_outputs_kernel   o of (chunk, head, value columns): Q S, decay and mask of the scores, then (Q K^T) V
 //
 // on the 32-bit matrix-core instructions v_mfma_f32_32x32x2_f32 and, in the walk, v_mfma_f32_16x16x4_f32 (which add in the same order).
 // head_norm_gate_kernel then divides every head's output by its root mean square and applies the weight and the output gate.
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 #include "gemm_wide.h"
 
@@ -56,6 +57,7 @@ struct MemArgs {
   float* mc;               // [H][chunks + 1] m in front of every chunk, and at the end
   float* keep;             // [H][chunks] what a chunk leaves of the state in front of it
   float* w;                // [H][chunks][64] weight of a token's key and value in the state behind its chunk, zero past the last; null: no walk
+  float* scores;           // [chunks][H][64][64] q . k of a chunk's tokens, not decayed; nothing past the diagonal's 16 x 16 tiles
   float* Sc;               // [chunks + 1][H][DP][VP]
   float* nc;               // [chunks + 1][H][DP]
 };
@@ -152,61 +154,171 @@ struct MaxPlus {
   double F, M;
 };
 __device__ __forceinline__ MaxPlus then(const MaxPlus& x, const MaxPlus& y) { return {x.F + y.F, fmax(x.M + y.F, y.M)}; }
+// Lane l's value becomes that of lanes 0 .. l one after the other (of LANES in a row).
+template <int LANES>
+__device__ __forceinline__ MaxPlus scan_lanes(MaxPlus v, int lane) {
+#pragma unroll
+  for (int off = 1; off < LANES; off <<= 1) {
+    const MaxPlus up = {__shfl_up(v.F, off, 64), __shfl_up(v.M, off, 64)};
+    if (lane >= off) v = then(up, v);
+  }
+  return v;
+}
 
-__global__ __launch_bounds__(1024) void mlstm_gates_kernel(const MemArgs a) {
-  __shared__ double sF[1024];
-  __shared__ double sM[1024];
-  const int tid = threadIdx.x, h = blockIdx.x;
+// One head's gates.  A thread takes a stretch of tokens, four of them at a time; up to four stay in its registers.
+constexpr int kHeldChunks = 1024;                      // chunks whose ends stay in LDS
+struct GatesLds {
+  MaxPlus stretches[16];
+  double F_end[kHeldChunks];                           // F of a chunk's last token
+  float m_front[kHeldChunks + 1];                      // m in front of it
+};
+__device__ __forceinline__ void head_gates(const MemArgs& a, int h, GatesLds& lds) {
+  constexpr int U = 4;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int per = (a.T + 1023) / 1024, t0 = min(tid * per, a.T), t1 = min(t0 + per, a.T);
   const float m_in = a.pos == 0 ? 0.f : a.m[(a.pos & 1) * a.H + h];
   double* F = a.F + (int64_t)h * a.T;
   float* li = a.i + (int64_t)h * a.T;
   float* mt = a.mt + (int64_t)h * a.T;
   float* mc = a.mc + (int64_t)h * (a.chunks + 1);
+  double f[U];                                         // of the four at hand: f, then F
+  float i[U];
   MaxPlus run = {0.0, -1e30};
-  for (int t = t0; t < t1; t++) {
-    const float* row = a.rows + (int64_t)t * a.ld_row;
-    const float f = log_forget_gate(a, row[a.f_off + h]), i = log_input_gate(a, row[a.i_off + h]);
-    run = then(run, {(double)f, (double)i});
-    F[t] = (double)f;                                   // becomes the running sum below
-    li[t] = i;
+  for (int t = t0; t < t1; t += U) {
+    float zf[U], zi[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (u >= per) break;                             // (a line of memory each)
+      const float* row = a.rows + (int64_t)min(t + u, a.T - 1) * a.ld_row;
+      zf[u] = row[a.f_off + h];
+      zi[u] = row[a.i_off + h];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (t + u >= t1) break;
+      f[u] = (double)log_forget_gate(a, zf[u]);
+      i[u] = log_input_gate(a, zi[u]);
+      run = then(run, {f[u], (double)i[u]});
+      if (per > U) F[t + u] = f[u];                    // becomes the running sum below
+      li[t + u] = i[u];
+    }
   }
-  sF[tid] = run.F;
-  sM[tid] = run.M;
+  // what lies in front of a thread's stretch: the waves before its own, and their lanes before its own
+  const MaxPlus upto = scan_lanes<64>(run, lane);
+  if (lane == 63) lds.stretches[wave] = upto;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {            // inclusive scan over the threads' stretches
-    MaxPlus mine = {sF[tid], sM[tid]};
-    if (tid >= off) mine = then({sF[tid - off], sM[tid - off]}, mine);
-    __syncthreads();
-    sF[tid] = mine.F;
-    sM[tid] = mine.M;
-    __syncthreads();
-  }
-  const MaxPlus before = tid > 0 ? MaxPlus{sF[tid - 1], sM[tid - 1]} : MaxPlus{0.0, -1e30};
+  const MaxPlus waves = scan_lanes<16>(lds.stretches[lane & 15], lane & 15);
+  MaxPlus before = {__shfl(waves.F, max(wave - 1, 0), 64), __shfl(waves.M, max(wave - 1, 0), 64)};
+  if (wave == 0) before = MaxPlus{0.0, -1e30};
+  const MaxPlus own = {__shfl_up(upto.F, 1, 64), __shfl_up(upto.M, 1, 64)};
+  if (lane > 0) before = then(before, own);
   double sum = before.F, m = fmax((double)m_in + before.F, before.M);
-  for (int t = t0; t < t1; t++) {
-    if (t % kChunk == 0) mc[t / kChunk] = (float)m;
-    const double f = F[t];
-    sum += f;
-    m = fmax(m + f, (double)li[t]);
-    F[t] = sum;
-    mt[t] = (float)m;
-    if (t == a.T - 1) {
-      mc[a.chunks] = (float)m;
-      a.m[((a.pos + a.T) & 1) * a.H + h] = (float)m;
+  auto front = [&](int c) {
+    mc[c] = (float)m;
+    if (c <= kHeldChunks) lds.m_front[c] = (float)m;
+  };
+  auto again = [&](int t) {                            // a longer stretch's next four
+    if (per > U)
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        f[u] = F[min(t + u, a.T - 1)];
+        i[u] = li[min(t + u, a.T - 1)];
+      }
+  };
+  for (int t = t0; t < t1; t += U) {
+    again(t);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (t + u >= t1) break;
+      if ((t + u) % kChunk == 0) front((t + u) / kChunk);
+      sum += f[u];
+      m = fmax(m + f[u], (double)i[u]);
+      f[u] = sum;
+      F[t + u] = sum;
+      mt[t + u] = (float)m;
+      const bool last = t + u == a.T - 1;
+      if ((last || (t + u) % kChunk == kChunk - 1) && (t + u) / kChunk < kHeldChunks) lds.F_end[(t + u) / kChunk] = sum;
+      if (last) {
+        front(a.chunks);
+        a.m[((a.pos + a.T) & 1) * a.H + h] = (float)m;
+      }
     }
   }
   __syncthreads();
-  for (int c = tid; c < a.chunks; c += 1024) {
-    const double start = c > 0 ? F[c * kChunk - 1] : 0.0, end = F[min((c + 1) * kChunk, a.T) - 1];
-    a.keep[(int64_t)h * a.chunks + c] = expf((float)(end - start + (double)mc[c] - (double)mc[c + 1]));
-  }
+  auto F_end = [&](int c) { return c < kHeldChunks ? lds.F_end[c] : F[min((c + 1) * kChunk, a.T) - 1]; };
+  auto m_front = [&](int c) { return (double)(c <= kHeldChunks ? lds.m_front[c] : mc[c]); };
+  for (int c = tid; c < a.chunks; c += 1024)
+    a.keep[(int64_t)h * a.chunks + c] = expf((float)(F_end(c) - (c > 0 ? F_end(c - 1) : 0.0) + m_front(c) - m_front(c + 1)));
   if (!a.w) return;
-  for (int t = tid; t < a.chunks * kChunk; t += 1024) {
-    const int c = t / kChunk, last = min((c + 1) * kChunk, a.T) - 1;
-    // in fours of tokens, a token of every four beside those of the others
-    a.w[((int64_t)h * a.chunks + c) * kChunk + 16 * (t & 3) + ((t & (kChunk - 1)) >> 2)] = t <= last ? expf((float)(F[last] - F[t] + (double)li[t] - (double)mc[c + 1])) : 0.f;
+  // in fours of tokens, a token of every four beside those of the others
+  auto put_weight = [&](int t, float w) { a.w[((int64_t)h * a.chunks + t / kChunk) * kChunk + 16 * (t & 3) + ((t & (kChunk - 1)) >> 2)] = w; };
+  for (int t = t0; t < t1; t += U) {
+    again(t);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (t + u >= t1) break;
+      const int c = (t + u) / kChunk;
+      put_weight(t + u, expf((float)(F_end(c) - f[u] + (double)i[u] - m_front(c + 1))));
+    }
   }
+  for (int t = a.T + tid; t < a.chunks * kChunk; t += 1024) put_weight(t, 0.f);
+}
+
+// The scores Q K^T of one (chunk, head), the 16 x 16 tiles up to the diagonal; a wave has one tile of them.
+constexpr int kScoreRow = 64 + 4;                      // floats of a row in LDS: sixteen rows' 16-byte pieces lie in different banks
+__device__ __forceinline__ void chunk_scores(const MemArgs& a, int item, float* lds) {
+  float *qs = lds, *ks = lds + kChunk * kScoreRow;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = item / a.H, h = item % a.H;
+  const int first = c * kChunk, x = 4 * (tid & 15), at = (tid >> 4) * kScoreRow + x;
+  const float* row = a.rows + (int64_t)(first + min(tid >> 4, a.T - first - 1)) * a.ld_row + (int64_t)h * a.DP;
+  constexpr int AHEAD = 4;                             // 64 dims each, requested together
+  f32x4_t q[AHEAD], k[AHEAD];
+  const int tr = wave < 1 ? 0 : wave < 3 ? 1 : wave < 6 ? 2 : 3, tc = wave - tr * (tr + 1) / 2;
+  f32x4_t p = {0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < a.DP; d += 64 * AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      const int du = min(d + 64 * u + x, a.DP - 4);
+      q[u] = *reinterpret_cast<const f32x4_t*>(row + du);
+      k[u] = *reinterpret_cast<const f32x4_t*>(row + a.k_off + du);
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      const int d0 = d + 64 * u;
+      if (d0 >= a.DP) break;
+      if (d0 + x >= a.DP) q[u] = k[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      __syncthreads();
+      *reinterpret_cast<f32x4_t*>(qs + at) = q[u] * a.q_scale;
+      *reinterpret_cast<f32x4_t*>(ks + at) = k[u];
+      __syncthreads();
+      if (wave < 10) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          const int place = 16 * s + 4 * (lane >> 4);
+          const f32x4_t fq = *reinterpret_cast<const f32x4_t*>(qs + (16 * tr + (lane & 15)) * kScoreRow + place);
+          const f32x4_t fk = *reinterpret_cast<const f32x4_t*>(ks + (16 * tc + (lane & 15)) * kScoreRow + place);
+#pragma unroll
+          for (int e = 0; e < 4; e++) p = __builtin_amdgcn_mfma_f32_16x16x4f32(fq[e], fk[e], p, 0, 0, 0);
+        }
+      }
+    }
+  }
+  if (wave < 10) {
+    float* to = a.scores + (int64_t)item * (kChunk * kChunk) + (16 * tr + 4 * (lane >> 4)) * kChunk + 16 * tc + (lane & 15);
+#pragma unroll
+    for (int e = 0; e < 4; e++) to[e * kChunk] = p[e];
+  }
+}
+
+// Grid = (chunks + 1, heads).  The first H workgroups: the heads' gates, a chain of short steps; the others, meanwhile: a chunk's and head's scores, which need no gate.
+// us, four heads of 256 x 512, 1531 tokens: gates alone 11.3 (three trips to memory for a second token, which are one
+// now), both 9.4, the scores by themselves 6.4 of that.
+__global__ __launch_bounds__(1024) void mlstm_gates_kernel(const MemArgs a) {
+  __shared__ __align__(16) float lds[2 * kChunk * kScoreRow];
+  static_assert(sizeof(GatesLds) <= sizeof(lds), "either of them");
+  const int block = blockIdx.x + gridDim.x * blockIdx.y;
+  if (block < a.H) head_gates(a, block, *reinterpret_cast<GatesLds*>(lds));
+  else chunk_scores(a, block - a.H, lds);
 }
 
 // Grid = (64 x 64 tiles of a head's state, heads, chunks); wave w: rows 32 (w >> 1), columns 32 (w & 1) of the tile.
@@ -509,151 +621,166 @@ __global__ __launch_bounds__(StateTile<ROWS>::kThreads, ROWS == 64 ? 4 : 2) void
   dh::arrive_and_wait<0>();                            // nothing may be in flight towards LDS when the workgroup ends
 }
 
-// Grid = (chunks, heads, groups of 64 TN value columns); wave w: tokens 32 (w >> 1), columns 32 TN (w & 1) + 0 .. 32 TN - 1.
-template <int TN>
-__global__ __launch_bounds__(256) void mlstm_outputs_kernel(const MemArgs a) {
-  constexpr int BV = 64 * TN, BD = 32, ROW = BD + 4, VROW = BV + 4, PROW = kChunk + 4;
+// 2^y of a double, in f32: the whole part goes into the exponent, so that the f32 exponential sees at most a half.
+__device__ __forceinline__ float exp2_of(double y) {
+  const double whole = __builtin_rint(y);
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((float)(y - whole)), (int)whole);
+}
+
+// o of 64 tokens x 64 value columns of a (chunk, head): Q S over dim, decayed, plus the decayed and masked scores times V; four waves of 32 x 32.
+// Grid: x = eight (chunk, head) pairs, one a die, under the column groups; y and z = eights of pairs.  So the column groups of a pair follow one
+// another on a die, whose L2 then holds its rows and scores.
+// Bound by the 32-bit matrix cores (160 instructions of 64 cycles a wave) and by what a step does besides: 64 dims' rows go through registers into LDS
+// in front of each quarter of the products, requested by offsets that are computed once (address arithmetic at every step took as long as the products).
+// us, four heads of 256 x 512, 1531 tokens (24 chunks: 768 workgroups, three a compute unit) 28 against 46.6 with Q K^T in here, once for each 128
+// columns (384 workgroups of twice the columns), and exponentials by expf; 40 tokens, four heads of 128 x 256, 8.6 against 14.4.
+// FAR: 64 rows span more than 4 GB.
+template <bool FAR>
+__global__ __launch_bounds__(256, 3) void mlstm_outputs_kernel(const MemArgs a) {
+  using Offset = std::conditional_t<FAR, uint64_t, uint32_t>;
+  // rows of LDS: read across rows (queries, scores) or across columns of rows four apart (states, values)
+  constexpr int BD = 64, ROW = kScoreRow, VROW = 64 + 8;
+  constexpr double kLog2e = 1.4426950408889634;
   __shared__ __align__(16) float qs[kChunk * ROW];
-  __shared__ __align__(16) float ks[kChunk * ROW];
-  __shared__ __align__(16) float sv[kChunk * VROW];    // state rows, later the values
-  __shared__ __align__(16) float ps[kChunk * PROW];
-  __shared__ double Fl[kChunk];
-  __shared__ float il[kChunk];
-  __shared__ float ml[kChunk];
+  __shared__ __align__(16) float sv[kChunk * VROW];
+  __shared__ __align__(16) double decay_to[kChunk];    // a score's decay: 2^(to[t] + from[s])
+  __shared__ __align__(16) double decay_from[kChunk];
   __shared__ float inter[kChunk];                      // what the state before the chunk has decayed to, per token
-  __shared__ float nq[kChunk];                         // n_start . q
-  __shared__ float nl[BD];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = blockIdx.x, h = blockIdx.y, v0 = BV * blockIdx.z;
+  __shared__ float least[kChunk];                      // e^-m
+  __shared__ float factor[kChunk];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int group = blockIdx.x >> 3, ch = (blockIdx.x & 7) + 8 * (blockIdx.y + gridDim.y * blockIdx.z), v0 = 64 * group;
+  if (ch >= a.chunks * a.H) return;
+  const int c = ch / a.H, h = ch - c * a.H;
   const int first = c * kChunk, count = min(kChunk, a.T - first);
-  const int wt = 32 * (wave >> 1), wc = 32 * TN * (wave & 1), ws = 32 * (wave & 1);
-  const float* Sc = a.Sc + ((int64_t)c * a.H + h) * a.DP * a.VP;
-  const float* nc = a.nc + ((int64_t)c * a.H + h) * a.DP;
+  // (the waves of the first 32 tokens have half of the scores: every other column group turns them round)
+  const int wt = 32 * ((wave >> 1) ^ (group & 1)), wc = 32 * (wave & 1);
+  // a thread's rows r0 + 16 r and its columns x .. x + 3 of every 64; offsets in bytes from bases all threads share
+  const int r0 = tid >> 4, x = 4 * (tid & 15), v = min(v0 + x, a.VP - 4);
+  const float *q_base = a.rows + (int64_t)first * a.ld_row + (int64_t)h * a.DP, *s_base = a.Sc + (int64_t)ch * a.DP * a.VP, *n_base = a.nc + (int64_t)ch * a.DP;
+  Offset q_off[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) q_off[r] = 4 * ((Offset)min(r0 + 16 * r, count - 1) * (Offset)a.ld_row + x);
+  const Offset s_off = 4 * ((Offset)r0 * a.VP + v);
+  f32x4_t qr[4], sr[4], nr;
+  auto at = [](const float* base, Offset off) { return *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const char*>(base) + off); };
+  // (where dims are no multiple of 64 the last step reads up to 32 dims past them, of what follows in a row and in the workspace, and drops them)
+  auto request = [&](int d0) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) qr[r] = at(q_base + d0, q_off[r]);
+#pragma unroll
+    for (int r = 0; r < 4; r++) sr[r] = at(s_base + (int64_t)(d0 + 16 * r) * a.VP, s_off);
+    nr = at(n_base + d0, 4 * x);
+  };
+  request(0);
   if (tid < kChunk) {
     const int t = first + min(tid, count - 1);
     const double F_start = first > 0 ? a.F[(int64_t)h * a.T + first - 1] : 0.0, F = a.F[(int64_t)h * a.T + t];
     const float m = a.mt[(int64_t)h * a.T + t];
-    Fl[tid] = F;
-    il[tid] = a.i[(int64_t)h * a.T + t];
-    ml[tid] = m;
+    decay_to[tid] = (F - (double)m) * kLog2e;
+    decay_from[tid] = ((double)a.i[(int64_t)h * a.T + t] - F) * kLog2e;
     inter[tid] = expf((float)(F - F_start + (double)a.mc[(int64_t)h * (a.chunks + 1) + c] - (double)m));
+    least[tid] = expf(-m);
   }
-  f32x16_t p, o[TN];
+  f32x16_t o;
 #pragma unroll
-  for (int e = 0; e < 16; e++) p[e] = 0.f;
+  for (int e = 0; e < 16; e++) o[e] = 0.f;
+  float dot[4] = {0.f, 0.f, 0.f, 0.f};                 // n_start . q of the thread's rows
+  auto store = [&] {
 #pragma unroll
-  for (int j = 0; j < TN; j++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[j][e] = 0.f;
-  float dot = 0.f;                                     // token tid >> 2, every fourth dim from tid & 3 on
-
-  f32x4_t qr[2], kr[2], sr[2 * TN];
-  float nr = 0.f;
-  auto load = [&](int d0) {
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-      const int x = tid + 256 * r, tok = first + min(x >> 3, count - 1), d = d0 + 4 * (x & 7);
-      const float* row = a.rows + (int64_t)tok * a.ld_row + (int64_t)h * a.DP + d;
-      qr[r] = *reinterpret_cast<const f32x4_t*>(row);
-      kr[r] = *reinterpret_cast<const f32x4_t*>(row + a.k_off);
+    for (int r = 0; r < 4; r++) {
+      *reinterpret_cast<f32x4_t*>(&qs[(r0 + 16 * r) * ROW + x]) = qr[r];
+      *reinterpret_cast<f32x4_t*>(&sv[(r0 + 16 * r) * VROW + x]) = sr[r];
     }
-#pragma unroll
-    for (int r = 0; r < 2 * TN; r++) {
-      const int x = tid + 256 * r, d = d0 + x / (BV / 4), v = v0 + 4 * (x % (BV / 4));
-      sr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (v < a.VP) sr[r] = *reinterpret_cast<const f32x4_t*>(Sc + (int64_t)d * a.VP + v);
-    }
-    if (tid < BD) nr = nc[d0 + tid];
   };
-  load(0);
-  for (int d0 = 0; d0 < a.DP; d0 += BD) {
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-      const int x = tid + 256 * r;
-      qr[r] *= a.q_scale;
-      *reinterpret_cast<f32x4_t*>(&qs[(x >> 3) * ROW + 4 * (x & 7)]) = qr[r];
-      *reinterpret_cast<f32x4_t*>(&ks[(x >> 3) * ROW + 4 * (x & 7)]) = kr[r];
-    }
-#pragma unroll
-    for (int r = 0; r < 2 * TN; r++) {
-      const int x = tid + 256 * r;
-      *reinterpret_cast<f32x4_t*>(&sv[x / (BV / 4) * VROW + 4 * (x % (BV / 4))]) = sr[r];
-    }
-    if (tid < BD) nl[tid] = nr;
-    __syncthreads();
-    if (d0 + BD < a.DP) load(d0 + BD);
-#pragma unroll
-    for (int s = 0; s < BD / 8; s++) {
+  // o += rows of qs times columns of sv over so many eights of either; the next eight are read while these are multiplied
+  auto multiply = [&](auto eights) {
+    constexpr int N = decltype(eights)::value;
+    f32x4_t fq[2], fs[2];
+    auto read = [&](int s) {
       const int d = 8 * s + 4 * (lane >> 5);
-      const f32x4_t fq = *reinterpret_cast<const f32x4_t*>(&qs[(wt + (lane & 31)) * ROW + d]);
-      const f32x4_t fk = *reinterpret_cast<const f32x4_t*>(&ks[(ws + (lane & 31)) * ROW + d]);
+      fq[s & 1] = *reinterpret_cast<const f32x4_t*>(&qs[(wt + (lane & 31)) * ROW + d]);
 #pragma unroll
-      for (int e = 0; e < 4; e++) p = __builtin_amdgcn_mfma_f32_32x32x2f32(fq[e], fk[e], p, 0, 0, 0);
+      for (int e = 0; e < 4; e++) fs[s & 1][e] = sv[(d + e) * VROW + wc + (lane & 31)];
+    };
+    read(0);
 #pragma unroll
-      for (int j = 0; j < TN; j++)
+    for (int s = 0; s < N; s++) {
+      if (s + 1 < N) read(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fq[e], sv[(d + e) * VROW + wc + 32 * j + (lane & 31)], o[j], 0, 0, 0);
+      for (int e = 0; e < 4; e++) o = __builtin_amdgcn_mfma_f32_32x32x2f32(fq[s & 1][e], fs[s & 1][e], o, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int d0 = 0; d0 < a.DP; d0 += BD) {
+    if (d0 + BD > a.DP) {                              // the upper half of these dims is not there (sizes are multiples of 32)
+      if (x >= 32) {
+        nr = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; r++) qr[r] = nr;
+      }
+      sr[2] = sr[3] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int d = 0; d < BD; d += 4) dot = fmaf(qs[(tid >> 2) * ROW + d + (tid & 3)], nl[d + (tid & 3)], dot);
-  }
-  dot = dh::group_combine<1, 4>(dot, dh::AddOp());
-  if ((tid & 3) == 0) nq[tid >> 2] = dot;
-  // decayed scores: accumulator element e holds token wt + 8 (e / 4) + 4 (lane >> 5) + e % 4, earlier token ws + (lane & 31)
-  {
-    const int s = ws + (lane & 31);
-    const double base = (double)il[s] - Fl[s];
+    for (int r = 0; r < 4; r++) {
+      qr[r] *= a.q_scale;
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const int t = wt + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      const float w = s <= t && s < count ? expf((float)(Fl[t] + base - (double)ml[t])) : 0.f;
-      ps[t * PROW + s] = w * p[e];
+      for (int e = 0; e < 4; e++) dot[r] = fmaf(qr[r][e], nr[e], dot[r]);
     }
-  }
-  __syncthreads();                                     // scores are there; the last state rows have been consumed
+    __syncthreads();
+    store();
+    __syncthreads();
+    // the next dims' rows, behind the last ones scores and values
+    if (d0 + BD < a.DP) {
+      request(d0 + BD);
+    } else {
+      const float *p_base = a.scores + (int64_t)ch * (kChunk * kChunk), *v_base = q_base + (a.v_off + (int64_t)h * (a.VP - a.DP) + v - x);
 #pragma unroll
-  for (int r = 0; r < 4 * TN; r++) {
-    const int x = tid + 256 * r, tok = first + min(x / (BV / 4), count - 1), v = v0 + 4 * (x % (BV / 4));
-    f32x4_t vv = {0.f, 0.f, 0.f, 0.f};
-    if (v < a.VP) vv = *reinterpret_cast<const f32x4_t*>(a.rows + (int64_t)tok * a.ld_row + a.v_off + (int64_t)h * a.VP + v);
-    *reinterpret_cast<f32x4_t*>(&sv[x / (BV / 4) * VROW + 4 * (x % (BV / 4))]) = vv;
+      for (int r = 0; r < 4; r++) {
+        qr[r] = at(p_base + 16 * kChunk * r, 16 * tid);
+        sr[r] = at(v_base, q_off[r]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(std::integral_constant<int, BD / 8>{});
   }
-  // a token's normaliser and with it the factor of its outputs
-  float sum = 0.f;
-  for (int s = tid & 3; s < kChunk; s += 4) sum += ps[(tid >> 2) * PROW + s];
-  sum = dh::group_combine<1, 4>(sum, dh::AddOp());
+  // decayed scores (nothing of what lies past the diagonal is a score), and with their sums the factor of a token's outputs
+  double from[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) from[e] = decay_from[x + e];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int t = r0 + 16 * r;
+    const double to = decay_to[t];
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const float decayed = exp2_of(to + from[e]) * qr[r][e];
+      qr[r][e] = x + e <= t && x + e < count ? decayed : 0.f;
+      sum += qr[r][e];
+    }
+    sum = dh::group_combine<1, 16>(sum, dh::AddOp());
+    const float nq = dh::group_combine<1, 16>(dot[r], dh::AddOp());
+    if (x == 0) factor[t] = 1.0f / (fmaxf(fabsf(fmaf(inter[t], nq, sum)), least[t]) + kDenominatorEps);
+    if (t >= count) sr[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();
+  store();
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 16; e++) o[e] *= inter[wt + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)];
+  if (__builtin_amdgcn_readfirstlane(wt)) multiply(std::integral_constant<int, kChunk / 8>{});
+  else multiply(std::integral_constant<int, kChunk / 16>{});         // tokens 0 .. 31 have no scores past them
+#pragma unroll
+  for (int e = 0; e < 16; e++) o[e] *= factor[wt + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)];
+  const int col = v0 + wc + (lane & 31);
+  if (col >= a.VP) return;
+  float* out = a.out + (int64_t)(first + wt + 4 * (lane >> 5)) * a.ld_out + (int64_t)h * a.VP + col;
 #pragma unroll
   for (int e = 0; e < 16; e++) {
-    const float f = inter[wt + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)];
-#pragma unroll
-    for (int j = 0; j < TN; j++) o[j][e] *= f;
-  }
-  __syncthreads();
-  if ((tid & 3) == 0) {
-    const int t = tid >> 2;
-    nq[t] = 1.0f / (fmaxf(fabsf(fmaf(inter[t], nq[t], sum)), expf(-ml[t])) + kDenominatorEps);
-  }
-#pragma unroll
-  for (int s = 0; s < kChunk / 8; s++) {
-    const int d = 8 * s + 4 * (lane >> 5);
-    const f32x4_t fp = *reinterpret_cast<const f32x4_t*>(&ps[(wt + (lane & 31)) * PROW + d]);
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fp[e], sv[(d + e) * VROW + wc + 32 * j + (lane & 31)], o[j], 0, 0, 0);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < TN; j++) {
-    const int v = v0 + wc + 32 * j + (lane & 31);
-    if (v >= a.VP) continue;
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const int t = wt + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      if (t < count) a.out[(int64_t)(first + t) * a.ld_out + (int64_t)h * a.VP + v] = o[j][e] * nq[t];
-    }
+    const int t = 8 * (e >> 2) + (e & 3);
+    if (wt + 4 * (lane >> 5) + t < count) out[(int64_t)t * a.ld_out] = o[e];
   }
 }
 
@@ -763,7 +890,8 @@ int dh_mlstm_step(const dh_mlstm* spec, const float* d_row, void* d_state, float
 size_t dh_mlstm_prefill_workspace_bytes(const dh_mlstm* s, int T) {
   if (!s || T <= 0) return 256;
   const size_t chunks = (size_t)dh::ceil_div(T, kChunk), HT = (size_t)s->H * T;
-  return up256(HT * 8) + 2 * up256(HT * 4) + 2 * up256((size_t)s->H * (chunks + 1) * 4) + up256((size_t)s->H * chunks * kChunk * 4) + up256((chunks + 1) * s->H * s->DP * 4) +
+  return up256(HT * 8) + 2 * up256(HT * 4) + 2 * up256((size_t)s->H * (chunks + 1) * 4) + up256((size_t)s->H * chunks * kChunk * 4) +
+         up256((size_t)s->H * chunks * kChunk * kChunk * 4) + up256((chunks + 1) * s->H * s->DP * 4) +
          up256((chunks + 1) * s->H * s->DP * s->VP * 4);
 }
 
@@ -797,13 +925,14 @@ int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, v
   a.mc = reinterpret_cast<float*>(take((size_t)spec->H * (a.chunks + 1) * 4));
   a.keep = reinterpret_cast<float*>(take((size_t)spec->H * (a.chunks + 1) * 4));
   a.w = reinterpret_cast<float*>(take((size_t)spec->H * a.chunks * kChunk * 4));
+  a.scores = reinterpret_cast<float*>(take((size_t)spec->H * a.chunks * kChunk * kChunk * 4));
   a.nc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * 4));
   a.Sc = reinterpret_cast<float*>(take((size_t)(a.chunks + 1) * spec->H * spec->DP * spec->VP * 4));
   // (more chunks than a grid's smaller dimensions hold have always been refused)
   if (a.chunks > 65535) return dh::fail(1, "[%s] %d tokens are too many for one portion", op, T);
   const int rows = walk_rows(*spec, a.chunks);
   if (!rows) a.w = nullptr;
-  hipLaunchKernelGGL(mlstm_gates_kernel, dim3(spec->H), dim3(1024), 0, dh::stream(), a);
+  hipLaunchKernelGGL(mlstm_gates_kernel, dim3(a.chunks + 1, spec->H), dim3(1024), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   if (rows) {
     if (int rc = rows == 64 ? launch_states<64>(op, a) : launch_states<32>(op, a)) return rc;
@@ -814,10 +943,11 @@ int dh_mlstm_prefill(const dh_mlstm* spec, const float* d_rows, void* d_state, v
     hipLaunchKernelGGL(mlstm_scan_kernel, dim3((unsigned)dh::ceil_div((int64_t)spec->DP * spec->VP + spec->DP, 1024), spec->H), dim3(256), 0, dh::stream(), a);
     DH_CHECK_LAUNCH(op);
   }
-  // wide column groups repeat Q K^T less often; narrow ones where those would not fill the device
-  const bool wide = spec->VP > 64 && (int64_t)a.chunks * spec->H * dh::ceil_div(spec->VP, 128) >= dh::num_cus();
-  if (wide) hipLaunchKernelGGL(mlstm_outputs_kernel<2>, dim3(a.chunks, spec->H, (unsigned)dh::ceil_div(spec->VP, 128)), dim3(256), 0, dh::stream(), a);
-  else hipLaunchKernelGGL(mlstm_outputs_kernel<1>, dim3(a.chunks, spec->H, (unsigned)dh::ceil_div(spec->VP, 64)), dim3(256), 0, dh::stream(), a);
+  const int64_t eights = dh::ceil_div((int64_t)a.chunks * spec->H, 8), deep = dh::ceil_div(eights, 65535);
+  // (a row of the workspace's states, 64 of which are offsets too, is never longer than one of these)
+  auto outputs = (int64_t)4 * kChunk * a.ld_row < (int64_t)1 << 32 ? mlstm_outputs_kernel<false> : mlstm_outputs_kernel<true>;
+  hipLaunchKernelGGL(outputs, dim3(8 * (unsigned)dh::ceil_div(spec->VP, 64), (unsigned)dh::ceil_div(eights, deep), (unsigned)deep), dim3(256), 0,
+                     dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   return 0;
 }

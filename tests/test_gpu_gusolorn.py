@@ -266,6 +266,48 @@ def test_memory_walks_give_the_bits_of_two_launches(L, H, D, V, T, start, rows, 
         assert state[v:].view(-1)[to * H + h] == own[D * (V + 2) + to], h
 
 
+@pytest.mark.parametrize("H,D,V,T,start,far", [(2, 32, 32, 1, 0, False), (9, 96, 96, 63, 3, False), (1, 160, 64, 65, 0, False), (3, 64, 160, 130, 5, False),
+                                               (1, 320, 32, 70, 2, False), (2, 96, 96, 67, 1, True)])
+def test_memory_outputs_of_a_portion(L, H, D, V, T, start, far):
+    """Outputs against the recurrence in 64 bits: dims and columns in whole and half tiles, last chunks of one to all tokens, pairs of chunk and head that
+    fill no eight, more dims than one batch of scores requests, and rows so far apart that 64 span more than 4 GB.  Every sum's roundings (dim products of
+    a query and the state or a key, 64 of a chunk's tokens with the score and the value, 66 a chunk in the state) on the sum of its terms' sizes."""
+    spec, qkv, ld = memory_spec(H, D, V)
+    g = torch.Generator(device="cuda").manual_seed(D + T)
+    x = torch.randn(T, ld, generator=g, device="cuda")
+    state = torch.randn(int(L.dh_mlstm_state_bytes(ctypes.byref(spec))) // 4, generator=g, device="cuda")
+    f = lambda t: t.double().cpu().numpy()
+    S, n, m = f(state[:H * D * V].view(H, D, V)), f(state[H * D * V:][:2 * H * D].view(2, H, D)[start & 1]), f(state[H * D * (V + 2):][:2 * H].view(2, H)[start & 1])
+    if not start:
+        S, n, m = 0 * S, 0 * n, 0 * m
+    q, k, v = (f(x[:, a:a + H * d]).reshape(T, H, d) for a, d in ((0, D), (H * D, D), (2 * H * D, V)))
+    zi, zf = f(x[:, qkv:qkv + H]), f(x[:, qkv + H:qkv + 2 * H])
+    SA, nA, want, bound = np.abs(S), np.abs(n), np.zeros((T, H, V)), np.zeros((T, H, V))
+    for t in range(T):
+        i, lf = 15 * np.tanh(zi[t] / 15), 15 * np.tanh(zf[t] / 15)
+        lf = np.minimum(lf, 0) - np.log1p(np.exp(-np.abs(lf)))
+        to = np.maximum(lf + m, i)
+        keep, put, m = np.exp(lf + m - to), np.exp(i - to), to
+        kv = k[t][:, :, None] * v[t][:, None, :]
+        S, SA = keep[:, None, None] * S + put[:, None, None] * kv, keep[:, None, None] * SA + put[:, None, None] * np.abs(kv)
+        n, nA = keep[:, None] * n + put[:, None] * k[t], keep[:, None] * nA + put[:, None] * np.abs(k[t])
+        qt = q[t] * D ** -0.5
+        den = np.maximum(np.abs((n * qt).sum(1)), np.exp(-m))[:, None] + 1e-6
+        want[t] = (S * qt[:, :, None]).sum(1) / den
+        bound[t] = ((SA * np.abs(qt)[:, :, None]).sum(1) + np.abs(want[t]) * (nA * np.abs(qt)).sum(1)[:, None]) / den
+    if far:
+        wide = torch.zeros(T, 1 << 24, device="cuda")          # 64 MB a row
+        wide[:, :ld] = x
+        x, spec.ld_row = wide, 1 << 24
+    ws = torch.full((int(L.dh_mlstm_prefill_workspace_bytes(ctypes.byref(spec), T)),), 255, dtype=torch.uint8, device="cuda")
+    out = torch.zeros(T, H * V, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_mlstm_prefill(ctypes.byref(spec), x.data_ptr(), state.data_ptr(), ws.data_ptr(), out.data_ptr(), H * V, T, start))
+    capi.check(L.dh_sync())
+    worst = (np.abs(f(out).reshape(T, H, V) - want) / bound).max()
+    assert worst <= (D + 2 * 64 + 66 * -(-T // 64)) * 2.0 ** -24, worst * 2.0 ** 24
+
+
 @pytest.mark.parametrize("live,before", [(1, 0), (2, 0), (4, 0), (1, 64)])
 def test_memory_state_of_few_live_tokens(L, live, before):
     """A chunk that few tokens count in (a portion of one, two or four tokens, and one whose last token closes the forget gate over 64 others)

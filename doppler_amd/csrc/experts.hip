@@ -11,8 +11,9 @@
 //
 // Decode: experts_up_kernel chooses the experts itself (every workgroup, from the few logits), norms the row and streams the
 // chosen gate and up rows; experts_down_kernel streams the chosen down matrices and the shared one side by side along k.
-// Prefill: experts_route_kernel, experts_sort_kernel (rows sorted by expert, table of row tiles), grouped products on the
-// matrix cores (dense_gemm.hip), experts_combine_kernel.
+// Prefill: experts_router_kernel (logits and choices) and experts_place_kernel (rows sorted by expert, table of row tiles), or for f32 operands, more than
+// 64 logits and long portions a product, experts_route_kernel and experts_sort_kernel; grouped products on the matrix cores (dense_gemm.hip);
+// experts_combine_kernel.
 #include <algorithm>
 #include <cfloat>
 
@@ -27,7 +28,8 @@ constexpr int kMaxExperts = 1024;
 struct StepArgs {
   const float* x;
   const float* norm;
-  const float* z;          // router logits [E], then the shared expert's
+  const uint16_t* router;  // [E and the shared expert's][K]
+  float* z;                // router logits [E], then the shared expert's
   const uint16_t* up;      // [E][2 ff][ld_in]
   const uint16_t* down;    // [E][hidden][ff]
   const uint16_t* shared_up;
@@ -73,40 +75,48 @@ __device__ __forceinline__ void choose_upto(const float* z, int E, int top, int*
       if (lane + 64 * j == id) v[j] = -INFINITY;
   }
 }
+// The same for up to 64 experts, a lane each: a lane's place is the number of experts in front of it.  The largest one after the other are `top` chains of
+// lane steps (0.3 us each), this a pass over the experts whose steps do not wait for one another (0.15 us for 16): experts_up and _down at hidden 1024,
+// four of 16 experts, 6.6 against 6.9 and 4.8 against 5.0 us.
+__device__ __forceinline__ void choose_by_places(const float* z, int E, int top, int* ids, float* zs) {
+  const int lane = threadIdx.x & 63;
+  const float own = z[min(lane, E - 1)], key = lane < E && own == own ? own : -INFINITY;
+  int place = 0;
+  for (int j0 = 0; j0 < E; j0 += 8) {                  // (lanes past the last expert are in front of none)
+#pragma unroll
+    for (int j = j0; j < j0 + 8; j++) {
+      const float other = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(key), j));
+      place += other > key || (other == key && j < lane) ? 1 : 0;
+    }
+  }
+  if (lane < E && place < top) {
+    ids[place] = lane;
+    zs[place] = own;
+  }
+}
 __device__ __forceinline__ void choose(const float* z, int E, int top, int* ids, float* zs) {
-  if (E <= 64) choose_upto<1>(z, E, top, ids, zs);
+  if (E <= 64 && E <= 32 * top) choose_by_places(z, E, top, ids, zs);
+  else if (E <= 64) choose_upto<1>(z, E, top, ids, zs);
   else if (E <= 256) choose_upto<4>(z, E, top, ids, zs);
   else choose_upto<kMaxExperts / 64>(z, E, top, ids, zs);
 }
 
 // A wave takes a gate and an up row at a time; the row sits in LDS as two planes of 16-byte pieces, as in the dense GEMV.
-template <int U>
+//
+// PR > 0: the router's logits are made here too, by every workgroup, four waves five rows each of at most 64 PR pieces, requested beside the row itself;
+// the first workgroup leaves them for experts_down_kernel.  A launch for seventeen sums (2.9 us and 1.4 in front of the next) against their weights once
+// more for each workgroup, from the L2: us, 17 rows of 1024 7.8 against 2.8 + 6.6, of 2048 14.8 against 3.4 + 14.2, and a gap between
+// launches less; from 4096 on the workgroups of a compute unit would read half a megabyte of them.  A wave whose first columns are the shared expert's requests those at once as well.
+constexpr int kRouterRows = 5;                         // of a wave
+template <int U, int PR>
 __global__ __launch_bounds__(256) void experts_up_kernel(const StepArgs a, int iters) {
   extern __shared__ __align__(16) float4 planes[];       // [2][K / 8]
   __shared__ float red[4];
+  __shared__ float logits_s[4 * kRouterRows];
   __shared__ int ids[kMaxTop];
   __shared__ float zs[kMaxTop];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int np = a.K >> 3, nstages = (np + 64 * U - 1) / (64 * U);
-  const float4* xg = reinterpret_cast<const float4*>(a.x);
-  float ss = 0.f;
-  for (int i = tid; i < (a.K >> 2); i += 256) {
-    const float4 v = xg[i];
-    ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss); ss = fmaf(v.w, v.w, ss);
-  }
-  ss = dh::wave_sum_uniform(ss);
-  if (lane == 0) red[wave] = ss;
-  if (wave == 0) choose(a.z, a.E, a.top, ids, zs);
-  __syncthreads();
-  const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)a.hidden + a.eps);
-  for (int i = tid; i < (a.K >> 2); i += 256) {
-    float4 v = xg[i];
-    const float4 w = reinterpret_cast<const float4*>(a.norm)[i];
-    v.x = v.x * inv * w.x; v.y = v.y * inv * w.y; v.z = v.z * inv * w.z; v.w = v.w * inv * w.w;
-    planes[(i & 1) * np + (i >> 1)] = v;
-  }
-  __syncthreads();
-  const int total = a.top * a.ff + a.shared_ff;
+  const int np = a.K >> 3, nstages = (np + 64 * U - 1) / (64 * U), total = a.top * a.ff + a.shared_ff;
   uint4 cur[2][U], nxt[2][U];
   auto load = [&](int unit, uint4 (&dst)[2][U]) {
     const int it = unit / nstages, st = unit - it * nstages;
@@ -124,7 +134,86 @@ __global__ __launch_bounds__(256) void experts_up_kernel(const StepArgs a, int i
       }
     }
   };
-  load(0, cur);
+  const float4 *xg = reinterpret_cast<const float4*>(a.x), *wg = reinterpret_cast<const float4*>(a.norm);
+  auto scaled = [](const float4& v, float f, const float4& w) { return make_float4(v.x * f * w.x, v.y * f * w.y, v.z * f * w.z, v.w * f * w.w); };
+  auto squares = [](const float4& v, float ss) {
+    ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss);
+    return fmaf(v.w, v.w, ss);
+  };
+  const float* z = a.z;
+  if constexpr (PR > 0) {
+    constexpr int XV = (PR + 1) / 2;                     // pieces of the row a thread holds
+    const int rows = a.E + (a.shared_ff ? 1 : 0), nx = a.K >> 2;
+    const bool ahead = (int)blockIdx.x * 4 >= a.top * a.ff;
+    float4 xv[XV], wv[XV];
+    uint4 rw[kRouterRows][PR];
+#pragma unroll
+    for (int j = 0; j < XV; j++) {
+      xv[j] = xg[min(tid + 256 * j, nx - 1)];
+      wv[j] = wg[min(tid + 256 * j, nx - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < kRouterRows; i++)
+#pragma unroll
+      for (int u = 0; u < PR; u++)
+        rw[i][u] = reinterpret_cast<const uint4*>(a.router + (int64_t)min(wave + 4 * i, rows - 1) * a.K)[min(lane + 64 * u, np - 1)];
+    if (ahead) load(0, cur);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < XV; j++)
+      if (tid + 256 * j < nx) ss = squares(xv[j], ss);
+    ss = dh::wave_sum_uniform(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)a.hidden + a.eps);
+#pragma unroll
+    for (int j = 0; j < XV; j++) {
+      const int i = tid + 256 * j;
+      if (i < nx) planes[(i & 1) * np + (i >> 1)] = scaled(xv[j], inv, wv[j]);
+    }
+    __syncthreads();
+    float sum[kRouterRows] = {};
+#pragma unroll
+    for (int u = 0; u < PR; u++) {
+      const int p = min(lane + 64 * u, np - 1);
+      float4 xa = planes[p], xb = planes[np + p];
+      if (lane + 64 * u >= np) xa = xb = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int i = 0; i < kRouterRows; i++) {
+        const uint4 w = rw[i][u];
+        float s = sum[i];
+        s = fmaf(xa.x, dh::bf16_low(w.x), s); s = fmaf(xa.y, dh::bf16_high(w.x), s);
+        s = fmaf(xa.z, dh::bf16_low(w.y), s); s = fmaf(xa.w, dh::bf16_high(w.y), s);
+        s = fmaf(xb.x, dh::bf16_low(w.z), s); s = fmaf(xb.y, dh::bf16_high(w.z), s);
+        s = fmaf(xb.z, dh::bf16_low(w.w), s); s = fmaf(xb.w, dh::bf16_high(w.w), s);
+        sum[i] = s;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kRouterRows; i++) {
+      const float s = dh::wave_sum_uniform(sum[i]);
+      if (lane == 0) {
+        logits_s[wave + 4 * i] = s;
+        if (blockIdx.x == 0 && wave + 4 * i < rows) a.z[wave + 4 * i] = s;
+      }
+    }
+    __syncthreads();
+    z = logits_s;
+    if (wave == 0) choose(z, a.E, a.top, ids, zs);
+    __syncthreads();
+    if (!ahead) load(0, cur);
+  } else {
+    float ss = 0.f;
+    for (int i = tid; i < (a.K >> 2); i += 256) ss = squares(xg[i], ss);
+    ss = dh::wave_sum_uniform(ss);
+    if (lane == 0) red[wave] = ss;
+    if (wave == 0) choose(z, a.E, a.top, ids, zs);
+    __syncthreads();
+    const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)a.hidden + a.eps);
+    for (int i = tid; i < (a.K >> 2); i += 256) planes[(i & 1) * np + (i >> 1)] = scaled(xg[i], inv, wg[i]);
+    __syncthreads();
+    load(0, cur);
+  }
   float acc[2] = {0.f, 0.f};
   int st = 0, it = 0;
   for (int unit = 0; unit < iters * nstages; unit++) {
@@ -149,7 +238,7 @@ __global__ __launch_bounds__(256) void experts_up_kernel(const StepArgs a, int i
       const int col = (it * (int)gridDim.x + (int)blockIdx.x) * 4 + wave;
       if (lane == 0 && col < total) {
         if (col >= a.top * a.ff) {
-          a.act[col] = dh::clamped_glu(g, u, a.shared_limit) * sigmoid_f(a.z[a.E]);
+          a.act[col] = dh::clamped_glu(g, u, a.shared_limit) * sigmoid_f(z[a.E]);
         } else {
           const float s = sigmoid_f(zs[col / a.ff]);
           a.act[col] = dh::clamped_glu(s * g, s * u, a.limit);
@@ -270,21 +359,180 @@ __global__ __launch_bounds__(256) void experts_down_kernel(const StepArgs a, int
 
 // ------------------------------------------------------------------ portions
 
+// A token's choices from its logits, by one wave.
+__device__ __forceinline__ void route_token(const float* z, int t, int E, int top, int shared, int* id_s, float* z_s, int* __restrict__ ids,
+                                            float* __restrict__ weights, float* __restrict__ sg) {
+  const int lane = threadIdx.x & 63;
+  choose(z, E, top, id_s, z_s);
+  __builtin_amdgcn_wave_barrier();
+  if (lane < top) {
+    ids[(int64_t)t * top + lane] = id_s[lane];
+    weights[(int64_t)t * top + lane] = sigmoid_f(z_s[lane]);
+  }
+  if (shared && lane == 0) sg[t] = sigmoid_f(z[E]);
+}
+
+// Logits of sixteen tokens, up to 16 NT of them each, and the tokens' choices.  Few columns over a long k are one trip to memory and a short product: each of
+// the waves takes every sixteenth 32 of k straight from memory into its fragments of v_mfma_f32_16x16x32_bf16, four of them requested together, and
+// the waves' sums meet in LDS in wave order.  What the places need goes out with the choices: slot, a choice's rank among the group's of its expert (in any
+// order), and counts [groups][E].  us, 1531 rows of 2048, 16 experts and a shared one: 8.1, against 6.1 + 5.3 + 4.8 for a product
+// with k in slices, the slices' sum and the choices; 40 rows of 1024 8 against 6.6 + 3.3.
+constexpr int kRouterLogits = 64;
+template <int NT>
+constexpr int kRouterWaves = NT <= 2 ? 16 : 8;         // (the sums of sixteen would not fit the LDS)
+template <int NT>
+__global__ __launch_bounds__(64 * kRouterWaves<NT>) void experts_router_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ router, int K, int T, int E, int top,
+                                                             int shared, int* __restrict__ ids, float* __restrict__ weights, float* __restrict__ sg,
+                                                             int* __restrict__ slot, int* __restrict__ counts) {
+  constexpr int WAVES = kRouterWaves<NT>, AHEAD = 64 / WAVES, ROW = 16 * NT + 4;
+  __shared__ __align__(16) float sums[WAVES][16][ROW];
+  __shared__ int id_s[WAVES][kMaxTop];
+  __shared__ float z_s[WAVES][kMaxTop];
+  __shared__ int count[kRouterLogits];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, t0 = 16 * blockIdx.x, n = E + shared;
+  // a lane's row of either operand and its eight of every 32 k
+  const uint16_t* a = h + (int64_t)min(t0 + (lane & 15), T - 1) * K + 8 * (lane >> 4);
+  const uint16_t* b[NT];
+#pragma unroll
+  for (int j = 0; j < NT; j++) b[j] = router + (int64_t)min(16 * j + (lane & 15), n - 1) * K + 8 * (lane >> 4);
+  dh::f32x4_t acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; j++) acc[j] = dh::f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 32 * wave; k0 < K; k0 += 32 * WAVES * AHEAD) {
+    dh::bf16x8_t fa[AHEAD], fb[AHEAD][NT];
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      const int at = min(k0 + 32 * WAVES * u, K - 32);
+      fa[u] = *reinterpret_cast<const dh::bf16x8_t*>(a + at);
+#pragma unroll
+      for (int j = 0; j < NT; j++) fb[u][j] = *reinterpret_cast<const dh::bf16x8_t*>(b[j] + at);
+    }
+    __builtin_amdgcn_sched_barrier(0);                 // (left alone the compiler requests each when it is due)
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      if (k0 + 32 * WAVES * u >= K) fa[u] = dh::bf16x8_t{};
+#pragma unroll
+      for (int j = 0; j < NT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[u], fb[u][j], acc[j], 0, 0, 0);
+    }
+  }
+  // accumulator element e of a lane: token 4 (lane / 16) + e, logit lane % 16
+#pragma unroll
+  for (int j = 0; j < NT; j++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) sums[wave][4 * (lane >> 4) + e][16 * j + (lane & 15)] = acc[j][e];
+  __syncthreads();
+  for (int i = tid; i < 16 * 16 * NT; i += 64 * WAVES) {
+    const int t = i / (16 * NT), c = i % (16 * NT);
+    float z = sums[0][t][c];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) z += sums[w][t][c];
+    sums[0][t][c] = z;                                 // (read by this thread alone)
+  }
+  if (tid < kRouterLogits) count[tid] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16 / WAVES; i++) {
+    const int t = (16 / WAVES) * wave + i;
+    if (t0 + t >= T) continue;
+    route_token(sums[0][t], t0 + t, E, top, shared, id_s[wave], z_s[wave], ids, weights, sg);
+    if (lane < top) slot[(int64_t)(t0 + t) * top + lane] = atomicAdd(&count[id_s[wave][lane]], 1);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  if (tid < E) counts[(int64_t)blockIdx.x * E + tid] = count[tid];
+}
+
 // One wave per token.
 __global__ __launch_bounds__(256) void experts_route_kernel(const float* __restrict__ z, int64_t ld_z, int T, int E, int top, int shared,
                                                             int* __restrict__ ids, float* __restrict__ weights, float* __restrict__ sg) {
   __shared__ int id_s[4][kMaxTop];
   __shared__ float z_s[4][kMaxTop];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, t = blockIdx.x * 4 + wave;
-  if (t >= T) return;
-  const float* row = z + (int64_t)t * ld_z;
-  choose(row, E, top, id_s[wave], z_s[wave]);
-  __builtin_amdgcn_wave_barrier();
-  if (lane < top) {
-    ids[(int64_t)t * top + lane] = id_s[wave][lane];
-    weights[(int64_t)t * top + lane] = sigmoid_f(z_s[wave][lane]);
+  const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
+  if (t < T) route_token(z + (int64_t)t * ld_z, t, E, top, shared, id_s[wave], z_s[wave], ids, weights, sg);
+}
+
+// Sorted places of the router kernel's choices, by workgroups of 64 tokens (four of its groups): every one of them adds up the groups' counts of every
+// expert, in all and in front of its own tokens.  A few short steps on many compute units (6124 choices of 16 experts 5.1 us, 160 choices 3.5), where
+// experts_sort_kernel takes one unit through all choices twice (9.9 and 5.5); it stays for more groups than a workgroup adds up in passing, more
+// experts, and choices that do not come in groups.
+constexpr int kPlacedGroups = 256;                     // 4096 tokens
+__global__ __launch_bounds__(256) void experts_place_kernel(const int* __restrict__ ids, const float* __restrict__ weights, const int* __restrict__ counts, int n, int top,
+                                                            int E, int groups, int tile_rows, int max_tiles, int* __restrict__ off, int* __restrict__ slot,
+                                                            int* __restrict__ row_token, float* __restrict__ row_weight, int* __restrict__ tiles) {
+  constexpr int GROUPS = 4, CHOICES = 16 * GROUPS, BATCH = 4;        // of a workgroup; CHOICES for each of a token's `top`
+  __shared__ int part[2][256];                         // sums of a thread's groups: all of them, and those in front
+  __shared__ int at[GROUPS][kRouterLogits];            // where a group's rows of an expert begin
+  const int tid = threadIdx.x, g0 = GROUPS * blockIdx.x, i0 = CHOICES * top * blockIdx.x, mine = min(CHOICES * top, n - i0);
+  const int shift = E <= 16 ? 4 : E <= 32 ? 5 : 6, parts = 256 >> shift, e = tid & ((1 << shift) - 1);
+  int id[BATCH], rank[BATCH];
+  float w[BATCH];
+  auto read = [&](int j) {
+#pragma unroll
+    for (int k = 0; k < BATCH; k++) {
+      const int i = i0 + min(j + 256 * k, mine - 1);
+      id[k] = ids[i];
+      rank[k] = slot[i];
+      w[k] = weights[i];
+    }
+  };
+  read(tid);
+  int all = 0, front = 0;
+#pragma unroll 4
+  for (int g = tid >> shift; g < groups; g += parts) {
+    const int c = e < E ? counts[g * E + e] : 0;
+    all += c;
+    front += g < g0 ? c : 0;
   }
-  if (shared && lane == 0) sg[t] = sigmoid_f(row[E]);
+  part[0][tid] = all;
+  part[1][tid] = front;
+  __syncthreads();
+  if (tid < 64) {                                      // lane: an expert
+    all = front = 0;
+    if (tid < E)
+      for (int k = 0; k < parts; k++) {
+        all += part[0][tid + (k << shift)];
+        front += part[1][tid + (k << shift)];
+      }
+    const int my_tiles = (all + tile_rows - 1) / tile_rows;
+    int rows = all, upto = my_tiles;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int a = __shfl_up(rows, o, 64), b = __shfl_up(upto, o, 64);
+      if (tid >= o) {
+        rows += a;
+        upto += b;
+      }
+    }
+    const int first = rows - all;
+    int next = first + front;
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+      at[g][tid] = next;
+      if (tid < E && g0 + g < groups) next += counts[(g0 + g) * E + tid];
+    }
+    if (blockIdx.x == 0) {
+      if (tid < E) off[tid] = first;
+      if (tid == E - 1) off[E] = n;
+      for (int k = 0; k < my_tiles; k++) {
+        tiles[2 * (upto - my_tiles + k)] = tid;
+        tiles[2 * (upto - my_tiles + k) + 1] = k * tile_rows;
+      }
+      for (int k = __shfl(upto, 63, 64) + tid; k < max_tiles; k += 64) tiles[2 * k] = -1;
+    }
+  }
+  __syncthreads();
+  for (int j = tid; j < mine; j += 256 * BATCH) {
+    if (j != tid) read(j);
+#pragma unroll
+    for (int k = 0; k < BATCH; k++) {
+      const int own = j + 256 * k, i = i0 + own;
+      if (own >= mine) break;
+      const int to = at[own / (16 * top)][id[k]] + rank[k];
+      slot[i] = to;
+      row_token[to] = i / top;
+      row_weight[to] = w[k];
+    }
+  }
 }
 
 // One workgroup: rows sorted by expert.  slot[i]: sorted place of choice i = token * top + k; row_token, row_weight by place.
@@ -452,11 +700,8 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace) {
   if (spec->K > 32768 || total > 32768) return dh::fail(1, "[%s] rows of %d and %lld elements: at most 32768 fit one workgroup", op, spec->K, (long long)total);
   float* z = static_cast<float*>(d_workspace);
   float* act = reinterpret_cast<float*>(static_cast<char*>(d_workspace) + up256((size_t)logits(spec) * 4));
-  if (int rc = dh_dense_gemv(d_x, spec->d_norm, spec->hidden, spec->eps, spec->d_router, spec->K, logits(spec), spec->K, 1.f, nullptr, nullptr, z,
-                             logits(spec), nullptr, DH_ACT_NONE))
-    return rc;
   StepArgs a{};
-  a.x = d_x; a.norm = spec->d_norm; a.z = z;
+  a.x = d_x; a.norm = spec->d_norm; a.z = z; a.router = static_cast<const uint16_t*>(spec->d_router);
   a.up = static_cast<const uint16_t*>(spec->d_up); a.down = static_cast<const uint16_t*>(spec->d_down);
   a.shared_up = static_cast<const uint16_t*>(spec->d_shared_up); a.shared_down = static_cast<const uint16_t*>(spec->d_shared_down);
   a.ls = spec->d_layer_scale; a.act = act; a.out = d_x;
@@ -464,7 +709,7 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace) {
   a.eps = spec->eps; a.limit = spec->limit; a.shared_limit = spec->shared_limit;
   static bool attr_set = false;
   if (!attr_set) {
-    for (const void* k : {reinterpret_cast<const void*>(experts_up_kernel<4>), reinterpret_cast<const void*>(experts_down_kernel<1, 8>)})
+    for (const void* k : {reinterpret_cast<const void*>(experts_up_kernel<4, 0>), reinterpret_cast<const void*>(experts_down_kernel<1, 8>)})
       DH_CHECK_HIP(op, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 32768 * 4));
     attr_set = true;
   }
@@ -475,7 +720,13 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace) {
   };
   int iters = 1;
   dim3 grid = plan(dh::ceil_div(total, 4), spec->K, &iters);
-  hipLaunchKernelGGL(experts_up_kernel<4>, grid, dim3(256), (size_t)spec->K * 4, dh::stream(), a, iters);
+  const bool with_router = logits(spec) <= 4 * kRouterRows && spec->K <= 2048;
+  if (!with_router)
+    if (int rc = dh_dense_gemv(d_x, spec->d_norm, spec->hidden, spec->eps, spec->d_router, spec->K, logits(spec), spec->K, 1.f, nullptr, nullptr, z,
+                               logits(spec), nullptr, DH_ACT_NONE))
+      return rc;
+  auto up = !with_router ? experts_up_kernel<4, 0> : spec->K <= 1024 ? experts_up_kernel<4, 2> : experts_up_kernel<4, 4>;
+  hipLaunchKernelGGL(up, grid, dim3(256), (size_t)spec->K * 4, dh::stream(), a, iters);
   DH_CHECK_LAUNCH(op);
   grid = plan(dh::ceil_div(spec->hidden, 4), total, &iters);
   hipLaunchKernelGGL((experts_down_kernel<1, 8>), grid, dim3(256), (size_t)total * 4, dh::stream(), a, iters);
@@ -519,15 +770,29 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   auto f32 = [&](size_t at) { return reinterpret_cast<float*>(w + at); };
   auto i32 = [&](size_t at) { return reinterpret_cast<int*>(w + at); };
   const int n = T * spec->top;
-  if (int rc = dh_dense_matmul(d_h, operand, spec->K, spec->d_router, spec->K, T, logits(spec), spec->K, 1.f, nullptr, nullptr, f32(p.z), p.ld_z,
-                               logits(spec), nullptr, 0, 0, DH_ACT_NONE))
-    return rc;
-  hipLaunchKernelGGL(experts_route_kernel, dim3((unsigned)dh::ceil_div(T, 4)), dim3(256), 0, dh::stream(), f32(p.z), (int64_t)p.ld_z, T, spec->experts,
-                     spec->top, spec->shared_ff > 0 ? 1 : 0, i32(p.ids), f32(p.weights), f32(p.sg));
-  DH_CHECK_LAUNCH(op);
-  hipLaunchKernelGGL(experts_sort_kernel, dim3(1), dim3(1024), 0, dh::stream(), i32(p.ids), f32(p.weights), n, spec->top, spec->experts, p.tile_rows,
-                     p.max_tiles, i32(p.off), i32(p.slot), i32(p.row_token), f32(p.row_weight), i32(p.tiles));
-  DH_CHECK_LAUNCH(op);
+  const int shared_logit = spec->shared_ff > 0 ? 1 : 0, groups = (int)dh::ceil_div(T, 16);
+  if (operand == DH_BF16 && logits(spec) <= kRouterLogits && groups <= kPlacedGroups) {
+    const int tiles = (int)dh::ceil_div(logits(spec), 16);
+    auto kern = tiles == 1 ? experts_router_kernel<1> : tiles == 2 ? experts_router_kernel<2> : experts_router_kernel<4>;
+    int* counts = i32(p.z);                            // (no logits go to memory)
+    hipLaunchKernelGGL(kern, dim3(groups), dim3(64 * (tiles <= 2 ? kRouterWaves<2> : kRouterWaves<4>)), 0, dh::stream(), static_cast<const uint16_t*>(d_h),
+                       static_cast<const uint16_t*>(spec->d_router), spec->K, T, spec->experts, spec->top, shared_logit, i32(p.ids), f32(p.weights), f32(p.sg),
+                       i32(p.slot), counts);
+    DH_CHECK_LAUNCH(op);
+    hipLaunchKernelGGL(experts_place_kernel, dim3((unsigned)dh::ceil_div(groups, 4)), dim3(256), 0, dh::stream(), i32(p.ids), f32(p.weights), counts, n, spec->top,
+                       spec->experts, groups, p.tile_rows, p.max_tiles, i32(p.off), i32(p.slot), i32(p.row_token), f32(p.row_weight), i32(p.tiles));
+    DH_CHECK_LAUNCH(op);
+  } else {
+    if (int rc = dh_dense_matmul(d_h, operand, spec->K, spec->d_router, spec->K, T, logits(spec), spec->K, 1.f, nullptr, nullptr, f32(p.z), p.ld_z,
+                                 logits(spec), nullptr, 0, 0, DH_ACT_NONE))
+      return rc;
+    hipLaunchKernelGGL(experts_route_kernel, dim3((unsigned)dh::ceil_div(T, 4)), dim3(256), 0, dh::stream(), f32(p.z), (int64_t)p.ld_z, T, spec->experts,
+                       spec->top, shared_logit, i32(p.ids), f32(p.weights), f32(p.sg));
+    DH_CHECK_LAUNCH(op);
+    hipLaunchKernelGGL(experts_sort_kernel, dim3(1), dim3(1024), 0, dh::stream(), i32(p.ids), f32(p.weights), n, spec->top, spec->experts, p.tile_rows,
+                       p.max_tiles, i32(p.off), i32(p.slot), i32(p.row_token), f32(p.row_weight), i32(p.tiles));
+    DH_CHECK_LAUNCH(op);
+  }
   const uint16_t *up = static_cast<const uint16_t*>(spec->d_up), *down = static_cast<const uint16_t*>(spec->d_down);
   const uint16_t *shared_up = static_cast<const uint16_t*>(spec->d_shared_up), *shared_down = static_cast<const uint16_t*>(spec->d_shared_down);
   const bool shared = spec->shared_ff > 0, up_pair = together(spec, operand, p, T, true), down_pair = together(spec, operand, p, T, false);

@@ -654,6 +654,65 @@ def test_products_that_share_a_launch_give_the_bits_of_those_apart(L, K, E, top,
     assert torch.equal(a[:both], b[:both]) and not torch.equal(a, x0[:T])
 
 
+@pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(1, 64, 1, 1, 64, 0), (16, 128, 16, 4, 64, 0), (17, 1088, 15, 2, 64, 64), (65, 192, 31, 3, 64, 64), (63, 2048, 19, 2, 64, 64),
+                                                    (200, 2112, 20, 3, 64, 64), (4096, 64, 33, 1, 64, 0), (4097, 64, 64, 32, 64, 0), (130, 64, 63, 32, 64, 64),
+                                                    (50, 64, 64, 2, 64, 64), (9, 4160, 7, 7, 64, 0)])
+def test_choices_of_portions_and_steps(L, T, K, E, top, ff, shared_ff):
+    """Tokens' experts, weights and places against 64 bits, in portions around sixteen tokens, four groups of them and the most that are placed in groups, of
+    up to 16, 32 and 64 logits and one more, and the same rows one at a time, with the logits made beside the first products (20 of at most 2048) and in
+    front of them.  Rows whose choice is closer than the logits' rounding (4096 products of 2^-24, of unit size together) are left out; an error in a choice, a weight or
+    a place is of the size of the row, and the activations' rounding to bf16 2^-9 of it."""
+    g = torch.Generator(device="cuda").manual_seed(T + K + E)
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    x0, ls, norm = torch.randn(T, K, generator=g, device="cuda"), torch.randn(K, generator=g, device="cuda"), 1.0 + 0.1 * torch.randn(K, generator=g, device="cuda")
+    router, up, down = w(E + (shared_ff > 0), K), w(E, 2 * ff, K), w(E, K, ff)
+    s_up, s_down = (w(2 * shared_ff, K), w(K, shared_ff)) if shared_ff else (None, None)
+    spec = capi.Experts(K, K, E, top, ff, shared_ff, 1e-5, 7.0, 1.5, norm.data_ptr(), ls.data_ptr(), router.data_ptr(), up.data_ptr(), down.data_ptr(),
+                        s_up.data_ptr() if shared_ff else None, s_down.data_ptr() if shared_ff else None)
+
+    def glu(z, limit, scale):
+        z = (z * scale).view(len(z), z.shape[1] // 64, 2, 32)
+        gate, lin = (z[:, :, i].reshape(len(z), z.shape[1] * z.shape[3]) for i in (0, 1))
+        gate = gate.clamp(max=limit)
+        return gate * torch.sigmoid(1.702 * gate) * (lin.clamp(-limit, limit) + 1)
+
+    def reference(hd):
+        z = hd @ router.double().T
+        best, ids = z[:, :E].topk(top, dim=1)
+        rest = z[:, :E].scatter(1, ids, -1e9).max(dim=1).values
+        want = torch.zeros_like(hd)
+        if shared_ff:
+            want += (glu(hd @ s_up.double().T, 1.5, 1.0) * torch.sigmoid(z[:, E:])) @ s_down.double().T
+        for e in range(E):
+            at, place = (ids == e).nonzero(as_tuple=True)
+            if len(at):
+                want[at] += glu(hd[at] @ up[e].double().T, 7.0, torch.sigmoid(best[at, place])[:, None]) @ down[e].double().T
+        return want * ls.double(), best[:, -1] - rest > 4096 * 2.0 ** -24
+
+    def check(x, hd, rows):
+        want, clear = reference(hd)
+        assert clear.double().mean() > 0.9
+        off = (x[rows].double() - x0[rows].double() - want).norm(dim=1) - 2.0 ** -8 * want.norm(dim=1) - 2.0 ** -23 * x0[rows].double().norm(dim=1)
+        assert (off[clear] <= 0).all(), int(off.argmax())
+    h = torch.randn(T, K, generator=g, device="cuda").to(torch.bfloat16)
+    ws = torch.full((L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T),), 255, dtype=torch.uint8, device="cuda")
+    x = x0.clone()
+    torch.cuda.synchronize()
+    capi.check(L.dh_experts_prefill(ctypes.byref(spec), h.data_ptr(), capi.BF16, x.data_ptr(), K, ws.data_ptr(), T))
+    capi.check(L.dh_sync())
+    check(x, h.double(), slice(0, T))
+    n = min(T, 20)
+    ws = torch.full((L.dh_experts_step_workspace_bytes(ctypes.byref(spec)),), 255, dtype=torch.uint8, device="cuda")
+    x = x0.clone()
+    torch.cuda.synchronize()
+    for t in range(n):
+        capi.check(L.dh_experts_step(ctypes.byref(spec), x[t].data_ptr(), ws.data_ptr()))
+    capi.check(L.dh_sync())
+    xd = x0[:n].double()
+    check(x, xd * torch.rsqrt(xd.square().mean(dim=1, keepdim=True) + 1e-5) * norm.double(), slice(0, n))
+    assert torch.equal(x[n:], x0[n:])
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

@@ -171,6 +171,8 @@ SIGNATURES = {
     "dh_experts_prefill_workspace_bytes": (_SZ, [ctypes.POINTER(Experts), _I, _I]),
     "dh_experts_prefill_layout": (_I, [ctypes.POINTER(Experts), _I, _I, _I, ctypes.POINTER(ctypes.c_int64)]),
     "dh_experts_prefill": (_I, [ctypes.POINTER(Experts), _P, _I, _P, _I, _P, _I]),
+    "dh_attn_spec_decode_for": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _P, _P, _I, _P, _I, _P, _I, ctypes.POINTER(_I)]),
+    "dh_dense_gemv_attn": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _P, _P]),
     "dh_attn_spec_decode": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _P, _P, _I, _P, _I, _P]),
     "dh_rmsnorm": (_I, [_P, _P, _I, _P, _I, _I, _F, _I, _P, _P, _P, _F]),
     "dh_rmsnorm_sandwich_pair": (_I, [_P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _F, _I]),

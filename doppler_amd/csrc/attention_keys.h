@@ -17,6 +17,7 @@ struct DynKeys {
   int causal, start_pos;        // start_pos < 0: the query sits at the last key, kv_start + kv_len - 1
   int sliding_window, kv_start, qkv;
   int one_per_cu;               // workgroups per kv head that fill the device once
+  int wide;                     // splits of a wide launch (wide_splits)
 };
 struct KeyRange {
   int kbeg, kend, nsplit, start_pos;
@@ -36,6 +37,12 @@ __host__ __device__ inline int splits_for(int one_per_cu, int nkeys) {
   const int chunks_each = (tiles + wgs - 1) / wgs;
   return (tiles + chunks_each - 1) / chunks_each;
 }
+// The same for workgroups of eight waves, which take 128 keys at a time: few splits, for a consumer that reads all of them in every workgroup.
+constexpr int kAttnWideKeys = 128;
+__host__ __device__ inline int wide_splits(int one_per_cu, int nkeys) {
+  const int tiles = nkeys > 0 ? (nkeys + kAttnWideKeys - 1) / kAttnWideKeys : 1;
+  return tiles < one_per_cu ? tiles : one_per_cu;
+}
 // The largest split count any key count up to max_keys can ask for: the grid of a launch whose key
 // count is only known on the device.
 __host__ __device__ inline int max_splits_upto(int one_per_cu, int max_keys) {
@@ -54,7 +61,7 @@ __device__ inline KeyRange dyn_key_range(const DynKeys& d) {
   r.kend = kv_len;
   if (!d.qkv && d.causal) r.kend = min(r.kend, r.start_pos - d.kv_start + 1);
   if (d.sliding_window > 0 && r.start_pos >= d.sliding_window) r.kbeg = max(0, r.start_pos - d.sliding_window + 1 - d.kv_start);
-  r.nsplit = r.kend > r.kbeg ? splits_for(d.one_per_cu, r.kend - r.kbeg) : 0;
+  r.nsplit = r.kend <= r.kbeg ? 0 : d.wide ? wide_splits(d.one_per_cu, r.kend - r.kbeg) : splits_for(d.one_per_cu, r.kend - r.kbeg);
   return r;
 }
 

@@ -1,10 +1,13 @@
 // Shared by the two files that serve dh_attn_spec (attention_spec.hip, attention_prefill.hip).
 #pragma once
+#include "attention_keys.h"
 #include "dh_common.h"
 
 namespace dh {
 // Host-side validation of a spec: 0, or fail().
 int attn_spec_check(const char* op, const dh_attn_spec* s);
+// The key ranges of a step whose key count is read on the device.
+DynKeys attn_spec_keys(const dh_attn_spec* s, const uint32_t* kv_len, int max_kv_len, bool wide);
 // Key elements that all heads of a token share (a rotated part beside every head's own): head keys are [D own | dim shared],
 // row r of the shared part lies ld elements behind row r - 1.  dim 0: none.
 struct SharedKey {

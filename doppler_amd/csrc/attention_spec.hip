@@ -2,7 +2,9 @@
 // of different sizes (dh_attn_spec): decode steps, and prefill for what the matrix-core kernels
 // (attention_prefill.hip) do not serve (heads of more than 128 elements, f32 caches with few queries).
 //
-// attn_spec_kernel: grid = (kv head x query-head group, key split, query token), four waves.  Keys advance in chunks;
+// attn_spec_kernel: grid = (kv head x query-head group, key split, query token), four waves, or eight where the product behind merges the splits
+// (left_to_product).  A chain of trips to memory: 32 heads of 128 over 1024 keys took 9.3 us with two integer divisions and eight 64-bit products in
+// front of its loads and lane steps through LDS behind, 7.2 without (16 heads on eight waves 8.1 and 6.6).  Keys advance in chunks;
 // every wave takes its own keys of a chunk and keeps its own online-softmax state, so the loop has no barrier.
 // L lanes share a key: lane (slot, piece) holds elements 8 piece .. 8 piece + 7 of its key's row and of its value
 // row.  Scores are f32 dot products summed over the L lanes with DPP steps, so the lane that multiplies a value piece
@@ -31,8 +33,9 @@ struct SpecArgs {
   void* V;
   float* O;             // f32 output rows (or null)
   uint16_t* O16;        // bf16 output rows
-  float* ws;            // [H][nsplit of the launch][VD + 2]
+  float* ws;            // [H][nsplit of the launch][VD] sums, then as many pairs (maximum, weight)
   int64_t ld_qkv, ld_out;
+  int groups;           // of query heads that share a kv head, GT each
   int H, Hkv, G, D, VD, value_dim;      // D: key elements of a head, its own and the shared ones
   int own_d;                            // its own
   const void* KS;                       // rows of the shared ones, ld_shared apart
@@ -104,20 +107,22 @@ __device__ __forceinline__ float value_factor(const float (&v)[8], int value_dim
   return 1.0f / sqrtf(ss / (float)value_dim + eps);
 }
 
-template <typename KV, int L, int GT>
-__global__ __launch_bounds__(256) void attn_spec_kernel(const SpecArgs a_in) {
-  SpecArgs a = a_in;
+template <typename KV, int L, int GT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_spec_kernel(const SpecArgs a) {
   constexpr int SLOTS = 64 / L;                        // keys a wave handles per pass
   constexpr int NP = L >= 16 ? 4 : L / 4;              // passes per chunk
   constexpr int WK = SLOTS * NP;                       // keys per wave and chunk
-  constexpr int CH = 4 * WK;                           // keys per chunk
-  __shared__ float o_lds[4][GT][8 * L];
-  __shared__ float ml_lds[4][GT][2];
+  constexpr int CH = WAVES * WK;                       // keys per chunk
+  __shared__ float o_lds[WAVES][GT][8 * L];
+  __shared__ float ml_lds[WAVES][GT][2];
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int slot = lane / L, piece = lane % L;
-  const int groups = (a.G + GT - 1) / GT;
-  const int kvh = blockIdx.x / groups, hg = blockIdx.x % groups;
+  int kvh = blockIdx.x, hg = 0;
+  if (a.groups > 1) {
+    kvh = blockIdx.x / a.groups;
+    hg = blockIdx.x - kvh * a.groups;
+  }
   const int h0 = kvh * a.G + hg * GT, gn = min(GT, a.G - hg * GT);
   const int split = blockIdx.y, t = blockIdx.z;
   const int ws_stride = a.nsplit;
@@ -138,19 +143,27 @@ __global__ __launch_bounds__(256) void attn_spec_kernel(const SpecArgs a_in) {
   const bool has_k = 8 * piece < a.D, has_v = 8 * piece < a.VD;
   const int nchunks = (kend - kbeg + CH - 1) / CH;
 
+  // (addresses: a 64-bit base a lane, once, and a 32-bit row times a 32-bit stride)
+  const char *kfrom = reinterpret_cast<const char*>(Kc + (int64_t)kbeg * kstride), *vfrom = reinterpret_cast<const char*>(Vc + (int64_t)kbeg * vstride);
+  const uint32_t kbytes = (uint32_t)(kstride * sizeof(KV)), vbytes = (uint32_t)(vstride * sizeof(KV));
+  const int last = kend - 1 - a.append - kbeg;         // of the rows in the cache: the appended one is not there yet
   Piece<KV> kn[NP], vn[NP], knew, vnew;
-  auto load = [&](int c) {
 #pragma unroll
-    for (int n = 0; n < NP; n++) {
-      // keys past the end repeat the last one; the appended one is not in the cache yet
-      const int key = min(kbeg + c * CH + wave * WK + n * SLOTS + slot, kend - 1 - a.append);
-      kn[n].zero();
-      vn[n].zero();
-      if (key >= kbeg) {
-        if (has_k) kn[n].load(Kc + key * kstride);
-        if (has_v) vn[n].load(Vc + key * vstride);
-      }
-    }
+  for (int n = 0; n < NP; n++) {
+    kn[n].zero();
+    vn[n].zero();
+  }
+  auto load = [&](int c) {
+    if (last < 0) return;
+    uint32_t r[NP];
+#pragma unroll
+    for (int n = 0; n < NP; n++) r[n] = (uint32_t)min(c * CH + wave * WK + n * SLOTS + slot, last);      // keys past the end repeat the last one
+    if (has_k)
+#pragma unroll
+      for (int n = 0; n < NP; n++) kn[n].load(reinterpret_cast<const KV*>(kfrom + (uint64_t)r[n] * kbytes));
+    if (has_v)
+#pragma unroll
+      for (int n = 0; n < NP; n++) vn[n].load(reinterpret_cast<const KV*>(vfrom + (uint64_t)r[n] * vbytes));
   };
   if (split < nchunks) load(split);
 
@@ -253,10 +266,10 @@ __global__ __launch_bounds__(256) void attn_spec_kernel(const SpecArgs a_in) {
     l[g] = dh::group_combine<L, 64>(l[g], dh::AddOp());
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      // the mirrors reverse the pieces of a row: they serve uniform groups only, so pieces are added lane by lane
+      // (the mirrors reverse the pieces of a row: they serve uniform groups only; a rotation by eight and the rows' swaps keep a lane's piece)
       float v = acc[g][i];
-#pragma unroll
-      for (int off = L; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+      if (L <= 8) v += dh::dpp_lane<0x128>(v);
+      v = dh::group_combine<(L < 16 ? 16 : L), 64>(v, dh::AddOp());
       if (slot == 0) o_lds[wave][g][8 * piece + i] = v;
     }
     if (lane == 0) {
@@ -265,14 +278,14 @@ __global__ __launch_bounds__(256) void attn_spec_kernel(const SpecArgs a_in) {
     }
   }
   __syncthreads();
-  for (int o = tid; o < gn * a.VD; o += 256) {
+  for (int o = tid; o < gn * a.VD; o += 64 * WAVES) {
     const int g = o / a.VD, d = o - g * a.VD, h = h0 + g;
     float M = ml_lds[0][g][0];
 #pragma unroll
-    for (int w = 1; w < 4; w++) M = fmaxf(M, ml_lds[w][g][0]);
+    for (int w = 1; w < WAVES; w++) M = fmaxf(M, ml_lds[w][g][0]);
     float num = 0.f, den = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
+    for (int w = 0; w < WAVES; w++) {
       const float f = __builtin_amdgcn_exp2f(ml_lds[w][g][0] - M);
       num = fmaf(f, o_lds[w][g][d], num);
       den = fmaf(f, ml_lds[w][g][1], den);
@@ -284,27 +297,25 @@ __global__ __launch_bounds__(256) void attn_spec_kernel(const SpecArgs a_in) {
       if (a.O16) a.O16[at] = dh::f32_to_bf16_bits(y);
       else a.O[at] = y;
     } else {
-      float* w = a.ws + ((int64_t)h * ws_stride + split) * (a.VD + 2);
-      w[d] = num;
-      if (d == 0) {
-        w[a.VD] = M;
-        w[a.VD + 1] = den;
-      }
+      const int64_t part = (int64_t)h * ws_stride + split;
+      a.ws[part * a.VD + d] = num;
+      if (d == 0) reinterpret_cast<float2*>(a.ws + (int64_t)a.H * ws_stride * a.VD)[part] = make_float2(M, den);
     }
   }
 }
 
 // One workgroup per query head: the splits' partial outputs, rescaled to their common maximum, gated.
 __global__ __launch_bounds__(256) void attn_spec_merge_kernel(const float* __restrict__ ws, float* __restrict__ O,
-                                                              const float* __restrict__ gate, int VD, int nsplit,
+                                                              const float* __restrict__ gate, int H, int VD, int nsplit,
                                                               const DynKeys dyn) {
   __shared__ float f_s[1024];
   __shared__ float red[4];
   const int h = blockIdx.x, tid = threadIdx.x, wave = tid >> 6;
-  const float* base = ws + (int64_t)h * nsplit * (VD + 2);
+  const float* base = ws + (int64_t)h * nsplit * VD;
+  const float2* pairs = reinterpret_cast<const float2*>(ws + (int64_t)H * nsplit * VD) + (int64_t)h * nsplit;
   if (dyn.kv_len_ptr != nullptr) nsplit = dh::dyn_key_range(dyn).nsplit;
   float M = -FLT_MAX;
-  for (int s = tid; s < nsplit; s += 256) M = fmaxf(M, base[(int64_t)s * (VD + 2) + VD]);
+  for (int s = tid; s < nsplit; s += 256) M = fmaxf(M, pairs[s].x);
   M = dh::group_combine<1, 64>(M, dh::MaxOp());
   if ((tid & 63) == 0) red[wave] = M;
   __syncthreads();
@@ -312,9 +323,10 @@ __global__ __launch_bounds__(256) void attn_spec_merge_kernel(const float* __res
   __syncthreads();
   float den = 0.f;
   for (int s = tid; s < nsplit; s += 256) {
-    const float f = __builtin_amdgcn_exp2f(base[(int64_t)s * (VD + 2) + VD] - M);
+    const float2 part = pairs[s];
+    const float f = __builtin_amdgcn_exp2f(part.x - M);
     f_s[s] = f;
-    den = fmaf(f, base[(int64_t)s * (VD + 2) + VD + 1], den);
+    den = fmaf(f, part.y, den);
   }
   den = dh::wave_sum_uniform(den);
   if ((tid & 63) == 0) red[wave] = den;
@@ -324,7 +336,7 @@ __global__ __launch_bounds__(256) void attn_spec_merge_kernel(const float* __res
   for (int d = tid; d < VD; d += 256) {
     float num = 0.f;
 #pragma unroll 8
-    for (int s = 0; s < nsplit; s++) num = fmaf(f_s[s], base[(int64_t)s * (VD + 2) + d], num);
+    for (int s = 0; s < nsplit; s++) num = fmaf(f_s[s], base[(int64_t)s * VD + d], num);
     O[(int64_t)h * VD + d] = num * inv;
   }
 }
@@ -357,12 +369,12 @@ typedef void (*SpecKernel)(const SpecArgs);
 template <typename KV, int L>
 SpecKernel pick_heads(int gt) {
   switch (gt) {
-    case 1: return attn_spec_kernel<KV, L, 1>;
-    case 2: return attn_spec_kernel<KV, L, 2>;
-    case 4: return attn_spec_kernel<KV, L, 4>;
+    case 1: return attn_spec_kernel<KV, L, 1, 4>;
+    case 2: return attn_spec_kernel<KV, L, 2, 4>;
+    case 4: return attn_spec_kernel<KV, L, 4, 4>;
     default:
-      if constexpr (L < 64) return attn_spec_kernel<KV, L, 8>;
-      else return attn_spec_kernel<KV, L, 4>;
+      if constexpr (L < 64) return attn_spec_kernel<KV, L, 8, 4>;
+      else return attn_spec_kernel<KV, L, 4, 4>;
   }
 }
 template <typename KV>
@@ -373,6 +385,13 @@ SpecKernel pick_lanes(int lanes, int gt) {
     case 32: return pick_heads<KV, 32>(gt);
     default: return pick_heads<KV, 64>(gt);
   }
+}
+// Eight waves: heads of up to 128 elements, one or two at once (more do not fit the registers), or null.
+template <typename KV>
+SpecKernel pick_wide(int lanes, int gt) {
+  if (lanes == 8) return gt == 1 ? attn_spec_kernel<KV, 8, 1, 8> : gt == 2 ? attn_spec_kernel<KV, 8, 2, 8> : nullptr;
+  if (lanes == 16) return gt == 1 ? attn_spec_kernel<KV, 16, 1, 8> : gt == 2 ? attn_spec_kernel<KV, 16, 2, 8> : nullptr;
+  return nullptr;
 }
 
 int lanes_for(int D, int VD) {
@@ -396,11 +415,66 @@ SpecArgs make_args(const dh_attn_spec* s, const float* qkv, void* K, void* V) {
   return a;
 }
 
-int launch_spec(const char* op, const dh_attn_spec* s, const SpecArgs& a, int T) {
-  const int lanes = lanes_for(a.D, a.VD), gt = heads_at_once(a.G, lanes);
-  const dim3 grid((unsigned)(s->Hkv * dh::ceil_div(a.G, gt)), (unsigned)a.nsplit, (unsigned)T);
-  SpecKernel k = s->cache_dtype == DH_F16 ? pick_lanes<__half>(lanes, gt) : pick_lanes<float>(lanes, gt);
-  hipLaunchKernelGGL(k, grid, dim3(256), 0, dh::stream(), a);
+SpecKernel wide_kernel(const dh_attn_spec* s) {
+  const int lanes = lanes_for(s->D, s->VD), gt = heads_at_once(s->H / s->Hkv, lanes);
+  return s->cache_dtype == DH_F16 ? pick_wide<__half>(lanes, gt) : pick_wide<float>(lanes, gt);
+}
+
+int launch_spec(const char* op, const dh_attn_spec* s, const SpecArgs& args, int T, SpecKernel wide = nullptr) {
+  const int lanes = lanes_for(args.D, args.VD), gt = heads_at_once(args.G, lanes);
+  SpecArgs a = args;
+  a.groups = (int)dh::ceil_div(a.G, gt);
+  const dim3 grid((unsigned)(s->Hkv * a.groups), (unsigned)a.nsplit, (unsigned)T);
+  SpecKernel k = wide ? wide : s->cache_dtype == DH_F16 ? pick_lanes<__half>(lanes, gt) : pick_lanes<float>(lanes, gt);
+  hipLaunchKernelGGL(k, grid, dim3(wide ? 512 : 256), 0, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+
+// Whether the splits are left to the product of `rows` rows that reads the output (dh_dense_gemv_attn): every workgroup of it reads all of them, from the same
+// lines at the same time, which has to cost less than a launch that merges them (3.8 us and 1.4 in front of the next).  So there are few: a workgroup of
+// eight waves takes 128 keys.  By the most keys a step can have, so that enqueued and captured steps split alike.
+// us, attention + merge + product / attention of wide workgroups + product: 16 heads of 128, 1024 keys, 2048 x 8192 7.7 + 3.9 + 9.3 / 6.6 + 10.8; 16 of 64 in
+// f32, 1024 x 4096 6.7 + 3.7 + 5.2 / 6.0 + 6.7.  With 16 splits of 64 keys (128 KB) the product takes 23, with four of 256 10.2 and the attention 10.5.
+constexpr int kMergedBytes = 64 << 10;
+bool left_to_product(const dh_attn_spec* s, int most_keys, int rows, const void* ws) {
+  const int one_per_cu = dh::attn_one_per_cu(dh::num_cus(), s->Hkv);
+  return rows > 0 && most_keys > dh::kAttnTileKeys && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 && wide_kernel(s) &&
+         (int64_t)4 * s->H * dh::wide_splits(one_per_cu, most_keys) * s->VD * std::max<int64_t>(1, dh::ceil_div(rows, 8 * dh::num_cus())) <= kMergedBytes;
+}
+
+int decode(const char* op, const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out, int pos,
+           const uint32_t* d_kv_len, int max_kv_len, void* d_workspace, int rows, int* left) {
+  DH_REQUIRE_INIT(op);
+  if (int rc = dh::attn_spec_check(op, spec)) return rc;
+  if (pos < 0) return dh::fail(1, "[%s] the position must be non-negative", op);
+  if (d_kv_len && max_kv_len <= 0) return dh::fail(1, "[%s] max_kv_len must be positive with the key count on the device", op);
+  if (!d_qkv || !d_cache_k || !d_cache_v || !d_out || !d_workspace) return dh::fail(1, "[%s] null pointer", op);
+  if ((reinterpret_cast<uintptr_t>(d_qkv) | reinterpret_cast<uintptr_t>(d_cache_k) | reinterpret_cast<uintptr_t>(d_cache_v)) & 15)
+    return dh::fail(1, "[%s] pointers must be 16-byte aligned", op);
+  SpecArgs a = make_args(spec, d_qkv, d_cache_k, d_cache_v);
+  a.O = d_out; a.ld_out = (int64_t)spec->H * spec->VD; a.ws = static_cast<float*>(d_workspace);
+  a.append = 1; a.pos0 = pos;
+  const int most = d_kv_len || max_kv_len > pos ? max_kv_len : pos + 1, most_keys = spec->window > 0 ? std::min(most, spec->window) : most;
+  const bool wide = left_to_product(spec, most_keys, rows, d_workspace);
+  const int one_per_cu = dh::attn_one_per_cu(dh::num_cus(), spec->Hkv);
+  if (d_kv_len) {
+    a.dyn = dh::attn_spec_keys(spec, d_kv_len, max_kv_len, wide);
+    a.nsplit = wide ? dh::wide_splits(one_per_cu, most_keys) : dh::max_splits_upto(one_per_cu, most_keys);
+  } else {
+    a.kend = pos + 1;
+    a.kbeg = spec->window > 0 ? std::max(0, pos - spec->window + 1) : 0;
+    a.nsplit = wide ? dh::wide_splits(one_per_cu, a.kend - a.kbeg) : dh::splits_for(one_per_cu, a.kend - a.kbeg);
+    a.direct = a.nsplit == 1;
+  }
+  if (int rc = launch_spec(op, spec, a, 1, wide ? wide_kernel(spec) : nullptr)) return rc;
+  if (a.direct) return 0;
+  if (wide) {
+    *left = a.nsplit;
+    return 0;
+  }
+  hipLaunchKernelGGL(attn_spec_merge_kernel, dim3(spec->H), dim3(256), 0, dh::stream(), a.ws, d_out,
+                     spec->gate_offset >= 0 ? d_qkv + spec->gate_offset : nullptr, spec->H, spec->VD, a.nsplit, a.dyn);
   DH_CHECK_LAUNCH(op);
   return 0;
 }
@@ -408,6 +482,13 @@ int launch_spec(const char* op, const dh_attn_spec* s, const SpecArgs& a, int T)
 }  // namespace
 
 namespace dh {
+
+DynKeys attn_spec_keys(const dh_attn_spec* s, const uint32_t* kv_len, int max_kv_len, bool wide) {
+  DynKeys d{};
+  d.kv_len_ptr = kv_len; d.max_kv_len = max_kv_len; d.causal = 1; d.start_pos = -1;
+  d.sliding_window = s->window; d.kv_start = 0; d.qkv = 1; d.one_per_cu = attn_one_per_cu(num_cus(), s->Hkv); d.wide = wide;
+  return d;
+}
 
 int attn_spec_check(const char* op, const dh_attn_spec* s) {
   if (!s) return fail(1, "[%s] null spec", op);
@@ -474,36 +555,15 @@ int dh_attn_spec_kv_write(const dh_attn_spec* spec, const float* d_qkv, void* d_
 
 int dh_attn_spec_decode(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
                         int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace) {
-  const char* op = "dh_attn_spec_decode";
-  DH_REQUIRE_INIT(op);
-  if (int rc = dh::attn_spec_check(op, spec)) return rc;
-  if (pos < 0) return dh::fail(1, "[%s] the position must be non-negative", op);
-  if (d_kv_len && max_kv_len <= 0) return dh::fail(1, "[%s] max_kv_len must be positive with the key count on the device", op);
-  if (!d_qkv || !d_cache_k || !d_cache_v || !d_out || !d_workspace) return dh::fail(1, "[%s] null pointer", op);
-  if ((reinterpret_cast<uintptr_t>(d_qkv) | reinterpret_cast<uintptr_t>(d_cache_k) | reinterpret_cast<uintptr_t>(d_cache_v)) & 15)
-    return dh::fail(1, "[%s] pointers must be 16-byte aligned", op);
-  SpecArgs a = make_args(spec, d_qkv, d_cache_k, d_cache_v);
-  a.O = d_out; a.ld_out = (int64_t)spec->H * spec->VD; a.ws = static_cast<float*>(d_workspace);
-  a.append = 1; a.pos0 = pos;
-  const int one_per_cu = dh::attn_one_per_cu(dh::num_cus(), spec->Hkv);
-  if (d_kv_len) {
-    a.dyn.kv_len_ptr = d_kv_len; a.dyn.max_kv_len = max_kv_len; a.dyn.causal = 1; a.dyn.start_pos = -1;
-    a.dyn.sliding_window = spec->window; a.dyn.kv_start = 0; a.dyn.qkv = 1; a.dyn.one_per_cu = one_per_cu;
-    const int keys = spec->window > 0 ? std::min(max_kv_len, spec->window) : max_kv_len;
-    a.nsplit = dh::max_splits_upto(one_per_cu, keys);
-  } else {
-    a.kend = pos + 1;
-    a.kbeg = spec->window > 0 ? std::max(0, pos - spec->window + 1) : 0;
-    a.nsplit = dh::splits_for(one_per_cu, a.kend - a.kbeg);
-    a.direct = a.nsplit == 1;
-  }
-  if (int rc = launch_spec(op, spec, a, 1)) return rc;
-  if (!a.direct) {
-    hipLaunchKernelGGL(attn_spec_merge_kernel, dim3(spec->H), dim3(256), 0, dh::stream(), a.ws, d_out,
-                       spec->gate_offset >= 0 ? d_qkv + spec->gate_offset : nullptr, spec->VD, a.nsplit, a.dyn);
-    DH_CHECK_LAUNCH(op);
-  }
-  return 0;
+  return decode("dh_attn_spec_decode", spec, d_qkv, d_cache_k, d_cache_v, d_out, pos, d_kv_len, max_kv_len, d_workspace, 0, nullptr);
+}
+
+int dh_attn_spec_decode_for(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
+                            int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace, int rows, int* left) {
+  const char* op = "dh_attn_spec_decode_for";
+  if (rows <= 0 || !left) return dh::fail(1, "[%s] a product of %d rows, or no place for the splits left", op, rows);
+  *left = 0;
+  return decode(op, spec, d_qkv, d_cache_k, d_cache_v, d_out, pos, d_kv_len, max_kv_len, d_workspace, rows, left);
 }
 
 }  // extern "C"

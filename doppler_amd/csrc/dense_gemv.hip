@@ -12,12 +12,16 @@
 // Outputs as in the multi-row product (dense_gemm.hip): columns below n_first with bias, column scale and residual, the rest
 // through an activation; or the argmax over all of them (output head).
 //
+// The ATTN form merges an attention's key splits (attention_spec.hip) into the front of the row: a launch less in front of the product.  A wave makes the
+// factors of a few heads' splits (up to 64: a lane each) from their maxima and weights, while the sums travel.
+//
 // The HEADS form reads the raw outputs of a layer's heads instead: each head divided by its root mean square, weighted and
 // multiplied by the sigmoid of an output gate on its way into LDS.
 #include <algorithm>
 #include <cfloat>
 
 #include "argmax_device.h"
+#include "attention_spec.h"
 #include "dense_device.h"
 
 namespace {
@@ -26,6 +30,7 @@ using dh::Cand;
 
 constexpr int kMaxK = 32768;
 constexpr int kMaxHeads = 256;        // of the HEADS form
+constexpr int kAttnFactors = 16384;   // bytes of LDS for the factors of an ATTN form
 
 struct GemvArgs {
   const float* x;
@@ -45,12 +50,19 @@ struct GemvArgs {
   int act;
   const float* gate;          // HEADS form: one number per element; norm_weight has one too, eps is the heads'
   int heads, head_padded, head_size;
+  const float* splits;        // ATTN form: [attn_heads][nsplit][attn_dim] sums, then as many pairs (maximum, weight); head_gate one number a head, or null
+  const float* head_gate;
+  int attn_heads, attn_dim, nsplit;
+  dh::DynKeys keys;           // how many of the splits there are, where only the device knows
   int iters;                  // rows per wave
   float* part_val;            // argmax: per-workgroup candidates
   uint32_t* part_idx;
 };
 
-template <int U, int WAVES, int BATCH, bool ARGMAX, bool HEADS>
+// What the row is made of.
+enum RowForm { kPlainRow, kHeadsRow, kAttnRow };
+
+template <int U, int WAVES, int BATCH, bool ARGMAX, int FORM>
 __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   extern __shared__ __align__(16) float4 planes[];      // [2][K / 8]
   __shared__ float red[WAVES];
@@ -87,7 +99,71 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
   };
 
   // ---- the activation row
-  if constexpr (HEADS) {
+  if constexpr (FORM == kAttnRow) {
+    constexpr int HB = 4, SB = 8;                        // heads a wave, splits a piece that are requested at once
+    extern __shared__ __align__(16) float4 planes_and_factors[];
+    float* const factors = reinterpret_cast<float*>(planes_and_factors) + a.K;      // [heads][nsplit]
+    float* const inverse = factors + a.attn_heads * a.nsplit;                       // [heads]
+    const int vp = a.attn_dim >> 2, live = a.attn_heads * vp, pieces = a.K >> 2, stride = a.nsplit;
+    const float4 *sums = reinterpret_cast<const float4*>(a.splits), *xg = reinterpret_cast<const float4*>(a.x);
+    const float2* pairs = reinterpret_cast<const float2*>(a.splits + (int64_t)a.attn_heads * stride * a.attn_dim);
+    const int nsplit = a.keys.kv_len_ptr ? dh::dyn_key_range(a.keys).nsplit : stride;
+    // a thread's first piece of the heads' part (its first splits) and of the rest, a wave's first heads, the first weights
+    float2 pair[HB];
+    float gate[HB];
+    auto head_of = [&](int j) { return min(wave + WAVES * j, a.attn_heads - 1); };
+    auto pair_of = [&](int h) { return pairs[h * stride + max(min(lane, nsplit - 1), 0)]; };
+#pragma unroll
+    for (int j = 0; j < HB; j++) {
+      pair[j] = pair_of(head_of(j));
+      gate[j] = a.head_gate ? a.head_gate[head_of(j)] : 0.f;
+    }
+    float4 part[SB], rest[BATCH];
+    auto part_of = [&](int i, int s) { return sums[((i / vp) * stride + max(min(s, nsplit - 1), 0)) * vp + i % vp]; };
+    const int turned = (int)((tid + 64 * blockIdx.x) % THREADS);         // workgroups begin at different heads: they read the same lines
+#pragma unroll
+    for (int s = 0; s < SB; s++) part[s] = part_of(min(turned, live - 1), s);
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) rest[b] = xg[min(live + tid + THREADS * b, pieces - 1)];
+    load(0, cur, cur_terms);
+    auto make_factors = [&](int h, const float2& p, float g) {
+      const bool there = lane < nsplit;
+      const float M = dh::group_combine<1, 64>(there ? p.x : -FLT_MAX, dh::MaxOp());
+      const float f = there ? __builtin_amdgcn_exp2f(p.x - M) : 0.f;
+      const float den = dh::wave_sum_uniform(there ? fmaf(f, p.y, 0.f) : 0.f);
+      if (there) factors[h * stride + lane] = f;
+      if (lane == 0) inverse[h] = (den > 0.f ? 1.0f / den : 0.f) * (a.head_gate ? 1.0f / (1.0f + expf(-g)) : 1.0f);
+    };
+#pragma unroll
+    for (int j = 0; j < HB; j++)
+      if (wave + WAVES * j < a.attn_heads) make_factors(wave + WAVES * j, pair[j], gate[j]);
+    for (int h = wave + WAVES * HB; h < a.attn_heads; h += WAVES) make_factors(h, pair_of(h), a.head_gate ? a.head_gate[h] : 0.f);
+#pragma unroll
+    for (int b = 0; b < BATCH; b++) {
+      const int i = live + tid + THREADS * b;
+      if (i < pieces) planes[(i & 1) * np + (i >> 1)] = rest[b];
+    }
+    for (int i = live + tid + THREADS * BATCH; i < pieces; i += THREADS) planes[(i & 1) * np + (i >> 1)] = xg[i];
+    __syncthreads();
+    for (int i = turned; i < live; i += THREADS) {
+      const int h = i / vp;
+      float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int s0 = 0; s0 < nsplit; s0 += SB) {
+        if (i != turned || s0 > 0) {
+#pragma unroll
+          for (int s = 0; s < SB; s++) part[s] = part_of(i, s0 + s);
+        }
+#pragma unroll
+        for (int s = 0; s < SB; s++) {
+          if (s0 + s >= nsplit) break;
+          const float f = factors[h * stride + s0 + s];
+          y.x = fmaf(f, part[s].x, y.x); y.y = fmaf(f, part[s].y, y.y); y.z = fmaf(f, part[s].z, y.z); y.w = fmaf(f, part[s].w, y.w);
+        }
+      }
+      const float inv = inverse[h];
+      planes[(i & 1) * np + (i >> 1)] = make_float4(y.x * inv, y.y * inv, y.z * inv, y.w * inv);
+    }
+  } else if constexpr (FORM == kHeadsRow) {
     // weighted and gated on the way in; the squares are summed by eight lanes (whole heads: their sizes are multiples of 32), then by
     // head, and the row in LDS is scaled last: one trip to memory
     __shared__ float inv_s[kMaxHeads];
@@ -223,26 +299,27 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(const GemvArgs a) {
 }
 
 // BATCH: 16-byte pieces of the row that a thread requests in front of the weights.
-template <int U, int WAVES, int BATCH, bool ARGMAX, bool HEADS>
+template <int U, int WAVES, int BATCH, bool ARGMAX, int FORM>
 int launch(const char* op, GemvArgs a, int max_grid, int* parts) {
-  auto kern = gemv_kernel<U, WAVES, BATCH, ARGMAX, HEADS>;
+  auto kern = gemv_kernel<U, WAVES, BATCH, ARGMAX, FORM>;
   static bool attr_set = false;
   if (!attr_set) {
     DH_CHECK_HIP(op, hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         kMaxK * 4));
+                                         kMaxK * 4 + (FORM == kAttnRow ? kAttnFactors : 0)));
     attr_set = true;
   }
   if (ARGMAX) max_grid = std::min(max_grid, dh::kMaxParts);
   const int64_t groups = dh::ceil_div(a.N, WAVES);
   a.iters = (int)std::max<int64_t>(1, dh::ceil_div(groups, max_grid));
   const int grid = (int)dh::ceil_div(groups, a.iters);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WAVES), (size_t)a.K * 4, dh::stream(), a);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WAVES), (size_t)a.K * 4 + (FORM == kAttnRow ? (size_t)4 * a.attn_heads * (a.nsplit + 1) : 0),
+                     dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   if (parts) *parts = grid;
   return 0;
 }
 
-template <int WAVES, bool ARGMAX, bool HEADS>
+template <int WAVES, bool ARGMAX, int FORM>
 int launch_loads(const char* op, const GemvArgs& a, int max_grid, int* parts) {
   // a stage as long as the row: lanes past the end load nothing and multiply zeros (a row of 1024 in a stage of 4096 leaves a quarter
   // of the bytes in flight).  Four waves a workgroup are few, so long rows get long stages there, and gated heads where a row is all a wave
@@ -251,16 +328,17 @@ int launch_loads(const char* op, const GemvArgs& a, int max_grid, int* parts) {
   // Pieces: what a row up to the stage's length has for a thread.  Requests for more of them stand in front of the weights for nothing (us, two or
   // four pieces / one: norm 1536 x 1024 4.2 -> 3.9, 3080 x 1024 4.8 -> 4.6, 2050 x 2048 5.1 -> 4.9, heads 1024 x 1024 4.4 -> 4.2); output heads, with
   // many rows a wave, go better with two (32000 x 2048 21.1 against 22.0).  Longer rows: as many as registers allow (four workgroups of eight waves: 64).
+  constexpr bool HEADS = FORM == kHeadsRow;
   constexpr int BATCH = HEADS || WAVES == 4 ? 4 : 2;
-  if (a.K <= 1024) return launch<2, WAVES, ARGMAX ? 2 : 1, ARGMAX, HEADS>(op, a, max_grid, parts);
-  if (a.K <= 2048) return launch<4, WAVES, ARGMAX || WAVES == 4 ? 2 : 1, ARGMAX, HEADS>(op, a, max_grid, parts);
-  if constexpr (WAVES == 4) return launch<8, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
+  if (a.K <= 1024) return launch<2, WAVES, ARGMAX ? 2 : 1, ARGMAX, FORM>(op, a, max_grid, parts);
+  if (a.K <= 2048) return launch<4, WAVES, ARGMAX || WAVES == 4 ? 2 : 1, ARGMAX, FORM>(op, a, max_grid, parts);
+  if constexpr (WAVES == 4) return launch<8, WAVES, BATCH, ARGMAX, FORM>(op, a, max_grid, parts);
   if constexpr (HEADS) {
-    if (WAVES == 8 ? a.N <= 8 * dh::num_cus() : a.K > 4096) return launch<8, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
+    if (WAVES == 8 ? a.N <= 8 * dh::num_cus() : a.K > 4096) return launch<8, WAVES, BATCH, ARGMAX, FORM>(op, a, max_grid, parts);
   } else {
-    if (a.K <= 3072) return launch<3, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
+    if (a.K <= 3072) return launch<3, WAVES, BATCH, ARGMAX, FORM>(op, a, max_grid, parts);
   }
-  return launch<4, WAVES, BATCH, ARGMAX, HEADS>(op, a, max_grid, parts);
+  return launch<4, WAVES, BATCH, ARGMAX, FORM>(op, a, max_grid, parts);
 }
 
 // Rows of each of its workgroups that the busiest compute unit goes through, with at most `per_cu` workgroups on every one.
@@ -274,17 +352,18 @@ int64_t busiest(int64_t N, int waves, int per_cu) {
 // two rounds of 321, or one of 642; x 2560 8.9 -> 6.9 us, x 8192 17.4 -> 16.7).  us, N x K with four waves and stages of 4096 (or two rows of 2048) -> now,
 // weights from memory: 10256 x 2048 10.6 -> 9.8, 5136 x 1024 5.9 -> 4.5, 18464 x 4096 28.0 -> 25.8 (5.9 TB/s), 2050 x 8192 9.8 -> 9.1; with
 // a norm 5136 x 1024 6.3 -> 5.1, 5136 x 2048 8.1 -> 7.1; heads 32000 x 2048 27.1 -> 25.6, 32000 x 1024 18.6 -> 16.9.  A launch alone is about 4 of them.
-template <bool ARGMAX, bool HEADS = false>
+template <bool ARGMAX, int FORM = kPlainRow>
 int dispatch(const char* op, const GemvArgs& a, int* parts) {
+  constexpr bool HEADS = FORM == kHeadsRow;
   const int cus = dh::num_cus();
-  if (a.K > 8192) return launch<8, 8, HEADS ? 4 : 2, ARGMAX, HEADS>(op, a, a.K <= 16384 ? 2 * cus : cus, parts);
+  if (a.K > 8192) return launch<8, 8, HEADS ? 4 : 2, ARGMAX, FORM>(op, a, a.K <= 16384 ? 2 * cus : cus, parts);
   if constexpr (HEADS)          // three rows are read to prepare one
-    if (a.N >= 16 * cus) return launch_loads<16, ARGMAX, HEADS>(op, a, cus, parts);
+    if (a.N >= 16 * cus) return launch_loads<16, ARGMAX, FORM>(op, a, cus, parts);
   if (a.N >= 8 * cus) {
     const bool four = !HEADS && (a.K <= 2048 || busiest(a.N, 8, 4) < busiest(a.N, 8, 2));
-    return launch_loads<8, ARGMAX, HEADS>(op, a, four ? 4 * cus : 2 * cus, parts);
+    return launch_loads<8, ARGMAX, FORM>(op, a, four ? 4 * cus : 2 * cus, parts);
   }
-  return launch_loads<4, ARGMAX, HEADS>(op, a, 4 * cus, parts);
+  return launch_loads<4, ARGMAX, FORM>(op, a, 4 * cus, parts);
 }
 
 int check(const char* op, const float* x, const float* norm_weight, int hidden, float eps, const void* W, int ldw, int N, int K) {
@@ -346,7 +425,27 @@ int dh_dense_gemv_heads(const float* d_x, const float* d_gate, const float* d_we
   GemvArgs a = make_args(d_x, d_weight, 0, eps, d_W, ldw, N, K, 1.f);
   a.gate = d_gate; a.heads = H; a.head_padded = padded; a.head_size = size;
   a.col_scale = d_col_scale; a.residual = d_residual; a.C = d_C;
-  return dispatch<false, true>(op, a, nullptr);
+  return dispatch<false, kHeadsRow>(op, a, nullptr);
+}
+
+int dh_dense_gemv_attn(const dh_attn_spec* spec, const float* d_qkv, const void* d_workspace, int left, const uint32_t* d_kv_len, int max_kv_len,
+                       const float* d_x, const void* d_W, int ldw, int N, int K, const float* d_residual, float* d_C) {
+  const char* op = "dh_dense_gemv_attn";
+  DH_REQUIRE_INIT(op);
+  if (int rc = dh::attn_spec_check(op, spec)) return rc;
+  if (int rc = check(op, d_x, nullptr, 0, 0.f, d_W, ldw, N, K)) return rc;
+  if ((int64_t)spec->H * spec->VD > K || left <= 0 || left > 64 || (int64_t)4 * spec->H * (left + 1) > kAttnFactors)
+    return dh::fail(1, "[%s] %d splits of %d heads of %d elements in a row of %d", op, left, spec->H, spec->VD, K);
+  if (!d_qkv || !d_workspace || !d_C) return dh::fail(1, "[%s] null pointer", op);
+  if (reinterpret_cast<uintptr_t>(d_workspace) & 15) return dh::fail(1, "[%s] the workspace must be 16-byte aligned", op);
+  if (d_kv_len && max_kv_len <= 0) return dh::fail(1, "[%s] max_kv_len must be positive with the key count on the device", op);
+  if (d_x == d_C) return dh::fail(1, "[%s] the output must not be the activation row", op);
+  GemvArgs a = make_args(d_x, nullptr, 0, 0.f, d_W, ldw, N, K, 1.f);
+  a.residual = d_residual; a.C = d_C;
+  a.splits = static_cast<const float*>(d_workspace); a.head_gate = spec->gate_offset >= 0 ? d_qkv + spec->gate_offset : nullptr;
+  a.attn_heads = spec->H; a.attn_dim = spec->VD; a.nsplit = left;
+  if (d_kv_len) a.keys = dh::attn_spec_keys(spec, d_kv_len, max_kv_len, true);
+  return dispatch<false, kAttnRow>(op, a, nullptr);
 }
 
 int dh_dense_lmhead_argmax(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,

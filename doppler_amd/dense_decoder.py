@@ -7,8 +7,8 @@ the residual, so a layer is two products:
     [ q | k | v | gate | up ] = W_in norm(x)         one stacked product; `up` leaves it through the activation
     x += W_out [ attention | act ]                   output and down projections side by side along k
 
-    decode    norm + W_in (one GEMV) -> attention (appends the key and value itself) [-> merge of the key splits]
-              -> W_out + residual (one GEMV): 3-4 launches per layer, f32 activations throughout
+    decode    norm + W_in (one GEMV) -> attention (appends the key and value itself) [-> merge of many key splits]
+              -> W_out + residual (one GEMV, which merges few key splits): 3-4 launches per layer, f32 activations throughout
     prefill   norm into the operand type -> W_in (matrix cores) -> KV write -> attention -> W_out + residual
 
 compute "bf16": matrix-core operands in bf16, f16 KV cache, everything else f32.  compute "f32": the same launches with
@@ -212,10 +212,18 @@ class DenseDecoder(DecoderBase):
                                g["n"], g["kx"], 1.0, d["bias"].data_ptr(), None, self.qkv.data_ptr(), g["n_first"], act, d["act"]))
         else:
             self._enqueue_in(d, self.x.data_ptr(), self._wide_row().data_ptr(), capi.F32, self.qkv.data_ptr(), act, 1, g["k2"])
-        ck(L.dh_attn_spec_decode(ctypes.byref(d["spec"]), self.qkv.data_ptr(), d["cache_k"].data_ptr(),
-                                 d["cache_v"].data_ptr(), mixed.data_ptr(), pos, kv_len, self.max_seq,
-                                 self.attn_ws.data_ptr()))
-        if g["k2"] <= GEMV_MAX_K:
+        # the product behind merges the key splits itself where that is faster than a launch
+        spec, one_row, left = ctypes.byref(d["spec"]), g["k2"] <= GEMV_MAX_K, ctypes.c_int(0)
+        step = (spec, self.qkv.data_ptr(), d["cache_k"].data_ptr(), d["cache_v"].data_ptr(), mixed.data_ptr(), pos, kv_len, self.max_seq,
+                self.attn_ws.data_ptr())
+        if one_row:
+            ck(L.dh_attn_spec_decode_for(*step, c["hidden"], ctypes.byref(left)))
+        else:
+            ck(L.dh_attn_spec_decode(*step))
+        if left.value:
+            ck(L.dh_dense_gemv_attn(spec, self.qkv.data_ptr(), self.attn_ws.data_ptr(), left.value, kv_len, self.max_seq, mixed.data_ptr(),
+                                    d["w_out"].data_ptr(), g["k2"], c["hidden"], g["k2"], self.x.data_ptr(), self.x.data_ptr()))
+        elif one_row:
             ck(L.dh_dense_gemv(mixed.data_ptr(), None, 0, 0.0, d["w_out"].data_ptr(), g["k2"], c["hidden"], g["k2"], 1.0,
                                None, self.x.data_ptr(), self.x.data_ptr(), c["hidden"], None, capi.ACT_NONE))
         else:

@@ -463,6 +463,14 @@ int dh_attn_spec_prefill(const dh_attn_spec* spec, const float* d_qkv, const voi
 size_t dh_attn_spec_workspace_bytes(int H, int VD, int max_kv_len);
 int dh_attn_spec_decode(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
                         int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace);
+/* The same in front of a product of `rows` rows whose activation row d_out begins: *left is 0 and d_out written, or, where that is faster, the number of
+ * key splits left in the workspace, which dh_dense_gemv_attn merges while it reads its row. */
+int dh_attn_spec_decode_for(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
+                            int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace, int rows, int* left);
+/* C[N] = W [attention | x[H * VD ..]] + residual for the splits a dh_attn_spec_decode_for with the same spec, row, workspace and key count has left
+ * (d_residual may be NULL or d_C; otherwise as dh_dense_gemv). */
+int dh_dense_gemv_attn(const dh_attn_spec* spec, const float* d_qkv, const void* d_workspace, int left, const uint32_t* d_kv_len, int max_kv_len,
+                       const float* d_x, const void* d_W, int ldw, int N, int K, const float* d_residual, float* d_C);
 /* dh_attn_spec_prefill for keys that end in elements all heads share: head h's key at row r is [cache_k[r][h] (D elements) |
  * shared_k + r * ld_shared (shared_dim elements)], its query D + shared_dim floats at h * (D + shared_dim). */
 int dh_attn_spec_prefill_shared(const dh_attn_spec* spec, const float* d_qkv, const void* d_cache_k, const void* d_shared_k,

@@ -777,6 +777,53 @@ def test_decode_with_the_key_count_on_the_device(L, window):
     assert torch.equal(a.kc, b.kc) and torch.equal(a.vc, b.vc)
 
 
+@pytest.mark.parametrize("cache", ["f16", "f32"])
+@pytest.mark.parametrize("H,G,d,e,window,n,rows,ff,merged", [(4, 2, 64, 48, 0, 700, 2050, 72, True), (2, 2, 24, 40, 129, 400, 30, 0, True), (16, 8, 128, 128, 1024, 1200, 2048, 64, True),
+                                                             (40, 40, 64, 24, 300, 400, 1030, 704, True), (6, 2, 24, 40, 300, 400, 100, 8, False), (4, 2, 64, 64, 64, 300, 100, 0, False),
+                                                             (32, 16, 128, 128, 1024, 1100, 4096, 0, False), (3, 3, 40, 264, 0, 300, 64, 0, False)])
+def test_splits_left_to_the_product_behind(L, H, G, d, e, window, n, rows, ff, merged, cache):
+    """A step's attention and the product that reads it, the key splits merged by the product or by a launch of their own, and with the key count on the
+    device: one to eight splits of 128 keys, heads of up to 16 lanes one and two at a time, part of a wave's heads and more than four, other activations
+    beside the heads'; more heads at once, few keys, many bytes of splits and long heads are merged as ever.  The same 32-bit sums in another order: 24
+    roundings of the terms' sizes."""
+    a, b, c = (Attn(L, H, G, d, e, window, cache, n=n, seed=31) for _ in range(3))
+    wide, K = H * a.VD, (H * a.VD + ff + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(n)
+    W, x = (torch.randn(rows, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16), torch.randn(rows, generator=g, device="cuda")
+    inputs = [torch.randn(K, generator=g, device="cuda")]
+    inputs += [inputs[0].clone(), inputs[0].clone()]
+    src, took, kv = a.rows(), [], torch.zeros(1, dtype=torch.int32, device="cuda")
+    for t in (a, b, c):
+        capi.check(L.dh_attn_spec_kv_write(ctypes.byref(t.spec), src.data_ptr(), t.kc.data_ptr(), t.vc.data_ptr(), n, 0))
+    for p in sorted({0, 1, 63, 64, 127, 128, 129, 255, 256, n // 2, n - 1}):
+        outs = []
+        for t, mixed, on_device in ((a, inputs[0], None), (b, inputs[1], False), (c, inputs[2], True)):
+            step = (ctypes.byref(t.spec), src.data_ptr() + 4 * t.ld * p, t.kc.data_ptr(), t.vc.data_ptr(), mixed.data_ptr())
+            left, y = ctypes.c_int(-1), x.clone()
+            kv.fill_(p + 1)
+            torch.cuda.synchronize()
+            where = (0, kv.data_ptr(), n) if on_device else (p, None, n)
+            if on_device is None:
+                capi.check(L.dh_attn_spec_decode(*step, *where, t.ws.data_ptr()))
+            else:
+                capi.check(L.dh_attn_spec_decode_for(*step, *where, t.ws.data_ptr(), rows, ctypes.byref(left)))
+                took.append(left.value)
+            if left.value > 0:
+                mixed[:wide] = float("nan")                    # what lies there is not read
+                torch.cuda.synchronize()
+                capi.check(L.dh_dense_gemv_attn(step[0], step[1], t.ws.data_ptr(), left.value, where[1], n, mixed.data_ptr(), W.data_ptr(), K, rows, K,
+                                                y.data_ptr(), y.data_ptr()))
+            else:
+                capi.check(L.dh_dense_gemv(mixed.data_ptr(), None, 0, 0.0, W.data_ptr(), K, rows, K, 1.0, None, y.data_ptr(), y.data_ptr(), rows, None, capi.ACT_NONE))
+            capi.check(L.dh_sync())
+            outs.append(y.double())
+        size = x.abs().double() + W.abs().double() @ inputs[0].abs().double()
+        for y in outs[1:]:
+            assert ((y - outs[0]).abs() <= 24 * 2.0 ** -24 * size).all(), p
+    assert (max(took) > 0) == merged
+    assert torch.equal(a.kc, b.kc) and torch.equal(a.vc, b.vc) and torch.equal(a.kc, c.kc)
+
+
 def test_prefill_output_in_bf16(L):
     a = Attn(L, 6, 2, 24, 40, 30, "f16", n=70, seed=13)
     f = a.run([70])

@@ -24,6 +24,7 @@ class DopplerHipError(RuntimeError):
 _P = ctypes.c_void_p
 _I = ctypes.c_int
 _I64 = ctypes.c_int64
+_U32 = ctypes.c_uint32
 _F = ctypes.c_float
 _SZ = ctypes.c_size_t
 
@@ -126,6 +127,10 @@ SIGNATURES = {
     "dh_f16w_matmul": (_I, [_P, _P, _P, _I, _I, _I, _F]),
     "dh_lmhead_argmax_workspace_bytes": (_SZ, [_I]),
     "dh_lmhead_argmax_f16": (_I, [_P, _P, _I, _I, _I64, _F, _P, _P, _I, _P]),
+    "dh_lmhead_argmax_f16_rmsnorm_read": (_I, [_P, _P, _F, _I, _P, _I, _I, _I64, _F, _P, _P, _I, _P, _P]),
+    "dh_dense_lmhead_argmax_read": (_I, [_P, _P, _I, _F, _P, _I, _I, _I, _F, _P, _P, _I, _P, _P]),
+    "dh_embed_sum_words": (_I, [_P, _U32, _U32, _U32, _P, _I, _P, _I64, _I64, _I64, _P, _I, _P, _I, _I, _I]),
+    "dh_gather_f16_words": (_I, [_P, _U32, _U32, _U32, _P, _P, _I, _I]),
     "dh_lmhead_argmax_f16_rmsnorm": (_I, [_P, _P, _F, _I, _P, _I, _I, _I64, _F, _P, _P, _I, _P]),
     "dh_attn_decode_workspace_bytes": (_SZ, [_I, _I, _I]),
     "dh_attn_prefill": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _F, _I]),

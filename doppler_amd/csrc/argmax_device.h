@@ -8,7 +8,7 @@ constexpr int kMaxParts = 2048;    // per-workgroup candidates a head leaves for
 
 // Folds `parts` candidates (one workgroup) and writes the token; ties go to the lowest index (lmhead.hip).
 int launch_argmax_final(const char* op, const float* part_val, const uint32_t* part_idx, int parts, uint32_t* token_out,
-                        int out_index);
+                        int out_index, uint32_t* also = nullptr);
 
 struct Cand {
   float v;

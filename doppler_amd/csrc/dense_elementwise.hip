@@ -15,25 +15,30 @@ struct EmbedArgs {
   int64_t buckets, mul_prev, mul_cur;
   int vocab, max_positions, ld_out, hidden, start_pos;
   const uint32_t* kv_len;
+  // ONE form: a token from the host, whose id, key count and the token before it go to `words` on the way
+  uint32_t* words;
+  uint32_t id, count, before;
+  int64_t bigram_row;
 };
 
 // Grid = (tokens, slices of 2048 columns): eight columns per thread with 16-byte loads where the rows are aligned for
 // them, else one column at a time.  Rows that do not exist (id or position out of range) count as zeros, so no id read on
 // the device can send a load outside the tables.
-template <bool VEC>
+__host__ __device__ inline int64_t bigram_row(uint32_t prev, uint32_t cur, int64_t mul_prev, int64_t mul_cur, int64_t buckets) {
+  const int64_t row = (int64_t)((uint64_t)(int64_t)prev * (uint64_t)mul_prev + (uint64_t)(int64_t)cur * (uint64_t)mul_cur) % buckets;
+  return row < 0 ? row + buckets : row;
+}
+template <bool VEC, bool ONE>
 __global__ __launch_bounds__(256) void embed_sum_kernel(const EmbedArgs a) {
   const int t = blockIdx.x;
-  const int64_t p = a.kv_len ? (int64_t)*a.kv_len - 1 : (int64_t)a.start_pos + t;
-  const uint32_t id = a.ids[t];
+  const int64_t p = !ONE && a.kv_len ? (int64_t)*a.kv_len - 1 : (int64_t)a.start_pos + t;
+  const uint32_t id = ONE ? a.id : a.ids[t];
+  if (ONE && blockIdx.y == 0 && threadIdx.x < 3) a.words[threadIdx.x] = threadIdx.x == 0 ? a.id : threadIdx.x == 1 ? a.count : a.before;
   const uint16_t* e = id < (uint32_t)a.vocab ? a.embed + (int64_t)id * a.hidden : nullptr;
   const uint16_t* b = nullptr;
   if (a.bigram) {
-    int64_t row = a.buckets;
-    if (p > 0) {
-      const uint32_t prev = t > 0 ? a.ids[t - 1] : *a.prev;
-      row = ((int64_t)prev * a.mul_prev + (int64_t)id * a.mul_cur) % a.buckets;
-      if (row < 0) row += a.buckets;
-    }
+    int64_t row = ONE ? a.bigram_row : a.buckets;
+    if (!ONE && p > 0) row = bigram_row(t > 0 ? a.ids[t - 1] : *a.prev, id, a.mul_prev, a.mul_cur, a.buckets);
     b = a.bigram + row * a.hidden;
   }
   const uint16_t* q = a.pos && p >= 0 && p < a.max_positions ? a.pos + p * a.hidden : nullptr;
@@ -123,35 +128,49 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
 
 extern "C" {
 
-int dh_embed_sum(const uint32_t* d_ids, int index_offset, const uint32_t* d_prev, const void* d_embed, int vocab,
-                 const void* d_bigram, int64_t buckets, int64_t mul_prev, int64_t mul_cur, const void* d_pos,
-                 int max_positions, float* d_out, int ld_out, int T, int hidden, int start_pos, const uint32_t* d_kv_len) {
-  const char* op = "dh_embed_sum";
+static int embed_sum(const char* op, EmbedArgs a, int T, bool one) {
   DH_REQUIRE_INIT(op);
-  if (T <= 0 || hidden <= 0 || vocab <= 0) return dh::fail(1, "[%s] Dimensions must be positive: T=%d, hidden=%d, vocab=%d", op, T, hidden, vocab);
-  if (index_offset < 0 || start_pos < 0) return dh::fail(1, "[%s] indexOffset and startPos must be non-negative", op);
-  if (ld_out < hidden) return dh::fail(1, "[%s] ld_out=%d is shorter than hidden=%d", op, ld_out, hidden);
-  if (!d_ids || !d_embed || !d_out) return dh::fail(1, "[%s] null pointer", op);
-  if (d_kv_len && T != 1) return dh::fail(1, "[%s] the device key count serves one token, got T=%d", op, T);
-  if (d_bigram && buckets <= 0) return dh::fail(1, "[%s] buckets must be positive", op);
-  if (d_bigram && !d_prev && (start_pos > 0 || d_kv_len)) return dh::fail(1, "[%s] the token before position %d is needed", op, start_pos);
-  if (d_pos && (max_positions <= 0 || (!d_kv_len && start_pos + T > max_positions)))
-    return dh::fail(1, "[%s] positions %d..%d are outside the table of %d", op, start_pos, start_pos + T - 1, max_positions);
+  if (T <= 0 || a.hidden <= 0 || a.vocab <= 0) return dh::fail(1, "[%s] Dimensions must be positive: T=%d, hidden=%d, vocab=%d", op, T, a.hidden, a.vocab);
+  if (a.start_pos < 0) return dh::fail(1, "[%s] indexOffset and startPos must be non-negative", op);
+  if (a.ld_out < a.hidden) return dh::fail(1, "[%s] ld_out=%d is shorter than hidden=%d", op, a.ld_out, a.hidden);
+  if (!(one ? (const void*)a.words : a.ids) || !a.embed || !a.out) return dh::fail(1, "[%s] null pointer", op);
+  if (a.kv_len && T != 1) return dh::fail(1, "[%s] the device key count serves one token, got T=%d", op, T);
+  if (a.bigram && a.buckets <= 0) return dh::fail(1, "[%s] buckets must be positive", op);
+  if (!one && a.bigram && !a.prev && (a.start_pos > 0 || a.kv_len)) return dh::fail(1, "[%s] the token before position %d is needed", op, a.start_pos);
+  if (a.pos && (a.max_positions <= 0 || (!a.kv_len && a.start_pos + T > a.max_positions)))
+    return dh::fail(1, "[%s] positions %d..%d are outside the table of %d", op, a.start_pos, a.start_pos + T - 1, a.max_positions);
+  if (one && a.bigram) a.bigram_row = a.start_pos > 0 ? bigram_row(a.before, a.id, a.mul_prev, a.mul_cur, a.buckets) : a.buckets;
+  const bool vec = a.hidden % 8 == 0 && a.ld_out % 4 == 0 &&
+                   ((reinterpret_cast<uintptr_t>(a.embed) | reinterpret_cast<uintptr_t>(a.bigram) | reinterpret_cast<uintptr_t>(a.pos) |
+                     reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
+  auto kern = vec ? one ? embed_sum_kernel<true, true> : embed_sum_kernel<true, false> : one ? embed_sum_kernel<false, true> : embed_sum_kernel<false, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)T, (unsigned)dh::ceil_div(a.hidden, 2048)), dim3(256), 0, dh::stream(), a);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+static EmbedArgs embed_args(const void* d_embed, int vocab, const void* d_bigram, int64_t buckets, int64_t mul_prev, int64_t mul_cur, const void* d_pos,
+                            int max_positions, float* d_out, int ld_out, int hidden, int start_pos) {
   EmbedArgs a{};
-  a.ids = d_ids + index_offset; a.prev = d_prev;
   a.embed = static_cast<const uint16_t*>(d_embed); a.bigram = static_cast<const uint16_t*>(d_bigram);
   a.pos = static_cast<const uint16_t*>(d_pos);
   a.out = d_out; a.buckets = buckets; a.mul_prev = mul_prev; a.mul_cur = mul_cur;
   a.vocab = vocab; a.max_positions = max_positions; a.ld_out = ld_out; a.hidden = hidden; a.start_pos = start_pos;
-  a.kv_len = d_kv_len;
-  const bool vec = hidden % 8 == 0 && ld_out % 4 == 0 &&
-                   ((reinterpret_cast<uintptr_t>(d_embed) | reinterpret_cast<uintptr_t>(d_bigram) | reinterpret_cast<uintptr_t>(d_pos) |
-                     reinterpret_cast<uintptr_t>(d_out)) & 15) == 0;
-  const dim3 grid((unsigned)T, (unsigned)dh::ceil_div(hidden, 2048));
-  if (vec) hipLaunchKernelGGL(embed_sum_kernel<true>, grid, dim3(256), 0, dh::stream(), a);
-  else hipLaunchKernelGGL(embed_sum_kernel<false>, grid, dim3(256), 0, dh::stream(), a);
-  DH_CHECK_LAUNCH(op);
-  return 0;
+  return a;
+}
+
+int dh_embed_sum(const uint32_t* d_ids, int index_offset, const uint32_t* d_prev, const void* d_embed, int vocab,
+                 const void* d_bigram, int64_t buckets, int64_t mul_prev, int64_t mul_cur, const void* d_pos,
+                 int max_positions, float* d_out, int ld_out, int T, int hidden, int start_pos, const uint32_t* d_kv_len) {
+  EmbedArgs a = embed_args(d_embed, vocab, d_bigram, buckets, mul_prev, mul_cur, d_pos, max_positions, d_out, ld_out, hidden, index_offset < 0 ? -1 : start_pos);
+  a.ids = d_ids ? d_ids + std::max(0, index_offset) : nullptr; a.prev = d_prev; a.kv_len = d_kv_len;
+  return embed_sum("dh_embed_sum", a, T, false);
+}
+
+int dh_embed_sum_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_embed, int vocab, const void* d_bigram, int64_t buckets,
+                       int64_t mul_prev, int64_t mul_cur, const void* d_pos, int max_positions, float* d_out, int ld_out, int hidden, int pos) {
+  EmbedArgs a = embed_args(d_embed, vocab, d_bigram, buckets, mul_prev, mul_cur, d_pos, max_positions, d_out, ld_out, hidden, pos);
+  a.words = d_words; a.id = id; a.count = kv_len; a.before = before;
+  return embed_sum("dh_embed_sum_words", a, 1, true);
 }
 
 int dh_rmsnorm_rows(const float* d_x, int ld_x, const uint32_t* d_rows, const float* d_weight, void* d_out, int out_dtype,

@@ -448,10 +448,9 @@ int dh_dense_gemv_attn(const dh_attn_spec* spec, const float* d_qkv, const void*
   return dispatch<false, kAttnRow>(op, a, nullptr);
 }
 
-int dh_dense_lmhead_argmax(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,
-                           int vocab, int K, float alpha, void* d_workspace, uint32_t* d_token_out, int output_index,
-                           float* d_logits_out) {
-  const char* op = "dh_dense_lmhead_argmax";
+static int lmhead_argmax(const char* op, const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,
+                         int vocab, int K, float alpha, void* d_workspace, uint32_t* d_token_out, int output_index,
+                         float* d_logits_out, uint32_t* also) {
   DH_REQUIRE_INIT(op);
   if (int rc = check(op, d_x, d_norm_weight, hidden, eps, d_W, ldw, vocab, K)) return rc;
   if (!d_workspace || !d_token_out) return dh::fail(1, "[%s] null pointer", op);
@@ -462,7 +461,25 @@ int dh_dense_lmhead_argmax(const float* d_x, const float* d_norm_weight, int hid
   a.part_idx = reinterpret_cast<uint32_t*>(static_cast<char*>(d_workspace) + (size_t)dh::kMaxParts * 4);
   int parts = 0;
   if (int rc = dispatch<true>(op, a, &parts)) return rc;
-  return dh::launch_argmax_final(op, a.part_val, a.part_idx, parts, d_token_out, output_index);
+  return dh::launch_argmax_final(op, a.part_val, a.part_idx, parts, d_token_out, output_index, also);
+}
+
+int dh_dense_lmhead_argmax(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,
+                           int vocab, int K, float alpha, void* d_workspace, uint32_t* d_token_out, int output_index,
+                           float* d_logits_out) {
+  return lmhead_argmax("dh_dense_lmhead_argmax", d_x, d_norm_weight, hidden, eps, d_W, ldw, vocab, K, alpha, d_workspace, d_token_out, output_index,
+                       d_logits_out, nullptr);
+}
+
+int dh_dense_lmhead_argmax_read(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,
+                                int vocab, int K, float alpha, void* d_workspace, uint32_t* d_token_out, int output_index,
+                                float* d_logits_out, uint32_t* host_token) {
+  const char* op = "dh_dense_lmhead_argmax_read";
+  DH_REQUIRE_INIT(op);
+  if (!host_token) return dh::fail(1, "[%s] no place for the token", op);
+  return dh::read_with(op, host_token, 1, [&](uint32_t* also) {
+    return lmhead_argmax(op, d_x, d_norm_weight, hidden, eps, d_W, ldw, vocab, K, alpha, d_workspace, d_token_out, output_index, d_logits_out, also);
+  });
 }
 
 }  // extern "C"

@@ -1,6 +1,7 @@
 // Shared host-side plumbing of libdopplerhip: error reporting, the single stream every op
 // enqueues on, and launch helpers.  gfx950 only.
 #pragma once
+#include <functional>
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -64,6 +65,9 @@ inline double tuning_double(const char* name, double dflt) {
   const char* e = tuning_env(name);
   return e ? atof(e) : dflt;
 }
+
+// Runs `enqueue` with the address of n words of pinned host memory that its launches write, waits for the stream and copies them out.
+int read_with(const char* op, uint32_t* host_dst, int n, const std::function<int(uint32_t*)>& enqueue);
 
 // ---- planning (dh_q4k_matmul_plan) ------------------------------------------------------------
 // While a plan is being made on this thread the dispatchers run as usual on the shape alone: ready()

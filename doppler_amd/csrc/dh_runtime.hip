@@ -144,6 +144,14 @@ float* widened_activations(size_t* bytes) {
   *bytes = g_widened_a ? kWidenedABytes : 0;
   return g_widened_a;
 }
+int read_with(const char* op, uint32_t* host_dst, int n, const std::function<int(uint32_t*)>& enqueue) {
+  if (g_capturing) return fail(1, "[%s] not possible while a graph is being captured (it waits for the stream)", op);
+  std::lock_guard<std::mutex> lock(g_words_mu);
+  if (int rc = enqueue(g_words)) return rc;
+  DH_CHECK_HIP(op, hipStreamSynchronize(g_stream));
+  for (int i = 0; i < n; i++) host_dst[i] = static_cast<volatile uint32_t*>(g_words)[i];
+  return check_kernel_status(op);
+}
 uint32_t* kernel_status_word() { return g_kstatus; }
 int check_kernel_status(const char* op) {
   if (!g_kstatus) return 0;
@@ -367,13 +375,11 @@ int dh_read_words(uint32_t* host_dst, const void* d_src, size_t offset, int n) {
   if (n < 1 || n > kMaxWords) return dh::fail(1, "[dh_read_words] 1..%d words, got %d", kMaxWords, n);
   if (!host_dst || !d_src) return dh::fail(1, "[dh_read_words] null pointer");
   if ((reinterpret_cast<uintptr_t>(d_src) + offset) & 3) return dh::fail(1, "[dh_read_words] the source must be 4-byte aligned");
-  std::lock_guard<std::mutex> lock(g_words_mu);
-  hipLaunchKernelGGL(read_words_kernel, dim3(1), dim3(64), 0, g_stream,
-                     reinterpret_cast<const uint32_t*>(static_cast<const char*>(d_src) + offset), g_words, n);
-  DH_CHECK_LAUNCH("dh_read_words");
-  DH_CHECK_HIP("dh_read_words", hipStreamSynchronize(g_stream));
-  for (int i = 0; i < n; i++) host_dst[i] = static_cast<volatile uint32_t*>(g_words)[i];
-  return dh::check_kernel_status("dh_read_words");
+  return dh::read_with("dh_read_words", host_dst, n, [&](uint32_t* pinned) {
+    hipLaunchKernelGGL(read_words_kernel, dim3(1), dim3(64), 0, g_stream, reinterpret_cast<const uint32_t*>(static_cast<const char*>(d_src) + offset), pinned, n);
+    DH_CHECK_LAUNCH("dh_read_words");
+    return 0;
+  });
 }
 
 int dh_event_synchronize(void* ev) {

@@ -415,6 +415,14 @@ __global__ __launch_bounds__(256) void gather_f16_kernel(const uint32_t* __restr
   out[i] = id >= vocab ? 0.0f : __half2float(table[(int64_t)id * hidden + d]);
 }
 
+// The row of one token from the host, whose id, key count and the token before it go to `words` on the way.
+__global__ __launch_bounds__(256) void gather_f16_words_kernel(uint32_t* words, uint32_t id, uint32_t kv_len, uint32_t before, const __half* __restrict__ table,
+                                                               float* __restrict__ out, int hidden, uint32_t vocab) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < 3) words[i] = i == 0 ? id : i == 1 ? kv_len : before;
+  if (i < hidden) out[i] = id >= vocab ? 0.0f : __half2float(table[(int64_t)id * hidden + i]);
+}
+
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }
 __device__ __forceinline__ float gelu_f(float x) {
   const float inner = 0.7978845608f * (x + 0.044715f * x * x * x);
@@ -820,6 +828,17 @@ int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int 
   const int64_t total = (int64_t)T * hidden;
   hipLaunchKernelGGL(gather_f16_kernel, dim3(grid_for(total)), dim3(256), 0, dh::stream(), d_ids,
                      static_cast<const __half*>(d_table), d_out, total, hidden, (uint32_t)vocab, index_offset);
+  DH_CHECK_LAUNCH(op);
+  return 0;
+}
+
+int dh_gather_f16_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_table, float* d_out, int hidden, int vocab) {
+  const char* op = "dh_gather_f16_words";
+  DH_REQUIRE_INIT(op);
+  if (hidden <= 0 || vocab <= 0) return dh::fail(1, "[%s] hiddenSize/vocabSize must be positive", op);
+  if (!d_words || !d_table || !d_out) return dh::fail(1, "[%s] null pointer", op);
+  hipLaunchKernelGGL(gather_f16_words_kernel, dim3((unsigned)dh::ceil_div(std::max(hidden, 3), 256)), dim3(256), 0, dh::stream(), d_words, id, kv_len, before,
+                     static_cast<const __half*>(d_table), d_out, hidden, (uint32_t)vocab);
   DH_CHECK_LAUNCH(op);
   return 0;
 }

@@ -11,6 +11,7 @@
 #include <cfloat>
 
 #include "argmax_device.h"
+#include "dense_device.h"
 #include "dh_common.h"
 
 namespace {
@@ -239,18 +240,53 @@ __global__ __launch_bounds__(256) void argmax_scan_kernel(const float* __restric
 }
 
 // Phase 2: one workgroup folds the per-workgroup candidates and writes the token.
+__device__ __forceinline__ uint32_t wave_lowest(uint32_t v) {
+  auto dpp = [](uint32_t x, auto ctrl) { return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, decltype(ctrl)::value, 0xF, 0xF, false); };
+  v = min(v, dpp(v, std::integral_constant<int, 0xB1>{}));      // quad_perm 1,0,3,2 and 2,3,0,1, then mirrors
+  v = min(v, dpp(v, std::integral_constant<int, 0x4E>{}));
+  v = min(v, dpp(v, std::integral_constant<int, 0x141>{}));
+  v = min(v, dpp(v, std::integral_constant<int, 0x140>{}));
+  auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = min((uint32_t)a[0], (uint32_t)a[1]);
+  auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return min((uint32_t)b[0], (uint32_t)b[1]);
+}
+// One trip to memory (all of a thread's candidates are requested together) and lane steps without LDS: 4.6 -> 4.0 us for 1000 candidates, the write to the host among them.
+// also: pinned host memory that gets the token too, or null.
 __global__ __launch_bounds__(256) void argmax_final_kernel(const float* __restrict__ part_val,
                                                            const uint32_t* __restrict__ part_idx, int parts,
-                                                           uint32_t* __restrict__ token_out, int out_index) {
+                                                           uint32_t* __restrict__ token_out, int out_index, uint32_t* also) {
+  constexpr int PER = dh::kMaxParts / 256;
   __shared__ float sv[4];
   __shared__ uint32_t si[4];
+  float v[PER];
+  uint32_t id[PER];
+#pragma unroll
+  for (int k = 0; k < PER; k++) {                        // (past the end the last one again)
+    const int i = min((int)threadIdx.x + 256 * k, parts - 1);
+    v[k] = part_val[i];
+    id[k] = part_idx[i];
+  }
   Cand best{-3.402823e+38f, 0xFFFFFFFFu};
-  for (int i = threadIdx.x; i < parts; i += 256)
-    if (beats(part_val[i], part_idx[i], best.v, best.i)) { best.v = part_val[i]; best.i = part_idx[i]; }
-  const Cand c = block_best_256(best, sv, si);
+#pragma unroll
+  for (int k = 0; k < PER; k++)
+    if (beats(v[k], id[k], best.v, best.i)) { best.v = v[k]; best.i = id[k]; }
+  const float most = dh::group_combine<1, 64>(best.v, dh::MaxOp());
+  const uint32_t first = wave_lowest(best.v == most ? best.i : 0xFFFFFFFFu);
+  if ((threadIdx.x & 63) == 0) {
+    sv[threadIdx.x >> 6] = most;
+    si[threadIdx.x >> 6] = first;
+  }
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  Cand c{sv[0], si[0]};
+  for (int w = 1; w < 4; w++)
+    if (beats(sv[w], si[w], c.v, c.i)) { c.v = sv[w]; c.i = si[w]; }
   // nothing beat the neutral start (every logit <= -3.4e38, NaN, or masked): index 0, as the
   // reference kernel's (NEG_INF, 0) start does
-  if (threadIdx.x == 0) token_out[out_index] = c.i == 0xFFFFFFFFu ? 0u : c.i;
+  const uint32_t token = c.i == 0xFFFFFFFFu ? 0u : c.i;
+  token_out[out_index] = token;
+  if (also) __hip_atomic_store(also, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <int MT, bool ARGMAX>
@@ -288,8 +324,8 @@ int check_f16w_shape(const char* op, int M, int N, int K) {
 
 namespace dh {
 int launch_argmax_final(const char* op, const float* part_val, const uint32_t* part_idx, int parts, uint32_t* token_out,
-                        int out_index) {
-  hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(256), 0, stream(), part_val, part_idx, parts, token_out, out_index);
+                        int out_index, uint32_t* also) {
+  hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(256), 0, stream(), part_val, part_idx, parts, token_out, out_index, also);
   DH_CHECK_LAUNCH(op);
   return 0;
 }
@@ -331,7 +367,7 @@ size_t dh_lmhead_argmax_workspace_bytes(int vocab) {
 
 static int lmhead_argmax_impl(const char* op, const float* d_h, const float* d_norm_weight, float eps, int weight_offset,
                               const void* d_E, int vocab, int hidden, int64_t pad_token_id, float logit_softcap,
-                              void* d_workspace, uint32_t* d_token_out, int output_index, float* d_logits_out) {
+                              void* d_workspace, uint32_t* d_token_out, int output_index, float* d_logits_out, uint32_t* also = nullptr) {
   DH_REQUIRE_INIT(op);
   if (int rc = check_f16w_shape(op, 1, vocab, hidden)) return rc;
   if (!d_h || !d_E || !d_workspace || !d_token_out) return dh::fail(1, "[%s] null pointer", op);
@@ -353,10 +389,7 @@ static int lmhead_argmax_impl(const char* op, const float* d_h, const float* d_n
   a.norm_weight = d_norm_weight; a.norm_eps = eps; a.norm_weight_offset = weight_offset;
   int parts = 0;
   if (int rc = launch_gemv<1, true>(a, &parts, op)) return rc;
-  hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(256), 0, dh::stream(), a.part_val, a.part_idx, parts,
-                     d_token_out, output_index);
-  DH_CHECK_LAUNCH(op);
-  return 0;
+  return dh::launch_argmax_final(op, a.part_val, a.part_idx, parts, d_token_out, output_index, also);
 }
 
 int dh_lmhead_argmax_f16(const float* d_h, const void* d_E, int vocab, int hidden, int64_t pad_token_id,
@@ -375,6 +408,18 @@ int dh_lmhead_argmax_f16_rmsnorm(const float* d_h, const float* d_norm_weight, f
                             d_workspace, d_token_out, output_index, d_logits_out);
 }
 
+int dh_lmhead_argmax_f16_rmsnorm_read(const float* d_h, const float* d_norm_weight, float eps, int weight_offset,
+                                      const void* d_E, int vocab, int hidden, int64_t pad_token_id, float logit_softcap,
+                                      void* d_workspace, uint32_t* d_token_out, int output_index, float* d_logits_out, uint32_t* host_token) {
+  const char* op = "dh_lmhead_argmax_f16_rmsnorm_read";
+  DH_REQUIRE_INIT(op);
+  if (!d_norm_weight || !host_token) return dh::fail(1, "[%s] null norm weight, or no place for the token", op);
+  return dh::read_with(op, host_token, 1, [&](uint32_t* also) {
+    return lmhead_argmax_impl(op, d_h, d_norm_weight, eps, weight_offset, d_E, vocab, hidden, pad_token_id, logit_softcap, d_workspace, d_token_out,
+                              output_index, d_logits_out, also);
+  });
+}
+
 size_t dh_argmax_workspace_bytes(void) { return (size_t)kMaxParts * 8; }
 
 int dh_argmax(const float* d_logits, int vocab, int64_t pad_token_id, float logit_softcap, void* d_workspace,
@@ -390,10 +435,7 @@ int dh_argmax(const float* d_logits, int vocab, int64_t pad_token_id, float logi
   hipLaunchKernelGGL(argmax_scan_kernel, dim3(parts), dim3(256), 0, dh::stream(), d_logits, vocab, pad_token_id,
                      logit_softcap, pv, pi);
   DH_CHECK_LAUNCH(op);
-  hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(256), 0, dh::stream(), pv, pi, parts, d_token_out,
-                     output_index);
-  DH_CHECK_LAUNCH(op);
-  return 0;
+  return dh::launch_argmax_final(op, pv, pi, parts, d_token_out, output_index);
 }
 
 }  // extern "C"

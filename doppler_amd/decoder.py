@@ -45,6 +45,7 @@ class DecoderBase:
 
     A model provides
         _enqueue_embed(ids_ptr, prev_ptr, pos, device_kv_len)   one token's embedding into the step's residual row
+        _enqueue_embed_words(words, pos)                        the same of a token from the host, whose words go to self.ids on the way
         _enqueue_stack(pos, device_kv_len)                      its layers
         _step_row()                                             the step's final residual row (device address)
         _enqueue_head(row_ptr, out_index, logits_ptr)           output head of a row: token (and logits)
@@ -102,12 +103,14 @@ class DecoderBase:
         return int(self.history[pos - 1]) if pos > 0 else 0
 
     def enqueue_step(self, pos, want_logits=False, from_device_token=False, in_index=0, out_index=0,
-                     device_kv_len=False):
+                     device_kv_len=False, host_words=None, read=False):
         """Enqueue one decode step for the token id in self.ids[0] (or, when from_device_token,
         the argmax an earlier step left in self.token[in_index]) at position `pos`; the new
         token goes to self.token[out_index].  No host synchronisation.  device_kv_len: the
         attention kernels take the key count (position + 1) from self.ids[1] instead of `pos`, so
-        that the enqueued step, captured into a graph, serves every later position as it is."""
+        that the enqueued step, captured into a graph, serves every later position as it is.
+        host_words (see step_words): the token comes from there instead of self.ids[0], and those words go to self.ids on the
+        way.  read: waits and returns the new token (out_index 0)."""
         if not 0 <= pos < self.max_seq:
             # the ops take no cache capacity: a position past the caches would write K/V and read
             # the position tables out of bounds
@@ -119,9 +122,27 @@ class DecoderBase:
         else:
             ids_ptr, prev_ptr = self.ids.data_ptr(), self.ids.data_ptr() + 8
         self._input_ptr = ids_ptr
-        self._enqueue_embed(ids_ptr, prev_ptr, pos, device_kv_len)
+        if host_words is None:
+            self._enqueue_embed(ids_ptr, prev_ptr, pos, device_kv_len)
+        else:
+            self._enqueue_embed_words(host_words, pos)
         self._enqueue_stack(pos, device_kv_len)
-        self._enqueue_head(self._step_row(), out_index, self.logits.data_ptr() if want_logits else None)
+        logits_ptr = self.logits.data_ptr() if want_logits else None
+        if read:
+            return self._head_token(self._step_row(), logits_ptr)
+        self._enqueue_head(self._step_row(), out_index, logits_ptr)
+
+    def _head_token(self, row_ptr, logits_ptr):
+        """The output head of a row, and its token on the host."""
+        self._enqueue_head(row_ptr, 0, logits_ptr)
+        return self.read_token()
+
+    def step_words(self, token, pos):
+        """What a step takes from the host besides its position: token id, key count (none: captured steps alone read it) and the token
+        before it."""
+        words = int(token), 0, self._before(pos)
+        self._remember(pos, token)
+        return words
 
     def set_token(self, token, kv_len=None, pos=None):
         """Token id of the step (and with it the key count of a captured step and the token
@@ -151,12 +172,14 @@ class DecoderBase:
         the finiteness status beside it when the guard is on).
         sampling = dict(temperature, topK, randomSeed): top-k temperature sampling from the
         step's logits instead of the fused greedy argmax."""
-        self.set_token(token, pos=pos)
+        words = self.step_words(token, pos)
+        if sampling is None and not self.finiteness_guard:
+            return self.enqueue_step(pos, want_logits, host_words=words, read=True)
         out_index = 0
         if self.finiteness_guard:
             self._reset_finiteness()
             out_index = self.TOKEN_RING - 1
-        self.enqueue_step(pos, want_logits or sampling is not None, out_index=out_index)
+        self.enqueue_step(pos, want_logits or sampling is not None, out_index=out_index, host_words=words)
         if sampling is not None:
             self._enqueue_sample(sampling, out_index)
         if not self.finiteness_guard:
@@ -346,9 +369,10 @@ class DecoderBase:
             return np.stack(out) if out else np.empty((0, self.cfg["vocab"]), np.float32)
         # logits of the last prompt token only
         last = base + (ids.size - 1) * stride * 4
-        self._enqueue_head(last, 0, self.logits.data_ptr() if (want_logits or sampling is not None) else None)
-        if sampling is not None:
-            self._enqueue_sample(sampling)
+        if sampling is None:
+            return self._head_token(last, self.logits.data_ptr() if want_logits else None)
+        self._enqueue_head(last, 0, self.logits.data_ptr())
+        self._enqueue_sample(sampling)
         return self.read_token()
 
     def _logit_rows(self, base, stride, rows):
@@ -372,8 +396,7 @@ class DecoderBase:
             raise ValueError("token ids must be in 0..%d" % (self.cfg["vocab"] - 1))
         pos = self.length
         if len(tokens) == 1 and all(w == 0 for w in want):
-            self.set_token(tokens[0], pos=pos)
-            self.enqueue_step(pos, want_logits=len(want) > 0)
+            self.enqueue_step(pos, want_logits=len(want) > 0, host_words=self.step_words(tokens[0], pos))
             out = np.tile(self.read_logits(), (len(want), 1)) if len(want) else np.empty((0, self.cfg["vocab"]), np.float32)
         else:
             out = self.prefill(tokens, pos, chunk=chunk, want=list(want))
@@ -514,8 +537,21 @@ class HipDecoder(DecoderBase):
         capi.check(self.L.dh_gather_f16(ids_ptr, self.embed.data_ptr(), self.x.data_ptr(), 1, self.cfg["hidden"],
                                         self.cfg["vocab"], 0))
 
+    def _enqueue_embed_words(self, words, pos):
+        capi.check(self.L.dh_gather_f16_words(self.ids.data_ptr(), *words, self.embed.data_ptr(), self.x.data_ptr(), self.cfg["hidden"],
+                                              self.cfg["vocab"]))
+
     def _step_row(self):
         return self.x.data_ptr()
+
+    def _head_token(self, row_ptr, logits_ptr):
+        c = self.cfg
+        if c["hidden"] > 4096 or c["hidden"] % 8:
+            return super()._head_token(row_ptr, logits_ptr)
+        capi.check(self.L.dh_lmhead_argmax_f16_rmsnorm_read(row_ptr, self.final_norm.data_ptr(), c["eps"], 0, self.embed.data_ptr(), c["vocab"],
+                                                            c["hidden"], -1, 0.0, self.lm_ws.data_ptr(), self.token.data_ptr(), 0, logits_ptr,
+                                                            self._host_token.ctypes.data))
+        return int(self._host_token[0])
 
     def _enqueue_stack(self, pos, device_kv_len):
         if self.chain_gemvs and self.fuse_norm and not self.finiteness_guard:

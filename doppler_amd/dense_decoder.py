@@ -188,8 +188,20 @@ class DenseDecoder(DecoderBase):
         capi.check(self.L.dh_embed_sum(ids_ptr, 0, prev_ptr, *self._embed_args(), self.x.data_ptr(), self.kx, 1,
                                        self.cfg["hidden"], pos, self.ids.data_ptr() + 4 if device_kv_len else None))
 
+    def _enqueue_embed_words(self, words, pos):
+        capi.check(self.L.dh_embed_sum_words(self.ids.data_ptr(), *words, *self._embed_args(), self.x.data_ptr(), self.kx, self.cfg["hidden"], pos))
+
     def _step_row(self):
         return self.x.data_ptr()
+
+    def _head_token(self, row_ptr, logits_ptr):
+        if self.kx > GEMV_MAX_K:
+            return super()._head_token(row_ptr, logits_ptr)
+        c = self.cfg
+        capi.check(self.L.dh_dense_lmhead_argmax_read(row_ptr, self.final_norm.data_ptr(), c["hidden"], c["eps"], self.head.data_ptr(), self.kx,
+                                                      c["vocab"], self.kx, c["logit_scale"], self.lm_ws.data_ptr(), self.token.data_ptr(), 0,
+                                                      logits_ptr, self._host_token.ctypes.data))
+        return int(self._host_token[0])
 
     def _enqueue_stack(self, pos, device_kv_len):
         L, c, ck = self.L, self.cfg, capi.check

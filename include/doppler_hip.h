@@ -278,6 +278,11 @@ int dh_lmhead_argmax_f16_rmsnorm(const float* d_h, const float* d_norm_weight, f
                                  const void* d_E, int vocab, int hidden, int64_t pad_token_id,
                                  float logit_softcap, void* d_workspace, uint32_t* d_token_out,
                                  int output_index, float* d_logits_out);
+/* The same, and the token brought to the host as dh_read_words would (it waits, reports and refuses like that), without a launch for it. */
+int dh_lmhead_argmax_f16_rmsnorm_read(const float* d_h, const float* d_norm_weight, float eps, int weight_offset,
+                                      const void* d_E, int vocab, int hidden, int64_t pad_token_id,
+                                      float logit_softcap, void* d_workspace, uint32_t* d_token_out,
+                                      int output_index, float* d_logits_out, uint32_t* host_token);
 
 /* ---- attention ----
  * Decode attention of one query token over an f16 KV cache.  Replaces
@@ -413,6 +418,10 @@ int dh_dense_gemv_heads(const float* d_x, const float* d_gate, const float* d_we
 int dh_dense_lmhead_argmax(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,
                            int vocab, int K, float alpha, void* d_workspace, uint32_t* d_token_out, int output_index,
                            float* d_logits_out);
+/* ... and the token to the host, as dh_lmhead_argmax_f16_rmsnorm_read. */
+int dh_dense_lmhead_argmax_read(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw,
+                                int vocab, int K, float alpha, void* d_workspace, uint32_t* d_token_out, int output_index,
+                                float* d_logits_out, uint32_t* host_token);
 
 /* out[t] = embed[id_t] + bigram[row_t] + pos[p_t], bf16 tables of `hidden` columns, f32 sum; p_t = start_pos + t, or
  * with d_kv_len (key count on the device, T = 1) *d_kv_len - 1.  row_t = (id_{t-1} * mul_prev + id_t * mul_cur) mod
@@ -422,6 +431,12 @@ int dh_dense_lmhead_argmax(const float* d_x, const float* d_norm_weight, int hid
 int dh_embed_sum(const uint32_t* d_ids, int index_offset, const uint32_t* d_prev, const void* d_embed, int vocab,
                  const void* d_bigram, int64_t buckets, int64_t mul_prev, int64_t mul_cur, const void* d_pos,
                  int max_positions, float* d_out, int ld_out, int T, int hidden, int start_pos, const uint32_t* d_kv_len);
+
+/* One token from the host: dh_set_words of (id, kv_len, before) to d_words and dh_embed_sum of id at position pos, `before` the token in front of it, in
+ * one launch. */
+int dh_embed_sum_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_embed, int vocab, const void* d_bigram,
+                       int64_t buckets, int64_t mul_prev, int64_t mul_cur, const void* d_pos, int max_positions, float* d_out, int ld_out,
+                       int hidden, int pos);
 
 /* RMSNorm of n rows into the operand type of the product that reads them: out[r] = norm(x[rows ? rows[r] : r]),
  * columns hidden .. ld_out - 1 zero.  out_dtype DH_BF16 or DH_F32. */
@@ -660,6 +675,9 @@ int dh_scale(const float* d_in, float* d_out, int64_t n, float scale);
  * (gather_f16.wgsl:35-66). */
 int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int T, int hidden,
                   int vocab, int index_offset);
+
+/* One token from the host: dh_set_words of (id, kv_len, before) to d_words and the row of id, in one launch. */
+int dh_gather_f16_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_table, float* d_out, int hidden, int vocab);
 
 /* out = clamp(act(gate) * up).  Replaces runSiLU with `gate` (src/gpu/kernels/silu.js:95,
  * silu.wgsl:100-106) and runGeLU with `gate` (gelu.wgsl:60-65). */

@@ -33,3 +33,61 @@ def test_words_refusals():
     for n, p, off, message in ((0, d.data_ptr(), 0, "words"), (17, d.data_ptr(), 0, "words"), (1, None, 0, "null"), (1, d.data_ptr(), 2, "aligned")):
         assert L.dh_set_words(p, off, w.ctypes.data, n) == 1 and message in L.dh_last_error().decode()
         assert L.dh_read_words(w.ctypes.data, p, off, n) == 1 and message in L.dh_last_error().decode()
+
+
+@pytest.mark.parametrize("hidden,buckets,pos", [(8, 0, 0), (13, 11, 0), (2056, 11, 5), (64, 1 << 40, 3)])
+def test_words_and_embedding_in_one_launch(hidden, buckets, pos):
+    """The words and rows that two launches leave, aligned and not, in one and two slices of columns, with the row the token before it picks."""
+    L = capi.init(torch.cuda.current_device())
+    vocab, positions, g = 50, 9, torch.Generator(device="cuda").manual_seed(hidden)
+    table = lambda rows, t: torch.randn(rows, hidden, generator=g, device="cuda").to(t)
+    embed, bigram, places, half = table(vocab, torch.bfloat16), table(12, torch.bfloat16), table(positions, torch.bfloat16), table(vocab, torch.float16)
+    mul = (3, 5) if buckets < 100 else (0, 1 << 39)                                  # (row 0 or half of the buckets: only the first exists here)
+    ld = (hidden + 63) // 64 * 64
+    for token in (0, 49, 50, 4) if buckets < 100 else (4, 48):
+        words = np.array([token, 0, 7], np.uint32)
+        args = (embed.data_ptr(), vocab, bigram.data_ptr() if buckets else None, buckets, *mul, places.data_ptr(), positions)
+        ids, got = (torch.full((4,), 9, dtype=torch.int32, device="cuda") for _ in range(2))
+        outs = [torch.full((ld,), 3.0, device="cuda") for _ in range(4)]
+        torch.cuda.synchronize()
+        capi.check(L.dh_set_words(ids.data_ptr(), 0, words.ctypes.data, 3))
+        capi.check(L.dh_embed_sum(ids.data_ptr(), 0, ids.data_ptr() + 8, *args, outs[0].data_ptr(), ld, 1, hidden, pos, None))
+        capi.check(L.dh_embed_sum_words(got.data_ptr(), token, 0, 7, *args, outs[1].data_ptr(), ld, hidden, pos))
+        capi.check(L.dh_sync())
+        assert torch.equal(outs[0], outs[1]) and torch.equal(ids, got)
+        got.fill_(9)
+        torch.cuda.synchronize()
+        capi.check(L.dh_gather_f16(ids.data_ptr(), half.data_ptr(), outs[2].data_ptr(), 1, hidden, vocab, 0))
+        capi.check(L.dh_gather_f16_words(got.data_ptr(), token, 0, 7, half.data_ptr(), outs[3].data_ptr(), hidden, vocab))
+        capi.check(L.dh_sync())
+        assert torch.equal(outs[2], outs[3]) and torch.equal(ids, got)
+
+
+@pytest.mark.parametrize("vocab", [1, 7, 2048, 2049, 32000, 70001])
+def test_token_of_a_head_on_the_host(vocab):
+    """The token both heads leave on the device and bring to the host is their logits' first maximum, with one to all of the candidates a final
+    reduction takes, among equal ones in other waves and threads, and 0 where no logit is a number."""
+    L = capi.init(torch.cuda.current_device())
+    K, g = 64, torch.Generator(device="cuda").manual_seed(vocab)
+    row, ones, eps = torch.randn(K, generator=g, device="cuda"), torch.ones(K, device="cuda"), 1e-6
+    ws = torch.zeros(int(L.dh_lmhead_argmax_workspace_bytes(vocab)), dtype=torch.uint8, device="cuda")
+    token, logits, host = torch.zeros(2, dtype=torch.int32, device="cuda"), torch.zeros(vocab, device="cuda"), np.zeros(1, np.uint32)
+    for case in range(4):
+        W = torch.randn(vocab, K, generator=g, device="cuda")
+        if case in (1, 2) and vocab > 1:                                       # equal rows, the largest by far
+            at = torch.randint(0, vocab, (5,), generator=g, device="cuda") if case == 1 else torch.tensor([vocab - 1, vocab // 2], device="cuda")
+            W[at] = 20.0 * row
+        if case == 3:
+            W[:] = float("nan")
+        for dtype in (torch.float16, torch.bfloat16):
+            E = W.to(dtype)
+            token.fill_(-1)
+            torch.cuda.synchronize()
+            if dtype == torch.float16:
+                capi.check(L.dh_lmhead_argmax_f16_rmsnorm_read(row.data_ptr(), ones.data_ptr(), eps, 0, E.data_ptr(), vocab, K, -1, 0.0, ws.data_ptr(),
+                                                               token.data_ptr(), 1, logits.data_ptr(), host.ctypes.data))
+            else:
+                capi.check(L.dh_dense_lmhead_argmax_read(row.data_ptr(), ones.data_ptr(), K, eps, E.data_ptr(), K, vocab, K, 1.0, ws.data_ptr(),
+                                                         token.data_ptr(), 1, logits.data_ptr(), host.ctypes.data))
+            want = 0 if case == 3 else int((logits == logits.max()).nonzero()[0])
+            assert token.tolist() == [-1, want] and host[0] == want, (case, dtype)

@@ -128,6 +128,7 @@ SIGNATURES = {
     "dh_lmhead_argmax_workspace_bytes": (_SZ, [_I]),
     "dh_lmhead_argmax_f16": (_I, [_P, _P, _I, _I, _I64, _F, _P, _P, _I, _P]),
     "dh_lmhead_argmax_f16_rmsnorm_read": (_I, [_P, _P, _F, _I, _P, _I, _I, _I64, _F, _P, _P, _I, _P, _P]),
+    "dh_dense_matmul_normed": (_I, [_P, _I, _I, _P, _I, _I, _I, _I, _P, _P, _P, _I, _P, _F, _P, _I, _I]),
     "dh_dense_lmhead_argmax_read": (_I, [_P, _P, _I, _F, _P, _I, _I, _I, _F, _P, _P, _I, _P, _P]),
     "dh_embed_sum_words": (_I, [_P, _U32, _U32, _U32, _P, _I, _P, _I64, _I64, _I64, _P, _I, _P, _I, _I, _I]),
     "dh_gather_f16_words": (_I, [_P, _U32, _U32, _U32, _P, _P, _I, _I]),
@@ -175,6 +176,7 @@ SIGNATURES = {
     "dh_experts_step": (_I, [ctypes.POINTER(Experts), _P, _P]),
     "dh_experts_prefill_workspace_bytes": (_SZ, [ctypes.POINTER(Experts), _I, _I]),
     "dh_experts_prefill_layout": (_I, [ctypes.POINTER(Experts), _I, _I, _I, ctypes.POINTER(ctypes.c_int64)]),
+    "dh_experts_prefill_normed": (_I, [ctypes.POINTER(Experts), _P, _I, _P, _I, _P, _I, _P, _F, _P, _I]),
     "dh_experts_prefill": (_I, [ctypes.POINTER(Experts), _P, _I, _P, _I, _P, _I]),
     "dh_attn_spec_decode_for": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _P, _P, _I, _P, _I, _P, _I, ctypes.POINTER(_I)]),
     "dh_dense_gemv_attn": (_I, [ctypes.POINTER(AttnSpec), _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _P, _P]),

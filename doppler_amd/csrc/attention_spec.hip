@@ -345,9 +345,10 @@ __global__ __launch_bounds__(256) void attn_spec_merge_kernel(const float* __res
 template <typename KV>
 __global__ __launch_bounds__(256) void kv_write_kernel(const SpecArgs a, int T) {
   const int lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (item >= (int64_t)T * a.Hkv) return;              // wave-uniform
-  const int t = (int)(item / a.Hkv), kvh = (int)(item % a.Hkv);
+  // (token and head of a wave's item without a division of 64 bits, which took longer than the rest in front of the loads)
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), item = 4 * blockIdx.x + wave;
+  const int t = (int)(item / (uint32_t)a.Hkv), kvh = (int)(item - (uint32_t)t * (uint32_t)a.Hkv);
+  if (t >= T) return;                                  // wave-uniform
   const float* row = a.qkv + (int64_t)t * a.ld_qkv;
   float k[8] = {}, v[8] = {};
   if (8 * lane < a.D) load8(row + a.k_off + (int64_t)kvh * a.D + 8 * lane, k);

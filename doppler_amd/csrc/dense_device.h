@@ -61,6 +61,46 @@ __device__ __forceinline__ float group_combine(float v, Op op) {
   return v;
 }
 
+// A row that 256 threads hold, four elements at 4 (tid + 1024 j / 4) each (zeros past `hidden`, a multiple of 4 and at most 8192), over its root mean square and
+// times w, in the operand type of the product that reads it; columns hidden .. ld_out - 1 zero.
+constexpr int kNormPieces = 8;
+template <bool BF16>
+__device__ __forceinline__ void store_normed_row(const float4 (&xv)[kNormPieces], int hidden, const float* __restrict__ w, float eps, float* red, void* __restrict__ out,
+                                                 int64_t base, int ld_out) {
+  const int tid = threadIdx.x;
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < kNormPieces; j++) {
+    ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss);
+    ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss);
+  }
+  ss = wave_sum_uniform(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)hidden + eps);
+  auto put = [&](int i, float v) {
+    if (BF16) static_cast<uint16_t*>(out)[base + i] = f32_to_bf16_bits(v);
+    else static_cast<float*>(out)[base + i] = v;
+  };
+#pragma unroll
+  for (int j = 0; j < kNormPieces; j++) {
+    const int i = 4 * (tid + 256 * j);
+    if (i >= hidden) continue;
+    const float4 wv = *reinterpret_cast<const float4*>(w + i);
+    const float y[4] = {xv[j].x * inv * wv.x, xv[j].y * inv * wv.y, xv[j].z * inv * wv.z, xv[j].w * inv * wv.w};
+    if (BF16 && (ld_out & 3) == 0) {
+      uint2 two;
+      two.x = (uint32_t)f32_to_bf16_bits(y[0]) | ((uint32_t)f32_to_bf16_bits(y[1]) << 16);
+      two.y = (uint32_t)f32_to_bf16_bits(y[2]) | ((uint32_t)f32_to_bf16_bits(y[3]) << 16);
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + base + i) = two;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++) put(i + e, y[e]);
+    }
+  }
+  for (int i = hidden + tid; i < ld_out; i += 256) put(i, 0.f);
+}
+
 // Workgroup index -> tile index such that each of the eight XCDs (which the hardware deals workgroups to in turn)
 // gets a contiguous run of tiles and its L2 sees their shared operands.
 __device__ __forceinline__ int xcd_contiguous(int id, int total) {

@@ -78,49 +78,28 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
   __shared__ float red[4];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const float* xr = x + (int64_t)(rows ? rows[blockIdx.x] : blockIdx.x) * ld_x;
-  const bool vec = (ld_x & 3) == 0 && (hidden & 3) == 0 && hidden <= 8192;
-  float4 xv[8];
-  float ss = 0.f;
-  if (vec) {
+  const int64_t base = (int64_t)blockIdx.x * ld_out;
+  if ((ld_x & 3) == 0 && (hidden & 3) == 0 && hidden <= 1024 * dh::kNormPieces) {
+    float4 xv[dh::kNormPieces];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < dh::kNormPieces; j++) {
       const int i = 4 * (tid + 256 * j);
       xv[j] = i < hidden ? *reinterpret_cast<const float4*>(xr + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-      ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss);
-      ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss);
     }
-  } else {
-    for (int i = tid; i < hidden; i += 256) ss = fmaf(xr[i], xr[i], ss);
+    dh::store_normed_row<BF16>(xv, hidden, w, eps, red, out, base, ld_out);
+    return;
   }
+  float ss = 0.f;
+  for (int i = tid; i < hidden; i += 256) ss = fmaf(xr[i], xr[i], ss);
   ss = dh::wave_sum_uniform(ss);
   if (lane == 0) red[wave] = ss;
   __syncthreads();
   const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)hidden + eps);
-  const int64_t base = (int64_t)blockIdx.x * ld_out;
   auto put = [&](int i, float v) {
     if (BF16) static_cast<uint16_t*>(out)[base + i] = dh::f32_to_bf16_bits(v);
     else static_cast<float*>(out)[base + i] = v;
   };
-  if (vec) {
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int i = 4 * (tid + 256 * j);
-      if (i >= hidden) continue;
-      const float4 wv = *reinterpret_cast<const float4*>(w + i);
-      const float y[4] = {xv[j].x * inv * wv.x, xv[j].y * inv * wv.y, xv[j].z * inv * wv.z, xv[j].w * inv * wv.w};
-      if (BF16 && (ld_out & 3) == 0) {
-        uint2 two;
-        two.x = (uint32_t)dh::f32_to_bf16_bits(y[0]) | ((uint32_t)dh::f32_to_bf16_bits(y[1]) << 16);
-        two.y = (uint32_t)dh::f32_to_bf16_bits(y[2]) | ((uint32_t)dh::f32_to_bf16_bits(y[3]) << 16);
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + base + i) = two;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; e++) put(i + e, y[e]);
-      }
-    }
-  } else {
-    for (int i = tid; i < hidden; i += 256) put(i, xr[i] * inv * w[i]);
-  }
+  for (int i = tid; i < hidden; i += 256) put(i, xr[i] * inv * w[i]);
   for (int i = hidden + tid; i < ld_out; i += 256) put(i, 0.f);
 }
 

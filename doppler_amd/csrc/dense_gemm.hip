@@ -55,6 +55,12 @@ struct GemmArgs {
   float* parts;           // [slices][M][N] raw sums instead of the outputs, or null
   int k_slice;            // k extent of a slice (a multiple of 64); K when there is one
   dh::ExpertRows rows;    // GROUPED and GLU forms
+  // the first output's rows normed as well, where a reduce launch holds them whole (done: it did), or null
+  const float* norm_weight;
+  float norm_eps;
+  void* normed;           // [M][ld_normed]
+  int normed_dtype, ld_normed;
+  bool* norm_done;
 };
 
 // Second outputs a kernel is compiled for: none (the first without or with a residual), one activation, or whatever the arguments say.
@@ -501,6 +507,36 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
   }
 }
 
+// The same where all columns are a first output's and the rows are normed behind it: one workgroup a row (N a multiple of 4, at most 8192, everything
+// aligned).  The norm's launch was 3.1 us and 1.4 in front of the next: 301 rows of 1024 in three slices 4.4 + 3.1 -> 5.0 us.
+template <bool BF16>
+__global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(const GemmArgs a, int slices) {
+  __shared__ float red[4];
+  const int m = blockIdx.x;
+  const int64_t total = (int64_t)a.M * a.N;
+  const float *p = a.parts + (int64_t)m * a.N, *res = a.residual ? a.residual + (int64_t)m * a.ldc : nullptr;
+  float* c = a.C + (int64_t)m * a.ldc;
+  float4 x[dh::kNormPieces];
+#pragma unroll
+  for (int j = 0; j < dh::kNormPieces; j++) {
+    const int n = 4 * (threadIdx.x + 256 * j);
+    x[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (n >= a.N) continue;
+    f32x4_t bias = {0.f, 0.f, 0.f, 0.f}, scale = {1.f, 1.f, 1.f, 1.f}, residual = bias, s = bias;
+    if (a.bias) bias = *reinterpret_cast<const f32x4_t*>(a.bias + n);
+    if (a.col_scale) scale = *reinterpret_cast<const f32x4_t*>(a.col_scale + n);
+    if (res) residual = *reinterpret_cast<const f32x4_t*>(res + n);
+#pragma unroll 4
+    for (int k = 0; k < slices; k++) s += *reinterpret_cast<const f32x4_t*>(p + k * total + n);
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = first_output(a, PutTerms{bias[e], scale[e], residual[e]}, s[e]);
+    x[j] = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(c + n) = x[j];
+  }
+  dh::store_normed_row<BF16>(x, a.N, a.norm_weight, a.norm_eps, red, a.normed, (int64_t)m * a.ld_normed, a.ld_normed);
+}
+
 // Tiles of the 16-bit products, and what they cost in ns: a k step (64 elements) `alone` with few workgroups on the device, `one` with one
 // on every compute unit, `full` with as many as fit (the two larger tiles: one, which takes more than half of the LDS); outside the k
 // loop `start`, and `again` for every further round of workgroups.  The device slows its clock under matrix-core load, so a step gets
@@ -589,6 +625,15 @@ int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
   return 0;
 }
 int launch_reduce(const char* op, const GemmArgs& a, int slices) {
+  if (a.norm_weight && a.n_first == a.N && a.N % 4 == 0 && a.N <= 1024 * dh::kNormPieces && a.ldc % 4 == 0 &&
+      ((reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.residual) | reinterpret_cast<uintptr_t>(a.bias) |
+        reinterpret_cast<uintptr_t>(a.col_scale)) & 15) == 0) {
+    auto kern = a.normed_dtype == DH_BF16 ? gemm_reduce_norm_kernel<true> : gemm_reduce_norm_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(a.M), dim3(256), 0, dh::stream(), a, slices);
+    DH_CHECK_LAUNCH(op);
+    *a.norm_done = true;
+    return 0;
+  }
   const bool vec = a.N % 4 == 0;
   const int64_t columns = vec ? a.N / 4 : a.N;
   int log2_wide = 8;
@@ -649,7 +694,9 @@ TileChoice choose_16bit(int64_t M, int64_t N, int64_t K, bool erf) {
 }
 
 // A product whose rows are out of reach goes in halves.
-int dense_16bit(const char* op, const GemmArgs& a, bool f16) {
+int dense_16bit(const char* op, const GemmArgs& whole, bool f16) {
+  GemmArgs a = whole;
+  if ((a.M > 1 && !within_reach(a.M, a.lda, a.K)) || (a.N > 1 && !within_reach(a.N, a.ldw, a.K))) a.norm_weight = nullptr;      // (its rows are not whole there)
   if (a.M > 1 && !within_reach(a.M, a.lda, a.K)) {
     GemmArgs low = a, high = a;
     const int64_t m = low.M = a.M / 2;
@@ -872,10 +919,9 @@ extern "C" int dh_dense_matmul(const void* d_A, int a_dtype, int lda, const void
                                 c2_dtype, ldc2, activation);
 }
 
-extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K,
-                                      float alpha, const float* d_bias, const float* d_col_scale, const float* d_residual,
-                                      float* d_C, int ldc, int n_first, void* d_C2, int c2_dtype, int ldc2, int activation) {
-  const char* op = "dh_dense_matmul";
+static int dense_matmul(const char* op, const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K,
+                        float alpha, const float* d_bias, const float* d_col_scale, const float* d_residual,
+                        float* d_C, int ldc, int n_first, void* d_C2, int c2_dtype, int ldc2, int activation, const GemmArgs& norm) {
   DH_REQUIRE_INIT(op);
   if (M <= 0 || N <= 0 || K <= 0) return dh::fail(1, "[%s] Dimensions must be positive: M=%d, N=%d, K=%d", op, M, N, K);
   if (K % 64) return dh::fail(1, "[%s] K=%d must be a multiple of 64 (zero-padded)", op, K);
@@ -890,13 +936,37 @@ extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, con
     return dh::fail(1, "[%s] the second output needs %d columns of bf16, f16 or f32 (ldc2=%d, dtype %d)", op, N - n_first, ldc2, c2_dtype);
   if ((reinterpret_cast<uintptr_t>(d_A) | reinterpret_cast<uintptr_t>(d_W)) & 15)
     return dh::fail(1, "[%s] activation and weight pointers must be 16-byte aligned", op);
-  GemmArgs a{};
+  GemmArgs a = norm;
   a.A = d_A; a.W = static_cast<const uint16_t*>(d_W); a.lda = lda; a.ldw = ldw;
   a.M = M; a.N = N; a.K = K; a.alpha = alpha; a.bias = d_bias; a.residual = d_residual; a.col_scale = d_col_scale;
   a.C = d_C; a.ldc = ldc; a.n_first = n_first;
   a.C2 = d_C2; a.ldc2 = ldc2; a.c2_dtype = c2_dtype; a.act = activation;
   if (a_dtype == DH_F32) return dense_f32(op, a);
   return dense_16bit(op, a, a_dtype == DH_F16);
+}
+
+extern "C" int dh_dense_matmul_scaled(const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K,
+                                      float alpha, const float* d_bias, const float* d_col_scale, const float* d_residual,
+                                      float* d_C, int ldc, int n_first, void* d_C2, int c2_dtype, int ldc2, int activation) {
+  return dense_matmul("dh_dense_matmul", d_A, a_dtype, lda, d_W, ldw, M, N, K, alpha, d_bias, d_col_scale, d_residual, d_C, ldc, n_first, d_C2, c2_dtype, ldc2,
+                      activation, GemmArgs{});
+}
+
+extern "C" int dh_dense_matmul_normed(const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K, const float* d_col_scale,
+                                      const float* d_residual, float* d_C, int ldc, const float* d_norm_weight, float eps, void* d_normed, int normed_dtype,
+                                      int ld_normed) {
+  const char* op = "dh_dense_matmul_normed";
+  DH_REQUIRE_INIT(op);
+  if (normed_dtype != DH_BF16 && normed_dtype != DH_F32) return dh::fail(1, "[%s] normed rows must be bf16 or f32, got dtype %d", op, normed_dtype);
+  if (!d_norm_weight || !d_normed) return dh::fail(1, "[%s] null pointer", op);
+  if (ld_normed < N || !(eps >= 0.f)) return dh::fail(1, "[%s] normed rows of %d do not hold %d elements, or eps is negative", op, ld_normed, N);
+  if ((reinterpret_cast<uintptr_t>(d_norm_weight) | reinterpret_cast<uintptr_t>(d_normed) | reinterpret_cast<uintptr_t>(d_C)) & 15)
+    return dh::fail(1, "[%s] pointers must be 16-byte aligned", op);
+  bool done = false;
+  GemmArgs norm{};
+  norm.norm_weight = d_norm_weight; norm.norm_eps = eps; norm.normed = d_normed; norm.normed_dtype = normed_dtype; norm.ld_normed = ld_normed; norm.norm_done = &done;
+  if (int rc = dense_matmul(op, d_A, a_dtype, lda, d_W, ldw, M, N, K, 1.f, nullptr, d_col_scale, d_residual, d_C, ldc, N, nullptr, 0, 0, DH_ACT_NONE, norm)) return rc;
+  return done ? 0 : dh_rmsnorm_rows(d_C, ldc, nullptr, d_norm_weight, d_normed, normed_dtype, ld_normed, M, N, eps);
 }
 
 extern "C" int dh_dense_matmul_layout(int M, int N, int K, int a_dtype, int form, int num_cus, int64_t* out3) {

@@ -622,6 +622,42 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __res
   }
 }
 
+// The same where nothing is added behind it, and the rows normed for the product that reads them: one workgroup a row (at most 8192 columns, a multiple of
+// four, x and ls aligned).  Against a launch of the norm's own, us: 1531 rows of 2048 18.9 + 5.6 -> 17.1, 40 of 1024 4.3 + 3.1 -> 4.8.
+template <bool BF16>
+__global__ __launch_bounds__(256) void experts_combine_norm_kernel(const float* __restrict__ y, int64_t ld_y, const int* __restrict__ slot, int top,
+                                                                   const float* __restrict__ shared, const float* __restrict__ ls, float* __restrict__ x,
+                                                                   int64_t ld_x, int hidden, const float* __restrict__ norm, float eps, void* __restrict__ normed,
+                                                                   int ld_normed) {
+  __shared__ float red[4];
+  const int t = blockIdx.x;
+  const int* places = slot + (int64_t)t * top;
+  float* row = x + (int64_t)t * ld_x;
+  float4 out[dh::kNormPieces];
+#pragma unroll
+  for (int j = 0; j < dh::kNormPieces; j++) {
+    const int i = 4 * (threadIdx.x + 256 * j);
+    out[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i >= hidden) continue;
+    const float4 old = *reinterpret_cast<const float4*>(row + i);
+    float4 s = out[j], own = s, f = make_float4(1.f, 1.f, 1.f, 1.f);
+    if (shared) own = *reinterpret_cast<const float4*>(shared + (int64_t)t * ld_y + i);
+    if (ls) f = *reinterpret_cast<const float4*>(ls + i);
+#pragma unroll 4
+    for (int k = 0; k < top; k++) {
+      const float4 v = *reinterpret_cast<const float4*>(y + (int64_t)places[k] * ld_y + i);
+      s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+    }
+    auto sum = [&](float f, float s, float own, float old) {
+      const float v = fmaf(f, s, old);
+      return shared ? fmaf(own, f, 0.f) + v : v;
+    };
+    out[j] = make_float4(sum(f.x, s.x, own.x, old.x), sum(f.y, s.y, own.y, old.y), sum(f.z, s.z, own.z, old.z), sum(f.w, s.w, own.w, old.w));
+    *reinterpret_cast<float4*>(row + i) = out[j];
+  }
+  dh::store_normed_row<BF16>(out, hidden, norm, eps, red, normed, (int64_t)t * ld_normed, ld_normed);
+}
+
 size_t up256(size_t n) { return (n + 255) / 256 * 256; }
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -680,6 +716,16 @@ dh::ExpertProduct shared_product(const dh_experts* s, const PortionSpace& p, int
 bool together(const dh_experts* s, int operand, const PortionSpace& p, int T, bool glu) {
   return s->shared_ff > 0 && operand == DH_BF16 && dh::experts_together(routed_product(s, p, T, glu), shared_product(s, p, T, glu), glu);
 }
+
+// The norm of the rows a portion leaves, for the product that reads them next, or nothing; done: the last launch made it.
+struct NextNorm {
+  const float* weight = nullptr;
+  float eps = 0.f;
+  void* normed = nullptr;
+  int ld = 0;
+  bool* done = nullptr;
+};
+int prefill(const char* op, const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T, const NextNorm& next);
 
 }  // namespace
 
@@ -751,7 +797,25 @@ int dh_experts_prefill_layout(const dh_experts* spec, int operand, int T, int nu
 }
 
 int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T) {
-  const char* op = "dh_experts_prefill";
+  return prefill("dh_experts_prefill", spec, d_h, operand, d_x, ld_x, d_workspace, T, NextNorm{});
+}
+
+int dh_experts_prefill_normed(const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T, const float* d_norm_weight,
+                              float eps, void* d_normed, int ld_normed) {
+  const char* op = "dh_experts_prefill_normed";
+  DH_REQUIRE_INIT(op);
+  if (!d_norm_weight || !d_normed) return dh::fail(1, "[%s] null pointer", op);
+  if (!aligned(d_norm_weight) || !aligned(d_normed)) return dh::fail(1, "[%s] pointers must be 16-byte aligned", op);
+  if (spec && (ld_normed < spec->hidden || !(eps >= 0.f))) return dh::fail(1, "[%s] normed rows of %d do not hold %d elements, or eps is negative", op, ld_normed, spec->hidden);
+  bool done = false;
+  if (int rc = prefill(op, spec, d_h, operand, d_x, ld_x, d_workspace, T, NextNorm{d_norm_weight, eps, d_normed, ld_normed, &done})) return rc;
+  return done ? 0 : dh_rmsnorm_rows(d_x, ld_x, nullptr, d_norm_weight, d_normed, operand, ld_normed, T, spec->hidden, eps);
+}
+
+}  // extern "C"
+
+namespace {
+int prefill(const char* op, const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T, const NextNorm& next) {
   DH_REQUIRE_INIT(op);
   if (int rc = check(op, spec)) return rc;
   if (T <= 0 || ld_x < spec->hidden) return dh::fail(1, "[%s] %d rows %d apart", op, T, ld_x);
@@ -762,8 +826,8 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   if (operand == DH_BF16 && T > 1 && (int64_t)T * spec->K >= (int64_t)1 << 31) {
     // gathered rows are addressed by 32-bit byte offsets: more than 4 GB of them go in two portions
     const int half = T / 2;
-    if (int rc = dh_experts_prefill(spec, d_h, operand, d_x, ld_x, d_workspace, half)) return rc;
-    return dh_experts_prefill(spec, static_cast<const uint16_t*>(d_h) + (int64_t)half * spec->K, operand, d_x + (int64_t)half * ld_x, ld_x, d_workspace, T - half);
+    if (int rc = prefill(op, spec, d_h, operand, d_x, ld_x, d_workspace, half, NextNorm{})) return rc;
+    return prefill(op, spec, static_cast<const uint16_t*>(d_h) + (int64_t)half * spec->K, operand, d_x + (int64_t)half * ld_x, ld_x, d_workspace, T - half, NextNorm{});
   }
   const PortionSpace p = portion_space(spec, operand, T);
   char* w = static_cast<char*>(d_workspace);
@@ -816,6 +880,15 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   } else {
     if (int rc = dh::experts_down(op, routed_down.rows, w + p.act, operand, spec->ff, down, spec->ff, spec->hidden, spec->ff, f32(p.y), p.ld_y)) return rc;
   }
+  if (next.weight && (!shared || down_pair) && spec->hidden % 4 == 0 && spec->hidden <= 1024 * dh::kNormPieces && ld_x % 4 == 0 && aligned(d_x) &&
+      aligned(spec->d_layer_scale)) {
+    auto kern = operand == DH_BF16 ? experts_combine_norm_kernel<true> : experts_combine_norm_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, dh::stream(), f32(p.y), (int64_t)p.ld_y, i32(p.slot), spec->top, down_pair ? f32(p.shared_y) : nullptr,
+                       spec->d_layer_scale, d_x, (int64_t)ld_x, spec->hidden, next.weight, next.eps, next.normed, next.ld);
+    DH_CHECK_LAUNCH(op);
+    *next.done = true;
+    return 0;
+  }
   hipLaunchKernelGGL(experts_combine_kernel, dim3(T, (unsigned)dh::ceil_div(spec->hidden, 1024)), dim3(256), 0, dh::stream(), f32(p.y), (int64_t)p.ld_y,
                      i32(p.slot), spec->top, down_pair ? f32(p.shared_y) : nullptr, spec->d_layer_scale, d_x, (int64_t)ld_x, spec->hidden);
   DH_CHECK_LAUNCH(op);
@@ -827,4 +900,4 @@ int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, flo
   return 0;
 }
 
-}  // extern "C"
+}  // namespace

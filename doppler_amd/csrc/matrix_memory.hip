@@ -789,11 +789,10 @@ template <typename OUT>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ gate,
                                                              int64_t ld_gate, const float* __restrict__ w, OUT* __restrict__ out,
                                                              int64_t ld_out, int rows, int H, int VP, int size, float eps) {
-  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (item >= (int64_t)rows * H) return;
-  const int64_t t = item / H;
-  const int h = (int)(item % H);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), item = 4 * blockIdx.x + wave, row = item / (uint32_t)H;
+  const int lane = threadIdx.x & 63, h = (int)(item - row * (uint32_t)H);
+  if (row >= (uint32_t)rows) return;
+  const int64_t t = row;
   const float* xr = x + t * ld_x + (int64_t)h * VP;
   float ss = 0.f;
   for (int i = 4 * lane; i < VP; i += 256) {

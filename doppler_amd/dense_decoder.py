@@ -263,16 +263,22 @@ class DenseDecoder(DecoderBase):
 
     # ------------------------------------------------------------------ several rows at once
 
-    def _enqueue_in(self, d, x, normed, operand, qkv, act, rows, ld_act):
-        """[q | k | v | gate] rows and activated `up` rows of the residual rows at x."""
+    def _enqueue_in(self, d, x, normed, operand, qkv, act, rows, ld_act, ready=False):
+        """[q | k | v | gate] rows and activated `up` rows of the residual rows at x (ready: their normed rows are there)."""
         g, c = d["geo"], self.cfg
-        capi.check(self.L.dh_rmsnorm_rows(x, self.kx, None, d["norm"].data_ptr(), normed, operand, self.kx, rows, c["hidden"], c["eps"]))
+        if not ready:
+            capi.check(self.L.dh_rmsnorm_rows(x, self.kx, None, d["norm"].data_ptr(), normed, operand, self.kx, rows, c["hidden"], c["eps"]))
         capi.check(self.L.dh_dense_matmul(normed, operand, self.kx, d["w_in"].data_ptr(), g["kx"], rows, g["n"], g["kx"], 1.0,
                                           d["bias"].data_ptr(), None, qkv, g["n_first"], g["n_first"], act, operand, ld_act,
                                           d["act"]))
 
-    def _enqueue_out(self, d, mixed, operand, x, rows):
+    def _enqueue_out(self, d, mixed, operand, x, rows, norm=None, normed=None):
+        """x += the layer's output; norm: the weights of the norm that comes next, whose rows go to `normed`."""
         g, Hd = d["geo"], self.cfg["hidden"]
+        if norm is not None:
+            capi.check(self.L.dh_dense_matmul_normed(mixed, operand, g["k2"], d["w_out"].data_ptr(), g["k2"], rows, Hd, g["k2"], None, x, x, self.kx,
+                                                     norm.data_ptr(), self.cfg["eps"], normed, operand, self.kx))
+            return
         capi.check(self.L.dh_dense_matmul(mixed, operand, g["k2"], d["w_out"].data_ptr(), g["k2"], rows, Hd, g["k2"], 1.0, None, x,
                                           x, self.kx, Hd, None, 0, 0, capi.ACT_NONE))
 
@@ -292,19 +298,21 @@ class DenseDecoder(DecoderBase):
         ck(L.dh_upload(b["ids"].data_ptr(), 0, up.ctypes.data, up.nbytes))
         ck(L.dh_embed_sum(b["ids"].data_ptr(), 1, b["ids"].data_ptr(), *self._embed_args(), x, self.kx, T, c["hidden"], pos, None))
         elem = b["normed"].element_size()
-        for d in self.layers:
+        ready = False        # whether the layer before has left this one's normed rows
+        for d, after in zip(self.layers, self.layers[1:] + [None]):
             if isinstance(d, SequentialLayer):
-                d.rows(x, T, pos)
+                ready = d.rows(x, T, pos, ready, after.parts[0] if isinstance(after, SequentialLayer) else None)
                 continue
             g = d["geo"]
             mixed = b["mixed"][self._mixed_key(g)].data_ptr()
             self._enqueue_in(d, x, b["normed"].data_ptr(), self.operand, b["qkv"].data_ptr(),
-                             mixed + elem * g["attn_cols"] if g["ff"] else None, T, g["k2"])
+                             mixed + elem * g["attn_cols"] if g["ff"] else None, T, g["k2"], ready)
             ck(L.dh_attn_spec_kv_write(ctypes.byref(d["spec"]), b["qkv"].data_ptr(), d["cache_k"].data_ptr(),
                                        d["cache_v"].data_ptr(), T, pos))
             ck(L.dh_attn_spec_prefill(ctypes.byref(d["spec"]), b["qkv"].data_ptr(), d["cache_k"].data_ptr(),
                                       d["cache_v"].data_ptr(), mixed, self.operand, g["k2"], T, pos))
-            self._enqueue_out(d, mixed, self.operand, x, T)
+            ready = after is not None and not isinstance(after, SequentialLayer)
+            self._enqueue_out(d, mixed, self.operand, x, T, after["norm"] if ready else None, b["normed"].data_ptr())
         return x, self.kx
 
     def _logit_rows(self, base, stride, rows):

@@ -8,7 +8,7 @@
                     ExpertsFF         sigmoid-routed experts with clamped gates, and a gated shared expert
 
 A sublayer stacks and pads its own tensors (zeros: padded rows and columns contribute nothing), owns its cache rows or state, and
-runs on the decoder's residual in two ways: step() for one token, rows() for a portion.  Projections that read the normed row are one
+runs on the decoder's residual in two ways: step() for one token, rows() for a portion (which may leave the next sublayer's normed rows).  Projections that read the normed row are one
 product; the layer scale and the residual belong to the epilogue of the last one.
 """
 import ctypes
@@ -90,17 +90,25 @@ class _Sublayer:
                                                    k, 1.0, bias, self.ls_ptr if residual else None, x_out if residual else None, x_out,
                                                    n if act_out is None else 0, act_out, act))
 
-    def _normed_rows(self, x, count):
-        """Normed residual rows in the operand type."""
+    def _normed_rows(self, x, count, ready=False):
+        """Normed residual rows in the operand type (ready: the sublayer before has left them)."""
         d = self.dec
         out = d.scratch.rows("normed", self.kx, count, d.operand_torch)
+        if ready:
+            return out
         capi.check(d.L.dh_rmsnorm_rows(x, self.kx, None, self.norm.data_ptr(), out, d.operand, self.kx, count, self.hidden, self.eps))
         return out
 
-    def _out_rows(self, a, k, w, x, count):
-        """x += ls * W a over rows of k elements."""
+    def _out_rows(self, a, k, w, x, count, then):
+        """x += ls * W a over rows of k elements; then: the next sublayer, or None.  Returns whether its normed rows are there."""
+        if then is not None:
+            d = self.dec
+            capi.check(d.L.dh_dense_matmul_normed(a, d.operand, k, w.data_ptr(), k, count, self.hidden, k, self.ls_ptr, x, x, self.kx, then.norm.data_ptr(),
+                                                  self.eps, d.scratch.rows("normed", self.kx, count, d.operand_torch), d.operand, self.kx))
+            return True
         capi.check(self.dec.L.dh_dense_matmul_scaled(a, self.dec.operand, k, w.data_ptr(), k, count, self.hidden, k, 1.0, None, self.ls_ptr, x,
                                                      x, self.kx, self.hidden, None, 0, 0, capi.ACT_NONE))
+        return False
 
     def state(self):
         """Recurrent buffers."""
@@ -162,9 +170,9 @@ class LatentAttention(_Sublayer):
         capi.check(d.L.dh_latent_decode(self.ref, row, self.cache.data_ptr(), mixed, pos, kv_len, d.max_seq, d.scratch.space("latent_decode", 1)))
         self._gemv(mixed, False, self.w_out, self.hidden, self.k2, residual=True)
 
-    def rows(self, x, count, pos):
+    def rows(self, x, count, pos, ready=False, then=None):
         d = self.dec
-        normed = self._normed_rows(x, count)
+        normed = self._normed_rows(x, count, ready)
         rows = d.scratch.rows("rows", self.ld, count, torch.float32)
         capi.check(d.L.dh_dense_matmul(normed, d.operand, self.kx, self.w_in.data_ptr(), self.kx, count, self.n_in, self.kx, 1.0, None, None, rows,
                                        self.ld, self.n_in, None, 0, 0, capi.ACT_NONE))
@@ -172,7 +180,7 @@ class LatentAttention(_Sublayer):
         mixed = d.scratch.rows("mixed_rows", self.k2, count, d.operand_torch)
         ws = d.scratch.space("latent_prefill", d.L.dh_latent_prefill_workspace_bytes(self.ref, count, pos))
         capi.check(d.L.dh_latent_prefill(self.ref, rows, self.cache.data_ptr(), ws, mixed, d.operand, self.k2, count, pos))
-        self._out_rows(mixed, self.k2, self.w_out, x, count)
+        return self._out_rows(mixed, self.k2, self.w_out, x, count, then)
 
     def step_bytes(self, ctx):
         m = self.m
@@ -234,9 +242,9 @@ class MatrixMemory(_Sublayer):
         self._norm_gate(o, row, mixed, capi.F32, 1)
         self._gemv(mixed, False, self.w_out, self.hidden, self.k2, residual=True)
 
-    def rows(self, x, count, pos):
+    def rows(self, x, count, pos, ready=False, then=None):
         d = self.dec
-        normed = self._normed_rows(x, count)
+        normed = self._normed_rows(x, count, ready)
         rows = d.scratch.rows("rows", self.n_in, count, torch.float32)
         capi.check(d.L.dh_dense_matmul(normed, d.operand, self.kx, self.w_in.data_ptr(), self.kx, count, self.n_in, self.kx, 1.0,
                                        self.bias.data_ptr(), None, rows, self.n_in, self.n_in, None, 0, 0, capi.ACT_NONE))
@@ -245,7 +253,7 @@ class MatrixMemory(_Sublayer):
         capi.check(d.L.dh_mlstm_prefill(self.ref, rows, self.memory.data_ptr(), ws, o, self.o_width, count, pos))
         mixed = d.scratch.rows("mixed_rows", self.k2, count, d.operand_torch)
         self._norm_gate(o, rows, mixed, d.operand, count)
-        self._out_rows(mixed, self.k2, self.w_out, x, count)
+        return self._out_rows(mixed, self.k2, self.w_out, x, count, then)
 
     def step_bytes(self, ctx):
         m = self.m
@@ -270,13 +278,13 @@ class DenseFF(_Sublayer):
         self._gemv(d.x.data_ptr(), True, self.up, self.ff, self.kx, act_out=act, act=self.act)
         self._gemv(act, False, self.down, self.hidden, self.ffp, residual=True)
 
-    def rows(self, x, count, pos):
+    def rows(self, x, count, pos, ready=False, then=None):
         d = self.dec
-        normed = self._normed_rows(x, count)
+        normed = self._normed_rows(x, count, ready)
         act = d.scratch.rows("act_rows", self.ffp, count, d.operand_torch)
         capi.check(d.L.dh_dense_matmul(normed, d.operand, self.kx, self.up.data_ptr(), self.kx, count, self.ff, self.kx, 1.0, None, None, None, 0, 0,
                                        act, d.operand, self.ffp, self.act))
-        self._out_rows(act, self.ffp, self.down, x, count)
+        return self._out_rows(act, self.ffp, self.down, x, count, then)
 
     def step_bytes(self, ctx):
         return 4 * self.hidden * self.ff
@@ -321,11 +329,15 @@ class ExpertsFF(_Sublayer):
         d = self.dec
         capi.check(d.L.dh_experts_step(self.ref, d.x.data_ptr(), d.scratch.space("experts_step", self.ws_bytes)))
 
-    def rows(self, x, count, pos):
+    def rows(self, x, count, pos, ready=False, then=None):
         d = self.dec
-        normed = self._normed_rows(x, count)
+        normed = self._normed_rows(x, count, ready)
         ws = d.scratch.space("experts_prefill", d.L.dh_experts_prefill_workspace_bytes(self.ref, d.operand, count))
+        if then is not None:
+            capi.check(d.L.dh_experts_prefill_normed(self.ref, normed, d.operand, x, self.kx, ws, count, then.norm.data_ptr(), self.eps, normed, self.kx))
+            return True
         capi.check(d.L.dh_experts_prefill(self.ref, normed, d.operand, x, self.kx, ws, count))
+        return False
 
     def step_bytes(self, ctx):
         m = self.m
@@ -352,9 +364,11 @@ class SequentialLayer:
         for p in self.parts:
             p.step(pos, kv_len)
 
-    def rows(self, x, count, pos):
-        for p in self.parts:
-            p.rows(x, count, pos)
+    def rows(self, x, count, pos, ready=False, then=None):
+        """A portion; ready: its first normed rows are there; then: the next layer's first sublayer, or None.  Returns whether that one's are."""
+        for p, after in zip(self.parts, self.parts[1:] + [then]):
+            ready = p.rows(x, count, pos, ready, after)
+        return ready
 
     def state(self):
         return [t for p in self.parts for t in p.state()]

@@ -409,6 +409,11 @@ int dh_dense_gemv(const float* d_x, const float* d_norm_weight, int hidden, floa
 int dh_dense_gemv_scaled(const float* d_x, const float* d_norm_weight, int hidden, float eps, const void* d_W, int ldw, int N,
                          int K, float alpha, const float* d_bias, const float* d_col_scale, const float* d_residual, float* d_C,
                          int n_first, float* d_C2, int activation);
+/* C [M][N] = (A W^T) * d_col_scale + d_residual (either may be NULL, the residual may be C) in f32, and its rows normed for the product that reads them,
+ * as dh_rmsnorm_rows would: d_normed [M][ld_normed], DH_BF16 or DH_F32.  One launch fewer where the product's k is cut into slices. */
+int dh_dense_matmul_normed(const void* d_A, int a_dtype, int lda, const void* d_W, int ldw, int M, int N, int K, const float* d_col_scale,
+                           const float* d_residual, float* d_C, int ldc, const float* d_norm_weight, float eps, void* d_normed, int normed_dtype,
+                           int ld_normed);
 /* C = (W y) * col_scale + residual with y the gated, normed heads of dh_head_norm_gate: x_h / rms(x_h) * weight * sigmoid(gate); at most
  * 256 heads of `padded` floats (a multiple of 32), K >= H * padded. */
 int dh_dense_gemv_heads(const float* d_x, const float* d_gate, const float* d_weight, int H, int padded, int size, float eps, const void* d_W,
@@ -580,6 +585,10 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace);
 /* T rows: d_h their normed rows [T][K] in the operand type (DH_BF16 or DH_F32), d_x the residual rows. */
 size_t dh_experts_prefill_workspace_bytes(const dh_experts* spec, int operand, int T);
 int dh_experts_prefill(const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T);
+/* The same, and the rows of x it leaves normed for the product that reads them, as dh_rmsnorm_rows would: d_normed [T][ld_normed] of the operand type, which may
+ * be d_h. */
+int dh_experts_prefill_normed(const dh_experts* spec, const void* d_h, int operand, float* d_x, int ld_x, void* d_workspace, int T, const float* d_norm_weight,
+                              float eps, void* d_normed, int ld_normed);
 /* How dh_experts_prefill would multiply a portion: out3 = rows of the routed experts' tiles, whether the shared expert's gate and up product goes in
  * their launch, whether its down product does.  For tests that have to reach every form; needs no device. */
 int dh_experts_prefill_layout(const dh_experts* spec, int operand, int T, int num_cus, int64_t* out3);

@@ -713,6 +713,49 @@ def test_choices_of_portions_and_steps(L, T, K, E, top, ff, shared_ff):
     assert torch.equal(x[n:], x0[n:])
 
 
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F32])
+@pytest.mark.parametrize("M,N,K,sliced", [(40, 1024, 3072, True), (1, 260, 4096, True), (33, 8192, 4096, None), (17, 8196, 4096, None), (5, 102, 4096, True), (700, 1024, 256, False)])
+def test_products_that_leave_normed_rows(L, M, N, K, sliced, dtype):
+    """The bits of a product and a norm: rows in one to eight pieces a thread and longer ones, columns that are no multiple of four, padding behind a row,
+    products in k slices and whole, with a column scale and the residual in place."""
+    out, t = (ctypes.c_int64 * 3)(), torch.bfloat16 if dtype == capi.BF16 else torch.float32
+    capi.check(L.dh_dense_matmul_layout(M, N, K, dtype, 0, 0, out))
+    assert sliced is None or (out[2] > 1) == sliced
+    g = torch.Generator(device="cuda").manual_seed(N)
+    A, W = torch.randn(M, K, generator=g, device="cuda").to(t), (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16)
+    ld, scale, w = (N + 63) // 64 * 64, torch.randn(N, generator=g, device="cuda"), torch.randn((N + 63) // 64 * 64, generator=g, device="cuda")
+    x = torch.randn(M, ld, generator=g, device="cuda")
+    y, a, b = x.clone(), (torch.full((M, ld), 7.0, dtype=t, device="cuda")), torch.full((M, ld), 7.0, dtype=t, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_dense_matmul_scaled(A.data_ptr(), dtype, K, W.data_ptr(), K, M, N, K, 1.0, None, scale.data_ptr(), x.data_ptr(), x.data_ptr(), ld, N, None, 0, 0, capi.ACT_NONE))
+    capi.check(L.dh_rmsnorm_rows(x.data_ptr(), ld, None, w.data_ptr(), a.data_ptr(), dtype, ld, M, N, 1e-5))
+    capi.check(L.dh_dense_matmul_normed(A.data_ptr(), dtype, K, W.data_ptr(), K, M, N, K, scale.data_ptr(), y.data_ptr(), y.data_ptr(), ld, w.data_ptr(), 1e-5, b.data_ptr(),
+                                        dtype, ld))
+    capi.check(L.dh_sync())
+    assert torch.equal(x, y) and torch.equal(a, b) and not b[:, N:].any()
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F32])
+@pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(40, 256, 8, 2, 64, 128), (1531, 1024, 4, 2, 512, 1024), (1000, 1024, 5, 2, 512, 1024), (50, 192, 4, 4, 64, 0), (3, 8256, 2, 1, 64, 0)])
+def test_experts_that_leave_normed_rows(L, T, K, E, top, ff, shared_ff, dtype):
+    """The bits of the experts and a norm, in place of the rows they read: a shared expert whose product is in the sum, or comes behind it, or is not there."""
+    g, t = torch.Generator(device="cuda").manual_seed(T + K), torch.bfloat16 if dtype == capi.BF16 else torch.float32
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    h, x, ls, norm = torch.randn(T, K, generator=g, device="cuda").to(t), *(torch.randn(*s, generator=g, device="cuda") for s in ((T, K), (K,), (K,)))
+    router, up, down = w(E + (shared_ff > 0), K), w(E, 2 * ff, K), w(E, K, ff)
+    s_up, s_down = (w(2 * shared_ff, K), w(K, shared_ff)) if shared_ff else (None, None)
+    spec = capi.Experts(K, K, E, top, ff, shared_ff, 1e-5, 7.0, 1.5, norm.data_ptr(), ls.data_ptr(), router.data_ptr(), up.data_ptr(), down.data_ptr(),
+                        s_up.data_ptr() if shared_ff else None, s_down.data_ptr() if shared_ff else None)
+    ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), dtype, T), dtype=torch.uint8, device="cuda")
+    y, a = x.clone(), torch.empty(T, K, dtype=t, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_experts_prefill(ctypes.byref(spec), h.data_ptr(), dtype, x.data_ptr(), K, ws.data_ptr(), T))
+    capi.check(L.dh_rmsnorm_rows(x.data_ptr(), K, None, norm.data_ptr(), a.data_ptr(), dtype, K, T, K, 1e-5))
+    capi.check(L.dh_experts_prefill_normed(ctypes.byref(spec), h.data_ptr(), dtype, y.data_ptr(), K, ws.data_ptr(), T, norm.data_ptr(), 1e-5, h.data_ptr(), K))
+    capi.check(L.dh_sync())
+    assert torch.equal(x, y) and torch.equal(a, h)
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

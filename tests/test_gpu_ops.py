@@ -233,6 +233,25 @@ def test_matmul_f16_activations_at_an_odd_address(M):
     assert rel_l2(out.cpu().numpy().reshape(M, N), want) <= matmul_bar(M)
 
 
+@pytest.mark.parametrize("K,norm", [(8188, True), (8192, False), (8196, True), (8448, False), (12286, True), (16384, True)])
+def test_matmul_prompt_rows_of_any_length(K, norm):
+    """Rows on either side of where sixteen waves pack them, whole pieces and not; the largest element of row m is moved through the row, so
+    that every wave's share is once the one that sets the scale (each row by itself within the product's bar)."""
+    M, N = 17, 48
+    W, wb = q4k_weight(N, K, 1400 + K)
+    A, nw = synth.normal_f32((M, K), 1401 + K), 1.0 + 0.1 * synth.normal_f32((K,), 1402)
+    A[np.arange(1, M), np.arange(1, M) * (K - 1) // (M - 1)] = 3000.0
+    A[0] = 0.0
+    x = A.astype(np.float64)
+    if norm:
+        x = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * nw
+    kw = dict(normWeight=ops.tensorFromNumpy(nw), rmsNormEps=1e-6, useFusedRmsnormWideTile=True) if norm else {}
+    out = ops.readTensor(ops.runMatmul(ops.tensorFromNumpy(A), wb, M, N, K, outputDtype="f32", **kw)).reshape(M, N)
+    want = oracle.q4k_matmul(x.astype(np.float32), W, M, N, K)
+    assert not out[0].any()
+    assert max(rel_l2(out[m], want[m]) for m in range(1, M)) <= matmul_bar(M)
+
+
 def test_matmul_f16_activations_errors():
     W, wb = q4k_weight(8, 256, 1160)
     a = ops.tensorFromNumpy(np.zeros((1, 256), np.float16).view(np.uint16))
@@ -647,6 +666,22 @@ def test_gpu_sample_topk_matches_oracle():
         ops.runGPUSample(lt, V, temperature=1.0, topK=300, randomSeed=1)
     with pytest.raises(DopplerHipError, match="randomSeed"):
         ops.runGPUSample(lt, V, temperature=1.0, topK=5)
+
+
+@pytest.mark.parametrize("hidden,at", [(4, 0), (1020, 0), (1024, 0), (1028, 0), (4100, 0), (1024, 1), (1026, 0)])
+def test_gather_f16_pieces(hidden, at):
+    """Rows in pieces of four and element by element (odd rows, a table that is not on 8 bytes) are the table's own bits, zeros past it."""
+    import torch
+    vocab, L = 50, capi.init(0)
+    E = torch.from_numpy(synth.normal_f16_bits((vocab * hidden + 1,), seed=3300 + hidden, scale=0.02).view(np.int16)).cuda()
+    ids = np.array([7, 49, 0, 50, 4000000000, 31], np.uint32)
+    d_ids, out = torch.from_numpy(ids.view(np.int32)).cuda(), torch.full((5 * hidden + 8,), 3.0, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_gather_f16(d_ids.data_ptr(), E.data_ptr() + 2 * at, out.data_ptr(), 5, hidden, vocab, 1))
+    capi.check(L.dh_sync())
+    table = E.cpu().numpy().view(np.uint16)[at:at + vocab * hidden].reshape(vocab, hidden)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:5 * hidden].reshape(5, hidden), oracle.gather_f16(ids[1:], table, hidden, vocab)) and (got[5 * hidden:] == 3.0).all()
 
 
 def test_gather_f16_exact():

@@ -21,6 +21,7 @@
 #include <cfloat>
 
 #include "attention_keys.h"
+#include "dense_device.h"
 #include "dh_common.h"
 
 namespace {
@@ -56,6 +57,7 @@ struct AttnArgs {
   int rotary_half, interleaved, w_offset, use_norm;
   float eps;
   int c_new, j_new;     // chunk, and key within the chunk, of the appended position
+  int split_new;        // the split that meets it
   // ---- key count on the device (dh_attn_decode_kvlen, dh_attn_decode_qkv_kvlen): kbeg, kend, nsplit,
   // direct and, for the stacked-projection form, cos_row, sin_row, new_row, c_new, j_new above are
   // derived in the kernel from the word behind kv_len_ptr; the grid holds the splits of max_kv_len
@@ -81,71 +83,61 @@ typedef __attribute__((ext_vector_type(8))) _Float16 half8_t;
 // odd rows what the high parts left over, so that the two rows together carry q to ~22 bits.  Both
 // parts are rounded toward zero, two elements per instruction (the residual is exact in f32, so the
 // rounding mode of the high part does not matter).  sc = 0 gives a zero operand.
+struct QParts {
+  uint32_t high, low;        // two elements each
+};
+__device__ __forceinline__ QParts q_parts(const float x0, const float x1) {
+  const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+  const float h0 = __half2float(__ushort_as_half((unsigned short)(hi & 0xffffu)));
+  const float h1 = __half2float(__ushort_as_half((unsigned short)(hi >> 16)));
+  return QParts{hi, __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0 - h0, x1 - h1))};
+}
 __device__ __forceinline__ half8_t q_operand(const float (&qv)[8], const float sc, const bool odd) {
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
   u32x4 w;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const float x0 = qv[2 * i] * sc, x1 = qv[2 * i + 1] * sc;
-    const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-    const float h0 = __half2float(__ushort_as_half((unsigned short)(hi & 0xffffu)));
-    const float h1 = __half2float(__ushort_as_half((unsigned short)(hi >> 16)));
-    const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0 - h0, x1 - h1));
-    w[i] = odd ? lo : hi;
+    const QParts p = q_parts(qv[2 * i] * sc, qv[2 * i + 1] * sc);
+    w[i] = odd ? p.low : p.high;
   }
   return __builtin_bit_cast(half8_t, w);
 }
 typedef __attribute__((ext_vector_type(4))) float float4_t;
 
 
-// Reductions across the lanes of a 16-lane row with DPP row shifts (no LDS traffic): afterwards
-// the last lane of every aligned group of `span` lanes (span = 2, 4, 8 or 16) holds the
-// group's result.
-template <int CTRL>
-__device__ __forceinline__ float dpp_row(float old, float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-template <int SPAN>
-__device__ __forceinline__ float row_group_max(float v) {
-  if (SPAN > 1) v = fmaxf(v, dpp_row<0x111>(v, v));
-  if (SPAN > 2) v = fmaxf(v, dpp_row<0x112>(v, v));
-  if (SPAN > 4) v = fmaxf(v, dpp_row<0x114>(v, v));
-  if (SPAN > 8) v = fmaxf(v, dpp_row<0x118>(v, v));
-  return v;
-}
-template <int SPAN>
-__device__ __forceinline__ float row_group_sum(float v) {
-  if (SPAN > 1) v += dpp_row<0x111>(0.f, v);
-  if (SPAN > 2) v += dpp_row<0x112>(0.f, v);
-  if (SPAN > 4) v += dpp_row<0x114>(0.f, v);
-  if (SPAN > 8) v += dpp_row<0x118>(0.f, v);
-  return v;
-}
-
-// One workgroup = one chunk of 64 keys of one kv head (or several chunks, strided, for long
-// contexts), four waves, two barriers per chunk.
+// One group of four waves = one chunk of 64 keys of one kv head (or several chunks, strided, for long
+// contexts); no wave waits for another between the query rows and the end.
 //   scores   wave w takes keys 16w..16w+15: S = Q.K^T with v_mfma_f32_16x16x32_f16.  The A
 //            operand holds the G query heads of the kv head as rows (2g, 2g+1) = f16 high part
 //            and f16 residual of scale*q (so q keeps ~22 bits); the B operand is loaded from
 //            HBM directly in operand layout (lane (key, kg) reads 16 bytes of its key's row).
-//   softmax  every wave redoes the (tiny) online-softmax update for all heads from the scores
-//            in LDS, so no second exchange is needed: 64/GT lanes per head, GT keys per lane,
-//            DPP row reductions, the per-head maxima and sums travel through scalar registers.
-//   P.V      wave w owns output dims [D/4*w, D/4*(w+1)); lane (dq, kh) holds 4 dims of keys
-//            kh, kh+KH, ... in registers and accumulates them for all heads; the key groups
-//            meet in a wave-private LDS buffer at the end.
+//   softmax  the wave's own, over its sixteen keys: a key per lane, DPP row reductions.
+//   P.V      over the same sixteen keys: whole rows of V, 16 bytes a lane, eight sums per head and
+//            lane; the probabilities change lanes through the wave's own LDS.  In the end lane
+//            swaps add the lanes of a dim, LDS the waves.
 // K and V of the next chunk are requested before the current one is consumed.
-// (Keeping two chunks in flight instead of one changed nothing, 34.1 vs 33.3 us at 32768 keys, and
-// neither did 128-key chunks, 33.5 us: a workgroup's ~2 us per 64 keys is its own softmax and
-// P.V arithmetic plus LDS round trips with one wave per SIMD, not the wait for memory or the
-// barriers.)
+// A step's launch is a chain of trips (arguments, query rows, keys) and of what one wave does for its
+// chunk.  Waves that shared a chunk's softmax and split V by dims took two barriers and twice the
+// requests per chunk; q's two parts were made in every wave from whole rows; addresses were 64-bit
+// products: 6.5 -> 5.7 us with 2049 keys of 32/8 heads of 128 in a step of 36 layers (1644 -> 1609 us),
+// 4.7 -> 4.4 with 518 keys of 16/8 heads of 64 (685 -> 672 us); 32768 keys of 16/8 heads of 128 stay
+// at 24.3 us, 5.5 TB/s.
+// GROUPS: where a workgroup has more than one chunk a second group of four waves takes every other
+// one.  (Two groups on the former kernel were slower, 6.8 us at 2049 keys and 31.7 at 32768: a
+// compute unit's requests were the bound.)
 // GT: query heads per kv head rounded up to 1, 2, 4 or 8 (bounds the unrolled per-head code).
 // QKV: the step's q, k, v arrive raw (see the top of the file); the appended key is the last
 // visible one, so the lanes that would read its row, or a clamped copy of it, from the not yet
 // written cache are patched from registers.
-template <int D, int GT, bool QKV>
-__global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a_in) {
+template <int D, int GT, bool QKV, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS) void attn_decode_split_kernel(const AttnArgs a_in) {
   AttnArgs a = a_in;
+  // the arguments in one batch (left alone the compiler fetches them where they are first used: three trips in front of the first row)
+  asm volatile("" :: "s"(a.K), "s"(a.V), "s"(a.H), "s"(a.Hkv), "s"(a.G), "s"(a.kbeg), "s"(a.kend), "s"(a.nsplit), "s"(a.scale), "s"(a.softcap), "s"(a.kv_start),
+               "s"(a.ring_window), "s"(a.dyn.kv_len_ptr));
+  if (QKV)
+    asm volatile("" :: "s"(a.qkv), "s"(a.qw), "s"(a.kw), "s"(a.cos_row), "s"(a.sin_row), "s"(a.rotary_half), "s"(a.interleaved), "s"(a.w_offset), "s"(a.use_norm),
+                 "s"(a.c_new), "s"(a.j_new), "s"(a.split_new));
   // splits per query head in the workspace: the launch's split count, which with the key count on the
   // device is the largest any count can ask for, so that a reader finds a head's partial results
   // without knowing the count
@@ -162,60 +154,67 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
       a.new_row = (int64_t)row * a.Hkv * D;
       a.c_new = (r.kend - r.kbeg - 1) / kTileKeys;
       a.j_new = (r.kend - r.kbeg - 1) % kTileKeys;
+      a.split_new = a.c_new % a.nsplit;
     }
   }
   constexpr int STEPS = D / 32;          // MFMAs per 16 keys
-  constexpr int DW = D / 4;              // output dims per wave
-  constexpr int LPK = DW / 4;            // lanes per key in P.V (4 dims each)
-  constexpr int KH = 64 / LPK;           // key groups
-  constexpr int NJ = kTileKeys / KH;     // keys per lane
-  constexpr int LH = 64 / GT;            // softmax: lanes per head (each holds GT keys)
-  constexpr int SPAN = LH < 16 ? LH : 16;
-  __shared__ __align__(16) float s_lds[GT][kTileKeys];        // raw scores of the chunk
-  __shared__ __align__(16) float p_lds[4][GT][kTileKeys];     // per-wave probabilities
-  __shared__ __align__(16) float o_lds[4][KH][GT][DW];        // per-wave partial outputs
+  constexpr int WAVES = 4 * GROUPS;
+  constexpr int LPK = D / 8;             // P.V: lanes per key (8 dims each)
+  constexpr int NJ = LPK / 4;            // keys per lane: of the wave's 16, NJ r .. NJ r + NJ - 1
+  constexpr int N = 8 * GT;              // sums per lane
+  __shared__ __align__(16) float p_lds[WAVES][GT][16];          // a wave's probabilities
+  __shared__ float a_lds[WAVES][GT];                            // what its earlier sums are scaled by
+  __shared__ __align__(16) float o_lds[WAVES][GT][D];
+  __shared__ float2 ml_lds[WAVES][GT];
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int of_all = __builtin_amdgcn_readfirstlane(tid >> 6), group = of_all >> 2, wave = of_all & 3;
   const int kvh = blockIdx.x, split = blockIdx.y;
   const int G = a.G;
-  const int64_t row_stride = (int64_t)a.Hkv * D;   // halves between consecutive keys
+  const uint32_t row_bytes = (uint32_t)(a.Hkv * D) * 2u;   // between consecutive keys
   const int qrow = lane & 15, kg = lane >> 4;
-  const int dq = lane % LPK, kh = lane / LPK;
-  const int key_s = 16 * wave + (lane & 15);
+  const int d8 = lane % LPK, kh = lane / LPK;
+  const int key_s = 16 * wave + (lane & 15), key_v = 16 * wave + NJ * kh;
   const int nkeys_total = a.kend - a.kbeg;
   const int nchunks = (nkeys_total + kTileKeys - 1) / kTileKeys;
 
   uint4 kf[STEPS];
-  uint2 vf[NJ], vn[NJ];
-  // Requests this wave's 16 keys of K (into kf) and its dim slice of V (into vn) of chunk c.
+  uint4 vf[NJ], vn[NJ];
+  // Requests this wave's 16 keys of K (into kf) and of V (into vn) of chunk c.
 #define DH_ATTN_LOAD(c_)                                                                          \
   do {                                                                                            \
-    const int kbase_ = a.kbeg + (c_) * kTileKeys;                                                 \
-    const int nk_ = min(kTileKeys, a.kend - kbase_);                                              \
+    /* a group without a chunk asks for one row that is there: a condition around these loads */  \
+    /* would make the wait for the rows in front of them a wait for everything               */   \
+    const int kbase_ = a.kbeg + min((c_), nchunks - 1) * kTileKeys;                               \
+    const int nk_ = (c_) < nchunks ? min(kTileKeys, a.kend - kbase_) : 1;                         \
     /* first cache row of the chunk; in ring layout rows wrap at the window (a chunk never */     \
-    /* spans more keys than the window holds, so one conditional subtraction is enough)    */     \
+    /* spans more keys than the window holds, so one jump is enough).  What the lanes      */     \
+    /* share is scalar: a lane's address is one multiply-add behind a select               */     \
     int row0_ = a.kv_start + kbase_, wrap_ = 0x7fffffff;                                          \
     if (a.ring_window > 0) {                                                                      \
       row0_ = (int)((unsigned)row0_ % (unsigned)a.ring_window);                                   \
-      wrap_ = a.ring_window;                                                                      \
+      wrap_ = a.ring_window - row0_;                                                              \
     }                                                                                             \
-    int row_ = row0_ + min(key_s, nk_ - 1);                                                       \
-    row_ = row_ >= wrap_ ? row_ - wrap_ : row_;                                                   \
-    const __half* kp_ = a.K + (int64_t)row_ * row_stride + (int64_t)kvh * D + 8 * kg;             \
+    const int64_t at_ = (int64_t)row0_ * row_bytes + (int64_t)kvh * (2 * D);                      \
+    const int64_t jump_ = a.ring_window > 0 ? (int64_t)a.ring_window * row_bytes : 0;             \
+    const char* const k0_ = reinterpret_cast<const char*>(a.K) + at_;                             \
+    const char* const v0_ = reinterpret_cast<const char*>(a.V) + at_;                             \
+    const char* const k1_ = k0_ - jump_;                                                          \
+    const char* const v1_ = v0_ - jump_;                                                          \
+    const uint32_t i_ = (uint32_t)min(key_s, nk_ - 1);                                            \
+    const char* kp_ = ((int)i_ >= wrap_ ? k1_ : k0_) + (uint64_t)i_ * row_bytes + 16 * kg;        \
     _Pragma("unroll") for (int s = 0; s < STEPS; s++)                                             \
-      kf[s] = *reinterpret_cast<const uint4*>(kp_ + 32 * s);                                      \
+      kf[s] = *reinterpret_cast<const uint4*>(kp_ + 64 * s);                                      \
     _Pragma("unroll") for (int j = 0; j < NJ; j++) {                                              \
-      int r_ = row0_ + min(kh + KH * j, nk_ - 1);                                                 \
-      r_ = r_ >= wrap_ ? r_ - wrap_ : r_;                                                         \
-      vn[j] = *reinterpret_cast<const uint2*>(a.V + (int64_t)r_ * row_stride + (int64_t)kvh * D + \
-                                              DW * wave + 4 * dq);                                \
+      const uint32_t r_ = (uint32_t)min(key_v + j, nk_ - 1);                                      \
+      vn[j] = *reinterpret_cast<const uint4*>(((int)r_ >= wrap_ ? v1_ : v0_) + (uint64_t)r_ * row_bytes + 16 * d8); \
     }                                                                                             \
   } while (0)
 
   // The appended key/value in fragment form (QKV variant, owner workgroup): lanes whose key, or
   // whose clamped stand-in for a key past the end, is the appended one take it from here.
   uint4 knew[STEPS] = {};
-  uint2 vnew = make_uint2(0u, 0u);
+  uint4 vnew = make_uint4(0u, 0u, 0u, 0u);
 #define DH_ATTN_PATCH(c_)                                                                         \
   do {                                                                                            \
     if (QKV && (c_) == a.c_new) {                                                                 \
@@ -223,11 +222,12 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
         _Pragma("unroll") for (int s = 0; s < STEPS; s++) kf[s] = knew[s];                        \
       }                                                                                           \
       _Pragma("unroll") for (int j = 0; j < NJ; j++)                                              \
-        if (kh + KH * j >= a.j_new) vn[j] = vnew;                                                 \
+        if (key_v + j >= a.j_new) vn[j] = vnew;                                                   \
     }                                                                                             \
   } while (0)
 
-  if (!QKV && split < nchunks) DH_ATTN_LOAD(split);
+  int c = split + group * a.nsplit;
+  if (!QKV && split < nchunks) DH_ATTN_LOAD(c);
 
   // ---- query fragments (A operand): row = lane & 15 -> head row>>1, high part / residual
   half8_t qa[STEPS];
@@ -238,46 +238,61 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
     // layout through LDS.  Their loads go out before those of the first K/V chunk, so they
     // return first and the preparation runs under the latency of the cache reads.
     constexpr int EPL = D / 32;                       // elements per lane
-    constexpr int ROUNDS = (GT + 2 + 7) / 8;          // 8 half waves per round
-    __shared__ __align__(16) float q_rows[GT][D];
+    constexpr int ROUNDS = (GT + 2 + 8 * GROUPS - 1) / (8 * GROUPS);          // 8 GROUPS half waves per round
+    __shared__ __align__(16) __half q_rows[2][GT][D];  // the two parts of scale * q (see q_operand)
     __shared__ __align__(16) __half k_row[D];
     __shared__ __align__(16) __half v_row[D];
-    const bool owner = split == a.c_new % a.nsplit;
+    const bool owner = split == a.split_new;
     const int hl = lane & 31;
     const int rotary_dim = 2 * a.rotary_half;
     float rx[ROUNDS][EPL], rw[ROUNDS][EPL], rc[ROUNDS][EPL], rs[ROUNDS][EPL];
     int role[ROUNDS];                                  // 0 idle, 1 query head, 2 new key, 3 new value
+    typedef __attribute__((ext_vector_type(EPL))) float row_vec_t;
+    struct __attribute__((packed, aligned(4))) table_vec_t { float v[EPL]; };      // the tables' rows lie on any float
 #pragma unroll
     for (int r = 0; r < ROUNDS; r++) {
-      const int slot = 8 * r + 2 * wave + (lane >> 5);
+      const int slot = 8 * GROUPS * r + 2 * of_all + (lane >> 5);
       role[r] = slot < G ? 1 : (owner && slot == G) ? 2 : (owner && slot == G + 1) ? 3 : 0;
-      const int64_t row = role[r] == 1 ? kvh * G + slot : role[r] == 2 ? a.H + kvh : role[r] == 3 ? a.H + a.Hkv + kvh : 0;
-      const float* src = a.qkv + row * D + EPL * hl;
+      const int row = role[r] == 1 ? kvh * G + slot : role[r] == 2 ? a.H + kvh : role[r] == 3 ? a.H + a.Hkv + kvh : 0;
+      const float* src = a.qkv + (int64_t)row * D + EPL * hl;
       const float* wsrc = !a.use_norm ? nullptr : role[r] == 1 ? a.qw : role[r] == 2 ? a.kw : nullptr;
-      typedef __attribute__((ext_vector_type(EPL))) float row_vec_t;
       const row_vec_t xv = *reinterpret_cast<const row_vec_t*>(src);
       const row_vec_t wv = *reinterpret_cast<const row_vec_t*>((wsrc ? wsrc : a.qkv) + EPL * hl);
 #pragma unroll
       for (int i = 0; i < EPL; i++) {
-        const int e = EPL * hl + i;
-        const bool rotated = (role[r] == 1 || role[r] == 2) && e < rotary_dim;
-        const int p = a.interleaved ? e >> 1 : e & (a.rotary_half - 1);
         rx[r][i] = xv[i];
         rw[r][i] = wsrc ? wv[i] : 1.0f;
-        rc[r][i] = a.cos_row[rotated ? p : 0];
-        rs[r][i] = a.sin_row[rotated ? p : 0];
+      }
+      const bool turns = role[r] == 1 || role[r] == 2;
+      if (a.interleaved) {
+#pragma unroll
+        for (int i = 0; i < EPL; i++) {
+          const int e = EPL * hl + i;
+          const int p = turns && e < rotary_dim ? e >> 1 : 0;
+          rc[r][i] = a.cos_row[p];
+          rs[r][i] = a.sin_row[p];
+        }
+      } else {                  // a lane's elements are neighbours in the tables: the half is a power of two and no less than EPL
+        const int p = turns && EPL * hl < rotary_dim ? (EPL * hl) & (a.rotary_half - 1) : 0;
+        const table_vec_t cv = *reinterpret_cast<const table_vec_t*>(a.cos_row + p), sv = *reinterpret_cast<const table_vec_t*>(a.sin_row + p);
+#pragma unroll
+        for (int i = 0; i < EPL; i++) {
+          rc[r][i] = cv.v[i];
+          rs[r][i] = sv.v[i];
+        }
       }
     }
-    DH_ATTN_LOAD(split);        // never empty: there are no more splits than chunks
+    __builtin_amdgcn_sched_barrier(0);
+    DH_ATTN_LOAD(c);        // the first group's is never empty: there are no more splits than chunks
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < ROUNDS; r++) {
-      const int slot = 8 * r + 2 * wave + (lane >> 5);
+      const int slot = 8 * GROUPS * r + 2 * of_all + (lane >> 5);
       float y[EPL];
       float ss = 0.f;
 #pragma unroll
       for (int i = 0; i < EPL; i++) ss = fmaf(rx[r][i], rx[r][i], ss);
-#pragma unroll
-      for (int off = 1; off < 32; off <<= 1) ss += __shfl_xor(ss, off, 64);
+      ss = dh::group_combine<1, 32>(ss, dh::AddOp{});
       const bool normed = a.use_norm && (role[r] == 1 || role[r] == 2);
       const float inv = normed ? 1.0f / sqrtf(ss / (float)D + a.eps) : 1.0f;
 #pragma unroll
@@ -293,19 +308,39 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
           y[i + 1] = on ? x0 * rs[r][i + 1] + x1 * rc[r][i + 1] : x1;
         }
       } else {
-        const int pd = a.rotary_half / EPL;           // lanes between the partners (p, p + half)
+        const int pd = a.rotary_half / EPL;           // lanes between the partners (p, p + half): a power of two, 16 where the whole head turns
         const bool low = EPL * hl < a.rotary_half;
+        float other[EPL];
+        if (pd == 16) {
+#pragma unroll
+          for (int i = 0; i < EPL; i++) {
+            // of the pair, the result for the other sixteen lanes
+            auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(y[i]), __float_as_uint(y[i]), false, false);
+            other[i] = __uint_as_float((lane & 16) ? t[0] : t[1]);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < EPL; i++) other[i] = __shfl_xor(y[i], pd, 64);
+        }
 #pragma unroll
         for (int i = 0; i < EPL; i++) {
-          const float other = __shfl_xor(y[i], pd, 64);
-          const float x0 = low ? y[i] : other, x1 = low ? other : y[i];
+          const float x0 = low ? y[i] : other[i], x1 = low ? other[i] : y[i];
           const float rot = low ? x0 * rc[r][i] - x1 * rs[r][i] : x0 * rs[r][i] + x1 * rc[r][i];
           y[i] = rotates && EPL * hl + i < rotary_dim ? rot : y[i];
         }
       }
       if (role[r] == 1) {
+        // both parts of scale * q are made here, once, and not by every wave from the whole rows
+        typedef __attribute__((ext_vector_type(EPL / 2))) uint32_t part_vec_t;
+        part_vec_t hi, lo;
 #pragma unroll
-        for (int i = 0; i < EPL; i++) q_rows[min(slot, GT - 1)][EPL * hl + i] = y[i];
+        for (int i = 0; i < EPL / 2; i++) {
+          const QParts w = q_parts(y[2 * i] * a.scale, y[2 * i + 1] * a.scale);
+          hi[i] = w.high;
+          lo[i] = w.low;
+        }
+        *reinterpret_cast<part_vec_t*>(&q_rows[0][min(slot, GT - 1)][EPL * hl]) = hi;
+        *reinterpret_cast<part_vec_t*>(&q_rows[1][min(slot, GT - 1)][EPL * hl]) = lo;
       } else if (role[r] == 2 || role[r] == 3) {
         __half* lrow = role[r] == 2 ? k_row : v_row;
         __half* grow = (role[r] == 2 ? a.Kw : a.Vw) + a.new_row + (int64_t)kvh * D;
@@ -321,16 +356,14 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
     const bool live = (qrow >> 1) < G;
 #pragma unroll
     for (int s = 0; s < STEPS; s++) {
-      const float* qp = &q_rows[min(qrow >> 1, GT - 1)][32 * s + 8 * kg];
-      const float4 q0 = reinterpret_cast<const float4*>(qp)[0], q1 = reinterpret_cast<const float4*>(qp)[1];
-      const float qv[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-      qa[s] = q_operand(qv, live ? a.scale : 0.f, (qrow & 1) != 0);
+      const uint4 q = *reinterpret_cast<const uint4*>(&q_rows[qrow & 1][min(qrow >> 1, GT - 1)][32 * s + 8 * kg]);
+      qa[s] = __builtin_bit_cast(half8_t, live ? q : make_uint4(0u, 0u, 0u, 0u));
     }
     if (owner) {
 #pragma unroll
       for (int s = 0; s < STEPS; s++) knew[s] = *reinterpret_cast<const uint4*>(k_row + 32 * s + 8 * kg);
-      vnew = *reinterpret_cast<const uint2*>(v_row + DW * wave + 4 * dq);
-      DH_ATTN_PATCH(split);
+      vnew = *reinterpret_cast<const uint4*>(v_row + 8 * d8);
+      DH_ATTN_PATCH(c);
     }
   } else {
 #pragma unroll
@@ -345,17 +378,14 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
       }
     }
   }
-  float m_run[GT], l_run[GT], acc[GT][4];
+  // A wave is on its own from here to the end: its sixteen keys' scores, their softmax, their part of the sums.  Lane (key, kg) has heads
+  // 2 kg and 2 kg + 1 of its key, m is the same in the sixteen lanes of a kg, l a lane's own; lane (r, d8) adds 8 dims of NJ keys.
+  float m_run[2] = {-FLT_MAX, -FLT_MAX}, l_run[2] = {0.f, 0.f}, acc[N];
 #pragma unroll
-  for (int g = 0; g < GT; g++) {
-    m_run[g] = -FLT_MAX; l_run[g] = 0.f;
-    acc[g][0] = acc[g][1] = acc[g][2] = acc[g][3] = 0.f;
-  }
-  const int sm_g = lane / LH, sm_q = lane % LH;      // softmax role: head, key group
+  for (int n = 0; n < N; n++) acc[n] = 0.f;
 
-  for (int c = split; c < nchunks; c += a.nsplit) {
-    const int kbase = a.kbeg + c * kTileKeys;
-    const int nk = min(kTileKeys, a.kend - kbase);
+  for (bool first = true; c < nchunks; c += GROUPS * a.nsplit, first = false) {
+    const int nk = min(kTileKeys, a.kend - a.kbeg - c * kTileKeys);
     // ---- scores of 16 keys x G heads
     float4_t d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -363,112 +393,112 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(const AttnArgs a
       d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[s], __builtin_bit_cast(half8_t, kf[s]), d, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < NJ; j++) vf[j] = vn[j];
-    if (c + a.nsplit < nchunks) {
-      DH_ATTN_LOAD(c + a.nsplit);
-      DH_ATTN_PATCH(c + a.nsplit);
+    const int next = c + GROUPS * a.nsplit;
+    if (next < nchunks) {
+      DH_ATTN_LOAD(next);
+      DH_ATTN_PATCH(next);
     }
     // lane (key, kg) holds rows 4kg..4kg+3 = heads 2kg (high + residual), 2kg+1
-    {
-      float sc2[2] = {d[0] + d[1], d[2] + d[3]};
-      if (a.softcap > 0.f) {
+    float sc[2] = {d[0] + d[1], d[2] + d[3]};
+    if (a.softcap > 0.f) {
 #pragma unroll 1
-        for (int e = 0; e < 2; e++) sc2[e] = tanhf(sc2[e] / a.softcap) * a.softcap;
-      }
-      const bool valid = key_s < nk;
-      if (2 * kg < GT) s_lds[2 * kg][key_s] = valid ? sc2[0] : -FLT_MAX;
-      if (2 * kg + 1 < GT) s_lds[2 * kg + 1][key_s] = valid ? sc2[1] : -FLT_MAX;
+      for (int e = 0; e < 2; e++) sc[e] = tanhf(sc[e] / a.softcap) * a.softcap;
     }
-    __syncthreads();
-    // ---- online softmax: lane (head sm_g, group sm_q) owns keys sm_q*GT .. sm_q*GT + GT - 1
-    {
-      float sc[GT], pr[GT];
+    // ---- online softmax
+    const bool valid = key_s < nk;
 #pragma unroll
-      for (int i = 0; i < GT; i++) sc[i] = s_lds[sm_g][sm_q * GT + i];
-      float mx = sc[0];
-#pragma unroll
-      for (int i = 1; i < GT; i++) mx = fmaxf(mx, sc[i]);
-      mx = row_group_max<SPAN>(mx);
-      float m_new[GT], alpha[GT], my_m = 0.f;
-#pragma unroll
-      for (int g = 0; g < GT; g++) {
-        float m = m_run[g];
-#pragma unroll
-        for (int r = 0; r < LH / SPAN; r++)       // the head's rows (or its single group)
-          m = fmaxf(m, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx), g * LH + r * SPAN + SPAN - 1)));
-        m_new[g] = m;
-        alpha[g] = __expf(m_run[g] - m);
-        if (g == sm_g) my_m = m;
-      }
-      float ps = 0.f;
-#pragma unroll
-      for (int i = 0; i < GT; i++) {
-        pr[i] = sm_q * GT + i < nk ? __expf(sc[i] - my_m) : 0.f;
-        ps += pr[i];
-        p_lds[wave][sm_g][sm_q * GT + i] = pr[i];
-      }
-      ps = row_group_sum<SPAN>(ps);
-#pragma unroll
-      for (int g = 0; g < GT; g++) {
-        float t = 0.f;
-#pragma unroll
-        for (int r = 0; r < LH / SPAN; r++)
-          t += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ps), g * LH + r * SPAN + SPAN - 1));
-        l_run[g] = l_run[g] * alpha[g] + t;
-        m_run[g] = m_new[g];
-        acc[g][0] *= alpha[g]; acc[g][1] *= alpha[g]; acc[g][2] *= alpha[g]; acc[g][3] *= alpha[g];
+    for (int e = 0; e < 2; e++) {
+      const float m = fmaxf(m_run[e], dh::group_combine<1, 16>(valid ? sc[e] : -FLT_MAX, dh::MaxOp{}));
+      const float alpha = __expf(m_run[e] - m), p = valid ? __expf(sc[e] - m) : 0.f;
+      l_run[e] = l_run[e] * alpha + p;
+      m_run[e] = m;
+      if (2 * kg + e < GT) {
+        p_lds[of_all][2 * kg + e][qrow] = p;
+        if (!first && qrow == 0) a_lds[of_all][2 * kg + e] = alpha;
       }
     }
-    // ---- P.V for this wave's dims (p_lds[wave] is private to the wave: program order suffices)
+    // ---- P.V (both arrays are the wave's own: program order suffices)
+    if (!first) {
+#pragma unroll
+      for (int n = 0; n < N; n++) acc[n] *= a_lds[of_all][n >> 3];
+    }
+    float pr[GT][NJ];
+#pragma unroll
+    for (int g = 0; g < GT; g++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++) pr[g][j] = p_lds[of_all][g][NJ * kh + j];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-      const int key = kh + KH * j;
-      const __half2* h2 = reinterpret_cast<const __half2*>(&vf[j]);
-      const float2 v01 = __half22float2(h2[0]), v23 = __half22float2(h2[1]);
+      const half8_t v = __builtin_bit_cast(half8_t, vf[j]);
 #pragma unroll
-      for (int g = 0; g < GT; g++) {
-        const float p = p_lds[wave][g][key];
-        acc[g][0] = fmaf(p, v01.x, acc[g][0]);
-        acc[g][1] = fmaf(p, v01.y, acc[g][1]);
-        acc[g][2] = fmaf(p, v23.x, acc[g][2]);
-        acc[g][3] = fmaf(p, v23.y, acc[g][3]);
+      for (int i = 0; i < 8; i++) {
+        const float x = (float)v[i];
+#pragma unroll
+        for (int g = 0; g < GT; g++) acc[8 * g + i] = fmaf(pr[g][j], x, acc[8 * g + i]);
       }
     }
-    __syncthreads();     // s_lds is rewritten by the next chunk
   }
 #undef DH_ATTN_LOAD
 #undef DH_ATTN_PATCH
 
-  // ---- key groups meet in the wave's LDS buffer, then the split's (o, m, l) go out
+  // ---- the lanes of a dim meet: at each step a lane keeps the half of the sums that its bit says
 #pragma unroll
-  for (int g = 0; g < GT; g++)
-    *reinterpret_cast<float4*>(&o_lds[wave][kh][g][4 * dq]) = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+  for (int n = 0; n < N / 2; n++) {
+    auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[n]), __float_as_uint(acc[n + N / 2]), false, false);
+    acc[n] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+  }
 #pragma unroll
-  for (int t = 0; t < (GT * DW + 63) / 64; t++) {
-    const int o = lane + 64 * t, g = min(o / DW, GT - 1), dim = o % DW;
-    float v = 0.f;
+  for (int n = 0; n < N / 4; n++) {
+    auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[n]), __float_as_uint(acc[n + N / 4]), false, false);
+    acc[n] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+  }
+  int at = (lane >> 5) * (N / 2) + ((lane >> 4) & 1) * (N / 4);        // the first that this lane has in the end
+  if constexpr (D == 64) {
 #pragma unroll
-    for (int k = 0; k < KH; k++) v += o_lds[wave][k][g][dim];
-    if (o < GT * DW && g < G) {
-      const int h = kvh * G + g;
-      if (a.direct) {
-        float l = 0.f;
+    for (int n = 0; n < N / 8; n++) {                                   // (dpp 0x128: the lane eight further round its sixteen)
+      const float x = acc[n] + dh::dpp_lane<0x128>(acc[n]), y = acc[n + N / 8] + dh::dpp_lane<0x128>(acc[n + N / 8]);
+      acc[n] = (lane & 8) ? y : x;
+    }
+    at += ((lane >> 3) & 1) * (N / 8);
+  }
+  constexpr int KEPT = N * LPK / 64;
 #pragma unroll
-        for (int gg = 0; gg < GT; gg++) l = gg == g ? l_run[gg] : l;
-        a.O[(int64_t)h * D + DW * wave + dim] = l > 0.f ? v / l : 0.f;
-      } else {
-        a.ws[((int64_t)h * ws_stride + split) * (D + 2) + DW * wave + dim] = v;
+  for (int n = 0; n < KEPT; n++) o_lds[of_all][(at + n) >> 3][8 * d8 + ((at + n) & 7)] = acc[n];
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const float l = dh::group_combine<1, 16>(l_run[e], dh::AddOp{});
+    if (qrow == 0 && 2 * kg + e < GT) ml_lds[of_all][2 * kg + e] = make_float2(m_run[e], l);
+  }
+  __syncthreads();
+  // ---- the waves meet, and the split's (o, m, l) go out
+#pragma unroll
+  for (int t = 0; t < (GT * D + 64 * WAVES - 1) / (64 * WAVES); t++) {
+    const int o = tid + 64 * WAVES * t, g = o / D, dim = o % D;
+    if (o >= GT * D || g >= G) continue;
+    float2 ml[WAVES];
+    float m = -FLT_MAX, l = 0.f, v = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+      ml[w] = ml_lds[w][g];
+      m = fmaxf(m, ml[w].x);
+    }
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+      const float f = __expf(ml[w].x - m);
+      l = fmaf(f, ml[w].y, l);
+      v = fmaf(f, o_lds[w][g][dim], v);
+    }
+    const int64_t h = kvh * G + g;
+    if (a.direct) {
+      a.O[h * D + dim] = l > 0.f ? v / l : 0.f;
+    } else {
+      float* const part = a.ws + (h * ws_stride + split) * (D + 2);
+      part[dim] = v;
+      if (dim == 0) {
+        part[D] = m;
+        part[D + 1] = l;
       }
     }
-  }
-  if (!a.direct && wave == 0 && lane < G) {
-    float* w = a.ws + ((int64_t)(kvh * G + lane) * ws_stride + split) * (D + 2);
-    float mv = 0.f, lv = 0.f;
-#pragma unroll
-    for (int g = 0; g < GT; g++) {     // pick this lane's head without dynamic register indexing
-      if (g == lane) { mv = m_run[g]; lv = l_run[g]; }
-    }
-    w[D] = mv;
-    w[D + 1] = lv;
   }
 }
 
@@ -553,20 +583,28 @@ typedef void (*SplitKernel)(const AttnArgs);
 typedef void (*MergeKernel)(const float*, float*, int, const DynKeys);
 
 template <int D, bool QKV>
-SplitKernel split_kernel_for(int G) {
-  if (G <= 1) return attn_decode_split_kernel<D, 1, QKV>;
-  if (G <= 2) return attn_decode_split_kernel<D, 2, QKV>;
-  if (G <= 4) return attn_decode_split_kernel<D, 4, QKV>;
-  return attn_decode_split_kernel<D, 8, QKV>;
+SplitKernel split_kernel_for(int G, bool two) {
+  if (G <= 1) return two ? attn_decode_split_kernel<D, 1, QKV, 2> : attn_decode_split_kernel<D, 1, QKV, 1>;
+  if (G <= 2) return two ? attn_decode_split_kernel<D, 2, QKV, 2> : attn_decode_split_kernel<D, 2, QKV, 1>;
+  if (G <= 4) return two ? attn_decode_split_kernel<D, 4, QKV, 2> : attn_decode_split_kernel<D, 4, QKV, 1>;
+  return two ? attn_decode_split_kernel<D, 8, QKV, 2> : attn_decode_split_kernel<D, 8, QKV, 1>;
 }
-SplitKernel split_kernel_for(int D, bool qkv, int G) {
-  if (D == 64) return qkv ? split_kernel_for<64, true>(G) : split_kernel_for<64, false>(G);
-  return qkv ? split_kernel_for<128, true>(G) : split_kernel_for<128, false>(G);
+SplitKernel split_kernel_for(int D, bool qkv, int G, bool two) {
+  if (D == 64) return qkv ? split_kernel_for<64, true>(G, two) : split_kernel_for<64, false>(G, two);
+  return qkv ? split_kernel_for<128, true>(G, two) : split_kernel_for<128, false>(G, two);
+}
+// Whether a split has chunks for a second group of waves (2049 keys of 32/8 heads, two chunks a split: the step of 36 layers 1626 us with one
+// group, 1608 with two; 6000 keys 10.1 / 9.7 us; without a second chunk the group would only wait).  A call that is recorded for replays at other
+// positions has two at every length, since a replay changes the grid and not the kernel; the sums are the same.
+bool two_groups(const AttnArgs& a, bool recorded) {
+  const int keys = a.dyn.kv_len_ptr ? a.dyn.max_kv_len : a.kend - a.kbeg;
+  return recorded || dh::ceil_div(keys, kTileKeys) > a.nsplit;
 }
 MergeKernel merge_kernel_for(int D) { return D == 64 ? attn_decode_merge_kernel<64> : attn_decode_merge_kernel<128>; }
 
-int launch(const AttnArgs& a, int D, bool qkv, const char* op, bool merge = true) {
-  hipLaunchKernelGGL(split_kernel_for(D, qkv, a.G), dim3(a.Hkv, a.nsplit), dim3(256), 0, dh::stream(), a);
+int launch(const AttnArgs& a, int D, bool qkv, const char* op, bool merge = true, bool recorded = false) {
+  const bool two = two_groups(a, recorded);
+  hipLaunchKernelGGL(split_kernel_for(D, qkv, a.G, two), dim3(a.Hkv, a.nsplit), dim3(two ? 512 : 256), 0, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   if (!a.direct && merge) {
     hipLaunchKernelGGL(merge_kernel_for(D), dim3(a.H), dim3(D), 0, dh::stream(), a.ws, a.O, a.nsplit, a.dyn);
@@ -614,6 +652,7 @@ int build_args(const dh::GraphAttnCall& c, int delta, bool force_merge, AttnArgs
     a.new_row = row * c.Hkv * c.D;
     a.c_new = (nkeys - 1) / kTileKeys;
     a.j_new = (nkeys - 1) % kTileKeys;
+    a.split_new = a.c_new % a.nsplit;
   } else {
     a.Q = c.q;
   }
@@ -693,7 +732,7 @@ int attn_graph_bind(Graph* g) {
     }
     if (ci < g->n_attn) {
       const GraphAttnCall& c = g->attn[ci];
-      if (kp.func == reinterpret_cast<void*>(split_kernel_for(c.D, c.qkv != 0, c.H / c.Hkv))) {
+      if (kp.func == reinterpret_cast<void*>(split_kernel_for(c.D, c.qkv != 0, c.H / c.Hkv, true))) {
         g->attn[ci].split_node = order[i];
         want_merge = true;
       }
@@ -720,9 +759,9 @@ int attn_graph_set_position(Graph* g, int position) {
     AttnArgs* ap = &a;
     void* split_args[] = {ap};
     hipKernelNodeParams sp{};
-    sp.func = reinterpret_cast<void*>(split_kernel_for(c.D, c.qkv != 0, a.G));
+    sp.func = reinterpret_cast<void*>(split_kernel_for(c.D, c.qkv != 0, a.G, true));
     sp.gridDim = dim3(a.Hkv, a.nsplit);
-    sp.blockDim = dim3(256);
+    sp.blockDim = dim3(512);
     sp.sharedMemBytes = 0;
     sp.kernelParams = split_args;
     DH_CHECK_HIP("dh_graph_launch", hipGraphExecKernelNodeSetParams(g->exec, c.split_node, &sp));
@@ -808,7 +847,7 @@ static int attn_decode_impl(const char* op, const float* d_Q, const void* d_K, c
     return dh::fail(1, "[%s] numHeads=%d, headDim=%d with %d key splits needs %zu bytes of split partials, the "
                        "scratch holds %zu: use dh_attn_decode with a workspace", op, H, D, a.nsplit, ws_need, ws_capacity);
   dh::graph_note_attention(c);
-  return launch(a, D, false, op);
+  return launch(a, D, false, op, true, capturing);
 }
 
 int dh_attn_decode(const float* d_Q, const void* d_K, const void* d_V, float* d_O, int H, int Hkv, int D,
@@ -889,7 +928,7 @@ static int attn_decode_qkv_impl(const char* op, const float* d_qkv, const float*
     return launch(a, D, true, op, false);
   }
   dh::graph_note_attention(c);
-  return launch(a, D, true, op);
+  return launch(a, D, true, op, true, capturing);
 }
 
 int dh_attn_decode_qkv(const float* d_qkv, const float* d_q_weight, const float* d_k_weight, const float* d_cos,

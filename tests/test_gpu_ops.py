@@ -1232,6 +1232,14 @@ def test_attention_decode_from_qkv_options():
                                       ops.acquireBuffer(4096), ops.acquireBuffer(4096), 16, 8, 128, 0, rotaryDim=96)
 
 
+# 64 kv heads: four workgroups a head fill the device, so a fifth chunk of 64 keys is where a workgroup gets its second four waves; then last chunks
+# of one key and of all, an odd number of chunks (a second group that has none), three chunks a group, rings that end inside a chunk
+@pytest.mark.parametrize("H,D,pos,window", [(64, 128, 255, 0), (64, 128, 256, 0), (128, 64, 319, 0), (192, 128, 320, 0), (320, 64, 447, 0), (512, 128, 448, 0),
+                                            (64, 64, 1300, 0), (128, 128, 1700, 300), (512, 64, 290, 300), (256, 64, 2000, 513)])
+def test_attention_decode_of_two_groups(H, D, pos, window):
+    _fused_case(H, 64, D, pos, seed=5700 + pos, window=window, ring=window > 0)
+
+
 def test_attention_decode_from_qkv_matches_separate_ops_without_norm():
     H, Hkv, D, pos = 32, 8, 128, 700
     cos, sin = synth.rope_tables(D, pos + 1, 1e6)

@@ -20,6 +20,8 @@
 // Tried there: four activation buffers instead of two (no change: a fetch is not what a step waits for), the weights
 // dequantised to f16 in memory by a pre-pass for gemm_wide.h (the same at 2048 rows, slower below).
 //
+// Products of few rows take it too, on tiles of 32 or 64 rows whose waves share k (choose_narrow).
+//
 // q4k_gemm_kernel (the rest): a wave computes a 64 x 64 (or 32 x 32) quadrant with v_mfma_f32_32x32x16_f16, four waves a
 // 128 x 128 (64 x 64) tile, and a workgroup is one or two such groups stacked along M against the same weight tile.  K advances 64
 // at a time; a thread loads 8 or 16 nibble bytes of a row and the block header, and the weights of a tile are dequantised once
@@ -564,7 +566,8 @@ __global__ __launch_bounds__(256 * MG) void q4k_gemm_kernel(const GemmArgs a) {
 }
 
 // ---- the wide kernel
-// WM x WN waves; a wave computes 32 RA rows x 64 columns (DUAL: 32 columns of both matrices).
+// WM x WN waves; a wave computes 32 RA rows x 64 columns (DUAL: 32 columns of both matrices).  KG such groups of waves, each with tiles of its own,
+// take runs of the super-blocks; their sums meet in LDS at the end.
 template <int WM_, int WN_, int RA_>
 struct Q4Tile {
   static constexpr int WM = WM_, WN = WN_, RA = RA_;
@@ -577,21 +580,26 @@ struct Q4Tile {
   static_assert(kBufA % (1024 * kWaves) == 0 && kRowsWave <= 32 * WN && kRowsWave % 32 == 0, "whole loads; a wave fetches rows of one matrix");
 };
 
-template <class Tile, bool DUAL>
-__global__ __launch_bounds__(Tile::kThreads, 2) void q4k_wide_kernel(const GemmArgs a) {
+template <class Tile, bool DUAL, int KG>
+__global__ __launch_bounds__(Tile::kThreads * KG, 2) void q4k_wide_kernel(const GemmArgs a) {
   constexpr int RA = Tile::RA, WN = Tile::WN, NB = Tile::kRoundsB, NA = Tile::kRoundsA;
   constexpr int BN = DUAL ? Tile::kRows / 2 : Tile::kRows;
-  extern __shared__ __align__(16) char smem[];
+  extern __shared__ __align__(16) char smem_all[];
   __shared__ float rs_lds[Tile::BM];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = KG > 1 ? wave_all / Tile::kWaves : 0, wave = wave_all - group * Tile::kWaves;
+  char* const smem = smem_all + group * Tile::kLds;
   const int wm = wave / WN, wn = wave % WN;
   const int tile = dh::xcd_contiguous(blockIdx.x, a.tiles_m * a.tiles_n);
   const int m0 = (tile % a.tiles_m) * Tile::BM, n0 = (tile / a.tiles_m) * BN;
   const int fr = lane & 31, fh = lane >> 5;
-  const int kt0 = a.ksplit > 1 ? (int)blockIdx.z * a.kt_per_split : 0;    // a multiple of 4
-  const int nk = (a.ksplit > 1 ? min((a.K + BK - 1) / BK, kt0 + a.kt_per_split) : (a.K + BK - 1) / BK) - kt0;
+  const int kt_first = a.ksplit > 1 ? (int)blockIdx.z * a.kt_per_split : 0;    // a multiple of 4
+  const int steps = (a.ksplit > 1 ? min((a.K + BK - 1) / BK, kt_first + a.kt_per_split) : (a.K + BK - 1) / BK) - kt_first;
+  // a group's steps: whole super-blocks, at least one (the host sees to KG of them)
+  auto group_first = [&](int g) { return min((steps + 3) / 4 * g / KG * 4, steps); };
+  const int kt0 = kt_first + group_first(group), nk = group_first(group + 1) - group_first(group);
   const int sb0 = kt0 >> 2, sb_last = (kt0 + nk - 1) >> 2;
-  for (int r = threadIdx.x; r < Tile::BM; r += Tile::kThreads) rs_lds[r] = a.row_scale[min(m0 + r, a.M - 1)].y;
+  for (int r = threadIdx.x; r < Tile::BM; r += Tile::kThreads * KG) rs_lds[r] = a.row_scale[min(m0 + r, a.M - 1)].y;
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   // ---- fetches
@@ -723,9 +731,9 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void q4k_wide_kernel(const GemmA
         for (int f = 0; f < 2; f++)
 #pragma unroll
           for (int stage = 0; stage < 3; stage++)
-            if (n == (NM == 4 ? f + stage : 3 * f + stage)) dequant(stage, f, next_ks, src, dst);
+            if (n == (NM == 2 ? stage / 2 : NM == 4 ? f + stage : 3 * f + stage)) dequant(stage, f, next_ks, src, dst);
         if (ks == 1 || ks == 2) {
-          if (n == (NM == 4 ? 0 : 6)) bits = scale_bits(hdr[ks - 1], (C + 1) & 3);
+          if (n == (NM <= 4 ? 0 : 6)) bits = scale_bits(hdr[ks - 1], (C + 1) & 3);
           if (n == NM - 1) ps[Q][ks - 1] = pair_scales_f16(hdr[ks - 1], bits);
         }
       });
@@ -760,7 +768,39 @@ __global__ __launch_bounds__(Tile::kThreads, 2) void q4k_wide_kernel(const GemmA
     now = next;
     next = was;
   }
+  if constexpr (KG > 1) {                  // steps that other groups have more
+    int most = 0;
+#pragma unroll
+    for (int g = 0; g < KG; g++) most = max(most, group_first(g + 1) - group_first(g));
+    for (int i = nk; i < most; i++) dh::arrive_and_wait<0>();
+  }
   dh::arrive_and_wait<0>();                // nothing may be in flight towards LDS when the workgroup ends
+  if constexpr (KG > 1) {
+    // the other groups' sums go where their tiles were and are added in group order
+    static_assert(RA * 2 * 64 * Tile::kThreads <= Tile::kLds, "a group's sums fit where its tiles were");
+    auto sums_of = [&](int g) { return reinterpret_cast<float4*>(smem_all + g * Tile::kLds) + (wave * 64 + lane); };
+    if (group > 0) {
+#pragma unroll
+      for (int q = 0; q < 2 * RA; q++)
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) {
+          const float16_t& v = acc[q >> 1][q & 1];
+          sums_of(group)[(4 * q + e / 4) * Tile::kThreads] = make_float4(v[e], v[e + 1], v[e + 2], v[e + 3]);
+        }
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; g++)
+#pragma unroll
+      for (int q = 0; q < 2 * RA; q++)
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) {
+          float16_t& v = acc[q >> 1][q & 1];
+          const float4 other = sums_of(g)[(4 * q + e / 4) * Tile::kThreads];
+          v[e] += other.x; v[e + 1] += other.y; v[e + 2] += other.z; v[e + 3] += other.w;
+        }
+  }
 
   store_results<DUAL, DUAL ? RA : 2 * RA>(
       a, m0, [&](int q, int matrix, int e) { return DUAL ? acc[q][matrix][e] : acc[q >> 1][q & 1][e]; },
@@ -848,14 +888,14 @@ int launch_gemm_cfg(const GemmArgs& a, const char* op) {
   return a.ksplit > 1 ? launch_reduce(a, op) : 0;
 }
 
-template <class Tile, bool DUAL>
+template <class Tile, bool DUAL, int KG = 1>
 int launch_wide(GemmArgs a, const char* op) {
-  auto kern = q4k_wide_kernel<Tile, DUAL>;
-  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLds);
+  auto kern = q4k_wide_kernel<Tile, DUAL, KG>;
+  static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, KG * Tile::kLds);
   DH_CHECK_HIP(op, set);
   a.tiles_m = (int)dh::ceil_div(a.M, Tile::BM);
   a.tiles_n = (int)dh::ceil_div(a.N, DUAL ? Tile::kRows / 2 : Tile::kRows);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n), 1, (unsigned)std::max(1, a.ksplit)), dim3(Tile::kThreads), Tile::kLds, dh::stream(), a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n), 1, (unsigned)std::max(1, a.ksplit)), dim3(Tile::kThreads * KG), KG * Tile::kLds, dh::stream(), a);
   DH_CHECK_LAUNCH(op);
   return 0;
 }
@@ -902,15 +942,18 @@ WideChoice choose_wide(int64_t M, int64_t N, int64_t K, bool dual) {
 // Steps of 64 k in a piece.
 int64_t steps_per_piece(int64_t K, int pieces) { return dh::ceil_div(dh::ceil_div(K, BK), 4 * pieces) * 4; }
 
+void cut(GemmArgs& a, int pieces) {
+  if (pieces <= 1) return;
+  a.kt_per_split = (int)steps_per_piece(a.K, pieces);
+  a.ksplit = (int)dh::ceil_div(dh::ceil_div(a.K, BK), a.kt_per_split);
+  size_t ws_bytes = 0;
+  if (a.ksplit > 1) a.partial = dh::splitk_workspace(&ws_bytes);
+}
+
 template <bool DUAL>
 int launch_wide_best(GemmArgs a, const char* op) {
   const WideChoice pick = choose_wide(a.M, a.N, a.K, DUAL);
-  if (pick.pieces > 1) {
-    a.kt_per_split = (int)steps_per_piece(a.K, pick.pieces);
-    a.ksplit = (int)dh::ceil_div(dh::ceil_div(a.K, BK), a.kt_per_split);
-    size_t ws_bytes = 0;
-    if (a.ksplit > 1) a.partial = dh::splitk_workspace(&ws_bytes);
-  }
+  cut(a, pick.pieces);
   int rc;
   switch (pick.tile) {
     case 0: rc = launch_wide<Q4Tile<2, 4, 4>, DUAL>(a, op); break;
@@ -921,15 +964,54 @@ int launch_wide_best(GemmArgs a, const char* op) {
   return rc || a.ksplit <= 1 ? rc : launch_reduce(a, op);
 }
 
-// Products of enough work, or of enough tiles, go to q4k_wide_kernel: where a step's latency counts instead of its throughput the other
+// Products of enough work, or of enough tiles, go to q4k_wide_kernel's large tiles: where a step's latency counts instead of its throughput the other
 // kernel is ahead, because its waves share one dequantised tile (us, that one / the wide one, weights from memory: 128 x 1152 x 6912 20 / 28,
-// 512 x 1152 x 6912 33.2 / 33.2, 64 x 4096 x 4096 23.5 / 24.7, but 1024 x 2048 x 1024 25.3 / 24.3, 200 x 6144 x 4096 39.5 / 37.3, 512 x 4096 x 12288
+// 512 x 1152 x 6912 33.2 / 33.2, but 1024 x 2048 x 1024 25.3 / 24.3, 200 x 6144 x 4096 39.5 / 37.3, 512 x 4096 x 12288
 // 142 / 82; a threshold of the product's size, as the costs of the other kernel are not in the table: over 236 shapes 1.5 % behind the best).  Pairs of
-// few steps stay there at any height (2048 x 1024 x 512 18 / 21, 1024 x 2048 x 1024 22 / 24), and up to 64 rows as long as its 64-row tiles
-// are resident at once (64 x 12288 x 4096 44 / 50, 48 x 16000 x 4096 44 / 51, but 64 x 20000 x 4096 80 / 62).
+// few steps stay there at any height (2048 x 1024 x 512 18 / 21, 1024 x 2048 x 1024 22 / 24).
 bool takes_wide(int64_t M, int64_t N, int64_t K, bool dual) {
-  if (dual && M <= 64 && dh::ceil_div(N, 64) <= dh::num_cus()) return false;
   return dh::ceil_div(M, 256) * dh::ceil_div(N, 128) >= dh::num_cus() || (double)M * N * K * (dual ? 2 : 1) >= (M >= 1024 && !dual ? 2e9 : 5e9);
+}
+
+// Few rows: q4k_wide_kernel on tiles of 32 or 64 rows x 128 weight rows (two waves), two such groups along k (three: 35.3 -> 37.8 us for the
+// pair of 64 x 12288 x 4096, their waves do not divide among four SIMDs).  There a weight is dequantised once, in the registers of the wave that
+// multiplies it, and read from LDS as nibbles; q4k_gemm_kernel writes and reads it there as f16 and reads the activations for every 32 columns: 72 KB a
+// step of 64 k, which at 128 bytes a clock is most of its 0.6 us, whatever the number of rows.  us with packing and reduction, weights from memory, before
+// / now: pairs 16 x 12288 x 4096 42.6 / 30.3, 64 x 12288 x 4096 44 / 35, 40 x 6144 x 2048 24.3 / 18.0, 33 x 3072 x 1024 14.5 / 12.0, 512 x 1024 x 4096 40.8 / 30.3;
+// products 16 x 4096 x 4096 17.6 / 14.5, 20 x 4096 x 12288 29.2 / 21.6, 64 x 12288 x 2048 25.0 / 18.2, 16 x 28672 x 4096 51 / 30.
+// What a super-block costs a group was fitted to those (3.0 us on 32 rows, 3.7 on 64), as long as the tiles run at once.  Where the lines lie: pairs of
+// over 512 rows (796 x 1536 x 1472 27.7 / 28.2) or under 1024 k on 64-row tiles (170 x 5000 x 640 13.3 / 14.1), products of under 8e6 weights or 2048 columns (64 x 2048 x 2048 12.0 / 13.2, 16 x 2048 x 3072 11.8 / 12.3,
+// but 16 x 2048 x 4096 16.1 / 12.6; 54 x 1536 x 5504 15.3 / 16.4), of over 64 rows that take long (122 x 8448 x 8448 42 / 54, 67 x 6208 x 8320 32.6 / 36.9, but
+// 100 x 12000 x 2000 27.1 / 21.0, 128 x 2048 x 6144 25.3 / 21.3).
+constexpr int kNarrowGroups = 2;
+struct NarrowChoice {
+  int bm, pieces;                // rows of a tile (0: another kernel serves the product), pieces of K
+};
+NarrowChoice choose_narrow(int64_t M, int64_t N, int64_t K, bool dual) {
+  const int64_t cus = dh::num_cus(), blocks = dh::ceil_div(K, kQK);
+  if (blocks < kNarrowGroups) return {0, 1};
+  if (dual ? M > 512 : M > 128 || N < 2048 || N * K < 8000000) return {0, 1};
+  size_t ws_bytes = 0;
+  (void)dh::splitk_workspace(&ws_bytes);
+  const int64_t most = dual ? 1 : std::min<int64_t>({kMaxSplit, blocks / kNarrowGroups, std::max<int64_t>(1, ws_bytes / ((size_t)M * N * sizeof(float)))});
+  NarrowChoice best{0, 1};
+  double least = !dual && M > 64 ? 20000.0 : 1e30;
+  for (int bm = 32; bm <= 64; bm += 32) {
+    const int64_t groups = dh::ceil_div(M, bm) * dh::ceil_div(N, dual ? 64 : 128);
+    if (dual && bm == 64 && K < 1024) break;
+    for (int64_t s = 1; s <= most; s++) {
+      const int64_t each = steps_per_piece(K, (int)s) / 4, pieces = dh::ceil_div(blocks, each), rounds = dh::ceil_div(groups * pieces, cus);
+      if (rounds > (M <= 32 && s == 1 ? 2 : 1)) break;
+      if (blocks - each * (pieces - 1) < kNarrowGroups) continue;         // the last piece, too, has a super-block for each group
+      double t = (double)rounds * dh::ceil_div(each, kNarrowGroups) * (bm == 32 ? 3000.0 : 3700.0);
+      if (pieces > 1) t += 3500.0 + 4.0 * M * N * (2 * pieces + 1) / 4000.0;
+      if (t < least) {
+        least = t;
+        best = NarrowChoice{bm, (int)s};
+      }
+    }
+  }
+  return best;
 }
 
 // 128 x 128 tiles when they occupy at least half of the compute units (their higher matrix-core
@@ -981,6 +1063,11 @@ int launch_gemm(GemmArgs a, const char* op) {
   a.row_scale = scales;
   a.Apk = packed;
   a.ksplit = 1;
+  if (const NarrowChoice pick = choose_narrow(a.M, a.N, a.K, DUAL); pick.bm > 0) {
+    cut(a, pick.pieces);
+    const int rc = pick.bm == 32 ? launch_wide<Q4Tile<1, 2, 1>, DUAL, kNarrowGroups>(a, op) : launch_wide<Q4Tile<1, 2, 2>, DUAL, kNarrowGroups>(a, op);
+    return rc || a.ksplit <= 1 ? rc : launch_reduce(a, op);
+  }
   if (takes_wide(a.M, a.N, a.K, DUAL)) return launch_wide_best<DUAL>(a, op);
   // The other kernel: for the fused gate/up pair 128 x 64 tiles (eight waves), then 128 x 128 (four waves, two workgroups per compute
   // unit) when those occupy at least half of the compute units, else 64 x 64.
@@ -1073,7 +1160,7 @@ int q4k_gemm_gate_up(const char* op, const float* A, const uint8_t* Wg, const ui
 extern "C" int dh_q4k_gemm_layout(int M, int N, int K, int dual, int num_cus, int64_t* out4) {
   if (!out4 || M < 16 || N <= 0 || K <= 0) return 0;
   dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
-  const int wide = takes_wide(M, N, K, dual != 0) ? 1 : 0;
+  const int wide = takes_wide(M, N, K, dual != 0) && choose_narrow(M, N, K, dual != 0).bm == 0 ? 1 : 0;
   const WideChoice pick = choose_wide(M, N, K, dual != 0);
   dh::plan_end();
   const int64_t steps = dh::ceil_div(K, BK);
@@ -1081,4 +1168,14 @@ extern "C" int dh_q4k_gemm_layout(int M, int N, int K, int dual, int num_cus, in
   const int64_t out[4] = {kWide[pick.tile].bm, kWide[pick.tile].rows, rows_per_wave[pick.tile], dh::ceil_div(steps, steps_per_piece(K, pick.pieces))};
   for (int i = 0; i < 4; i++) out4[i] = wide ? out[i] : 0;
   return wide;
+}
+
+extern "C" int dh_q4k_gemm_narrow_layout(int M, int N, int K, int dual, int num_cus, int64_t* out2) {
+  if (!out2 || M < 16 || N <= 0 || K <= 0) return 0;
+  dh::plan_begin(num_cus > 0 ? num_cus : dh::ready() ? dh::num_cus() : 256);
+  const NarrowChoice pick = choose_narrow(M, N, K, dual != 0);
+  dh::plan_end();
+  out2[0] = pick.bm;
+  out2[1] = pick.bm ? dh::ceil_div(dh::ceil_div(K, BK), steps_per_piece(K, pick.pieces)) : 0;
+  return pick.bm ? 1 : 0;
 }

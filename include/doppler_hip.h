@@ -171,6 +171,8 @@ int dh_q4k_gemv_layout(int M, int N, int K, int normed, int dual, int num_cus, i
  * a tile, weight rows of a tile (of both matrices of a pair), rows of a wave, pieces K is cut into }.  Returns 1, or 0 with zeros where the
  * kernel for smaller products serves the shape.  For tests that have to reach every tile; needs no device. */
 int dh_q4k_gemm_layout(int M, int N, int K, int dual, int num_cus, int64_t* out4);
+/* The same for the tiles of few rows (dh_q4k_gemm_layout returns 0 for what takes them): out2 = { rows of a tile (32, 64), pieces K is cut into }. */
+int dh_q4k_gemm_narrow_layout(int M, int N, int K, int dual, int num_cus, int64_t* out2);
 
 /* out[M,inter] = clamp(act(x.Wgate^T) * (x.Wup^T) * alpha).
  * Replaces runFusedFFN/recordFusedFFN, src/gpu/kernels/fused_ffn.js:501,605

@@ -149,6 +149,8 @@ int dh_embed_sum_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t
                        int64_t mul_prev, int64_t mul_cur, const void* d_pos, int max_positions, float* d_out, int ld_out, int hidden, int pos) {
   EmbedArgs a = embed_args(d_embed, vocab, d_bigram, buckets, mul_prev, mul_cur, d_pos, max_positions, d_out, ld_out, hidden, pos);
   a.words = d_words; a.id = id; a.count = kv_len; a.before = before;
+  DH_REQUIRE_INIT("dh_embed_sum_words");
+  if (dh::capturing_graph()) return dh::fail(1, "[dh_embed_sum_words] not possible while a graph is being captured (a replay would set the same words)");
   return embed_sum("dh_embed_sum_words", a, 1, true);
 }
 

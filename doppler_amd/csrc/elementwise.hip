@@ -856,6 +856,7 @@ int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int 
 int dh_gather_f16_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_table, float* d_out, int hidden, int vocab) {
   const char* op = "dh_gather_f16_words";
   DH_REQUIRE_INIT(op);
+  if (dh::capturing_graph()) return dh::fail(1, "[%s] not possible while a graph is being captured (a replay would set the same words)", op);
   if (hidden <= 0 || vocab <= 0) return dh::fail(1, "[%s] hiddenSize/vocabSize must be positive", op);
   if (!d_words || !d_table || !d_out) return dh::fail(1, "[%s] null pointer", op);
   hipLaunchKernelGGL(gather_f16_words_kernel, dim3((unsigned)dh::ceil_div(std::max(hidden, 3), 256)), dim3(256), 0, dh::stream(), d_words, id, kv_len, before,

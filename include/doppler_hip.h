@@ -440,7 +440,7 @@ int dh_embed_sum(const uint32_t* d_ids, int index_offset, const uint32_t* d_prev
                  int max_positions, float* d_out, int ld_out, int T, int hidden, int start_pos, const uint32_t* d_kv_len);
 
 /* One token from the host: dh_set_words of (id, kv_len, before) to d_words and dh_embed_sum of id at position pos, `before` the token in front of it, in
- * one launch. */
+ * one launch; refused while a graph is being captured, like dh_set_words. */
 int dh_embed_sum_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_embed, int vocab, const void* d_bigram,
                        int64_t buckets, int64_t mul_prev, int64_t mul_cur, const void* d_pos, int max_positions, float* d_out, int ld_out,
                        int hidden, int pos);
@@ -687,7 +687,7 @@ int dh_scale(const float* d_in, float* d_out, int64_t n, float scale);
 int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int T, int hidden,
                   int vocab, int index_offset);
 
-/* One token from the host: dh_set_words of (id, kv_len, before) to d_words and the row of id, in one launch. */
+/* One token from the host: dh_set_words of (id, kv_len, before) to d_words and the row of id, in one launch; refused while a graph is being captured. */
 int dh_gather_f16_words(uint32_t* d_words, uint32_t id, uint32_t kv_len, uint32_t before, const void* d_table, float* d_out, int hidden, int vocab);
 
 /* out = clamp(act(gate) * up).  Replaces runSiLU with `gate` (src/gpu/kernels/silu.js:95,

@@ -1,4 +1,6 @@
 """Words of a step that travel as launch arguments and come back through pinned memory."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -61,6 +63,24 @@ def test_words_and_embedding_in_one_launch(hidden, buckets, pos):
         capi.check(L.dh_gather_f16_words(got.data_ptr(), token, 0, 7, half.data_ptr(), outs[3].data_ptr(), hidden, vocab))
         capi.check(L.dh_sync())
         assert torch.equal(outs[2], outs[3]) and torch.equal(ids, got)
+
+
+def test_words_of_a_token_are_refused_while_a_graph_is_captured():
+    """A replay would set the same words: the refusal of dh_set_words, in front of anything that would go into the graph."""
+    L = capi.init(torch.cuda.current_device())
+    half, out, ids = torch.ones(8, 8, dtype=torch.float16, device="cuda"), torch.full((64,), 3.0, device="cuda"), torch.full((4,), 9, dtype=torch.int32, device="cuda")
+    cleared, g = torch.ones(64, device="cuda"), ctypes.c_void_p()
+    torch.cuda.synchronize()
+    capi.check(L.dh_graph_begin())
+    refused = [(L.dh_gather_f16_words(ids.data_ptr(), 1, 0, 0, half.data_ptr(), out.data_ptr(), 8, 8), L.dh_last_error().decode()),
+               (L.dh_embed_sum_words(ids.data_ptr(), 1, 0, 0, half.data_ptr(), 8, None, 0, 0, 0, None, 0, out.data_ptr(), 64, 8, 0), L.dh_last_error().decode())]
+    capi.check(L.dh_fill_zero(cleared.data_ptr(), 0, 256))
+    capi.check(L.dh_graph_end(0, ctypes.byref(g)))
+    assert all(rc == 1 and "captured" in message for rc, message in refused)
+    capi.check(L.dh_graph_launch(g, 0))
+    capi.check(L.dh_sync())
+    assert not cleared.any() and (out == 3).all() and (ids == 9).all()
+    capi.check(L.dh_graph_destroy(g))
 
 
 @pytest.mark.parametrize("vocab", [1, 7, 2048, 2049, 32000, 70001])

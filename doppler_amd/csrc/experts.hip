@@ -410,7 +410,11 @@ __global__ __launch_bounds__(64 * kRouterWaves<NT>) void experts_router_kernel(c
     __builtin_amdgcn_sched_barrier(0);                 // (left alone the compiler requests each when it is due)
 #pragma unroll
     for (int u = 0; u < AHEAD; u++) {
-      if (k0 + 32 * WAVES * u >= K) fa[u] = dh::bf16x8_t{};
+      if (k0 + 32 * WAVES * u >= K) {                  // (both: an infinite weight times nothing is no number)
+        fa[u] = dh::bf16x8_t{};
+#pragma unroll
+        for (int j = 0; j < NT; j++) fb[u][j] = dh::bf16x8_t{};
+      }
 #pragma unroll
       for (int j = 0; j < NT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[u], fb[u][j], acc[j], 0, 0, 0);
     }

@@ -756,6 +756,27 @@ def test_experts_that_leave_normed_rows(L, T, K, E, top, ff, shared_ff, dtype):
     assert torch.equal(x, y) and torch.equal(a, h)
 
 
+@pytest.mark.parametrize("K", [256, 1024, 2112])
+def test_an_infinite_router_weight_is_a_large_one(L, K):
+    """Its logits are infinite, of either sign, not lost: the bits of a weight whose sigmoids are 0 and 1 as well.  It stands among the last of k, whose
+    neighbours past the end are read in its place."""
+    T, E, top, ff = 40, 8, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(K)
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    h, x, norm = torch.randn(T, K, generator=g, device="cuda").to(torch.bfloat16), torch.randn(T, K, generator=g, device="cuda"), torch.ones(K, device="cuda")
+    router, up, down = w(E, K), w(E, 2 * ff, K), w(E, K, ff)
+    spec = capi.Experts(K, K, E, top, ff, 0, 1e-5, 7.0, 0.0, norm.data_ptr(), None, router.data_ptr(), up.data_ptr(), down.data_ptr(), None, None)
+    ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ctypes.byref(spec), capi.BF16, T), dtype=torch.uint8, device="cuda")
+    outs = []
+    for value in (1e30, float("inf")):
+        router[3, K - 7] = value
+        outs.append(x.clone())
+        torch.cuda.synchronize()
+        capi.check(L.dh_experts_prefill(ctypes.byref(spec), h.data_ptr(), capi.BF16, outs[-1].data_ptr(), K, ws.data_ptr(), T))
+        capi.check(L.dh_sync())
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

@@ -172,6 +172,12 @@ __global__ __launch_bounds__(256) void experts_up_kernel(const StepArgs a, int i
       if (i < nx) planes[(i & 1) * np + (i >> 1)] = scaled(xv[j], inv, wv[j]);
     }
     __syncthreads();
+    if (np < 64 * PR)                                    // past the row's end both operands are nothing: an infinite weight times nothing is no number
+#pragma unroll
+      for (int u = 0; u < PR; u++)
+#pragma unroll
+        for (int i = 0; i < kRouterRows; i++)
+          if (lane + 64 * u >= np) rw[i][u] = make_uint4(0, 0, 0, 0);
     float sum[kRouterRows] = {};
 #pragma unroll
     for (int u = 0; u < PR; u++) {

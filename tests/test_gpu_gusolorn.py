@@ -777,6 +777,27 @@ def test_an_infinite_router_weight_is_a_large_one(L, K):
     assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
 
 
+@pytest.mark.parametrize("K", [256, 960, 1024, 1536, 2048, 2112])
+def test_an_infinite_router_weight_of_a_step_is_a_large_one(L, K):
+    """The same of one row, whatever launch its logits are made in: rows that end inside a lane's pieces, on them, and longer ones."""
+    E, top, ff = 8, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(K)
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    x, norm = torch.randn(K, generator=g, device="cuda"), torch.ones(K, device="cuda")
+    router, up, down = w(E, K), w(E, 2 * ff, K), w(E, K, ff)
+    spec = capi.Experts(K, K, E, top, ff, 0, 1e-5, 7.0, 0.0, norm.data_ptr(), None, router.data_ptr(), up.data_ptr(), down.data_ptr(), None, None)
+    ws = torch.empty(L.dh_experts_step_workspace_bytes(ctypes.byref(spec)), dtype=torch.uint8, device="cuda")
+    for sign in (1, -1):
+        outs = []
+        for value in (1e30, float("inf")):
+            router[3, K - 7] = value
+            outs.append(sign * x)
+            torch.cuda.synchronize()
+            capi.check(L.dh_experts_step(ctypes.byref(spec), outs[-1].data_ptr(), ws.data_ptr()))
+            capi.check(L.dh_sync())
+        assert torch.isfinite(outs[0]).all() and torch.equal(*outs), sign
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

@@ -89,9 +89,12 @@ __device__ __forceinline__ void choose_by_places(const float* z, int E, int top,
       place += other > key || (other == key && j < lane) ? 1 : 0;
     }
   }
+  // choices behind the last logit above -infinity: the first number's expert again, for nothing (as above, where no number of 64 leaves the first as it is)
+  const unsigned long long numbers = __builtin_amdgcn_ballot_w64(lane < E && own == own);
   if (lane < E && place < top) {
-    ids[place] = lane;
-    zs[place] = own;
+    const bool lost = key == -INFINITY;
+    ids[place] = !lost ? lane : numbers ? __builtin_ctzll(numbers) : 0;
+    zs[place] = !lost || (numbers == 0 && E == 64 && place == 0) ? own : -INFINITY;
   }
 }
 __device__ __forceinline__ void choose(const float* z, int E, int top, int* ids, float* zs) {

@@ -798,6 +798,44 @@ def test_an_infinite_router_weight_of_a_step_is_a_large_one(L, K):
         assert torch.isfinite(outs[0]).all() and torch.equal(*outs), sign
 
 
+@pytest.mark.parametrize("E,top", [(8, 4), (8, 8), (20, 3), (64, 4), (64, 1), (70, 4)])
+def test_logits_that_are_not_numbers_weigh_nothing(L, E, top):
+    """Where fewer logits than are chosen are numbers, the rest of the choices add nothing: the bits of logits of -1e30, in steps and in prompts of either
+    type.  (Sums of 0 behind the numbers' experts, which come first either way.)"""
+    T, K, ff = 20, 128, 64
+    g = torch.Generator(device="cuda").manual_seed(E + top)
+    w = lambda *shape: (torch.randn(*shape, generator=g, device="cuda") / shape[-1] ** 0.5).to(torch.bfloat16)
+    rows, norm = torch.randn(T, K, generator=g, device="cuda"), torch.ones(K, device="cuda")
+    rows[:, 5] = 1.0
+    router, up, down = w(E, K), w(E, 2 * ff, K), w(E, K, ff)
+    spec = capi.Experts(K, K, E, top, ff, 0, 1e-5, 7.0, 0.0, norm.data_ptr(), None, router.data_ptr(), up.data_ptr(), down.data_ptr(), None, None)
+    ref = ctypes.byref(spec)
+    for numbers in ([], [1], [E - 1, 2], [0, 3, E // 2]):
+        if not numbers and E == 64:            # (a lane each and no number among them: the first choice weighs as its logit does)
+            continue
+        lost = torch.ones(E, dtype=torch.bool, device="cuda")
+        lost[numbers] = False
+        kept, outs = router.clone(), []
+        for value in (-1e30, float("nan")):
+            router[lost, 5] = value
+            out = [rows[0].clone()]
+            ws = torch.empty(L.dh_experts_step_workspace_bytes(ref), dtype=torch.uint8, device="cuda")
+            torch.cuda.synchronize()
+            capi.check(L.dh_experts_step(ref, out[0].data_ptr(), ws.data_ptr()))
+            capi.check(L.dh_sync())
+            for operand, t in ((capi.BF16, torch.bfloat16), (capi.F32, torch.float32)):
+                h, x = rows.to(t), rows.clone()
+                ws = torch.empty(L.dh_experts_prefill_workspace_bytes(ref, operand, T), dtype=torch.uint8, device="cuda")
+                torch.cuda.synchronize()
+                capi.check(L.dh_experts_prefill(ref, h.data_ptr(), operand, x.data_ptr(), K, ws.data_ptr(), T))
+                capi.check(L.dh_sync())
+                out.append(x)
+            outs.append(out)
+        router.copy_(kept)
+        for k, (a, b) in enumerate(zip(*outs)):
+            assert torch.isfinite(a).all() and torch.equal(a, b), (numbers, k)
+
+
 def test_equal_logits_go_to_the_lower_expert(L, tmp_path):
     x = rng(22).standard_normal((40, 64))
 

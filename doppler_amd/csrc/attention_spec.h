@@ -8,6 +8,10 @@ namespace dh {
 int attn_spec_check(const char* op, const dh_attn_spec* s);
 // The key ranges of a step whose key count is read on the device.
 DynKeys attn_spec_keys(const dh_attn_spec* s, const uint32_t* kv_len, int max_kv_len, bool wide);
+// What a product that merges a step's key splits (dense_gemv.hip) takes of them: a lane each makes a head's factors, which stand in LDS beside the row.
+constexpr int kMergedSplits = 64;
+constexpr int kMergedFactors = 16384;      // bytes
+inline bool product_merges(int heads, int splits) { return splits <= kMergedSplits && (int64_t)4 * heads * (splits + 1) <= kMergedFactors; }
 // Key elements that all heads of a token share (a rotated part beside every head's own): head keys are [D own | dim shared],
 // row r of the shared part lies ld elements behind row r - 1.  dim 0: none.
 struct SharedKey {

@@ -13,7 +13,7 @@
 // through an activation; or the argmax over all of them (output head).
 //
 // The ATTN form merges an attention's key splits (attention_spec.hip) into the front of the row: a launch less in front of the product.  A wave makes the
-// factors of a few heads' splits (up to 64: a lane each) from their maxima and weights, while the sums travel.
+// factors of a few heads' splits (a lane each) from their maxima and weights, while the sums travel.
 //
 // The HEADS form reads the raw outputs of a layer's heads instead: each head divided by its root mean square, weighted and
 // multiplied by the sigmoid of an output gate on its way into LDS.
@@ -30,7 +30,6 @@ using dh::Cand;
 
 constexpr int kMaxK = 32768;
 constexpr int kMaxHeads = 256;        // of the HEADS form
-constexpr int kAttnFactors = 16384;   // bytes of LDS for the factors of an ATTN form
 
 struct GemvArgs {
   const float* x;
@@ -305,7 +304,7 @@ int launch(const char* op, GemvArgs a, int max_grid, int* parts) {
   static bool attr_set = false;
   if (!attr_set) {
     DH_CHECK_HIP(op, hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         kMaxK * 4 + (FORM == kAttnRow ? kAttnFactors : 0)));
+                                         kMaxK * 4 + (FORM == kAttnRow ? dh::kMergedFactors : 0)));
     attr_set = true;
   }
   if (ARGMAX) max_grid = std::min(max_grid, dh::kMaxParts);
@@ -434,7 +433,7 @@ int dh_dense_gemv_attn(const dh_attn_spec* spec, const float* d_qkv, const void*
   DH_REQUIRE_INIT(op);
   if (int rc = dh::attn_spec_check(op, spec)) return rc;
   if (int rc = check(op, d_x, nullptr, 0, 0.f, d_W, ldw, N, K)) return rc;
-  if ((int64_t)spec->H * spec->VD > K || left <= 0 || left > 64 || (int64_t)4 * spec->H * (left + 1) > kAttnFactors)
+  if ((int64_t)spec->H * spec->VD > K || left <= 0 || !dh::product_merges(spec->H, left))
     return dh::fail(1, "[%s] %d splits of %d heads of %d elements in a row of %d", op, left, spec->H, spec->VD, K);
   if (!d_qkv || !d_workspace || !d_C) return dh::fail(1, "[%s] null pointer", op);
   if (reinterpret_cast<uintptr_t>(d_workspace) & 15) return dh::fail(1, "[%s] the workspace must be 16-byte aligned", op);

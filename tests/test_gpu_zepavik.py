@@ -824,6 +824,40 @@ def test_splits_left_to_the_product_behind(L, H, G, d, e, window, n, rows, ff, m
     assert torch.equal(a.kc, b.kc) and torch.equal(a.vc, b.vc) and torch.equal(a.kc, c.kc)
 
 
+@pytest.mark.parametrize("H,G,d,e,n,merged", [(2, 2, 64, 64, 8400, False), (3, 3, 64, 64, 8400, False), (4, 2, 32, 32, 9000, False), (1, 1, 64, 128, 8320, False),
+                                              (1, 1, 64, 64, 8192, True), (2, 1, 32, 32, 8150, True)])
+def test_few_heads_over_many_keys(L, H, G, d, e, n, merged):
+    """Splits of few small heads are few bytes at any number of them; the product behind merges up to 64 of a head.  The product against 64 bits over the
+    layer's outputs: 32-bit sums of n keys and of K columns, no chain of which is longer than one in 32 of the terms, each a rounding of the sizes."""
+    a = Attn(L, H, G, d, e, 0, "f32", n=n, seed=61, bias=False, gate=False)
+    rows, K = 64, (H * a.VD + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(n)
+    W, src = (torch.randn(rows, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16), a.rows()
+    kv, spec = torch.zeros(1, dtype=torch.int32, device="cuda"), ctypes.byref(a.spec)
+    capi.check(L.dh_attn_spec_kv_write(spec, src.data_ptr(), a.kc.data_ptr(), a.vc.data_ptr(), n, 0))
+    q = dev(a.q).double()
+    for p in sorted({8127, 8128, 8191, 8192, n - 1} & set(range(n))):
+        k, v = a.kc[:p + 1].double(), a.vc[:p + 1].double()
+        o = torch.zeros(H, a.VD, dtype=torch.float64, device="cuda")
+        for h in range(H):
+            o[h] = torch.softmax(k[:, h * G // H, :d] @ q[p, h] * a.scale, 0) @ v[:, h * G // H]
+        want = W[:, :H * a.VD].double() @ o.reshape(-1)
+        size = W[:, :H * a.VD].double().abs() @ v.abs().amax(0).repeat_interleave(H // G, 0).reshape(-1)
+        for on_device in (False, True):
+            left, mixed, y = ctypes.c_int(-1), torch.zeros(K, device="cuda"), torch.zeros(rows, device="cuda")
+            kv.fill_(p + 1)
+            torch.cuda.synchronize()
+            row, where = src.data_ptr() + 4 * a.ld * p, (0, kv.data_ptr(), n) if on_device else (p, None, n)
+            capi.check(L.dh_attn_spec_decode_for(spec, row, a.kc.data_ptr(), a.vc.data_ptr(), mixed.data_ptr(), *where, a.ws.data_ptr(), rows, ctypes.byref(left)))
+            assert (left.value > 0) == merged and left.value <= 64
+            if merged:
+                capi.check(L.dh_dense_gemv_attn(spec, row, a.ws.data_ptr(), left.value, where[1], n, mixed.data_ptr(), W.data_ptr(), K, rows, K, None, y.data_ptr()))
+            else:
+                capi.check(L.dh_dense_gemv(mixed.data_ptr(), None, 0, 0.0, W.data_ptr(), K, rows, K, 1.0, None, None, y.data_ptr(), rows, None, capi.ACT_NONE))
+            capi.check(L.dh_sync())
+            assert ((y.double() - want).abs() <= (n / 32 + K / 32) * 2.0 ** -24 * size).all(), (p, on_device)
+
+
 def test_prefill_output_in_bf16(L):
     a = Attn(L, 6, 2, 24, 40, 30, "f16", n=70, seed=13)
     f = a.run([70])

@@ -8,6 +8,8 @@ namespace dh {
 int attn_spec_check(const char* op, const dh_attn_spec* s);
 // The key ranges of a step whose key count is read on the device.
 DynKeys attn_spec_keys(const dh_attn_spec* s, const uint32_t* kv_len, int max_kv_len, bool wide);
+// Splits of a wide launch for a step that can see `keys` keys at most.
+int attn_spec_wide_splits(const dh_attn_spec* s, int keys);
 // What a product that merges a step's key splits (dense_gemv.hip) takes of them: a lane each makes a head's factors, which stand in LDS beside the row.
 constexpr int kMergedSplits = 64;
 constexpr int kMergedFactors = 16384;      // bytes

@@ -440,7 +440,7 @@ int launch_spec(const char* op, const dh_attn_spec* s, const SpecArgs& args, int
 // Few small heads have few bytes at any number of splits, but no more of them than the product takes (product_merges).
 constexpr int kMergedBytes = 64 << 10;
 bool left_to_product(const dh_attn_spec* s, int most_keys, int rows, const void* ws) {
-  const int splits = dh::wide_splits(dh::attn_one_per_cu(dh::num_cus(), s->Hkv), most_keys);
+  const int splits = dh::attn_spec_wide_splits(s, most_keys);
   return rows > 0 && most_keys > dh::kAttnTileKeys && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 && wide_kernel(s) && dh::product_merges(s->H, splits) &&
          (int64_t)4 * s->H * splits * s->VD * std::max<int64_t>(1, dh::ceil_div(rows, 8 * dh::num_cus())) <= kMergedBytes;
 }
@@ -462,7 +462,7 @@ int decode(const char* op, const dh_attn_spec* spec, const float* d_qkv, void* d
   const int one_per_cu = dh::attn_one_per_cu(dh::num_cus(), spec->Hkv);
   if (d_kv_len) {
     a.dyn = dh::attn_spec_keys(spec, d_kv_len, max_kv_len, wide);
-    a.nsplit = wide ? dh::wide_splits(one_per_cu, most_keys) : dh::max_splits_upto(one_per_cu, most_keys);
+    a.nsplit = wide ? dh::attn_spec_wide_splits(spec, most_keys) : dh::max_splits_upto(one_per_cu, most_keys);
   } else {
     a.kend = pos + 1;
     a.kbeg = spec->window > 0 ? std::max(0, pos - spec->window + 1) : 0;
@@ -490,6 +490,10 @@ DynKeys attn_spec_keys(const dh_attn_spec* s, const uint32_t* kv_len, int max_kv
   d.kv_len_ptr = kv_len; d.max_kv_len = max_kv_len; d.causal = 1; d.start_pos = -1;
   d.sliding_window = s->window; d.kv_start = 0; d.qkv = 1; d.one_per_cu = attn_one_per_cu(num_cus(), s->Hkv); d.wide = wide;
   return d;
+}
+
+int attn_spec_wide_splits(const dh_attn_spec* s, int keys) {
+  return wide_splits(attn_one_per_cu(num_cus(), s->Hkv), s->window > 0 ? std::min(keys, s->window) : keys);
 }
 
 int attn_spec_check(const char* op, const dh_attn_spec* s) {

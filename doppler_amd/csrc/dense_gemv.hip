@@ -438,6 +438,9 @@ int dh_dense_gemv_attn(const dh_attn_spec* spec, const float* d_qkv, const void*
   if (!d_qkv || !d_workspace || !d_C) return dh::fail(1, "[%s] null pointer", op);
   if (reinterpret_cast<uintptr_t>(d_workspace) & 15) return dh::fail(1, "[%s] the workspace must be 16-byte aligned", op);
   if (d_kv_len && max_kv_len <= 0) return dh::fail(1, "[%s] max_kv_len must be positive with the key count on the device", op);
+  // (the device's count decides how many are read, up to this many)
+  if (d_kv_len && left != dh::attn_spec_wide_splits(spec, max_kv_len))
+    return dh::fail(1, "[%s] %d splits are not those of up to %d keys", op, left, max_kv_len);
   if (d_x == d_C) return dh::fail(1, "[%s] the output must not be the activation row", op);
   GemvArgs a = make_args(d_x, nullptr, 0, 0.f, d_W, ldw, N, K, 1.f);
   a.residual = d_residual; a.C = d_C;

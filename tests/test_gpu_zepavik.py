@@ -858,6 +858,22 @@ def test_few_heads_over_many_keys(L, H, G, d, e, n, merged):
             assert ((y.double() - want).abs() <= (n / 32 + K / 32) * 2.0 ** -24 * size).all(), (p, on_device)
 
 
+def test_splits_of_another_count_are_refused(L):
+    """The device's key count says how many splits a product reads: they have to be those of the most keys it can be."""
+    a = Attn(L, 4, 2, 64, 48, 0, n=700, seed=9)
+    src, W, x, y, left = a.rows(), torch.zeros(64, 192, dtype=torch.bfloat16, device="cuda"), torch.zeros(192, device="cuda"), torch.zeros(64, device="cuda"), ctypes.c_int()
+    count = torch.full((1,), 700, dtype=torch.int32, device="cuda")
+    capi.check(L.dh_attn_spec_kv_write(ctypes.byref(a.spec), src.data_ptr(), a.kc.data_ptr(), a.vc.data_ptr(), 700, 0))
+    torch.cuda.synchronize()
+    capi.check(L.dh_attn_spec_decode_for(ctypes.byref(a.spec), src.data_ptr() + 4 * a.ld * 699, a.kc.data_ptr(), a.vc.data_ptr(), x.data_ptr(), 0, count.data_ptr(), 700,
+                                         a.ws.data_ptr(), 64, ctypes.byref(left)))
+    merge = lambda splits, most: L.dh_dense_gemv_attn(ctypes.byref(a.spec), src.data_ptr() + 4 * a.ld * 699, a.ws.data_ptr(), splits, count.data_ptr(), most, x.data_ptr(),
+                                                    W.data_ptr(), 192, 64, 192, None, y.data_ptr())
+    for splits, most in ((left.value - 1, 700), (left.value + 1, 700), (left.value, 1100), (0, 700)):
+        assert merge(splits, most) != 0 and "splits" in L.dh_last_error().decode()
+    assert merge(left.value, 700) == 0 and L.dh_sync() == 0
+
+
 def test_prefill_output_in_bf16(L):
     a = Attn(L, 6, 2, 24, 40, 30, "f16", n=70, seed=13)
     f = a.run([70])

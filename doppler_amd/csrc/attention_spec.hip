@@ -27,6 +27,11 @@ using dh::KeyRange;
 
 constexpr float kLog2e = 1.4426950408889634f;
 
+// A split's maximum and weight.  A workspace may begin on any float.
+struct __attribute__((packed, aligned(4))) SplitPair {
+  float most, weight;
+};
+
 struct SpecArgs {
   const float* qkv;     // projection rows [T][ld_qkv]
   void* K;
@@ -299,7 +304,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_spec_kernel(const SpecArgs a)
     } else {
       const int64_t part = (int64_t)h * ws_stride + split;
       a.ws[part * a.VD + d] = num;
-      if (d == 0) reinterpret_cast<float2*>(a.ws + (int64_t)a.H * ws_stride * a.VD)[part] = make_float2(M, den);
+      if (d == 0) reinterpret_cast<SplitPair*>(a.ws + (int64_t)a.H * ws_stride * a.VD)[part] = SplitPair{M, den};
     }
   }
 }
@@ -312,10 +317,10 @@ __global__ __launch_bounds__(256) void attn_spec_merge_kernel(const float* __res
   __shared__ float red[4];
   const int h = blockIdx.x, tid = threadIdx.x, wave = tid >> 6;
   const float* base = ws + (int64_t)h * nsplit * VD;
-  const float2* pairs = reinterpret_cast<const float2*>(ws + (int64_t)H * nsplit * VD) + (int64_t)h * nsplit;
+  const SplitPair* pairs = reinterpret_cast<const SplitPair*>(ws + (int64_t)H * nsplit * VD) + (int64_t)h * nsplit;
   if (dyn.kv_len_ptr != nullptr) nsplit = dh::dyn_key_range(dyn).nsplit;
   float M = -FLT_MAX;
-  for (int s = tid; s < nsplit; s += 256) M = fmaxf(M, pairs[s].x);
+  for (int s = tid; s < nsplit; s += 256) M = fmaxf(M, pairs[s].most);
   M = dh::group_combine<1, 64>(M, dh::MaxOp());
   if ((tid & 63) == 0) red[wave] = M;
   __syncthreads();
@@ -323,10 +328,10 @@ __global__ __launch_bounds__(256) void attn_spec_merge_kernel(const float* __res
   __syncthreads();
   float den = 0.f;
   for (int s = tid; s < nsplit; s += 256) {
-    const float2 part = pairs[s];
-    const float f = __builtin_amdgcn_exp2f(part.x - M);
+    const SplitPair part = pairs[s];
+    const float f = __builtin_amdgcn_exp2f(part.most - M);
     f_s[s] = f;
-    den = fmaf(f, part.y, den);
+    den = fmaf(f, part.weight, den);
   }
   den = dh::wave_sum_uniform(den);
   if ((tid & 63) == 0) red[wave] = den;

@@ -481,7 +481,7 @@ int dh_attn_spec_prefill(const dh_attn_spec* spec, const float* d_qkv, const voi
 /* One step from its raw projection row: key and value are appended at row `pos`, the token attends to its window;
  * d_out is [H * VD] f32.  d_kv_len (may be NULL): the key count pos + 1 is read from device memory instead, at most
  * max_kv_len (a captured step then replays at every position).  d_workspace: dh_attn_spec_workspace_bytes(H, VD,
- * max_kv_len or pos + 1). */
+ * max_kv_len or pos + 1), on a multiple of 4 bytes (dh_attn_spec_decode_for leaves splits only in one on a multiple of 16). */
 size_t dh_attn_spec_workspace_bytes(int H, int VD, int max_kv_len);
 int dh_attn_spec_decode(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
                         int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace);

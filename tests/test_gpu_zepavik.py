@@ -874,6 +874,28 @@ def test_splits_of_another_count_are_refused(L):
     assert merge(left.value, 700) == 0 and L.dh_sync() == 0
 
 
+def test_a_workspace_on_any_float(L):
+    """Splits in a workspace that begins on a multiple of four bytes: the bits of one on a multiple of sixteen, and with a product behind a launch merges them."""
+    outs = []
+    for off in (0, 4, 8, 12):
+        a = Attn(L, 4, 2, 64, 48, 0, n=700, seed=9)
+        src, ws = a.rows(), torch.zeros(a.ws.numel() + 16, dtype=torch.uint8, device="cuda")
+        capi.check(L.dh_attn_spec_kv_write(ctypes.byref(a.spec), src.data_ptr(), a.kc.data_ptr(), a.vc.data_ptr(), 700, 0))
+        for p in (130, 699):
+            step, left = (ctypes.byref(a.spec), src.data_ptr() + 4 * a.ld * p, a.kc.data_ptr(), a.vc.data_ptr()), ctypes.c_int(-1)
+            for rows in (0, 64):
+                out = torch.zeros(4 * 48, device="cuda")
+                torch.cuda.synchronize()
+                if rows and off:
+                    capi.check(L.dh_attn_spec_decode_for(*step, out.data_ptr(), p, None, 700, ws.data_ptr() + off, rows, ctypes.byref(left)))
+                    assert left.value == 0
+                else:
+                    capi.check(L.dh_attn_spec_decode(*step, out.data_ptr(), p, None, 700, ws.data_ptr() + off))
+                capi.check(L.dh_sync())
+                outs.append((p, out))
+    assert all(torch.equal(o, next(x for q, x in outs if q == p)) for p, o in outs)
+
+
 def test_prefill_output_in_bf16(L):
     a = Attn(L, 6, 2, 24, 40, 30, "f16", n=70, seed=13)
     f = a.run([70])

@@ -148,9 +148,9 @@ __global__ __launch_bounds__(64 * WAVES) void attn_spec_kernel(const SpecArgs a)
   const bool has_k = 8 * piece < a.D, has_v = 8 * piece < a.VD;
   const int nchunks = (kend - kbeg + CH - 1) / CH;
 
-  // (addresses: a 64-bit base a lane, once, and a 32-bit row times a 32-bit stride)
+  // (addresses: a 64-bit base a lane, once, and a 32-bit row times a 32-bit stride in pieces of sixteen bytes, of which rows of any cache are made)
   const char *kfrom = reinterpret_cast<const char*>(Kc + (int64_t)kbeg * kstride), *vfrom = reinterpret_cast<const char*>(Vc + (int64_t)kbeg * vstride);
-  const uint32_t kbytes = (uint32_t)(kstride * sizeof(KV)), vbytes = (uint32_t)(vstride * sizeof(KV));
+  const uint32_t kpieces = (uint32_t)(kstride * sizeof(KV) / 16), vpieces = (uint32_t)(vstride * sizeof(KV) / 16);
   const int last = kend - 1 - a.append - kbeg;         // of the rows in the cache: the appended one is not there yet
   Piece<KV> kn[NP], vn[NP], knew, vnew;
 #pragma unroll
@@ -165,10 +165,10 @@ __global__ __launch_bounds__(64 * WAVES) void attn_spec_kernel(const SpecArgs a)
     for (int n = 0; n < NP; n++) r[n] = (uint32_t)min(c * CH + wave * WK + n * SLOTS + slot, last);      // keys past the end repeat the last one
     if (has_k)
 #pragma unroll
-      for (int n = 0; n < NP; n++) kn[n].load(reinterpret_cast<const KV*>(kfrom + (uint64_t)r[n] * kbytes));
+      for (int n = 0; n < NP; n++) kn[n].load(reinterpret_cast<const KV*>(kfrom + 16 * ((uint64_t)r[n] * kpieces)));
     if (has_v)
 #pragma unroll
-      for (int n = 0; n < NP; n++) vn[n].load(reinterpret_cast<const KV*>(vfrom + (uint64_t)r[n] * vbytes));
+      for (int n = 0; n < NP; n++) vn[n].load(reinterpret_cast<const KV*>(vfrom + 16 * ((uint64_t)r[n] * vpieces)));
   };
   if (split < nchunks) load(split);
 

@@ -896,6 +896,25 @@ def test_a_workspace_on_any_float(L):
     assert all(torch.equal(o, next(x for q, x in outs if q == p)) for p, o in outs)
 
 
+def test_shared_key_rows_four_gigabytes_apart(L):
+    """Row strides whose bytes no longer fit 32 bits: the bits of rows beside one another."""
+    H, D, S, VD, T, far = 2, 8, 8, 8, 2, 1 << 30
+    g = torch.Generator(device="cuda").manual_seed(5)
+    ld = H * (D + S) + 16
+    qkv, kc, vc, ks = (torch.randn(T, n, generator=g, device="cuda") for n in (ld, D, VD, S))
+    spec = capi.AttnSpec(H, 1, D, VD, VD, 0, capi.F32, 0, H * (D + S), H * (D + S) + 8, -1, ld, D ** -0.5, 1e-5, None, None)
+    apart, outs = torch.empty(far + S, device="cuda"), []
+    apart[:S], apart[far:] = ks[0], ks[1]
+    for rows, stride in ((ks, S), (apart, far)):
+        o = torch.zeros(T, H * VD, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_attn_spec_prefill_shared(ctypes.byref(spec), qkv.data_ptr(), kc.data_ptr(), rows.data_ptr(), S, stride, vc.data_ptr(), o.data_ptr(),
+                                                 capi.F32, H * VD, T, 0))
+        capi.check(L.dh_sync())
+        outs.append(o)
+    assert outs[0].abs().sum() > 0 and torch.equal(*outs)
+
+
 def test_prefill_output_in_bf16(L):
     a = Attn(L, 6, 2, 24, 40, 30, "f16", n=70, seed=13)
     f = a.run([70])

@@ -843,7 +843,8 @@ int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int 
     return dh::fail(1, "[%s] numTokens/hiddenSize/vocabSize must be positive", op);
   if (!d_ids || !d_table || !d_out) return dh::fail(1, "[%s] null pointer", op);
   const int64_t total = (int64_t)T * hidden;
-  if ((hidden & 3) == 0 && hidden < (1 << 24) && (reinterpret_cast<uintptr_t>(d_table) & 7) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0)
+  // (a workgroup a row: a launch has less than 2^32 threads along a dimension)
+  if ((hidden & 3) == 0 && hidden < (1 << 24) && T < (1 << 24) && (reinterpret_cast<uintptr_t>(d_table) & 7) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0)
     hipLaunchKernelGGL(gather_f16_pieces_kernel, dim3((unsigned)T, (unsigned)dh::ceil_div(hidden, 1024)), dim3(256), 0, dh::stream(), d_ids,
                        static_cast<const __half*>(d_table), d_out, hidden, (uint32_t)vocab, index_offset);
   else

@@ -65,6 +65,19 @@ def test_words_and_embedding_in_one_launch(hidden, buckets, pos):
         assert torch.equal(outs[2], outs[3]) and torch.equal(ids, got)
 
 
+def test_more_rows_than_a_grid_has_workgroups_of():
+    """Rows of four elements: at 2^24 of them a workgroup each is more threads than a launch can have."""
+    L = capi.init(torch.cuda.current_device())
+    T, table = 1 << 24, torch.arange(32, device="cuda").to(torch.float16).reshape(8, 4)
+    ids = (torch.arange(T, device="cuda") % 11).to(torch.int32)
+    out = torch.zeros(T, 4, device="cuda")
+    torch.cuda.synchronize()
+    capi.check(L.dh_gather_f16(ids.data_ptr(), table.data_ptr(), out.data_ptr(), T, 4, 8, 0))
+    capi.check(L.dh_sync())
+    want = torch.cat([table.float(), torch.zeros(3, 4, device="cuda")])[ids.long()]
+    assert torch.equal(out, want)
+
+
 def test_words_of_a_token_are_refused_while_a_graph_is_captured():
     """A replay would set the same words: the refusal of dh_set_words, in front of anything that would go into the graph."""
     L = capi.init(torch.cuda.current_device())

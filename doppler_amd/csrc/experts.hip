@@ -11,8 +11,8 @@
 //
 // Decode: experts_up_kernel chooses the experts itself (every workgroup, from the few logits), norms the row and streams the
 // chosen gate and up rows; experts_down_kernel streams the chosen down matrices and the shared one side by side along k.
-// Prefill: experts_router_kernel (logits and choices) and experts_place_kernel (rows sorted by expert, table of row tiles), or for f32 operands, more than
-// 64 logits and long portions a product, experts_route_kernel and experts_sort_kernel; grouped products on the matrix cores (dense_gemm.hip);
+// Prefill: experts_router_kernel (logits and choices) and experts_place_kernel (rows sorted by expert, table of row tiles), or for f32 operands, many
+// logits, long rows and long portions (routes_itself) a product, experts_route_kernel and experts_sort_kernel; grouped products on the matrix cores (dense_gemm.hip);
 // experts_combine_kernel.
 #include <algorithm>
 #include <cfloat>
@@ -386,14 +386,12 @@ __device__ __forceinline__ void route_token(const float* z, int t, int E, int to
 // the waves' sums meet in LDS in wave order.  What the places need goes out with the choices: slot, a choice's rank among the group's of its expert (in any
 // order), and counts [groups][E].  us, 1531 rows of 2048, 16 experts and a shared one: 8.1, against 6.1 + 5.3 + 4.8 for a product
 // with k in slices, the slices' sum and the choices; 40 rows of 1024 8 against 6.6 + 3.3.
-constexpr int kRouterLogits = 64;
+constexpr int kRouterLogits = 32, kRouterWaves = 16;
 template <int NT>
-constexpr int kRouterWaves = NT <= 2 ? 16 : 8;         // (the sums of sixteen would not fit the LDS)
-template <int NT>
-__global__ __launch_bounds__(64 * kRouterWaves<NT>) void experts_router_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ router, int K, int T, int E, int top,
+__global__ __launch_bounds__(64 * kRouterWaves) void experts_router_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ router, int K, int T, int E, int top,
                                                              int shared, int* __restrict__ ids, float* __restrict__ weights, float* __restrict__ sg,
                                                              int* __restrict__ slot, int* __restrict__ counts) {
-  constexpr int WAVES = kRouterWaves<NT>, AHEAD = 64 / WAVES, ROW = 16 * NT + 4;
+  constexpr int WAVES = kRouterWaves, AHEAD = 64 / WAVES, ROW = 16 * NT + 4;
   __shared__ __align__(16) float sums[WAVES][16][ROW];
   __shared__ int id_s[WAVES][kMaxTop];
   __shared__ float z_s[WAVES][kMaxTop];
@@ -443,13 +441,9 @@ __global__ __launch_bounds__(64 * kRouterWaves<NT>) void experts_router_kernel(c
   }
   if (tid < kRouterLogits) count[tid] = 0;
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 16 / WAVES; i++) {
-    const int t = (16 / WAVES) * wave + i;
-    if (t0 + t >= T) continue;
-    route_token(sums[0][t], t0 + t, E, top, shared, id_s[wave], z_s[wave], ids, weights, sg);
-    if (lane < top) slot[(int64_t)(t0 + t) * top + lane] = atomicAdd(&count[id_s[wave][lane]], 1);
-    __builtin_amdgcn_wave_barrier();
+  if (t0 + wave < T) {
+    route_token(sums[0][wave], t0 + wave, E, top, shared, id_s[wave], z_s[wave], ids, weights, sg);
+    if (lane < top) slot[(int64_t)(t0 + wave) * top + lane] = atomicAdd(&count[id_s[wave][lane]], 1);
   }
   __syncthreads();
   if (tid < E) counts[(int64_t)blockIdx.x * E + tid] = count[tid];
@@ -476,7 +470,7 @@ __global__ __launch_bounds__(256) void experts_place_kernel(const int* __restric
   __shared__ int part[2][256];                         // sums of a thread's groups: all of them, and those in front
   __shared__ int at[GROUPS][kRouterLogits];            // where a group's rows of an expert begin
   const int tid = threadIdx.x, g0 = GROUPS * blockIdx.x, i0 = CHOICES * top * blockIdx.x, mine = min(CHOICES * top, n - i0);
-  const int shift = E <= 16 ? 4 : E <= 32 ? 5 : 6, parts = 256 >> shift, e = tid & ((1 << shift) - 1);
+  const int shift = E <= 16 ? 4 : 5, parts = 256 >> shift, e = tid & ((1 << shift) - 1);
   int id[BATCH], rank[BATCH];
   float w[BATCH];
   auto read = [&](int j) {
@@ -520,8 +514,9 @@ __global__ __launch_bounds__(256) void experts_place_kernel(const int* __restric
     int next = first + front;
 #pragma unroll
     for (int g = 0; g < GROUPS; g++) {
+      if (tid >= E) break;
       at[g][tid] = next;
-      if (tid < E && g0 + g < groups) next += counts[(g0 + g) * E + tid];
+      if (g0 + g < groups) next += counts[(g0 + g) * E + tid];
     }
     if (blockIdx.x == 0) {
       if (tid < E) off[tid] = first;
@@ -546,6 +541,14 @@ __global__ __launch_bounds__(256) void experts_place_kernel(const int* __restric
       row_weight[to] = w[k];
     }
   }
+}
+
+// Where the two kernels above stand in for a product, its slices' sum, the choices and the sort.  Every workgroup reads the whole router, and with more
+// logits twice the accumulators' rows, where a product spreads a long k over the device; what the sort saves grows with the tokens.  Whole portions of 64
+// wide experts in us, product and sort / these: 16 logits, 200 tokens, k 2048 36.7 / 33.6, 4096 56.5 / 55.8, 5120 64.2 / 66.5; 32 logits k 2048 42.8 / 41.7,
+// 3072 51.1 / 55.1, 4096 58.9 / 63.0, with 4096 tokens 222.5 / 220.0 (17: 212.0 / 201.8); 64 logits, 200 tokens, k 256 22.7 / 31.7, 2048 43.5 / 48.9.
+bool routes_itself(int logits, int K, int T) {
+  return logits <= kRouterLogits && T <= 16 * kPlacedGroups && (K <= 2048 || (K <= 4096 && (logits <= 16 || T > 1024)));
 }
 
 // One workgroup: rows sorted by expert.  slot[i]: sorted place of choice i = token * top + k; row_token, row_weight by place.
@@ -848,11 +851,10 @@ int prefill(const char* op, const dh_experts* spec, const void* d_h, int operand
   auto i32 = [&](size_t at) { return reinterpret_cast<int*>(w + at); };
   const int n = T * spec->top;
   const int shared_logit = spec->shared_ff > 0 ? 1 : 0, groups = (int)dh::ceil_div(T, 16);
-  if (operand == DH_BF16 && logits(spec) <= kRouterLogits && groups <= kPlacedGroups) {
-    const int tiles = (int)dh::ceil_div(logits(spec), 16);
-    auto kern = tiles == 1 ? experts_router_kernel<1> : tiles == 2 ? experts_router_kernel<2> : experts_router_kernel<4>;
+  if (operand == DH_BF16 && routes_itself(logits(spec), spec->K, T)) {
+    auto kern = logits(spec) <= 16 ? experts_router_kernel<1> : experts_router_kernel<2>;
     int* counts = i32(p.z);                            // (no logits go to memory)
-    hipLaunchKernelGGL(kern, dim3(groups), dim3(64 * (tiles <= 2 ? kRouterWaves<2> : kRouterWaves<4>)), 0, dh::stream(), static_cast<const uint16_t*>(d_h),
+    hipLaunchKernelGGL(kern, dim3(groups), dim3(64 * kRouterWaves), 0, dh::stream(), static_cast<const uint16_t*>(d_h),
                        static_cast<const uint16_t*>(spec->d_router), spec->K, T, spec->experts, spec->top, shared_logit, i32(p.ids), f32(p.weights), f32(p.sg),
                        i32(p.slot), counts);
     DH_CHECK_LAUNCH(op);

@@ -713,6 +713,14 @@ def test_choices_of_portions_and_steps(L, T, K, E, top, ff, shared_ff):
     assert torch.equal(x[n:], x0[n:])
 
 
+@pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(40, 2048, 31, 2, 64, 64), (40, 2048, 33, 2, 64, 0), (40, 2112, 16, 2, 64, 0), (40, 2112, 16, 2, 64, 64), (1024, 2112, 32, 3, 64, 0),
+                                                    (1025, 2112, 31, 3, 64, 64), (20, 4096, 15, 2, 64, 64), (1025, 4096, 32, 2, 64, 0), (1025, 4160, 16, 2, 64, 0)])
+def test_choices_on_either_side_of_a_product(L, T, K, E, top, ff, shared_ff):
+    """Portions whose logits are made with the choices, and their neighbours whose logits are a product's: 32 logits, 2048 and 4096 of k, 16 logits and 1024
+    tokens between."""
+    test_choices_of_portions_and_steps(L, T, K, E, top, ff, shared_ff)
+
+
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F32])
 @pytest.mark.parametrize("M,N,K,sliced", [(40, 1024, 3072, True), (1, 260, 4096, True), (33, 8192, 4096, None), (17, 8196, 4096, None), (5, 102, 4096, True), (700, 1024, 256, False)])
 def test_products_that_leave_normed_rows(L, M, N, K, sliced, dtype):

@@ -76,8 +76,10 @@ __device__ __forceinline__ void choose_upto(const float* z, int E, int top, int*
   }
 }
 // The same for up to 64 experts, a lane each: a lane's place is the number of experts in front of it.  The largest one after the other are `top` chains of
-// lane steps (0.3 us each), this a pass over the experts whose steps do not wait for one another (0.15 us for 16): experts_up and _down at hidden 1024,
-// four of 16 experts, 6.6 against 6.9 and 4.8 against 5.0 us.
+// lane steps (0.3 us each), this a pass over the experts whose steps do not wait for one another: experts_up and _down at hidden 1024, four of 16 experts,
+// 6.6 against 6.9 and 4.8 against 5.0 us.  It costs by the experts and the other by the choices: a portion of eight tokens, us, the largest one after the other /
+// this, 8 of 8 experts 25.6 / 24.7, 3 of 16 23.3 / 23.3, 2 of 16 23.2 / 23.3, 6 of 32 24.7 / 24.7, 2 of 32 23.2 / 23.8, 8 of 48 25.6 / 25.7, 8 of 64 25.4 / 25.8,
+// 2 of 64 22.7 / 24.0.
 __device__ __forceinline__ void choose_by_places(const float* z, int E, int top, int* ids, float* zs) {
   const int lane = threadIdx.x & 63;
   const float own = z[min(lane, E - 1)], key = lane < E && own == own ? own : -INFINITY;
@@ -98,7 +100,7 @@ __device__ __forceinline__ void choose_by_places(const float* z, int E, int top,
   }
 }
 __device__ __forceinline__ void choose(const float* z, int E, int top, int* ids, float* zs) {
-  if (E <= 64 && E <= 32 * top) choose_by_places(z, E, top, ids, zs);
+  if (E <= 64 && E <= 5 * top) choose_by_places(z, E, top, ids, zs);
   else if (E <= 64) choose_upto<1>(z, E, top, ids, zs);
   else if (E <= 256) choose_upto<4>(z, E, top, ids, zs);
   else choose_upto<kMaxExperts / 64>(z, E, top, ids, zs);

@@ -806,7 +806,7 @@ def test_an_infinite_router_weight_of_a_step_is_a_large_one(L, K):
         assert torch.isfinite(outs[0]).all() and torch.equal(*outs), sign
 
 
-@pytest.mark.parametrize("E,top", [(8, 4), (8, 8), (20, 3), (64, 4), (64, 1), (70, 4)])
+@pytest.mark.parametrize("E,top", [(8, 4), (8, 8), (15, 3), (16, 3), (20, 3), (64, 13), (64, 4), (64, 1), (70, 4)])
 def test_logits_that_are_not_numbers_weigh_nothing(L, E, top):
     """Where fewer logits than are chosen are numbers, the rest of the choices add nothing: the bits of logits of -1e30, in steps and in prompts of either
     type.  (Sums of 0 behind the numbers' experts, which come first either way.)"""

@@ -676,6 +676,15 @@ __global__ __launch_bounds__(256) void experts_combine_norm_kernel(const float* 
   dh::store_normed_row<BF16>(out, hidden, norm, eps, red, normed, (int64_t)t * ld_normed, ld_normed);
 }
 
+// Where a step's first kernel makes the logits too (20 are what its waves hold).  Four pieces of a row leave three workgroups to a compute unit's registers, and
+// a fourth would wait for one of them to end; and what a launch saves is more than twenty rows' reading only where there are few workgroups or the rows are long.
+// us, logits in a launch / in the kernel, four of the experts: 20 logits, 768 workgroups, k 256 12.3 / 12.1, 1536 15.8 / 15.1, 2048 17.0 / 15.8; 1024 workgroups,
+// k 256 12.8 / 13.2, 512 13.2 / 13.3, 1024 14.3 / 13.5, 1536 16.8 / 20.0, 2048 18.2 / 20.7; 17 logits, 784 workgroups, k 1024 13.9 / 12.2, 2048 17.4 / 18.3;
+// 16 logits, 1024 workgroups, k 256 12.8 / 12.7; 9 logits, 528 workgroups, k 1024 13.2 / 10.5, 2048 16.3 / 13.3.
+bool router_beside(int logits, int K, int workgroups) {
+  return logits <= 4 * kRouterRows && K <= 2048 && (workgroups <= 3 * dh::num_cus() || (K <= 1024 && (logits <= 16 || K >= 512)));
+}
+
 size_t up256(size_t n) { return (n + 255) / 256 * 256; }
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -784,7 +793,7 @@ int dh_experts_step(const dh_experts* spec, float* d_x, void* d_workspace) {
   };
   int iters = 1;
   dim3 grid = plan(dh::ceil_div(total, 4), spec->K, &iters);
-  const bool with_router = logits(spec) <= 4 * kRouterRows && spec->K <= 2048;
+  const bool with_router = router_beside(logits(spec), spec->K, (int)grid.x);
   if (!with_router)
     if (int rc = dh_dense_gemv(d_x, spec->d_norm, spec->hidden, spec->eps, spec->d_router, spec->K, logits(spec), spec->K, 1.f, nullptr, nullptr, z,
                                logits(spec), nullptr, DH_ACT_NONE))

@@ -713,6 +713,14 @@ def test_choices_of_portions_and_steps(L, T, K, E, top, ff, shared_ff):
     assert torch.equal(x[n:], x0[n:])
 
 
+@pytest.mark.parametrize("K,E,top,ff,shared_ff", [(448, 20, 4, 1024, 0), (448, 16, 4, 1024, 0), (512, 19, 4, 960, 192), (1024, 17, 2, 2048, 0), (1088, 8, 3, 1024, 0),
+                                                  (1088, 8, 3, 1024, 64), (2048, 20, 1, 3072, 0)])
+def test_step_logits_beside_many_products(L, K, E, top, ff, shared_ff):
+    """Steps whose logits are made with the first products, and their neighbours with a launch for them: 768 and 1024 workgroups, rows around 512 and 1024, 16 to
+    20 logits."""
+    test_choices_of_portions_and_steps(L, 5, K, E, top, ff, shared_ff)
+
+
 @pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(40, 2048, 31, 2, 64, 64), (40, 2048, 33, 2, 64, 0), (40, 2112, 16, 2, 64, 0), (40, 2112, 16, 2, 64, 64), (1024, 2112, 32, 3, 64, 0),
                                                     (1025, 2112, 31, 3, 64, 64), (20, 4096, 15, 2, 64, 64), (1025, 4096, 32, 2, 64, 0), (1025, 4160, 16, 2, 64, 0)])
 def test_choices_on_either_side_of_a_product(L, T, K, E, top, ff, shared_ff):

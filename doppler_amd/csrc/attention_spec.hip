@@ -442,11 +442,14 @@ int launch_spec(const char* op, const dh_attn_spec* s, const SpecArgs& args, int
 // eight waves takes 128 keys.  By the most keys a step can have, so that enqueued and captured steps split alike.
 // us, attention + merge + product / attention of wide workgroups + product: 16 heads of 128, 1024 keys, 2048 x 8192 7.7 + 3.9 + 9.3 / 6.6 + 10.8; 16 of 64 in
 // f32, 1024 x 4096 6.7 + 3.7 + 5.2 / 6.0 + 6.7.  With 16 splits of 64 keys (128 KB) the product takes 23, with four of 256 10.2 and the attention 10.5.
-// Few small heads have few bytes at any number of splits, but no more of them than the product takes (product_merges).
+// Few small heads have few bytes at any number of splits, but no more of them than the product takes (product_merges).  And a wave of the product makes four
+// heads' factors at once (HB there): more than its four or eight waves have would be another trip to memory, 32 heads of 64 in front of 2048 x 2048 (eight waves)
+// 11.4 / 10.1, of 2000 x 2048 (four) 10.0 / 12.3, 64 of 64 of 2000 x 4096 14.7 / 20.3.
+// The call does not know the product's columns: where more than 4096 rows have few of them its callers keep to dh_attn_spec_decode (dense_decoder.py).
 constexpr int kMergedBytes = 64 << 10;
 bool left_to_product(const dh_attn_spec* s, int most_keys, int rows, const void* ws) {
   const int splits = dh::attn_spec_wide_splits(s, most_keys);
-  return rows > 0 && most_keys > dh::kAttnTileKeys && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 && wide_kernel(s) && dh::product_merges(s->H, splits) &&
+  return rows > 0 && s->H <= (rows >= 8 * dh::num_cus() ? 32 : 16) && most_keys > dh::kAttnTileKeys && (reinterpret_cast<uintptr_t>(ws) & 15) == 0 && wide_kernel(s) && dh::product_merges(s->H, splits) &&
          (int64_t)4 * s->H * splits * s->VD * std::max<int64_t>(1, dh::ceil_div(rows, 8 * dh::num_cus())) <= kMergedBytes;
 }
 

@@ -224,11 +224,12 @@ class DenseDecoder(DecoderBase):
                                g["n"], g["kx"], 1.0, d["bias"].data_ptr(), None, self.qkv.data_ptr(), g["n_first"], act, d["act"]))
         else:
             self._enqueue_in(d, self.x.data_ptr(), self._wide_row().data_ptr(), capi.F32, self.qkv.data_ptr(), act, 1, g["k2"])
-        # the product behind merges the key splits itself where that is faster than a launch
+        # the product behind merges the key splits itself where that is faster than a launch (rows of few columns: every workgroup of many merges for little
+        # work of its own; us, a launch / the product: 8192 x 512 10.9 / 12.9, x 1536 14.2 / 15.7, x 4288 21.5 / 19.4)
         spec, one_row, left = ctypes.byref(d["spec"]), g["k2"] <= GEMV_MAX_K, ctypes.c_int(0)
         step = (spec, self.qkv.data_ptr(), d["cache_k"].data_ptr(), d["cache_v"].data_ptr(), mixed.data_ptr(), pos, kv_len, self.max_seq,
                 self.attn_ws.data_ptr())
-        if one_row:
+        if one_row and (c["hidden"] <= 4096 or g["k2"] >= 3072):
             ck(L.dh_attn_spec_decode_for(*step, c["hidden"], ctypes.byref(left)))
         else:
             ck(L.dh_attn_spec_decode(*step))

@@ -486,7 +486,8 @@ size_t dh_attn_spec_workspace_bytes(int H, int VD, int max_kv_len);
 int dh_attn_spec_decode(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
                         int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace);
 /* The same in front of a product of `rows` rows whose activation row d_out begins: *left is 0 and d_out written, or, where that is faster, the number of
- * key splits left in the workspace, which dh_dense_gemv_attn merges while it reads its row. */
+ * key splits left in the workspace, which dh_dense_gemv_attn merges while it reads its row (more than 4096 rows: of at least 3072 columns, which the call
+ * cannot see). */
 int dh_attn_spec_decode_for(const dh_attn_spec* spec, const float* d_qkv, void* d_cache_k, void* d_cache_v, float* d_out,
                             int pos, const uint32_t* d_kv_len, int max_kv_len, void* d_workspace, int rows, int* left);
 /* C[N] = W [attention | x[H * VD ..]] + residual for the splits a dh_attn_spec_decode_for with the same spec, row, workspace and key count has left

@@ -779,11 +779,12 @@ def test_decode_with_the_key_count_on_the_device(L, window):
 
 @pytest.mark.parametrize("cache", ["f16", "f32"])
 @pytest.mark.parametrize("H,G,d,e,window,n,rows,ff,merged", [(4, 2, 64, 48, 0, 700, 2050, 72, True), (2, 2, 24, 40, 129, 400, 30, 0, True), (16, 8, 128, 128, 1024, 1200, 2048, 64, True),
-                                                             (40, 40, 64, 24, 300, 400, 1030, 704, True), (6, 2, 24, 40, 300, 400, 100, 8, False), (4, 2, 64, 64, 64, 300, 100, 0, False),
+                                                             (40, 40, 64, 24, 300, 400, 1030, 704, False), (16, 16, 64, 24, 300, 400, 1030, 704, True), (18, 6, 64, 24, 300, 400, 1030, 704, False),
+                                                             (32, 32, 64, 24, 300, 400, 2050, 704, True), (33, 33, 64, 24, 300, 400, 2050, 704, False), (6, 2, 24, 40, 300, 400, 100, 8, False), (4, 2, 64, 64, 64, 300, 100, 0, False),
                                                              (32, 16, 128, 128, 1024, 1100, 4096, 0, False), (3, 3, 40, 264, 0, 300, 64, 0, False)])
 def test_splits_left_to_the_product_behind(L, H, G, d, e, window, n, rows, ff, merged, cache):
     """A step's attention and the product that reads it, the key splits merged by the product or by a launch of their own, and with the key count on the
-    device: one to eight splits of 128 keys, heads of up to 16 lanes one and two at a time, part of a wave's heads and more than four, other activations
+    device: one to eight splits of 128 keys, heads of up to 16 lanes one and two at a time, part of a wave's heads and all four of them in products of four and of eight waves, other activations
     beside the heads'; more heads at once, few keys, many bytes of splits and long heads are merged as ever.  The same 32-bit sums in another order: 24
     roundings of the terms' sizes."""
     a, b, c = (Attn(L, H, G, d, e, window, cache, n=n, seed=31) for _ in range(3))
@@ -856,6 +857,24 @@ def test_few_heads_over_many_keys(L, H, G, d, e, n, merged):
                 capi.check(L.dh_dense_gemv(mixed.data_ptr(), None, 0, 0.0, W.data_ptr(), K, rows, K, 1.0, None, None, y.data_ptr(), rows, None, capi.ACT_NONE))
             capi.check(L.dh_sync())
             assert ((y.double() - want).abs() <= (n / 32 + K / 32) * 2.0 ** -24 * size).all(), (p, on_device)
+
+
+def test_splits_in_front_of_a_product_of_other_rows(L):
+    """More heads than a product's waves make factors of at once: the bits of a product of eight waves that has the same rows and more."""
+    a, K = Attn(L, 32, 32, 64, 24, 300, n=400, seed=31), 32 * 24
+    g = torch.Generator(device="cuda").manual_seed(3)
+    W, src, x = (torch.randn(2050, K, generator=g, device="cuda") / K ** 0.5).to(torch.bfloat16), a.rows(), torch.zeros(K, device="cuda")
+    left, row, spec = ctypes.c_int(), src.data_ptr() + 4 * a.ld * 399, ctypes.byref(a.spec)
+    torch.cuda.synchronize()
+    capi.check(L.dh_attn_spec_kv_write(spec, src.data_ptr(), a.kc.data_ptr(), a.vc.data_ptr(), 400, 0))
+    capi.check(L.dh_attn_spec_decode_for(spec, row, a.kc.data_ptr(), a.vc.data_ptr(), x.data_ptr(), 399, None, 400, a.ws.data_ptr(), 2050, ctypes.byref(left)))
+    outs = []
+    for rows in (2050, 100):
+        outs.append(torch.zeros(rows, device="cuda"))
+        torch.cuda.synchronize()
+        capi.check(L.dh_dense_gemv_attn(spec, row, a.ws.data_ptr(), left.value, None, 400, x.data_ptr(), W.data_ptr(), K, rows, K, None, outs[-1].data_ptr()))
+        capi.check(L.dh_sync())
+    assert left.value > 1 and outs[0].abs().sum() > 0 and torch.equal(outs[0][:100], outs[1])
 
 
 def test_splits_of_another_count_are_refused(L):

@@ -61,16 +61,20 @@ __device__ __forceinline__ float group_combine(float v, Op op) {
   return v;
 }
 
-// A row that 256 threads hold, four elements at 4 (tid + 1024 j / 4) each (zeros past `hidden`, a multiple of 4 and at most 8192), over its root mean square and
+// A row that 256 threads hold, four elements at 4 (tid + 256 j) each (zeros past `hidden`, a multiple of 4 and at most 1024 PIECES), over its root mean square and
 // times w, in the operand type of the product that reads it; columns hidden .. ld_out - 1 zero.
 constexpr int kNormPieces = 8;
-template <bool BF16>
-__device__ __forceinline__ void store_normed_row(const float4 (&xv)[kNormPieces], int hidden, const float* __restrict__ w, float eps, float* red, void* __restrict__ out,
+// Pieces where a row is made of several in the same launch.  Longer rows take a wide launch and the norm's: one workgroup's trips through 8192 columns of a few
+// rows took longer than the launch they saved (products in slices with their norm, us, apart / in one, from 8192 columns: 16 x 4096 19.3 / 18.1, 5 x 5120
+// 21.3 / 23.0, 16 x 6144 24.2 / 25.5, 33 x 8192 32.1 / 33.4; from 4096 200 x 7168 33.2 / 32.8).
+constexpr int kMadePieces = 4;
+template <bool BF16, int PIECES>
+__device__ __forceinline__ void store_normed_row(const float4 (&xv)[PIECES], int hidden, const float* __restrict__ w, float eps, float* red, void* __restrict__ out,
                                                  int64_t base, int ld_out) {
   const int tid = threadIdx.x;
   float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < kNormPieces; j++) {
+  for (int j = 0; j < PIECES; j++) {
     ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss);
     ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss);
   }
@@ -83,7 +87,7 @@ __device__ __forceinline__ void store_normed_row(const float4 (&xv)[kNormPieces]
     else static_cast<float*>(out)[base + i] = v;
   };
 #pragma unroll
-  for (int j = 0; j < kNormPieces; j++) {
+  for (int j = 0; j < PIECES; j++) {
     const int i = 4 * (tid + 256 * j);
     if (i >= hidden) continue;
     const float4 wv = *reinterpret_cast<const float4*>(w + i);

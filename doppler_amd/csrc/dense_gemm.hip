@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a, int 
   }
 }
 
-// The same where all columns are a first output's and the rows are normed behind it: one workgroup a row (N a multiple of 4, at most 8192, everything
+// The same where all columns are a first output's and the rows are normed behind it: one workgroup a row (N a multiple of 4, at most 4096, everything
 // aligned).  The norm's launch was 3.1 us and 1.4 in front of the next: 301 rows of 1024 in three slices 4.4 + 3.1 -> 5.0 us.
 template <bool BF16>
 __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(const GemmArgs a, int slices) {
@@ -516,9 +516,9 @@ __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(const GemmArgs a,
   const int64_t total = (int64_t)a.M * a.N;
   const float *p = a.parts + (int64_t)m * a.N, *res = a.residual ? a.residual + (int64_t)m * a.ldc : nullptr;
   float* c = a.C + (int64_t)m * a.ldc;
-  float4 x[dh::kNormPieces];
+  float4 x[dh::kMadePieces];
 #pragma unroll
-  for (int j = 0; j < dh::kNormPieces; j++) {
+  for (int j = 0; j < dh::kMadePieces; j++) {
     const int n = 4 * (threadIdx.x + 256 * j);
     x[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (n >= a.N) continue;
@@ -625,7 +625,7 @@ int launch_16bit_kernel(const char* op, GemmArgs a, int slices) {
   return 0;
 }
 int launch_reduce(const char* op, const GemmArgs& a, int slices) {
-  if (a.norm_weight && a.n_first == a.N && a.N % 4 == 0 && a.N <= 1024 * dh::kNormPieces && a.ldc % 4 == 0 &&
+  if (a.norm_weight && a.n_first == a.N && a.N % 4 == 0 && a.N <= 1024 * dh::kMadePieces && a.ldc % 4 == 0 &&
       ((reinterpret_cast<uintptr_t>(a.C) | reinterpret_cast<uintptr_t>(a.residual) | reinterpret_cast<uintptr_t>(a.bias) |
         reinterpret_cast<uintptr_t>(a.col_scale)) & 15) == 0) {
     auto kern = a.normed_dtype == DH_BF16 ? gemm_reduce_norm_kernel<true> : gemm_reduce_norm_kernel<false>;

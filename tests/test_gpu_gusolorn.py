@@ -752,6 +752,13 @@ def test_products_that_leave_normed_rows(L, M, N, K, sliced, dtype):
 
 
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F32])
+@pytest.mark.parametrize("M,N,K", [(3, 4092, 4096), (20, 4096, 4096), (20, 4100, 4096), (9, 5120, 8192)])
+def test_products_around_the_longest_rows_that_are_normed_with_them(L, M, N, K, dtype):
+    test_products_that_leave_normed_rows(L, M, N, K, None, dtype)
+
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F32])
 @pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(40, 256, 8, 2, 64, 128), (1531, 1024, 4, 2, 512, 1024), (1000, 1024, 5, 2, 512, 1024), (50, 192, 4, 4, 64, 0), (3, 8256, 2, 1, 64, 0)])
 def test_experts_that_leave_normed_rows(L, T, K, E, top, ff, shared_ff, dtype):
     """The bits of the experts and a norm, in place of the rows they read: a shared expert whose product is in the sum, or comes behind it, or is not there."""

@@ -640,8 +640,10 @@ __global__ __launch_bounds__(256) void experts_combine_kernel(const float* __res
   }
 }
 
-// The same where nothing is added behind it, and the rows normed for the product that reads them: one workgroup a row (at most 8192 columns, a multiple of
-// four, x and ls aligned).  Against a launch of the norm's own, us: 1531 rows of 2048 18.9 + 5.6 -> 17.1, 40 of 1024 4.3 + 3.1 -> 4.8.
+// The same where nothing is added behind it, and the rows normed for the product that reads them: one workgroup a row (at most 4096 columns, a multiple of
+// four, x and ls aligned).  Against a launch of the norm's own, us: 1531 rows of 2048 18.9 + 5.6 -> 17.1, 40 of 1024 4.3 + 3.1 -> 4.8.  What a thread adds up one
+// after the other is its pieces times the choices: whole portions of 16 tokens, apart / in one, 32 choices of 3072 columns 59.6 / 57.3, of 4096 66.9 / 68.1, of 8192 97.4
+// / 112.3, 16 of 4096 60.4 / 60.2, of 6144 76.3 / 79.2, two of 8192 72.1 / 74.8.
 template <bool BF16>
 __global__ __launch_bounds__(256) void experts_combine_norm_kernel(const float* __restrict__ y, int64_t ld_y, const int* __restrict__ slot, int top,
                                                                    const float* __restrict__ shared, const float* __restrict__ ls, float* __restrict__ x,
@@ -651,9 +653,9 @@ __global__ __launch_bounds__(256) void experts_combine_norm_kernel(const float* 
   const int t = blockIdx.x;
   const int* places = slot + (int64_t)t * top;
   float* row = x + (int64_t)t * ld_x;
-  float4 out[dh::kNormPieces];
+  float4 out[dh::kMadePieces];
 #pragma unroll
-  for (int j = 0; j < dh::kNormPieces; j++) {
+  for (int j = 0; j < dh::kMadePieces; j++) {
     const int i = 4 * (threadIdx.x + 256 * j);
     out[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (i >= hidden) continue;
@@ -675,6 +677,7 @@ __global__ __launch_bounds__(256) void experts_combine_norm_kernel(const float* 
   }
   dh::store_normed_row<BF16>(out, hidden, norm, eps, red, normed, (int64_t)t * ld_normed, ld_normed);
 }
+bool sums_in_passing(int hidden, int top) { return hidden <= 1024 * dh::kMadePieces && (int64_t)hidden * top <= 3 << 15; }
 
 // Where a step's first kernel makes the logits too (20 are what its waves hold).  Four pieces of a row leave three workgroups to a compute unit's registers, and
 // a fourth would wait for one of them to end; and what a launch saves is more than twenty rows' reading only where there are few workgroups or the rows are long.
@@ -906,7 +909,7 @@ int prefill(const char* op, const dh_experts* spec, const void* d_h, int operand
   } else {
     if (int rc = dh::experts_down(op, routed_down.rows, w + p.act, operand, spec->ff, down, spec->ff, spec->hidden, spec->ff, f32(p.y), p.ld_y)) return rc;
   }
-  if (next.weight && (!shared || down_pair) && spec->hidden % 4 == 0 && spec->hidden <= 1024 * dh::kNormPieces && ld_x % 4 == 0 && aligned(d_x) &&
+  if (next.weight && (!shared || down_pair) && spec->hidden % 4 == 0 && sums_in_passing(spec->hidden, spec->top) && ld_x % 4 == 0 && aligned(d_x) &&
       aligned(spec->d_layer_scale)) {
     auto kern = operand == DH_BF16 ? experts_combine_norm_kernel<true> : experts_combine_norm_kernel<false>;
     hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, dh::stream(), f32(p.y), (int64_t)p.ld_y, i32(p.slot), spec->top, down_pair ? f32(p.shared_y) : nullptr,

@@ -757,7 +757,6 @@ def test_products_around_the_longest_rows_that_are_normed_with_them(L, M, N, K, 
     test_products_that_leave_normed_rows(L, M, N, K, None, dtype)
 
 
-
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F32])
 @pytest.mark.parametrize("T,K,E,top,ff,shared_ff", [(40, 256, 8, 2, 64, 128), (1531, 1024, 4, 2, 512, 1024), (1000, 1024, 5, 2, 512, 1024), (50, 192, 4, 4, 64, 0), (3, 8256, 2, 1, 64, 0)])
 def test_experts_that_leave_normed_rows(L, T, K, E, top, ff, shared_ff, dtype):
@@ -777,6 +776,11 @@ def test_experts_that_leave_normed_rows(L, T, K, E, top, ff, shared_ff, dtype):
     capi.check(L.dh_experts_prefill_normed(ctypes.byref(spec), h.data_ptr(), dtype, y.data_ptr(), K, ws.data_ptr(), T, norm.data_ptr(), 1e-5, h.data_ptr(), K))
     capi.check(L.dh_sync())
     assert torch.equal(x, y) and torch.equal(a, h)
+
+
+@pytest.mark.parametrize("T,K,E,top", [(17, 3072, 32, 32), (17, 3136, 32, 32), (5, 4096, 24, 24), (5, 4096, 25, 25), (9, 4160, 3, 2)])
+def test_experts_around_the_longest_rows_that_are_normed_with_them(L, T, K, E, top):
+    test_experts_that_leave_normed_rows(L, T, K, E, top, 64, 0, capi.BF16)
 
 
 @pytest.mark.parametrize("K", [256, 1024, 2112])

@@ -973,6 +973,17 @@ bool takes_wide(int64_t M, int64_t N, int64_t K, bool dual) {
   return dh::ceil_div(M, 256) * dh::ceil_div(N, 128) >= dh::num_cus() || (double)M * N * K * (dual ? 2 : 1) >= (M >= 1024 && !dual ? 2e9 : 5e9);
 }
 
+// Pieces of K with which 128 x 128 tiles of q4k_gemm_kernel occupy half of the compute units, or 0 where no number of them does.
+int big_tile_pieces(int64_t M, int64_t N, int64_t K) {
+  const int64_t cus = dh::num_cus(), tiles = dh::ceil_div(M, 128) * dh::ceil_div(N, 128);
+  if (2 * tiles >= cus) return 1;
+  size_t ws_bytes = 0;
+  (void)dh::splitk_workspace(&ws_bytes);
+  int64_t pieces = std::min<int64_t>({8, cus / tiles, dh::ceil_div(K, BK) / 8});
+  while (pieces > 1 && (size_t)pieces * M * N * sizeof(float) > ws_bytes) pieces--;
+  return pieces > 1 && 2 * tiles * pieces >= cus ? (int)pieces : 0;
+}
+
 // Few rows: q4k_wide_kernel on tiles of 32 or 64 rows x 128 weight rows (two waves), two such groups along k (three: 35.3 -> 37.8 us for the
 // pair of 64 x 12288 x 4096, their waves do not divide among four SIMDs).  There a weight is dequantised once, in the registers of the wave that
 // multiplies it, and read from LDS as nibbles; q4k_gemm_kernel writes and reads it there as f16 and reads the activations for every 32 columns: 72 KB a
@@ -981,7 +992,10 @@ bool takes_wide(int64_t M, int64_t N, int64_t K, bool dual) {
 // products 16 x 4096 x 4096 17.6 / 14.5, 20 x 4096 x 12288 29.2 / 21.6, 64 x 12288 x 2048 25.0 / 18.2, 16 x 28672 x 4096 51 / 30.
 // What a super-block costs a group was fitted to those (3.0 us on 32 rows, 3.7 on 64), as long as the tiles run at once.  Where the lines lie: pairs of
 // over 512 rows (796 x 1536 x 1472 27.7 / 28.2) or under 1024 k on 64-row tiles (170 x 5000 x 640 13.3 / 14.1), products of under 8e6 weights or 2048 columns (64 x 2048 x 2048 12.0 / 13.2, 16 x 2048 x 3072 11.8 / 12.3,
-// but 16 x 2048 x 4096 16.1 / 12.6; 54 x 1536 x 5504 15.3 / 16.4), of over 64 rows that take long (122 x 8448 x 8448 42 / 54, 67 x 6208 x 8320 32.6 / 36.9, but
+// but 16 x 2048 x 4096 16.1 / 12.6; 54 x 1536 x 5504 15.3 / 16.4), where the other kernel has 64 x 64 tiles, whose pieces of K overlap one another's waits (20 x
+// 2609 x 3172 12.6 / 16.0, 59 x 3612 x 2388 14.1 / 16.4, 32 x 16227 x 716 10.8 / 11.7, and with its 128-row tiles 26 x 3998 x 2228 16.8 / 14.3; of over 64 rows it
+// has two of them, 70 x 16044 x 612 12.0 / 13.5, 122 x 3957 x 2480 18.3 / 19.6, but from 1024 to 2047 k 94 x 7832 x 1040 16.0 / 12.4, 119 x 4521 x 1872 17.7 / 15.9), of
+// over 64 rows that take long (122 x 8448 x 8448 42 / 54, 67 x 6208 x 8320 32.6 / 36.9, but
 // 100 x 12000 x 2000 27.1 / 21.0, 128 x 2048 x 6144 25.3 / 21.3).
 constexpr int kNarrowGroups = 2;
 struct NarrowChoice {
@@ -991,6 +1005,7 @@ NarrowChoice choose_narrow(int64_t M, int64_t N, int64_t K, bool dual) {
   const int64_t cus = dh::num_cus(), blocks = dh::ceil_div(K, kQK);
   if (blocks < kNarrowGroups) return {0, 1};
   if (dual ? M > 512 : M > 128 || N < 2048 || N * K < 8000000) return {0, 1};
+  if (!dual && K >= 512 && !(M > 64 && K >= 1024 && K < 2048) && big_tile_pieces(M, N, K) == 0) return {0, 1};
   size_t ws_bytes = 0;
   (void)dh::splitk_workspace(&ws_bytes);
   const int64_t most = dual ? 1 : std::min<int64_t>({kMaxSplit, blocks / kNarrowGroups, std::max<int64_t>(1, ws_bytes / ((size_t)M * N * sizeof(float)))});
@@ -1088,13 +1103,10 @@ int launch_gemm(GemmArgs a, const char* op) {
     // 128 x 128 tiles with K cut into pieces when that fills the compute units: their matrix-core
     // share is higher than that of 64 x 64 tiles
     if (env_big) {
-      const int nkt = (a.K + BK - 1) / BK;
+      const int nkt = (a.K + BK - 1) / BK, split = big_tile_pieces(a.M, a.N, a.K);
       size_t ws_bytes = 0;
       float* ws = dh::splitk_workspace(&ws_bytes);
-      int split = (int)std::min<int64_t>(8, dh::num_cus() / std::max<int64_t>(1, big_tiles));
-      split = std::min(split, nkt / 8);
-      while (split > 1 && (size_t)split * a.M * a.N * sizeof(float) > ws_bytes) split--;
-      if (split > 1 && ws && big_tiles * split * 2 >= dh::num_cus()) {
+      if (split > 1 && ws) {
         a.kt_per_split = (int)dh::ceil_div(nkt, split);
         a.ksplit = (int)dh::ceil_div(nkt, a.kt_per_split);
         a.partial = ws;

@@ -993,15 +993,17 @@ def test_prefill_products_of_the_wide_kernel(M, N, K, pair, f16_out, tile):
 
 
 # Few rows: tiles of 32 and 64 rows, two groups of waves along k.  Rows that end a tile and begin one, ragged columns, runs of super-blocks that two
-# groups and several pieces do not share evenly, K off the 64 and the 256; the least K and two rounds of tiles.
+# groups and several pieces do not share evenly, K off the 64 and the 256; the least K and two rounds of tiles.  Where they are taken ends at products of the other
+# kernel's 64 x 64 tiles, but for more than 64 rows from 1024 to 2047 k.
 # (Two rounds with K = 513: a column of one super-block and one weight more takes its error from the f16 rounding of a few scales, and the largest of 33001 such
 # is 4.23e-3 of its column, on these tiles and on q4k_gemm_kernel's alike to the last digit; with three super-blocks 2.23e-3, the same on both.  A pair's
 # columns, products of two such, reach 6.29e-3 among 20001 of 29 x 300, again on both: its rounds are the plain product's, and it has 4099.)
 NARROW_PRODUCTS = [
-    (16, 4096, 4096, False, False, (32, 8)), (17, 2100, 3990, False, True, (32, 8)), (31, 16130, 500, False, False, (32, 1)), (33, 2049, 4100, False, False, (32, 6)),
+    (16, 4096, 4096, False, False, (32, 8)), (17, 2100, 3990, False, True, None), (17, 2100, 4102, False, True, (32, 6)), (20, 16400, 612, False, False, (32, 1)), (31, 16130, 500, False, False, (32, 1)), (33, 2049, 4100, False, False, (32, 6)),
     (32, 33001, 513, False, False, (32, 1)), (64, 28672, 324, False, False, (64, 1)), (65, 11999, 1540, False, True, (64, 1)), (128, 2048, 6144, False, False, (64, 6)),
     (18, 70, 513, True, False, (32, 1)), (32, 129, 260, True, False, (32, 1)), (29, 4099, 300, True, False, (32, 1)), (95, 130, 4700, True, False, (32, 1)),
-    (64, 12288, 1100, True, False, (64, 1)), (129, 4099, 1029, True, False, (64, 1)), (1024, 1030, 1300, True, False, None)]
+    (64, 12288, 1100, True, False, (64, 1)), (129, 4099, 1029, True, False, (64, 1)), (1024, 1030, 1300, True, False, None), (20, 16200, 612, False, False, None),
+    (70, 7400, 1100, False, False, (32, 1)), (70, 3960, 2100, False, True, None), (26, 3998, 2228, False, False, (32, 3)), (26, 3960, 2228, False, False, None)]
 
 
 @pytest.mark.parametrize("M,N,K,pair,f16_out,tile", NARROW_PRODUCTS)

@@ -597,8 +597,12 @@ SplitKernel split_kernel_for(int D, bool qkv, int G, bool two) {
 // group, 1608 with two; 6000 keys 10.1 / 9.7 us; without a second chunk the group would only wait).  A call that is recorded for replays at other
 // positions has two at every length, since a replay changes the grid and not the kernel; the sums are the same.
 bool two_groups(const AttnArgs& a, bool recorded) {
-  const int keys = a.dyn.kv_len_ptr ? a.dyn.max_kv_len : a.kend - a.kbeg;
-  return recorded || dh::ceil_div(keys, kTileKeys) > a.nsplit;
+  int keys = a.kend - a.kbeg, splits = a.nsplit;
+  if (a.dyn.kv_len_ptr) {                              // (the launch has the splits of any count; what is visible is bounded by the window)
+    keys = a.dyn.sliding_window > 0 ? std::min(a.dyn.max_kv_len, a.dyn.sliding_window) : a.dyn.max_kv_len;
+    splits = splits_for(a.dyn.one_per_cu, keys);
+  }
+  return recorded || dh::ceil_div(keys, kTileKeys) > splits;
 }
 MergeKernel merge_kernel_for(int D) { return D == 64 ? attn_decode_merge_kernel<64> : attn_decode_merge_kernel<128>; }
 

@@ -992,6 +992,27 @@ def test_prefill_products_of_the_wide_kernel(M, N, K, pair, f16_out, tile):
     assert worst.max().item() < 4e-3 and ((got - want).norm(dim=0) / want.norm(dim=0)).max().item() < 4e-3
 
 
+@pytest.mark.parametrize("window", [64, 2047, 2048, 2049, 2112, 0])
+def test_decode_attention_in_a_window_counted_on_the_device(window):
+    """A launch for any count up to 6000 and one for the count: windows of as many chunks as there are splits, and one more (the groups of waves that share a
+    split).  The same sums in at most 47 partial ones: as many roundings of the largest value."""
+    L = capi.init(torch.cuda.current_device())
+    H, Hkv, D, most = 16, 8, 64, 6000
+    g = torch.Generator(device="cuda").manual_seed(window)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    K, V, qkv, w, table = n(most, Hkv, D).half(), n(most, Hkv, D).half(), n((H + 2 * Hkv) * D), torch.ones(D, device="cuda"), torch.rand(2, most, D // 2, generator=g, device="cuda")
+    ws = torch.zeros(int(L.dh_attn_decode_workspace_bytes(H, D, most)), dtype=torch.uint8, device="cuda")
+    for count in (1, 63, 2048, 2050, 2113, most):
+        outs, kv = [torch.zeros(H, D, device="cuda") for _ in range(2)], torch.full((1,), count, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        args = (qkv.data_ptr(), w.data_ptr(), w.data_ptr(), table[0].data_ptr(), table[1].data_ptr(), K.data_ptr(), V.data_ptr())
+        tail = (D, 0, 1e-6, 0, 1, D ** -0.5, 0.0, window, 0, 0, ws.data_ptr())
+        capi.check(L.dh_attn_decode_qkv(*args, outs[0].data_ptr(), H, Hkv, D, count - 1, *tail))
+        capi.check(L.dh_attn_decode_qkv_kvlen(*args, outs[1].data_ptr(), H, Hkv, D, kv.data_ptr(), most, *tail))
+        capi.check(L.dh_sync())
+        assert outs[0].abs().sum() > 0 and (outs[0] - outs[1]).abs().max() <= 47 * 2.0 ** -24 * V.float().abs().max(), count
+
+
 # Few rows: tiles of 32 and 64 rows, two groups of waves along k.  Rows that end a tile and begin one, ragged columns, runs of super-blocks that two
 # groups and several pieces do not share evenly, K off the 64 and the 256; the least K and two rounds of tiles.  Where they are taken ends at products of the other
 # kernel's 64 x 64 tiles, but for more than 64 rows from 1024 to 2047 k.

@@ -416,7 +416,8 @@ __global__ __launch_bounds__(256) void gather_f16_kernel(const uint32_t* __restr
 }
 
 // The same, four elements a thread and a row's 1024 a workgroup: rows of whole pieces whose operands allow wide accesses.  A division of 64 bits
-// and two bytes a thread are what the other form spends its time on (2048 rows of 4096: 27.1 -> 13.1 us).
+// and two bytes a thread are what the other form spends its time on (2048 rows of 4096: 27.1 -> 13.1 us).  Rows of less than 256 leave most of a workgroup idle
+// (us, that form / this: 8000 rows of 4 1.9 / 3.3, of 64 2.4 / 3.4, of 128 3.2 / 3.6, of 192 4.1 / 3.8, 200 of 384 1.9 / 1.9, 2048 of 640 3.7 / 2.6).
 __global__ __launch_bounds__(256) void gather_f16_pieces_kernel(const uint32_t* __restrict__ ids, const __half* __restrict__ table, float* __restrict__ out, int hidden,
                                                                 uint32_t vocab, int index_offset) {
   const int d = 4 * (int)(blockIdx.y * 256 + threadIdx.x);
@@ -844,7 +845,7 @@ int dh_gather_f16(const uint32_t* d_ids, const void* d_table, float* d_out, int 
   if (!d_ids || !d_table || !d_out) return dh::fail(1, "[%s] null pointer", op);
   const int64_t total = (int64_t)T * hidden;
   // (a workgroup a row: a launch has less than 2^32 threads along a dimension)
-  if ((hidden & 3) == 0 && hidden < (1 << 24) && T < (1 << 24) && (reinterpret_cast<uintptr_t>(d_table) & 7) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0)
+  if ((hidden & 3) == 0 && hidden >= 256 && hidden < (1 << 24) && T < (1 << 24) && (reinterpret_cast<uintptr_t>(d_table) & 7) == 0 && (reinterpret_cast<uintptr_t>(d_out) & 15) == 0)
     hipLaunchKernelGGL(gather_f16_pieces_kernel, dim3((unsigned)T, (unsigned)dh::ceil_div(hidden, 1024)), dim3(256), 0, dh::stream(), d_ids,
                        static_cast<const __half*>(d_table), d_out, hidden, (uint32_t)vocab, index_offset);
   else

@@ -65,17 +65,33 @@ def test_words_and_embedding_in_one_launch(hidden, buckets, pos):
         assert torch.equal(outs[2], outs[3]) and torch.equal(ids, got)
 
 
-def test_more_rows_than_a_grid_has_workgroups_of():
-    """Rows of four elements: at 2^24 of them a workgroup each is more threads than a launch can have."""
+@pytest.mark.parametrize("hidden", [4, 250, 252, 256, 257, 260, 1024, 1028])
+def test_embedding_rows_of_any_length(hidden):
+    """A table's rows and zeros for ids outside it, element by element and in pieces, on tables and outputs that allow pieces and that do not."""
     L = capi.init(torch.cuda.current_device())
-    T, table = 1 << 24, torch.arange(32, device="cuda").to(torch.float16).reshape(8, 4)
+    table = torch.randn(9 * hidden + 1, device="cuda").half()
+    ids = torch.tensor([3, 0, 8, 9, 1 << 30, 8, 2], dtype=torch.int32, device="cuda")
+    for shift in (0, 1):
+        rows, out = table[shift:shift + 9 * hidden].view(9, hidden), torch.full((5 * hidden + 1,), 7.0, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_gather_f16(ids.data_ptr(), rows.data_ptr(), out.data_ptr() + 4 * shift, 5, hidden, 9, 2))
+        capi.check(L.dh_sync())
+        want = torch.cat([rows.float(), torch.zeros(1, hidden, device="cuda")])[[8, 9, 9, 8, 2]]
+        assert torch.equal(out[shift:shift + 5 * hidden].view(5, hidden), want) and out[-1 if not shift else 0] == 7.0
+
+
+def test_more_rows_than_a_grid_has_workgroups_of():
+    """At 2^24 rows a workgroup each is more threads than a launch can have, at one less it is not."""
+    L = capi.init(torch.cuda.current_device())
+    T = 1 << 24
     ids = (torch.arange(T, device="cuda") % 11).to(torch.int32)
-    out = torch.zeros(T, 4, device="cuda")
-    torch.cuda.synchronize()
-    capi.check(L.dh_gather_f16(ids.data_ptr(), table.data_ptr(), out.data_ptr(), T, 4, 8, 0))
-    capi.check(L.dh_sync())
-    want = torch.cat([table.float(), torch.zeros(3, 4, device="cuda")])[ids.long()]
-    assert torch.equal(out, want)
+    for rows, hidden in ((T, 4), (T - 1, 256)):
+        table, out = torch.arange(8 * hidden, device="cuda").to(torch.float16).reshape(8, hidden), torch.zeros(rows, hidden, device="cuda")
+        torch.cuda.synchronize()
+        capi.check(L.dh_gather_f16(ids.data_ptr(), table.data_ptr(), out.data_ptr(), rows, hidden, 8, 0))
+        capi.check(L.dh_sync())
+        want = torch.cat([table.float(), torch.zeros(3, hidden, device="cuda")])
+        assert all(torch.equal(out[a:a + (1 << 20)], want[ids[a:min(a + (1 << 20), rows)].long()]) for a in range(0, rows, 1 << 20))
 
 
 def test_words_of_a_token_are_refused_while_a_graph_is_captured():

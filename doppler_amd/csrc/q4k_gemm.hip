@@ -990,7 +990,9 @@ int big_tile_pieces(int64_t M, int64_t N, int64_t K) {
 // step of 64 k, which at 128 bytes a clock is most of its 0.6 us, whatever the number of rows.  us with packing and reduction, weights from memory, before
 // / now: pairs 16 x 12288 x 4096 42.6 / 30.3, 64 x 12288 x 4096 44 / 35, 40 x 6144 x 2048 24.3 / 18.0, 33 x 3072 x 1024 14.5 / 12.0, 512 x 1024 x 4096 40.8 / 30.3;
 // products 16 x 4096 x 4096 17.6 / 14.5, 20 x 4096 x 12288 29.2 / 21.6, 64 x 12288 x 2048 25.0 / 18.2, 16 x 28672 x 4096 51 / 30.
-// What a super-block costs a group was fitted to those (3.0 us on 32 rows, 3.7 on 64), as long as the tiles run at once.  Where the lines lie: pairs of
+// What a super-block costs a group was fitted to those (3.0 us on 32 rows, 3.7 on 64), as long as the tiles run at once, or on 32 rows in two rounds of more than
+// a short k (23 x 35392 x 296 13.5 / 15.4, 18 x 38689 x 532 17.6 / 18.3, 28 x 51643 x 788 23.6 / 23.2, 32 x 60197 x 1088 30.2 / 26.4; pairs 23 x 24571 x 312 13.4 /
+// 13.9, 25 x 25711 x 348 14.6 / 14.2, 16 x 21498 x 1520 33.3 / 25.1).  Where the lines lie: pairs of
 // over 512 rows (796 x 1536 x 1472 27.7 / 28.2) or under 1024 k on 64-row tiles (170 x 5000 x 640 13.3 / 14.1), products of under 8e6 weights or 2048 columns (64 x 2048 x 2048 12.0 / 13.2, 16 x 2048 x 3072 11.8 / 12.3,
 // but 16 x 2048 x 4096 16.1 / 12.6; 54 x 1536 x 5504 15.3 / 16.4), where the other kernel has 64 x 64 tiles, whose pieces of K overlap one another's waits (20 x
 // 2609 x 3172 12.6 / 16.0, 59 x 3612 x 2388 14.1 / 16.4, 32 x 16227 x 716 10.8 / 11.7, and with its 128-row tiles 26 x 3998 x 2228 16.8 / 14.3; of over 64 rows it
@@ -1016,7 +1018,7 @@ NarrowChoice choose_narrow(int64_t M, int64_t N, int64_t K, bool dual) {
     if (dual && bm == 64 && K < 1024) break;
     for (int64_t s = 1; s <= most; s++) {
       const int64_t each = steps_per_piece(K, (int)s) / 4, pieces = dh::ceil_div(blocks, each), rounds = dh::ceil_div(groups * pieces, cus);
-      if (rounds > (M <= 32 && s == 1 ? 2 : 1)) break;
+      if (rounds > (M <= 32 && s == 1 && K >= (dual ? 340 : 768) ? 2 : 1)) break;
       if (blocks - each * (pieces - 1) < kNarrowGroups) continue;         // the last piece, too, has a super-block for each group
       double t = (double)rounds * dh::ceil_div(each, kNarrowGroups) * (bm == 32 ? 3000.0 : 3700.0);
       if (pieces > 1) t += 3500.0 + 4.0 * M * N * (2 * pieces + 1) / 4000.0;

@@ -953,7 +953,7 @@ WIDE_PRODUCTS = [
     (1049, 1061, 1861, False, True, (128, 128, 64, 2)), (1829, 2215, 554, False, True, (128, 256, 64, 1)), (946, 1350, 4612, False, False, (128, 256, 64, 5)),
     (1582, 2529, 2601, False, False, (128, 256, 128, 1)), (1255, 1583, 7763, False, True, (128, 256, 128, 3)), (1703, 4807, 523, False, False, (256, 256, 128, 1)),
     (1538, 2528, 10169, False, False, (256, 256, 128, 2)), (525, 11517, 366, True, False, (128, 256, 64, 1)), (993, 2642, 953, True, False, (128, 256, 64, 1)), (1676, 1190, 2575, True, False, (128, 256, 128, 1)),
-    (1207, 3570, 582, True, False, (256, 256, 128, 1))]
+    (1207, 3570, 582, True, False, (256, 256, 128, 1)), (32, 33001, 513, False, False, (128, 256, 64, 1))]
 
 
 def wide_tile(M, N, K, pair, num_cus=0):
@@ -1016,12 +1016,12 @@ def test_decode_attention_in_a_window_counted_on_the_device(window):
 # Few rows: tiles of 32 and 64 rows, two groups of waves along k.  Rows that end a tile and begin one, ragged columns, runs of super-blocks that two
 # groups and several pieces do not share evenly, K off the 64 and the 256; the least K and two rounds of tiles.  Where they are taken ends at products of the other
 # kernel's 64 x 64 tiles, but for more than 64 rows from 1024 to 2047 k.
-# (Two rounds with K = 513: a column of one super-block and one weight more takes its error from the f16 rounding of a few scales, and the largest of 33001 such
-# is 4.23e-3 of its column, on these tiles and on q4k_gemm_kernel's alike to the last digit; with three super-blocks 2.23e-3, the same on both.  A pair's
-# columns, products of two such, reach 6.29e-3 among 20001 of 29 x 300, again on both: its rounds are the plain product's, and it has 4099.)
+# (A column of one super-block and one weight more takes its error from the f16 rounding of a few scales, and the largest of 33001 such is 4.23e-3 of its column, on
+# these tiles and on q4k_gemm_kernel's alike to the last digit; with three super-blocks 2.23e-3, the same on both.  A pair's columns, products of two such, reach
+# 6.29e-3 among 20001 of 29 x 300: a pair in two rounds is compared with the same columns in one, below.)
 NARROW_PRODUCTS = [
     (16, 4096, 4096, False, False, (32, 8)), (17, 2100, 3990, False, True, None), (17, 2100, 4102, False, True, (32, 6)), (20, 16400, 612, False, False, (32, 1)), (31, 16130, 500, False, False, (32, 1)), (33, 2049, 4100, False, False, (32, 6)),
-    (32, 33001, 513, False, False, (32, 1)), (64, 28672, 324, False, False, (64, 1)), (65, 11999, 1540, False, True, (64, 1)), (128, 2048, 6144, False, False, (64, 6)),
+    (32, 33001, 770, False, False, (32, 1)), (64, 28672, 324, False, False, (64, 1)), (65, 11999, 1540, False, True, (64, 1)), (128, 2048, 6144, False, False, (64, 6)),
     (18, 70, 513, True, False, (32, 1)), (32, 129, 260, True, False, (32, 1)), (29, 4099, 300, True, False, (32, 1)), (95, 130, 4700, True, False, (32, 1)),
     (64, 12288, 1100, True, False, (64, 1)), (129, 4099, 1029, True, False, (64, 1)), (1024, 1030, 1300, True, False, None), (20, 16200, 612, False, False, None),
     (70, 7400, 1100, False, False, (32, 1)), (70, 3960, 2100, False, True, None), (26, 3998, 2228, False, False, (32, 3)), (26, 3960, 2228, False, False, None)]
@@ -1032,6 +1032,28 @@ def test_prefill_products_of_few_rows(M, N, K, pair, f16_out, tile):
     out = (ctypes.c_int64 * 2)()
     assert (tuple(out) if capi.load().dh_q4k_gemm_narrow_layout(M, N, K, int(pair), 256, out) else None) == tile
     test_prefill_products_of_the_wide_kernel(M, N, K, pair, f16_out, None)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 16385, 340), (29, 20001, 340), (32, 32768, 1100)])
+def test_pairs_of_few_rows_in_two_rounds_of_tiles(M, N, K):
+    """The bits of the same columns in products of one round (which the shapes above compare with 64 bits): a column's sums do not depend on how many there are."""
+    L, out, row = capi.init(torch.cuda.current_device()), (ctypes.c_int64 * 2)(), synth.q4k_nbytes(1, K)
+    W = [torch.from_numpy(synth.q4k_tensor(N, K, seed=s)).cuda() for s in (1, 2)]
+    x, norm = torch.randn(M, K, device="cuda"), torch.rand(K, device="cuda")
+
+    def pair(first, columns):
+        y = torch.zeros(M, columns, device="cuda")
+        torch.cuda.synchronize()
+        assert L.dh_q4k_gemm_narrow_layout(M, columns, K, 1, 256, out) == 1
+        capi.check(L.dh_q4k_ffn_gate_up_rmsnorm(x.data_ptr(), norm.data_ptr(), 1e-5, 0, *(w.data_ptr() + first * row for w in W), y.data_ptr(), M, K, columns,
+                                                capi.ACT_SILU, 1.0, 0.0))
+        capi.check(L.dh_sync())
+        return y
+    half = N // 2
+    whole = pair(0, N)
+    assert L.dh_q4k_gemm_narrow_layout(M, N, 339, 1, 256, out) == 0            # (a shorter k does not pay for two rounds)
+    assert torch.isfinite(whole).all() and whole.abs().sum() > 0
+    assert torch.equal(whole[:, :half], pair(0, half)) and torch.equal(whole[:, half:], pair(half, N - half))
 
 
 def test_scale_of_a_part_holds_its_whole_shape():

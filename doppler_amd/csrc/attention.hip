@@ -120,8 +120,8 @@ typedef __attribute__((ext_vector_type(4))) float float4_t;
 // chunk.  Waves that shared a chunk's softmax and split V by dims took two barriers and twice the
 // requests per chunk; q's two parts were made in every wave from whole rows; addresses were 64-bit
 // products: 6.5 -> 5.7 us with 2049 keys of 32/8 heads of 128 in a step of 36 layers (1644 -> 1609 us),
-// 4.7 -> 4.4 with 518 keys of 16/8 heads of 64 (685 -> 672 us); 32768 keys of 16/8 heads of 128 stay
-// at 24.3 us, 5.5 TB/s.
+// 4.7 -> 4.4 with 518 keys of 16/8 heads of 64 (685 -> 672 us); 32768 keys of 16/8 heads of 128 29.0
+// -> 26.0 us, 5.2 TB/s.
 // GROUPS: where a workgroup has more than one chunk a second group of four waves takes every other
 // one.  (Two groups on the former kernel were slower, 6.8 us at 2049 keys and 31.7 at 32768: a
 // compute unit's requests were the bound.)

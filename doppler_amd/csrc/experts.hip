@@ -91,12 +91,17 @@ __device__ __forceinline__ void choose_by_places(const float* z, int E, int top,
       place += other > key || (other == key && j < lane) ? 1 : 0;
     }
   }
-  // choices behind the last logit above -infinity: the first number's expert again, for nothing (as above, where no number of 64 leaves the first as it is)
-  const unsigned long long numbers = __builtin_amdgcn_ballot_w64(lane < E && own == own);
   if (lane < E && place < top) {
-    const bool lost = key == -INFINITY;
-    ids[place] = !lost ? lane : numbers ? __builtin_ctzll(numbers) : 0;
-    zs[place] = !lost || (numbers == 0 && E == 64 && place == 0) ? own : -INFINITY;
+    ids[place] = lane;
+    zs[place] = own;
+  }
+  if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(key > -INFINITY)) < top) {
+    // choices behind the last logit above -infinity: the first number's expert again, for nothing (as above, where no number of 64 leaves the first as it is)
+    const unsigned long long numbers = __builtin_amdgcn_ballot_w64(lane < E && own == own);
+    if (lane < E && place < top && key == -INFINITY) {
+      ids[place] = numbers ? __builtin_ctzll(numbers) : 0;
+      if (numbers != 0 || E < 64 || place > 0) zs[place] = -INFINITY;
+    }
   }
 }
 __device__ __forceinline__ void choose(const float* z, int E, int top, int* ids, float* zs) {
@@ -177,18 +182,12 @@ __global__ __launch_bounds__(256) void experts_up_kernel(const StepArgs a, int i
       if (i < nx) planes[(i & 1) * np + (i >> 1)] = scaled(xv[j], inv, wv[j]);
     }
     __syncthreads();
-    if (np < 64 * PR)                                    // past the row's end both operands are nothing: an infinite weight times nothing is no number
-#pragma unroll
-      for (int u = 0; u < PR; u++)
-#pragma unroll
-        for (int i = 0; i < kRouterRows; i++)
-          if (lane + 64 * u >= np) rw[i][u] = make_uint4(0, 0, 0, 0);
     float sum[kRouterRows] = {};
 #pragma unroll
     for (int u = 0; u < PR; u++) {
-      const int p = min(lane + 64 * u, np - 1);
-      float4 xa = planes[p], xb = planes[np + p];
-      if (lane + 64 * u >= np) xa = xb = make_float4(0.f, 0.f, 0.f, 0.f);
+      const int p = lane + 64 * u;
+      if (p >= np) continue;                             // (an infinite weight read again past the row's end, times nothing, would be no number)
+      const float4 xa = planes[p], xb = planes[np + p];
 #pragma unroll
       for (int i = 0; i < kRouterRows; i++) {
         const uint4 w = rw[i][u];

@@ -1,7 +1,6 @@
 // Shared host-side plumbing of libdopplerhip: error reporting, the single stream every op
 // enqueues on, and launch helpers.  gfx950 only.
 #pragma once
-#include <functional>
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -66,8 +65,13 @@ inline double tuning_double(const char* name, double dflt) {
   return e ? atof(e) : dflt;
 }
 
-// Runs `enqueue` with the address of n words of pinned host memory that its launches write, waits for the stream and copies them out.
-int read_with(const char* op, uint32_t* host_dst, int n, const std::function<int(uint32_t*)>& enqueue);
+// Runs `enqueue` with the address of n words of pinned host memory that its launches write, waits for the stream and copies them out.  (A C entry calls this:
+// the callable stays where it is and nothing is allocated that could throw.)
+int read_with(const char* op, uint32_t* host_dst, int n, int (*enqueue)(void* callable, uint32_t* pinned), void* callable);
+template <class F>
+int read_with(const char* op, uint32_t* host_dst, int n, F enqueue) {
+  return read_with(op, host_dst, n, [](void* callable, uint32_t* pinned) { return (*static_cast<F*>(callable))(pinned); }, &enqueue);
+}
 
 // ---- planning (dh_q4k_matmul_plan) ------------------------------------------------------------
 // While a plan is being made on this thread the dispatchers run as usual on the shape alone: ready()

@@ -144,10 +144,10 @@ float* widened_activations(size_t* bytes) {
   *bytes = g_widened_a ? kWidenedABytes : 0;
   return g_widened_a;
 }
-int read_with(const char* op, uint32_t* host_dst, int n, const std::function<int(uint32_t*)>& enqueue) {
+int read_with(const char* op, uint32_t* host_dst, int n, int (*enqueue)(void*, uint32_t*), void* callable) {
   if (g_capturing) return fail(1, "[%s] not possible while a graph is being captured (it waits for the stream)", op);
   std::lock_guard<std::mutex> lock(g_words_mu);
-  if (int rc = enqueue(g_words)) return rc;
+  if (int rc = enqueue(callable, g_words)) return rc;
   DH_CHECK_HIP(op, hipStreamSynchronize(g_stream));
   for (int i = 0; i < n; i++) host_dst[i] = static_cast<volatile uint32_t*>(g_words)[i];
   return check_kernel_status(op);

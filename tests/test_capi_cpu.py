@@ -2,10 +2,11 @@
 and calls fail loudly (not silently) when no device has been initialised."""
 import os
 import re
+import subprocess
 
 import pytest
 
-from doppler_amd import capi
+from doppler_amd import build, capi
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -24,6 +25,12 @@ def test_library_exports_every_declared_symbol():
     lib = capi.load()
     for name in header_symbols():
         assert hasattr(lib, name), name
+
+
+def test_no_entry_holds_a_callable_that_allocates():
+    """A copy of what a callable captured is memory whose lack would be thrown through a C entry."""
+    names = subprocess.run(["nm", "-D", "--undefined-only", build.LIB], capture_output=True, text=True, check=True).stdout
+    assert "hipMalloc" in names and "bad_function_call" not in names
 
 
 def test_ops_fail_loudly_without_init():

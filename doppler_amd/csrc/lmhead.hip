@@ -259,6 +259,7 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const float* __restri
   constexpr int PER = dh::kMaxParts / 256;
   __shared__ float sv[4];
   __shared__ uint32_t si[4];
+  __shared__ int lost[4];
   float v[PER];
   uint32_t id[PER];
 #pragma unroll
@@ -273,15 +274,31 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const float* __restri
     if (beats(v[k], id[k], best.v, best.i)) { best.v = v[k]; best.i = id[k]; }
   const float most = dh::group_combine<1, 64>(best.v, dh::MaxOp());
   const uint32_t first = wave_lowest(best.v == most ? best.i : 0xFFFFFFFFu);
+  bool no_number = false;
+#pragma unroll
+  for (int k = 0; k < PER; k++) no_number |= v[k] != v[k];
+  const unsigned long long any = __builtin_amdgcn_ballot_w64(no_number);
   if ((threadIdx.x & 63) == 0) {
     sv[threadIdx.x >> 6] = most;
     si[threadIdx.x >> 6] = first;
+    lost[threadIdx.x >> 6] = any != 0;
   }
   __syncthreads();
-  if (threadIdx.x > 0) return;
   Cand c{sv[0], si[0]};
-  for (int w = 1; w < 4; w++)
-    if (beats(sv[w], si[w], c.v, c.i)) { c.v = sv[w]; c.i = si[w]; }
+  if (lost[0] | lost[1] | lost[2] | lost[3]) {
+    // what is no number is neither more nor less than a candidate, and its place decides: one after the other, in the order of the pairwise reduction
+    best = Cand{-3.402823e+38f, 0xFFFFFFFFu};
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+      if ((int)threadIdx.x + 256 * k < parts && beats(v[k], id[k], best.v, best.i)) { best.v = v[k]; best.i = id[k]; }
+    __syncthreads();
+    c = block_best_256(best, sv, si);
+    if (threadIdx.x > 0) return;
+  } else {
+    if (threadIdx.x > 0) return;
+    for (int w = 1; w < 4; w++)
+      if (beats(sv[w], si[w], c.v, c.i)) { c.v = sv[w]; c.i = si[w]; }
+  }
   // nothing beat the neutral start (every logit <= -3.4e38, NaN, or masked): index 0, as the
   // reference kernel's (NEG_INF, 0) start does
   const uint32_t token = c.i == 0xFFFFFFFFu ? 0u : c.i;

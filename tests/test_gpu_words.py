@@ -140,3 +140,36 @@ def test_token_of_a_head_on_the_host(vocab):
                                                          token.data_ptr(), 1, logits.data_ptr(), host.ctypes.data))
             want = 0 if case == 3 else int((logits == logits.max()).nonzero()[0])
             assert token.tolist() == [-1, want] and host[0] == want, (case, dtype)
+
+
+def test_logits_that_are_not_numbers():
+    """One of the candidates a head leaves is neither more nor less than another: its place decides, as it does inside a candidate's workgroup.  256 candidates of
+    which a few are no numbers, against the pairwise reduction by halves: lanes, then waves."""
+    L = capi.init(torch.cuda.current_device())
+
+    def beats(a, b):
+        return a[0] > b[0] or (not a[0] < b[0] and a[1] < b[1])
+
+    def fold(c):                                             # 64 lanes, the first one's view: the other half's best against its own half's
+        lanes = list(c)
+        for off in (32, 16, 8, 4, 2, 1):
+            lanes = [lanes[i ^ off] if beats(lanes[i ^ off], lanes[i]) else lanes[i] for i in range(64)]
+        return lanes[0]
+    g = np.random.default_rng(5)
+    ws = torch.zeros(int(L.dh_argmax_workspace_bytes()), dtype=torch.uint8, device="cuda")
+    token = torch.zeros(1, dtype=torch.int32, device="cuda")
+    for trial in range(24):
+        # a stretch of 256 logits a candidate; one logit of a stretch stands out, so that what a workgroup leaves does not depend on its own order
+        big = g.choice(np.array([np.nan, np.inf, 3.0, 4.0, 5.0], np.float32), 256, p=[(0.02, 0.3)[trial % 2], 0.02, 0.2, 0.2, (0.56, 0.28)[trial % 2]])
+        logits = np.full(65536, -np.inf, np.float32)
+        logits[np.arange(256) * 256] = big                  # (the first of a stretch: an infinity below it is less, and a number's place before it)
+        want = [(float(big[i]), 256 * i) for i in range(256)]
+        waves = [fold(want[64 * w:64 * w + 64]) for w in range(4)]
+        best = waves[0]
+        for w in waves[1:]:
+            best = w if beats(w, best) else best
+        d = torch.from_numpy(logits).cuda()
+        torch.cuda.synchronize()
+        capi.check(L.dh_argmax(d.data_ptr(), 65536, -1, 0.0, ws.data_ptr(), token.data_ptr(), 0))
+        capi.check(L.dh_sync())
+        assert token.item() == best[1], trial

@@ -296,7 +296,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_spec_kernel(const SpecArgs a)
       den = fmaf(f, ml_lds[w][g][1], den);
     }
     if (a.direct) {
-      float y = den > 0.f ? num / den : 0.f;
+      // (no weights, of keys that are no numbers: what a merge of splits of 64 keys would leave, and nothing where those are one)
+      float y = den > 0.f ? num / den : WAVES > 4 && kend - kbeg > dh::kAttnTileKeys ? num * 0.f : 0.f;
       if (a.gate_off >= 0) y *= sigmoid_f(row[a.gate_off + h]);
       const int64_t at = (int64_t)t * a.ld_out + (int64_t)h * a.VD + d;
       if (a.O16) a.O16[at] = dh::f32_to_bf16_bits(y);

@@ -877,6 +877,39 @@ def test_splits_in_front_of_a_product_of_other_rows(L):
     assert left.value > 1 and outs[0].abs().sum() > 0 and torch.equal(outs[0][:100], outs[1])
 
 
+@pytest.mark.parametrize("what", ["key", "value", "query", "new key"])
+def test_what_is_no_number_is_none_behind_a_product_either(L, what):
+    """A lost element of a key, a value or the step's row: the product's outputs are lost in front of a product as they are behind a merge of their own, in one
+    split of 128 keys, in several, and where 64 keys are one."""
+    n, H, G, d = 300, 4, 2, 64
+    W = torch.ones(70, H * d, dtype=torch.bfloat16, device="cuda")
+    for p in (5, 62, 63, 64, 100, 127, 128, 200, 299):
+        ys = []
+        for rows in (0, 70):
+            a = Attn(L, H, G, d, d, 0, n=n, seed=3, bias=False)
+            src = a.rows()
+            capi.check(L.dh_attn_spec_kv_write(ctypes.byref(a.spec), src.data_ptr(), a.kc.data_ptr(), a.vc.data_ptr(), n, 0))
+            capi.check(L.dh_sync())
+            if what == "key": a.kc[p // 2, 1, 7] = float("nan")
+            if what == "value": a.vc[p // 2, 1, 7] = float("nan")
+            if what == "query": src[p, 2 * d + 3] = float("nan")
+            if what == "new key": src[p, a.ko + d + 3] = float("nan")
+            x, y, left = torch.zeros(H * d, device="cuda"), torch.zeros(70, device="cuda"), ctypes.c_int(0)
+            torch.cuda.synchronize()
+            step = (ctypes.byref(a.spec), src.data_ptr() + 4 * a.ld * p, a.kc.data_ptr(), a.vc.data_ptr(), x.data_ptr(), p, None, n, a.ws.data_ptr())
+            if rows:
+                capi.check(L.dh_attn_spec_decode_for(*step, rows, ctypes.byref(left)))
+            else:
+                capi.check(L.dh_attn_spec_decode(*step))
+            if left.value:
+                capi.check(L.dh_dense_gemv_attn(*step[:2], a.ws.data_ptr(), left.value, None, n, x.data_ptr(), W.data_ptr(), H * d, 70, H * d, None, y.data_ptr()))
+            else:
+                capi.check(L.dh_dense_gemv(x.data_ptr(), None, 0, 0.0, W.data_ptr(), H * d, 70, H * d, 1.0, None, None, y.data_ptr(), 70, None, capi.ACT_NONE))
+            capi.check(L.dh_sync())
+            ys.append(y)
+        assert torch.equal(ys[0].isnan(), ys[1].isnan()), p
+
+
 def test_splits_of_another_count_are_refused(L):
     """The device's key count says how many splits a product reads: they have to be those of the most keys it can be."""
     a = Attn(L, 4, 2, 64, 48, 0, n=700, seed=9)
